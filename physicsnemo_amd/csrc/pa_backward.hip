@@ -18,6 +18,7 @@
 //   d x_mid[n,:] = sum_s d z[n,s] Ws[s,:]
 #include "pa_common.h"
 #include "pa_host.h"
+#include "pa_mfma_ops.h"
 
 namespace pa {
 namespace backward {
@@ -162,6 +163,156 @@ __global__ __launch_bounds__(kAttnBwdThreads) void slice_attention_backward_kern
   for (int s = t; s < S; s += kAttnBwdThreads) {
     float acc = 0.f;
     for (int d = 0; d < D; ++d) acc = fmaf(dtok[s * D1 + d], tok[s * D1 + d], acc);
+    d_norm[(int64_t)bh * S + s] = -acc / slice_norm[(int64_t)bh * S + s];
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// slice_attention_backward_mfma_kernel: the same gradients with every product on v_mfma_f32_32x32x2_f32 (fp32 products
+// and sums).  One workgroup of 8 waves per (b, h); all operands sit in LDS as fp32, S and D padded with zeros to whole
+// 32 x 32 tiles, rows one word longer than a tile multiple so that both the row-wise and the column-wise operand reads
+// fall on 32 different banks; the waves share the output tiles of each step.  P and dSc live in LDS too, or (SCRATCH:
+// S = 128 does not leave room) in the caller's 2 S^2 floats per (b, h), which stay in the L2.
+// Bound by the latency of its ten dependent steps (B * H workgroups, 8 for one sample of an eight-head layer): the
+// kernel above spends 155 us on S = 64, D = 32 at 8 workgroups, where a thread walks its products one fma at a time
+// through LDS reads; the tiles take 35 us (B = 8: 147 -> 30 us; 32 workgroups of S = 32, D = 16: 27 -> 17 us).
+// ------------------------------------------------------------------------------------------------
+constexpr int kAttnMfmaWaves = kAttnBwdThreads / 64;
+
+struct AttnTiles {
+  int SP, DP, D1, S1, nS, nD;
+  __host__ __device__ AttnTiles(int S, int D) {
+    SP = (S + 31) / 32 * 32;
+    DP = (D + 31) / 32 * 32;
+    D1 = DP + 1;
+    S1 = SP + 1;
+    nS = SP / 32;
+    nD = DP / 32;
+  }
+  __host__ __device__ size_t words(bool scratch) const {
+    return (size_t)8 * SP * D1 + (size_t)3 * DP * D1 + (scratch ? 0 : (size_t)2 * SP * S1);
+  }
+};
+
+// 32 x 32 tile of A . B: element (row, k) of A at a[row * ar + k * ak], (k, column) of B at b[column * bc + k * bk]
+__device__ __forceinline__ mfma::f32x16 tile_product(const float *a, int ar, int ak, const float *b, int bc, int bk, int K,
+                                                     mfma::f32x16 acc) {
+  const int lane = threadIdx.x & 63, i = lane & 31, g = lane >> 5;
+  a += i * ar + g * ak;
+  b += i * bc + g * bk;
+  for (int k0 = 0; k0 < K; k0 += 32) {  // K: whole tiles
+#pragma unroll
+    for (int k = 0; k < 32; k += 2)
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[(k0 + k) * ak], b[(k0 + k) * bk], acc, 0, 0, 0);
+  }
+  return acc;
+}
+
+template <bool SCRATCH>
+__global__ __launch_bounds__(kAttnBwdThreads) void slice_attention_backward_mfma_kernel(
+    const float *__restrict__ slice_token, const float *__restrict__ slice_norm, const float *__restrict__ w_qkv,
+    const float *__restrict__ d_out_token, float *__restrict__ scratch, float *__restrict__ d_num,
+    float *__restrict__ d_norm, float *__restrict__ d_wqkv_part, int D, int S) {
+  using mfma::f32x16;
+  extern __shared__ float lds[];
+  const AttnTiles d(S, D);
+  const int SD = d.SP * d.D1, D1 = d.D1, PS = SCRATCH ? S : d.S1;  // PS: row stride of P and dSc
+  float *tok = lds, *dO = tok + SD, *q = dO + SD, *k = q + SD, *v = k + SD, *dq = v + SD, *dk = dq + SD, *dv = dk + SD;
+  float *wq = dv + SD;  // q|k|v weights, three blocks of DP rows
+  const int bh = blockIdx.x, t = threadIdx.x, lane = t & 63, i = lane & 31, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  float *P = SCRATCH ? scratch + (int64_t)bh * 2 * S * S : wq + 3 * d.DP * D1;
+  float *dSc = P + (int64_t)d.SP * PS;
+  f32x16 zero;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) zero[r] = 0.f;
+  auto put = [&](float *dst, int stride, const f32x16 &c, float scale) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) dst[mfma::rowmap(r, g) * stride + i] = c[r] * scale;
+  };
+
+  for (int u = t; u < d.SP * d.DP; u += kAttnBwdThreads) {
+    const int s = u / d.DP, e = u - s * d.DP;
+    const bool ok = s < S && e < D;
+    tok[s * D1 + e] = ok ? slice_token[((int64_t)bh * S + s) * D + e] : 0.f;
+    dO[s * D1 + e] = ok ? d_out_token[((int64_t)bh * S + s) * D + e] : 0.f;
+  }
+  for (int u = t; u < 3 * d.DP * d.DP; u += kAttnBwdThreads) {
+    const int row = u / d.DP, c = u - row * d.DP, m = row / d.DP, e = row - m * d.DP;
+    wq[row * D1 + c] = (e < D && c < D) ? w_qkv[(int64_t)(m * D + e) * D + c] : 0.f;
+  }
+  __syncthreads();
+  for (int job = wave; job < d.nS * 3 * d.nD; job += kAttnMfmaWaves) {  // q | k | v = tok W^T
+    const int ts = job / (3 * d.nD), te = job - ts * 3 * d.nD, m = te / d.nD, e0 = (te - m * d.nD) * 32;
+    const f32x16 c = tile_product(tok + ts * 32 * D1, D1, 1, wq + (m * d.DP + e0) * D1, D1, 1, d.DP, zero);
+    put((m == 0 ? q : m == 1 ? k : v) + ts * 32 * D1 + e0, D1, c, 1.f);
+  }
+  __syncthreads();
+  const float scale = rsqrtf((float)D);
+  for (int job = wave; job < 2 * d.nS * d.nS; job += kAttnMfmaWaves) {  // scores = q k^T / sqrt(D), dP = dO v^T
+    const int ts = (job >> 1) / d.nS, tu = (job >> 1) - ts * d.nS;
+    const bool dp = job & 1;
+    const f32x16 c = tile_product((dp ? dO : q) + ts * 32 * D1, D1, 1, (dp ? v : k) + tu * 32 * D1, D1, 1, d.DP, zero);
+    put((dp ? dSc : P) + ts * 32 * PS + tu * 32, PS, c, dp ? 1.f : scale);
+  }
+  __syncthreads();
+  for (int s = wave; s < d.SP; s += kAttnMfmaWaves) {  // softmax rows and their backward; rows and columns beyond S: 0
+    float *pr = P + s * PS, *dr = dSc + s * PS;
+    float mx = -INFINITY;
+    for (int u = lane; u < S; u += 64) mx = fmaxf(mx, pr[u]);
+    mx = wave_max(mx);
+    float sum = 0.f;
+    for (int u = lane; u < S; u += 64) sum += expf(pr[u] - mx);
+    const float inv = s < S ? 1.f / wave_sum(sum) : 0.f;
+    float delta = 0.f;
+    for (int u = lane; u < S; u += 64) delta = fmaf(expf(pr[u] - mx) * inv, dr[u], delta);
+    delta = wave_sum(delta);
+    for (int u = lane; u < d.SP; u += 64) {
+      const float p = u < S ? expf(pr[u] - mx) * inv : 0.f;
+      pr[u] = p;
+      dr[u] = u < S ? p * (dr[u] - delta) * scale : 0.f;
+    }
+  }
+  __syncthreads();
+  for (int job = wave; job < 3 * d.nS * d.nD; job += kAttnMfmaWaves) {  // dq = dSc k, dk = dSc^T q, dv = P^T dO
+    const int m = job % 3, rest = job / 3, ts = rest / d.nD, e0 = (rest - ts * d.nD) * 32;
+    const float *a = (m == 2 ? P : dSc) + ts * 32 * (m == 0 ? PS : 1);
+    const float *b = (m == 0 ? k : m == 1 ? q : dO) + e0;
+    const f32x16 c = tile_product(a, m == 0 ? PS : 1, m == 0 ? 1 : PS, b, 1, D1, d.SP, zero);
+    put((m == 0 ? dq : m == 1 ? dk : dv) + ts * 32 * D1 + e0, D1, c, 1.f);
+  }
+  __syncthreads();
+  float *dtok = q;  // q is no longer needed
+  const int njobs = d.nS * d.nD;
+  for (int job = wave; job < njobs + 3 * d.nD * d.nD; job += kAttnMfmaWaves) {
+    if (job < njobs) {  // d tok = dq Wq + dk Wk + dv Wv
+      const int ts = job / d.nD, e0 = (job - ts * d.nD) * 32;
+      f32x16 c = zero;
+#pragma unroll
+      for (int m = 0; m < 3; ++m)
+        c = tile_product((m == 0 ? dq : m == 1 ? dk : dv) + ts * 32 * D1, D1, 1, wq + m * d.DP * D1 + e0, 1, D1, d.DP, c);
+      put(dtok + ts * 32 * D1 + e0, D1, c, 1.f);
+    } else {  // dW = d(q|k|v)^T tok
+      const int w = job - njobs, m = w / (d.nD * d.nD), rest = w - m * d.nD * d.nD, te = rest / d.nD, td = rest - te * d.nD;
+      const f32x16 c =
+          tile_product((m == 0 ? dq : m == 1 ? dk : dv) + te * 32, 1, D1, tok + td * 32, 1, D1, d.SP, zero);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int e = te * 32 + mfma::rowmap(r, g), dd = td * 32 + i;
+        if (e < D && dd < D) d_wqkv_part[((int64_t)bh * 3 + m) * D * D + e * D + dd] = c[r];
+      }
+    }
+  }
+  __syncthreads();
+  for (int u = t; u < S * D; u += kAttnBwdThreads) {
+    const int s = u / D, e = u - s * D;
+    const float inv = slice_norm ? 1.f / slice_norm[(int64_t)bh * S + s] : 1.f;
+    d_num[(int64_t)bh * S * D + u] = dtok[s * D1 + e] * inv;
+  }
+  if (!slice_norm) return;
+  for (int s = t; s < S; s += kAttnBwdThreads) {
+    float acc = 0.f;
+    for (int e = 0; e < D; ++e) acc = fmaf(dtok[s * D1 + e], tok[s * D1 + e], acc);
     d_norm[(int64_t)bh * S + s] = -acc / slice_norm[(int64_t)bh * S + s];
   }
 }
@@ -496,6 +647,19 @@ size_t attention_lds_bytes(const pa_shape &s) {
 int slice_attention(const pa_shape &s, const pa_params &p, const float *slice_token, const float *slice_norm,
                     const float *d_out_token, float *scratch, float *d_num, float *d_norm, float *d_wqkv_part,
                     hipStream_t st) {
+  // The MFMA form wherever its operands fit the LDS (S <= 64 at D <= 32, or P and dSc in the scratch where S is a whole
+  // number of tiles, which covers S = 128 at D <= 32); the fma form beyond.
+  const AttnTiles tiles((int)s.S, (int)s.D);
+  const bool in_scratch = tiles.words(false) * 4 > kMaxLdsBytes;
+  if (!in_scratch || (s.S % 32 == 0 && tiles.words(true) * 4 <= kMaxLdsBytes)) {
+    const size_t bytes = tiles.words(in_scratch) * 4;
+    auto kernel = in_scratch ? slice_attention_backward_mfma_kernel<true> : slice_attention_backward_mfma_kernel<false>;
+    int rc = allow_dynamic_lds(kernel, bytes);
+    if (rc) return rc;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(s.B * s.H)), dim3(kAttnBwdThreads), bytes, st, slice_token, slice_norm,
+                       p.qkv_project_weight, d_out_token, scratch, d_num, d_norm, d_wqkv_part, (int)s.D, (int)s.S);
+    return launch_status();
+  }
   const size_t lds = attention_lds_bytes(s);
   int rc = allow_dynamic_lds(slice_attention_backward_kernel, lds);
   if (rc) return rc;

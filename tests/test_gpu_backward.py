@@ -75,6 +75,36 @@ def test_slice_attention_backward_stage():
     assert_fp32_close(d_w, w_r.grad, "d qkv weight")
 
 
+@pytest.mark.parametrize("S,D", [(1, 8), (16, 32), (33, 16), (64, 32), (64, 64), (128, 32), (96, 40), (100, 32), (128, 64)])
+@pytest.mark.parametrize("with_norm", [False, True])
+def test_slice_attention_backward_tiles(S, D, with_norm):
+    """The slice-attention backward over the shapes where its 32 x 32 tiles are ragged, where the S x S matrices move
+    from LDS to the scratch (S = 128) and where the fma kernel takes over: against autograd in float64."""
+    announce("slice attention backward", S, D, with_norm)
+    B, H = 2, 2
+    torch.manual_seed(S + D)
+    tok, d_out = torch.randn(B, H, S, D), torch.randn(B, H, S, D)
+    wqkv = torch.randn(3 * D, D) / D ** 0.5
+    norm = torch.rand(B, H, S) + 0.5
+    num_r = (tok.double() * norm.double()[..., None]).requires_grad_(True)
+    nrm_r, w_r = norm.double().requires_grad_(True), wqkv.double().requires_grad_(True)
+    tok_r = num_r / nrm_r[..., None]
+    q, k, v = (tok_r @ w_r.t()).chunk(3, dim=-1)
+    out = torch.softmax(q @ k.transpose(-1, -2) / D ** 0.5, dim=-1) @ v
+    d_tok_r, = torch.autograd.grad((out * d_out.double()).sum(), tok_r, retain_graph=True)
+    (out * d_out.double()).sum().backward()
+    dims = PF.LayerDims(B, 100, H * D, H, D, S)
+    if not PF.backward_supported(torch.float32, dims):
+        pytest.skip("shape outside the backward kernels' range")
+    params = {"qkv_project_weight": wqkv.cuda().contiguous()}
+    d_num, d_norm, d_w = PF.slice_attention_backward(tok.cuda(), norm.cuda() if with_norm else None, d_out.cuda(), params,
+                                                     dims)
+    assert_fp32_close(d_num, num_r.grad if with_norm else d_tok_r, "d slice numerators / tokens")
+    if with_norm:
+        assert_fp32_close(d_norm, nrm_r.grad, "d slice norms")
+    assert_fp32_close(d_w, w_r.grad, "d qkv weight")
+
+
 def test_bf16_layer_gradients():
     announce("bf16 backward (autocast)")
     ref, hip = make_pair("irregular", 256, 8, 32, 64, sharpen=2.0)
