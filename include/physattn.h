@@ -434,6 +434,17 @@ int pa_cols_gemm(int64_t rows, const void *a, int64_t lda, int64_t cols_a, const
 int64_t pa_cols_gemm_f32_chunks(int64_t rows, int64_t cols_a, int64_t cols_b);
 int pa_cols_gemm_f32(int64_t rows, const void *a, int64_t lda, int64_t cols_a, const void *b, int64_t ldb,
                      int64_t cols_b, float *partials, float *col_sum_partials, void *stream);
+/* The whole weight gradient of a Linear (or of a grid convolution) in one call, partial sums added up:
+ *   out[i][j] = sum_m a[m][i] * b[m][j],  col_sums[i] = sum_m a[m][i]  (NULL to skip), both float32;
+ * a (rows, cols_a) = d out, b (rows, cols_b) = the input, contiguous rows, bf16 or float32, 16-byte aligned.  With `grid`
+ * (conv_k > 0, B * N = rows) b is gathered per tap and out is (cols_a, cols_b, taps), a convolution weight's layout.
+ * Served (else PA_ERR_UNSUPPORTED): bf16 with both widths multiples of 32 and >= 128, or cols_a a multiple of 32 (of 256
+ * beyond 256) and cols_b in {32, 64, 128, 256} (no grid); float32 with both multiples of 4 and >= 16; without a grid
+ * also one width <= 16 against a multiple of 4 (>= 16).  Same sums on every call (fixed order). */
+int64_t pa_weight_grad_workspace_bytes(int dtype, int64_t rows, int64_t cols_a, int64_t cols_b, const pa_shape *grid);
+int pa_weight_grad(int dtype, int64_t rows, const void *a, int64_t cols_a, const void *b, int64_t cols_b,
+                   const pa_shape *grid, void *workspace, int64_t workspace_bytes, float *out, float *col_sums,
+                   void *stream);
 /* bf16 Linear over the rows of `in` (B, N, c_in) -> H*32 columns, weight (H*32, c_in) bf16, bias float32 or NULL:
  * `out` natural (B, N, H*32) and/or `out_pack` in the packed layout of PA_BUF_FX_PACK (either may be NULL). */
 int pa_rows_gemm_packed(const pa_shape *shape, int64_t c_in, const void *in, const void *weight, const float *bias,

@@ -36,7 +36,7 @@ EXPORTED = [
     "pa_static_scratch_bytes", "pa_slice_reduce_static",
     "pa_preprocess_query", "pa_preprocess_workspace_bytes", "pa_preprocess_forward",
     "pa_block_query", "pa_block_workspace_bytes", "pa_block_forward", "pa_markers_enabled",
-    "pa_mfma_project_softmax_reduce_clocked",
+    "pa_mfma_project_softmax_reduce_clocked", "pa_weight_grad_workspace_bytes", "pa_weight_grad",
 ]
 
 PA_BUF_BLOB, PA_BUF_FX_PACK, PA_BUF_W_PACK, PA_BUF_PARTIALS, PA_BUF_TOKP = range(5)
@@ -253,6 +253,11 @@ def load() -> ctypes.CDLL:
     lib.pa_mfma_slice_softmax_backward.argtypes = [ps, pp] + [c_void_p] * 12
     lib.pa_cols_gemm_chunks.restype = c_int64
     lib.pa_cols_gemm_chunks.argtypes = [c_int64, c_int64]
+    lib.pa_weight_grad_workspace_bytes.restype = c_int64
+    lib.pa_weight_grad_workspace_bytes.argtypes = [c_int, c_int64, c_int64, c_int64, ps]
+    lib.pa_weight_grad.restype = c_int
+    lib.pa_weight_grad.argtypes = [c_int, c_int64, c_void_p, c_int64, c_void_p, c_int64, ps, c_void_p, c_int64, c_void_p,
+                                   c_void_p, c_void_p]
     lib.pa_cols_gemm.restype = c_int
     lib.pa_cols_gemm.argtypes = [c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p]
     lib.pa_residual_layernorm.restype = c_int

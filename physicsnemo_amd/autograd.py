@@ -5,8 +5,9 @@ The reference has no backward code of its own (autograd differentiates physics_a
 this is the same gradient, assembled from
   * hand-written kernels for everything specific to the layer (slice softmax, slice sums, slice attention,
     deslice and their adjoints, the input-gradient GEMMs / transposed convolutions), and
-  * the weight gradients ``d out^T . in`` (products over the point axis) on the library's own MFMA kernel for bf16
-    shapes it serves, and on the GEMM library behind ``torch.matmul`` otherwise (fp32, convolutions, odd widths).
+  * the weight gradients ``d out^T . in`` (products over the point axis; for the structured layers against the
+    neighbours at every tap) on the library's own MFMA kernels for the shapes they serve, and on the GEMM library
+    behind ``torch.matmul`` otherwise (odd widths).
 """
 from __future__ import annotations
 
@@ -30,6 +31,7 @@ def _aligned(t: torch.Tensor) -> torch.Tensor:
 def _wgrad(d_out: torch.Tensor, inp: torch.Tensor):
     """(d W, d b) = (d out^T . in, column sums of d out) over all rows: one pass of the library's MFMA kernel where it
     serves the shape, else the GEMM library and a reduction."""
+    d_out, inp = d_out.contiguous(), inp.contiguous()
     if PF.cols_gemm_supported(d_out, inp):
         return PF.cols_gemm(d_out, inp, col_sums=True)
     ca, cb = d_out.shape[-1], inp.shape[-1]
@@ -46,15 +48,22 @@ def _wgrad(d_out: torch.Tensor, inp: torch.Tensor):
     return _rows(d_out).t() @ _rows(inp), _rows(d_out).sum(0, dtype=torch.float32)
 
 
-def _conv_weight_grad(d_out: torch.Tensor, x: torch.Tensor, grid: tuple, k: int) -> torch.Tensor:
-    """d W[o, c, taps...] = sum over grid points of d_out[p, o] * x[p + tap - k//2, c] (zero outside the grid).
+def _conv_weight_grad(d_out: torch.Tensor, x: torch.Tensor, dims):
+    """(d W, d b) of a grid convolution: d W[o, c, taps...] = sum over grid points of d_out[p, o] * x[p + tap - k//2, c]
+    (zero outside the grid), d b[o] = sum d_out[p, o].
 
-    d_out (B, N, O), x (B, N, C) channels-last over `grid`; returns (O, C, k, ..., k) in d_out's dtype."""
+    d_out (B, N, O), x (B, N, C) channels-last over the grid of `dims`.  One pass of the library's kernel where it serves
+    the widths; otherwise the GEMM library on the unfolded input (2-D) or tap by tap."""
+    if PF.cols_gemm_supported(d_out, x, dims):
+        return PF.cols_gemm(d_out, x, col_sums=True, grid=dims)
+    k = dims.conv_k
+    grid = (dims.grid_h, dims.grid_w) + ((dims.grid_d,) if dims.grid_d > 0 else ())
+    d_b = _rows(d_out).sum(0, dtype=torch.float32)
     B, O, C, nd, pad = x.shape[0], d_out.shape[-1], x.shape[-1], len(grid), k // 2
     if nd == 2:
         # one product against the unfolded (im2col) input: its columns are ordered (c, u, v) like the weight
         cols = torch.nn.functional.unfold(x.reshape(B, *grid, C).permute(0, 3, 1, 2), k, padding=pad)  # (B, C k k, N)
-        return (_rows(d_out).t() @ cols.transpose(1, 2).reshape(-1, C * k * k)).reshape(O, C, k, k)
+        return (_rows(d_out).t() @ cols.transpose(1, 2).reshape(-1, C * k * k)).reshape(O, C, k, k), d_b
     dg, xg = d_out.reshape(B, *grid, O), x.reshape(B, *grid, C)
     dW = torch.zeros((O, C) + (k,) * nd, dtype=d_out.dtype, device=x.device)
     for tap in itertools.product(range(k), repeat=nd):
@@ -65,7 +74,7 @@ def _conv_weight_grad(d_out: torch.Tensor, x: torch.Tensor, grid: tuple, k: int)
         out_sl = (slice(None),) + tuple(slice(a, b) for a, b in zip(lo, hi))
         in_sl = (slice(None),) + tuple(slice(a + u - pad, b + u - pad) for a, b, u in zip(lo, hi, tap))
         dW[(slice(None), slice(None)) + tap] = dg[out_sl].reshape(-1, O).t() @ xg[in_sl].reshape(-1, C)
-    return dW
+    return dW, d_b
 
 
 def _torch_conv_layout(w_flat: torch.Tensor, O: int, C: int, taps: tuple, dims) -> torch.Tensor:
@@ -117,8 +126,7 @@ def _finish_backward(ctx, x, dy, out_x, d_wqkv, d_proj, d_z, d_temp, x_mid, temp
         w_t = w_both.flip(dims=tuple(range(2, 2 + len(grid)))).transpose(0, 1)  # (C, 2HD, k, ...)
         w_t = (w_t.movedim(1, -1) if dims.conv_tap_major else w_t).contiguous()
         dx = PF.rows_gemm(d_proj, w_t, None, dims, 2 * HD, C) if ctx.needs_input_grad[0] else None
-        d_w_in = _conv_weight_grad(d_proj, x, grid, k)
-        d_b_in = _rows(d_proj).sum(0, dtype=torch.float32)
+        d_w_in, d_b_in = _conv_weight_grad(d_proj, x, dims)
 
     grads = (d_w_in[:HD], d_b_in[:HD], d_w_in[HD:], d_b_in[HD:], d_ws, d_bs, d_temp, d_wqkv, d_wo, d_bo)
     grads = tuple(gr.reshape(p.shape).to(p.dtype) if gr is not None and ctx.needs_input_grad[param_offset + i] else None
@@ -228,8 +236,7 @@ def _plus_backward_tail(ctx, x, uniform, x_mid, w, tok_out, out_x, dy, g, d_num,
         w_t = _torch_conv_layout(wx, HD, C, (k,) * len(grid), dims).flip(dims=tuple(range(2, 2 + len(grid)))).transpose(0, 1)
         w_t = (w_t.movedim(1, -1) if dims.conv_tap_major else w_t).contiguous()
         dx = PF.rows_gemm(d_xm, w_t, None, dims, HD, C) if ctx.needs_input_grad[0] else None
-        d_wx = _conv_weight_grad(d_xm, x, grid, k)
-        d_bx = _rows(d_xm).sum(0, dtype=torch.float32)
+        d_wx, d_bx = _conv_weight_grad(d_xm, x, dims)
 
     grads = (d_wx, d_bx, d_ws, d_bs, d_temp, d_w1, d_b1, d_w2, d_b2, d_wqkv, d_wo, d_bo)
     grads = tuple(gr.reshape(p.shape).to(p.dtype) if gr is not None and ctx.needs_input_grad[first_param + i] else None
@@ -563,7 +570,7 @@ class PointCrossFunction(torch.autograd.Function):
 class LinearFunction(torch.autograd.Function):
     """torch.nn.functional.linear for the block MLP in bf16 training: the two row GEMMs (forward, input gradient) go to
     the GEMM library, the weight and bias gradients -- products over the huge row axis, where the library's kernels
-    leave most of the machine idle -- to `cols_gemm_kernel`, which also returns them in float32."""
+    leave most of the machine idle -- to the library's row-axis kernels, which also return them in float32."""
 
     @staticmethod
     def forward(ctx, x, weight, bias):
@@ -579,24 +586,47 @@ class LinearFunction(torch.autograd.Function):
         dx = (dy @ w16) if ctx.needs_input_grad[0] else None
         dw = db = None
         if ctx.needs_input_grad[1] or ctx.needs_input_grad[2]:
-            dy2, x2 = _rows(dy), _rows(x).contiguous()
-            if PF.cols_gemm_supported(dy2, x2):
-                dw, db = PF.cols_gemm(dy2, x2, col_sums=True)
-            elif PF.cols_gemm_supported(x2, dy2):  # wide output, narrow input: form (x^T dy) and transpose
-                dw = PF.cols_gemm(x2, dy2).t()
-                db = dy2.sum(0, dtype=torch.float32)
-            else:
-                dw, db = dy2.t() @ x2, dy2.sum(0, dtype=torch.float32)
+            dw, db = _wgrad(_rows(dy), _rows(x))
             dw = dw.to(ctx.param_dtypes[0])
             db = db.to(ctx.param_dtypes[1]) if ctx.param_dtypes[1] is not None else None
         return dx, dw, db
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
-    """Differentiable linear layer; on bf16 GPU tensors the weight gradient runs on the library's kernel."""
-    if x.is_cuda and x.dtype == torch.bfloat16:
+    """Differentiable linear layer; on bf16 / float32 GPU tensors the weight gradient runs on the library's kernels."""
+    if x.is_cuda and x.dtype in (torch.bfloat16, torch.float32) and x.numel() > 0:
         return LinearFunction.apply(x.contiguous(), weight, bias)
     return torch.nn.functional.linear(x, weight, bias)
+
+
+def compute_dtype(x: torch.Tensor) -> torch.dtype | None:
+    """The type a Linear of x runs in on the library's training path: bfloat16 under bf16 autocast, x's own float32 or
+    bfloat16 without autocast, None where the modules run as they are."""
+    if not x.is_cuda:
+        return None
+    if torch.is_autocast_enabled("cuda"):
+        return torch.bfloat16 if torch.get_autocast_dtype("cuda") == torch.bfloat16 else None
+    return x.dtype if x.dtype in (torch.bfloat16, torch.float32) else None
+
+
+def mlp(x: torch.Tensor, layers: torch.nn.Sequential) -> torch.Tensor:
+    """Linear -> activation -> Linear in training, as autocast would run it, on `linear`."""
+    dtype = compute_dtype(x)
+    if dtype is None:
+        return layers(x)
+    with torch.autocast("cuda", enabled=False):
+        h = linear(x.to(dtype), layers[0].weight, layers[0].bias)
+        return linear(layers[1](h), layers[2].weight, layers[2].bias)
+
+
+def layer_norm_linear(x: torch.Tensor, ln: torch.nn.LayerNorm, lin: torch.nn.Linear) -> torch.Tensor:
+    """lin(ln(x)) in training (the output head), as autocast would run it: LayerNorm statistics in float32, its result
+    rounded to the Linear's type."""
+    dtype = compute_dtype(x)
+    if dtype is None or x.dtype != dtype:
+        return lin(ln(x))
+    with torch.autocast("cuda", enabled=False):
+        return linear(layer_norm(x, ln), lin.weight, lin.bias)
 
 
 class LayerNormFunction(torch.autograd.Function):

@@ -762,8 +762,35 @@ int pa_cols_gemm_f32(int64_t rows, const void *a, int64_t lda, int64_t cols_a, c
   if (!rows_ok(rows) || !cols_ok(lda) || !cols_ok(ldb)) return PA_ERR_UNSUPPORTED;
   if (!a || !b || !partials) return PA_ERR_NULL;
   if (!aligned16(a) || !aligned16(b) || !aligned16(partials)) return PA_ERR_ALIGN;
-  return pa::gemm::cols_gemm_f32(a, lda, cols_a, b, ldb, cols_b, rows, partials, col_sum_partials, compute_units(),
+  return pa::gemm::cols_gemm_f32(a, lda, cols_a, b, ldb, cols_b, rows, nullptr, partials, col_sum_partials, compute_units(),
                                  static_cast<hipStream_t>(stream));
+}
+
+static int weight_grad_taps(const pa_shape *grid, int64_t rows) {  // > 0, or an error
+  if (!grid || grid->conv_k == 0) return 1;
+  const int rc = check_shape(PA_F32, grid);
+  if (rc) return rc;
+  return grid->B * grid->N == rows ? pa::grid_taps(grid).taps : PA_ERR_DIMS;
+}
+
+int64_t pa_weight_grad_workspace_bytes(int dtype, int64_t rows, int64_t cols_a, int64_t cols_b, const pa_shape *grid) {
+  if (rows <= 0 || cols_a <= 0 || cols_b <= 0) return PA_ERR_DIMS;
+  if (!rows_ok(rows) || !cols_ok(cols_a) || !cols_ok(cols_b)) return PA_ERR_UNSUPPORTED;
+  const int taps = weight_grad_taps(grid, rows);
+  if (taps <= 0) return taps;
+  return pa::wgrad::workspace_bytes(dtype, rows, cols_a, cols_b, taps, compute_units());
+}
+
+int pa_weight_grad(int dtype, int64_t rows, const void *a, int64_t cols_a, const void *b, int64_t cols_b,
+                   const pa_shape *grid, void *workspace, int64_t workspace_bytes, float *out, float *col_sums,
+                   void *stream) {
+  const int64_t need = pa_weight_grad_workspace_bytes(dtype, rows, cols_a, cols_b, grid);
+  if (need < 0) return (int)need;
+  if (!a || !b || !workspace || !out) return PA_ERR_NULL;
+  if (workspace_bytes < need) return PA_ERR_SCRATCH;
+  if (!aligned16(a) || !aligned16(b) || !aligned16(workspace)) return PA_ERR_ALIGN;
+  return pa::wgrad::product(dtype, rows, a, cols_a, cols_a, b, cols_b, cols_b, grid && grid->conv_k > 0 ? grid : nullptr,
+                            workspace, out, col_sums, compute_units(), static_cast<hipStream_t>(stream));
 }
 
 int pa_mfma_backward_query(const pa_shape *shape) {

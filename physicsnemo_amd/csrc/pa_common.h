@@ -125,6 +125,32 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// Geometry of a grid convolution's neighbourhood: ks^2 taps (ks^3 with gd > 0) around every point of a gh x gw (x gd)
+// grid, N points per batch element; ks = 0: none.
+struct GridTaps {
+  int ks, taps, N, gh, gw, gd;
+};
+// row of the neighbour of row m at a tap, -1 outside the grid
+__device__ __forceinline__ int64_t grid_neighbour(const GridTaps &t, int64_t m, int tap) {
+  const int ksd = t.gd > 0 ? t.ks : 1, gd = t.gd > 0 ? t.gd : 1, pad = t.ks / 2;
+  const int uv = tap / ksd, z = tap - uv * ksd, u = uv / t.ks, v = uv - u * t.ks;
+  const int64_t b = m / t.N;
+  int n = (int)(m - b * t.N);
+  const int l = n % gd;
+  n /= gd;
+  const int i = n / t.gw, j = n - i * t.gw;
+  const int ii = i + u - pad, jj = j + v - pad, ll = l + (t.gd > 0 ? z - pad : 0);
+  if (ii < 0 || ii >= t.gh || jj < 0 || jj >= t.gw || ll < 0 || ll >= gd) return -1;
+  return b * t.N + ((int64_t)ii * t.gw + jj) * gd + ll;
+}
+inline GridTaps grid_taps(const pa_shape *s) {
+  GridTaps t{0, 1, 1, 1, 1, 0};
+  if (!s || s->conv_k <= 0) return t;
+  t.ks = (int)s->conv_k, t.N = (int)s->N, t.gh = (int)s->grid_h, t.gw = (int)s->grid_w, t.gd = (int)s->grid_d;
+  t.taps = t.ks * t.ks * (t.gd > 0 ? t.ks : 1);
+  return t;
+}
+
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 }  // namespace pa

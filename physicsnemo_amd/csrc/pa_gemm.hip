@@ -446,13 +446,14 @@ constexpr int kF32Tile = 128, kF32Rows = 32;
 
 __global__ __launch_bounds__(256) void cols_gemm_f32_kernel(const float *__restrict__ A, int lda, int OA,
                                                             const float *__restrict__ B, int ldb, int OB, int64_t M,
-                                                            int64_t rows_per_chunk, float *__restrict__ partials,
-                                                            float *__restrict__ col_sums) {
+                                                            int64_t rows_per_chunk, GridTaps grid,
+                                                            float *__restrict__ partials, float *__restrict__ col_sums) {
   __shared__ float As[2][kF32Rows][kF32Tile];
   __shared__ float Bs[2][kF32Rows][kF32Tile];
   const int t = threadIdx.x, lane = t & 63, i = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int oa0 = blockIdx.y * kF32Tile, ob0 = blockIdx.z * kF32Tile;
+  const int nob = (OB + kF32Tile - 1) / kF32Tile, tap = blockIdx.z / nob;
+  const int oa0 = blockIdx.y * kF32Tile, ob0 = (blockIdx.z - tap * nob) * kF32Tile;
   const int64_t m_begin = (int64_t)blockIdx.x * rows_per_chunk;
   const int64_t m_end = min(M, m_begin + rows_per_chunk);
   const int wa = (wave & 1) * 64, wb = (wave >> 1) * 64;  // this wave's sub-block of the tile
@@ -476,7 +477,8 @@ __global__ __launch_bounds__(256) void cols_gemm_f32_kernel(const float *__restr
       pa[k] = pb[k] = float4{0.f, 0.f, 0.f, 0.f};
       if (m < m_end) {
         if (oa0 + sc < OA) pa[k] = *reinterpret_cast<const float4 *>(A + m * lda + oa0 + sc);
-        if (ob0 + sc < OB) pb[k] = *reinterpret_cast<const float4 *>(B + m * ldb + ob0 + sc);
+        const int64_t mb = grid.ks > 0 ? grid_neighbour(grid, m, tap) : m;
+        if (ob0 + sc < OB && mb >= 0) pb[k] = *reinterpret_cast<const float4 *>(B + mb * ldb + ob0 + sc);
       }
     }
   };
@@ -507,7 +509,8 @@ __global__ __launch_bounds__(256) void cols_gemm_f32_kernel(const float *__restr
     buf ^= 1;
   }
   // C/D layout: lane (i, g) holds column ob = i, register r holds row oa = rowmap(r, g)
-  float *dst = partials + (int64_t)blockIdx.x * OA * OB;
+  const int64_t ld = (int64_t)grid.taps * OB;
+  float *dst = partials + (int64_t)blockIdx.x * OA * ld + (int64_t)tap * OB;
 #pragma unroll
   for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -516,7 +519,7 @@ __global__ __launch_bounds__(256) void cols_gemm_f32_kernel(const float *__restr
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int oa = oa0 + wa + 32 * u + mfma::rowmap(r, g);
-        if (oa < OA && ob < OB) dst[(int64_t)oa * OB + ob] = acc[u][v][r];
+        if (oa < OA && ob < OB) dst[(int64_t)oa * ld + ob] = acc[u][v][r];
       }
     }
   if (col_sums && blockIdx.z == 0 && (wave >> 1) == 0) {
@@ -529,147 +532,31 @@ __global__ __launch_bounds__(256) void cols_gemm_f32_kernel(const float *__restr
   }
 }
 
+// Two workgroups per compute unit in all, and no more chunks than pay for their partial results: 32 rows of a tile take
+// about 2 us, a partial of n values about 2 n ps to write and read back, their sum is smallest at sqrt(3e4 M / n).
 int64_t cols_gemm_f32_chunks(int64_t M, int64_t OA, int64_t OB, int num_cu) {
   const int64_t tiles = ((OA + kF32Tile - 1) / kF32Tile) * ((OB + kF32Tile - 1) / kF32Tile);
-  int64_t g = (3 * (int64_t)num_cu + tiles - 1) / tiles;  // about three workgroups per compute unit in all
-  const int64_t cap = (M + 1023) / 1024;                  // at least 1024 rows per chunk
+  int64_t g = 2 * (int64_t)num_cu / tiles, best = 1;
+  while ((best + 1) * (best + 1) <= 30000 * M / (OA * OB)) ++best;
+  if (g > best) g = best;
+  const int64_t cap = (M + 63) / 64;
   if (g > cap) g = cap;
   return g < 1 ? 1 : g;
 }
 
+// `shape` with conv_k > 0: B's rows are the neighbours at every tap, the partials [g][oa][tap][ob]
 int cols_gemm_f32(const void *A, int64_t lda, int64_t OA, const void *B, int64_t ldb, int64_t OB, int64_t M,
-                  float *partials, float *col_sums, int num_cu, hipStream_t st) {
+                  const pa_shape *shape, float *partials, float *col_sums, int num_cu, hipStream_t st) {
   if (OA <= 0 || OB <= 0 || OA % 4 != 0 || OB % 4 != 0 || lda % 4 != 0 || ldb % 4 != 0) return PA_ERR_UNSUPPORTED;
-  const int64_t G = cols_gemm_f32_chunks(M, OA, OB, num_cu);
+  const GridTaps grid_geom = grid_taps(shape);
+  const int64_t G = cols_gemm_f32_chunks(M, OA, OB * grid_geom.taps, num_cu);
   int64_t per = (M + G - 1) / G;
   per = (per + kF32Rows - 1) / kF32Rows * kF32Rows;
-  const dim3 grid((unsigned)G, (unsigned)((OA + kF32Tile - 1) / kF32Tile), (unsigned)((OB + kF32Tile - 1) / kF32Tile));
+  const dim3 grid((unsigned)G, (unsigned)((OA + kF32Tile - 1) / kF32Tile),
+                  (unsigned)((OB + kF32Tile - 1) / kF32Tile * grid_geom.taps));
   hipLaunchKernelGGL(cols_gemm_f32_kernel, grid, dim3(256), 0, st, static_cast<const float *>(A), (int)lda, (int)OA,
-                     static_cast<const float *>(B), (int)ldb, (int)OB, M, per, partials, col_sums);
+                     static_cast<const float *>(B), (int)ldb, (int)OB, M, per, grid_geom, partials, col_sums);
   return launch_status();
-}
-
-// ------------------------------------------------------------------------------------------------
-// cols_gemm_lds_kernel: the same product with the transposition done by the LDS read instead of on the matrix
-// cores.  A workgroup (8 waves, 4 along A's columns x 2 along B's) owns a 256 x 256 block of P for its chunk of rows;
-// 32 rows of both operands at a time are staged in LDS as they lie in memory (16-byte loads and writes; row stride 288
-// elements), and a lane receives its operand -- eight consecutive rows m of one column -- from two transposing reads
-// (ds_read_b64_tr_b16: within a group of 16 lanes, lane l receives element l % 4 of what lanes l / 4, 4 + l / 4,
-// 8 + l / 4, 12 + l / 4 address; lane L addresses row m0 + L / 4, columns c0 + 4 (L % 4) .. + 3, so lane l ends up with
-// column c0 + l of rows m0 .. m0 + 3).  With 144 words between rows the four rows a half-wave reads fall on four
-// different quarters of the banks.  Wave tile 64 x 128: 6 operand fragments (12 reads) feed 8 MFMAs.
-// grid (G row chunks, ceil(OA / 256)); OB <= 256.
-// ------------------------------------------------------------------------------------------------
-constexpr int kColsLd = 288;
-
-__global__ __launch_bounds__(512) void cols_gemm_lds_kernel(const uint16_t *__restrict__ A, int lda, int OA,
-                                                            const uint16_t *__restrict__ B, int ldb, int OB, int64_t M,
-                                                            int64_t per, float *__restrict__ partials,
-                                                            float *__restrict__ col_sums) {
-  typedef short v4i16 __attribute__((ext_vector_type(4)));
-  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-  typedef __attribute__((address_space(3))) v4i16 *lds_v4i16;
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  extern __shared__ u32x4 cols_smem[];
-  uint16_t *As = reinterpret_cast<uint16_t *>(cols_smem);  // [2][32 * kColsLd]
-  uint16_t *Bs = As + 2 * 32 * kColsLd;                     // [2][32 * kColsLd]
-  const int t = threadIdx.x, lane = t & 63, g = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int wa = (wave & 3) * 64, wb = (wave >> 2) * 128;
-  const int oa0 = blockIdx.y * 256;
-  const int64_t blk0 = (int64_t)blockIdx.x * per, nblk = (M + 31) / 32;
-  const int64_t blk1 = blk0 + per < nblk ? blk0 + per : nblk;
-
-  f32x16 acc[2][4];
-#pragma unroll
-  for (int u = 0; u < 2; ++u)
-#pragma unroll
-    for (int v = 0; v < 4; ++v)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[u][v][r] = 0.f;
-  float csum[2] = {0.f, 0.f};
-
-  // staging: 32 rows x 32 units of 8 columns per operand = 1024 units, two per thread
-  const int sr = t >> 5, su = (t & 31) * 8;  // row (and row + 16), first column of the unit
-  u32x4 pa[2], pb[2];
-  auto fetch = [&](int64_t blk) {
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const int64_t m = blk * 32 + sr + 16 * k;
-      pa[k] = pb[k] = u32x4{0, 0, 0, 0};
-      if (m < M) {
-        if (oa0 + su < OA) pa[k] = *reinterpret_cast<const u32x4 *>(A + m * lda + oa0 + su);
-        if (su < OB) pb[k] = *reinterpret_cast<const u32x4 *>(B + m * ldb + su);
-      }
-    }
-  };
-  auto stage = [&](int buf) {
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      *reinterpret_cast<u32x4 *>(&As[(buf * 32 + sr + 16 * k) * kColsLd + su]) = pa[k];
-      *reinterpret_cast<u32x4 *>(&Bs[(buf * 32 + sr + 16 * k) * kColsLd + su]) = pb[k];
-    }
-  };
-  // this lane's address inside a 32-row tile for the rows 8 g .. 8 g + 3 of k-step 0 and the 16 columns its group
-  // of lanes stands for (see above); k-step, upper four rows and column tile are constant offsets
-  const int l16 = lane & 15, q1 = (lane >> 4) & 1;
-  const int lane_off = (8 * g + (l16 >> 2)) * kColsLd + 16 * q1 + 4 * (l16 & 3);
-  auto operand = [&](const uint16_t *tile, int ks, int col) {  // rows 16 ks + 8 g .. + 7 of column col + (lane & 31)
-    const uint16_t *p = tile + lane_off + 16 * ks * kColsLd + col;
-    const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16)(uintptr_t)p));
-    const u32x2 hi =
-        __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16)(uintptr_t)(p + 4 * kColsLd)));
-    return u32x4{lo[0], lo[1], hi[0], hi[1]};
-  };
-  const bf16x2 ones = {(__bf16)1.f, (__bf16)1.f};
-  if (blk0 < blk1) fetch(blk0);
-  int buf = 0;
-  for (int64_t blk = blk0; blk < blk1; ++blk) {
-    stage(buf);
-    __syncthreads();
-    if (blk + 1 < blk1) fetch(blk + 1);
-    const uint16_t *at = As + buf * 32 * kColsLd, *bt = Bs + buf * 32 * kColsLd;
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      u32x4 af[2], bf[4];
-#pragma unroll
-      for (int u = 0; u < 2; ++u) af[u] = operand(at, ks, wa + 32 * u);
-#pragma unroll
-      for (int v = 0; v < 4; ++v) bf[v] = operand(bt, ks, wb + 32 * v);
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[u][v] = mfma::mma(af[u], bf[v], acc[u][v]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t word = af[u][j];
-          csum[u] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, word), ones, csum[u], false);
-        }
-      }
-    }
-    buf ^= 1;
-  }
-  const int i = lane & 31;
-  float *dst = partials + (int64_t)blockIdx.x * OA * OB;
-#pragma unroll
-  for (int u = 0; u < 2; ++u)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int ob = wb + 32 * v + i;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int oa = oa0 + wa + 32 * u + mfma::rowmap(r, g);
-        if (oa < OA && ob < OB) dst[(int64_t)oa * OB + ob] = acc[u][v][r];
-      }
-    }
-  if (col_sums && (wave >> 2) == 0) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const float total = csum[u] + __shfl_xor(csum[u], 32, 64);
-      const int oa = oa0 + wa + 32 * u + i;
-      if (g == 0 && oa < OA) col_sums[(int64_t)blockIdx.x * OA + oa] = total;
-    }
-  }
 }
 
 // the partial results stay small next to the rows a chunk reads
@@ -689,14 +576,8 @@ int cols_gemm(const void *A, int64_t lda, int64_t OA, const void *B, int64_t ldb
   const int64_t per = (nblk + G - 1) / G;
   const dim3 grid((unsigned)G, (unsigned)((OA + 255) / 256)), block((unsigned)((OA < 256 ? OA : 256) * 2));
   const uint16_t *a = static_cast<const uint16_t *>(A), *b = static_cast<const uint16_t *>(B);
-  if (OA >= 128 && OB >= 128 && OB <= 256) {  // wide products: the LDS-gather kernel (its 256 x 256 tile would idle on narrow ones)
-    const size_t lds = (size_t)4 * 32 * kColsLd * 2;
-    const int rc = allow_dynamic_lds(cols_gemm_lds_kernel, lds);
-    if (rc) return rc;
-    hipLaunchKernelGGL(cols_gemm_lds_kernel, dim3((unsigned)G, (unsigned)((OA + 255) / 256)), dim3(512), lds, st, a,
-                       (int)lda, (int)OA, b, (int)ldb, (int)OB, M, per, partials, col_sums);
-    return launch_status();
-  }
+  if (OA >= 128 && OB >= 128 && OB <= 256)  // wide products (the 256 x 256 tile would idle on narrow ones)
+    return wgrad::launch_wide(A, lda, OA, B, ldb, OB, M, G, nullptr, partials, col_sums, st);
 #define PA_COLS(NBV) \
   hipLaunchKernelGGL((cols_gemm_kernel<NBV>), grid, block, 0, st, a, (int)lda, (int)OA, b, (int)ldb, M, per, partials, col_sums)
   switch (OB / 32) {

@@ -76,8 +76,18 @@ int cols_gemm(const void *A, int64_t lda, int64_t OA, const void *B, int64_t ldb
 // the same for float32 operands (fp32 MFMA)
 int64_t cols_gemm_f32_chunks(int64_t M, int64_t OA, int64_t OB, int num_cu);
 int cols_gemm_f32(const void *A, int64_t lda, int64_t OA, const void *B, int64_t ldb, int64_t OB, int64_t M,
-                  float *partials, float *col_sums, int num_cu, hipStream_t st);
+                  const pa_shape *shape, float *partials, float *col_sums, int num_cu, hipStream_t st);
 }  // namespace gemm
+
+namespace wgrad {
+// out[oa][ob] (grid: [oa][ob][tap]) = sum_m A[m][oa] B[m][ob] and the column sums of A; `workspace`: workspace_bytes()
+int64_t workspace_bytes(int dtype, int64_t M, int64_t OA, int64_t OB, int taps, int num_cu);
+int product(int dtype, int64_t M, const void *A, int64_t lda, int64_t OA, const void *B, int64_t ldb, int64_t OB,
+            const pa_shape *grid, void *workspace, float *out, float *col_sums, int num_cu, hipStream_t st);
+// the bf16 tile kernel alone, G partial results
+int launch_wide(const void *A, int64_t lda, int64_t OA, const void *B, int64_t ldb, int64_t OB, int64_t M, int64_t G,
+                const pa_shape *grid, float *partials, float *col_sums, hipStream_t st);
+}  // namespace wgrad
 
 namespace general {
 int dequant_e4m3(const void *in, const float *scale, void *out, int64_t rows, int64_t cols, hipStream_t st);

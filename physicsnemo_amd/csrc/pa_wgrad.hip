@@ -1,0 +1,475 @@
+// Weight gradients: products over the row axis  P[oa][ob] = sum_m A[m][oa] B[m][ob]  with A = d out, B = the layer's
+// input (or, for a grid convolution, its neighbours: one product per tap), plus the column sums of A (the bias
+// gradient).  The row axis is cut into chunks, each leaves one partial result, and one small kernel adds the partials up
+// in index order, so results do not depend on the launch.
+//
+//   wgrad_kernel          bf16, up to 256 x 256 of P per workgroup, operands staged by direct global -> LDS loads
+//   narrow_wgrad_kernel   one side with at most 16 columns (input features, output channels), bf16 or fp32
+//   sum_partials_kernel   the fixed-order total, for both results of a call in one launch
+// The fp32 tile kernel (cols_gemm_f32_kernel) and the narrower bf16 one (cols_gemm_kernel) are in pa_gemm.hip.
+#include "pa_common.h"
+#include "pa_host.h"
+#include "pa_mfma_ops.h"
+
+namespace pa {
+namespace wgrad {
+
+using mfma::f32x16;
+using mfma::u32x2;
+using mfma::u32x4;
+
+__device__ const uint32_t kZeroUnit[4] = {0u, 0u, 0u, 0u};
+
+// ------------------------------------------------------------------------------------------------
+// wgrad_kernel: a workgroup (8 waves, 4 along A's columns x 2 along B's, wave tile 64 x 128) owns a 256 x 256 block of P
+// for its chunk of rows.  32 rows of both operands (32 KB) are one stage; four stages form a ring in LDS, filled by
+// global_load_lds three stages ahead (96 KB in flight per CU, which is what the memory latency asks for at this rate),
+// one barrier per stage.  A lane receives its operand -- eight consecutive rows of one column -- from two transposing
+// reads (ds_read_b64_tr_b16: within a group of 16 lanes, lane l receives element l % 4 of what lanes l / 4, 4 + l / 4,
+// 8 + l / 4, 12 + l / 4 address).  The direct loads write 1 KB contiguously, so the rows cannot be padded apart;
+// instead position p of row r holds the 16-byte unit p ^ 4 (r % 4), which puts the four rows a half-wave reads on four
+// different quarters of the banks.
+// Workgroups that share a chunk of rows (the blocks of columns, the taps) are placed on the same XCD next to each
+// other, so that the operand they share is read from memory once.
+// Bound by HBM, 2 (OA + OB) bytes per row, where P is one or two blocks: 512 x 256 over 1 048 576 rows 0.35 ms = 4.6 TB/s
+// (the copy of 1 GiB reaches 5.1); with register staging one stage ahead and twice the workgroups it took 0.44 ms.
+// A 3 x 3 convolution's 512 x 256 x 9 over 32 768 grid points: 109 us (im2col and the GEMM library: 590 us).
+// ------------------------------------------------------------------------------------------------
+constexpr int kStages = 4, kStageBytes = 32 * 1024;
+
+struct Args {
+  const uint16_t *A, *B;
+  int lda, ldb, OA, OB;
+  int64_t M;
+  int per;             // 32-row blocks per chunk
+  int chunks, ny, nz;  // row chunks; 256-column blocks of A; (tap, 256-column block of B)
+  float *partials;     // [chunk][OA][taps][OB]
+  float *col_sums;     // [chunk][OA] or NULL
+  GridTaps grid;       // grid convolution: B's row for point m and a tap is the neighbour there, zero outside the grid
+};
+
+__device__ __forceinline__ void load_unit_to_lds(const void *p, unsigned dst) {  // lane l's 16 bytes land at dst + 16 l
+  asm volatile(
+      "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %0, off" ::"v"(p), "s"(dst)
+      : "memory");
+}
+
+template <bool CONV>
+__global__ __launch_bounds__(512) void wgrad_kernel(Args a) {
+  typedef short v4i16 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) v4i16 *lds_v4i16;
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  extern __shared__ u32x4 ring[];  // [stage][A 32 rows x 512 bytes | B 32 rows x 512 bytes]
+  const int t = threadIdx.x, lane = t & 63, i = lane & 31, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int wa = (wave & 3) * 64, wb = (wave >> 2) * 128;
+  // the (chunk, tile) pairs in chunk-major order are dealt out to the XCDs (= workgroup id mod 8) in eight equal runs
+  const int tiles = a.ny * a.nz, item = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const int chunk = item / tiles, tile = item - chunk * tiles;
+  if (chunk >= a.chunks) return;
+  const int oa0 = (tile % a.ny) * 256, zt = tile / a.ny, nob = (a.OB + 255) / 256;
+  const int tap = CONV ? zt / nob : 0, ob0 = (CONV ? zt % nob : zt) * 256;
+  const int64_t nblk = (a.M + 31) / 32, blk0 = (int64_t)chunk * a.per;
+  const int64_t blk1 = blk0 + a.per < nblk ? blk0 + a.per : nblk;
+
+  f32x16 acc[2][4];
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[u][v][r] = 0.f;
+  float csum[2] = {0.f, 0.f};
+  const bool sums = a.col_sums != nullptr && zt == 0 && wb == 0;
+
+  // this wave stages rows 4 wave .. + 3 of both operands, two rows per load: lane l carries position l % 32 of row
+  // 4 wave + 2 k + l / 32, i.e. unit (l % 32) ^ 4 (row % 4); units past the operand's last column re-read its first one
+  int ua[2], ub[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int unit = i ^ (4 * (2 * k + g));
+    ua[k] = oa0 + unit * 8 < a.OA ? oa0 + unit * 8 : oa0;
+    ub[k] = ob0 + unit * 8 < a.OB ? ob0 + unit * 8 : ob0;
+  }
+  const unsigned lds0 = (unsigned)(uintptr_t)ring + wave * 2048;
+  // Convolution: the neighbour of row m at this tap is row m + shift where it lies inside the grid.  The grid coordinates
+  // of a lane's two rows are divided out once and then advanced by the 32 rows of a stage with carries.
+  int ci[2], cj[2], cl[2], du = 0, dv = 0, dz = 0, si = 0, sj = 0, sl = 0;
+  int64_t shift = 0;
+  const int gw = a.grid.gw, gh = a.grid.gh, gd = a.grid.gd > 0 ? a.grid.gd : 1;
+  if constexpr (CONV) {
+    const int ksd = a.grid.gd > 0 ? a.grid.ks : 1, uv = tap / ksd, pad = a.grid.ks / 2;
+    du = uv / a.grid.ks - pad, dv = uv % a.grid.ks - pad, dz = a.grid.gd > 0 ? tap % ksd - pad : 0;
+    shift = ((int64_t)du * gw + dv) * gd + dz;
+    si = 32 / (gw * gd), sj = 32 / gd % gw, sl = 32 % gd;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      int n = (int)((blk0 * 32 + wave * 4 + 2 * k + g) % a.grid.N);
+      cl[k] = n % gd;
+      n /= gd;
+      ci[k] = n / gw;
+      cj[k] = n - ci[k] * gw;
+    }
+  }
+  const uint16_t *pa[2], *pb[2];
+  auto fetch = [&](int64_t blk) {  // past the chunk's end: its last block again, so that every stage counts four loads
+    const unsigned dst = lds0 + (unsigned)((blk - blk0) & (kStages - 1)) * kStageBytes;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      if (blk < blk1) {
+        const int64_t m = blk * 32 + wave * 4 + 2 * k + g, mc = m < a.M ? m : a.M - 1;
+        pa[k] = a.A + mc * a.lda + ua[k];
+        pb[k] = a.B + mc * a.ldb + ub[k];
+        if constexpr (CONV) {
+          const int ii = ci[k] + du, jj = cj[k] + dv, ll = cl[k] + dz;
+          const bool in = m < a.M && (unsigned)ii < (unsigned)gh && (unsigned)jj < (unsigned)gw && (unsigned)ll < (unsigned)gd;
+          pb[k] = in ? pb[k] + shift * a.ldb : reinterpret_cast<const uint16_t *>(kZeroUnit);
+          cl[k] += sl;
+          cj[k] += sj;
+          ci[k] += si;
+          if (cl[k] >= gd) cl[k] -= gd, ++cj[k];
+          if (cj[k] >= gw) cj[k] -= gw, ++ci[k];
+          while (ci[k] >= gh) ci[k] -= gh;
+        }
+      }
+      load_unit_to_lds(pa[k], dst + k * 1024);
+      load_unit_to_lds(pb[k], dst + 16384 + k * 1024);
+    }
+  };
+  // reads: rows 16 ks + 8 g + l16 / 4 (+ 4); 16-byte units of 8 columns, see above
+  const int l16 = lane & 15, q1 = (lane >> 4) & 1, rr = l16 >> 2;
+  const int row_off = (8 * g + rr) * 512 + 32 * q1 + 8 * (l16 & 3);
+  auto operand = [&](const char *base, int ks, int col) {  // rows 16 ks + 8 g .. + 7 of column col + lane % 32
+    const char *p = base + row_off + 16 * ks * 512 + 64 * ((col >> 5) ^ rr);
+    const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16)(uintptr_t)p));
+    const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16)(uintptr_t)(p + 4 * 512)));
+    return u32x4{lo[0], lo[1], hi[0], hi[1]};
+  };
+  const bf16x2 ones = {(__bf16)1.f, (__bf16)1.f};
+
+  if (blk0 < blk1) {
+    fetch(blk0);
+    fetch(blk0 + 1);
+    fetch(blk0 + 2);
+  }
+  for (int64_t blk = blk0; blk < blk1; ++blk) {
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // this wave's share of the stage; the two younger stay in flight
+    __syncthreads();
+    fetch(blk + 3);  // into the stage multiplied one step ago, which every wave is past
+    const char *at = reinterpret_cast<const char *>(ring) + ((blk - blk0) & (kStages - 1)) * kStageBytes;
+    const char *bt = at + 16384;
+    const int valid = (int)(a.M - blk * 32 < 32 ? a.M - blk * 32 : 32);  // rows of this block
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      u32x4 af[2], bf[4];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) af[u] = operand(at, ks, wa + 32 * u);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) bf[v] = operand(bt, ks, wb + 32 * v);
+      if (valid < 32) {  // the last rows of all: those beyond M hold a repeated row and must not count
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int r = 16 * ks + 8 * g + 2 * j;
+            const uint32_t word = af[u][j];
+            af[u][j] = r + 1 < valid ? word : r < valid ? (word & 0xffffu) : 0u;
+          }
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[u][v] = mfma::mma(af[u], bf[v], acc[u][v]);
+        if (sums) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const uint32_t word = af[u][j];
+            csum[u] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, word), ones, csum[u], false);
+          }
+        }
+      }
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be landing in LDS when the workgroup ends
+  const int64_t ld = (int64_t)(CONV ? a.grid.taps : 1) * a.OB;
+  float *dst = a.partials + (int64_t)chunk * a.OA * ld + (int64_t)tap * a.OB;
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int ob = ob0 + wb + 32 * v + i;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int oa = oa0 + wa + 32 * u + mfma::rowmap(r, g);
+        if (oa < a.OA && ob < a.OB) dst[(int64_t)oa * ld + ob] = acc[u][v][r];
+      }
+    }
+  if (sums) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const float total = csum[u] + __shfl_xor(csum[u], 32, 64);
+      const int oa = oa0 + wa + 32 * u + i;
+      if (g == 0 && oa < a.OA) a.col_sums[(int64_t)chunk * a.OA + oa] = total;
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// narrow_wgrad_kernel: P[w][n] = sum_m W[m][w] V[m][n] with n < NN <= 16.  A thread keeps 4 columns of W against all
+// columns of V in registers, four rows in flight per workgroup; V's rows pass through LDS as fp32 (64 at a time) and are
+// read as broadcasts.  Also the column sums of W and of V.  Bound by reading W once.
+// ------------------------------------------------------------------------------------------------
+struct NarrowArgs {
+  const void *W, *V;
+  int ldw, ldv, OW, ON;
+  int64_t M, per;      // rows per chunk
+  float *partials;     // [chunk][OW][ON] (swap = 0) or [chunk][ON][OW] (swap = 1)
+  float *sums_w, *sums_v;  // [chunk][OW], [chunk][ON]; NULL: not wanted
+  int swap;
+};
+
+template <typename T, int NN>
+__global__ __launch_bounds__(256) void narrow_wgrad_kernel(NarrowArgs a) {
+  constexpr int ROWS = 64;
+  __shared__ float vs[ROWS][NN];
+  __shared__ float red[3][64][4 * NN + 5];
+  typedef typename std::conditional<sizeof(T) == 2, u32x2, u32x4>::type quad;
+  const T *W = static_cast<const T *>(a.W), *V = static_cast<const T *>(a.V);
+  const int t = threadIdx.x, cg = t & 63, rl = t >> 6, c0 = blockIdx.y * 256 + 4 * cg;
+  const bool live = c0 < a.OW;
+  const int64_t m0 = (int64_t)blockIdx.x * a.per, m1 = m0 + a.per < a.M ? m0 + a.per : a.M;
+  float acc[4][NN], sw[4] = {0.f, 0.f, 0.f, 0.f}, sv = 0.f;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+#pragma unroll
+    for (int n = 0; n < NN; ++n) acc[k][n] = 0.f;
+  for (int64_t mb = m0; mb < m1; mb += ROWS) {
+    __syncthreads();
+    for (int e = t; e < ROWS * NN; e += 256) {
+      const int r = e / NN, n = e - r * NN;
+      vs[r][n] = (mb + r < m1 && n < a.ON) ? load_as_f32(V + (mb + r) * a.ldv + n) : 0.f;
+    }
+    __syncthreads();
+    quad w[ROWS / 4];
+#pragma unroll
+    for (int k = 0; k < ROWS / 4; ++k) {
+      const int64_t m = mb + 4 * k + rl;
+      w[k] = quad{};
+      if (live && m < m1) w[k] = *reinterpret_cast<const quad *>(W + m * a.ldw + c0);
+    }
+#pragma unroll
+    for (int k = 0; k < ROWS / 4; ++k) {
+      float x[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if constexpr (sizeof(T) == 2) {
+          const uint32_t word = w[k][j >> 1];
+          x[j] = __uint_as_float((j & 1) ? (word & 0xffff0000u) : (word << 16));
+        } else {
+          const uint32_t word = w[k][j];
+          x[j] = __uint_as_float(word);
+        }
+        sw[j] += x[j];
+      }
+      const float *v = vs[4 * k + rl];
+#pragma unroll
+      for (int n = 0; n < NN; ++n)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j][n] = fmaf(x[j], v[n], acc[j][n]);
+    }
+    if (a.sums_v && blockIdx.y == 0 && t < NN)
+      for (int r = 0; r < ROWS; ++r) sv += vs[r][t];
+  }
+  if (rl > 0) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+      for (int n = 0; n < NN; ++n) red[rl - 1][cg][j * NN + n] = acc[j][n];
+      red[rl - 1][cg][4 * NN + j] = sw[j];
+    }
+  }
+  __syncthreads();
+  const int64_t chunk = blockIdx.x;
+  if (rl == 0 && live) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+      for (int n = 0; n < NN; ++n) {
+        const float v = ((acc[j][n] + red[0][cg][j * NN + n]) + red[1][cg][j * NN + n]) + red[2][cg][j * NN + n];
+        if (n < a.ON)
+          a.partials[chunk * a.OW * a.ON + (a.swap ? (int64_t)n * a.OW + c0 + j : (int64_t)(c0 + j) * a.ON + n)] = v;
+      }
+      if (a.sums_w)
+        a.sums_w[chunk * a.OW + c0 + j] =
+            ((sw[j] + red[0][cg][4 * NN + j]) + red[1][cg][4 * NN + j]) + red[2][cg][4 * NN + j];
+    }
+  }
+  if (a.sums_v && blockIdx.y == 0 && t < a.ON) a.sums_v[chunk * a.ON + t] = sv;
+}
+
+// ------------------------------------------------------------------------------------------------
+// sum_partials_kernel: dst[e] = sum_g src[g][e], two results in one launch.  A workgroup takes 32 consecutive elements
+// x 8 interleaved eighths of the partials and adds the eighths up through LDS, always in the same order.
+// taps > 1: the first result is [oa][tap][ob] and leaves as [oa][ob][tap], the order of a convolution's weight.
+// ------------------------------------------------------------------------------------------------
+struct SumArgs {
+  const float *src[2];
+  float *dst[2];
+  int64_t n[2];
+  int64_t blocks0;  // workgroups of the first result
+  int G, taps, OB;
+};
+
+__global__ __launch_bounds__(256) void sum_partials_kernel(SumArgs a) {
+  __shared__ float part[8][32];
+  const int z = (int64_t)blockIdx.x >= a.blocks0 ? 1 : 0;
+  const int64_t e = ((int64_t)blockIdx.x - (z ? a.blocks0 : 0)) * 32 + (threadIdx.x & 31), n = a.n[z];
+  const int part_id = threadIdx.x >> 5;
+  float s = 0.f;
+  if (e < n) {
+    const float *p = a.src[z] + e;
+#pragma unroll 8
+    for (int g = part_id; g < a.G; g += 8) s += p[(int64_t)g * n];
+  }
+  part[part_id][threadIdx.x & 31] = s;
+  __syncthreads();
+  if (part_id == 0 && e < n) {
+    float v = s;
+#pragma unroll
+    for (int k = 1; k < 8; ++k) v += part[k][threadIdx.x];
+    int64_t at = e;
+    if (z == 0 && a.taps > 1) {
+      const int64_t oa = e / (a.taps * (int64_t)a.OB), rest = e - oa * a.taps * a.OB, tap = rest / a.OB, ob = rest - tap * a.OB;
+      at = (oa * a.OB + ob) * a.taps + tap;
+    }
+    a.dst[z][at] = v;
+  }
+}
+
+// ================================================================================================
+// host side
+// ================================================================================================
+// Row chunks of a product of `tiles` workgroups per chunk: every workgroup resident at once (one 128 KB ring per CU), and
+// not so many that writing and re-reading the partial results costs more than the shorter chunks save: a chunk of r rows
+// takes about r 20 ns, a partial of n values about 2 n ps, and their sum is smallest at G = sqrt(1e4 M / n).
+int64_t chunks_for(int64_t M, int64_t tiles, int64_t n, int num_cu) {
+  const int64_t nblk = (M + 31) / 32;
+  int64_t g = num_cu / tiles;
+  int64_t best = 1;
+  while ((best + 1) * (best + 1) <= 10000 * M / n) ++best;
+  if (g > best) g = best;
+  if (g > nblk) g = nblk;
+  return g < 1 ? 1 : g;
+}
+
+static bool wide(int64_t OA, int64_t OB) { return OA % 32 == 0 && OB % 32 == 0 && OA >= 128 && OB >= 128; }
+
+enum class Form { none, wide_bf16, tiles_bf16, tiles_f32, narrow };
+
+static Form form_of(int dtype, int64_t OA, int64_t OB, int taps) {
+  if (OA <= 0 || OB <= 0) return Form::none;
+  if (dtype == PA_F32) {
+    if (OA % 4 == 0 && OB % 4 == 0 && OA >= 16 && OB >= 16) return Form::tiles_f32;
+  } else if (dtype == PA_BF16) {
+    if (wide(OA, OB)) return Form::wide_bf16;
+    if (taps == 1 && OA % 32 == 0 && (OA <= 256 || OA % 256 == 0) && (OB == 32 || OB == 64 || OB == 128 || OB == 256))
+      return Form::tiles_bf16;
+  }
+  if (taps == 1 && ((OB <= 16 && OA % 4 == 0 && OA >= 16) || (OA <= 16 && OB % 4 == 0 && OB >= 16))) return Form::narrow;
+  return Form::none;
+}
+
+static int64_t chunks_of(Form f, int64_t M, int64_t OA, int64_t OB, int taps, int num_cu) {
+  switch (f) {
+    case Form::wide_bf16: return chunks_for(M, ((OA + 255) / 256) * ((OB + 255) / 256) * taps, OA * OB * taps, num_cu);
+    case Form::tiles_bf16: return gemm::cols_gemm_chunks(M, OA, num_cu);
+    case Form::tiles_f32: return gemm::cols_gemm_f32_chunks(M, OA, OB * taps, num_cu);
+    case Form::narrow: {
+      const int64_t w = OA > OB ? OA : OB;
+      int64_t g = 4 * (int64_t)num_cu / ((w + 255) / 256);
+      const int64_t cap = (M + 127) / 128;
+      if (g > cap) g = cap;
+      return g < 1 ? 1 : g;
+    }
+    default: return 0;
+  }
+}
+
+int64_t workspace_bytes(int dtype, int64_t M, int64_t OA, int64_t OB, int taps, int num_cu) {
+  const Form f = form_of(dtype, OA, OB, taps);
+  if (f == Form::none) return PA_ERR_UNSUPPORTED;
+  return chunks_of(f, M, OA, OB, taps, num_cu) * (OA * OB * taps + OA) * 4;
+}
+
+template <typename T>
+static int launch_narrow(const NarrowArgs &a, int64_t G, hipStream_t st) {
+  const dim3 grid((unsigned)G, (unsigned)((a.OW + 255) / 256));
+  if (a.ON <= 4) hipLaunchKernelGGL((narrow_wgrad_kernel<T, 4>), grid, dim3(256), 0, st, a);
+  else if (a.ON <= 8) hipLaunchKernelGGL((narrow_wgrad_kernel<T, 8>), grid, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((narrow_wgrad_kernel<T, 16>), grid, dim3(256), 0, st, a);
+  return launch_status();
+}
+
+int launch_wide(const void *A, int64_t lda, int64_t OA, const void *B, int64_t ldb, int64_t OB, int64_t M, int64_t G,
+                const pa_shape *grid, float *partials, float *col_sums, hipStream_t st) {
+  Args a{};
+  a.A = static_cast<const uint16_t *>(A);
+  a.B = static_cast<const uint16_t *>(B);
+  a.lda = (int)lda, a.ldb = (int)ldb, a.OA = (int)OA, a.OB = (int)OB;
+  a.M = M;
+  a.per = (int)(((M + 31) / 32 + G - 1) / G);
+  a.grid = grid_taps(grid);
+  a.chunks = (int)G;
+  a.ny = (int)((OA + 255) / 256);
+  a.nz = (int)((OB + 255) / 256) * a.grid.taps;
+  a.partials = partials, a.col_sums = col_sums;
+  auto kernel = grid ? wgrad_kernel<true> : wgrad_kernel<false>;
+  const size_t lds = (size_t)kStages * kStageBytes;
+  if (int rc = allow_dynamic_lds(kernel, lds)) return rc;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((G * a.ny * a.nz + 7) / 8 * 8)), dim3(512), lds, st, a);
+  return launch_status();
+}
+
+int product(int dtype, int64_t M, const void *A, int64_t lda, int64_t OA, const void *B, int64_t ldb, int64_t OB,
+            const pa_shape *grid, void *workspace, float *out, float *col_sums, int num_cu, hipStream_t st) {
+  const int taps = grid_taps(grid).taps;
+  const Form f = form_of(dtype, OA, OB, taps);
+  if (f == Form::none) return PA_ERR_UNSUPPORTED;
+  const int64_t G = chunks_of(f, M, OA, OB, taps, num_cu), n = OA * OB * taps;
+  float *partials = static_cast<float *>(workspace), *sums = col_sums ? partials + G * n : nullptr;
+  int rc = PA_OK;
+  switch (f) {
+    case Form::wide_bf16: rc = launch_wide(A, lda, OA, B, ldb, OB, M, G, grid, partials, sums, st); break;
+    case Form::tiles_bf16: rc = gemm::cols_gemm(A, lda, OA, B, ldb, OB, M, partials, sums, num_cu, st); break;
+    case Form::tiles_f32: rc = gemm::cols_gemm_f32(A, lda, OA, B, ldb, OB, M, grid, partials, sums, num_cu, st); break;
+    default: {
+      NarrowArgs a{};
+      const bool a_wide = OB <= 16 && OA >= 16 && OA % 4 == 0;
+      a.W = a_wide ? A : B, a.V = a_wide ? B : A;
+      a.ldw = (int)(a_wide ? lda : ldb), a.ldv = (int)(a_wide ? ldb : lda);
+      a.OW = (int)(a_wide ? OA : OB), a.ON = (int)(a_wide ? OB : OA);
+      a.M = M, a.per = (M + G - 1) / G;
+      a.partials = partials;
+      (a_wide ? a.sums_w : a.sums_v) = sums;
+      a.swap = a_wide ? 0 : 1;
+      rc = dtype == PA_F32 ? launch_narrow<float>(a, G, st) : launch_narrow<bf16>(a, G, st);
+    }
+  }
+  if (rc) return rc;
+  SumArgs s{};
+  s.src[0] = partials, s.dst[0] = out, s.n[0] = n;
+  s.blocks0 = (n + 31) / 32;
+  int64_t blocks = s.blocks0;
+  if (col_sums) {
+    s.src[1] = sums, s.dst[1] = col_sums, s.n[1] = OA;
+    blocks += (OA + 31) / 32;
+  }
+  s.G = (int)G, s.taps = taps, s.OB = (int)OB;
+  hipLaunchKernelGGL(sum_partials_kernel, dim3((unsigned)blocks), dim3(256), 0, st, s);
+  return launch_status();
+}
+
+}  // namespace wgrad
+}  // namespace pa

@@ -614,40 +614,40 @@ def mfma_backward_supported(dtype: torch.dtype, dims: LayerDims) -> bool:
     return bool(rc)
 
 
-def cols_gemm_supported(a: torch.Tensor, b: torch.Tensor) -> bool:
-    ca, cb = a.shape[-1], b.shape[-1]
-    if a.dtype == torch.float32 and b.dtype == torch.float32:  # fp32 MFMA kernel: worth it from a few thousand rows on
-        return a.is_cuda and ca % 4 == 0 and cb % 4 == 0 and a.numel() // ca >= 4096
-    return (a.dtype == torch.bfloat16 and b.dtype == torch.bfloat16 and a.is_cuda and ca % 32 == 0
-            and (ca <= 256 or ca % 256 == 0) and cb in (32, 64, 128, 256))
+def cols_gemm_supported(a: torch.Tensor, b: torch.Tensor, grid: LayerDims | None = None) -> bool:
+    """True if `cols_gemm` serves d out = a (..., ca), input = b (..., cb) (see pa_weight_grad for the shapes)."""
+    if not (a.is_cuda and a.dtype == b.dtype and a.dtype in (torch.float32, torch.bfloat16)) or a.numel() == 0:
+        return False
+    if a.data_ptr() % 16 or b.data_ptr() % 16:
+        return False
+    ca = a.shape[-1]
+    return _lib.load().pa_weight_grad_workspace_bytes(_lib.dtype_code(a.dtype), a.numel() // ca, ca, b.shape[-1],
+                                                      byref(grid.c()) if grid is not None else None) > 0
 
 
-def cols_gemm(a: torch.Tensor, b: torch.Tensor, col_sums: bool = False):
+def cols_gemm(a: torch.Tensor, b: torch.Tensor, col_sums: bool = False, grid: LayerDims | None = None):
     """a^T . b over the leading (row) axes: bf16 or float32 (..., ca) and (..., cb) with equal row counts -> float32
-    (ca, cb).
-
-    The weight-gradient product d W = d out^T . in on the MFMA kernel `cols_gemm_kernel`; with `col_sums` the column
-    sums of a (the matching bias gradient) come back as well, from the same pass."""
+    (ca, cb): the weight-gradient product d W = d out^T . in.  With `grid` (the dims of a structured layer) b's rows are
+    gathered at every tap of its convolution and the result is (ca, cb, k, ..., k).  With `col_sums` the column sums of
+    a (the matching bias gradient) come back as well, from the same pass."""
     _need_cuda(a, b)
     lib = _lib.load()
     ca, cb = a.shape[-1], b.shape[-1]
     rows = a.numel() // ca
     if b.numel() // cb != rows:
         raise ValueError("cols_gemm needs the same number of rows on both sides")
-    a, b = a.contiguous(), b.contiguous()
-    if a.dtype == torch.float32:
-        chunks = lib.pa_cols_gemm_f32_chunks(rows, ca, cb)
-        partials = torch.empty(int(chunks), ca, cb, dtype=torch.float32, device=a.device)
-        sums = torch.empty(int(chunks), ca, dtype=torch.float32, device=a.device) if col_sums else None
-        _lib.check(lib.pa_cols_gemm_f32(rows, a.data_ptr(), ca, ca, b.data_ptr(), cb, cb, partials.data_ptr(),
-                                        _lib.ptr(sums), _lib.current_stream_ptr(a.device)), "pa_cols_gemm_f32")
-        return (partials.sum(0), sums.sum(0)) if col_sums else partials.sum(0)
-    chunks = lib.pa_cols_gemm_chunks(rows, ca)
-    partials = torch.empty(int(chunks), ca, cb, dtype=torch.float32, device=a.device)
-    sums = torch.empty(int(chunks), ca, dtype=torch.float32, device=a.device) if col_sums else None
-    _lib.check(lib.pa_cols_gemm(rows, a.data_ptr(), ca, ca, b.data_ptr(), cb, cb, partials.data_ptr(), _lib.ptr(sums),
-                                _lib.current_stream_ptr(a.device)), "pa_cols_gemm")
-    return (partials.sum(0), sums.sum(0)) if col_sums else partials.sum(0)
+    code = _lib.dtype_code(a.dtype)
+    geom = byref(grid.c()) if grid is not None else None
+    nbytes = lib.pa_weight_grad_workspace_bytes(code, rows, ca, cb, geom)
+    if nbytes < 0:
+        _lib.check(int(nbytes), "pa_weight_grad_workspace_bytes")
+    workspace = torch.empty(int(nbytes), dtype=torch.uint8, device=a.device)
+    taps = (grid.conv_k,) * (3 if grid.grid_d > 0 else 2) if grid is not None and grid.conv_k > 0 else ()
+    out = torch.empty(ca, cb, *taps, dtype=torch.float32, device=a.device)
+    sums = torch.empty(ca, dtype=torch.float32, device=a.device) if col_sums else None
+    _lib.check(lib.pa_weight_grad(code, rows, a.data_ptr(), ca, b.data_ptr(), cb, geom, workspace.data_ptr(), int(nbytes),
+                                  out.data_ptr(), _lib.ptr(sums), _lib.current_stream_ptr(a.device)), "pa_weight_grad")
+    return (out, sums) if col_sums else out
 
 
 def rows_gemm(inp, weight, bias, dims: LayerDims, c_in: int, c_out: int, gelu: bool = False):

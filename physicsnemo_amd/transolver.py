@@ -82,7 +82,7 @@ class Mlp(nn.Module):
                     PF.preprocess_supported(dtype, rows, lin1.in_features, lin1.out_features, lin2.out_features)):
                 w1, b1, w2, b2 = self._kernel_params(dtype, x.device)
                 return PF.preprocess_forward(x.to(dtype).contiguous(), w1, b1, w2, b2)
-        return self.layers(x)
+        return PA.mlp(x, self.layers) if needs_grad and len(self.layers) == 3 else self.layers(x)
 
 
 class PositionalEmbedding(nn.Module):
@@ -213,15 +213,8 @@ class TransolverBlock(nn.Module):
         return torch.is_grad_enabled() and (fx.requires_grad or any(p.requires_grad for p in self.parameters()))
 
     def _mlp_with_grad(self, normed: torch.Tensor) -> torch.Tensor:
-        """ln_mlp1[1] in training; under bf16 autocast its Linears use `autograd.linear` (weight gradients on the
-        library's row-axis kernel), otherwise the module as it is."""
-        mlp = self.ln_mlp1[1]
-        if normed.is_cuda and torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16:
-            lin1, act, lin2 = mlp.layers[0], mlp.layers[1], mlp.layers[2]
-            with torch.autocast("cuda", enabled=False):
-                h = PA.linear(normed.to(torch.bfloat16), lin1.weight, lin1.bias)
-                return PA.linear(act(h), lin2.weight, lin2.bias)
-        return mlp(normed)
+        """ln_mlp1[1] in training: its Linears use `autograd.linear` (weight gradients on the library's kernels)."""
+        return PA.mlp(normed, self.ln_mlp1[1].layers)
 
     def forward_chain(self, fx: torch.Tensor, normed_in: torch.Tensor | None, next_ln: nn.LayerNorm | None):
         """One block inside a chain of blocks: takes LayerNorm_1(fx) if the previous stage already produced it and
@@ -539,7 +532,7 @@ class Transolver(nn.Module):
                 if normed is not None and on_library:
                     fx = self._library_linear(normed, block.ln_mlp2[1])  # output head (:305-307)
                 else:
-                    fx = block.ln_mlp2[1](normed) if normed is not None else block.ln_mlp2(fx)
+                    fx = block.ln_mlp2[1](normed) if normed is not None else PA.layer_norm_linear(fx, *block.ln_mlp2)
             else:
                 fx, normed = block.forward_chain(fx, normed, self.blocks[k + 1].ln_1)
         if unflatten_output:

@@ -1,6 +1,7 @@
 """Backward pass of the HIP layer against autograd over the fp32 oracle (the oracle's own gradient is pinned by
 finite differences in test_oracle_closed_forms.py).  Bars: fp32 gradients rtol 1e-4 with atol = 1e-4 * max|ref|
 per tensor; bf16 gradients rel-L2 <= 3e-2 against the fp32 reference gradients."""
+import numpy as np
 import pytest
 import torch
 
@@ -261,6 +262,46 @@ def test_cols_gemm_float32(rows, ca, cb):
     assert got.shape == (ca, cb) and got.dtype == torch.float32
     assert_fp32_close(got, want.float(), "a^T b", rtol=1e-4)
     assert torch.equal(got, PF.cols_gemm(a, b))  # fixed summation order
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,ca,cb", [
+    (1, 256, 256), (33, 128, 128), (4097, 1024, 256), (2500, 256, 1024), (100001, 512, 288), (777, 160, 416),  # tile kernels
+    (5, 512, 5), (100003, 512, 7), (3001, 4, 256), (64, 1, 64), (9000, 260, 16), (129, 16, 300),               # one narrow side
+])
+def test_weight_gradient_shapes(dtype, rows, ca, cb):
+    """Row counts around the 32-row stages and the chunks, widths around the 256-column blocks, both narrow sides:
+    against float64, to the rounding of an fp32 sum of `rows` products (about sqrt(rows) 6e-8 of the rms entry)."""
+    announce("weight gradient", dtype, rows, ca, cb)
+    torch.manual_seed(rows + ca)
+    a = torch.randn(rows, ca, device="cuda").to(dtype)
+    b = (torch.randn(rows, cb, device="cuda") + 0.1).to(dtype)
+    if not PF.cols_gemm_supported(a, b):
+        pytest.skip("width pair left to the GEMM library")
+    got, sums = PF.cols_gemm(a, b, col_sums=True)
+    assert_fp32_close(got, (a.double().t() @ b.double()).float(), "a^T b", rtol=1e-4)
+    assert_fp32_close(sums, a.double().sum(0).float(), "column sums", rtol=1e-4)
+    assert torch.equal(got, PF.cols_gemm(a, b))
+
+
+@pytest.mark.parametrize("dtype,C,O", [(torch.bfloat16, 256, 512), (torch.bfloat16, 128, 128), (torch.float32, 128, 256),
+                                       (torch.float32, 36, 20)])
+@pytest.mark.parametrize("grid,k", [((13, 9), 3), ((40, 33), 5), ((4, 6, 5), 3), ((1, 50), 3)])
+def test_conv_weight_gradient(dtype, C, O, grid, k):
+    """The convolution form (neighbours gathered per tap, zero outside the grid) against torch's convolution backward."""
+    announce("conv weight gradient", dtype, C, O, grid, k)
+    torch.manual_seed(C + k)
+    B, N = 2, int(np.prod(grid))
+    g, x = torch.randn(B, N, O, device="cuda").to(dtype), torch.randn(B, N, C, device="cuda").to(dtype)
+    dims = PF.LayerDims(B, N, C, 4, 32, 32, grid[0], grid[1], k, grid[2] if len(grid) == 3 else 0, 1)
+    assert PF.cols_gemm_supported(g, x, dims)
+    dw, db = PF.cols_gemm(g, x, col_sums=True, grid=dims)
+    w = torch.zeros(O, C, *(k,) * len(grid), dtype=torch.float64, requires_grad=True)
+    conv = torch.nn.functional.conv2d if len(grid) == 2 else torch.nn.functional.conv3d
+    y = conv(x.double().cpu().transpose(1, 2).reshape(B, C, *grid), w, padding=k // 2)
+    y.backward(g.double().cpu().transpose(1, 2).reshape(B, O, *grid))
+    assert_fp32_close(dw, w.grad, "d weight")
+    assert_fp32_close(db, g.double().sum((0, 1)), "d bias")
 
 
 def test_bf16_model_training_step_runs_the_mfma_backward():
