@@ -455,15 +455,47 @@ int pa_mfma_slice_weighted_sum(const pa_shape *shape, const void *w_pack, const 
                                float *sums, void *stream);
 /* out_x (B, N, H*32) bf16 = deslice of the attended tokens (PA.py:492-495), the input of d W_out = dy^T out_x. */
 int pa_mfma_deslice(const pa_shape *shape, const void *w_pack, const void *tokp, void *out_x, void *stream);
-/* Per-point part of the backward pass, as pa_slice_softmax_backward but with the slice weights taken from w_pack.
- * tables: scratch of pa_mfma_backward_tables_bytes(shape) bytes; d_temperature_partials: float32,
- * pa_mfma_backward_groups(shape) * H elements (sum over the first index). */
+/* Scratch bytes and gradient floats of pa_point_backward for layers without the Transolver++ temperature. */
 int64_t pa_mfma_backward_tables_bytes(const pa_shape *shape);
 int64_t pa_mfma_backward_groups(const pa_shape *shape);
-int pa_mfma_slice_softmax_backward(const pa_shape *shape, const pa_params *p, const void *x_mid, const void *fx_mid,
-                                   const void *d_out_x, const void *w_pack, const float *out_slice_token,
-                                   const float *d_num, const float *d_norm, void *tables, void *d_proj, void *d_z,
-                                   float *d_temperature_partials, void *stream);
+
+/* ---- backward pieces for bf16 layers with 32-wide heads (D = 32, C = 32 H in {128, 256, 512}, S in {16, 32, 64, 128}) ----
+ * Per-point part: x_mid, fx_mid, d_out_x bf16 rows (B, N, H*32), the attended tokens (NULL: no deslice term), d num and
+ * d nrm -> d_proj (B, N, 2*H*32) = [d x_mid | d fx_mid] and grads (float32): d W_slice (S, 32), d b_slice (S),
+ * d temperature (H).  The slice weights are formed again from x_mid.  plus != NULL (Transolver++, PA.py:166-170,
+ * :530-532): fx_mid is x_mid, `uniform` (B, N, H, S) bf16 the samples behind the noise, d_proj (B, N, H*32) holds the sum
+ * of both gradients, and grads go on with proj_temperature's d W1 (S, 32), d b1 (S), d w2 (S), d b2 (1). */
+int64_t pa_point_backward_grads(const pa_shape *shape, int plus);
+int64_t pa_point_backward_workspace_bytes(const pa_shape *shape, int plus);
+int pa_point_backward(const pa_shape *shape, const pa_params *p, const pa_plus_params *plus, const void *x_mid,
+                      const void *fx_mid, const void *d_out_x, const void *uniform, const float *out_slice_token,
+                      const float *d_num, const float *d_norm, void *workspace, int64_t workspace_bytes, void *d_proj,
+                      float *grads, void *stream);
+/* From the output gradient dy (B, N, C) bf16 and the packed slice weights of the forward: d (attended tokens)
+ * (B, H, S, 32), d W_out (C, H*32) and d b_out (C), all float32.  out_linear_weight (C, H*32) bf16. */
+int64_t pa_output_backward_workspace_bytes(const pa_shape *shape);
+int pa_output_backward(const pa_shape *shape, const void *w_pack, const void *dy, const float *out_slice_token,
+                       const void *out_linear_weight, void *workspace, int64_t workspace_bytes, float *d_out_slice_token,
+                       float *d_out_linear_weight, float *d_out_linear_bias, void *stream);
+
+/* ---- training of such a layer in two calls --------------------------------------------------------
+ * Parameters: the three large weights in `weight_dtype` (PA_F32 or PA_BF16) in torch's layout (convolution weights
+ * (H*32, C, k, ..); shape->conv_tap_major must be 1, it names the kernels' order), everything else float32.  The forward
+ * leaves in `saved` (PA_TRAIN_SAVED bytes) what the backward reads; the parameters are not read again except the small
+ * float32 ones.  grads (PA_TRAIN_GRADS bytes, float32): d in_project_x.weight, d in_project_fx.weight (not with plus),
+ * their biases in the same order, d out_linear.weight, d out_linear.bias, d qkv_project.weight (96, 32), then grads of
+ * pa_point_backward.  dx (B, N, C) bf16 or NULL.  Replaces autograd over PA.py:501-558. */
+#define PA_TRAIN_SAVED 0    /* kept from the forward to the backward call */
+#define PA_TRAIN_FORWARD 1  /* workspace of the forward call */
+#define PA_TRAIN_BACKWARD 2 /* workspace of the backward call */
+#define PA_TRAIN_GRADS 3
+int64_t pa_layer_train_bytes(const pa_shape *shape, int plus, int which);
+int pa_layer_train_forward(const pa_shape *shape, int weight_dtype, const pa_params *p, const pa_plus_params *plus,
+                           const void *x, const void *uniform, void *y, void *saved, void *workspace,
+                           int64_t workspace_bytes, void *stream);
+int pa_layer_train_backward(const pa_shape *shape, const pa_params *p, const pa_plus_params *plus, const void *x,
+                            const void *uniform, const void *dy, const void *saved, void *dx, float *grads, void *workspace,
+                            int64_t workspace_bytes, void *stream);
 
 /* ---- block MLP ---------------------------------------------------------------------------------- */
 

@@ -30,7 +30,9 @@ EXPORTED = [
     "pa_layer_forward_plus_workspace_bytes", "pa_layer_forward_plus", "pa_flare_forward_mfma_supported",
     "pa_flare_forward_mfma_workspace_bytes", "pa_flare_forward_mfma",
     "pa_mfma_backward_query", "pa_rows_gemm_packed", "pa_mfma_slice_weighted_sum", "pa_mfma_deslice",
-    "pa_mfma_backward_tables_bytes", "pa_mfma_backward_groups", "pa_mfma_slice_softmax_backward",
+    "pa_mfma_backward_tables_bytes", "pa_mfma_backward_groups", "pa_point_backward_grads",
+    "pa_point_backward_workspace_bytes", "pa_point_backward", "pa_output_backward_workspace_bytes", "pa_output_backward",
+    "pa_layer_train_bytes", "pa_layer_train_forward", "pa_layer_train_backward",
     "pa_cols_gemm_chunks", "pa_cols_gemm", "pa_residual_layernorm",
     "pa_mfma_layer_forward", "pa_rows_gemm_act", "pa_layernorm_backward_groups", "pa_layernorm_backward",
     "pa_static_scratch_bytes", "pa_slice_reduce_static",
@@ -39,6 +41,7 @@ EXPORTED = [
     "pa_mfma_project_softmax_reduce_clocked", "pa_weight_grad_workspace_bytes", "pa_weight_grad",
 ]
 
+PA_TRAIN_SAVED, PA_TRAIN_FORWARD, PA_TRAIN_BACKWARD, PA_TRAIN_GRADS = range(4)
 PA_BUF_BLOB, PA_BUF_FX_PACK, PA_BUF_W_PACK, PA_BUF_PARTIALS, PA_BUF_TOKP = range(5)
 
 
@@ -249,8 +252,23 @@ def load() -> ctypes.CDLL:
     lib.pa_mfma_backward_tables_bytes.argtypes = [ps]
     lib.pa_mfma_backward_groups.restype = c_int64
     lib.pa_mfma_backward_groups.argtypes = [ps]
-    lib.pa_mfma_slice_softmax_backward.restype = c_int
-    lib.pa_mfma_slice_softmax_backward.argtypes = [ps, pp] + [c_void_p] * 12
+    pplus = POINTER(PaPlusParams)
+    lib.pa_point_backward_grads.restype = c_int64
+    lib.pa_point_backward_grads.argtypes = [ps, c_int]
+    lib.pa_point_backward_workspace_bytes.restype = c_int64
+    lib.pa_point_backward_workspace_bytes.argtypes = [ps, c_int]
+    lib.pa_point_backward.restype = c_int
+    lib.pa_point_backward.argtypes = [ps, pp, pplus] + [c_void_p] * 8 + [c_int64] + [c_void_p] * 3
+    lib.pa_output_backward_workspace_bytes.restype = c_int64
+    lib.pa_output_backward_workspace_bytes.argtypes = [ps]
+    lib.pa_output_backward.restype = c_int
+    lib.pa_output_backward.argtypes = [ps] + [c_void_p] * 5 + [c_int64] + [c_void_p] * 4
+    lib.pa_layer_train_bytes.restype = c_int64
+    lib.pa_layer_train_bytes.argtypes = [ps, c_int, c_int]
+    lib.pa_layer_train_forward.restype = c_int
+    lib.pa_layer_train_forward.argtypes = [ps, c_int, pp, pplus] + [c_void_p] * 5 + [c_int64, c_void_p]
+    lib.pa_layer_train_backward.restype = c_int
+    lib.pa_layer_train_backward.argtypes = [ps, pp, pplus] + [c_void_p] * 7 + [c_int64, c_void_p]
     lib.pa_cols_gemm_chunks.restype = c_int64
     lib.pa_cols_gemm_chunks.argtypes = [c_int64, c_int64]
     lib.pa_weight_grad_workspace_bytes.restype = c_int64

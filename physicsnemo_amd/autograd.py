@@ -98,18 +98,27 @@ def _slice_weight_grad(d_z: torch.Tensor, x_mid: torch.Tensor, H: int, S: int, D
     return _wgrad(d_z.reshape(-1, S), x_mid.reshape(-1, D))
 
 
-def _finish_backward(ctx, x, dy, out_x, d_wqkv, d_proj, d_z, d_temp, x_mid, temperature, param_offset=3):
+def _finish_backward(ctx, x, dy, out_x, d_wqkv, d_proj, d_z, d_temp, x_mid, temperature, param_offset=3, slice_grads=None,
+                     out_grads=None):
     """Everything after the layer-specific kernels: d x (input-gradient GEMM / transposed convolution) and the weight
     and bias gradients, which are plain GEMMs / column sums over the point axis.  Returns (d x, None, None, the ten
-    parameter gradients); `param_offset`: position of the first parameter among the Function's inputs."""
+    parameter gradients); `param_offset`: position of the first parameter among the Function's inputs.  `slice_grads`,
+    `out_grads`: (d weight, d bias) of in_project_slice (with d temperature masked) and of out_linear where the kernels
+    before this left them."""
     dims, kp = ctx.dims, ctx.kparams
     B, N, C, H, D, S = dims.B, dims.N, dims.C, dims.H, dims.D, dims.S
     HD = H * D
     linear = PF.LayerDims(B, N, C, H, D, S)
-    d_wo, d_bo = _wgrad(dy, out_x) if out_x is not None else (None, None)  # None: no out_linear (context projector)
-    d_ws, d_bs = _slice_weight_grad(d_z, x_mid, H, S, D)
-    t = temperature.reshape(-1)
-    d_temp = d_temp * ((t >= 0.5) & (t <= 5.0)).to(d_temp.dtype)
+    if out_grads is not None:
+        d_wo, d_bo = out_grads
+    else:
+        d_wo, d_bo = _wgrad(dy, out_x) if out_x is not None else (None, None)  # None: no out_linear (context projector)
+    if slice_grads is not None:
+        d_ws, d_bs = slice_grads
+    else:
+        d_ws, d_bs = _slice_weight_grad(d_z, x_mid, H, S, D)
+        t = temperature.reshape(-1)
+        d_temp = d_temp * ((t >= 0.5) & (t <= 5.0)).to(d_temp.dtype)
 
     k = dims.conv_k
     wx, wf = kp["in_project_x_weight"], kp["in_project_fx_weight"]
@@ -167,43 +176,58 @@ class PhysicsAttentionFunction(torch.autograd.Function):
         return _finish_backward(ctx, x, dy, out_x, d_wqkv, d_proj, d_z, d_temp, x_mid, temperature)
 
 
-class PhysicsAttentionMfmaFunction(torch.autograd.Function):
-    """The same gradient on the bf16 MFMA kernels (irregular variant, D = 32, C in {128, 256}, S <= 64).
+_LAYER_PARAMS = ("in_project_x_weight", "in_project_x_bias", "in_project_fx_weight", "in_project_fx_bias",
+                 "in_project_slice_weight", "in_project_slice_bias", "temperature", "qkv_project_weight",
+                 "out_linear_weight", "out_linear_bias")
+_PLUS_PARAMS = ("in_project_x_weight", "in_project_x_bias", "in_project_slice_weight", "in_project_slice_bias", "temperature",
+                "proj_temperature_0_weight", "proj_temperature_0_bias", "proj_temperature_2_weight",
+                "proj_temperature_2_bias", "qkv_project_weight", "out_linear_weight", "out_linear_bias")
+_LARGE = ("in_project_x_weight", "in_project_fx_weight", "out_linear_weight")
 
-    The forward is the inference path (fused projection / softmax / aggregation kernel, slice attention, deslice +
-    out_linear) with its packed slice weights kept; the backward recomputes x_mid / fx_mid with one MFMA GEMM and reads
-    the slice weights in their packed form."""
+
+def _layer_train_forward(ctx, x, uniform, dims, names, params):
+    """Forward of a bf16 layer with 32-wide heads in one library call; ctx keeps what the backward call reads."""
+    large = torch.bfloat16 if all(p.dtype == torch.bfloat16 for n, p in zip(names, params) if n in _LARGE) else torch.float32
+    kp = {n: p.detach().to(large if n in _LARGE else torch.float32).contiguous() for n, p in zip(names, params)}
+    y, saved = PF.layer_train_forward(x, uniform, kp, dims)
+    ctx.save_for_backward(x, uniform, saved, *params)
+    ctx.dims, ctx.names, ctx.kparams = dims, names, kp
+    return y
+
+
+def _layer_train_backward(ctx, dy, first_param):
+    x, uniform, saved, *params = ctx.saved_tensors
+    dx, grads = PF.layer_train_backward(x, uniform, dy.to(x.dtype).contiguous(), saved, ctx.kparams, ctx.dims,
+                                        ctx.needs_input_grad[0])
+    return dx, tuple(grads[n].view(p.shape).to(p.dtype) if need else None
+                     for n, p, need in zip(ctx.names, params, ctx.needs_input_grad[first_param:]))
+
+
+class PhysicsAttentionMfmaFunction(torch.autograd.Function):
+    """The same gradient on the bf16 MFMA kernels (32-wide heads: irregular and structured variants), one library call
+    forward and one backward; the parameters go to the library as they are (`kparams` is not read)."""
 
     @staticmethod
-    def forward(ctx, x, dims, kparams, wx, bx, wf, bf, ws, bs, temperature, wqkv, wo, bo):
-        st = PF.MfmaStages(kparams, dims, x.device)
-        st.pack_params()
-        if st.fused_groups > 0:
-            st.project_softmax_reduce(x)
-        else:
-            st.project_softmax(x)
-            st.slice_reduce()
-        st.combine_attention()
-        y = torch.empty_like(x)
-        st.deslice_project(y)
-        ctx.save_for_backward(x, temperature)
-        ctx.stages, ctx.dims, ctx.kparams = st, dims, kparams
-        ctx.param_like = (wx, bx, wf, bf, ws, bs, temperature, wqkv, wo, bo)
-        return y
+    def forward(ctx, x, dims, kparams, *params):
+        return _layer_train_forward(ctx, x, None, dims, _LAYER_PARAMS, params)
 
     @staticmethod
     def backward(ctx, dy):
-        x, temperature = ctx.saved_tensors
-        st, dims, kp = ctx.stages, ctx.dims, ctx.kparams
-        C, HD, D = dims.C, dims.H * dims.D, dims.D
-        dy = dy.to(x.dtype).contiguous()
-        g, g_pack = st.rows_gemm_packed(dy, kp["out_linear_weight"].view(C, HD).t().contiguous(), None)
-        x_mid, fx_mid = PF.project_inputs(x, kp, dims)
-        d_tok_out = st.slice_weighted_sum(g_pack)[..., :D].contiguous()
-        d_num, d_norm, d_wqkv = PF.slice_attention_backward(st.tok, st.norm, d_tok_out, kp, dims)
-        out_x = st.deslice()
-        d_proj, d_z, d_temp = st.slice_softmax_backward(x_mid, fx_mid, g, d_num, d_norm)
-        return _finish_backward(ctx, x, dy, out_x, d_wqkv, d_proj, d_z, d_temp, x_mid, temperature)
+        dx, grads = _layer_train_backward(ctx, dy, 3)
+        return (dx, None, None) + grads
+
+
+class PhysicsAttentionPlusMfmaFunction(torch.autograd.Function):
+    """`PhysicsAttentionPlusFunction` on the bf16 MFMA kernels (32-wide heads)."""
+
+    @staticmethod
+    def forward(ctx, x, uniform, dims, *params):
+        return _layer_train_forward(ctx, x, uniform, dims, _PLUS_PARAMS, params)
+
+    @staticmethod
+    def backward(ctx, dy):
+        dx, grads = _layer_train_backward(ctx, dy, 3)
+        return (dx, None, None) + grads
 
 
 def _plus_backward_tail(ctx, x, uniform, x_mid, w, tok_out, out_x, dy, g, d_num, d_norm, d_wqkv, first_param):
@@ -376,14 +400,13 @@ class GALEFunction(torch.autograd.Function):
         dy = dy.to(x.dtype).contiguous()
         linear = PF.LayerDims(dims.B, dims.N, C, dims.H, D, dims.S)
         w_out_t = kp["out_linear_weight"].view(C, HD).t().contiguous()
+        g = PF.rows_gemm(dy, w_out_t, None, linear, C, HD)
         if ctx.mfma:
             st = ctx.stages
-            g, g_pack = st.rows_gemm_packed(dy, w_out_t, None)
             x_mid, fx_mid = PF.project_inputs(x, kp, dims)
-            d_out_tok = st.slice_weighted_sum(g_pack)[..., :D].contiguous()
+            d_out_tok, d_wo, d_bo = PF.output_backward(st.w_pack, dy, ctx.out_tok, kp["out_linear_weight"], dims)
         else:
             x_mid, fx_mid, w, out_x = ctx.saved_tensors[2:]
-            g = PF.rows_gemm(dy, w_out_t, None, linear, C, HD)
             d_out_tok = PF.slice_weighted_sum(w, g, dims)[..., :D].contiguous()
         # slice-token stage: PyTorch's graph of the forward
         out_graph, tok_leaf, ctx_leaf, stage_params = ctx.graph
@@ -396,13 +419,13 @@ class GALEFunction(torch.autograd.Function):
         # tok = num / nrm
         d_num = (d_tok / ctx.norm[..., None]).contiguous()
         d_norm = (-(d_tok * ctx.tok).sum(-1) / ctx.norm).contiguous()
+        # qkv_project.weight takes part in the token stage only: its gradient comes with `d_stage`
         if ctx.mfma:
-            out_x = st.deslice()
-            d_proj, d_z, d_temp = st.slice_softmax_backward(x_mid, fx_mid, g, d_num, d_norm)
+            d_proj, d_ws, d_bs, d_temp = PF.point_backward(x_mid, fx_mid, g, ctx.out_tok, d_num, d_norm, kp, dims)
+            base = _finish_backward(ctx, x, dy, None, None, d_proj, None, d_temp, x_mid, temperature, 6, (d_ws, d_bs), (d_wo, d_bo))
         else:
             d_proj, d_z, d_temp = PF.slice_softmax_backward(x_mid, fx_mid, w, g, ctx.out_tok, d_num, d_norm, kp, dims)
-        # qkv_project.weight takes part in the token stage only: its gradient comes with `d_stage`
-        base = _finish_backward(ctx, x, dy, out_x, None, d_proj, d_z, d_temp, x_mid, temperature, param_offset=6)
+            base = _finish_backward(ctx, x, dy, out_x, None, d_proj, d_z, d_temp, x_mid, temperature, param_offset=6)
         return (base[0], d_context, None, None, None, None) + base[3:] + tuple(d_stage)
 
 
@@ -424,7 +447,6 @@ class SliceTokensFunction(torch.autograd.Function):
                 st.slice_reduce()
             st.combine_attention()
             tok, norm = st.tok.clone(), st.norm
-            ctx.stages = st
             ctx.save_for_backward(x, temperature, tok, norm)
         else:
             x_mid, fx_mid = PF.project_inputs(x, kparams, dims)
@@ -444,15 +466,14 @@ class SliceTokensFunction(torch.autograd.Function):
         d_norm = (-(d_tok * tok).sum(-1) / norm).contiguous()
         g = torch.zeros(dims.B, dims.N, dims.H * dims.D, dtype=x.dtype, device=x.device)
         if ctx.mfma:
-            st = ctx.stages
-            st.tok_out.zero_()
             x_mid, fx_mid = PF.project_inputs(x, kp, dims)
-            d_proj, d_z, d_temp = st.slice_softmax_backward(x_mid, fx_mid, g, d_num, d_norm)
+            d_proj, d_ws, d_bs, d_temp = PF.point_backward(x_mid, fx_mid, g, None, d_num, d_norm, kp, dims)
+            base = _finish_backward(ctx, x, None, None, None, d_proj, None, d_temp, x_mid, temperature, 3, (d_ws, d_bs))
         else:
             x_mid, fx_mid, w = ctx.saved_tensors[4:]
             d_proj, d_z, d_temp = PF.slice_softmax_backward(x_mid, fx_mid, w, g, torch.zeros_like(tok), d_num, d_norm,
                                                             kp, dims)
-        base = _finish_backward(ctx, x, None, None, None, d_proj, d_z, d_temp, x_mid, temperature)
+            base = _finish_backward(ctx, x, None, None, None, d_proj, d_z, d_temp, x_mid, temperature)
         return base[:3] + base[3:10]
 
 

@@ -799,19 +799,9 @@ int pa_mfma_backward_query(const pa_shape *shape) {
   return pa::mfma::backward_supported(*shape) && check_backward_shape(PA_BF16, shape) == PA_OK ? 1 : 0;
 }
 
-int64_t pa_mfma_backward_tables_bytes(const pa_shape *shape) {
-  int rc = check_shape(PA_BF16, shape);
-  if (rc) return rc;
-  if (!pa::mfma::backward_supported(*shape)) return PA_ERR_UNSUPPORTED;
-  return pa::mfma::backward_tables_bytes(*shape);
-}
+int64_t pa_mfma_backward_tables_bytes(const pa_shape *shape) { return pa_point_backward_workspace_bytes(shape, 0); }
 
-int64_t pa_mfma_backward_groups(const pa_shape *shape) {
-  int rc = check_shape(PA_BF16, shape);
-  if (rc) return rc;
-  if (!pa::mfma::backward_supported(*shape)) return PA_ERR_UNSUPPORTED;
-  return pa::mfma::backward_groups(*shape, compute_units()) * shape->B;
-}
+int64_t pa_mfma_backward_groups(const pa_shape *shape) { return pa_point_backward_grads(shape, 0); }
 
 int pa_rows_gemm_packed(const pa_shape *shape, int64_t c_in, const void *in, const void *weight, const float *bias,
                         void *out, void *out_pack, void *stream) {
@@ -849,23 +839,117 @@ int pa_mfma_deslice(const pa_shape *shape, const void *w_pack, const void *tokp,
   return pa::mfma::deslice_natural(*shape, w_pack, tokp, out_x, compute_units(), static_cast<hipStream_t>(stream));
 }
 
-int pa_mfma_slice_softmax_backward(const pa_shape *shape, const pa_params *p, const void *x_mid, const void *fx_mid,
-                                   const void *d_out_x, const void *w_pack, const float *out_slice_token,
-                                   const float *d_num, const float *d_norm, void *tables, void *d_proj, void *d_z,
-                                   float *d_temperature_partials, void *stream) {
+static int check_point_backward(const pa_shape *shape) {
   int rc = check_shape(PA_BF16, shape);
   if (rc) return rc;
-  if (!pa::mfma::backward_supported(*shape)) return PA_ERR_UNSUPPORTED;
+  return pa::mfma::point_backward_supported(*shape) ? PA_OK : PA_ERR_UNSUPPORTED;
+}
+
+int64_t pa_point_backward_grads(const pa_shape *shape, int plus) {
+  const int rc = check_point_backward(shape);
+  return rc ? rc : pa::mfma::point_backward_grads(*shape, plus != 0);
+}
+
+int64_t pa_point_backward_workspace_bytes(const pa_shape *shape, int plus) {
+  const int rc = check_point_backward(shape);
+  return rc ? rc : pa::mfma::point_backward_workspace_bytes(*shape, plus != 0, compute_units());
+}
+
+static bool plus_complete(const pa_plus_params *q) {
+  return q->proj_temperature_0_weight && q->proj_temperature_0_bias && q->proj_temperature_2_weight && q->proj_temperature_2_bias;
+}
+
+int pa_point_backward(const pa_shape *shape, const pa_params *p, const pa_plus_params *plus, const void *x_mid,
+                      const void *fx_mid, const void *d_out_x, const void *uniform, const float *out_slice_token,
+                      const float *d_num, const float *d_norm, void *workspace, int64_t workspace_bytes, void *d_proj,
+                      float *grads, void *stream) {
+  const int64_t need = pa_point_backward_workspace_bytes(shape, plus ? 1 : 0);
+  if (need < 0) return (int)need;
   if (!p || !p->in_project_slice_weight || !p->in_project_slice_bias || !p->temperature) return PA_ERR_NULL;
-  if (!x_mid || !fx_mid || !d_out_x || !w_pack || !out_slice_token || !d_num || !d_norm || !tables || !d_proj || !d_z ||
-      !d_temperature_partials)
-    return PA_ERR_NULL;
-  if (!aligned16(x_mid) || !aligned16(fx_mid) || !aligned16(d_out_x) || !aligned16(w_pack) || !aligned16(tables) ||
-      !aligned16(d_proj) || !aligned16(d_z))
+  if (!x_mid || (!plus && !fx_mid) || !d_out_x || !d_num || !d_norm || !workspace || !d_proj || !grads) return PA_ERR_NULL;
+  if (plus && (!uniform || !plus_complete(plus))) return PA_ERR_NULL;
+  if (workspace_bytes < need) return PA_ERR_WORKSPACE;
+  if (!aligned16(x_mid) || !aligned16(fx_mid) || !aligned16(d_out_x) || !aligned16(uniform) || !aligned16(workspace) ||
+      !aligned16(d_proj))
     return PA_ERR_ALIGN;
-  return pa::mfma::slice_softmax_backward(*shape, *p, x_mid, fx_mid, d_out_x, w_pack, out_slice_token, d_num, d_norm, tables,
-                                          d_proj, d_z, d_temperature_partials, compute_units(),
-                                          static_cast<hipStream_t>(stream));
+  return pa::mfma::point_backward(*shape, *p, plus, x_mid, fx_mid, d_out_x, uniform, out_slice_token, d_num, d_norm,
+                                  workspace, d_proj, grads, compute_units(), static_cast<hipStream_t>(stream));
+}
+
+int64_t pa_output_backward_workspace_bytes(const pa_shape *shape) {
+  const int rc = check_point_backward(shape);
+  return rc ? rc : pa::wgrad::output_backward_workspace_bytes(*shape, compute_units());
+}
+
+int pa_output_backward(const pa_shape *shape, const void *w_pack, const void *dy, const float *out_slice_token,
+                       const void *out_linear_weight, void *workspace, int64_t workspace_bytes, float *d_out_slice_token,
+                       float *d_out_linear_weight, float *d_out_linear_bias, void *stream) {
+  const int64_t need = pa_output_backward_workspace_bytes(shape);
+  if (need < 0) return (int)need;
+  if (!w_pack || !dy || !out_slice_token || !out_linear_weight || !workspace || !d_out_slice_token || !d_out_linear_weight ||
+      !d_out_linear_bias)
+    return PA_ERR_NULL;
+  if (workspace_bytes < need) return PA_ERR_WORKSPACE;
+  if (!aligned16(w_pack) || !aligned16(dy) || !aligned16(workspace)) return PA_ERR_ALIGN;
+  return pa::wgrad::output_backward(*shape, w_pack, dy, out_slice_token, out_linear_weight, workspace, d_out_slice_token,
+                                    d_out_linear_weight, d_out_linear_bias, compute_units(), static_cast<hipStream_t>(stream));
+}
+
+static int check_layer_train(const pa_shape *shape, int plus) {
+  int rc = check_shape(PA_BF16, shape);
+  if (rc) return rc;
+  return pa::train::supported(*shape, plus != 0) ? PA_OK : PA_ERR_UNSUPPORTED;
+}
+
+int64_t pa_layer_train_bytes(const pa_shape *shape, int plus, int which) {
+  const int rc = check_layer_train(shape, plus);
+  if (rc) return rc;
+  switch (which) {
+    case PA_TRAIN_SAVED: return pa::train::saved_bytes(*shape, plus != 0);
+    case PA_TRAIN_FORWARD: return pa::train::forward_workspace_bytes(*shape, plus != 0, compute_units());
+    case PA_TRAIN_BACKWARD: return pa::train::backward_workspace_bytes(*shape, plus != 0, compute_units());
+    case PA_TRAIN_GRADS: return pa::train::grad_floats(*shape, plus != 0) * 4;
+    default: return PA_ERR_UNSUPPORTED;
+  }
+}
+
+static int check_train_params(const pa_params *p, const pa_plus_params *plus) {
+  if (!p || !p->in_project_x_weight || !p->in_project_x_bias || !p->in_project_slice_weight || !p->in_project_slice_bias ||
+      !p->temperature || !p->qkv_project_weight || !p->out_linear_weight || !p->out_linear_bias)
+    return PA_ERR_NULL;
+  if (!plus) return p->in_project_fx_weight && p->in_project_fx_bias ? PA_OK : PA_ERR_NULL;
+  return plus_complete(plus) ? PA_OK : PA_ERR_NULL;
+}
+
+int pa_layer_train_forward(const pa_shape *shape, int weight_dtype, const pa_params *p, const pa_plus_params *plus,
+                           const void *x, const void *uniform, void *y, void *saved, void *workspace,
+                           int64_t workspace_bytes, void *stream) {
+  Range entry("pa_layer_train_forward");
+  int rc = check_layer_train(shape, plus ? 1 : 0);
+  if (rc) return rc;
+  if (weight_dtype != PA_F32 && weight_dtype != PA_BF16) return PA_ERR_UNSUPPORTED;
+  if ((rc = check_train_params(p, plus))) return rc;
+  if (!x || (plus && !uniform) || !y || !saved || !workspace) return PA_ERR_NULL;
+  if (!aligned16(x) || !aligned16(uniform) || !aligned16(y) || !aligned16(saved) || !aligned16(workspace)) return PA_ERR_ALIGN;
+  if (workspace_bytes < pa::train::forward_workspace_bytes(*shape, plus != nullptr, compute_units())) return PA_ERR_WORKSPACE;
+  return pa::train::forward(*shape, weight_dtype, *p, plus, x, uniform, y, saved, workspace, compute_units(),
+                            static_cast<hipStream_t>(stream));
+}
+
+int pa_layer_train_backward(const pa_shape *shape, const pa_params *p, const pa_plus_params *plus, const void *x,
+                            const void *uniform, const void *dy, const void *saved, void *dx, float *grads, void *workspace,
+                            int64_t workspace_bytes, void *stream) {
+  Range entry("pa_layer_train_backward");
+  int rc = check_layer_train(shape, plus ? 1 : 0);
+  if (rc) return rc;
+  if ((rc = check_train_params(p, plus))) return rc;
+  if (!x || (plus && !uniform) || !dy || !saved || !grads || !workspace) return PA_ERR_NULL;
+  if (!aligned16(x) || !aligned16(uniform) || !aligned16(dy) || !aligned16(saved) || !aligned16(dx) || !aligned16(grads) ||
+      !aligned16(workspace))
+    return PA_ERR_ALIGN;
+  if (workspace_bytes < pa::train::backward_workspace_bytes(*shape, plus != nullptr, compute_units())) return PA_ERR_WORKSPACE;
+  return pa::train::backward(*shape, *p, plus, x, uniform, dy, saved, dx, grads, workspace, compute_units(),
+                             static_cast<hipStream_t>(stream));
 }
 
 int64_t pa_mfma_buffer_bytes(const pa_shape *shape, int which) {
@@ -1526,7 +1610,7 @@ int pa_layer_forward_plus(int dtype, const pa_shape *shape, const pa_params *p, 
   a.pack_heads = (int)s.H;
   if (!pa::gemm::serves(a, 1, 2)) return PA_ERR_UNSUPPORTED;
   if ((rc = pa::gemm::launch(a, 1, PA_BF16, st))) return rc;
-  if ((rc = pa::mfma::slice_softmax_pack_plus(s, *p, *plus, x_mid, uniform, wp, compute_units(), st))) return rc;
+  if ((rc = pa::mfma::slice_softmax_pack_plus(s, *p, *plus, x_mid, uniform, wp, false, compute_units(), st))) return rc;
   if ((rc = pa::mfma::slice_reduce(s, wp, fxp, partials, st))) return rc;
   if ((rc = pa::mfma::combine_attention(s, *p, nullptr, partials, sp.G, tok, norm, tok_out, tokp, st))) return rc;
   if (pa::mfma::supported(dtype, s) && p->out_linear_bias) {

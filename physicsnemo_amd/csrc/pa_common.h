@@ -51,7 +51,18 @@ __device__ __forceinline__ float gelu_logistic(float x) {
   return x * __builtin_amdgcn_rcpf(1.f + e);
 }
 
-// its derivative: Phi(v) + v phi(v)
+// Phi(x) of the logistic form above, and the derivative of GELU from it: Phi(x) + x phi(x)
+__device__ __forceinline__ float gelu_logistic_phi(float x) {
+  const float x2 = fminf(x * x, 81.f);
+  float p = fmaf(-3.51902394e-04f * -2.f * kLog2e, x2, 3.70080200e-02f * -2.f * kLog2e);
+  p = fmaf(p, x2, 7.97505275e-01f * -2.f * kLog2e);
+  return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x * p));
+}
+__device__ __forceinline__ float gelu_grad_from_phi(float x, float phi) {
+  return fmaf(x * 0.3989422804014327f, __builtin_amdgcn_exp2f(x * x * (-0.5f * kLog2e)), phi);
+}
+
+// the derivative of gelu_erf: Phi(v) + v phi(v)
 __device__ __forceinline__ float gelu_erf_grad(float v) {
   return 0.5f * (1.f + erff(v * 0.70710678118654752f)) + v * 0.3989422804014327f * expf(-0.5f * v * v);
 }

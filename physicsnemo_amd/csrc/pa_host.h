@@ -87,7 +87,24 @@ int product(int dtype, int64_t M, const void *A, int64_t lda, int64_t OA, const 
 // the bf16 tile kernel alone, G partial results
 int launch_wide(const void *A, int64_t lda, int64_t OA, const void *B, int64_t ldb, int64_t OB, int64_t M, int64_t G,
                 const pa_shape *grid, float *partials, float *col_sums, hipStream_t st);
+int sum_rows(const float *src, int64_t rows, int64_t n, float *dst, hipStream_t st);
+int64_t output_backward_workspace_bytes(const pa_shape &s, int num_cu);
+int output_backward(const pa_shape &s, const void *w_pack, const void *dy, const float *out_token, const void *w_out,
+                    void *workspace, float *d_out_token, float *d_w_out, float *d_b_out, int num_cu, hipStream_t st);
 }  // namespace wgrad
+
+namespace train {
+// training of a bf16 layer (32-wide heads): see pa_layer_train_forward / _backward
+bool supported(const pa_shape &s, bool plus);
+int64_t saved_bytes(const pa_shape &s, bool plus);
+int64_t forward_workspace_bytes(const pa_shape &s, bool plus, int num_cu);
+int64_t backward_workspace_bytes(const pa_shape &s, bool plus, int num_cu);
+int64_t grad_floats(const pa_shape &s, bool plus);
+int forward(const pa_shape &s, int weight_dtype, const pa_params &p, const pa_plus_params *plus, const void *x,
+            const void *uniform, void *y, void *saved, void *workspace, int num_cu, hipStream_t st);
+int backward(const pa_shape &s, const pa_params &p, const pa_plus_params *plus, const void *x, const void *uniform,
+             const void *dy, const void *saved, void *dx, float *grads, void *workspace, int num_cu, hipStream_t st);
+}  // namespace train
 
 namespace general {
 int dequant_e4m3(const void *in, const float *scale, void *out, int64_t rows, int64_t cols, hipStream_t st);
@@ -208,7 +225,7 @@ int ball_query_cells(int64_t B, int64_t Np, int64_t Nq, int64_t K, float radius,
 namespace mfma {
 bool staged_supported(int dtype, const pa_shape &s);
 int slice_softmax_pack_plus(const pa_shape &s, const pa_params &p, const pa_plus_params &pp, const void *x_mid,
-                            const void *uniform, void *w_pack, int num_cu, hipStream_t st);
+                            const void *uniform, void *w_pack, bool split, int num_cu, hipStream_t st);
 int slice_softmax_pack(const pa_shape &s, const pa_params &p, const void *x_mid, void *w_pack, int num_cu,
                        hipStream_t st);
 // the same weights recomputed where they are used, never stored: token sums (softmax_reduce_groups partials) and
@@ -221,12 +238,14 @@ int deslice_recompute(const pa_shape &s, const pa_params &p, const void *x_mid, 
                       void *out_x, int num_cu, hipStream_t st);
 bool backward_supported(const pa_shape &s);
 int64_t backward_groups(const pa_shape &s, int num_cu);
-int64_t backward_tables_bytes(const pa_shape &s);
 int deslice_natural(const pa_shape &s, const void *w_pack, const void *tokp, void *out_x, int num_cu, hipStream_t st);
-int slice_softmax_backward(const pa_shape &s, const pa_params &p, const void *x_mid, const void *fx_mid,
-                           const void *d_out_x, const void *w_pack, const float *out_token, const float *d_num,
-                           const float *d_norm, void *tables, void *d_proj, void *d_z, float *dT_part, int num_cu,
-                           hipStream_t st);
+bool point_backward_supported(const pa_shape &s);
+int64_t point_backward_grads(const pa_shape &s, bool plus);
+int64_t point_backward_workspace_bytes(const pa_shape &s, bool plus, int num_cu);
+int point_backward(const pa_shape &s, const pa_params &p, const pa_plus_params *plus, const void *x_mid,
+                   const void *fx_mid, const void *d_out_x, const void *uniform, const float *out_token,
+                   const float *d_num, const float *d_norm, void *workspace, void *d_proj, float *grads, int num_cu,
+                   hipStream_t st);
 bool supported(int dtype, const pa_shape &s);
 int64_t tiles_per_batch(const pa_shape &s);
 int64_t reduce_groups(const pa_shape &s);

@@ -16,10 +16,24 @@ namespace mfma {
 // ------------------------------------------------------------------------------------------------
 // slice_softmax_pack_kernel: grid (G, B, head groups), one wave per head of the group; wave h walks the batch's
 // 32-point tiles g, g + G, ...
-//   logits^T (S x 32 pts) = W_slice (A, LDS, k = d in natural order) . x_mid^T (B = the points' rows, 16-byte loads)
+//   logits^T (S x 32 pts) = W_slice (A, LDS, k = d in natural order) . x_mid^T (B = the points' rows, 16-byte loads);
+//   W_slice as bf16(W) + bf16(W - bf16(W)): the training forward this serves keeps the float32 weight's 16 leading bits
 //   softmax over s in the base-2 domain: in-lane over the accumulator registers plus one exchange with lane ^ 32
 //   -> w_pack (the layout kernel (a) of the fused path writes); rows beyond N get zero weight.
 // ------------------------------------------------------------------------------------------------
+// eight consecutive float32 values (NULL: zeros) as bf16 and as the bf16 remainders of that rounding
+__device__ __forceinline__ void split_fragment(const float *src, u32x4 &hi, u32x4 &lo) {
+  bf16x8 h, l;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float v = src ? src[j] : 0.f;
+    h[j] = (__bf16)v;
+    l[j] = (__bf16)(v - (float)h[j]);
+  }
+  hi = __builtin_bit_cast(u32x4, h);
+  lo = __builtin_bit_cast(u32x4, l);
+}
+
 template <int S>
 __global__ __launch_bounds__(512) void slice_softmax_pack_kernel(const uint16_t *__restrict__ x_mid,
                                                                  const float *__restrict__ w_slice,
@@ -27,7 +41,7 @@ __global__ __launch_bounds__(512) void slice_softmax_pack_kernel(const uint16_t 
                                                                  const float *__restrict__ temperature,
                                                                  u32x4 *__restrict__ w_pack, int64_t N, int tpb, int H) {
   constexpr int ST = (S + 31) / 32, NCH = S / 16;
-  __shared__ u32x4 wsl[ST * 2 * 64];
+  __shared__ u32x4 wsl[2 * ST * 2 * 64];  // bf16(W), then the remainders
   __shared__ float bsl[ST * 32];
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -37,10 +51,7 @@ __global__ __launch_bounds__(512) void slice_softmax_pack_kernel(const uint16_t 
   for (int u = tid; u < ST * 2 * 64; u += blockDim.x) {
     const int ul = u & 63, ui = ul & 31, ug = ul >> 5, f = u >> 6, st = f >> 1, kk = f & 1;
     const int s = 32 * st + ui;
-    bf16x8 e;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) e[j] = (__bf16)(s < S ? w_slice[s * 32 + 16 * kk + 8 * ug + j] : 0.f);
-    wsl[u] = __builtin_bit_cast(u32x4, e);
+    split_fragment(s < S ? w_slice + s * 32 + 16 * kk + 8 * ug : nullptr, wsl[u], wsl[ST * 2 * 64 + u]);
   }
   for (int s = tid; s < ST * 32; s += blockDim.x) bsl[s] = s < S ? b_slice[s] : -1e30f;  // slices beyond S: weight 0
   __syncthreads();
@@ -56,8 +67,11 @@ __global__ __launch_bounds__(512) void slice_softmax_pack_kernel(const uint16_t 
     for (int st = 0; st < ST; ++st) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) lg[st][r] = bsl[32 * st + rowmap(r, g)];
-      lg[st] = mma(wsl[(st * 2 + 0) * 64 + lane], xm0, lg[st]);
-      lg[st] = mma(wsl[(st * 2 + 1) * 64 + lane], xm1, lg[st]);
+#pragma unroll
+      for (int lo = 0; lo < 2; ++lo) {
+        lg[st] = mma(wsl[((lo * ST + st) * 2 + 0) * 64 + lane], xm0, lg[st]);
+        lg[st] = mma(wsl[((lo * ST + st) * 2 + 1) * 64 + lane], xm1, lg[st]);
+      }
     }
     float mx = -INFINITY;
 #pragma unroll
@@ -92,7 +106,8 @@ __global__ __launch_bounds__(512) void slice_softmax_pack_kernel(const uint16_t 
 //   w        = softmax_s((logits[s] - log(-log(u[s] + 1e-8) + 1e-8)) / temp)             u: the caller's U[0,1) samples
 // `uniform` (B, N, H, S) bf16 in natural layout: a lane reads its slices (runs of four) with 8-byte loads.
 // ------------------------------------------------------------------------------------------------
-template <int S>
+// SPLIT: both weights with their bf16 remainders (training; inference multiplies with the rounded weights)
+template <int S, bool SPLIT>
 __global__ __launch_bounds__(512) void slice_softmax_pack_plus_kernel(
     const uint16_t *__restrict__ x_mid, const uint16_t *__restrict__ uniform, const float *__restrict__ w_slice,
     const float *__restrict__ b_slice, const float *__restrict__ temperature, const float *__restrict__ pt_w1,
@@ -100,8 +115,9 @@ __global__ __launch_bounds__(512) void slice_softmax_pack_plus_kernel(
     u32x4 *__restrict__ w_pack, int64_t N, int tpb, int H) {
   constexpr int ST = (S + 31) / 32, NCH = S / 16;
   constexpr float kLn2 = 0.6931471805599453f;
-  __shared__ u32x4 wsl[ST * 2 * 64];
-  __shared__ u32x4 w1l[ST * 2 * 64];
+  constexpr int NP = SPLIT ? 2 : 1;
+  __shared__ u32x4 wsl[NP * ST * 2 * 64];
+  __shared__ u32x4 w1l[NP * ST * 2 * 64];
   __shared__ float bsl[ST * 32], b1l[ST * 32], w2l[ST * 32];
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -111,14 +127,13 @@ __global__ __launch_bounds__(512) void slice_softmax_pack_plus_kernel(
   for (int u = tid; u < ST * 2 * 64; u += blockDim.x) {
     const int ul = u & 63, ui = ul & 31, ug = ul >> 5, f = u >> 6, st = f >> 1, kk = f & 1;
     const int s = 32 * st + ui;
-    bf16x8 e, e1;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      e[j] = (__bf16)(s < S ? w_slice[s * 32 + 16 * kk + 8 * ug + j] : 0.f);
-      e1[j] = (__bf16)(s < S ? pt_w1[s * 32 + 16 * kk + 8 * ug + j] : 0.f);
+    u32x4 lo, lo1;
+    split_fragment(s < S ? w_slice + s * 32 + 16 * kk + 8 * ug : nullptr, wsl[u], lo);
+    split_fragment(s < S ? pt_w1 + s * 32 + 16 * kk + 8 * ug : nullptr, w1l[u], lo1);
+    if constexpr (SPLIT) {
+      wsl[(NP - 1) * ST * 2 * 64 + u] = lo;
+      w1l[(NP - 1) * ST * 2 * 64 + u] = lo1;
     }
-    wsl[u] = __builtin_bit_cast(u32x4, e);
-    w1l[u] = __builtin_bit_cast(u32x4, e1);
   }
   for (int s = tid; s < ST * 32; s += blockDim.x) {
     bsl[s] = s < S ? b_slice[s] : -1e30f;  // slices beyond S: weight 0
@@ -141,8 +156,11 @@ __global__ __launch_bounds__(512) void slice_softmax_pack_plus_kernel(
       f32x16 hd;
 #pragma unroll
       for (int r = 0; r < 16; ++r) hd[r] = b1l[32 * st + rowmap(r, g)];
-      hd = mma(w1l[(st * 2 + 0) * 64 + lane], xm0, hd);
-      hd = mma(w1l[(st * 2 + 1) * 64 + lane], xm1, hd);
+#pragma unroll
+      for (int q = 0; q < NP; ++q) {
+        hd = mma(w1l[((q * ST + st) * 2 + 0) * 64 + lane], xm0, hd);
+        hd = mma(w1l[((q * ST + st) * 2 + 1) * 64 + lane], xm1, hd);
+      }
 #pragma unroll
       for (int r = 0; r < 16; ++r) a2 = fmaf(w2l[32 * st + rowmap(r, g)], gelu_logistic(hd[r]), a2);
     }
@@ -156,8 +174,11 @@ __global__ __launch_bounds__(512) void slice_softmax_pack_plus_kernel(
     for (int st = 0; st < ST; ++st) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) lg[st][r] = bsl[32 * st + rowmap(r, g)];
-      lg[st] = mma(wsl[(st * 2 + 0) * 64 + lane], xm0, lg[st]);
-      lg[st] = mma(wsl[(st * 2 + 1) * 64 + lane], xm1, lg[st]);
+#pragma unroll
+      for (int q = 0; q < NP; ++q) {
+        lg[st] = mma(wsl[((q * ST + st) * 2 + 0) * 64 + lane], xm0, lg[st]);
+        lg[st] = mma(wsl[((q * ST + st) * 2 + 1) * 64 + lane], xm1, lg[st]);
+      }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int s0 = 32 * st + 8 * q + 4 * g;  // slices rowmap(4 q .. 4 q + 3, g)
@@ -394,7 +415,7 @@ int slice_softmax_pack(const pa_shape &s, const pa_params &p, const void *x_mid,
 }
 
 int slice_softmax_pack_plus(const pa_shape &s, const pa_params &p, const pa_plus_params &pp, const void *x_mid,
-                            const void *uniform, void *w_pack, int num_cu, hipStream_t st) {
+                            const void *uniform, void *w_pack, bool split, int num_cu, hipStream_t st) {
   const int waves = (int)(s.H < 8 ? s.H : 8);
   if (s.H % waves != 0) return PA_ERR_UNSUPPORTED;
   const int groups = (int)(s.H / waves);
@@ -404,7 +425,8 @@ int slice_softmax_pack_plus(const pa_shape &s, const pa_params &p, const pa_plus
   if (gx < 1) gx = 1;
   const dim3 grid((unsigned)gx, (unsigned)s.B, (unsigned)groups), block((unsigned)(waves * 64));
 #define PA_LAUNCH_SSPP(SS)                                                                                          \
-  hipLaunchKernelGGL((slice_softmax_pack_plus_kernel<SS>), grid, block, 0, st, static_cast<const uint16_t *>(x_mid), \
+  hipLaunchKernelGGL((split ? slice_softmax_pack_plus_kernel<SS, true> : slice_softmax_pack_plus_kernel<SS, false>), grid, \
+                     block, 0, st, static_cast<const uint16_t *>(x_mid),                                             \
                      static_cast<const uint16_t *>(uniform), p.in_project_slice_weight, p.in_project_slice_bias,     \
                      p.temperature, pp.proj_temperature_0_weight, pp.proj_temperature_0_bias,                        \
                      pp.proj_temperature_2_weight, pp.proj_temperature_2_bias, static_cast<u32x4 *>(w_pack), s.N,    \

@@ -1,0 +1,265 @@
+// Training of a bf16 layer with 32-wide heads (irregular, structured and Transolver++ variants) as two sequences of the
+// library's kernels: the forward keeps what the backward needs in one buffer, the backward leaves every gradient.
+// Per-point intermediates that only link two products are formed again or folded away instead of stored:
+//   d tok' and d W_out come from sum_n w[n, h, s] dy[n, :] (pa_wgrad.hip), so neither out_x nor a reduction over d out_x
+//   is formed; d W_slice, d b_slice are summed inside the per-point kernel, so d z is never stored (pa_mfma_bwd.hip); the
+//   irregular layer's projections are computed again in the backward pass.
+#include "pa_common.h"
+#include "pa_host.h"
+#include "pa_mfma_ops.h"
+
+namespace pa {
+namespace train {
+
+// ------------------------------------------------------------------------------------------------
+// prepare_weights_kernel: the three large weights as the two passes read them, bf16, from float32 or bf16 parameters in
+// torch's layout, 32 x 32 tiles turned around through LDS (grid x: tiles, y: taps):
+//   w_in   [projection][o][tap][c]          w_in_t  [c][taps - 1 - tap][projection HD + o]   (the transposed convolution)
+//   w_out  [c][o]                           w_out_t [o][c]
+// ------------------------------------------------------------------------------------------------
+struct PrepareArgs {
+  const void *w[3];  // in_project_x, in_project_fx (or NULL), out_linear
+  uint16_t *w_in, *w_in_t, *w_out, *w_out_t;
+  int C, HD, taps, nproj;
+};
+
+template <typename T>
+__global__ __launch_bounds__(256) void prepare_weights_kernel(PrepareArgs a) {
+  __shared__ float tile[32][33];
+  const int t = threadIdx.x, col = t & 31, row0 = t >> 5;
+  const int tc = a.C / 32, th = a.HD / 32, per = th * tc;
+  int id = blockIdx.x;
+  const int which = id / per;  // 0 .. nproj - 1: an input projection, nproj: out_linear
+  id -= which * per;
+  const bool out = which == a.nproj;
+  const int tap = blockIdx.y;
+  if (out && tap > 0) return;
+  const int r0 = 32 * (out ? id / th : id / tc), c0 = 32 * (out ? id % th : id % tc);  // rows, columns of the tile
+  const T *src = static_cast<const T *>(a.w[out ? 2 : which]);
+  const int64_t ld = out ? a.HD : (int64_t)a.C * a.taps;
+  const int step = out ? 1 : a.taps;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int r = row0 + 8 * k;
+    tile[r][col] = load_as_f32(src + (r0 + r) * ld + (int64_t)(c0 + col) * step + (out ? 0 : tap));
+  }
+  __syncthreads();
+  const int O2 = a.nproj * a.HD;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int r = row0 + 8 * k;
+    const uint16_t straight = f32_to_bf16_bits(tile[r][col]), turned = f32_to_bf16_bits(tile[col][r]);
+    if (out) {
+      a.w_out[(int64_t)(r0 + r) * a.HD + c0 + col] = straight;
+      a.w_out_t[(int64_t)(c0 + r) * a.C + r0 + col] = turned;
+    } else {
+      a.w_in[((int64_t)(which * a.HD + r0 + r) * a.taps + tap) * a.C + c0 + col] = straight;
+      a.w_in_t[((int64_t)(c0 + r) * a.taps + (a.taps - 1 - tap)) * O2 + which * a.HD + r0 + col] = turned;
+    }
+  }
+}
+
+static int64_t round_up(int64_t v) { return (v + 255) / 256 * 256; }
+
+// ---- buffer plans ----
+struct Saved {  // kept from the forward to the backward pass
+  int64_t w_in, w_in_t, w_out, w_out_t, w_pack, tok, norm, tok_out, x_mid, fx_mid, total;
+};
+struct Scratch {
+  int64_t blob, fx_pack, partials, tokp, out_x, total;                                     // forward
+  int64_t g, x_mid, fx_mid, d_proj, d_tok, d_num, d_norm, attn, parts, work, total_backward;  // backward
+  int64_t work_bytes;
+};
+
+static bool fused(const pa_shape &s, bool plus) { return !plus && mfma::supported(PA_BF16, s); }
+
+bool supported(const pa_shape &s, bool plus) {
+  if (s.conv_k != 0 && s.conv_tap_major != 1) return false;
+  if (!mfma::point_backward_supported(s)) return false;
+  return backward::attention_lds_bytes(s) <= kMaxLdsBytes;
+}
+
+static Saved plan_saved(const pa_shape &s, bool plus) {
+  const int64_t HD = s.H * 32, taps = grid_taps(&s).taps, np = plus ? 1 : 2, tiles = s.B * mfma::tiles_per_batch(s);
+  Saved p{};
+  int64_t off = 0;
+  auto take = [&](int64_t bytes) {
+    const int64_t at = off;
+    off += round_up(bytes);
+    return at;
+  };
+  p.w_in = take(np * HD * taps * s.C * 2);
+  p.w_in_t = take(np * HD * taps * s.C * 2);
+  p.w_out = take(HD * s.C * 2);
+  p.w_out_t = take(HD * s.C * 2);
+  p.w_pack = take(tiles * s.H * (s.S / 16) * 1024);
+  p.tok = take(s.B * s.H * s.S * 32 * 4);
+  p.norm = take(s.B * s.H * s.S * 4);
+  p.tok_out = take(s.B * s.H * s.S * 32 * 4);
+  if (!fused(s, plus)) {
+    p.x_mid = take(s.B * s.N * HD * 2);
+    if (!plus) p.fx_mid = take(s.B * s.N * HD * 2);
+  }
+  p.total = off;
+  return p;
+}
+
+static int64_t forward_groups(const pa_shape &s, bool plus, int num_cu) {
+  return fused(s, plus) && mfma::fuse_reduce(s) ? mfma::project_groups(s, num_cu, true) : mfma::reduce_groups(s);
+}
+
+static Scratch plan_scratch(const pa_shape &s, bool plus, int num_cu) {
+  const int64_t HD = s.H * 32, M = s.B * s.N, tiles = s.B * mfma::tiles_per_batch(s), BHS = s.B * s.H * s.S;
+  Scratch p{};
+  int64_t off = 0;
+  auto take = [&](int64_t bytes) {
+    const int64_t at = off;
+    off += round_up(bytes);
+    return at;
+  };
+  p.blob = take(s.C <= 256 ? mfma::blob_bytes(s) : 0);
+  p.fx_pack = take(tiles * s.H * 2 * 1024);
+  p.partials = take((forward_groups(s, plus, num_cu) + 1) * BHS * 33 * 4);
+  p.tokp = take(mfma::tokp_bytes(s));
+  p.out_x = take(s.C <= 256 ? 0 : M * HD * 2);
+  p.total = off;
+
+  off = 0;
+  const int np = plus ? 1 : 2;
+  p.g = take(M * HD * 2);
+  if (fused(s, plus)) {
+    p.x_mid = take(M * HD * 2);
+    p.fx_mid = take(M * HD * 2);
+  }
+  p.d_proj = take(M * np * HD * 2);
+  p.d_tok = take(BHS * 32 * 4);
+  p.d_num = take(BHS * 32 * 4);
+  p.d_norm = take(BHS * 4);
+  p.attn = take(s.B * s.H * 2 * s.S * s.S * 4);
+  p.parts = take(s.B * s.H * 3 * 32 * 32 * 4);
+  p.work_bytes = wgrad::workspace_bytes(PA_BF16, M, np * HD, s.C, grid_taps(&s).taps, num_cu);
+  auto more = [&](int64_t bytes) { p.work_bytes = bytes > p.work_bytes ? bytes : p.work_bytes; };
+  more(wgrad::output_backward_workspace_bytes(s, num_cu));
+  more(mfma::point_backward_workspace_bytes(s, plus, num_cu));
+  p.work = take(p.work_bytes);
+  p.total_backward = off;
+  return p;
+}
+
+int64_t saved_bytes(const pa_shape &s, bool plus) { return plan_saved(s, plus).total; }
+int64_t forward_workspace_bytes(const pa_shape &s, bool plus, int num_cu) { return plan_scratch(s, plus, num_cu).total; }
+int64_t backward_workspace_bytes(const pa_shape &s, bool plus, int num_cu) {
+  return plan_scratch(s, plus, num_cu).total_backward;
+}
+
+// gradients in one float buffer: d in_project_x (then d in_project_fx) weights, their biases, d W_out, d b_out, d W_qkv,
+// then the per-point kernel's (d W_slice, d b_slice, d temperature, Transolver++: d W1, d b1, d w2, d b2)
+int64_t grad_floats(const pa_shape &s, bool plus) {
+  const int64_t HD = s.H * 32, np = plus ? 1 : 2;
+  return np * HD * s.C * grid_taps(&s).taps + np * HD + s.C * HD + s.C + 3 * 32 * 32 + mfma::point_backward_grads(s, plus);
+}
+
+// `p` for the kernels behind prepare_weights: the bf16 copies in the saved buffer
+static pa_params prepared(const pa_shape &s, const pa_params &p, bool plus, char *sv, const Saved &sp) {
+  pa_params q = p;
+  q.in_project_x_weight = sv + sp.w_in;
+  q.in_project_fx_weight = plus ? nullptr : sv + sp.w_in + s.H * 32 * s.C * grid_taps(&s).taps * 2;
+  q.out_linear_weight = sv + sp.w_out;
+  q.in_project_x_scale = q.in_project_fx_scale = q.out_linear_scale = nullptr;
+  return q;
+}
+
+int forward(const pa_shape &s, int weight_dtype, const pa_params &params, const pa_plus_params *plus, const void *x,
+            const void *uniform, void *y, void *saved, void *workspace, int num_cu, hipStream_t st) {
+  const bool pl = plus != nullptr;
+  const Saved sp = plan_saved(s, pl);
+  const Scratch sc = plan_scratch(s, pl, num_cu);
+  char *sv = static_cast<char *>(saved), *ws = static_cast<char *>(workspace);
+  const int taps = grid_taps(&s).taps;
+  PrepareArgs pa{};
+  pa.w[0] = params.in_project_x_weight, pa.w[1] = params.in_project_fx_weight, pa.w[2] = params.out_linear_weight;
+  pa.w_in = reinterpret_cast<uint16_t *>(sv + sp.w_in), pa.w_in_t = reinterpret_cast<uint16_t *>(sv + sp.w_in_t);
+  pa.w_out = reinterpret_cast<uint16_t *>(sv + sp.w_out), pa.w_out_t = reinterpret_cast<uint16_t *>(sv + sp.w_out_t);
+  pa.C = (int)s.C, pa.HD = (int)(s.H * 32), pa.taps = taps, pa.nproj = pl ? 1 : 2;
+  const dim3 grid((unsigned)((pa.nproj + 1) * (s.C / 32) * s.H), (unsigned)taps);
+  if (weight_dtype == PA_F32) hipLaunchKernelGGL(prepare_weights_kernel<float>, grid, dim3(256), 0, st, pa);
+  else hipLaunchKernelGGL(prepare_weights_kernel<bf16>, grid, dim3(256), 0, st, pa);
+  int rc = launch_status();
+  if (rc) return rc;
+  const pa_params p = prepared(s, params, pl, sv, sp);
+  void *blob = ws + sc.blob, *fx_pack = ws + sc.fx_pack, *tokp = ws + sc.tokp, *w_pack = sv + sp.w_pack;
+  float *partials = reinterpret_cast<float *>(ws + sc.partials), *tok = reinterpret_cast<float *>(sv + sp.tok),
+        *norm = reinterpret_cast<float *>(sv + sp.norm), *tok_out = reinterpret_cast<float *>(sv + sp.tok_out);
+  const int64_t G = forward_groups(s, pl, num_cu);
+  const float *fx_bias = nullptr;
+  if (fused(s, pl)) {
+    if ((rc = mfma::pack_params(s, p, blob, st))) return rc;
+    const bool one = mfma::fuse_reduce(s);
+    if ((rc = mfma::project_softmax(s, blob, x, fx_pack, w_pack, one ? partials : nullptr, num_cu, st))) return rc;
+    if (!one && (rc = mfma::slice_reduce(s, w_pack, fx_pack, partials, st))) return rc;
+    fx_bias = p.in_project_fx_bias;
+  } else {
+    void *x_mid = sv + sp.x_mid, *fx_mid = pl ? nullptr : sv + sp.fx_mid;
+    GemmArgs a{};
+    a.in = x;
+    a.w[0] = p.in_project_x_weight, a.w[1] = p.in_project_fx_weight;
+    a.bias[0] = p.in_project_x_bias, a.bias[1] = p.in_project_fx_bias;
+    a.out[0] = x_mid, a.out[1] = fx_mid;
+    a.out_pack[pl ? 0 : 1] = fx_pack;
+    a.M = s.B * s.N;
+    a.N = (int)s.N, a.C = (int)s.C, a.O = (int)(s.H * 32);
+    a.gh = (int)s.grid_h, a.gw = (int)s.grid_w, a.gd = (int)s.grid_d, a.ks = (int)s.conv_k;
+    a.w_tap_major = 1;
+    a.K = taps * (int)s.C;
+    a.pack_tpb = (int)mfma::tiles_per_batch(s), a.pack_heads = (int)s.H;
+    if (!gemm::serves(a, pl ? 1 : 2, 2)) return PA_ERR_UNSUPPORTED;
+    if ((rc = gemm::launch(a, pl ? 1 : 2, PA_BF16, st))) return rc;
+    rc = pl ? mfma::slice_softmax_pack_plus(s, p, *plus, x_mid, uniform, w_pack, true, num_cu, st)
+            : mfma::slice_softmax_pack(s, p, x_mid, w_pack, num_cu, st);
+    if (rc) return rc;
+    if ((rc = mfma::slice_reduce(s, w_pack, fx_pack, partials, st))) return rc;
+    if (s.C <= 256 && (rc = mfma::pack_out_linear(s, p.out_linear_weight, nullptr, p.out_linear_bias, blob, st))) return rc;
+  }
+  if ((rc = mfma::combine_attention(s, p, fx_bias, partials, G, tok, norm, tok_out, tokp, st))) return rc;
+  if (s.C <= 256) return mfma::deslice_project(s, blob, w_pack, tokp, y, nullptr, num_cu, st);
+  if ((rc = mfma::deslice_natural(s, w_pack, tokp, ws + sc.out_x, num_cu, st))) return rc;
+  return general::out_linear(PA_BF16, s, p, ws + sc.out_x, y, st);
+}
+
+int backward(const pa_shape &s, const pa_params &params, const pa_plus_params *plus, const void *x, const void *uniform,
+             const void *dy, const void *saved, void *dx, float *grads, void *workspace, int num_cu, hipStream_t st) {
+  const bool pl = plus != nullptr;
+  const Saved sp = plan_saved(s, pl);
+  const Scratch sc = plan_scratch(s, pl, num_cu);
+  char *sv = static_cast<char *>(const_cast<void *>(saved)), *ws = static_cast<char *>(workspace);
+  const pa_params p = prepared(s, params, pl, sv, sp);
+  const int64_t HD = s.H * 32, M = s.B * s.N, taps = grid_taps(&s).taps, np = pl ? 1 : 2;
+  float *d_w_in = grads, *d_b_in = d_w_in + np * HD * s.C * taps, *d_w_out = d_b_in + np * HD, *d_b_out = d_w_out + s.C * HD,
+        *d_wqkv = d_b_out + s.C, *small = d_wqkv + 3 * 32 * 32;
+  const float *tok = reinterpret_cast<float *>(sv + sp.tok), *norm = reinterpret_cast<float *>(sv + sp.norm),
+              *tok_out = reinterpret_cast<float *>(sv + sp.tok_out);
+  float *d_tok = reinterpret_cast<float *>(ws + sc.d_tok), *d_num = reinterpret_cast<float *>(ws + sc.d_num),
+        *d_norm = reinterpret_cast<float *>(ws + sc.d_norm), *parts = reinterpret_cast<float *>(ws + sc.parts);
+  void *g = ws + sc.g, *d_proj = ws + sc.d_proj, *work = ws + sc.work;
+  pa_shape lin = s;
+  lin.conv_k = lin.grid_h = lin.grid_w = lin.grid_d = 0;
+  int rc = wgrad::output_backward(s, sv + sp.w_pack, dy, tok_out, p.out_linear_weight, work, d_tok, d_w_out, d_b_out, num_cu, st);
+  if (rc) return rc;
+  if ((rc = backward::slice_attention(s, p, tok, norm, d_tok, reinterpret_cast<float *>(ws + sc.attn), d_num, d_norm, parts, st)))
+    return rc;
+  if ((rc = wgrad::sum_rows(parts, s.B * s.H, 3 * 32 * 32, d_wqkv, st))) return rc;
+  if ((rc = general::rows_gemm(PA_BF16, lin, s.C, HD, dy, sv + sp.w_out_t, nullptr, 0, g, st))) return rc;
+  const void *x_mid = sv + sp.x_mid, *fx_mid = pl ? nullptr : sv + sp.fx_mid;
+  if (fused(s, pl)) {
+    x_mid = ws + sc.x_mid, fx_mid = ws + sc.fx_mid;
+    if ((rc = general::project_inputs(PA_BF16, s, p, x, ws + sc.x_mid, ws + sc.fx_mid, st))) return rc;
+  }
+  if ((rc = mfma::point_backward(s, p, plus, x_mid, fx_mid, g, uniform, tok_out, d_num, d_norm, work, d_proj, small, num_cu, st)))
+    return rc;
+  if (dx && (rc = general::rows_gemm(PA_BF16, s, np * HD, s.C, d_proj, sv + sp.w_in_t, nullptr, 0, dx, st))) return rc;
+  return wgrad::product(PA_BF16, M, d_proj, np * HD, np * HD, x, s.C, s.C, s.conv_k > 0 ? &s : nullptr, work, d_w_in, d_b_in,
+                        num_cu, st);
+}
+
+}  // namespace train
+}  // namespace pa

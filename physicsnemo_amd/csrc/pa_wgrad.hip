@@ -42,10 +42,15 @@ struct Args {
   int lda, ldb, OA, OB;
   int64_t M;
   int per;             // 32-row blocks per chunk
-  int chunks, ny, nz;  // row chunks; 256-column blocks of A; (tap, 256-column block of B)
+  int chunks, batches; // row chunks (of each batch element, 1 unless A is packed)
+  int ny, nz;          // 256-column blocks of A; (tap, 256-column block of B)
   float *partials;     // [chunk][OA][taps][OB]
   float *col_sums;     // [chunk][OA] or NULL
   GridTaps grid;       // grid convolution: B's row for point m and a tap is the neighbour there, zero outside the grid
+  // packed A (the slice weights of the MFMA kernels): [batch][tile of 32 points][chunk of 16 columns][lane] 16 bytes, the
+  // chunk's lane (point p, half g) holding columns 4 g .. + 3 and 8 + 4 g .. + 3; chunks and M count per batch then
+  const u32x4 *pack;
+  int tpb, tile_units;  // tiles per batch, 16-byte units of a tile
 };
 
 __device__ __forceinline__ void load_unit_to_lds(const void *p, unsigned dst) {  // lane l's 16 bytes land at dst + 16 l
@@ -56,8 +61,13 @@ __device__ __forceinline__ void load_unit_to_lds(const void *p, unsigned dst) { 
       : "memory");
 }
 
-template <bool CONV>
+// MODE 0: A and B are rows.  1: B gathered per tap of a convolution.  2: A packed, batch by batch; the chunks of a stage
+// are copied as they lie, the 16-byte units permuted within a chunk so that the transposing reads of a half-wave (4
+// points x 4 groups of slices x 2 chunks) fall on all banks: unit (p, g) of chunk c at position 32 g + (p ^ 4 g ^ 8 (c & 1)).
+// Slice weights of points beyond N are zero, so B's rows there only need to be readable; col_sums are B's columns.
+template <int MODE>
 __global__ __launch_bounds__(512) void wgrad_kernel(Args a) {
+  constexpr bool CONV = MODE == 1, PACKED = MODE == 2;
   typedef short v4i16 __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) v4i16 *lds_v4i16;
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -68,10 +78,11 @@ __global__ __launch_bounds__(512) void wgrad_kernel(Args a) {
   // the (chunk, tile) pairs in chunk-major order are dealt out to the XCDs (= workgroup id mod 8) in eight equal runs
   const int tiles = a.ny * a.nz, item = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   const int chunk = item / tiles, tile = item - chunk * tiles;
-  if (chunk >= a.chunks) return;
+  if (chunk >= a.chunks * a.batches) return;
   const int oa0 = (tile % a.ny) * 256, zt = tile / a.ny, nob = (a.OB + 255) / 256;
   const int tap = CONV ? zt / nob : 0, ob0 = (CONV ? zt % nob : zt) * 256;
-  const int64_t nblk = (a.M + 31) / 32, blk0 = (int64_t)chunk * a.per;
+  const int batch = PACKED ? chunk / a.chunks : 0;
+  const int64_t nblk = (a.M + 31) / 32, blk0 = (int64_t)(chunk - batch * a.chunks) * a.per;
   const int64_t blk1 = blk0 + a.per < nblk ? blk0 + a.per : nblk;
 
   f32x16 acc[2][4];
@@ -81,8 +92,8 @@ __global__ __launch_bounds__(512) void wgrad_kernel(Args a) {
     for (int v = 0; v < 4; ++v)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[u][v][r] = 0.f;
-  float csum[2] = {0.f, 0.f};
-  const bool sums = a.col_sums != nullptr && zt == 0 && wb == 0;
+  float csum[4] = {0.f, 0.f, 0.f, 0.f};
+  const bool sums = a.col_sums != nullptr && (PACKED ? oa0 == 0 && wa == 0 : zt == 0 && wb == 0);
 
   // this wave stages rows 4 wave .. + 3 of both operands, two rows per load: lane l carries position l % 32 of row
   // 4 wave + 2 k + l / 32, i.e. unit (l % 32) ^ 4 (row % 4); units past the operand's last column re-read its first one
@@ -120,8 +131,14 @@ __global__ __launch_bounds__(512) void wgrad_kernel(Args a) {
     for (int k = 0; k < 2; ++k) {
       if (blk < blk1) {
         const int64_t m = blk * 32 + wave * 4 + 2 * k + g, mc = m < a.M ? m : a.M - 1;
-        pa[k] = a.A + mc * a.lda + ua[k];
-        pb[k] = a.B + mc * a.ldb + ub[k];
+        if constexpr (PACKED) {
+          const int c = 2 * wave + k, cs = oa0 + 16 * c < a.OA ? oa0 / 16 + c : oa0 / 16;
+          pa[k] = reinterpret_cast<const uint16_t *>(a.pack + ((int64_t)batch * a.tpb + blk) * a.tile_units + cs * 64 +
+                                                     32 * g + (i ^ (4 * g) ^ (8 * k)));
+        } else {
+          pa[k] = a.A + mc * a.lda + ua[k];
+        }
+        pb[k] = a.B + ((int64_t)batch * a.M + mc) * a.ldb + ub[k];
         if constexpr (CONV) {
           const int ii = ci[k] + du, jj = cj[k] + dv, ll = cl[k] + dz;
           const bool in = m < a.M && (unsigned)ii < (unsigned)gh && (unsigned)jj < (unsigned)gw && (unsigned)ll < (unsigned)gd;
@@ -147,7 +164,32 @@ __global__ __launch_bounds__(512) void wgrad_kernel(Args a) {
     const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16)(uintptr_t)(p + 4 * 512)));
     return u32x4{lo[0], lo[1], hi[0], hi[1]};
   };
+  // packed A: points 16 ks + 8 g + l16 / 4 (+ 4), group l16 % 4 of the chunk's four groups of four slices
+  const int gu = l16 & 1, pk_base = q1 * 1024 + 512 * gu + 8 * ((l16 >> 1) & 1) + 16 * ((8 * (g ^ q1)) + rr);
+  auto packed_operand = [&](const char *base, int ks, int col) {
+    const char *p = base + (col >> 4) * 1024 + 256 * ks + pk_base;
+    const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16)(uintptr_t)(p + 64 * gu)));
+    const u32x2 hi =
+        __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16)(uintptr_t)(p + 64 * (1 ^ gu))));
+    return u32x4{lo[0], lo[1], hi[0], hi[1]};
+  };
   const bf16x2 ones = {(__bf16)1.f, (__bf16)1.f};
+  auto masked = [&](u32x4 v, int ks, int valid) {  // rows >= valid of a 32-row block to zero
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int r = 16 * ks + 8 * g + 2 * j;
+      const uint32_t word = v[j];
+      v[j] = r + 1 < valid ? word : r < valid ? (word & 0xffffu) : 0u;
+    }
+    return v;
+  };
+  auto add_columns = [&](u32x4 v, float &s) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t word = v[j];
+      s = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, word), ones, s, false);
+    }
+  };
 
   if (blk0 < blk1) {
     fetch(blk0);
@@ -165,29 +207,24 @@ __global__ __launch_bounds__(512) void wgrad_kernel(Args a) {
     for (int ks = 0; ks < 2; ++ks) {
       u32x4 af[2], bf[4];
 #pragma unroll
-      for (int u = 0; u < 2; ++u) af[u] = operand(at, ks, wa + 32 * u);
+      for (int u = 0; u < 2; ++u) af[u] = PACKED ? packed_operand(at, ks, wa + 32 * u) : operand(at, ks, wa + 32 * u);
 #pragma unroll
       for (int v = 0; v < 4; ++v) bf[v] = operand(bt, ks, wb + 32 * v);
-      if (valid < 32) {  // the last rows of all: those beyond M hold a repeated row and must not count
+      if (!PACKED && valid < 32) {  // the last rows of all: those beyond M hold a repeated row and must not count
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int r = 16 * ks + 8 * g + 2 * j;
-            const uint32_t word = af[u][j];
-            af[u][j] = r + 1 < valid ? word : r < valid ? (word & 0xffffu) : 0u;
-          }
+        for (int u = 0; u < 2; ++u) af[u] = masked(af[u], ks, valid);
       }
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int v = 0; v < 4; ++v) acc[u][v] = mfma::mma(af[u], bf[v], acc[u][v]);
-        if (sums) {
+      if (sums) {
+        if constexpr (PACKED) {
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const uint32_t word = af[u][j];
-            csum[u] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, word), ones, csum[u], false);
-          }
+          for (int v = 0; v < 4; ++v) add_columns(valid < 32 ? masked(bf[v], ks, valid) : bf[v], csum[v]);
+        } else {
+#pragma unroll
+          for (int u = 0; u < 2; ++u) add_columns(af[u], csum[u]);
         }
       }
     }
@@ -208,10 +245,10 @@ __global__ __launch_bounds__(512) void wgrad_kernel(Args a) {
     }
   if (sums) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < (PACKED ? 4 : 2); ++u) {
       const float total = csum[u] + __shfl_xor(csum[u], 32, 64);
-      const int oa = oa0 + wa + 32 * u + i;
-      if (g == 0 && oa < a.OA) a.col_sums[(int64_t)chunk * a.OA + oa] = total;
+      const int col = (PACKED ? ob0 + wb : oa0 + wa) + 32 * u + i, ncol = PACKED ? a.OB : a.OA;
+      if (g == 0 && col < ncol) a.col_sums[(int64_t)chunk * ncol + col] = total;
     }
   }
 }
@@ -311,7 +348,8 @@ __global__ __launch_bounds__(256) void narrow_wgrad_kernel(NarrowArgs a) {
 
 // ------------------------------------------------------------------------------------------------
 // sum_partials_kernel: dst[e] = sum_g src[g][e], two results in one launch.  A workgroup takes 32 consecutive elements
-// x 8 interleaved eighths of the partials and adds the eighths up through LDS, always in the same order.
+// x 8 interleaved eighths of the partials and adds the eighths up through LDS, always in the same order.  blockIdx.y: a
+// batch of such sums of the first result ([batch][g][e] -> [batch][e]); the second one is formed by batch 0.
 // taps > 1: the first result is [oa][tap][ob] and leaves as [oa][ob][tap], the order of a convolution's weight.
 // ------------------------------------------------------------------------------------------------
 struct SumArgs {
@@ -319,19 +357,20 @@ struct SumArgs {
   float *dst[2];
   int64_t n[2];
   int64_t blocks0;  // workgroups of the first result
-  int G, taps, OB;
+  int G[2], taps, OB;
 };
 
 __global__ __launch_bounds__(256) void sum_partials_kernel(SumArgs a) {
   __shared__ float part[8][32];
   const int z = (int64_t)blockIdx.x >= a.blocks0 ? 1 : 0;
+  if (z && blockIdx.y > 0) return;
   const int64_t e = ((int64_t)blockIdx.x - (z ? a.blocks0 : 0)) * 32 + (threadIdx.x & 31), n = a.n[z];
-  const int part_id = threadIdx.x >> 5;
+  const int part_id = threadIdx.x >> 5, G = a.G[z];
   float s = 0.f;
   if (e < n) {
-    const float *p = a.src[z] + e;
+    const float *p = a.src[z] + (int64_t)blockIdx.y * G * n + e;
 #pragma unroll 8
-    for (int g = part_id; g < a.G; g += 8) s += p[(int64_t)g * n];
+    for (int g = part_id; g < G; g += 8) s += p[(int64_t)g * n];
   }
   part[part_id][threadIdx.x & 31] = s;
   __syncthreads();
@@ -339,12 +378,70 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(SumArgs a) {
     float v = s;
 #pragma unroll
     for (int k = 1; k < 8; ++k) v += part[k][threadIdx.x];
-    int64_t at = e;
+    int64_t at = (int64_t)blockIdx.y * n + e;
     if (z == 0 && a.taps > 1) {
       const int64_t oa = e / (a.taps * (int64_t)a.OB), rest = e - oa * a.taps * a.OB, tap = rest / a.OB, ob = rest - tap * a.OB;
       at = (oa * a.OB + ob) * a.taps + tap;
     }
     a.dst[z][at] = v;
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// token_grad_kernel: what the layer's output gradient says about the slice tokens and out_linear, from the sums
+// P[b][h S + s][c] = sum_n w[n, h, s] dy[n, c] (the packed product above) instead of from per-point d out_x and out_x:
+//   d tok'[b, h, s, d] = sum_c P[b, h, s, c] W_out[c, 32 h + d]              workgroups 0 .. B H ceil(S / 32) - 1
+//   d W_out[c, 32 h + d] = sum_b sum_s P[b, h, s, c] tok'[b, h, s, d]        the others, one per (h, 32 rows c)
+// Four waves per 32 x 32 result tile on fp32 MFMA, each a quarter of the reduction, added up in order through LDS.  Bound
+// by latency (P is a few hundred KB): the quarters' loads are all in flight at once, which takes 60 us (one wave per
+// tile) to 15 us at B = 1, S = 64, C = 256.
+// ------------------------------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void token_grad_kernel(const float *__restrict__ P, const uint16_t *__restrict__ w_out,
+                                                         const float *__restrict__ out_token, float *__restrict__ d_token,
+                                                         float *__restrict__ d_w_out, int B, int H, int S, int C) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  __shared__ float part[3][16][64];
+  const int lane = threadIdx.x & 63, i = lane & 31, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ST = (S + 31) / 32, HD = H * 32, first = B * H * ST;
+  f32x16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  const bool to_token = (int)blockIdx.x < first;
+  const int e = blockIdx.x - first, st = blockIdx.x % ST, bh = blockIdx.x / ST, h = to_token ? bh % H : e % H, c0 = e / H * 32;
+  if (to_token) {
+    const int s = 32 * st + i, cw = C / 4;
+    const float *row = P + ((int64_t)bh * S + (s < S ? s : S - 1)) * C + wave * cw + 4 * g;
+    const uint16_t *wcol = w_out + (int64_t)(wave * cw + 4 * g) * HD + 32 * h + i;
+#pragma unroll 8
+    for (int c = 0; c < cw; c += 8) {  // lane half g supplies c + 4 g .. + 3, one pair (c + m, c + 4 + m) per MFMA
+      const f32x4 p4 = *reinterpret_cast<const f32x4 *>(row + c);
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(p4[m], bf16_bits_to_f32(wcol[(int64_t)(c + m) * HD]), acc, 0, 0, 0);
+    }
+  } else {
+    const int sw = S / 4;
+    for (int b = 0; b < B; ++b) {
+      const int64_t at = ((int64_t)b * H + h) * S + wave * sw + g;
+      const float *p = P + at * C + c0 + i, *tk = out_token + at * 32 + i;
+#pragma unroll 8
+      for (int s = 0; s < sw; s += 2)
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(p[(int64_t)s * C], tk[s * 32], acc, 0, 0, 0);
+    }
+  }
+  if (wave > 0) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) part[wave - 1][r][lane] = acc[r];
+  }
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const float v = ((acc[r] + part[0][r][lane]) + part[1][r][lane]) + part[2][r][lane];
+    const int row = mfma::rowmap(r, g);
+    if (!to_token) d_w_out[(int64_t)(c0 + row) * HD + 32 * h + i] = v;
+    else if (32 * st + row < S) d_token[((int64_t)bh * S + 32 * st + row) * 32 + i] = v;
   }
 }
 
@@ -421,11 +518,11 @@ int launch_wide(const void *A, int64_t lda, int64_t OA, const void *B, int64_t l
   a.M = M;
   a.per = (int)(((M + 31) / 32 + G - 1) / G);
   a.grid = grid_taps(grid);
-  a.chunks = (int)G;
+  a.chunks = (int)G, a.batches = 1;
   a.ny = (int)((OA + 255) / 256);
   a.nz = (int)((OB + 255) / 256) * a.grid.taps;
   a.partials = partials, a.col_sums = col_sums;
-  auto kernel = grid ? wgrad_kernel<true> : wgrad_kernel<false>;
+  auto kernel = grid ? wgrad_kernel<1> : wgrad_kernel<0>;
   const size_t lds = (size_t)kStages * kStageBytes;
   if (int rc = allow_dynamic_lds(kernel, lds)) return rc;
   hipLaunchKernelGGL(kernel, dim3((unsigned)((G * a.ny * a.nz + 7) / 8 * 8)), dim3(512), lds, st, a);
@@ -466,8 +563,62 @@ int product(int dtype, int64_t M, const void *A, int64_t lda, int64_t OA, const 
     s.src[1] = sums, s.dst[1] = col_sums, s.n[1] = OA;
     blocks += (OA + 31) / 32;
   }
-  s.G = (int)G, s.taps = taps, s.OB = (int)OB;
+  s.G[0] = s.G[1] = (int)G, s.taps = taps, s.OB = (int)OB;
   hipLaunchKernelGGL(sum_partials_kernel, dim3((unsigned)blocks), dim3(256), 0, st, s);
+  return launch_status();
+}
+
+// dst[e] = sum over `rows` rows of n floats
+int sum_rows(const float *src, int64_t rows, int64_t n, float *dst, hipStream_t st) {
+  SumArgs s{};
+  s.src[0] = src, s.dst[0] = dst, s.n[0] = n, s.G[0] = (int)rows, s.taps = 1;
+  s.blocks0 = (n + 31) / 32;
+  hipLaunchKernelGGL(sum_partials_kernel, dim3((unsigned)s.blocks0), dim3(256), 0, st, s);
+  return launch_status();
+}
+
+// ---- the layer's output gradient against the packed slice weights ----
+static int64_t output_chunks(const pa_shape &s, int num_cu) {  // row chunks per batch element
+  const int64_t HS = s.H * s.S, tiles = ((HS + 255) / 256) * ((s.C + 255) / 256), tpb = (s.N + 31) / 32;
+  int64_t g = chunks_for(s.N, tiles * s.B, HS * s.C, num_cu);
+  if (g > tpb) g = tpb;
+  return g < 1 ? 1 : g;
+}
+
+int64_t output_backward_workspace_bytes(const pa_shape &s, int num_cu) {
+  const int64_t G = output_chunks(s, num_cu), n = s.H * s.S * s.C;
+  return (s.B * n * (G + 1) + s.B * G * s.C) * 4;
+}
+
+// dy (B, N, C) bf16, w_pack and out_token of the forward, w_out (C, H*32) bf16 -> d tok' (B,H,S,32), d W_out, d b_out
+int output_backward(const pa_shape &s, const void *w_pack, const void *dy, const float *out_token, const void *w_out,
+                    void *workspace, float *d_out_token, float *d_w_out, float *d_b_out, int num_cu, hipStream_t st) {
+  const int64_t G = output_chunks(s, num_cu), HS = s.H * s.S, n = HS * s.C;
+  float *P = static_cast<float *>(workspace), *partials = P + s.B * n, *sums = partials + s.B * G * n;
+  Args a{};
+  a.B = static_cast<const uint16_t *>(dy);
+  a.pack = static_cast<const u32x4 *>(w_pack);
+  a.ldb = (int)s.C, a.OA = (int)HS, a.OB = (int)s.C;
+  a.M = s.N, a.tpb = (int)((s.N + 31) / 32), a.tile_units = (int)(HS / 16 * 64);
+  a.per = (int)((a.tpb + G - 1) / G);
+  a.grid = grid_taps(nullptr);
+  a.chunks = (int)G, a.batches = (int)s.B;
+  a.ny = (int)((HS + 255) / 256), a.nz = (int)((s.C + 255) / 256);
+  a.partials = partials, a.col_sums = sums;
+  const size_t lds = (size_t)kStages * kStageBytes;
+  int rc = allow_dynamic_lds(wgrad_kernel<2>, lds);
+  if (rc) return rc;
+  hipLaunchKernelGGL(wgrad_kernel<2>, dim3((unsigned)((s.B * G * a.ny * a.nz + 7) / 8 * 8)), dim3(512), lds, st, a);
+  if ((rc = launch_status())) return rc;
+  SumArgs sa{};
+  sa.src[0] = partials, sa.dst[0] = P, sa.n[0] = n, sa.G[0] = (int)G, sa.taps = 1;
+  sa.blocks0 = (n + 31) / 32;
+  sa.src[1] = sums, sa.dst[1] = d_b_out, sa.n[1] = s.C, sa.G[1] = (int)(s.B * G);
+  hipLaunchKernelGGL(sum_partials_kernel, dim3((unsigned)(sa.blocks0 + (s.C + 31) / 32), (unsigned)s.B), dim3(256), 0, st, sa);
+  if ((rc = launch_status())) return rc;
+  const int64_t wgs = s.B * s.H * ((s.S + 31) / 32) + s.H * (s.C / 32);
+  hipLaunchKernelGGL(token_grad_kernel, dim3((unsigned)wgs), dim3(256), 0, st, P, static_cast<const uint16_t *>(w_out),
+                     out_token, d_out_token, d_w_out, (int)s.B, (int)s.H, (int)s.S, (int)s.C);
   return launch_status();
 }
 

@@ -569,24 +569,6 @@ class MfmaStages:
                                             out_x.data_ptr(), self._stream()), "pa_mfma_deslice")
         return out_x
 
-    def slice_softmax_backward(self, x_mid, fx_mid, d_out_x, d_num, d_norm):
-        """Returns (d_proj (B,N,2HD) = [d x_mid | d fx_mid], d_z (B,N,H,S), d clamp(temperature) (H) float32)."""
-        _need_cuda(x_mid, fx_mid, d_out_x, d_num, d_norm)
-        d = self.dims
-        nbytes = self.lib.pa_mfma_backward_tables_bytes(byref(self.shape))
-        groups = self.lib.pa_mfma_backward_groups(byref(self.shape))
-        if nbytes < 0 or groups < 0:
-            _lib.check(int(min(nbytes, groups)), "pa_mfma_backward_tables_bytes")
-        tables = torch.empty(int(nbytes), dtype=torch.uint8, device=self.device)
-        d_proj = torch.empty(d.B, d.N, 2 * d.H * 32, dtype=torch.bfloat16, device=self.device)
-        d_z = torch.empty(d.B, d.N, d.H, d.S, dtype=torch.bfloat16, device=self.device)
-        dT = torch.empty(int(groups), d.H, dtype=torch.float32, device=self.device)
-        _lib.check(self.lib.pa_mfma_slice_softmax_backward(
-            byref(self.shape), byref(self.cparams), x_mid.data_ptr(), fx_mid.data_ptr(), d_out_x.data_ptr(),
-            self.w_pack.data_ptr(), self.tok_out.data_ptr(), d_num.data_ptr(), d_norm.data_ptr(), tables.data_ptr(),
-            d_proj.data_ptr(), d_z.data_ptr(), dT.data_ptr(), self._stream()), "pa_mfma_slice_softmax_backward")
-        return d_proj, d_z, dT.sum(0)
-
     def deslice_project(self, y, residual=None, ln_weight=None, ln_bias=None, ln_eps=1e-5, ln_out=None):
         tail = _c_tail(residual, ln_weight, ln_bias, ln_eps, ln_out)
         _lib.check(self.lib.pa_mfma_deslice_project(byref(self.shape), self.blob.data_ptr(), self.w_pack.data_ptr(),
@@ -612,6 +594,98 @@ def mfma_backward_supported(dtype: torch.dtype, dims: LayerDims) -> bool:
     if rc < 0:
         _lib.check(rc, "pa_mfma_backward_query")
     return bool(rc)
+
+
+def _c_plus(params: dict):
+    return byref(_lib.PaPlusParams(*[_lib.ptr(params[k]) for k, _ in _lib.PaPlusParams._fields_]))
+
+
+def point_backward(x_mid, fx_mid, d_out_x, tok_out, d_num, d_norm, params, dims: LayerDims):
+    """Per-point part of the backward pass for bf16 layers with 32-wide heads.  Returns (d_proj (B,N,2HD) = [d x_mid |
+    d fx_mid], d W_slice (S, D), d b_slice (S), d temperature (H)); tok_out None: no deslice term."""
+    _need_cuda(x_mid, fx_mid, d_out_x, tok_out, d_num, d_norm)
+    lib, shape, S, D, H = _lib.load(), dims.c(), dims.S, dims.D, dims.H
+    nbytes = lib.pa_point_backward_workspace_bytes(byref(shape), 0)
+    if nbytes < 0:
+        _lib.check(int(nbytes), "pa_point_backward_workspace_bytes")
+    workspace = torch.empty(int(nbytes), dtype=torch.uint8, device=x_mid.device)
+    d_proj = torch.empty(dims.B, dims.N, 2 * H * D, dtype=x_mid.dtype, device=x_mid.device)
+    grads = torch.empty(lib.pa_point_backward_grads(byref(shape), 0), dtype=torch.float32, device=x_mid.device)
+    _lib.check(lib.pa_point_backward(
+        byref(shape), byref(_c_params(params)), None, x_mid.data_ptr(), fx_mid.data_ptr(), d_out_x.data_ptr(), None,
+        _lib.ptr(tok_out), d_num.data_ptr(), d_norm.data_ptr(), workspace.data_ptr(), int(nbytes), d_proj.data_ptr(),
+        grads.data_ptr(), _lib.current_stream_ptr(x_mid.device)), "pa_point_backward")
+    return d_proj, grads[:S * D].view(S, D), grads[S * D:S * D + S], grads[S * D + S:]
+
+
+def output_backward(w_pack, dy, tok_out, w_out, dims: LayerDims):
+    """From dy (B,N,C) bf16 and the forward's packed slice weights: (d tok_out (B,H,S,D), d W_out (C,HD), d b_out (C))."""
+    _need_cuda(w_pack, dy, tok_out, w_out)
+    lib, shape = _lib.load(), dims.c()
+    nbytes = lib.pa_output_backward_workspace_bytes(byref(shape))
+    if nbytes < 0:
+        _lib.check(int(nbytes), "pa_output_backward_workspace_bytes")
+    f32 = dict(dtype=torch.float32, device=dy.device)
+    workspace = torch.empty(int(nbytes), dtype=torch.uint8, device=dy.device)
+    d_tok, d_w = torch.empty(dims.B, dims.H, dims.S, dims.D, **f32), torch.empty(dims.C, dims.H * dims.D, **f32)
+    d_b = torch.empty(dims.C, **f32)
+    _lib.check(lib.pa_output_backward(byref(shape), w_pack.data_ptr(), dy.data_ptr(), tok_out.data_ptr(), w_out.data_ptr(),
+                                      workspace.data_ptr(), int(nbytes), d_tok.data_ptr(), d_w.data_ptr(), d_b.data_ptr(),
+                                      _lib.current_stream_ptr(dy.device)), "pa_output_backward")
+    return d_tok, d_w, d_b
+
+
+def layer_train_supported(dtype: torch.dtype, dims: LayerDims, plus: bool = False) -> bool:
+    """True where a layer trains in the two library calls below (bf16, 32-wide heads)."""
+    if dtype != torch.bfloat16:
+        return False
+    return _lib.load().pa_layer_train_bytes(byref(dims.c()), 1 if plus else 0, _lib.PA_TRAIN_SAVED) > 0
+
+
+def layer_train_forward(x, uniform, params: dict, dims: LayerDims):
+    """(y, saved) of a bf16 layer.  `params`: the layer's own parameters under the names of `pa_params` /
+    `pa_plus_params`, the three large weights all float32 or all bfloat16 in torch's layout, the rest float32."""
+    _need_cuda(x, uniform)
+    lib, shape, plus = _lib.load(), dims.c(), uniform is not None
+    nbytes = lib.pa_layer_train_bytes(byref(shape), int(plus), _lib.PA_TRAIN_FORWARD)
+    if nbytes < 0:
+        _lib.check(int(nbytes), "pa_layer_train_bytes")
+    saved = torch.empty(lib.pa_layer_train_bytes(byref(shape), int(plus), _lib.PA_TRAIN_SAVED), dtype=torch.uint8, device=x.device)
+    workspace = torch.empty(int(nbytes), dtype=torch.uint8, device=x.device)
+    y = torch.empty(dims.B, dims.N, dims.C, dtype=x.dtype, device=x.device)
+    _lib.check(lib.pa_layer_train_forward(
+        byref(shape), _lib.dtype_code(params["out_linear_weight"].dtype), byref(_c_params(params)),
+        _c_plus(params) if plus else None, x.data_ptr(), _lib.ptr(uniform), y.data_ptr(), saved.data_ptr(),
+        workspace.data_ptr(), int(nbytes), _lib.current_stream_ptr(x.device)), "pa_layer_train_forward")
+    return y, saved
+
+
+def layer_train_backward(x, uniform, dy, saved, params: dict, dims: LayerDims, need_dx: bool = True):
+    """(dx or None, gradients by parameter name, float32 views of one buffer) of `layer_train_forward`."""
+    _need_cuda(x, uniform, dy, saved)
+    lib, shape, plus = _lib.load(), dims.c(), uniform is not None
+    nbytes = lib.pa_layer_train_bytes(byref(shape), int(plus), _lib.PA_TRAIN_BACKWARD)
+    if nbytes < 0:
+        _lib.check(int(nbytes), "pa_layer_train_bytes")
+    workspace = torch.empty(int(nbytes), dtype=torch.uint8, device=x.device)
+    grads = torch.empty(lib.pa_layer_train_bytes(byref(shape), int(plus), _lib.PA_TRAIN_GRADS) // 4, dtype=torch.float32,
+                        device=x.device)
+    dx = torch.empty_like(x) if need_dx else None
+    _lib.check(lib.pa_layer_train_backward(
+        byref(shape), byref(_c_params(params)), _c_plus(params) if plus else None, x.data_ptr(), _lib.ptr(uniform),
+        dy.data_ptr(), saved.data_ptr(), _lib.ptr(dx), grads.data_ptr(), workspace.data_ptr(), int(nbytes),
+        _lib.current_stream_ptr(x.device)), "pa_layer_train_backward")
+    C, HD, S, D, H = dims.C, dims.H * dims.D, dims.S, dims.D, dims.H
+    taps = dims.conv_k ** (3 if dims.grid_d > 0 else 2) if dims.conv_k > 0 else 1
+    proj = ["in_project_x"] + ([] if plus else ["in_project_fx"])
+    sizes = [(n + "_weight", HD * C * taps) for n in proj] + [(n + "_bias", HD) for n in proj]
+    sizes += [("out_linear_weight", C * HD), ("out_linear_bias", C), ("qkv_project_weight", 3 * D * D),
+              ("in_project_slice_weight", S * D), ("in_project_slice_bias", S), ("temperature", H)]
+    if plus:
+        sizes += [("proj_temperature_0_weight", S * D), ("proj_temperature_0_bias", S), ("proj_temperature_2_weight", S),
+                  ("proj_temperature_2_bias", 1)]
+    parts = grads.split([n for _, n in sizes])
+    return dx, {name: part for (name, _), part in zip(sizes, parts)}
 
 
 def cols_gemm_supported(a: torch.Tensor, b: torch.Tensor, grid: LayerDims | None = None) -> bool:

@@ -19,7 +19,8 @@ import torch
 import torch.nn as nn
 
 from . import functional as PF
-from .autograd import PhysicsAttentionFunction, PhysicsAttentionMfmaFunction, PhysicsAttentionPlusFunction
+from .autograd import (PhysicsAttentionFunction, PhysicsAttentionMfmaFunction, PhysicsAttentionPlusFunction,
+                       PhysicsAttentionPlusMfmaFunction)
 
 __all__ = ["PhysicsAttentionBase", "PhysicsAttentionIrregularMesh", "PhysicsAttentionStructuredMesh2D",
            "PhysicsAttentionStructuredMesh3D"]
@@ -159,10 +160,11 @@ class PhysicsAttentionBase(nn.Module):
         dims = self.layer_dims(x)
         if not PF.backward_supported(x.dtype, dims):
             raise RuntimeError(f"the backward kernels do not serve this shape: {dims}")
-        fn = PhysicsAttentionMfmaFunction if PF.mfma_backward_supported(x.dtype, dims) else PhysicsAttentionFunction
+        on_mfma = PF.layer_train_supported(x.dtype, dims)
+        fn = PhysicsAttentionMfmaFunction if on_mfma else PhysicsAttentionFunction
         return fn.apply(
-            x, dims, self.kernel_params(x.dtype, x.device), self.in_project_x.weight, self.in_project_x.bias,
-            self.in_project_fx.weight, self.in_project_fx.bias, self.in_project_slice.weight,
+            x, dims, None if on_mfma else self.kernel_params(x.dtype, x.device), self.in_project_x.weight,
+            self.in_project_x.bias, self.in_project_fx.weight, self.in_project_fx.bias, self.in_project_slice.weight,
             self.in_project_slice.bias, self.temperature, self.qkv_project.weight, self.out_linear.weight,
             self.out_linear.bias)
 
@@ -173,12 +175,13 @@ class PhysicsAttentionBase(nn.Module):
             raise RuntimeError(f"the backward kernels do not serve this shape: {dims}")
         if noise_u is None:
             noise_u = torch.rand((dims.B, dims.N, dims.H, dims.S), dtype=x.dtype, device=x.device)
-        pt = self.proj_temperature
-        return PhysicsAttentionPlusFunction.apply(
-            x, noise_u.detach().to(x.dtype).contiguous(), dims, self.kernel_params(x.dtype, x.device),
-            self.in_project_x.weight, self.in_project_x.bias, self.in_project_slice.weight, self.in_project_slice.bias,
-            self.temperature, pt[0].weight, pt[0].bias, pt[2].weight, pt[2].bias, self.qkv_project.weight,
-            self.out_linear.weight, self.out_linear.bias)
+        noise_u, pt = noise_u.detach().to(x.dtype).contiguous(), self.proj_temperature
+        params = (self.in_project_x.weight, self.in_project_x.bias, self.in_project_slice.weight, self.in_project_slice.bias,
+                  self.temperature, pt[0].weight, pt[0].bias, pt[2].weight, pt[2].bias, self.qkv_project.weight,
+                  self.out_linear.weight, self.out_linear.bias)
+        if PF.layer_train_supported(x.dtype, dims, plus=True):
+            return PhysicsAttentionPlusMfmaFunction.apply(x, noise_u, dims, *params)
+        return PhysicsAttentionPlusFunction.apply(x, noise_u, dims, self.kernel_params(x.dtype, x.device), *params)
 
     @staticmethod
     def _wants_fp16(x: torch.Tensor) -> bool:

@@ -209,6 +209,49 @@ def test_bf16_mfma_backward_matches_oracle_and_general_path(B, N, C, S):
     assert t[0] == 0.0  # 0.3 is below the clamp: no gradient
 
 
+@pytest.mark.parametrize("variant,C,S,B,N,grid", [
+    ("irregular", 512, 64, 2, 333, None), ("irregular", 512, 128, 1, 100, None), ("irregular", 128, 64, 1, 1, None),
+    ("plus", 256, 64, 2, 1001, None), ("plus", 128, 16, 1, 63, None), ("plus", 128, 32, 3, 257, None),
+    ("plus", 512, 64, 1, 96, None), ("plus", 256, 128, 1, 130, None),
+    ("structured2d", 256, 64, 2, 21 * 17, (21, 17)), ("structured2d", 128, 16, 1, 33, (3, 11)),
+    ("structured2d", 512, 32, 1, 40, (8, 5)), ("structured3d", 256, 128, 1, 210, (5, 6, 7)),
+])
+def test_bf16_training_kernels_over_variants(variant, C, S, B, N, grid):
+    """Forward and backward of the bf16 training calls where their tiles, head groups and table forms change: every
+    parameter tensor and the input gradient against the fp32 oracle (bf16 data: 3e-2; the few scalars, sums of cancelling
+    terms, only have to be finite)."""
+    announce("bf16 training kernels", variant, C, S, B, N, grid)
+    H = C // 32
+    torch.manual_seed(S + N)
+    plus = variant == "plus"
+    if plus:
+        ref = to.OraclePhysicsAttentionIrregularMesh(C, heads=H, dim_head=32, slice_num=S, plus=True)
+        hip = pn.PhysicsAttentionIrregularMesh(C, heads=H, dim_head=32, slice_num=S, use_te=False, plus=True)
+        hip.load_state_dict(ref.state_dict())
+        hip = hip.cuda()
+    else:
+        ref, hip = make_pair(variant, C, H, 32, S, spatial=grid, sharpen=2.0)
+    ref.train(), hip.train()
+    xb = torch.randn(B, N, C).bfloat16()
+    probe = torch.randn(B, N, C).bfloat16()
+    u = torch.rand(B, N, H, S).bfloat16()
+    assert PF.layer_train_supported(torch.bfloat16, hip.layer_dims(xb.cuda()), plus)
+
+    def run(m, x, probe, u):
+        x = x.clone().requires_grad_(True)
+        y = m.forward_with_noise(x, u) if plus else m(x)
+        y.backward(probe)
+        return y.detach(), {"x": x.grad, **{n: p.grad for n, p in m.named_parameters()}}
+
+    y_ref, want = run(ref, xb.float(), probe.float(), u.float())
+    y, got = run(hip, xb.cuda(), probe.cuda(), u.cuda())
+    assert_rel_l2(y, y_ref, "y (training forward)", tol=1e-2)
+    for name in want:
+        assert torch.isfinite(got[name]).all(), name
+        if want[name].numel() >= 32 and N > 1:
+            assert_rel_l2(got[name], want[name], f"grad {name}", tol=3e-2)
+
+
 def test_mfma_deslice_natural_layout():
     announce("MFMA deslice to natural layout")
     ref, hip = make_pair("irregular", 256, 8, 32, 64, sharpen=2.0)
