@@ -600,11 +600,11 @@ int pa_residual_layernorm(int dtype, int64_t rows, int64_t C, void *y, const pa_
 
 /* Backward of LayerNorm over the last axis (TR.py:210, :300-307; the reference relies on autograd): x, dy, dx (rows, C)
  * in the activation dtype, C a multiple of 4 (float32) / 8 (bf16) and <= 1024; the statistics are recomputed from x.
- * partials: float32 (pa_layernorm_backward_groups(rows), 2, C): [g][0][:] = that group's share of d gamma,
- * [g][1][:] of d beta; the caller adds them up over g. */
+ * dx = add + (gradient through the LayerNorm), add (rows, C) or NULL: the gradient that reaches x past it.
+ * grads (2, C) float32: d gamma, d beta; partials: pa_layernorm_backward_groups(rows) * 2 C floats of scratch. */
 int64_t pa_layernorm_backward_groups(int64_t rows);
-int pa_layernorm_backward(int dtype, int64_t rows, int64_t C, const void *x, const void *dy, const float *gamma,
-                          float eps, void *dx, float *partials, void *stream);
+int pa_layernorm_backward(int dtype, int64_t rows, int64_t C, const void *x, const void *dy, const void *add,
+                          const float *gamma, float eps, void *dx, float *partials, float *grads, void *stream);
 
 /* ---- whole layer ------------------------------------------------------------------------------ */
 

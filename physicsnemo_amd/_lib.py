@@ -287,8 +287,7 @@ def load() -> ctypes.CDLL:
     lib.pa_layernorm_backward_groups.restype = c_int64
     lib.pa_layernorm_backward_groups.argtypes = [c_int64]
     lib.pa_layernorm_backward.restype = c_int
-    lib.pa_layernorm_backward.argtypes = [c_int, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p,
-                                          c_void_p]
+    lib.pa_layernorm_backward.argtypes = [c_int, c_int64, c_int64] + [c_void_p] * 4 + [c_float] + [c_void_p] * 4
     _lib = lib
     return lib
 

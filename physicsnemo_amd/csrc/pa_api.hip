@@ -702,13 +702,13 @@ int64_t pa_layernorm_backward_groups(int64_t rows) {
   return pa::general::layernorm_backward_groups(rows);
 }
 
-int pa_layernorm_backward(int dtype, int64_t rows, int64_t C, const void *x, const void *dy, const float *gamma, float eps,
-                          void *dx, float *partials, void *stream) {
+int pa_layernorm_backward(int dtype, int64_t rows, int64_t C, const void *x, const void *dy, const void *add,
+                          const float *gamma, float eps, void *dx, float *partials, float *grads, void *stream) {
   if (dtype != PA_F32 && dtype != PA_BF16) return PA_ERR_UNSUPPORTED;
   if (rows <= 0 || C <= 0 || C > 1024) return PA_ERR_DIMS;
-  if (!x || !dy || !gamma || !dx || !partials) return PA_ERR_NULL;
-  if (!aligned16(x) || !aligned16(dy) || !aligned16(dx)) return PA_ERR_ALIGN;
-  return pa::general::layernorm_backward(dtype, rows, C, x, dy, gamma, eps, dx, partials,
+  if (!x || !dy || !gamma || !dx || !partials || !grads) return PA_ERR_NULL;
+  if (!aligned16(x) || !aligned16(dy) || !aligned16(add) || !aligned16(dx)) return PA_ERR_ALIGN;
+  return pa::general::layernorm_backward(dtype, rows, C, x, dy, add, gamma, eps, dx, partials, grads,
                                          static_cast<hipStream_t>(stream));
 }
 

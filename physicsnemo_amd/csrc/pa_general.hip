@@ -9,6 +9,8 @@
 //   slice_combine_attn_kernel fixed-order combine, / (norm + 1e-2), qkv, softmax(q k^T / sqrt D) v   (LDS resident)
 //   deslice_kernel            out_x[n,h,:] = sum_s w[n,h,s] * tok'[h,s,:]
 //   residual_ln_kernel        fx_new = y + residual; ln_out = LayerNorm(fx_new)
+#include <type_traits>
+
 #include "pa_common.h"
 #include "pa_host.h"
 
@@ -738,176 +740,241 @@ __global__ __launch_bounds__(256) void residual_ln_kernel(T *__restrict__ y, con
   }
 }
 
-// residual_ln_vec_kernel: the same with 16-byte accesses for rows that are whole 16-byte units (C % UE == 0,
-// C <= 64 * UPL * UE): lane l owns units l, l + 64, ... of its row and keeps them in registers between the passes.
-template <typename T, int UPL>
-__global__ __launch_bounds__(256) void residual_ln_vec_kernel(T *__restrict__ y, const T *__restrict__ residual,
-                                                              const float *__restrict__ gamma,
-                                                              const float *__restrict__ beta, float eps,
-                                                              T *__restrict__ ln_out, int64_t M, int C) {
-  constexpr int UE = 16 / sizeof(T);
-  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-  const int lane = threadIdx.x & 63;
-  const int units = C / UE;
-  float gam[UPL][UE], bet[UPL][UE];  // this lane's LayerNorm parameters stay in registers across its rows
+// Rows of whole 16-byte units (C % UE == 0): LPR lanes share a row, the smallest power of two that gives every unit a lane
+// (all 64 with UPL units each for rows beyond 64 units), so a wave works on 64 / LPR rows at once, every lane of an access
+// carries data, and the row sums are exchanges inside the group.  The next rows are fetched while these are worked on.
+template <int LPR>
+__device__ __forceinline__ float group_sum(float v) {
+#pragma unroll
+  for (int off = LPR / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+template <typename T>
+struct RowUnit {
+  static constexpr int UE = 16 / sizeof(T);
+  typedef uint32_t vec __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ void unpack(vec v, float (&f)[UE]) {
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+      for (int e = 0; e < UE; ++e) {
+        const uint32_t w = v[e];
+        f[e] = __uint_as_float(w);
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < UE; ++e) {
+        const uint32_t w = v[e >> 1];
+        f[e] = __uint_as_float((e & 1) ? (w & 0xffff0000u) : (w << 16));
+      }
+    }
+  }
+  static __device__ __forceinline__ vec pack(const float (&f)[UE]) {
+    vec v;
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+      for (int e = 0; e < UE; ++e) v[e] = __float_as_uint(f[e]);
+    } else {
+#pragma unroll
+      for (int w = 0; w < 4; ++w)
+        v[w] = (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)f[2 * w]) |
+               ((uint32_t)__builtin_bit_cast(uint16_t, (__bf16)f[2 * w + 1]) << 16);
+    }
+    return v;
+  }
+};
+
+// residual_ln_rows_kernel: y <- y + residual (if given), ln_out = LayerNorm(y) (if given).  Bound by HBM: 262 144 bf16
+// rows of 256 channels without a residual 56 us = 4.8 TB/s (one row per wave with half of its lanes idle: 88 us).
+template <typename T, int LPR, int UPL>
+__global__ __launch_bounds__(256) void residual_ln_rows_kernel(T *__restrict__ y, const T *__restrict__ residual,
+                                                               const float *__restrict__ gamma,
+                                                               const float *__restrict__ beta, float eps,
+                                                               T *__restrict__ ln_out, int64_t M, int C) {
+  using U = RowUnit<T>;
+  using vec = typename U::vec;
+  constexpr int UE = U::UE, RPW = 64 / LPR;
+  const int lane = threadIdx.x & 63, l = lane % LPR, sub = lane / LPR, units = C / UE;
+  float gam[UPL][UE], bet[UPL][UE];
 #pragma unroll
   for (int k = 0; k < UPL; ++k)
 #pragma unroll
     for (int e = 0; e < UE; ++e) {
-      const int c = (lane + 64 * k) * UE + e;
+      const int c = (l + LPR * k) * UE + e;
       gam[k][e] = (ln_out && c < C) ? gamma[c] : 1.f;
       bet[k][e] = (ln_out && c < C) ? beta[c] : 0.f;
     }
-  // one wave per row at a time; the grid is sized to the machine and every wave walks rows a grid apart
-  for (int64_t m = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); m < M; m += (int64_t)gridDim.x * 4) {
-  T *yr = y + m * C;
-  float v[UPL][UE];
-  float sum = 0.f;
+  const float inv_c = 1.f / (float)C;
+  const int64_t step = (int64_t)gridDim.x * 4 * RPW;
+  int64_t mw = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW;  // the wave's first row
+  auto fetch = [&](int64_t m, vec(&a)[UPL], vec(&r)[UPL]) {
 #pragma unroll
-  for (int k = 0; k < UPL; ++k) {
-    const int u = lane + 64 * k;
-    if (u < units) {
-      u32x4 a = *reinterpret_cast<const u32x4 *>(yr + u * UE);
-      const T *ae = reinterpret_cast<const T *>(&a);
+    for (int k = 0; k < UPL; ++k) {
+      a[k] = r[k] = vec{0, 0, 0, 0};
+      if (m < M && l + LPR * k < units) {
+        a[k] = *reinterpret_cast<const vec *>(y + m * C + (l + LPR * k) * UE);
+        if (residual) r[k] = *reinterpret_cast<const vec *>(residual + m * C + (l + LPR * k) * UE);
+      }
+    }
+  };
+  vec a[UPL], r[UPL];
+  if (mw < M) fetch(mw + sub, a, r);
+  for (; mw < M; mw += step) {
+    const int64_t m = mw + sub;
+    vec an[UPL], rn[UPL];
+    fetch(m + step, an, rn);
+    float v[UPL][UE], sum = 0.f;
+#pragma unroll
+    for (int k = 0; k < UPL; ++k) {
+      U::unpack(a[k], v[k]);
       if (residual) {
-        u32x4 r = *reinterpret_cast<const u32x4 *>(residual + m * C + u * UE);
-        const T *re = reinterpret_cast<const T *>(&r);
-        alignas(16) T o[UE];
+        float rv[UE];
+        U::unpack(r[k], rv);
 #pragma unroll
-        for (int e = 0; e < UE; ++e) {
-          v[k][e] = round_to(yr, load_as_f32(ae + e) + load_as_f32(re + e));
-          store_from_f32(o + e, v[k][e]);
-        }
-        *reinterpret_cast<u32x4 *>(yr + u * UE) = *reinterpret_cast<const u32x4 *>(o);
-      } else {
-#pragma unroll
-        for (int e = 0; e < UE; ++e) v[k][e] = load_as_f32(ae + e);
+        for (int e = 0; e < UE; ++e) v[k][e] += rv[e];
+        const vec o = U::pack(v[k]);
+        U::unpack(o, v[k]);  // the sum as it is stored
+        if (m < M && l + LPR * k < units) *reinterpret_cast<vec *>(y + m * C + (l + LPR * k) * UE) = o;
       }
 #pragma unroll
       for (int e = 0; e < UE; ++e) sum += v[k][e];
     }
-  }
-  if (!ln_out) continue;
-  const float mean = wave_sum(sum) / (float)C;
-  float sq = 0.f;
+    if (ln_out) {
+      const float mean = group_sum<LPR>(sum) * inv_c;
+      float sq = 0.f;
 #pragma unroll
-  for (int k = 0; k < UPL; ++k)
-    if (lane + 64 * k < units) {
+      for (int k = 0; k < UPL; ++k)
+        if (l + LPR * k < units) {
 #pragma unroll
-      for (int e = 0; e < UE; ++e) {
-        const float d = v[k][e] - mean;
-        sq = fmaf(d, d, sq);
+          for (int e = 0; e < UE; ++e) {
+            const float d = v[k][e] - mean;
+            sq = fmaf(d, d, sq);
+          }
+        }
+      const float rstd = rsqrtf(group_sum<LPR>(sq) * inv_c + eps);
+#pragma unroll
+      for (int k = 0; k < UPL; ++k) {
+#pragma unroll
+        for (int e = 0; e < UE; ++e) v[k][e] = (v[k][e] - mean) * rstd * gam[k][e] + bet[k][e];
+        if (m < M && l + LPR * k < units) *reinterpret_cast<vec *>(ln_out + m * C + (l + LPR * k) * UE) = U::pack(v[k]);
       }
     }
-  const float rstd = rsqrtf(wave_sum(sq) / (float)C + eps);
 #pragma unroll
-  for (int k = 0; k < UPL; ++k) {
-    const int u = lane + 64 * k;
-    if (u < units) {
-      alignas(16) T o[UE];
-#pragma unroll
-      for (int e = 0; e < UE; ++e)
-        store_from_f32(o + e, (v[k][e] - mean) * rstd * gam[k][e] + bet[k][e]);
-      *reinterpret_cast<u32x4 *>(ln_out + m * C + u * UE) = *reinterpret_cast<const u32x4 *>(o);
+    for (int k = 0; k < UPL; ++k) {
+      a[k] = an[k];
+      r[k] = rn[k];
     }
-  }
   }
 }
 
-// layernorm_backward_kernel: backward of y = (x - mean) * rstd * gamma + beta over rows of whole 16-byte units.
-//   xh = (x - mean) rstd;  g = dy gamma;  dx = rstd (g - mean_c(g) - xh mean_c(g xh));  d gamma = sum_rows dy xh;
-//   d beta = sum_rows dy.   One wave per row at a time (statistics recomputed from x), lane l owns units l, l + 64, ...;
-// every wave accumulates d gamma / d beta of its columns over the rows it walks, the four waves of a workgroup add up
-// through LDS and each workgroup leaves one partial [2][C] (the caller adds the partials in index order).
-template <typename T, int UPL>
-__global__ __launch_bounds__(256) void layernorm_backward_kernel(const T *__restrict__ x, const T *__restrict__ dy,
-                                                                 const float *__restrict__ gamma, float eps,
-                                                                 T *__restrict__ dx, float *__restrict__ partials,
-                                                                 int64_t M, int C) {
-  constexpr int UE = 16 / sizeof(T);
-  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// layernorm_backward_rows_kernel: backward of y = (x - mean) rstd gamma + beta.
+//   xh = (x - mean) rstd;  g = dy gamma;  dx = [add +] rstd (g - mean_c(g) - xh mean_c(g xh));  d gamma = sum_rows dy xh;
+//   d beta = sum_rows dy (statistics recomputed from x; `add`: the gradient that reaches x past the LayerNorm).
+// Every lane sums d gamma / d beta of its columns over the rows it walks, the groups and waves of a workgroup add up in
+// order through LDS, each workgroup leaves one partial [2][C].  Bound by HBM: 262 144 bf16 rows of 256 channels 73 us =
+// 5.5 TB/s (one row per wave: 128 us).
+template <typename T, int LPR, int UPL>
+__global__ __launch_bounds__(256) void layernorm_backward_rows_kernel(const T *__restrict__ x, const T *__restrict__ dy,
+                                                                      const T *__restrict__ add,
+                                                                      const float *__restrict__ gamma, float eps,
+                                                                      T *__restrict__ dx, float *__restrict__ partials,
+                                                                      int64_t M, int C) {
+  using U = RowUnit<T>;
+  using vec = typename U::vec;
+  constexpr int UE = U::UE, RPW = 64 / LPR;
   extern __shared__ float red[];  // [4 waves][2][C]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int units = C / UE;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l = lane % LPR, sub = lane / LPR, units = C / UE;
   float gam[UPL][UE], dg[UPL][UE], db[UPL][UE];
 #pragma unroll
   for (int k = 0; k < UPL; ++k)
 #pragma unroll
     for (int e = 0; e < UE; ++e) {
-      const int c = (lane + 64 * k) * UE + e;
+      const int c = (l + LPR * k) * UE + e;
       gam[k][e] = c < C ? gamma[c] : 0.f;
       dg[k][e] = db[k][e] = 0.f;
     }
   const float inv_c = 1.f / (float)C;
-  for (int64_t m = (int64_t)blockIdx.x * 4 + wave; m < M; m += (int64_t)gridDim.x * 4) {
-    float xv[UPL][UE], gv[UPL][UE];
-    float sum = 0.f;
+  const int64_t step = (int64_t)gridDim.x * 4 * RPW;
+  int64_t mw = ((int64_t)blockIdx.x * 4 + wave) * RPW;
+  auto fetch = [&](int64_t m, vec(&a)[UPL], vec(&d)[UPL], vec(&p)[UPL]) {
 #pragma unroll
     for (int k = 0; k < UPL; ++k) {
-      const int u = lane + 64 * k;
-#pragma unroll
-      for (int e = 0; e < UE; ++e) xv[k][e] = gv[k][e] = 0.f;
-      if (u < units) {
-        u32x4 a = *reinterpret_cast<const u32x4 *>(x + m * C + u * UE);
-        u32x4 d = *reinterpret_cast<const u32x4 *>(dy + m * C + u * UE);
-        const T *ae = reinterpret_cast<const T *>(&a), *de = reinterpret_cast<const T *>(&d);
-#pragma unroll
-        for (int e = 0; e < UE; ++e) {
-          xv[k][e] = load_as_f32(ae + e);
-          gv[k][e] = load_as_f32(de + e);  // dy for now
-          sum += xv[k][e];
-        }
+      a[k] = d[k] = p[k] = vec{0, 0, 0, 0};
+      if (m < M && l + LPR * k < units) {
+        const int64_t at = m * C + (l + LPR * k) * UE;
+        a[k] = *reinterpret_cast<const vec *>(x + at);
+        d[k] = *reinterpret_cast<const vec *>(dy + at);
+        if (add) p[k] = *reinterpret_cast<const vec *>(add + at);
       }
     }
-    const float mean = wave_sum(sum) * inv_c;
+  };
+  vec a[UPL], d[UPL], p[UPL];
+  if (mw < M) fetch(mw + sub, a, d, p);
+  for (; mw < M; mw += step) {
+    const int64_t m = mw + sub;
+    vec an[UPL], dn[UPL], pn[UPL];
+    fetch(m + step, an, dn, pn);
+    float xv[UPL][UE], gv[UPL][UE], sum = 0.f;
+#pragma unroll
+    for (int k = 0; k < UPL; ++k) {
+      U::unpack(a[k], xv[k]);
+      U::unpack(d[k], gv[k]);
+#pragma unroll
+      for (int e = 0; e < UE; ++e) sum += xv[k][e];
+    }
+    const float mean = group_sum<LPR>(sum) * inv_c;
     float sq = 0.f;
 #pragma unroll
     for (int k = 0; k < UPL; ++k)
-      if (lane + 64 * k < units) {
+      if (l + LPR * k < units) {
 #pragma unroll
         for (int e = 0; e < UE; ++e) {
           const float dlt = xv[k][e] - mean;
           sq = fmaf(dlt, dlt, sq);
         }
       }
-    const float rstd = rsqrtf(wave_sum(sq) * inv_c + eps);
+    const float rstd = rsqrtf(group_sum<LPR>(sq) * inv_c + eps);
     float s1 = 0.f, s2 = 0.f;
 #pragma unroll
     for (int k = 0; k < UPL; ++k)
-      if (lane + 64 * k < units) {
 #pragma unroll
-        for (int e = 0; e < UE; ++e) {
-          const float xh = (xv[k][e] - mean) * rstd, dyv = gv[k][e];
-          dg[k][e] = fmaf(dyv, xh, dg[k][e]);
-          db[k][e] += dyv;
-          const float g = dyv * gam[k][e];
-          xv[k][e] = xh;
-          gv[k][e] = g;
-          s1 += g;
-          s2 = fmaf(g, xh, s2);
-        }
+      for (int e = 0; e < UE; ++e) {  // lanes without a unit and rows beyond M hold dy = 0
+        const float xh = (xv[k][e] - mean) * rstd, dyv = gv[k][e], gg = dyv * gam[k][e];
+        dg[k][e] = fmaf(dyv, xh, dg[k][e]);
+        db[k][e] += dyv;
+        xv[k][e] = xh;
+        gv[k][e] = gg;
+        s1 += gg;
+        s2 = fmaf(gg, xh, s2);
       }
-    s1 = wave_sum(s1) * inv_c;
-    s2 = wave_sum(s2) * inv_c;
+    s1 = group_sum<LPR>(s1) * inv_c;
+    s2 = group_sum<LPR>(s2) * inv_c;
 #pragma unroll
     for (int k = 0; k < UPL; ++k) {
-      const int u = lane + 64 * k;
-      if (u < units) {
-        alignas(16) T o[UE];
+      float o[UE], pv[UE];
+      U::unpack(p[k], pv);
 #pragma unroll
-        for (int e = 0; e < UE; ++e) store_from_f32(o + e, rstd * (gv[k][e] - s1 - xv[k][e] * s2));
-        *reinterpret_cast<u32x4 *>(dx + m * C + u * UE) = *reinterpret_cast<const u32x4 *>(o);
-      }
+      for (int e = 0; e < UE; ++e) o[e] = fmaf(rstd, gv[k][e] - s1 - xv[k][e] * s2, pv[e]);
+      if (m < M && l + LPR * k < units) *reinterpret_cast<vec *>(dx + m * C + (l + LPR * k) * UE) = U::pack(o);
+      a[k] = an[k];
+      d[k] = dn[k];
+      p[k] = pn[k];
     }
   }
 #pragma unroll
   for (int k = 0; k < UPL; ++k)
 #pragma unroll
     for (int e = 0; e < UE; ++e) {
-      const int c = (lane + 64 * k) * UE + e;
-      if (c < C) {
-        red[(wave * 2 + 0) * C + c] = dg[k][e];
-        red[(wave * 2 + 1) * C + c] = db[k][e];
+      float vg = dg[k][e], vb = db[k][e];
+#pragma unroll
+      for (int off = 32; off >= LPR; off >>= 1) {  // the wave's groups
+        vg += __shfl_xor(vg, off, 64);
+        vb += __shfl_xor(vb, off, 64);
+      }
+      const int c = (l + LPR * k) * UE + e;
+      if (sub == 0 && c < C) {
+        red[(wave * 2 + 0) * C + c] = vg;
+        red[(wave * 2 + 1) * C + c] = vb;
       }
     }
   __syncthreads();
@@ -1233,59 +1300,67 @@ int deslice(int dtype, const pa_shape &s, const void *w, const float *out_token,
   return dtype == PA_F32 ? deslice_t<float>(s, w, out_token, out_x, st) : deslice_t<bf16>(s, w, out_token, out_x, st);
 }
 
+// f(integral constants LPR, UPL) for rows of `units` 16-byte units; false: longer than the kernels' 256 units
+template <class F>
+static bool for_row_units(int units, F &&f) {
+  using std::integral_constant;
+  const auto one = integral_constant<int, 1>{};
+  if (units <= 4) f(integral_constant<int, 4>{}, one);
+  else if (units <= 8) f(integral_constant<int, 8>{}, one);
+  else if (units <= 16) f(integral_constant<int, 16>{}, one);
+  else if (units <= 32) f(integral_constant<int, 32>{}, one);
+  else if (units <= 64) f(integral_constant<int, 64>{}, one);
+  else if (units <= 128) f(integral_constant<int, 64>{}, integral_constant<int, 2>{});
+  else if (units <= 256) f(integral_constant<int, 64>{}, integral_constant<int, 4>{});
+  else return false;
+  return true;
+}
+
 template <typename T>
 static int residual_ln_t(const pa_shape &s, void *y, const pa_block_tail &tail, hipStream_t st) {
   const int64_t M = s.B * s.N;
   const int C = (int)s.C;
   constexpr int UE = 16 / sizeof(T);
-  dim3 grid((unsigned)((M + 3) / 4));
-  const dim3 vgrid((unsigned)std::min<int64_t>((M + 3) / 4, 256 * 16));  // the vector kernel's waves walk the rows
   T *yp = static_cast<T *>(y), *lo = static_cast<T *>(tail.ln_out);
   const T *res = static_cast<const T *>(tail.residual);
   const bool vec = C % UE == 0 && aligned16(y) && aligned16(tail.residual) && aligned16(tail.ln_out);
-  const int upl = (C / UE + 63) / 64;
-  if (vec && upl <= 1)
-    hipLaunchKernelGGL((residual_ln_vec_kernel<T, 1>), vgrid, dim3(256), 0, st, yp, res, tail.ln_gamma, tail.ln_beta,
-                       tail.ln_eps, lo, M, C);
-  else if (vec && upl <= 2)
-    hipLaunchKernelGGL((residual_ln_vec_kernel<T, 2>), vgrid, dim3(256), 0, st, yp, res, tail.ln_gamma, tail.ln_beta,
-                       tail.ln_eps, lo, M, C);
-  else if (vec && upl <= 4)
-    hipLaunchKernelGGL((residual_ln_vec_kernel<T, 4>), vgrid, dim3(256), 0, st, yp, res, tail.ln_gamma, tail.ln_beta,
-                       tail.ln_eps, lo, M, C);
-  else
-    hipLaunchKernelGGL((residual_ln_kernel<T>), grid, dim3(256), 0, st, yp, res, tail.ln_gamma, tail.ln_beta,
-                       tail.ln_eps, lo, M, C);
+  if (vec && for_row_units(C / UE, [&](auto lpr, auto upl) {
+        constexpr int LPR = decltype(lpr)::value, UPL = decltype(upl)::value, RPB = 4 * (64 / LPR);
+        const dim3 grid((unsigned)std::min<int64_t>((M + RPB - 1) / RPB, 256 * 8));
+        hipLaunchKernelGGL((residual_ln_rows_kernel<T, LPR, UPL>), grid, dim3(256), 0, st, yp, res, tail.ln_gamma,
+                           tail.ln_beta, tail.ln_eps, lo, M, C);
+      }))
+    return launch_status();
+  hipLaunchKernelGGL((residual_ln_kernel<T>), dim3((unsigned)((M + 3) / 4)), dim3(256), 0, st, yp, res, tail.ln_gamma,
+                     tail.ln_beta, tail.ln_eps, lo, M, C);
   return launch_status();
 }
 
-int64_t layernorm_backward_groups(int64_t rows) { return std::min<int64_t>((rows + 3) / 4, 256 * 8); }
+// workgroups (partial sums): every wave walks several rows, so that the partials stay few next to the rows
+int64_t layernorm_backward_groups(int64_t rows) { return std::min<int64_t>((rows + 15) / 16, 256 * 4); }
 
 template <typename T>
-static int layernorm_backward_t(int64_t rows, int C, const void *x, const void *dy, const float *gamma, float eps, void *dx,
-                                float *partials, hipStream_t st) {
+static int layernorm_backward_t(int64_t rows, int C, const void *x, const void *dy, const void *add, const float *gamma,
+                                float eps, void *dx, float *partials, hipStream_t st) {
   constexpr int UE = 16 / sizeof(T);
   if (C % UE != 0) return PA_ERR_UNSUPPORTED;
-  const int upl = (C / UE + 63) / 64;
   const dim3 grid((unsigned)layernorm_backward_groups(rows));
   const size_t lds = (size_t)8 * C * 4;
-  const T *xp = static_cast<const T *>(x), *dp = static_cast<const T *>(dy);
-  T *op = static_cast<T *>(dx);
-  if (upl <= 1)
-    hipLaunchKernelGGL((layernorm_backward_kernel<T, 1>), grid, dim3(256), lds, st, xp, dp, gamma, eps, op, partials, rows, C);
-  else if (upl <= 2)
-    hipLaunchKernelGGL((layernorm_backward_kernel<T, 2>), grid, dim3(256), lds, st, xp, dp, gamma, eps, op, partials, rows, C);
-  else if (upl <= 4)
-    hipLaunchKernelGGL((layernorm_backward_kernel<T, 4>), grid, dim3(256), lds, st, xp, dp, gamma, eps, op, partials, rows, C);
-  else
-    return PA_ERR_UNSUPPORTED;
-  return launch_status();
+  const bool ok = for_row_units(C / UE, [&](auto lpr, auto upl) {
+    constexpr int LPR = decltype(lpr)::value, UPL = decltype(upl)::value;
+    hipLaunchKernelGGL((layernorm_backward_rows_kernel<T, LPR, UPL>), grid, dim3(256), lds, st, static_cast<const T *>(x),
+                       static_cast<const T *>(dy), static_cast<const T *>(add), gamma, eps, static_cast<T *>(dx), partials,
+                       rows, C);
+  });
+  return ok ? launch_status() : PA_ERR_UNSUPPORTED;
 }
 
-int layernorm_backward(int dtype, int64_t rows, int64_t C, const void *x, const void *dy, const float *gamma, float eps,
-                       void *dx, float *partials, hipStream_t st) {
-  return dtype == PA_F32 ? layernorm_backward_t<float>(rows, (int)C, x, dy, gamma, eps, dx, partials, st)
-                         : layernorm_backward_t<bf16>(rows, (int)C, x, dy, gamma, eps, dx, partials, st);
+// grads (2, C): d gamma, d beta; partials: layernorm_backward_groups(rows) * 2 C floats of scratch; add may be NULL
+int layernorm_backward(int dtype, int64_t rows, int64_t C, const void *x, const void *dy, const void *add, const float *gamma,
+                       float eps, void *dx, float *partials, float *grads, hipStream_t st) {
+  const int rc = dtype == PA_F32 ? layernorm_backward_t<float>(rows, (int)C, x, dy, add, gamma, eps, dx, partials, st)
+                                 : layernorm_backward_t<bf16>(rows, (int)C, x, dy, add, gamma, eps, dx, partials, st);
+  return rc ? rc : wgrad::sum_rows(partials, layernorm_backward_groups(rows), 2 * C, grads, st);
 }
 
 int residual_ln(int dtype, const pa_shape &s, void *y, const pa_block_tail &tail, hipStream_t st) {

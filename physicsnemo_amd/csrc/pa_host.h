@@ -127,8 +127,8 @@ int combine_attention(const pa_shape &s, const pa_params &p, const float *partia
 int deslice(int dtype, const pa_shape &s, const void *w, const float *out_token, void *out_x, hipStream_t st);
 int residual_ln(int dtype, const pa_shape &s, void *y, const pa_block_tail &tail, hipStream_t st);
 int64_t layernorm_backward_groups(int64_t rows);
-int layernorm_backward(int dtype, int64_t rows, int64_t C, const void *x, const void *dy, const float *gamma, float eps,
-                       void *dx, float *partials, hipStream_t st);
+int layernorm_backward(int dtype, int64_t rows, int64_t C, const void *x, const void *dy, const void *add, const float *gamma,
+                       float eps, void *dx, float *partials, float *grads, hipStream_t st);
 }  // namespace general
 
 namespace conv {

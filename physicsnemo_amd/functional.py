@@ -279,20 +279,20 @@ def layernorm_supported(x: torch.Tensor) -> bool:
     return x.shape[-1] % unit == 0 and x.shape[-1] <= 1024
 
 
-def layernorm_backward(x, dy, ln_weight, ln_eps=1e-5):
-    """(dx, d gamma, d beta) of LayerNorm over the last axis; x, dy in the activation dtype, gamma float32."""
-    _need_cuda(x, dy, ln_weight)
+def layernorm_backward(x, dy, ln_weight, ln_eps=1e-5, add=None):
+    """(dx, d gamma, d beta) of LayerNorm over the last axis; x, dy in the activation dtype, gamma float32.  `add`: a
+    gradient that reaches x past the LayerNorm, summed into dx."""
+    _need_cuda(x, dy, ln_weight, add)
     lib = _lib.load()
     C = x.shape[-1]
     rows = x.numel() // C
-    groups = lib.pa_layernorm_backward_groups(rows)
-    partials = torch.empty(int(groups), 2, C, dtype=torch.float32, device=x.device)
+    partials = torch.empty(int(lib.pa_layernorm_backward_groups(rows)) * 2 * C, dtype=torch.float32, device=x.device)
+    grads = torch.empty(2, C, dtype=torch.float32, device=x.device)
     dx = torch.empty_like(x)
-    _lib.check(lib.pa_layernorm_backward(_lib.dtype_code(x.dtype), rows, C, x.data_ptr(), dy.data_ptr(),
+    _lib.check(lib.pa_layernorm_backward(_lib.dtype_code(x.dtype), rows, C, x.data_ptr(), dy.data_ptr(), _lib.ptr(add),
                                          ln_weight.data_ptr(), float(ln_eps), dx.data_ptr(), partials.data_ptr(),
-                                         _lib.current_stream_ptr(x.device)), "pa_layernorm_backward")
-    sums = partials.sum(0)
-    return dx, sums[0], sums[1]
+                                         grads.data_ptr(), _lib.current_stream_ptr(x.device)), "pa_layernorm_backward")
+    return dx, grads[0], grads[1]
 
 
 def mlp_supported(dtype: torch.dtype, rows: int, C: int, F: int) -> bool:

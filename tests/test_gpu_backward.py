@@ -441,6 +441,31 @@ def test_layernorm_and_linear_autograd_functions(dtype, rows, C):
         assert_rel_l2(lin.bias.grad, p2.bfloat16().float().reshape(-1, 256).sum(0), "linear db", tol=1e-2)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,C", [(1, 8), (7, 16), (1001, 64), (300, 96), (4099, 256), (63, 520), (130, 1024)])
+def test_layernorm_row_groups(dtype, rows, C):
+    """The row kernels where the lanes sharing a row change (4 .. 64 and several units per lane) and rows run out inside a
+    wave: forward with a residual, backward with a gradient past the LayerNorm, against float64."""
+    announce("layernorm row groups", dtype, rows, C)
+    torch.manual_seed(rows + C)
+    y, res, dy, add = (torch.randn(rows, C, device="cuda").to(dtype) for _ in range(4))
+    gam, bet = torch.randn(C, device="cuda"), torch.randn(C, device="cuda")
+    fx, out = PF.residual_layernorm(y.clone(), residual=res, ln_weight=gam, ln_bias=bet)
+    want_fx = (y.double() + res.double()).to(dtype)
+    assert torch.equal(fx, (y.float() + res.float()).to(dtype))
+    x = want_fx.double().requires_grad_(True)
+    g64, b64 = gam.double().requires_grad_(True), bet.double().requires_grad_(True)
+    ln = torch.nn.functional.layer_norm(x, (C,), g64, b64)
+    ln.backward(dy.double())
+    dx, dg, db = PF.layernorm_backward(want_fx, dy, gam, add=add)
+    # bf16 results carry one rounding (2^-9 of the value), fp32 ones a few of the row sums' 2^-24
+    tol = 4e-3 if dtype == torch.bfloat16 else 1e-6
+    assert_rel_l2(out, ln.detach(), "LayerNorm", tol=tol)
+    assert_rel_l2(dx, x.grad + add.double(), "dx + add", tol=tol)
+    assert_rel_l2(dg, g64.grad, "d gamma", tol=1e-5)
+    assert_rel_l2(db, b64.grad, "d beta", tol=1e-5)
+
+
 def test_output_dropout_in_training_matches_the_reference_site():
     """The reference applies nn.Dropout to the layer output in training mode (physics_attention.py:499): kept entries
     are y / (1 - p), the rest zero, gradients flow through the kept entries only; eval mode is the identity."""
