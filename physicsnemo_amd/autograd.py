@@ -640,6 +640,50 @@ def mlp(x: torch.Tensor, layers: torch.nn.Sequential) -> torch.Tensor:
         return linear(layers[1](h), layers[2].weight, layers[2].bias)
 
 
+class MlpResidualFunction(torch.autograd.Function):
+    """residual + Linear(gelu(Linear(x))) of a bf16 block in one kernel that keeps the hidden layer on chip; the backward
+    forms the hidden layer again from x, so nothing of it is kept between the passes (2 x 2 F bytes per row)."""
+
+    @staticmethod
+    def forward(ctx, x, residual, w1, b1, w2, b2):
+        w1_16, w2_16 = (w.detach().to(torch.bfloat16).contiguous() for w in (w1, w2))
+        b1_32, b2_32 = (b.detach().float().contiguous() for b in (b1, b2))
+        ctx.save_for_backward(x, w1_16, b1_32, w2_16)
+        ctx.param_dtypes = tuple(p.dtype for p in (w1, b1, w2, b2))
+        return PF.mlp_forward_packed(x, PF.mlp_pack(w1_16, w2_16), b1_32, b2_32, residual=residual)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, w1, b1, w2 = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        dy16 = _aligned(dy)
+        if torch.is_grad_enabled():  # create_graph: the same formulas as tensor ops, which can be differentiated again
+            h = torch.nn.functional.linear(x, w1, b1.to(x.dtype))
+            act, dh = torch.nn.functional.gelu(h), torch.ops.aten.gelu_backward(dy16 @ w2, h)
+        else:
+            act, dh = PF.mlp_backward(x, dy16, w1, b1, w2)
+        dx = dh @ w1 if need[0] else None
+        d_w1, d_b1 = _wgrad(_rows(dh), _rows(x)) if need[2] or need[3] else (None, None)
+        d_w2, d_b2 = _wgrad(_rows(dy16), _rows(act)) if need[4] or need[5] else (None, None)
+        grads = (g.to(t) if n else None for g, t, n in zip((d_w1, d_b1, d_w2, d_b2), ctx.param_dtypes, need[2:]))
+        return (dx, dy if need[1] else None, *grads)
+
+
+def norm_mlp_residual(x: torch.Tensor, ln: torch.nn.LayerNorm, layers: torch.nn.Sequential) -> torch.Tensor:
+    """x + Mlp(LayerNorm(x)) in training, as autocast would run it: on the fused MLP kernels where they serve the rows,
+    else on `layer_norm` and `mlp`."""
+    lin1, act, lin2 = layers[0], layers[1], layers[2]
+    normed, x = layer_norm_residual(x, ln)
+    C = x.shape[-1]
+    if (len(layers) == 3 and compute_dtype(normed) == normed.dtype == x.dtype == torch.bfloat16 and
+            isinstance(act, torch.nn.GELU) and act.approximate == "none" and lin1.bias is not None and
+            lin2.bias is not None and lin1.in_features == lin2.out_features == C and
+            PF.mlp_backward_supported(x.dtype, x.numel() // C, C, lin1.out_features)):
+        with torch.autocast("cuda", enabled=False):
+            return MlpResidualFunction.apply(_aligned(normed), _aligned(x), lin1.weight, lin1.bias, lin2.weight, lin2.bias)
+    return mlp(normed, layers) + x
+
+
 def layer_norm_linear(x: torch.Tensor, ln: torch.nn.LayerNorm, lin: torch.nn.Linear) -> torch.Tensor:
     """lin(ln(x)) in training (the output head), as autocast would run it: LayerNorm statistics in float32, its result
     rounded to the Linear's type."""
@@ -670,8 +714,43 @@ class LayerNormFunction(torch.autograd.Function):
         return dx, dg.to(ctx.param_dtypes[0]), db.to(ctx.param_dtypes[1]), None
 
 
+class LayerNormResidualFunction(torch.autograd.Function):
+    """(LayerNorm(x), x): the gradient of the second output, the residual stream going on, is added to that of the
+    LayerNorm by the backward kernel instead of by a pass of its own."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias, eps):
+        ctx.set_materialize_grads(False)
+        w32, b32 = weight.detach().float().contiguous(), bias.detach().float().contiguous()
+        rows = x.contiguous()
+        _, out = PF.residual_layernorm(rows, ln_weight=w32, ln_bias=b32, ln_eps=eps)
+        ctx.save_for_backward(rows, w32)
+        ctx.eps, ctx.param_dtypes = eps, (weight.dtype, bias.dtype)
+        return out, x.view_as(x)
+
+    @staticmethod
+    def backward(ctx, dy, d_pass):
+        if dy is None:
+            return d_pass, None, None, None
+        x, w32 = ctx.saved_tensors
+        add = None if d_pass is None else _aligned(d_pass.to(x.dtype))
+        dx, dg, db = PF.layernorm_backward(x, dy.to(x.dtype).contiguous(), w32, ctx.eps, add)
+        return dx, dg.to(ctx.param_dtypes[0]), db.to(ctx.param_dtypes[1]), None
+
+
+def _layer_norm_served(x: torch.Tensor, ln: torch.nn.LayerNorm) -> bool:
+    return len(ln.normalized_shape) == 1 and ln.elementwise_affine and ln.bias is not None and PF.layernorm_supported(x)
+
+
+def layer_norm_residual(x: torch.Tensor, ln: torch.nn.LayerNorm):
+    """(LayerNorm(x), x) for a pre-norm block: use the second element as the residual stream."""
+    if _layer_norm_served(x, ln) and x.requires_grad and torch.is_grad_enabled():
+        return LayerNormResidualFunction.apply(x, ln.weight, ln.bias, ln.eps)
+    return layer_norm(x, ln), x
+
+
 def layer_norm(x: torch.Tensor, ln: torch.nn.LayerNorm) -> torch.Tensor:
     """Differentiable LayerNorm: the library's kernels where they serve the rows, the module itself otherwise."""
-    if len(ln.normalized_shape) == 1 and ln.elementwise_affine and ln.bias is not None and PF.layernorm_supported(x):
+    if _layer_norm_served(x, ln):
         return LayerNormFunction.apply(x, ln.weight, ln.bias, ln.eps)
     return ln(x)

@@ -1110,6 +1110,26 @@ int pa_mlp_forward_packed(int dtype, int64_t rows, int64_t C, int64_t F, const v
                           compute_units(), static_cast<hipStream_t>(stream));
 }
 
+int64_t pa_mlp_backward_workspace_bytes(int dtype, int64_t rows, int64_t C, int64_t F) {
+  if (rows <= 0 || C <= 0 || F <= 0) return PA_ERR_DIMS;
+  if (dtype != PA_BF16 || rows > PA_MAX_ROWS || !pa::mlp::hidden_backward_supported(rows, C, F)) return PA_ERR_UNSUPPORTED;
+  return round_up(pa::mlp::hidden_backward_blob_bytes(C, F), 256);
+}
+
+int pa_mlp_backward(int dtype, int64_t rows, int64_t C, int64_t F, const pa_mlp_params *p, const void *u, const void *dy,
+                    void *act, void *d_hidden, void *workspace, int64_t workspace_bytes, void *stream) {
+  Range entry("pa_mlp_backward");
+  const int64_t need = pa_mlp_backward_workspace_bytes(dtype, rows, C, F);
+  if (need < 0) return (int)need;
+  if (!p || !p->w1 || !p->b1 || !p->w2 || !u || !dy || !act || !d_hidden || !workspace) return PA_ERR_NULL;
+  if (!aligned16(p->w1) || !aligned16(p->w2) || !aligned16(u) || !aligned16(dy) || !aligned16(act) || !aligned16(d_hidden) ||
+      !aligned16(workspace))
+    return PA_ERR_ALIGN;
+  if (workspace_bytes < need) return PA_ERR_WORKSPACE;
+  return pa::mlp::hidden_backward(rows, C, F, p->w1, p->b1, p->w2, u, dy, act, d_hidden, workspace, compute_units(),
+                                  static_cast<hipStream_t>(stream));
+}
+
 int pa_mlp_input_ln_query(int dtype, int64_t rows, int64_t C, int64_t F) {
   if (rows <= 0 || rows > PA_MAX_ROWS || C <= 0 || F <= 0) return 0;
   return pa::mlp::input_ln_supported(dtype, rows, C, F) ? 1 : 0;

@@ -9,6 +9,9 @@
 
 #include "pa_common.h"
 
+#include <type_traits>
+#include <utility>
+
 namespace pa {
 namespace mfma {
 
@@ -34,6 +37,41 @@ __device__ __forceinline__ u32x4 pack_half(const f32x16 &v, float scale = 1.f) {
 }
 
 __device__ __forceinline__ uint16_t to_bf16_bits(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
+
+// 2 floats -> 2 bf16 (round to nearest even), the first in the low half
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  bf16x2 o;
+  o[0] = (__bf16)a;
+  o[1] = (__bf16)b;
+  return __builtin_bit_cast(uint32_t, o);
+}
+
+// Four direct global -> LDS loads of 64 x 16 bytes each (no registers): the wave's lanes read sbase + 1024 q + 16 lane
+// (q = 0..3) and the data land at LDS byte address lds + 1024 q + 16 lane; the instruction offset advances the
+// global and the LDS address alike.  sbase and lds are wave-uniform.  The loads are asynchronous and counted by
+// vmcnt; their data must not be read before a wait and a barrier.
+__device__ __forceinline__ void load_4k_to_lds(const void *sbase, unsigned lane16, unsigned lds) {
+  asm volatile(
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %0\n\t"
+      "global_load_lds_dwordx4 %1, %0 offset:1024\n\t"
+      "global_load_lds_dwordx4 %1, %0 offset:2048\n\t"
+      "global_load_lds_dwordx4 %1, %0 offset:3072" ::"s"(sbase),
+      "v"(lane16), "s"(lds)
+      : "memory");
+}
+
+// f(integral_constant<int, 0>{}), ..., f(integral_constant<int, N - 1>{}): a loop whose index is a constant expression
+template <class F, int... I>
+__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F &&f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
 
 // value of lane l combined with the value of lane l ^ 32, without a trip through LDS: v_permlane32_swap hands every
 // lane the lower-half and the upper-half value of its column

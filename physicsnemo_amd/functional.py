@@ -461,6 +461,34 @@ def mlp_forward_packed(u, packed, b1, b2, residual=None, ln_weight=None, ln_bias
     return y if ln_out is None else (y, ln_out)
 
 
+def mlp_backward_supported(dtype: torch.dtype, rows: int, C: int, F: int) -> bool:
+    """True if `mlp_backward` serves this shape (bfloat16, C = 256) and `mlp_forward` does."""
+    if dtype != torch.bfloat16 or rows <= 0 or not mlp_supported(dtype, rows, C, F):
+        return False
+    return _lib.load().pa_mlp_backward_workspace_bytes(_lib.PA_BF16, rows, C, F) > 0
+
+
+def mlp_backward(u, dy, w1, b1, w2):
+    """(gelu(w1 . u + b1), d hidden), each (..., F): what the weight and input gradients of `mlp_forward` are products of.
+
+    u, dy (..., C), w1 (F, C), w2 (C, F) bfloat16; b1 float32."""
+    _need_cuda(u, dy, w1, b1, w2)
+    lib = _lib.load()
+    C, F = w1.shape[1], w1.shape[0]
+    rows = u.numel() // C
+    nbytes = lib.pa_mlp_backward_workspace_bytes(_lib.PA_BF16, rows, C, F)
+    if nbytes < 0:
+        _lib.check(int(nbytes), "pa_mlp_backward_workspace_bytes")
+    workspace = torch.empty(int(nbytes), dtype=torch.uint8, device=u.device)
+    act = torch.empty(*u.shape[:-1], F, dtype=u.dtype, device=u.device)
+    dh = torch.empty_like(act)
+    params = _lib.PaMlpParams(_lib.ptr(w1), _lib.ptr(b1), _lib.ptr(w2), None)
+    _lib.check(lib.pa_mlp_backward(_lib.PA_BF16, rows, C, F, byref(params), u.data_ptr(), dy.data_ptr(), act.data_ptr(),
+                                   dh.data_ptr(), workspace.data_ptr(), int(nbytes), _lib.current_stream_ptr(u.device)),
+               "pa_mlp_backward")
+    return act, dh
+
+
 class MfmaStages:
     """The bf16 MFMA kernels one by one (pa_mfma_* entry points) with their opaque buffers held as torch tensors.
 

@@ -212,18 +212,14 @@ class TransolverBlock(nn.Module):
     def _needs_grad(self, fx: torch.Tensor) -> bool:
         return torch.is_grad_enabled() and (fx.requires_grad or any(p.requires_grad for p in self.parameters()))
 
-    def _mlp_with_grad(self, normed: torch.Tensor) -> torch.Tensor:
-        """ln_mlp1[1] in training: its Linears use `autograd.linear` (weight gradients on the library's kernels)."""
-        return PA.mlp(normed, self.ln_mlp1[1].layers)
-
     def forward_chain(self, fx: torch.Tensor, normed_in: torch.Tensor | None, next_ln: nn.LayerNorm | None):
         """One block inside a chain of blocks: takes LayerNorm_1(fx) if the previous stage already produced it and
         returns (fx_out, next_ln(fx_out) or None).  Same arithmetic as `forward` (reference :300-303)."""
         if self._needs_grad(fx):
             # training: the layer's autograd path, LayerNorms / MLP as differentiable tensor ops (reference :300-303)
-            x_in = normed_in if normed_in is not None else PA.layer_norm(fx, self.ln_1)
+            x_in, fx = (normed_in, fx) if normed_in is not None else PA.layer_norm_residual(fx, self.ln_1)
             fx1 = self.Attn(x_in) + fx
-            return self._mlp_with_grad(PA.layer_norm(fx1, self.ln_mlp1[0])) + fx1, None
+            return PA.norm_mlp_residual(fx1, self.ln_mlp1[0], self.ln_mlp1[1].layers), None
         x_in = normed_in if normed_in is not None else self.ln_1(fx)
         whole = self._whole_block(x_in, fx, next_ln)
         if whole is not None:

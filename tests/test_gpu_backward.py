@@ -7,6 +7,7 @@ import torch
 
 from oracle import torch_oracle as to
 import physicsnemo_amd as pn
+from physicsnemo_amd import autograd as PA
 from physicsnemo_amd import functional as PF
 from gpu_util import announce, assert_fp32_close, assert_rel_l2, make_pair
 
@@ -464,6 +465,44 @@ def test_layernorm_row_groups(dtype, rows, C):
     assert_rel_l2(dx, x.grad + add.double(), "dx + add", tol=tol)
     assert_rel_l2(dg, g64.grad, "d gamma", tol=1e-5)
     assert_rel_l2(db, b64.grad, "d beta", tol=1e-5)
+
+
+@pytest.mark.parametrize("rows,F", [(1, 64), (255, 128), (257, 1024), (2000, 192), (70_001, 256)])
+def test_mlp_residual_block(rows, F):
+    """x + Mlp(LayerNorm(x)) of a bf16 block, forward and all gradients, at partial row blocks, with the hidden units
+    split between workgroups and not, and with more items than workgroups, against float64."""
+    announce("mlp residual", rows, F)
+    torch.manual_seed(rows)
+    C = 256
+    ln = torch.nn.LayerNorm(C).cuda()
+    layers = torch.nn.Sequential(torch.nn.Linear(C, F), torch.nn.GELU(), torch.nn.Linear(F, C)).cuda()
+    with torch.no_grad():
+        ln.weight.add_(0.3 * torch.randn_like(ln.weight))
+        for lin in (layers[0], layers[2]):
+            lin.weight.copy_(lin.weight.bfloat16().float())
+    x = torch.randn(rows, C, device="cuda").bfloat16().requires_grad_(True)
+    dy = torch.randn(rows, C, device="cuda").bfloat16()
+    assert PF.mlp_backward_supported(x.dtype, rows, C, F)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = PA.norm_mlp_residual(x, ln, layers)
+    y.backward(dy)
+    import copy
+    ln64, layers64 = copy.deepcopy(ln).double(), copy.deepcopy(layers).double()
+    ln64.zero_grad(), layers64.zero_grad()
+    x64 = x.detach().double().requires_grad_(True)
+    y64 = x64 + layers64(ln64(x64))
+    y64.backward(dy.double())
+    # every chain carries at most four bf16 roundings (LayerNorm, hidden layer or its gradient, result, sum): 2^-9 each
+    # at most, 2^-9 / sqrt(3) on the average
+    assert_rel_l2(y.detach(), y64.detach(), "y", tol=4e-3)
+    assert_rel_l2(x.grad, x64.grad, "dx", tol=5e-3)
+    for (name, p), q in zip(list(ln.named_parameters()) + list(layers.named_parameters()),
+                            list(ln64.parameters()) + list(layers64.parameters())):
+        assert p.grad.dtype == torch.float32
+        assert_rel_l2(p.grad, q.grad, "d " + name, tol=6e-3)
+    # create_graph takes the same formulas as tensor ops
+    (gx,) = torch.autograd.grad(PA.norm_mlp_residual(x, ln.bfloat16(), layers.bfloat16()), x, dy, create_graph=True)
+    assert_rel_l2(gx.detach(), x64.grad, "dx, create_graph", tol=1e-2)
 
 
 def test_output_dropout_in_training_matches_the_reference_site():
