@@ -63,6 +63,15 @@ __device__ __forceinline__ void load_4k_to_lds(const void *sbase, unsigned lane1
       : "memory");
 }
 
+// One such load with a 16-byte address per lane: lane l's unit lands at dst + 16 l.
+__device__ __forceinline__ void load_unit_to_lds(const void *p, unsigned dst) {  // lane l's 16 bytes land at dst + 16 l
+  asm volatile(
+      "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %0, off" ::"v"(p), "s"(dst)
+      : "memory");
+}
+
 // f(integral_constant<int, 0>{}), ..., f(integral_constant<int, N - 1>{}): a loop whose index is a constant expression
 template <class F, int... I>
 __device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {

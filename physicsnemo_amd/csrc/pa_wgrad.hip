@@ -15,6 +15,7 @@ namespace pa {
 namespace wgrad {
 
 using mfma::f32x16;
+using mfma::load_unit_to_lds;
 using mfma::u32x2;
 using mfma::u32x4;
 
@@ -52,14 +53,6 @@ struct Args {
   const u32x4 *pack;
   int tpb, tile_units;  // tiles per batch, 16-byte units of a tile
 };
-
-__device__ __forceinline__ void load_unit_to_lds(const void *p, unsigned dst) {  // lane l's 16 bytes land at dst + 16 l
-  asm volatile(
-      "s_mov_b32 m0, %1\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, off" ::"v"(p), "s"(dst)
-      : "memory");
-}
 
 // MODE 0: A and B are rows.  1: B gathered per tap of a convolution.  2: A packed, batch by batch; the chunks of a stage
 // are copied as they lie, the 16-byte units permuted within a chunk so that the transposing reads of a half-wave (4
