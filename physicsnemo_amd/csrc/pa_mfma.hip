@@ -726,7 +726,8 @@ __global__ __launch_bounds__(64 * ((S + 31) / 32)) void slice_attention_kernel(c
 // TAIL (compile time): 0 plain, 1 residual + LayerNorm, 2 residual only, 3 LayerNorm only.
 // MASKED = false: the steady-state kernel, full tiles only; its loop body has no branch around a memory
 // operation and issues the next tile's loads right after the last use of the current ones, so every wait
-// counts exactly the younger operations.  MASKED = true: the ragged last tile of each batch (one per workgroup).
+// counts exactly the younger operations.  MASKED = true: one tile per workgroup, the last `nfull` tiles of each batch: the
+// ragged one, or, where a workgroup per tile fits the chip, all of them in one launch (2 x 1 000 points: 5.9 us against 6.1 + 4.7).
 // ------------------------------------------------------------------------------------------------
 template <int C, int S, int TAIL, bool MASKED>
 __global__ __launch_bounds__(C * 2) void deslice_project_kernel(const u32x4 *__restrict__ blob, const u32x4 *__restrict__ w_pack,
@@ -766,8 +767,8 @@ __global__ __launch_bounds__(C * 2) void deslice_project_kernel(const u32x4 *__r
 
   // item -> (batch, tile-in-batch): full tiles for the steady-state kernel, the last (ragged) tile otherwise
   int64_t item = blockIdx.x;
-  int64_t b = MASKED ? item : item / nfull;
-  int64_t t = MASKED ? (int64_t)tpb - 1 : item - b * nfull;
+  int64_t b = item / nfull;
+  int64_t t = item - b * nfull + (MASKED ? tpb - nfull : 0);
   u32x4 wcur[NCH];
   rowvec rcur[ROWS];
   {
@@ -1271,7 +1272,8 @@ static int deslice_project_t(const pa_shape &s, const void *blob, const void *w_
   const float *gm = tail ? tail->ln_gamma : nullptr, *bt = tail ? tail->ln_beta : nullptr;
   const float eps = tail ? tail->ln_eps : 0.f;
   uint16_t *lo = static_cast<uint16_t *>(tail ? tail->ln_out : nullptr);
-  if (nfull > 0) {
+  const bool ragged = s.N % 32 != 0, at_once = ragged && s.B * tpb <= num_cu;
+  if (nfull > 0 && !at_once) {
     static int per_cu = 0;  // resident workgroups per CU for this instantiation
     if (per_cu == 0) {
       int nb = 0;
@@ -1288,9 +1290,10 @@ static int deslice_project_t(const pa_shape &s, const void *blob, const void *w_
     int rc = launch_status();
     if (rc) return rc;
   }
-  if (s.N % 32 != 0) {
-    hipLaunchKernelGGL((deslice_project_kernel<C, S, TAIL, true>), dim3((unsigned)s.B), dim3(C * 2), 0, st, bl, wp, tp, yo,
-                       res, gm, bt, eps, lo, s.N, (int)tpb, nfull, s.B);
+  if (ragged) {
+    const int per = at_once ? (int)tpb : 1;
+    hipLaunchKernelGGL((deslice_project_kernel<C, S, TAIL, true>), dim3((unsigned)(s.B * per)), dim3(C * 2), 0, st, bl, wp, tp,
+                       yo, res, gm, bt, eps, lo, s.N, (int)tpb, per, s.B * per);
     return launch_status();
   }
   return PA_OK;
