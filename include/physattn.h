@@ -583,7 +583,8 @@ typedef struct pa_block_head {
  * x (B,N,C) is LayerNorm_1(fx_in), which the caller has from the block before (or pa_preprocess_forward);
  * next: ln_gamma / ln_beta / ln_eps / ln_out of the LayerNorm that follows (ln_1 of the next block, or ln_mlp2[0]),
  * residual must be NULL; next may be NULL.  fx1 and its LayerNorm are never stored.
- * Served where pa_block_query() is 1: float32, C = 128, 8 heads of 16, 32 slices, F a multiple of 128 (up to 1024).
+ * Served where pa_block_query() is 1: float32, 32 slices and either C = 128, 8 heads of 16, F a multiple of 128 (up to
+ * 1024), or an irregular mesh with C = 32 or 64 in heads of 8 or 16 and F a multiple of 32 whose weights fit LDS.
  * workspace: pa_block_workspace_bytes(). */
 int pa_block_query(int dtype, const pa_shape *shape, int64_t F);
 int64_t pa_block_workspace_bytes(int dtype, const pa_shape *shape, int64_t F);

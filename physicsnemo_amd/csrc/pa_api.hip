@@ -1400,14 +1400,39 @@ int pa_layer_forward(int dtype, const pa_shape *shape, const pa_params *p, const
   return rc;
 }
 
+// Workspace plan of a narrow block
+struct NarrowPlan {
+  int64_t off_w, off_partials, off_tok, off_norm, off_tok_out, total, G;
+};
+
+static NarrowPlan plan_narrow(const pa_shape &s) {
+  NarrowPlan p{};
+  const int64_t BHS = s.B * s.H * s.S;
+  int64_t off = 0;
+  auto take = [&](int64_t bytes) {
+    const int64_t at = off;
+    off += round_up(bytes, 256);
+    return at;
+  };
+  p.G = pa::narrow::groups(s, compute_units());
+  p.off_w = take(s.B * s.N * s.H * s.S * 4);
+  p.off_partials = take((p.G + 1) * BHS * (s.D + 1) * 4);  // one more: where the combine pass leaves the sum
+  p.off_tok = take(BHS * s.D * 4);
+  p.off_norm = take(BHS * 4);
+  p.off_tok_out = take(BHS * s.D * 4);
+  p.total = off;
+  return p;
+}
+
 int pa_block_query(int dtype, const pa_shape *shape, int64_t F) {
   if (check_shape(dtype, shape)) return 0;
-  return pa::f32rows::block_supported(dtype, *shape, F) ? 1 : 0;
+  return pa::f32rows::block_supported(dtype, *shape, F) || pa::narrow::block_supported(dtype, *shape, F) ? 1 : 0;
 }
 
 int64_t pa_block_workspace_bytes(int dtype, const pa_shape *shape, int64_t F) {
   int rc = check_shape(dtype, shape);
   if (rc) return rc;
+  if (pa::narrow::block_supported(dtype, *shape, F)) return plan_narrow(*shape).total;
   if (!pa::f32rows::block_supported(dtype, *shape, F)) return PA_ERR_UNSUPPORTED;
   return plan_general(dtype, *shape).total + round_up(pa::f32rows::block_blob_bytes(F), 256);
 }
@@ -1432,11 +1457,21 @@ int pa_block_forward(int dtype, const pa_shape *shape, const pa_params *p, const
     if (!aligned16(head->weight)) return PA_ERR_ALIGN;
   }
   const pa_shape &s = *shape;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  char *ws = static_cast<char *>(workspace);
+  if (pa::narrow::block_supported(dtype, s, mlp->F)) {
+    const NarrowPlan np = plan_narrow(s);
+    if (workspace_bytes < np.total) return PA_ERR_WORKSPACE;
+    auto at = [&](int64_t off) { return reinterpret_cast<float *>(ws + off); };
+    if ((rc = pa::narrow::front(s, *p, x, at(np.off_w), at(np.off_partials), compute_units(), st))) return rc;
+    if ((rc = pa::general::combine_attention(s, *p, at(np.off_partials), np.G, at(np.off_tok), at(np.off_norm),
+                                             at(np.off_tok_out), st)))
+      return rc;
+    return pa::narrow::block_tail(s, *p, *mlp, at(np.off_w), at(np.off_tok_out), fx_in, fx_out, next, head, compute_units(), st);
+  }
   if (!pa::f32rows::block_supported(dtype, s, mlp->F)) return PA_ERR_UNSUPPORTED;
   const GeneralPlan plan = plan_general(dtype, s);
   if (workspace_bytes < plan.total + pa::f32rows::block_blob_bytes(mlp->F)) return PA_ERR_WORKSPACE;
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  char *ws = static_cast<char *>(workspace);
   void *x_mid = ws + plan.off_x_mid, *fx_mid = ws + plan.off_fx_mid, *w = ws + plan.off_w;
   float *partials = reinterpret_cast<float *>(ws + plan.off_partials);
   float *tok = reinterpret_cast<float *>(ws + plan.off_tok), *norm = reinterpret_cast<float *>(ws + plan.off_norm);

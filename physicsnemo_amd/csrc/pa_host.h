@@ -174,6 +174,18 @@ int premlp_forward(int64_t rows, int64_t c_in, int64_t F, const void *w1, const 
                    const float *b2, const void *u, void *y, const pa_block_tail *tail, void *blob, hipStream_t st);
 }  // namespace f32rows
 
+namespace narrow {
+// float32 blocks of 32 or 64 channels (heads of 8 or 16, 32 slices, irregular mesh): `front` leaves the slice weights
+// (B, N, H, S) and groups() partial token sums as the general combine kernels read them, block_tail is
+// f32rows::block_tail for these widths
+bool block_supported(int dtype, const pa_shape &s, int64_t F);
+int64_t groups(const pa_shape &s, int num_cu);
+int front(const pa_shape &s, const pa_params &p, const void *x, float *w, float *partials, int num_cu, hipStream_t st);
+int block_tail(const pa_shape &s, const pa_params &p, const pa_block_mlp &m, const float *w, const float *out_token,
+               const void *fx_in, void *fx_out, const pa_block_tail *next, const pa_block_head *head, int num_cu,
+               hipStream_t st);
+}  // namespace narrow
+
 namespace backward {
 size_t attention_lds_bytes(const pa_shape &s);
 int slice_attention(const pa_shape &s, const pa_params &p, const float *slice_token, const float *slice_norm,

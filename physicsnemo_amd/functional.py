@@ -327,7 +327,8 @@ def mlp_forward(u, w1, b1, w2, b2, residual=None, ln_weight=None, ln_bias=None, 
 
 
 def block_supported(dtype: torch.dtype, dims: LayerDims, F: int) -> bool:
-    """True if `block_forward` serves the shape (float32, C = 128, 8 heads of 16, 32 slices, F a multiple of 128)."""
+    """True if `block_forward` serves the shape (float32, 32 slices: C = 128 in 8 heads of 16, F a multiple of 128; or
+    C = 32 / 64 in heads of 8 / 16 on an irregular mesh, F a multiple of 32)."""
     if dtype != torch.float32:
         return False
     return bool(_lib.load().pa_block_query(_lib.PA_F32, byref(dims.c()), F))

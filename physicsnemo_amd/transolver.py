@@ -242,8 +242,8 @@ class TransolverBlock(nn.Module):
 
     def _whole_block(self, x_in: torch.Tensor, fx: torch.Tensor, next_ln: nn.LayerNorm | None,
                      head: nn.Linear | None = None):
-        """The block behind ln_1 in one library call (pa_block_forward) where the shape is served (float32, hidden 128,
-        8 heads of 16, 32 slices), else None.  With `head` (the last block's ln_mlp2[1], up to 4 outputs) the second
+        """The block behind ln_1 in one library call (pa_block_forward) where the shape is served (float32, 32
+        slices; hidden 128 in heads of 16, or 32 / 64 channels on an irregular mesh), else None.  With `head` (the last block's ln_mlp2[1], up to 4 outputs) the second
         element of the result is the head's output instead of the LayerNorm."""
         attn, mlp = self.Attn, self.ln_mlp1[1]
         if not (x_in.is_cuda and x_in.dtype == torch.float32 and fx.dtype == torch.float32 and not self.fp8_weights

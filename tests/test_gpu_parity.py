@@ -140,6 +140,42 @@ def test_fp32_whole_block_in_one_call(spatial, B, mlp_ratio, last):
         assert_fp32_close(whole[1], want, "block output, head in the call")
 
 
+@pytest.mark.parametrize("C,H,B,N,mlp_ratio,last", [(64, 4, 3, 1001, 1, True), (64, 8, 1, 31, 2, False),
+                                                    (32, 4, 2, 33, 4, True), (32, 2, 1, 70_000, 1, False)])
+def test_fp32_narrow_block_in_one_call(C, H, B, N, mlp_ratio, last):
+    # 32 / 64 channels in heads of 8 / 16 on an irregular mesh: less than a tile, ragged tiles, several tiles per wave,
+    # several chunks of hidden features, the output head in the call; run twice
+    announce("fp32 narrow block", C, H, B, N, mlp_ratio, last)
+    torch.manual_seed(4)
+    kw = dict(mlp_ratio=mlp_ratio, last_layer=last, out_dim=3, slice_num=32)
+    ref = to.OracleTransolverBlock(H, C, **kw).eval()
+    hip = pn.TransolverBlock(H, C, 0.0, use_te=False, **kw).eval()
+    with torch.no_grad():
+        for ln in (ref.ln_1, ref.ln_mlp1[0]):
+            ln.weight.add_(0.2 * torch.randn(C))
+            ln.bias.add_(0.2 * torch.randn(C))
+        ref.Attn.in_project_slice.weight.mul_(2.0)
+        ref.Attn.temperature.copy_(torch.linspace(0.3, 6.0, H).view_as(ref.Attn.temperature))  # beyond both clamps
+    hip.load_state_dict(ref.state_dict())
+    hip = hip.cuda()
+    fx = torch.randn(B, N, C)
+    next_ln = hip.ln_mlp2[0] if last else torch.nn.LayerNorm(C).cuda()
+    head = hip.ln_mlp2[1] if last else None
+    with torch.no_grad():
+        want = ref(fx)
+        xc = fx.cuda()
+        normed = hip.ln_1(xc)
+        whole = hip._whole_block(normed, xc, next_ln, head=head)
+        assert whole is not None
+        again = hip._whole_block(normed, xc, next_ln, head=head)
+    assert all(torch.equal(a, b) for a, b in zip(whole, again))
+    if last:
+        assert_fp32_close(whole[1], want, "block output, head in the call")
+    else:
+        assert_fp32_close(whole[0], want, "block output")
+        assert_fp32_close(whole[1], torch.nn.functional.layer_norm(want, (C,)), "next LayerNorm")
+
+
 def test_fp32_fused_path_is_bit_reproducible():
     # the float32 kernels stream weights and rows through LDS rings with asynchronous loads and reduce the token sums
     # in a fixed order: repeated calls on the same inputs must agree to the bit (a race would show up here first);
