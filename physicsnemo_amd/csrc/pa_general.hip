@@ -482,10 +482,13 @@ __global__ __launch_bounds__(256) void slice_partial_kernel(const T *__restrict_
 // combine_partials_kernel: second pass of the reduction, parallel over outputs.  grid (ceil(n_out/64), B*H);
 // 64 outputs x 4 quarter-ranges of the G partials per workgroup; each thread adds its quarter in index order,
 // the four quarter sums are then added in a fixed order ((q0 + q1) + q2) + q3: bit-reproducible, no atomics.
+// Bound by the latency of the partials, which other XCDs wrote: 16 of a thread's loads are in flight at once.  256 partials
+// of 8 x 2 112 floats 5.1 us; one load at a time 17.5.
 // ------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void combine_partials_kernel(const float *__restrict__ partials, int G,
                                                                int64_t partial_stride, float *__restrict__ combined,
                                                                int n_out) {
+  constexpr int kAhead = 16;
   __shared__ float quarter[4][64];
   const int t = threadIdx.x, q = t >> 6, l = t & 63;
   const int o = blockIdx.x * 64 + l;
@@ -495,7 +498,13 @@ __global__ __launch_bounds__(256) void combine_partials_kernel(const float *__re
   float acc = 0.f;
   if (o < n_out) {
     const float *src = partials + (int64_t)bh * n_out + o;
-    for (int g = g0; g < g1; ++g) acc += src[(int64_t)g * partial_stride];
+    for (int g = g0; g < g1; g += kAhead) {  // kAhead loads in flight, added in index order
+      float v[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) v[u] = src[(int64_t)min(g + u, g1 - 1) * partial_stride];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) acc += g + u < g1 ? v[u] : 0.f;
+    }
   }
   quarter[q][l] = acc;
   __syncthreads();
