@@ -774,9 +774,13 @@ static int launch_t(const GemmArgs &a, int nsets, hipStream_t st) {
 
 template <typename T>
 static int launch_n(const GemmArgs &a, int nsets, hipStream_t st) {
-  if (a.O <= 64) return launch_t<T, 2>(a, nsets, st);
-  if (a.O <= 128) return launch_t<T, 4>(a, nsets, st);
-  return launch_t<T, 8>(a, nsets, st);
+  // the widest tile of outputs the shape fills, narrower ones where it leaves CUs without a workgroup (8 rows, 16 -> 2 x 256:
+  // 69 us on one 256-wide workgroup per set, 21 us on four 64-wide ones)
+  const int64_t rows = a.pack_tpb > 0 ? (a.M / a.N) * a.pack_tpb * 32 : a.M, row_tiles = (rows + kRows - 1) / kRows * nsets;
+  auto fills = [&](int nt) { return row_tiles * ((a.O + 32 * nt - 1) / (32 * nt)) >= 256; };
+  if (a.O > 128 && fills(8)) return launch_t<T, 8>(a, nsets, st);
+  if (a.O > 64 && fills(4)) return launch_t<T, 4>(a, nsets, st);
+  return launch_t<T, 2>(a, nsets, st);
 }
 
 int launch(const GemmArgs &a, int nsets, int dtype, hipStream_t st) {
