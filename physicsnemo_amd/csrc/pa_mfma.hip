@@ -599,7 +599,8 @@ __global__ __launch_bounds__(256) void slice_reduce_kernel(const u32x4 *__restri
 // (v_mfma_f32_32x32x2_f32: A lane (i, g) holds A[i][k = g], B lane (i, g) holds B[k = g][i], C/D as above).
 // One workgroup per (b, h), one wave per tile of 32 slices; lane (i, g) of wave w owns slice s = 32w + i.
 //   tok[s][:]  = num[s][:] / (cnt[s] + 1e-2)                                    -> slice_token, slice_norm
-//   q^T, k^T, v^T (32 e x 32 s) = Wq|k|v (A) . tok^T (B: lane <-> s, k <-> d)    registers <-> e = rowmap(r, g)
+// Bound by latency: the weights come as float4 with the sums, one trip to memory, 9.2 us at S = 64 (as 48 single floats 11.5).
+//   q^T, k^T, v^T (32 e x 32 s) = Wq|k|v (A) . tok^T (B: lane <-> s, k <-> d = rowmap(r, g))    registers <-> e = rowmap(r, g)
 //   k, v -> LDS; scores^T (keys x queries) = k (A, from LDS) . q^T: register r of q^T is directly the B operand of
 //   the step whose reduction pair is d = rowmap(r, 0 / 1)
 //   softmax over the keys: in-lane over registers and key tiles + one exchange with lane ^ 32
@@ -630,16 +631,33 @@ __global__ __launch_bounds__(64 * ((S + 31) / 32)) void slice_attention_kernel(c
   const float wsum = src[D], cnt = wsum + kSliceNormEps;
   // fx_bias (H*32, or NULL): bias of in_project_fx left out of the summed fx_mid: sum_n w (fx + b) = sum_n w fx + b sum_n w
   const float *fb = fx_bias ? fx_bias + (bh % heads) * D : nullptr;
-  float tk[16];  // tok[s][2kk + g]
+  // the weights are requested with the sums: rows e = 32m + i of Wqkv, channels d = rowmap(r, g), four at a time
+  float4 wr[3][4];
+  if (reinterpret_cast<uintptr_t>(w_qkv) & 15u) {  // a parameter that starts off a 16-byte boundary
 #pragma unroll
-  for (int kk = 0; kk < 16; ++kk) {
-    const float num = fb ? fmaf(fb[2 * kk + g], wsum, src[2 * kk + g]) : src[2 * kk + g];
-    tk[kk] = live ? num / cnt : 0.f;
+    for (int m = 0; m < 3; ++m)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float *p = w_qkv + (32 * m + i) * D + 8 * q + 4 * g;
+        wr[m][q] = float4{p[0], p[1], p[2], p[3]};
+      }
+  } else {
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) wr[m][q] = *reinterpret_cast<const float4 *>(w_qkv + (32 * m + i) * D + 8 * q + 4 * g);
+  }
+  float tk[16];  // tok[s][rowmap(r, g)]
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int d = rowmap(r, g);
+    const float num = fb ? fmaf(fb[d], wsum, src[d]) : src[d];
+    tk[r] = live ? num / cnt : 0.f;
   }
   if (live) {
     if (slice_token) {
 #pragma unroll
-      for (int kk = 0; kk < 16; ++kk) slice_token[((int64_t)bh * S + s) * D + 2 * kk + g] = tk[kk];
+      for (int r = 0; r < 16; ++r) slice_token[((int64_t)bh * S + s) * D + rowmap(r, g)] = tk[r];
     }
     if (slice_norm && g == 0) slice_norm[(int64_t)bh * S + s] = cnt;
   }
@@ -647,12 +665,12 @@ __global__ __launch_bounds__(64 * ((S + 31) / 32)) void slice_attention_kernel(c
   f32x16 qT, kT, vT;
 #pragma unroll
   for (int r = 0; r < 16; ++r) qT[r] = kT[r] = vT[r] = 0.f;
+  auto at = [](const float4 &v, int j) { return j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w; };
 #pragma unroll
-  for (int kk = 0; kk < 16; ++kk) {
-    const float *wr = w_qkv + i * D + 2 * kk + g;  // row e = 32m + i of Wqkv, column d = 2kk + g
-    qT = mma32(wr[0], tk[kk], qT);
-    kT = mma32(wr[32 * D], tk[kk], kT);
-    vT = mma32(wr[64 * D], tk[kk], vT);
+  for (int r = 0; r < 16; ++r) {
+    qT = mma32(at(wr[0][r >> 2], r & 3), tk[r], qT);
+    kT = mma32(at(wr[1][r >> 2], r & 3), tk[r], kT);
+    vT = mma32(at(wr[2][r >> 2], r & 3), tk[r], vT);
   }
   // q scaled for a base-2 softmax: exp(x / sqrt(D)) = exp2(x * log2e / sqrt(D))
   const float qscale = kLog2e * 0.17677669529663687f;
