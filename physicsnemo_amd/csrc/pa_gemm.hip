@@ -592,10 +592,11 @@ int cols_gemm(const void *A, int64_t lda, int64_t OA, const void *B, int64_t ldb
 }
 
 // ------------------------------------------------------------------------------------------------
-// conv_gemm_kernel: the bf16 grid convolutions as implicit GEMM (rows x taps * channels) . W^T with whole steps of 64
-// channels of one tap.  Workgroup: 8 waves, 128 rows x 256 outputs, wave tile 64 x 64.  One step of both operands
-// (48 KB) is a stage; three stages form a ring in LDS, filled two steps ahead by direct global -> LDS loads (the
-// neighbours' rows are gathered by their addresses, a unit of zeros outside the grid), one barrier per step.  The loads
+// conv_gemm_kernel: the grid convolutions as implicit GEMM (rows x taps * channels) . W^T with whole steps of 128 bytes of
+// channels (64 bf16, 32 float32) of one tap.  Workgroup: bf16 8 waves, 128 rows x 256 outputs, wave tile 64 x 64; float32
+// 4 waves, 64 x 128, wave tile 32 x 64 (two workgroups per CU).  One step of both operands (48 / 24 KB) is a stage; three
+// stages form a ring in LDS, filled two steps ahead by direct global -> LDS loads (the neighbours' rows are gathered by
+// their addresses, a unit of zeros outside the grid), one barrier per step.  The loads
 // write 8 rows of 128 bytes contiguously, so position p of row r holds the row's 16-byte unit p ^ (r % 8): the eight
 // lanes of an access phase then fall on all banks.
 // Outputs: rows as 16-byte pieces (the product formed as out^T, lanes <-> rows), or with `out_pack` the un-transposed
@@ -604,16 +605,26 @@ int cols_gemm(const void *A, int64_t lda, int64_t OA, const void *B, int64_t ldb
 // and 512 -> 256 (77 GFLOP each): 105 and 96 us against 254 and 219 us of rows_gemm_mfma_kernel (registers one step ahead, two
 // barriers per step, no ring); 1 640 points: 40 and 75 us against 107 and 183.
 // ------------------------------------------------------------------------------------------------
-constexpr int kConvRows = 128, kConvOut = 256, kConvStages = 3, kConvStageBytes = (kConvRows + kConvOut) * 128;
+// float32 is bound by v_mfma_f32_32x32x2_f32 and by whole workgroups per CU: 4 x 85 x 85 points, 128 -> 2 x 128 and
+// 256 -> 128 (17 GFLOP each): 190 and 189 us against 227 and 242; 720 points: 50 and 93 against 192 and 217.
+constexpr int kConvStages = 3;
+template <typename T>
+struct ConvTile {  // waves: two along the rows, WC along the outputs; a wave stages 16 rows and 32 weight rows of a step
+  static constexpr int RT = sizeof(T) == 2 ? 2 : 1, WC = sizeof(T) == 2 ? 4 : 2, kWaves = 2 * WC;
+  static constexpr int kRows = 64 * RT, kOut = 64 * WC, kStageBytes = (kRows + kOut) * 128, KB = 128 / (int)sizeof(T);
+};
 __device__ const uint32_t kZeroUnit[4] = {0u, 0u, 0u, 0u};
 
-__global__ __launch_bounds__(512) void conv_gemm_kernel(GemmArgs a) {
-  extern __shared__ u32x4 ring[];  // [stage][128 input rows | 256 weight rows] of 128 bytes
+template <typename T>
+__global__ __launch_bounds__((ConvTile<T>::kWaves * 64)) void conv_gemm_kernel(GemmArgs a) {
+  using Q = ConvTile<T>;
+  constexpr int RT = Q::RT, UE = Unit<T>::kElems;
+  extern __shared__ u32x4 ring[];  // [stage][kRows input rows | kOut weight rows] of 128 bytes
   const int z = blockIdx.z, t = threadIdx.x, lane = t & 63, i = lane & 31, g = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), wr = (wave & 1) * 64, wc = (wave >> 1) * 64;
-  const uint16_t *in = static_cast<const uint16_t *>(a.in);
-  const int64_t m0 = (int64_t)blockIdx.x * kConvRows;
-  const int o0 = blockIdx.y * kConvOut;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), wr = (wave & 1) * (32 * RT), wc = (wave >> 1) * 64;
+  const T *in = static_cast<const T *>(a.in);
+  const int64_t m0 = (int64_t)blockIdx.x * Q::kRows;
+  const int o0 = blockIdx.y * Q::kOut;
   const int gd = a.gd > 0 ? a.gd : 1, ksd = a.gd > 0 ? a.ks : 1, pad = a.ks / 2, pad_d = a.gd > 0 ? pad : 0;
   // rows are numbered as in rows_gemm_mfma_kernel: first real row of 32-row tile `tile`, and how many of its rows exist
   const unsigned tpb = a.pack_tpb > 0 ? (unsigned)a.pack_tpb : 0u;
@@ -625,7 +636,7 @@ __global__ __launch_bounds__(512) void conv_gemm_kernel(GemmArgs a) {
   };
   // this wave stages input rows 16 wave + 8 k + lane / 8 (k = 0, 1) and weight rows 32 wave + 8 k + lane / 8 (k = 0 .. 3)
   const int unit = (lane & 7) ^ (lane >> 3);
-  const uint16_t *base[2], *wp = static_cast<const uint16_t *>(a.w[z]) + (int64_t)(o0 + 32 * wave + (lane >> 3)) * a.K + 8 * unit;
+  const T *base[2], *wp = static_cast<const T *>(a.w[z]) + (int64_t)(o0 + 32 * wave + (lane >> 3)) * a.K + UE * unit;
   int ci[2], cj[2], cl[2];
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
@@ -639,25 +650,25 @@ __global__ __launch_bounds__(512) void conv_gemm_kernel(GemmArgs a) {
     n /= gd;
     ci[k] = local < count ? (int)(n / a.gw) : -(1 << 20);  // no row: never inside the grid
     cj[k] = (int)(n % a.gw);
-    base[k] = in + m * a.C + 8 * unit;
+    base[k] = in + m * a.C + UE * unit;
   }
-  const int nkb = a.K / 64, cblocks = a.C / 64;
+  const int nkb = a.K / Q::KB, cblocks = a.C / Q::KB;
   int fu = 0, fv = 0, fz = 0, fc = 0;  // tap and channel block of the step fetched next
   auto fetch = [&](int kb) {           // past the last step: that one again, so that every step counts six loads
-    const unsigned dst = (unsigned)(uintptr_t)ring + (unsigned)(kb % kConvStages) * kConvStageBytes;
-    const int64_t shift = (((int64_t)(fu - pad) * a.gw + fv - pad) * gd + fz - pad_d) * a.C + 64 * fc;  // the neighbour, from the row
+    const unsigned dst = (unsigned)(uintptr_t)ring + (unsigned)(kb % kConvStages) * Q::kStageBytes;
+    const int64_t shift = (((int64_t)(fu - pad) * a.gw + fv - pad) * gd + fz - pad_d) * a.C + Q::KB * fc;  // the neighbour, from the row
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const bool ok = ((unsigned)(ci[k] + fu - pad) < (unsigned)a.gh) & ((unsigned)(cj[k] + fv - pad) < (unsigned)a.gw) &
                       ((unsigned)(cl[k] + fz - pad_d) < (unsigned)gd);
-      const uint16_t *p = ok ? base[k] + shift : reinterpret_cast<const uint16_t *>(kZeroUnit);
+      const T *p = ok ? base[k] + shift : reinterpret_cast<const T *>(kZeroUnit);
       mfma::load_unit_to_lds(p, dst + (16 * wave + 8 * k) * 128);
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k)
-      mfma::load_unit_to_lds(wp + (int64_t)8 * k * a.K, dst + kConvRows * 128 + (32 * wave + 8 * k) * 128);
+      mfma::load_unit_to_lds(wp + (int64_t)8 * k * a.K, dst + Q::kRows * 128 + (32 * wave + 8 * k) * 128);
     if (kb + 1 < nkb) {
-      wp += 64;
+      wp += Q::KB;
       if (++fc == cblocks) {
         fc = 0;
         if (++fz == ksd) {
@@ -667,11 +678,11 @@ __global__ __launch_bounds__(512) void conv_gemm_kernel(GemmArgs a) {
       }
     }
   };
-  f32x16 acc[2][2];  // [output tile][row tile]
+  f32x16 acc[2][RT];  // [output tile][row tile]
 #pragma unroll
   for (int u = 0; u < 2; ++u)
 #pragma unroll
-    for (int v = 0; v < 2; ++v)
+    for (int v = 0; v < RT; ++v)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[u][v][r] = 0.f;
   u32x4 *pk = static_cast<u32x4 *>(a.out_pack[z]);
@@ -684,27 +695,35 @@ __global__ __launch_bounds__(512) void conv_gemm_kernel(GemmArgs a) {
       asm volatile("s_waitcnt vmcnt(6)" ::: "memory");  // this wave's share of the step; the next one stays in flight
       __syncthreads();
       fetch(kb + 2);  // into the stage multiplied one step ago, which every wave is past
-      const u32x4 *xs = ring + (kb % kConvStages) * (kConvStageBytes / 16) + wr * 8 + row_off;
-      const u32x4 *ws = ring + (kb % kConvStages) * (kConvStageBytes / 16) + (kConvRows + wc) * 8 + row_off;
+      const u32x4 *xs = ring + (kb % kConvStages) * (Q::kStageBytes / 16) + wr * 8 + row_off;
+      const u32x4 *ws = ring + (kb % kConvStages) * (Q::kStageBytes / 16) + (Q::kRows + wc) * 8 + row_off;
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
         const int at = (2 * ks + g) ^ swz;
-        const u32x4 w0 = ws[at], w1 = ws[32 * 8 + at], x0 = xs[at], x1 = xs[32 * 8 + at];
-        acc[0][0] = turned ? mfma::mma(w0, x0, acc[0][0]) : mfma::mma(x0, w0, acc[0][0]);
-        acc[0][1] = turned ? mfma::mma(w0, x1, acc[0][1]) : mfma::mma(x1, w0, acc[0][1]);
-        acc[1][0] = turned ? mfma::mma(w1, x0, acc[1][0]) : mfma::mma(x0, w1, acc[1][0]);
-        acc[1][1] = turned ? mfma::mma(w1, x1, acc[1][1]) : mfma::mma(x1, w1, acc[1][1]);
+        const u32x4 w[2] = {ws[at], ws[32 * 8 + at]};
+        u32x4 x[RT];
+#pragma unroll
+        for (int v = 0; v < RT; ++v) x[v] = xs[32 * 8 * v + at];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int v = 0; v < RT; ++v)
+            acc[u][v] = turned ? mma_unit(in, w[u], x[v], acc[u][v]) : mma_unit(in, x[v], w[u], acc[u][v]);
       }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be landing in LDS when the workgroup ends
   };
-  if (pk) multiply(std::false_type{});
-  else multiply(std::true_type{});
+  if constexpr (sizeof(T) == 2) {
+    if (pk) multiply(std::false_type{});
+    else multiply(std::true_type{});
+  } else {
+    multiply(std::true_type{});
+  }
 
-  uint16_t *out = static_cast<uint16_t *>(a.out[z]);
+  T *out = static_cast<T *>(a.out[z]);
   const float *bias = a.bias[z];
 #pragma unroll
-  for (int v = 0; v < 2; ++v) {
+  for (int v = 0; v < RT; ++v) {
     const unsigned tile = (unsigned)((m0 + wr) / 32) + v;
     int64_t first;
     int count;
@@ -718,7 +737,14 @@ __global__ __launch_bounds__(512) void conv_gemm_kernel(GemmArgs a) {
 #pragma unroll
           for (int r = 0; r < 16; ++r) c[r] += bias[oc + mfma::rowmap(r, g)];
         }
-        mfma::store_tile_natural(c, out + (first + (i < count ? i : 0)) * a.O + oc, g, i < count);
+        T *row = out + (first + (i < count ? i : 0)) * a.O + oc;
+        if constexpr (sizeof(T) == 2) {
+          mfma::store_tile_natural(c, reinterpret_cast<uint16_t *>(row), g, i < count);
+        } else if (i < count) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<float4 *>(row + 8 * q + 4 * g) = float4{c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]};
+        }
         continue;
       }
       const float bv = bias ? bias[oc + i] : 0.f;
@@ -727,7 +753,7 @@ __global__ __launch_bounds__(512) void conv_gemm_kernel(GemmArgs a) {
       if (out) {
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          if (mfma::rowmap(r, g) < count) out[(first + mfma::rowmap(r, g)) * a.O + oc + i] = mfma::to_bf16_bits(c[r]);
+          if (mfma::rowmap(r, g) < count) store_from_f32(out + (first + mfma::rowmap(r, g)) * a.O + oc + i, c[r]);
       }
       if (tpb && (int64_t)tile * 32 < a.M / a.N * tpb * 32) {
         pk[(((int64_t)tile * a.pack_heads + oc / 32) * 2 + 0) * 64 + lane] = mfma::pack_half<0>(c);
@@ -737,20 +763,24 @@ __global__ __launch_bounds__(512) void conv_gemm_kernel(GemmArgs a) {
   }
 }
 
-// whole steps of one tap (64 channels), whole workgroups of outputs; weights in the reduction's order
+// whole steps of one tap, whole workgroups of outputs; weights in the reduction's order
+template <typename T>
 static bool conv_serves(const GemmArgs &a, int nsets) {
-  if (a.ks <= 0 || a.act != 0 || !a.w_tap_major || a.C % 64 != 0 || a.O % kConvOut != 0 || a.K < 128) return false;
+  using Q = ConvTile<T>;
+  if (a.ks <= 0 || a.act != 0 || !a.w_tap_major || a.C % Q::KB != 0 || a.O % Q::kOut != 0 || a.K < 2 * Q::KB) return false;
   for (int z = 0; z < nsets; ++z)
-    if (!a.out_pack[z] && !aligned16(a.out[z])) return false;
+    if (a.out_pack[z] ? sizeof(T) != 2 : !aligned16(a.out[z])) return false;
   return true;
 }
 
+template <typename T>
 static int conv_launch(const GemmArgs &a, int nsets, hipStream_t st) {
+  using Q = ConvTile<T>;
   const int64_t rows = a.pack_tpb > 0 ? (a.M / a.N) * a.pack_tpb * 32 : a.M;
-  const size_t lds = (size_t)kConvStages * kConvStageBytes;
-  if (int rc = allow_dynamic_lds(conv_gemm_kernel, lds)) return rc;
-  const dim3 grid((unsigned)((rows + kConvRows - 1) / kConvRows), (unsigned)(a.O / kConvOut), (unsigned)nsets);
-  hipLaunchKernelGGL(conv_gemm_kernel, grid, dim3(512), lds, st, a);
+  const size_t lds = (size_t)kConvStages * Q::kStageBytes;
+  if (int rc = allow_dynamic_lds(conv_gemm_kernel<T>, lds)) return rc;
+  const dim3 grid((unsigned)((rows + Q::kRows - 1) / Q::kRows), (unsigned)(a.O / Q::kOut), (unsigned)nsets);
+  hipLaunchKernelGGL(conv_gemm_kernel<T>, grid, dim3(Q::kWaves * 64), lds, st, a);
   return launch_status();
 }
 
@@ -791,7 +821,8 @@ int launch(const GemmArgs &a, int nsets, int dtype, hipStream_t st) {
       cus = 256;
     return linear_launch(a, nsets, cus, st);
   }
-  if (dtype == PA_BF16 && conv_serves(a, nsets)) return conv_launch(a, nsets, st);
+  if (dtype == PA_BF16 && conv_serves<bf16>(a, nsets)) return conv_launch<bf16>(a, nsets, st);
+  if (dtype == PA_F32 && conv_serves<float>(a, nsets)) return conv_launch<float>(a, nsets, st);
   return dtype == PA_F32 ? launch_n<float>(a, nsets, st) : launch_n<bf16>(a, nsets, st);
 }
 

@@ -469,21 +469,23 @@ def test_layernorm_row_groups(dtype, rows, C):
 
 @pytest.mark.parametrize("grid,C,O,B,k", [((3, 5), 64, 256, 2, 3), ((16, 17), 256, 256, 1, 3), ((9, 30), 128, 512, 3, 5),
                                           ((4, 5, 7), 64, 256, 2, 3), ((33, 40), 512, 256, 1, 3)])
-def test_bf16_convolution_as_implicit_gemm(grid, C, O, B, k):
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_convolution_as_implicit_gemm(grid, C, O, B, k, dtype):
     """The ring-buffered convolution at partial row blocks, one and several channel blocks per tap, 2-D and 3-D,
     against float64."""
-    announce("conv gemm", grid, C, O, B, k)
+    announce("conv gemm", grid, C, O, B, k, dtype)
     torch.manual_seed(C + O)
     N = int(np.prod(grid))
     dims = PF.LayerDims(B, N, C, O // 32, 32, 32, grid[0], grid[1], k, grid[2] if len(grid) == 3 else 0, 1)
-    x = torch.randn(B, N, C, device="cuda").bfloat16()
-    w = (torch.randn(O, C, *(k,) * len(grid), device="cuda") / (C * k ** len(grid)) ** 0.5).bfloat16()
+    x = torch.randn(B, N, C, device="cuda").to(dtype)
+    w = (torch.randn(O, C, *(k,) * len(grid), device="cuda") / (C * k ** len(grid)) ** 0.5).to(dtype)
     bias = torch.randn(O, device="cuda")
     got = PF.rows_gemm(x, w.movedim(1, -1).contiguous(), bias, dims, C, O)
     conv = torch.nn.functional.conv2d if len(grid) == 2 else torch.nn.functional.conv3d
     want = conv(x.double().transpose(1, 2).reshape(B, C, *grid).cpu(), w.double().cpu(), bias.double().cpu(), padding=k // 2)
-    # one bf16 rounding of the result: at most 2^-9 of each value, 2^-9 / sqrt(3) on the average
-    assert_rel_l2(got, want.reshape(B, O, N).transpose(1, 2).float(), "conv", tol=2e-3)
+    # one bf16 rounding of the result: at most 2^-9 of each value, 2^-9 / sqrt(3) on the average; float32: the sums' own
+    # rounding, 2^-24 sqrt(terms) at 4 608 terms
+    assert_rel_l2(got, want.reshape(B, O, N).transpose(1, 2), "conv", tol=2e-3 if dtype == torch.bfloat16 else 4e-6)
 
 
 @pytest.mark.parametrize("rows,F", [(1, 64), (255, 128), (257, 1024), (2000, 192), (70_001, 256)])
