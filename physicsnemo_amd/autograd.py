@@ -93,7 +93,7 @@ def _slice_weight_grad(d_z: torch.Tensor, x_mid: torch.Tensor, H: int, S: int, D
     a, b = d_z.reshape(-1, H * S), x_mid.reshape(-1, H * D)
     if H > 1 and H * S <= 512 and PF.cols_gemm_supported(a, b):  # wider: the extra passes over x_mid cost more
         p, sums = PF.cols_gemm(a, b, col_sums=True)
-        dw = sum(p[h * S:(h + 1) * S, h * D:(h + 1) * D] for h in range(H))
+        dw = p.view(H, S, H, D).diagonal(dim1=0, dim2=2).sum(-1)
         return dw, sums.reshape(H, S).sum(0)
     return _wgrad(d_z.reshape(-1, S), x_mid.reshape(-1, D))
 

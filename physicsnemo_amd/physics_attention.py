@@ -109,11 +109,20 @@ class PhysicsAttentionBase(nn.Module):
         if hit == stamp:
             return self._kernel_param_cache["params"]
         with torch.no_grad():
-            params = {
-                name: _kernel_layout(p.detach()).to(device=device, dtype=dtype if big else torch.float32)
-                .contiguous().reshape(-1).clone()
-                for name, p, big in named
-            }
+            params = {}
+            for name, p, big in named:
+                if big:
+                    w = _kernel_layout(p.detach()).to(device=device, dtype=dtype).contiguous().reshape(-1)
+                    params[name] = w.clone() if w.data_ptr() == p.data_ptr() else w
+            # the small ones are copied together, each to a 16-byte boundary
+            small = [(name, p.detach().to(device=device, dtype=torch.float32).reshape(-1)) for name, p, big in named if not big]
+            gaps = [-v.numel() % 4 for _, v in small]
+            pad = torch.zeros(3, dtype=torch.float32, device=device) if any(gaps) else None
+            flat = torch.cat([part for (_, v), gap in zip(small, gaps) for part in ((v, pad[:gap]) if gap else (v,))])
+            at = 0
+            for (name, v), gap in zip(small, gaps):
+                params[name] = flat[at:at + v.numel()]
+                at += v.numel() + gap
             if fp8:
                 for name, p, big in named:
                     if big:
