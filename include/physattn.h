@@ -484,14 +484,15 @@ int pa_output_backward(const pa_shape *shape, const void *w_pack, const void *dy
  * leaves in `saved` (PA_TRAIN_SAVED bytes) what the backward reads; the parameters are not read again except the small
  * float32 ones.  grads (PA_TRAIN_GRADS bytes, float32): d in_project_x.weight, d in_project_fx.weight (not with plus),
  * their biases in the same order, d out_linear.weight, d out_linear.bias, d qkv_project.weight (96, 32), then grads of
- * pa_point_backward.  dx (B, N, C) bf16 or NULL.  Replaces autograd over PA.py:501-558. */
+ * pa_point_backward.  dx (B, N, C) bf16 or NULL.  tail (NULL, or C <= 256): the block's residual and LayerNorm on y, as in
+ * pa_layer_forward; the backward call takes the gradient of y.  Replaces autograd over PA.py:501-558. */
 #define PA_TRAIN_SAVED 0    /* kept from the forward to the backward call */
 #define PA_TRAIN_FORWARD 1  /* workspace of the forward call */
 #define PA_TRAIN_BACKWARD 2 /* workspace of the backward call */
 #define PA_TRAIN_GRADS 3
 int64_t pa_layer_train_bytes(const pa_shape *shape, int plus, int which);
 int pa_layer_train_forward(const pa_shape *shape, int weight_dtype, const pa_params *p, const pa_plus_params *plus,
-                           const void *x, const void *uniform, void *y, void *saved, void *workspace,
+                           const void *x, const void *uniform, void *y, const pa_block_tail *tail, void *saved, void *workspace,
                            int64_t workspace_bytes, void *stream);
 int pa_layer_train_backward(const pa_shape *shape, const pa_params *p, const pa_plus_params *plus, const void *x,
                             const void *uniform, const void *dy, const void *saved, void *dx, float *grads, void *workspace,

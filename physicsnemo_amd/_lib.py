@@ -271,7 +271,7 @@ def load() -> ctypes.CDLL:
     lib.pa_layer_train_bytes.restype = c_int64
     lib.pa_layer_train_bytes.argtypes = [ps, c_int, c_int]
     lib.pa_layer_train_forward.restype = c_int
-    lib.pa_layer_train_forward.argtypes = [ps, c_int, pp, pplus] + [c_void_p] * 5 + [c_int64, c_void_p]
+    lib.pa_layer_train_forward.argtypes = [ps, c_int, pp, pplus] + [c_void_p] * 3 + [pt] + [c_void_p] * 2 + [c_int64, c_void_p]
     lib.pa_layer_train_backward.restype = c_int
     lib.pa_layer_train_backward.argtypes = [ps, pp, pplus] + [c_void_p] * 7 + [c_int64, c_void_p]
     lib.pa_cols_gemm_chunks.restype = c_int64

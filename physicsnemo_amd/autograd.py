@@ -185,10 +185,15 @@ _PLUS_PARAMS = ("in_project_x_weight", "in_project_x_bias", "in_project_slice_we
 _LARGE = ("in_project_x_weight", "in_project_fx_weight", "out_linear_weight")
 
 
+def _train_params(names, params):
+    """The parameters as `layer_train_forward` takes them."""
+    large = torch.bfloat16 if all(p.dtype == torch.bfloat16 for n, p in zip(names, params) if n in _LARGE) else torch.float32
+    return {n: p.detach().to(large if n in _LARGE else torch.float32).contiguous() for n, p in zip(names, params)}
+
+
 def _layer_train_forward(ctx, x, uniform, dims, names, params):
     """Forward of a bf16 layer with 32-wide heads in one library call; ctx keeps what the backward call reads."""
-    large = torch.bfloat16 if all(p.dtype == torch.bfloat16 for n, p in zip(names, params) if n in _LARGE) else torch.float32
-    kp = {n: p.detach().to(large if n in _LARGE else torch.float32).contiguous() for n, p in zip(names, params)}
+    kp = _train_params(names, params)
     y, saved = PF.layer_train_forward(x, uniform, kp, dims)
     ctx.save_for_backward(x, uniform, saved, *params)
     ctx.dims, ctx.names, ctx.kparams = dims, names, kp
@@ -215,6 +220,41 @@ class PhysicsAttentionMfmaFunction(torch.autograd.Function):
     def backward(ctx, dy):
         dx, grads = _layer_train_backward(ctx, dy, 3)
         return (dx, None, None) + grads
+
+
+def _through_norm(y, w32, eps, d_y, d_normed, param_dtypes):
+    """(gradient of y, d weight, d bias) for the outputs y and LayerNorm(y)."""
+    if d_normed is None:
+        return (None if d_y is None else _aligned(d_y.to(y.dtype))), None, None
+    add = None if d_y is None else _aligned(d_y.to(y.dtype))
+    d, dg, db = PF.layernorm_backward(y, _aligned(d_normed.to(y.dtype)), w32, eps, add)
+    return d, dg.to(param_dtypes[0]), db.to(param_dtypes[1])
+
+
+class LayerResidualNormFunction(torch.autograd.Function):
+    """(y, LayerNorm(y)) for y = layer(x) + residual: `PhysicsAttentionMfmaFunction` with the block's residual and
+    following LayerNorm in the forward's last kernel, and the residual's gradient in the LayerNorm's backward kernel."""
+
+    @staticmethod
+    def forward(ctx, x, residual, dims, ln_w, ln_b, eps, *params):
+        ctx.set_materialize_grads(False)
+        kp = _train_params(_LAYER_PARAMS, params)
+        w32 = ln_w.detach().float().contiguous()
+        y, saved, normed = PF.layer_train_forward(x, None, kp, dims, residual, w32, ln_b.detach().float().contiguous(), eps)
+        ctx.save_for_backward(x, saved, y, w32, *params)
+        ctx.dims, ctx.kparams, ctx.eps, ctx.ln_dtypes = dims, kp, eps, (ln_w.dtype, ln_b.dtype)
+        return y, normed
+
+    @staticmethod
+    def backward(ctx, d_y, d_normed):
+        x, saved, y, w32, *params = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        d, dg, db = _through_norm(y, w32, ctx.eps, d_y, d_normed, ctx.ln_dtypes)
+        if d is None:
+            return (None,) * (6 + len(params))
+        dx, grads = PF.layer_train_backward(x, None, d, saved, ctx.kparams, ctx.dims, need[0])
+        return (dx, d if need[1] else None, None, dg, db, None) + tuple(
+            grads[n].view(p.shape).to(p.dtype) if wanted else None for n, p, wanted in zip(_LAYER_PARAMS, params, need[6:]))
 
 
 class PhysicsAttentionPlusMfmaFunction(torch.autograd.Function):
@@ -641,22 +681,37 @@ def mlp(x: torch.Tensor, layers: torch.nn.Sequential) -> torch.Tensor:
 
 
 class MlpResidualFunction(torch.autograd.Function):
-    """residual + Linear(gelu(Linear(x))) of a bf16 block in one kernel that keeps the hidden layer on chip; the backward
-    forms the hidden layer again from x, so nothing of it is kept between the passes (2 x 2 F bytes per row)."""
+    """(y, LayerNorm(y)) for y = residual + Linear(gelu(Linear(x))) of a bf16 block, in one kernel that keeps the hidden
+    layer on chip (ln_w None: y alone); the backward forms the hidden layer again from x, so nothing of it is kept between
+    the passes (2 x 2 F bytes per row)."""
 
     @staticmethod
-    def forward(ctx, x, residual, w1, b1, w2, b2):
+    def forward(ctx, x, residual, w1, b1, w2, b2, ln_w, ln_b, eps):
+        ctx.set_materialize_grads(False)
         w1_16, w2_16 = (w.detach().to(torch.bfloat16).contiguous() for w in (w1, w2))
         b1_32, b2_32 = (b.detach().float().contiguous() for b in (b1, b2))
-        ctx.save_for_backward(x, w1_16, b1_32, w2_16)
         ctx.param_dtypes = tuple(p.dtype for p in (w1, b1, w2, b2))
-        return PF.mlp_forward_packed(x, PF.mlp_pack(w1_16, w2_16), b1_32, b2_32, residual=residual)
+        packed = PF.mlp_pack(w1_16, w2_16)
+        if ln_w is None:
+            ctx.save_for_backward(x, w1_16, b1_32, w2_16)
+            return PF.mlp_forward_packed(x, packed, b1_32, b2_32, residual=residual)
+        w32 = ln_w.detach().float().contiguous()
+        y, normed = PF.mlp_forward_packed(x, packed, b1_32, b2_32, residual=residual, ln_weight=w32,
+                                          ln_bias=ln_b.detach().float().contiguous(), ln_eps=eps)
+        ctx.save_for_backward(x, w1_16, b1_32, w2_16, y, w32)
+        ctx.eps, ctx.ln_dtypes = eps, (ln_w.dtype, ln_b.dtype)
+        return y, normed
 
     @staticmethod
-    def backward(ctx, dy):
-        x, w1, b1, w2 = ctx.saved_tensors
+    def backward(ctx, dy, d_normed=None):
+        x, w1, b1, w2, *norm = ctx.saved_tensors
         need = ctx.needs_input_grad
-        dy16 = _aligned(dy)
+        d_ln = (None, None)
+        if norm:
+            dy, *d_ln = _through_norm(norm[0], norm[1], ctx.eps, dy, d_normed, ctx.ln_dtypes)
+        if dy is None:
+            return (None,) * 9
+        dy16 = _aligned(dy.to(x.dtype))
         if torch.is_grad_enabled():  # create_graph: the same formulas as tensor ops, which can be differentiated again
             h = torch.nn.functional.linear(x, w1, b1.to(x.dtype))
             act, dh = torch.nn.functional.gelu(h), torch.ops.aten.gelu_backward(dy16 @ w2, h)
@@ -666,22 +721,31 @@ class MlpResidualFunction(torch.autograd.Function):
         d_w1, d_b1 = _wgrad(_rows(dh), _rows(x)) if need[2] or need[3] else (None, None)
         d_w2, d_b2 = _wgrad(_rows(dy16), _rows(act)) if need[4] or need[5] else (None, None)
         grads = (g.to(t) if n else None for g, t, n in zip((d_w1, d_b1, d_w2, d_b2), ctx.param_dtypes, need[2:]))
-        return (dx, dy if need[1] else None, *grads)
+        return (dx, dy if need[1] else None, *grads, *d_ln, None)
 
 
-def norm_mlp_residual(x: torch.Tensor, ln: torch.nn.LayerNorm, layers: torch.nn.Sequential) -> torch.Tensor:
-    """x + Mlp(LayerNorm(x)) in training, as autocast would run it: on the fused MLP kernels where they serve the rows,
-    else on `layer_norm` and `mlp`."""
+def mlp_residual(normed: torch.Tensor, x: torch.Tensor, layers: torch.nn.Sequential, next_ln: torch.nn.LayerNorm | None = None):
+    """(x + Mlp(normed), next_ln of it or None) in training, as autocast would run it: on the fused MLP kernels where they
+    serve the rows (with the LayerNorm that follows in their tail), else on `mlp`."""
     lin1, act, lin2 = layers[0], layers[1], layers[2]
-    normed, x = layer_norm_residual(x, ln)
     C = x.shape[-1]
     if (len(layers) == 3 and compute_dtype(normed) == normed.dtype == x.dtype == torch.bfloat16 and
             isinstance(act, torch.nn.GELU) and act.approximate == "none" and lin1.bias is not None and
             lin2.bias is not None and lin1.in_features == lin2.out_features == C and
             PF.mlp_backward_supported(x.dtype, x.numel() // C, C, lin1.out_features)):
+        norm = (None, None, 0.0)
+        if next_ln is not None and _layer_norm_served(x, next_ln) and tuple(next_ln.normalized_shape) == (C,):
+            norm = (next_ln.weight, next_ln.bias, next_ln.eps)
         with torch.autocast("cuda", enabled=False):
-            return MlpResidualFunction.apply(_aligned(normed), _aligned(x), lin1.weight, lin1.bias, lin2.weight, lin2.bias)
-    return mlp(normed, layers) + x
+            out = MlpResidualFunction.apply(_aligned(normed), _aligned(x), lin1.weight, lin1.bias, lin2.weight, lin2.bias, *norm)
+        return out if norm[0] is not None else (out, None)
+    return mlp(normed, layers) + x, None
+
+
+def norm_mlp_residual(x: torch.Tensor, ln: torch.nn.LayerNorm, layers: torch.nn.Sequential) -> torch.Tensor:
+    """x + Mlp(LayerNorm(x)) in training, as autocast would run it."""
+    normed, x = layer_norm_residual(x, ln)
+    return mlp_residual(normed, x, layers)[0]
 
 
 def layer_norm_linear(x: torch.Tensor, ln: torch.nn.LayerNorm, lin: torch.nn.Linear) -> torch.Tensor:
@@ -690,8 +754,13 @@ def layer_norm_linear(x: torch.Tensor, ln: torch.nn.LayerNorm, lin: torch.nn.Lin
     dtype = compute_dtype(x)
     if dtype is None or x.dtype != dtype:
         return lin(ln(x))
+    return linear_as_autocast(layer_norm(x, ln), lin)
+
+
+def linear_as_autocast(x: torch.Tensor, lin: torch.nn.Linear) -> torch.Tensor:
+    """lin(x) in training on `linear`, for an x that is in the type autocast would run the Linear in."""
     with torch.autocast("cuda", enabled=False):
-        return linear(layer_norm(x, ln), lin.weight, lin.bias)
+        return linear(x, lin.weight, lin.bias)
 
 
 class LayerNormFunction(torch.autograd.Function):

@@ -922,7 +922,7 @@ static int check_train_params(const pa_params *p, const pa_plus_params *plus) {
 }
 
 int pa_layer_train_forward(const pa_shape *shape, int weight_dtype, const pa_params *p, const pa_plus_params *plus,
-                           const void *x, const void *uniform, void *y, void *saved, void *workspace,
+                           const void *x, const void *uniform, void *y, const pa_block_tail *tail, void *saved, void *workspace,
                            int64_t workspace_bytes, void *stream) {
   Range entry("pa_layer_train_forward");
   int rc = check_layer_train(shape, plus ? 1 : 0);
@@ -931,8 +931,10 @@ int pa_layer_train_forward(const pa_shape *shape, int weight_dtype, const pa_par
   if ((rc = check_train_params(p, plus))) return rc;
   if (!x || (plus && !uniform) || !y || !saved || !workspace) return PA_ERR_NULL;
   if (!aligned16(x) || !aligned16(uniform) || !aligned16(y) || !aligned16(saved) || !aligned16(workspace)) return PA_ERR_ALIGN;
+  if ((rc = check_tail(tail))) return rc;
+  if (tail_active(tail) && shape->C > 256) return PA_ERR_UNSUPPORTED;  // the tail rides on kernel (d)
   if (workspace_bytes < pa::train::forward_workspace_bytes(*shape, plus != nullptr, compute_units())) return PA_ERR_WORKSPACE;
-  return pa::train::forward(*shape, weight_dtype, *p, plus, x, uniform, y, saved, workspace, compute_units(),
+  return pa::train::forward(*shape, weight_dtype, *p, plus, x, uniform, y, tail_active(tail) ? tail : nullptr, saved, workspace, compute_units(),
                             static_cast<hipStream_t>(stream));
 }
 

@@ -170,7 +170,7 @@ static pa_params prepared(const pa_shape &s, const pa_params &p, bool plus, char
 }
 
 int forward(const pa_shape &s, int weight_dtype, const pa_params &params, const pa_plus_params *plus, const void *x,
-            const void *uniform, void *y, void *saved, void *workspace, int num_cu, hipStream_t st) {
+            const void *uniform, void *y, const pa_block_tail *tail, void *saved, void *workspace, int num_cu, hipStream_t st) {
   const bool pl = plus != nullptr;
   const Saved sp = plan_saved(s, pl);
   const Scratch sc = plan_scratch(s, pl, num_cu);
@@ -221,7 +221,7 @@ int forward(const pa_shape &s, int weight_dtype, const pa_params &params, const 
     if (s.C <= 256 && (rc = mfma::pack_out_linear(s, p.out_linear_weight, nullptr, p.out_linear_bias, blob, st))) return rc;
   }
   if ((rc = mfma::combine_attention(s, p, fx_bias, partials, G, tok, norm, tok_out, tokp, st))) return rc;
-  if (s.C <= 256) return mfma::deslice_project(s, blob, w_pack, tokp, y, nullptr, num_cu, st);
+  if (s.C <= 256) return mfma::deslice_project(s, blob, w_pack, tokp, y, tail, num_cu, st);
   if ((rc = mfma::deslice_natural(s, w_pack, tokp, ws + sc.out_x, num_cu, st))) return rc;
   return general::out_linear(PA_BF16, s, p, ws + sc.out_x, y, st);
 }

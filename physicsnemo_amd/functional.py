@@ -671,10 +671,10 @@ def layer_train_supported(dtype: torch.dtype, dims: LayerDims, plus: bool = Fals
     return _lib.load().pa_layer_train_bytes(byref(dims.c()), 1 if plus else 0, _lib.PA_TRAIN_SAVED) > 0
 
 
-def layer_train_forward(x, uniform, params: dict, dims: LayerDims):
-    """(y, saved) of a bf16 layer.  `params`: the layer's own parameters under the names of `pa_params` /
+def layer_train_forward(x, uniform, params: dict, dims: LayerDims, residual=None, ln_weight=None, ln_bias=None, ln_eps=1e-5):
+    """(y, saved) of a bf16 layer, with ln_weight (y + residual, saved, LayerNorm(y + residual)).  `params`: the layer's own parameters under the names of `pa_params` /
     `pa_plus_params`, the three large weights all float32 or all bfloat16 in torch's layout, the rest float32."""
-    _need_cuda(x, uniform)
+    _need_cuda(x, uniform, residual)
     lib, shape, plus = _lib.load(), dims.c(), uniform is not None
     nbytes = lib.pa_layer_train_bytes(byref(shape), int(plus), _lib.PA_TRAIN_FORWARD)
     if nbytes < 0:
@@ -682,11 +682,13 @@ def layer_train_forward(x, uniform, params: dict, dims: LayerDims):
     saved = torch.empty(lib.pa_layer_train_bytes(byref(shape), int(plus), _lib.PA_TRAIN_SAVED), dtype=torch.uint8, device=x.device)
     workspace = torch.empty(int(nbytes), dtype=torch.uint8, device=x.device)
     y = torch.empty(dims.B, dims.N, dims.C, dtype=x.dtype, device=x.device)
+    ln_out = torch.empty_like(y) if ln_weight is not None else None
+    tail = _c_tail(residual, ln_weight, ln_bias, ln_eps, ln_out)
     _lib.check(lib.pa_layer_train_forward(
         byref(shape), _lib.dtype_code(params["out_linear_weight"].dtype), byref(_c_params(params)),
-        _c_plus(params) if plus else None, x.data_ptr(), _lib.ptr(uniform), y.data_ptr(), saved.data_ptr(),
+        _c_plus(params) if plus else None, x.data_ptr(), _lib.ptr(uniform), y.data_ptr(), byref(tail), saved.data_ptr(),
         workspace.data_ptr(), int(nbytes), _lib.current_stream_ptr(x.device)), "pa_layer_train_forward")
-    return y, saved
+    return (y, saved) if ln_out is None else (y, saved, ln_out)
 
 
 def layer_train_backward(x, uniform, dy, saved, params: dict, dims: LayerDims, need_dx: bool = True):

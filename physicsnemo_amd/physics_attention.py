@@ -19,8 +19,8 @@ import torch
 import torch.nn as nn
 
 from . import functional as PF
-from .autograd import (PhysicsAttentionFunction, PhysicsAttentionMfmaFunction, PhysicsAttentionPlusFunction,
-                       PhysicsAttentionPlusMfmaFunction)
+from .autograd import (LayerResidualNormFunction, PhysicsAttentionFunction, PhysicsAttentionMfmaFunction,
+                       PhysicsAttentionPlusFunction, PhysicsAttentionPlusMfmaFunction, _aligned)
 
 __all__ = ["PhysicsAttentionBase", "PhysicsAttentionIrregularMesh", "PhysicsAttentionStructuredMesh2D",
            "PhysicsAttentionStructuredMesh3D"]
@@ -285,6 +285,25 @@ class PhysicsAttentionBase(nn.Module):
             x, self.kernel_params(x.dtype, x.device), self.layer_dims(x), residual=residual,
             ln_weight=ln.weight.detach().float().contiguous(), ln_bias=ln.bias.detach().float().contiguous(),
             ln_eps=ln.eps)
+
+    def forward_block_with_grad(self, x: torch.Tensor, residual: torch.Tensor, ln: nn.LayerNorm):
+        """Training: (self(x) + residual, its LayerNorm) with the add and the LayerNorm in the layer's last kernel, or None
+        where that does not serve the call (other types and widths, Transolver++, dropout, hooks on this module)."""
+        hooks = (self._forward_hooks, self._forward_pre_hooks, self._backward_hooks, self._backward_pre_hooks)
+        if (type(self).forward is not PhysicsAttentionBase.forward or any(hooks) or self.plus or self.fp8_weights or
+                (self.training and self.out_dropout.p > 0) or not x.is_cuda or x.ndim != 3 or x.numel() == 0 or
+                not x.dtype == residual.dtype == torch.bfloat16 or self._wants_fp16(x) or x.shape != residual.shape or
+                not (ln.elementwise_affine and ln.bias is not None and tuple(ln.normalized_shape) == (self.dim,))):
+            return None
+        self._validate(x)
+        x = self._prepare_input(x)
+        dims = self.layer_dims(x)
+        if dims.C > 256 or not PF.layer_train_supported(x.dtype, dims):
+            return None
+        return LayerResidualNormFunction.apply(
+            _aligned(x), _aligned(residual), dims, ln.weight, ln.bias, ln.eps, self.in_project_x.weight, self.in_project_x.bias,
+            self.in_project_fx.weight, self.in_project_fx.bias, self.in_project_slice.weight, self.in_project_slice.bias,
+            self.temperature, self.qkv_project.weight, self.out_linear.weight, self.out_linear.bias)
 
     def forward_stages(self, x: torch.Tensor) -> dict:
         """Stage-by-stage forward through the natural-layout entry points; returns every intermediate."""

@@ -21,7 +21,7 @@ import torch.nn as nn
 from . import autograd as PA
 from . import checkpoint as _ckpt
 from . import functional as PF
-from .physics_attention import (PhysicsAttentionIrregularMesh, PhysicsAttentionStructuredMesh2D,
+from .physics_attention import (PhysicsAttentionBase, PhysicsAttentionIrregularMesh, PhysicsAttentionStructuredMesh2D,
                                 PhysicsAttentionStructuredMesh3D)
 
 __all__ = ["Mlp", "TransolverBlock", "Transolver"]
@@ -218,8 +218,14 @@ class TransolverBlock(nn.Module):
         if self._needs_grad(fx):
             # training: the layer's autograd path, LayerNorms / MLP as differentiable tensor ops (reference :300-303)
             x_in, fx = (normed_in, fx) if normed_in is not None else PA.layer_norm_residual(fx, self.ln_1)
-            fx1 = self.Attn(x_in) + fx
-            return PA.norm_mlp_residual(fx1, self.ln_mlp1[0], self.ln_mlp1[1].layers), None
+            pair = None
+            if isinstance(self.Attn, PhysicsAttentionBase):
+                pair = self.Attn.forward_block_with_grad(x_in, fx, self.ln_mlp1[0])
+            if pair is None:
+                normed, fx1 = PA.layer_norm_residual(self.Attn(x_in) + fx, self.ln_mlp1[0])
+            else:
+                fx1, normed = pair
+            return PA.mlp_residual(normed, fx1, self.ln_mlp1[1].layers, next_ln)
         x_in = normed_in if normed_in is not None else self.ln_1(fx)
         whole = self._whole_block(x_in, fx, next_ln)
         if whole is not None:
@@ -527,6 +533,8 @@ class Transolver(nn.Module):
                 fx, normed = block.forward_chain(fx, normed, block.ln_mlp2[0])
                 if normed is not None and on_library:
                     fx = self._library_linear(normed, block.ln_mlp2[1])  # output head (:305-307)
+                elif normed is not None and PA.compute_dtype(fx) == normed.dtype:
+                    fx = PA.linear_as_autocast(normed, block.ln_mlp2[1])
                 else:
                     fx = block.ln_mlp2[1](normed) if normed is not None else PA.layer_norm_linear(fx, *block.ln_mlp2)
             else:

@@ -526,6 +526,42 @@ def test_mlp_residual_block(rows, F):
     assert_rel_l2(gx.detach(), x64.grad, "dx, create_graph", tol=1e-2)
 
 
+@pytest.mark.parametrize("C,S,B,N,grid", [(256, 64, 2, 1001, None), (128, 16, 1, 33, None), (256, 32, 1, 12 * 9, (12, 9))])
+def test_bf16_blocks_with_fused_tails_train_like_separate_ones(C, S, B, N, grid):
+    """A chain of two bf16 blocks and its head: residuals and LayerNorms in the layer's and the MLP's kernels are no
+    further from the float32 model than the same blocks with a hook on their layers, which makes the layer a call of its own."""
+    announce("fused training tails", C, S, B, N, grid)
+    torch.manual_seed(N)
+    kw = dict(functional_dim=3, embedding_dim=2, out_dim=3, n_layers=2, n_hidden=C, n_head=C // 32, mlp_ratio=2, slice_num=S,
+              structured_shape=grid, use_te=False)
+    model = pn.Transolver(**kw).cuda().train()
+    x, e = torch.randn(B, N, 3, device="cuda"), torch.rand(B, N, 2, device="cuda")
+    dy = torch.randn(B, N, 3, device="cuda")
+
+    def step(amp=True):
+        model.zero_grad(set_to_none=True)
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=amp):
+            out = model(x, e)
+        (out.float() * dy).sum().backward()
+        return out.detach().float(), {n: p.grad.clone() for n, p in model.named_parameters()}
+
+    out, got = step()
+    seen = []
+    handles = [b.Attn.register_forward_hook(lambda *a: seen.append(1)) for b in model.blocks]
+    apart_out, apart = step()
+    for h in handles:
+        h.remove()
+    assert len(seen) == 2
+    want_out, want = step(amp=False)
+    # both are bf16 chains of the same length; the fused one rounds no more often, so its error differs by chance only:
+    # over the thousands of elements of each of these vectors by a few per cent (a gradient of four elements alone, the
+    # temperature's at 33 points, can be off by any factor)
+    flat = lambda grads: torch.cat([grads[n].reshape(-1) for n in want]).cpu()
+    for got_v, apart_v, want_v in ((out, apart_out, want_out), (flat(got), flat(apart), flat(want))):
+        e_got, e_apart = to.rel_l2(got_v.cpu(), want_v.cpu()), to.rel_l2(apart_v.cpu(), want_v.cpu())
+        assert e_got <= 1.3 * e_apart, (e_got, e_apart)
+
+
 def test_output_dropout_in_training_matches_the_reference_site():
     """The reference applies nn.Dropout to the layer output in training mode (physics_attention.py:499): kept entries
     are y / (1 - p), the rest zero, gradients flow through the kept entries only; eval mode is the identity."""
