@@ -208,26 +208,38 @@ class GeoTransolver(nn.Module):
                              f"with shape {tuple(global_embedding.shape)}")
         embedding_states, local_bq, _ = self.context_builder.build_context(streams, local_positions, geometry,
                                                                            global_embedding)
-        x = [self.preprocess[i](t) for i, t in enumerate(streams)]
+        # without a gradient the first block's LayerNorm comes with the preprocess launch, and each block hands the next one
+        # LayerNorm_1 of its outputs (and the last one the output head its LayerNorm)
+        grad = torch.is_grad_enabled() and (any(t.requires_grad for t in streams) or
+                                            any(p.requires_grad for p in self.parameters()))
+        first_ln = None if grad or self.include_local_features or len(self.blocks) == 0 else self.blocks[0].ln_1
+        pairs = [m.forward_with_norm(t, first_ln) if first_ln is not None and type(m) is Mlp and
+                 not (m._forward_hooks or m._forward_pre_hooks) else (m(t), None) for m, t in zip(self.preprocess, streams)]
+        x, normed = [y for y, _ in pairs], [n for _, n in pairs]
         if self.include_local_features and local_bq is not None:
             x = [torch.cat([x[i], local_bq[i].to(x[i].dtype)], dim=-1) for i in range(len(x))]
         needs_grad = torch.is_grad_enabled() and (any(t.requires_grad for t in x)
                                                   or any(p.requires_grad for p in self.parameters()))
         chain = not needs_grad and all(t.is_cuda for t in x) and all(hasattr(b.Attn, "gale_params") for b in self.blocks)
         if chain:
-            # inference: each block hands the next one LayerNorm_1 of its outputs (computed in its MLP kernel's tail)
             if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16:
                 x = [t.to(torch.bfloat16) for t in x]
-            normed = None
+            if any(n is None or n.dtype != t.dtype for n, t in zip(normed, x)):
+                normed = None
             for k, block in enumerate(self.blocks):
-                next_ln = self.blocks[k + 1].ln_1 if k + 1 < len(self.blocks) else None
+                # the streams share a block's LayerNorm but have output heads of their own
+                head_ln = self.ln_mlp_out[0][0] if len(x) == 1 else None
+                next_ln = self.blocks[k + 1].ln_1 if k + 1 < len(self.blocks) else head_ln
                 x, normed = block.forward_chain(tuple(x), normed, embedding_states, next_ln)
         else:
+            normed = None
             for block in self.blocks:
                 x = block(tuple(x), embedding_states)
         point_features = list(x)
         # per-stream head: LayerNorm on the library kernel (forward and backward), then the output Linear
-        x = [self.ln_mlp_out[i][1](PA.layer_norm(t, self.ln_mlp_out[i][0])) for i, t in enumerate(x)]
+        if not (len(x) == 1 and normed is not None and len(self.blocks) > 0):
+            normed = [PA.layer_norm(t, self.ln_mlp_out[i][0]) for i, t in enumerate(x)]
+        x = [self.ln_mlp_out[i][1](n) for i, n in enumerate(normed)]
         if self.structured_shape is not None and unflatten_output:
             x = [t.reshape(t.shape[0], *self.structured_shape, -1) for t in x]
         out = x[0] if single_input else tuple(x)

@@ -69,6 +69,10 @@ class Mlp(nn.Module):
         return cache["params"]
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        return self.forward_with_norm(x, None)[0]
+
+    def forward_with_norm(self, x: torch.Tensor, ln: nn.LayerNorm | None):
+        """(self(x), ln(self(x))), the second element None where the LayerNorm does not ride on the library launch."""
         lin1, lin2 = self.layers[0], self.layers[2]
         act = self.layers[1]
         needs_grad = torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in self.parameters()))
@@ -81,8 +85,12 @@ class Mlp(nn.Module):
             if (dtype in (torch.float32, torch.bfloat16) and
                     PF.preprocess_supported(dtype, rows, lin1.in_features, lin1.out_features, lin2.out_features)):
                 w1, b1, w2, b2 = self._kernel_params(dtype, x.device)
-                return PF.preprocess_forward(x.to(dtype).contiguous(), w1, b1, w2, b2)
-        return PA.mlp(x, self.layers) if needs_grad and len(self.layers) == 3 else self.layers(x)
+                x = x.to(dtype).contiguous()
+                if ln is not None and ln.elementwise_affine and ln.bias is not None:
+                    return PF.preprocess_forward(x, w1, b1, w2, b2, ln_weight=ln.weight.detach().float().contiguous(),
+                                                 ln_bias=ln.bias.detach().float().contiguous(), ln_eps=ln.eps)
+                return PF.preprocess_forward(x, w1, b1, w2, b2), None
+        return (PA.mlp(x, self.layers) if needs_grad and len(self.layers) == 3 else self.layers(x)), None
 
 
 class PositionalEmbedding(nn.Module):
