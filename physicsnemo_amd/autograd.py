@@ -636,18 +636,22 @@ class LinearFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias):
         w16 = weight.to(x.dtype)
-        ctx.save_for_backward(x, w16)
+        ctx.save_for_backward(x, weight, w16)
         ctx.param_dtypes = (weight.dtype, bias.dtype if bias is not None else None)
         return torch.nn.functional.linear(x, w16, bias.to(x.dtype) if bias is not None else None)
 
     @staticmethod
     def backward(ctx, dy):
-        x, w16 = ctx.saved_tensors
+        x, weight, w16 = ctx.saved_tensors
         dy = dy.contiguous()
-        dx = (dy @ w16) if ctx.needs_input_grad[0] else None
+        again = torch.is_grad_enabled()  # create_graph: tensor ops on the inputs themselves, to be differentiated again
+        dx = (dy @ (weight.to(x.dtype) if again else w16)) if ctx.needs_input_grad[0] else None
         dw = db = None
         if ctx.needs_input_grad[1] or ctx.needs_input_grad[2]:
-            dw, db = _wgrad(_rows(dy), _rows(x))
+            if again:
+                dw, db = _rows(dy).float().t() @ _rows(x).float(), _rows(dy).sum(0, dtype=torch.float32)
+            else:
+                dw, db = _wgrad(_rows(dy), _rows(x))
             dw = dw.to(ctx.param_dtypes[0])
             db = db.to(ctx.param_dtypes[1]) if ctx.param_dtypes[1] is not None else None
         return dx, dw, db
@@ -662,18 +666,32 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> 
 
 def compute_dtype(x: torch.Tensor) -> torch.dtype | None:
     """The type a Linear of x runs in on the library's training path: bfloat16 under bf16 autocast, x's own float32 or
-    bfloat16 without autocast, None where the modules run as they are."""
-    if not x.is_cuda:
+    bfloat16 without autocast, None where the modules run as they are (also under torch.func transforms and forward-mode
+    differentiation, which the library's functions do not take part in)."""
+    if not x.is_cuda or torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0:
         return None
     if torch.is_autocast_enabled("cuda"):
         return torch.bfloat16 if torch.get_autocast_dtype("cuda") == torch.bfloat16 else None
     return x.dtype if x.dtype in (torch.bfloat16, torch.float32) else None
 
 
+def unhooked(*modules: torch.nn.Module) -> bool:
+    """True where calling the modules is their arithmetic and nothing more.  Hooks observe or change a module's values, and
+    `torch.nn.utils`' weight and spectral normalisation and pruning form the weight in one."""
+    return not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks for m in modules)
+
+
+def _linears_served(dtype: torch.dtype | None, *lins: torch.nn.Module) -> bool:
+    """True where `linear` does what calling the modules does in `dtype`; without autocast a Linear refuses an input whose
+    type is not its weight's."""
+    return dtype is not None and all(type(m) is torch.nn.Linear and unhooked(m) and
+                                     (torch.is_autocast_enabled("cuda") or m.weight.dtype == dtype) for m in lins)
+
+
 def mlp(x: torch.Tensor, layers: torch.nn.Sequential) -> torch.Tensor:
     """Linear -> activation -> Linear in training, as autocast would run it, on `linear`."""
     dtype = compute_dtype(x)
-    if dtype is None:
+    if len(layers) != 3 or not unhooked(layers) or not _linears_served(dtype, layers[0], layers[2]):
         return layers(x)
     with torch.autocast("cuda", enabled=False):
         h = linear(x.to(dtype), layers[0].weight, layers[0].bias)
@@ -727,10 +745,10 @@ class MlpResidualFunction(torch.autograd.Function):
 def mlp_residual(normed: torch.Tensor, x: torch.Tensor, layers: torch.nn.Sequential, next_ln: torch.nn.LayerNorm | None = None):
     """(x + Mlp(normed), next_ln of it or None) in training, as autocast would run it: on the fused MLP kernels where they
     serve the rows (with the LayerNorm that follows in their tail), else on `mlp`."""
-    lin1, act, lin2 = layers[0], layers[1], layers[2]
-    C = x.shape[-1]
-    if (len(layers) == 3 and compute_dtype(normed) == normed.dtype == x.dtype == torch.bfloat16 and
-            isinstance(act, torch.nn.GELU) and act.approximate == "none" and lin1.bias is not None and
+    C, dtype = x.shape[-1], compute_dtype(normed)
+    lin1, act, lin2 = layers if len(layers) == 3 else (None,) * 3
+    if (dtype == normed.dtype == x.dtype == torch.bfloat16 and unhooked(layers) and _linears_served(dtype, lin1, lin2) and
+            type(act) is torch.nn.GELU and unhooked(act) and act.approximate == "none" and lin1.bias is not None and
             lin2.bias is not None and lin1.in_features == lin2.out_features == C and
             PF.mlp_backward_supported(x.dtype, x.numel() // C, C, lin1.out_features)):
         norm = (None, None, 0.0)
@@ -752,13 +770,15 @@ def layer_norm_linear(x: torch.Tensor, ln: torch.nn.LayerNorm, lin: torch.nn.Lin
     """lin(ln(x)) in training (the output head), as autocast would run it: LayerNorm statistics in float32, its result
     rounded to the Linear's type."""
     dtype = compute_dtype(x)
-    if dtype is None or x.dtype != dtype:
+    if x.dtype != dtype or not unhooked(ln) or not _linears_served(dtype, lin):
         return lin(ln(x))
     return linear_as_autocast(layer_norm(x, ln), lin)
 
 
 def linear_as_autocast(x: torch.Tensor, lin: torch.nn.Linear) -> torch.Tensor:
-    """lin(x) in training on `linear`, for an x that is in the type autocast would run the Linear in."""
+    """lin(x) in training on `linear` where it serves the module, for an x in the type autocast would run it in."""
+    if not _linears_served(compute_dtype(x), lin):
+        return lin(x)
     with torch.autocast("cuda", enabled=False):
         return linear(x, lin.weight, lin.bias)
 

@@ -285,14 +285,14 @@ class GALEBlock(nn.Module):
     _mlp_residual = TransolverBlock._mlp_residual
 
     def _one(self, fx: torch.Tensor, attn: torch.Tensor, needs_grad: bool) -> torch.Tensor:
-        fx1 = attn + fx
-        if needs_grad:
-            return PA.norm_mlp_residual(fx1, self.ln_mlp1[0], self.ln_mlp1[1].layers)
+        fx1, mlp = attn + fx, self.ln_mlp1[1]
+        if needs_grad and type(mlp) is Mlp and PA.unhooked(mlp):
+            return PA.norm_mlp_residual(fx1, self.ln_mlp1[0], mlp.layers)
         normed = PA.layer_norm(fx1, self.ln_mlp1[0])
-        if self._mlp_kernel_serves(normed):
+        if not needs_grad and self._mlp_kernel_serves(normed):
             packed, b1, b2 = self._mlp_kernel_packed(normed.device, normed.dtype)
             return PF.mlp_forward_packed(normed, packed, b1, b2, residual=fx1.to(normed.dtype).contiguous())
-        return PA.mlp(normed, self.ln_mlp1[1].layers) + fx1
+        return mlp(normed) + fx1
 
     def forward_chain(self, fx: tuple, normed_in, global_context: torch.Tensor | None, next_ln: nn.LayerNorm | None):
         """Inference, one block inside a chain: takes LayerNorm_1 of every stream if the previous block produced it and

@@ -90,7 +90,7 @@ class Mlp(nn.Module):
                     return PF.preprocess_forward(x, w1, b1, w2, b2, ln_weight=ln.weight.detach().float().contiguous(),
                                                  ln_bias=ln.bias.detach().float().contiguous(), ln_eps=ln.eps)
                 return PF.preprocess_forward(x, w1, b1, w2, b2), None
-        return (PA.mlp(x, self.layers) if needs_grad and len(self.layers) == 3 else self.layers(x)), None
+        return (PA.mlp(x, self.layers) if needs_grad else self.layers(x)), None
 
 
 class PositionalEmbedding(nn.Module):
@@ -233,7 +233,10 @@ class TransolverBlock(nn.Module):
                 normed, fx1 = PA.layer_norm_residual(self.Attn(x_in) + fx, self.ln_mlp1[0])
             else:
                 fx1, normed = pair
-            return PA.mlp_residual(normed, fx1, self.ln_mlp1[1].layers, next_ln)
+            mlp = self.ln_mlp1[1]
+            if type(mlp) is not Mlp or not PA.unhooked(mlp):
+                return mlp(normed) + fx1, None
+            return PA.mlp_residual(normed, fx1, mlp.layers, next_ln)
         x_in = normed_in if normed_in is not None else self.ln_1(fx)
         whole = self._whole_block(x_in, fx, next_ln)
         if whole is not None:
@@ -538,13 +541,16 @@ class Transolver(nn.Module):
                         fx = whole[1]
                         continue
                     normed = x_in
-                fx, normed = block.forward_chain(fx, normed, block.ln_mlp2[0])
+                head = PA.unhooked(block.ln_mlp2, block.ln_mlp2[0]) or not block._needs_grad(fx)
+                fx, normed = block.forward_chain(fx, normed, block.ln_mlp2[0] if head else None)
                 if normed is not None and on_library:
                     fx = self._library_linear(normed, block.ln_mlp2[1])  # output head (:305-307)
                 elif normed is not None and PA.compute_dtype(fx) == normed.dtype:
                     fx = PA.linear_as_autocast(normed, block.ln_mlp2[1])
+                elif normed is not None:
+                    fx = block.ln_mlp2[1](normed)
                 else:
-                    fx = block.ln_mlp2[1](normed) if normed is not None else PA.layer_norm_linear(fx, *block.ln_mlp2)
+                    fx = PA.layer_norm_linear(fx, *block.ln_mlp2) if head else block.ln_mlp2(fx)
             else:
                 fx, normed = block.forward_chain(fx, normed, self.blocks[k + 1].ln_1)
         if unflatten_output:

@@ -1,6 +1,8 @@
 """Backward pass of the HIP layer against autograd over the fp32 oracle (the oracle's own gradient is pinned by
 finite differences in test_oracle_closed_forms.py).  Bars: fp32 gradients rtol 1e-4 with atol = 1e-4 * max|ref|
 per tensor; bf16 gradients rel-L2 <= 3e-2 against the fp32 reference gradients."""
+import copy
+
 import numpy as np
 import pytest
 import torch
@@ -9,6 +11,7 @@ from oracle import torch_oracle as to
 import physicsnemo_amd as pn
 from physicsnemo_amd import autograd as PA
 from physicsnemo_amd import functional as PF
+from physicsnemo_amd.transolver import Mlp
 from gpu_util import announce, assert_fp32_close, assert_rel_l2, make_pair
 
 pytestmark = pytest.mark.gpu
@@ -584,3 +587,67 @@ def test_output_dropout_in_training_matches_the_reference_site():
     blk = pn.TransolverBlock(2, 64, 0.25, mlp_ratio=2, slice_num=16, use_te=False).cuda().train()
     out = blk(x)
     assert out.shape == x.shape and torch.isfinite(out).all()
+
+
+def test_modules_with_hooks_are_called_in_training():
+    """Hooks on a block's MLP, its Linears and the output head run in a float32 training step (weight and spectral
+    normalisation form the weight in one), and the gradients are those of the step without hooks."""
+    announce("hooks in float32 training")
+    torch.manual_seed(0)
+    model = pn.Transolver(functional_dim=3, embedding_dim=2, out_dim=3, n_layers=2, n_hidden=64, n_head=4, mlp_ratio=2,
+                          slice_num=32, use_te=False).cuda().train()
+    x, e, dy = (torch.randn(2, 300, n, device="cuda") for n in (3, 2, 3))
+
+    def step():
+        model.zero_grad(set_to_none=True)
+        (model(x, e) * dy).sum().backward()
+        return {n: p.grad.clone() for n, p in model.named_parameters()}
+
+    want = step()
+    block, mlp = model.blocks[1], model.blocks[1].ln_mlp1[1]
+    hooked = [block.ln_mlp2, *block.ln_mlp2, mlp, mlp.layers, *mlp.layers, model.preprocess.layers[0]]
+    for m in hooked:
+        seen = []
+        handle = m.register_forward_hook(lambda *a: seen.append(1))
+        got = step()
+        handle.remove()
+        assert len(seen) == 1, m
+        for n in want:  # the same products in float32, in another order
+            assert_rel_l2(got[n], want[n].cpu(), n, tol=1e-4)
+    torch.nn.utils.parametrizations.weight_norm(mlp.layers[0])
+    want_w = mlp.layers[0].weight.detach().clone()
+    with torch.no_grad():
+        mlp.layers[0].parametrizations.weight.original0.mul_(2.0)
+    seen = []
+    handle = mlp.layers[0].register_forward_hook(lambda m, i, o: seen.append((i[0].detach(), o.detach(), m.bias.detach())))
+    step()
+    handle.remove()
+    inp, out, bias = seen[0]
+    assert_rel_l2(out, (inp @ (2.0 * want_w).t() + bias).cpu(), "normalised weight", tol=1e-5)
+
+
+def test_mlp_module_differentiates_twice_and_forward():
+    """An Mlp by itself, float32: gradients of gradients, forward mode, torch.func, and the refusal of another type."""
+    announce("second derivatives of the Mlp")
+    torch.manual_seed(0)
+    net = Mlp(4, 64, 8).cuda()
+    ref = copy.deepcopy(net).cpu().double()
+    x = torch.randn(5000, 4, device="cuda")
+
+    def second(m, x):
+        x = x.detach().requires_grad_(True)
+        (gx,) = torch.autograd.grad(m(x).square().sum(), x, create_graph=True)
+        return torch.autograd.grad(gx.square().sum(), [x, *m.parameters()])
+
+    for got, want in zip(second(net, x), second(ref, x.cpu().double())):
+        # float32 sums over 5 000 rows: 5000^0.5 * 2^-24 = 4e-6 of the terms, which cancel by up to ten
+        assert_rel_l2(got, want.float(), "second derivative", tol=4e-5)
+    t = torch.randn_like(x)
+    _, jvp = torch.func.jvp(net, (x,), (t,))
+    _, want = torch.func.jvp(ref, (x.cpu().double(),), (t.cpu().double(),))
+    assert_rel_l2(jvp.detach(), want.detach().float(), "jvp", tol=1e-5)
+    got = torch.func.vmap(torch.func.grad(lambda v: net(v).sum()))(x[:8])
+    want = torch.func.vmap(torch.func.grad(lambda v: ref(v).sum()))(x[:8].cpu().double())
+    assert_rel_l2(got, want.float(), "vmap of grad", tol=1e-5)
+    with pytest.raises(RuntimeError):
+        net(x.bfloat16())
