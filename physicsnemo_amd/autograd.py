@@ -186,14 +186,16 @@ _LARGE = ("in_project_x_weight", "in_project_fx_weight", "out_linear_weight")
 
 
 def _train_params(names, params):
-    """The parameters as `layer_train_forward` takes them."""
+    """The parameters as `layer_train_forward` takes them, each on a 16-byte boundary (a view into one flat vector of all
+    parameters need not start on one)."""
     large = torch.bfloat16 if all(p.dtype == torch.bfloat16 for n, p in zip(names, params) if n in _LARGE) else torch.float32
-    return {n: p.detach().to(large if n in _LARGE else torch.float32).contiguous() for n, p in zip(names, params)}
+    return {n: _aligned(p.detach().to(large if n in _LARGE else torch.float32)) for n, p in zip(names, params)}
 
 
 def _layer_train_forward(ctx, x, uniform, dims, names, params):
     """Forward of a bf16 layer with 32-wide heads in one library call; ctx keeps what the backward call reads."""
-    kp = _train_params(names, params)
+    x, kp = _aligned(x), _train_params(names, params)
+    uniform = None if uniform is None else _aligned(uniform)
     y, saved = PF.layer_train_forward(x, uniform, kp, dims)
     ctx.save_for_backward(x, uniform, saved, *params)
     ctx.dims, ctx.names, ctx.kparams = dims, names, kp
@@ -202,7 +204,7 @@ def _layer_train_forward(ctx, x, uniform, dims, names, params):
 
 def _layer_train_backward(ctx, dy, first_param):
     x, uniform, saved, *params = ctx.saved_tensors
-    dx, grads = PF.layer_train_backward(x, uniform, dy.to(x.dtype).contiguous(), saved, ctx.kparams, ctx.dims,
+    dx, grads = PF.layer_train_backward(x, uniform, _aligned(dy.to(x.dtype)), saved, ctx.kparams, ctx.dims,
                                         ctx.needs_input_grad[0])
     return dx, tuple(grads[n].view(p.shape).to(p.dtype) if need else None
                      for n, p, need in zip(ctx.names, params, ctx.needs_input_grad[first_param:]))
@@ -239,8 +241,8 @@ class LayerResidualNormFunction(torch.autograd.Function):
     def forward(ctx, x, residual, dims, ln_w, ln_b, eps, *params):
         ctx.set_materialize_grads(False)
         kp = _train_params(_LAYER_PARAMS, params)
-        w32 = ln_w.detach().float().contiguous()
-        y, saved, normed = PF.layer_train_forward(x, None, kp, dims, residual, w32, ln_b.detach().float().contiguous(), eps)
+        w32 = _aligned(ln_w.detach().float())
+        y, saved, normed = PF.layer_train_forward(x, None, kp, dims, residual, w32, _aligned(ln_b.detach().float()), eps)
         ctx.save_for_backward(x, saved, y, w32, *params)
         ctx.dims, ctx.kparams, ctx.eps, ctx.ln_dtypes = dims, kp, eps, (ln_w.dtype, ln_b.dtype)
         return y, normed
@@ -706,16 +708,16 @@ class MlpResidualFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, residual, w1, b1, w2, b2, ln_w, ln_b, eps):
         ctx.set_materialize_grads(False)
-        w1_16, w2_16 = (w.detach().to(torch.bfloat16).contiguous() for w in (w1, w2))
-        b1_32, b2_32 = (b.detach().float().contiguous() for b in (b1, b2))
+        w1_16, w2_16 = (_aligned(w.detach().to(torch.bfloat16)) for w in (w1, w2))
+        b1_32, b2_32 = (_aligned(b.detach().float()) for b in (b1, b2))
         ctx.param_dtypes = tuple(p.dtype for p in (w1, b1, w2, b2))
         packed = PF.mlp_pack(w1_16, w2_16)
         if ln_w is None:
             ctx.save_for_backward(x, w1_16, b1_32, w2_16)
             return PF.mlp_forward_packed(x, packed, b1_32, b2_32, residual=residual)
-        w32 = ln_w.detach().float().contiguous()
+        w32 = _aligned(ln_w.detach().float())
         y, normed = PF.mlp_forward_packed(x, packed, b1_32, b2_32, residual=residual, ln_weight=w32,
-                                          ln_bias=ln_b.detach().float().contiguous(), ln_eps=eps)
+                                          ln_bias=_aligned(ln_b.detach().float()), ln_eps=eps)
         ctx.save_for_backward(x, w1_16, b1_32, w2_16, y, w32)
         ctx.eps, ctx.ln_dtypes = eps, (ln_w.dtype, ln_b.dtype)
         return y, normed

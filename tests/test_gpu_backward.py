@@ -651,3 +651,31 @@ def test_mlp_module_differentiates_twice_and_forward():
     assert_rel_l2(got, want.float(), "vmap of grad", tol=1e-5)
     with pytest.raises(RuntimeError):
         net(x.bfloat16())
+
+
+@pytest.mark.parametrize("plus", [False, True])
+def test_bf16_training_takes_parameters_and_gradients_off_16_byte_boundaries(plus):
+    """Parameters that are views into one flat vector, an input and an output gradient that start one element into their
+    storage: bit for bit the results of the aligned call."""
+    announce("misaligned parameters", plus)
+    torch.manual_seed(0)
+    layer = pn.PhysicsAttentionIrregularMesh(128, heads=4, dim_head=32, slice_num=32, use_te=False, plus=plus).cuda().train()
+    x, dy = torch.randn(2, 2, 131, 128, device="cuda").bfloat16()
+    noise = torch.rand(2, 131, 4, 32, device="cuda").bfloat16()
+
+    def off(t):
+        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+        flat[1:] = t.detach().reshape(-1)
+        return flat[1:].view(t.shape)
+
+    def step(move):
+        xi = move(x).detach().requires_grad_(True)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = layer.forward_with_noise(xi, move(noise)) if plus else layer(xi)
+        return [y.detach()] + list(torch.autograd.grad(y, [xi, *layer.parameters()], move(dy), allow_unused=True))
+
+    want = step(lambda t: t)
+    for p in layer.parameters():
+        p.data = off(p.data)
+    for a, b in zip(step(off), want):
+        assert (a is None) == (b is None) and (a is None or torch.equal(a, b))
