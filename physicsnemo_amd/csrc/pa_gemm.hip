@@ -206,44 +206,54 @@ __global__ __launch_bounds__(256) void rows_gemm_mfma_kernel(GemmArgs a) {
 // row's 32 channels leave as 16-byte stores; with packing on, the un-transposed tile (lanes <-> channels) is formed
 // as well and written in the packed operand layout of the slice kernels.
 // Rows are numbered as in rows_gemm_mfma_kernel (padded per batch when pack_tpb > 0).
+// Bound by memory latency: a workgroup has one tile (16 KB at K = 256) on its way.  LEAN (K = 256, 256 columns per
+// workgroup, natural output only) fits 128 registers, so two workgroups share a CU and one's loads cover the other's:
+// 256 -> 2 x 256 at 1 048 576 rows 441 -> 394 us (4.1 TB/s), 256 -> 256 228 -> 212 us (5.1 TB/s).
 // ------------------------------------------------------------------------------------------------
-template <int KS>
-__global__ __launch_bounds__(512) void rows_linear_kernel(GemmArgs a) {
+template <int KS, bool LEAN>
+__global__ __launch_bounds__(512, LEAN ? 4 : 2) void rows_linear_kernel(GemmArgs a) {
   constexpr int K = 16 * KS, UPR = K / 8, ROWU = UPR + 1;
+  constexpr int PT = LEAN ? 32 * UPR / 512 : 4;  // 16-byte units a thread stages per tile, at most
   extern __shared__ u32x4 xs_all[];
   u32x4(*xs)[32 * ROWU] = reinterpret_cast<u32x4(*)[32 * ROWU]>(xs_all);  // two tile buffers
   const int z = blockIdx.z;
   const uint16_t *in = static_cast<const uint16_t *>(a.in);
   const uint16_t *W = static_cast<const uint16_t *>(a.w[z]);
   uint16_t *out = static_cast<uint16_t *>(a.out[z]);
-  u32x4 *pk = static_cast<u32x4 *>(a.out_pack[z]);
+  u32x4 *pk = LEAN ? nullptr : static_cast<u32x4 *>(a.out_pack[z]);
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int NT = blockDim.x;
+  const int NT = LEAN ? 512 : blockDim.x;
   const int o0 = blockIdx.y * 256 + wave * 32;  // this wave's output columns
 
   u32x4 wf[KS];  // W[o0 + i][16 ks + 8 g + j]: the A operand of out^T and the B operand of the un-transposed tile
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks)
     wf[ks] = *reinterpret_cast<const u32x4 *>(W + (int64_t)(o0 + i) * K + 16 * ks + 8 * g);
-  float bias_t[16];  // bias of channel rowmap(r, g) (out^T: registers <-> channels)
+  float bias_t[16];  // bias of channel rowmap(r, g) (out^T: registers <-> channels); LEAN reads it from LDS per tile
+  __shared__ float bias_s[LEAN ? 256 : 1];
+  if constexpr (LEAN) {
+    if (tid < 256) bias_s[tid] = a.bias[z] ? a.bias[z][blockIdx.y * 256 + tid] : 0.f;
+  } else {
 #pragma unroll
-  for (int r = 0; r < 16; ++r) bias_t[r] = a.bias[z] ? a.bias[z][o0 + mfma::rowmap(r, g)] : 0.f;
-  const float bias_n = a.bias[z] ? a.bias[z][o0 + i] : 0.f;
+    for (int r = 0; r < 16; ++r) bias_t[r] = a.bias[z] ? a.bias[z][o0 + mfma::rowmap(r, g)] : 0.f;
+  }
+  const float bias_n = !LEAN && a.bias[z] ? a.bias[z][o0 + i] : 0.f;
 
-  const int64_t padded = (int64_t)a.pack_tpb * 32;
-  const int64_t ntiles = a.pack_tpb > 0 ? (a.M / a.N) * a.pack_tpb : (a.M + 31) / 32;
+  const int tpb = LEAN ? 0 : a.pack_tpb;
+  const int64_t padded = (int64_t)tpb * 32;
+  const int64_t ntiles = tpb > 0 ? (a.M / a.N) * tpb : (a.M + 31) / 32;
   auto real_row = [&](int64_t vm) -> int64_t {
-    if (a.pack_tpb == 0) return vm < a.M ? vm : -1;
+    if (tpb == 0) return vm < a.M ? vm : -1;
     const int64_t b = vm / padded, n = vm - b * padded;
     return (n < a.N && b * a.N + n < a.M) ? b * a.N + n : -1;
   };
   // staging: unit idx = k * NT + tid of the tile -> row idx / UPR, position idx % UPR; 32 * UPR units per tile
   const int per_thread = (32 * UPR + NT - 1) / NT;
-  u32x4 stg[4];  // per_thread <= 4 for every supported (K, workgroup size) pair
+  u32x4 stg[PT];  // per_thread <= PT for every supported (K, workgroup size) pair
   auto stage_load = [&](int64_t tile) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < PT; ++k) {
       const int idx = k * NT + tid;
       stg[k] = u32x4{0, 0, 0, 0};
       if (k < per_thread && idx < 32 * UPR) {
@@ -255,7 +265,7 @@ __global__ __launch_bounds__(512) void rows_linear_kernel(GemmArgs a) {
   };
   auto stage_store = [&](int buf) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < PT; ++k) {
       const int idx = k * NT + tid;
       if (k < per_thread && idx < 32 * UPR) {
         const int rc = idx / UPR, pos = idx - rc * UPR;
@@ -278,7 +288,7 @@ __global__ __launch_bounds__(512) void rows_linear_kernel(GemmArgs a) {
     f32x16 acc_t, acc_n;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      acc_t[r] = bias_t[r];
+      acc_t[r] = LEAN ? bias_s[wave * 32 + mfma::rowmap(r, g)] : bias_t[r];
       acc_n[r] = bias_n;
     }
     if (pk) {
@@ -321,17 +331,25 @@ bool linear_serves(const GemmArgs &a, int nsets, size_t elem_bytes) {
 int linear_launch(const GemmArgs &a, int nsets, int num_cu, hipStream_t st) {
   const int64_t ntiles = a.pack_tpb > 0 ? (a.M / a.N) * a.pack_tpb : (a.M + 31) / 32;
   const int waves = (a.O < 256 ? a.O : 256) / 32;
-  // resident workgroups: the register-held weights leave room for one 8-wave workgroup per CU (two for K = 128)
-  int64_t gx = (a.K == 128 ? 2 : 1) * (int64_t)num_cu / (((a.O + 255) / 256) * nsets);
+  // resident workgroups: the register-held weights leave room for one 8-wave workgroup per CU, two for K = 128 and the
+  // lean form.  The second one of the lean form pays from eight tiles per CU on, where its weights (128 KB) are covered:
+  // 256 -> 256, two against one: 16 384 rows 12.0 / 9.1 us, 32 768 14.5 / 12.5; from 65 536 rows against one of the other
+  // form: 19.5 / 20.8, 1 048 576 rows 211 / 227.
+  const bool lean = a.K == 256 && a.O % 256 == 0 && a.pack_tpb == 0 && !a.out_pack[0] && !a.out_pack[nsets - 1];
+  const int64_t sides = (a.O + 255) / 256 * nsets;
+  int64_t gx = (a.K == 128 || (lean && ntiles * sides >= 8 * (int64_t)num_cu) ? 2 : 1) * (int64_t)num_cu / sides;
   if (gx < 1) gx = 1;
   if (gx > ntiles) gx = ntiles;
   const dim3 grid((unsigned)gx, (unsigned)((a.O + 255) / 256), (unsigned)nsets), block((unsigned)(waves * 64));
   const size_t lds = (size_t)2 * 32 * (a.K / 8 + 1) * 16;  // only K = 512 exceeds the default limit
-  if (int rc = allow_dynamic_lds(rows_linear_kernel<32>, a.K == 512 ? lds : 0)) return rc;
+  if (int rc = allow_dynamic_lds(rows_linear_kernel<32, false>, a.K == 512 ? lds : 0)) return rc;
   switch (a.K) {
-    case 128: hipLaunchKernelGGL((rows_linear_kernel<8>), grid, block, lds, st, a); break;
-    case 256: hipLaunchKernelGGL((rows_linear_kernel<16>), grid, block, lds, st, a); break;
-    case 512: hipLaunchKernelGGL((rows_linear_kernel<32>), grid, block, lds, st, a); break;
+    case 128: hipLaunchKernelGGL((rows_linear_kernel<8, false>), grid, block, lds, st, a); break;
+    case 256:
+      if (lean) hipLaunchKernelGGL((rows_linear_kernel<16, true>), grid, block, lds, st, a);
+      else hipLaunchKernelGGL((rows_linear_kernel<16, false>), grid, block, lds, st, a);
+      break;
+    case 512: hipLaunchKernelGGL((rows_linear_kernel<32, false>), grid, block, lds, st, a); break;
     default: return PA_ERR_UNSUPPORTED;
   }
   return launch_status();

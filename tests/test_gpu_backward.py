@@ -679,3 +679,17 @@ def test_bf16_training_takes_parameters_and_gradients_off_16_byte_boundaries(plu
         p.data = off(p.data)
     for a, b in zip(step(off), want):
         assert (a is None) == (b is None) and (a is None or torch.equal(a, b))
+
+
+@pytest.mark.parametrize("rows,c_out,bias", [(4096, 256, True), (4127, 256, False), (16387, 512, True), (33001, 256, True)])
+def test_row_gemm_of_256_inputs_with_two_workgroups_per_cu(rows, c_out, bias):
+    """The natural-output row GEMM at its smallest row count, ragged last tiles, fewer and more tiles than workgroups."""
+    announce("row GEMM, 256 inputs", rows, c_out, bias)
+    torch.manual_seed(rows)
+    x, w = torch.randn(1, rows, 256, device="cuda").bfloat16(), torch.randn(c_out, 256, device="cuda").bfloat16()
+    b = torch.randn(c_out, device="cuda") if bias else None
+    y = PF.rows_gemm(x, w, b, PF.LayerDims(1, rows, 256, 8, 32, 64), 256, c_out)
+    want = x[0].double().cpu() @ w.double().cpu().t() + (b.double().cpu() if bias else 0)
+    # float32 sums, rounded to bf16 once: at most half a unit in the last place (2^-9) of a value, sums far below it
+    err = (y[0].double().cpu() - want).abs()
+    assert (err <= 2.0 ** -8 * want.abs() + 1e-3).all()
