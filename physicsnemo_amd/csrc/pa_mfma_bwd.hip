@@ -55,8 +55,8 @@ __global__ __launch_bounds__(512) void deslice_natural_kernel(const u32x4 *__res
 //   per (b,h) tokA[(st*2 + kk)] = tok'[32st + i][16kk + 8g + j]                    A of d w, first half of k
 //            dnA[(st*2 + kk)]   = d num[32st + i][16kk + 8g + j]                   A of d w, second half of k
 //            dnT[cq]            = d num[16cq + rowmap(j, g)][i]                     A of d fx_mid
-// Slices >= S read as zero.  SPLIT tables carry the remainders t - bf16(t) in a second set of fragments behind each group, so that products with them keep 16 bits of the table: for the layer variants
-// (structured, Transolver++) whose backward multiplies with float32 tables elsewhere.
+// Slices >= S read as zero.  SPLIT tables carry the remainders t - bf16(t) in a second set of fragments behind each group,
+// so that products with them keep 16 bits of the table (point_split() says for which layers).
 // ------------------------------------------------------------------------------------------------
 struct BwdTablePlan {
   int st2, nch, group, nshared, nhead;  // fragments: of the two kinds, of a shared group, shared, per (b, h)
@@ -526,8 +526,10 @@ bool point_backward_supported(const pa_shape &s) {
 
 int64_t point_backward_grads(const pa_shape &s, bool plus) { return point_grads((int)s.S, (int)s.H, plus); }
 
-// The irregular layer multiplied with bf16 tables here before it had this kernel, the others with float32 ones
-static bool point_split(const pa_shape &s, bool plus) { return plus || s.conv_k > 0; }
+// Irregular layers of 128 and 256 channels multiply with bf16 tables, all others with float32 ones kept as bf16 and its
+// remainder: at 512 channels and 128 slices, 4 096 points, plain bf16 tables leave d b_slice 1.6e-2, d W_slice 1.0e-2 and
+// d W_x 6.9e-3 from float64, the split ones 2.7e-3, 2.2e-3 and 2.5e-3 (as fma loops on float32 tables do).
+static bool point_split(const pa_shape &s, bool plus) { return plus || s.conv_k > 0 || s.C == 512; }
 
 static int point_head_waves(const pa_shape &s, bool plus) {  // waves (heads) per workgroup
   const int most = point_waves((int)s.S, plus, point_split(s, plus));

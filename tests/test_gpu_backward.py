@@ -256,6 +256,50 @@ def test_bf16_training_kernels_over_variants(variant, C, S, B, N, grid):
             assert_rel_l2(got[name], want[name], f"grad {name}", tol=3e-2)
 
 
+@pytest.mark.parametrize("variant,C,S,B,N,grid", [
+    ("irregular", 512, 128, 1, 2048, None), ("irregular", 512, 32, 2, 1001, None), ("plus", 256, 64, 1, 4003, None),
+    ("plus", 128, 16, 2, 2001, None), ("structured2d", 256, 64, 1, 1200, (30, 40)), ("structured2d", 128, 32, 2, 660, (20, 33)),
+])
+def test_bf16_training_gradients_keep_float32_tables(variant, C, S, B, N, grid):
+    """Layers whose backward multiplies with float32 tables (slice weights, attended tokens, d num): every gradient, the
+    temperature's among them, against float64 at large weights that bf16 holds.  A chain has at most six independent
+    bf16 roundings of per-point values (x_mid, fx_mid, d out_x, d z, d x_mid, the result: 2^-9 / sqrt(3) = 1.1e-3 of a value
+    on the average each, 2.8e-3 together); 5e-3 leaves room for the cancellation in sums over the points, and gradients
+    of a few elements (temperature, last bias of proj_temperature) get 1e-2.  Tables rounded to bf16 put one and the same error into every point, which
+    the sums do not average: 0.7e-2 to 1.6e-2 at 512 channels."""
+    announce("float32 tables in bf16 training", variant, C, S, B, N, grid)
+    H = C // 32
+    plus = variant == "plus"
+    if plus:
+        torch.manual_seed(0)
+        ref = to.OraclePhysicsAttentionIrregularMesh(C, heads=H, dim_head=32, slice_num=S, plus=True)
+        hip = pn.PhysicsAttentionIrregularMesh(C, heads=H, dim_head=32, slice_num=S, use_te=False, plus=True).cuda()
+    else:
+        ref, hip = make_pair(variant, C, H, 32, S, spatial=grid)
+    with torch.no_grad():
+        for name, p in ref.named_parameters():
+            if name == "temperature":
+                p.copy_(0.6 + 0.8 * torch.rand_like(p))
+            elif name.split(".")[0] in ("in_project_x", "in_project_fx", "out_linear") and p.ndim > 1:
+                p.copy_(p.bfloat16().float())
+            elif name.endswith("bias"):
+                p.add_(0.1 * torch.randn_like(p))
+    hip.load_state_dict(ref.state_dict())
+    ref, hip = ref.double().train(), hip.train()
+    x, dy, u = torch.randn(B, N, C).bfloat16(), torch.randn(B, N, C).bfloat16(), torch.rand(B, N, H, S).bfloat16()
+    assert PF.layer_train_supported(torch.bfloat16, hip.layer_dims(x.cuda()), plus)
+
+    def run(m, x, dy, u):
+        x = x.clone().requires_grad_(True)
+        y = m.forward_with_noise(x, u) if plus else m(x)
+        y.backward(dy)
+        return {"y": y.detach(), "x": x.grad, **{n: p.grad for n, p in m.named_parameters()}}
+
+    want, got = run(ref, x.double(), dy.double(), u.double()), run(hip, x.cuda(), dy.cuda(), u.cuda())
+    for name in want:
+        assert_rel_l2(got[name], want[name], name, tol=1e-2 if want[name].numel() < 16 else 5e-3)
+
+
 def test_mfma_deslice_natural_layout():
     announce("MFMA deslice to natural layout")
     ref, hip = make_pair("irregular", 256, 8, 32, 64, sharpen=2.0)
