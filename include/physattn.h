@@ -527,6 +527,13 @@ int pa_mlp_forward(int dtype, int64_t rows, int64_t C, int64_t F, const pa_mlp_p
 int pa_mlp_pack(int dtype, int64_t C, int64_t F, const pa_mlp_params *p, void *packed, int64_t packed_bytes, void *stream);
 int pa_mlp_forward_packed(int dtype, int64_t rows, int64_t C, int64_t F, const void *packed, const float *b1,
                           const float *b2, const void *u, void *y, const pa_block_tail *tail, void *stream);
+/* The hidden layer's part of the MLP's backward pass, from the layer's input and the output's gradient alone:
+ *   act (rows, F) = gelu(w1 u + b1),  d_hidden (rows, F) = (w2^T dy) * gelu'(w1 u + b1);
+ * w1 (F, C), w2 (C, F), u, dy (rows, C) and the results bf16, 16-byte aligned; b1 float32; b2 is not read.  The weight
+ * gradients are dy^T act and d_hidden^T u, the input's d_hidden w1.  bf16, C = 256, F a multiple of 64 up to 8 192. */
+int64_t pa_mlp_backward_workspace_bytes(int dtype, int64_t rows, int64_t C, int64_t F);
+int pa_mlp_backward(int dtype, int64_t rows, int64_t C, int64_t F, const pa_mlp_params *p, const void *u, const void *dy,
+                    void *act, void *d_hidden, void *workspace, int64_t workspace_bytes, void *stream);
 /* pa_mlp_forward_packed for rows that still lack the LayerNorm in front of the Mlp: the kernel applies
  * LayerNorm(in_ln) to the rows of u as it turns them into operands, so `ln_mlp1[0]` of TransolverBlock (TR.py:303) costs
  * no pass over memory and its producer (the attention layer's tail) need not write a normalised copy.  With
@@ -534,14 +541,7 @@ int pa_mlp_forward_packed(int dtype, int64_t rows, int64_t C, int64_t F, const v
  * (pa_mlp_input_ln_query() == 1). */
 typedef struct pa_input_ln {
   const float *gamma; /* (C) */
-  const float *beta;  /* The hidden layer's part of the MLP's backward pass, from the layer's input and the output's gradient alone:
- *   act (rows, F) = gelu(w1 u + b1),  d_hidden (rows, F) = (w2^T dy) * gelu'(w1 u + b1);
- * w1 (F, C), w2 (C, F), u, dy (rows, C) and the results bf16, 16-byte aligned; b1 float32; b2 is not read.  The weight
- * gradients are dy^T act and d_hidden^T u, the input's d_hidden w1.  bf16, C = 256, F a multiple of 64 up to 8 192. */
-int64_t pa_mlp_backward_workspace_bytes(int dtype, int64_t rows, int64_t C, int64_t F);
-int pa_mlp_backward(int dtype, int64_t rows, int64_t C, int64_t F, const pa_mlp_params *p, const void *u, const void *dy,
-                    void *act, void *d_hidden, void *workspace, int64_t workspace_bytes, void *stream);
-/* (C) */
+  const float *beta;  /* (C) */
   float eps;
 } pa_input_ln;
 int pa_mlp_input_ln_query(int dtype, int64_t rows, int64_t C, int64_t F);

@@ -25,6 +25,18 @@ def test_library_loads_and_exports_every_declared_symbol():
     assert lib.pa_status_string(0) == b"ok"
 
 
+@pytest.mark.parametrize("compiler,ext", [(["gcc", "-std=c11", "-pedantic-errors"], "c"), (["g++", "-std=c++17"], "cpp")])
+def test_header_declares_every_symbol_to_c_and_cpp(tmp_path, compiler, ext):
+    """The public header is C; a unit that takes the address of every exported function finds a declaration of each."""
+    import subprocess
+    unit = tmp_path / f"unit.{ext}"
+    unit.write_text('#include "physattn.h"\ntypedef void (*fn)(void);\nfn all[] = {\n' +
+                    "".join(f"  (fn)&{name},\n" for name in sorted(_lib.EXPORTED)) + "};\n")
+    out = subprocess.run([*compiler, "-Wall", "-Werror", "-Wno-cast-function-type", "-fsyntax-only", "-I",
+                          os.path.join(ROOT, "include"), str(unit)], capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0, out.stderr
+
+
 def test_marker_ranges_follow_the_environment():
     """PA_ROCTX=1 turns the roctx ranges on (the marker library is opened at run time); without it they are off."""
     import subprocess
