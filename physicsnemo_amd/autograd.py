@@ -185,16 +185,17 @@ _PLUS_PARAMS = ("in_project_x_weight", "in_project_x_bias", "in_project_slice_we
 _LARGE = ("in_project_x_weight", "in_project_fx_weight", "out_linear_weight")
 
 
-def _train_params(names, params):
-    """The parameters as `layer_train_forward` takes them, each on a 16-byte boundary (a view into one flat vector of all
-    parameters need not start on one)."""
+def _train_params(names, params, device):
+    """The parameters as `layer_train_forward` takes them: on the input's device, each on a 16-byte boundary (a view into
+    one flat vector of all parameters need not start on one)."""
     large = torch.bfloat16 if all(p.dtype == torch.bfloat16 for n, p in zip(names, params) if n in _LARGE) else torch.float32
-    return {n: _aligned(p.detach().to(large if n in _LARGE else torch.float32)) for n, p in zip(names, params)}
+    return {n: _aligned(p.detach().to(device=device, dtype=large if n in _LARGE else torch.float32))
+            for n, p in zip(names, params)}
 
 
 def _layer_train_forward(ctx, x, uniform, dims, names, params):
     """Forward of a bf16 layer with 32-wide heads in one library call; ctx keeps what the backward call reads."""
-    x, kp = _aligned(x), _train_params(names, params)
+    x, kp = _aligned(x), _train_params(names, params, x.device)
     uniform = None if uniform is None else _aligned(uniform)
     y, saved = PF.layer_train_forward(x, uniform, kp, dims)
     ctx.save_for_backward(x, uniform, saved, *params)
@@ -240,7 +241,7 @@ class LayerResidualNormFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, residual, dims, ln_w, ln_b, eps, *params):
         ctx.set_materialize_grads(False)
-        kp = _train_params(_LAYER_PARAMS, params)
+        kp = _train_params(_LAYER_PARAMS, params, x.device)
         w32 = _aligned(ln_w.detach().float())
         y, saved, normed = PF.layer_train_forward(x, None, kp, dims, residual, w32, _aligned(ln_b.detach().float()), eps)
         ctx.save_for_backward(x, saved, y, w32, *params)

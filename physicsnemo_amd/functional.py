@@ -672,9 +672,12 @@ def layer_train_supported(dtype: torch.dtype, dims: LayerDims, plus: bool = Fals
 
 
 def layer_train_forward(x, uniform, params: dict, dims: LayerDims, residual=None, ln_weight=None, ln_bias=None, ln_eps=1e-5):
-    """(y, saved) of a bf16 layer, with ln_weight (y + residual, saved, LayerNorm(y + residual)).  `params`: the layer's own parameters under the names of `pa_params` /
-    `pa_plus_params`, the three large weights all float32 or all bfloat16 in torch's layout, the rest float32."""
-    _need_cuda(x, uniform, residual)
+    """(y, saved) of a bf16 layer, with ln_weight (y + residual, saved, LayerNorm(y + residual)).  `params`: the layer's own
+    parameters under the names of `pa_params` / `pa_plus_params`, the three large weights all float32 or all bfloat16 in
+    torch's layout, the rest float32."""
+    _need_cuda(x, uniform, residual, ln_weight, ln_bias, *params.values())
+    if uniform is not None and (uniform.dtype != x.dtype or uniform.shape != (dims.B, dims.N, dims.H, dims.S)):
+        raise ValueError("uniform samples must have the activation dtype and shape (B, N, H, S)")
     lib, shape, plus = _lib.load(), dims.c(), uniform is not None
     nbytes = lib.pa_layer_train_bytes(byref(shape), int(plus), _lib.PA_TRAIN_FORWARD)
     if nbytes < 0:
@@ -693,7 +696,7 @@ def layer_train_forward(x, uniform, params: dict, dims: LayerDims, residual=None
 
 def layer_train_backward(x, uniform, dy, saved, params: dict, dims: LayerDims, need_dx: bool = True):
     """(dx or None, gradients by parameter name, float32 views of one buffer) of `layer_train_forward`."""
-    _need_cuda(x, uniform, dy, saved)
+    _need_cuda(x, uniform, dy, saved, *params.values())
     lib, shape, plus = _lib.load(), dims.c(), uniform is not None
     nbytes = lib.pa_layer_train_bytes(byref(shape), int(plus), _lib.PA_TRAIN_BACKWARD)
     if nbytes < 0:

@@ -51,6 +51,17 @@ def test_marker_ranges_follow_the_environment():
         assert out.stdout.strip().splitlines()[-1] == expected, (value, out.stdout, out.stderr)
 
 
+def test_training_parameters_follow_the_input_to_its_device():
+    """A layer that was not moved to its input's device: no parameter reaches the kernels as a pointer of another one."""
+    from physicsnemo_amd import autograd as PA
+    for names in (PA._LAYER_PARAMS, PA._PLUS_PARAMS):
+        params = [torch.randn(2, 8) for _ in names]
+        moved = PA._train_params(names, params, torch.device("meta"))
+        assert list(moved) == list(names) and all(t.device.type == "meta" for t in moved.values())
+        with pytest.raises(RuntimeError, match="GPU tensors only"):  # what the entry point does with those of another device
+            PF._need_cuda(*PA._train_params(names, params, torch.device("cpu")).values())
+
+
 def _shape(**kw):
     base = dict(B=1, N=64, C=64, H=2, D=32, S=16, grid_h=0, grid_w=0, conv_k=0)
     base.update(kw)

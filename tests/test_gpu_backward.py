@@ -698,6 +698,24 @@ def test_mlp_module_differentiates_twice_and_forward():
 
 
 @pytest.mark.parametrize("plus", [False, True])
+def test_bf16_training_of_a_layer_left_on_the_host(plus):
+    """Parameters in host memory are copied to the input's device in the forward; their gradients cannot be delivered there
+    and the backward says so.  Uniform samples of another shape are refused."""
+    announce("layer left on the host", plus)
+    torch.manual_seed(0)
+    layer = pn.PhysicsAttentionIrregularMesh(128, heads=4, dim_head=32, slice_num=32, use_te=False, plus=plus).train()
+    x, noise = torch.randn(2, 131, 128, device="cuda").bfloat16(), torch.rand(2, 131, 4, 32, device="cuda").bfloat16()
+    run = lambda m: m.forward_with_noise(x, noise) if plus else m(x)
+    y = run(layer)
+    with pytest.raises(RuntimeError, match="device"):
+        y.backward(torch.ones_like(y))
+    assert torch.equal(run(copy.deepcopy(layer).cuda()), y)
+    if plus:
+        with pytest.raises(ValueError, match="uniform"):
+            layer.cuda().forward_with_noise(x, noise[:, :100])
+
+
+@pytest.mark.parametrize("plus", [False, True])
 def test_bf16_training_takes_parameters_and_gradients_off_16_byte_boundaries(plus):
     """Parameters that are views into one flat vector, an input and an output gradient that start one element into their
     storage: bit for bit the results of the aligned call."""
