@@ -942,7 +942,8 @@ __global__ __launch_bounds__(256) void layernorm_backward_rows_kernel(const T *_
           sq = fmaf(dlt, dlt, sq);
         }
       }
-    const float rstd = rsqrtf(group_sum<LPR>(sq) * inv_c + eps);
+    // rows beyond M hold zeros throughout; with eps = 0 their statistics alone would be infinite
+    const float rstd = m < M ? rsqrtf(group_sum<LPR>(sq) * inv_c + eps) : 0.f;
     float s1 = 0.f, s2 = 0.f;
 #pragma unroll
     for (int k = 0; k < UPL; ++k)

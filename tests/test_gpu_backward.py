@@ -514,6 +514,23 @@ def test_layernorm_row_groups(dtype, rows, C):
     assert_rel_l2(db, b64.grad, "d beta", tol=1e-5)
 
 
+@pytest.mark.parametrize("dtype,rows,C", [(torch.bfloat16, 1, 256), (torch.bfloat16, 2001, 256), (torch.float32, 7, 32),
+                                          (torch.float32, 1003, 64), (torch.bfloat16, 3, 40)])
+def test_layernorm_backward_without_eps(dtype, rows, C):
+    """eps = 0 with rows that do not fill the last wave: the rows that are not there add nothing to d gamma."""
+    announce("layernorm, eps 0", dtype, rows, C)
+    x, dy = (torch.randn(rows, C, device="cuda").to(dtype) for _ in range(2))
+    gam = torch.randn(C, device="cuda")
+    x64, g64 = x.double().requires_grad_(True), gam.double().requires_grad_(True)
+    b64 = torch.zeros_like(g64, requires_grad=True)
+    torch.nn.functional.layer_norm(x64, (C,), g64, b64, eps=0.0).backward(dy.double())
+    got = PF.layernorm_backward(x, dy, gam, ln_eps=0.0)
+    # as with an eps: one rounding of dx to its type, float32 sums
+    for g, want, tol in zip(got, (x64.grad, g64.grad, b64.grad), (4e-3 if dtype == torch.bfloat16 else 1e-6, 1e-5, 1e-5)):
+        assert torch.isfinite(g).all()
+        assert_rel_l2(g, want, "dx, d gamma, d beta", tol=tol)
+
+
 @pytest.mark.parametrize("grid,C,O,B,k", [((3, 5), 64, 256, 2, 3), ((16, 17), 256, 256, 1, 3), ((9, 30), 128, 512, 3, 5),
                                           ((4, 5, 7), 64, 256, 2, 3), ((33, 40), 512, 256, 1, 3)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
