@@ -281,6 +281,7 @@ class GALEBlock(nn.Module):
     fp8_weights = False  # the shared MLP helpers read it; GALE blocks are served in bf16 / float32 only
     _mlp_kernel_params = TransolverBlock._mlp_kernel_params
     _mlp_kernel_packed = TransolverBlock._mlp_kernel_packed
+    _mlp_is_plain = TransolverBlock._mlp_is_plain
     _mlp_kernel_serves = TransolverBlock._mlp_kernel_serves
     _mlp_residual = TransolverBlock._mlp_residual
 

@@ -186,10 +186,19 @@ class TransolverBlock(nn.Module):
                 self._mlp_cache["packed"] = PF.mlp_pack(w1, w2)
         return self._mlp_cache["packed"], b1, b2
 
+    def _mlp_is_plain(self) -> bool:
+        """True where calling ln_mlp1[1] is Linear, GELU, Linear on its own parameters and nothing more, as the kernels
+        compute it: no hooks (weight normalisation forms the weight in one), no replaced or parametrised module."""
+        mlp = self.ln_mlp1[1]
+        if type(mlp) is not Mlp or len(mlp.layers) != 3:
+            return False
+        lin1, act, lin2 = mlp.layers
+        return (type(lin1) is type(lin2) is nn.Linear and type(act) is nn.GELU and act.approximate == "none" and
+                PA.unhooked(mlp, mlp.layers, lin1, act, lin2))
+
     def _mlp_kernel_serves(self, normed: torch.Tensor) -> bool:
         mlp = self.ln_mlp1[1]
-        if not (normed.is_cuda and normed.dtype in (torch.bfloat16, torch.float32) and isinstance(mlp.layers[1], nn.GELU)
-                and mlp.layers[1].approximate == "none"):
+        if not (normed.is_cuda and normed.dtype in (torch.bfloat16, torch.float32) and self._mlp_is_plain()):
             return False
         if normed.dtype == torch.float32 and self.fp8_weights:
             return False
@@ -207,9 +216,9 @@ class TransolverBlock(nn.Module):
         dtype = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x_in.dtype
         if dtype != torch.bfloat16:
             return False
-        mlp = self.ln_mlp1[1]
-        if not (isinstance(mlp.layers[1], nn.GELU) and mlp.layers[1].approximate == "none"):
+        if not self._mlp_is_plain():
             return False
+        mlp = self.ln_mlp1[1]
         rows, C = x_in.numel() // x_in.shape[-1], x_in.shape[-1]
         if C != 256:
             # at 512 channels the MLP kernel runs one wave per SIMD and nothing hides the normalisation of its rows:
@@ -259,13 +268,12 @@ class TransolverBlock(nn.Module):
 
     def _whole_block(self, x_in: torch.Tensor, fx: torch.Tensor, next_ln: nn.LayerNorm | None,
                      head: nn.Linear | None = None):
-        """The block behind ln_1 in one library call (pa_block_forward) where the shape is served (float32, 32
-        slices; hidden 128 in heads of 16, or 32 / 64 channels on an irregular mesh), else None.  With `head` (the last block's ln_mlp2[1], up to 4 outputs) the second
-        element of the result is the head's output instead of the LayerNorm."""
+        """The block behind ln_1 in one library call (pa_block_forward) where the shape is served (float32, 32 slices;
+        hidden 128 in heads of 16, or 32 / 64 channels on an irregular mesh), else None.  With `head` (the last block's
+        ln_mlp2[1], up to 4 outputs) the second element of the result is the head's output instead of the LayerNorm."""
         attn, mlp = self.Attn, self.ln_mlp1[1]
         if not (x_in.is_cuda and x_in.dtype == torch.float32 and fx.dtype == torch.float32 and not self.fp8_weights
-                and not getattr(attn, "plus", False) and isinstance(mlp.layers[1], nn.GELU)
-                and mlp.layers[1].approximate == "none" and hasattr(attn, "layer_dims")):
+                and not getattr(attn, "plus", False) and hasattr(attn, "layer_dims") and self._mlp_is_plain()):
             return None
         if (attn.training and attn.out_dropout.p > 0) or torch.is_autocast_enabled("cuda"):
             return None  # autocast runs the layer in its own dtype: the separate calls handle that

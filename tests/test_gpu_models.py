@@ -188,3 +188,38 @@ def test_full_size_models_by_replication(name):
                               1.5 * tol))
     assert worst_oracle <= tol, worst_oracle
     assert worst_copy <= 1.5 * tol, worst_copy
+
+
+@pytest.mark.parametrize("C,heads,ratio,dtype", [(32, 4, 2, torch.float32), (64, 4, 1, torch.float32),
+                                                 (128, 8, 1, torch.float32), (256, 8, 2, torch.bfloat16)])
+def test_served_blocks_call_mlps_that_are_more_than_their_parameters(C, heads, ratio, dtype):
+    """Hooks on a block's MLP and its Linears run at inference, a normalised weight is the one of this call, and the
+    results are those of the block served whole."""
+    announce("MLP hooks at inference", C, dtype)
+    torch.manual_seed(0)
+    model = pn.Transolver(functional_dim=3, embedding_dim=2, out_dim=3, n_layers=2, n_hidden=C, n_head=heads, mlp_ratio=ratio,
+                          slice_num=32, use_te=False).cuda().eval()
+    x, e = torch.randn(2, 301, 3, device="cuda"), torch.rand(2, 301, 2, device="cuda")
+    amp = dtype == torch.bfloat16
+
+    def run():
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16, enabled=amp):
+            return model(x, e)
+
+    want, mlp = run(), model.blocks[1].ln_mlp1[1]
+    tol = 2e-2 if amp else 1e-5  # the same arithmetic in separate calls: bf16 roundings between them, or float32 sums
+    for m in (mlp, mlp.layers, *mlp.layers):
+        seen = []
+        handle = m.register_forward_hook(lambda *a: seen.append(1))
+        got = run()
+        handle.remove()
+        assert len(seen) == 1, m
+        assert_rel_l2(got, want, "output with a hook", tol=tol)
+    torch.nn.utils.parametrizations.weight_norm(mlp.layers[2])
+    assert_rel_l2(run(), want, "normalised weight", tol=tol)
+    with torch.no_grad():
+        mlp.layers[2].parametrizations.weight.original0.mul_(3.0)
+    got = run()
+    torch.nn.utils.parametrize.remove_parametrizations(mlp.layers[2], "weight")  # leaves the tripled weight
+    assert_rel_l2(got, run(), "tripled weight", tol=tol)
+    assert to.rel_l2(got.cpu(), want.cpu()) > 0.05
