@@ -321,9 +321,17 @@ class TransolverBlock(nn.Module):
                                          ln_bias=next_ln.bias.detach().float().contiguous(), ln_eps=next_ln.eps)
         return h + fx1, None
 
+    def _head_norm(self, fx: torch.Tensor) -> nn.LayerNorm | None:
+        """ln_mlp2[0] where it may ride on the kernel before it: in training ln_mlp2 is called as it is when it has hooks or
+        its first module is not a LayerNorm."""
+        ln = self.ln_mlp2[0]
+        if self._needs_grad(fx) and not (len(self.ln_mlp2) == 2 and type(ln) is nn.LayerNorm and PA.unhooked(self.ln_mlp2, ln)):
+            return None
+        return ln
+
     def forward(self, fx: torch.Tensor) -> torch.Tensor:
         if self.last_layer:
-            fx2, normed = self.forward_chain(fx, None, self.ln_mlp2[0])
+            fx2, normed = self.forward_chain(fx, None, self._head_norm(fx))
             return self.ln_mlp2[1](normed) if normed is not None else self.ln_mlp2(fx2)
         return self.forward_chain(fx, None, None)[0]
 
@@ -549,8 +557,8 @@ class Transolver(nn.Module):
                         fx = whole[1]
                         continue
                     normed = x_in
-                head = PA.unhooked(block.ln_mlp2, block.ln_mlp2[0]) or not block._needs_grad(fx)
-                fx, normed = block.forward_chain(fx, normed, block.ln_mlp2[0] if head else None)
+                head_ln = block._head_norm(fx)
+                fx, normed = block.forward_chain(fx, normed, head_ln)
                 if normed is not None and on_library:
                     fx = self._library_linear(normed, block.ln_mlp2[1])  # output head (:305-307)
                 elif normed is not None and PA.compute_dtype(fx) == normed.dtype:
@@ -558,7 +566,8 @@ class Transolver(nn.Module):
                 elif normed is not None:
                     fx = block.ln_mlp2[1](normed)
                 else:
-                    fx = PA.layer_norm_linear(fx, *block.ln_mlp2) if head else block.ln_mlp2(fx)
+                    fuse = head_ln is not None and block._needs_grad(fx)
+                    fx = PA.layer_norm_linear(fx, *block.ln_mlp2) if fuse else block.ln_mlp2(fx)
             else:
                 fx, normed = block.forward_chain(fx, normed, self.blocks[k + 1].ln_1)
         if unflatten_output:

@@ -687,6 +687,38 @@ def test_modules_with_hooks_are_called_in_training():
     assert_rel_l2(out, (inp @ (2.0 * want_w).t() + bias).cpu(), "normalised weight", tol=1e-5)
 
 
+def test_head_of_a_bf16_block_is_called_where_it_is_more_than_a_layernorm_and_a_linear():
+    """The last block by itself and in its model, bf16 training: hooks on ln_mlp2 and its modules run, a first module of
+    another kind is called."""
+    announce("hooks on the head of a bf16 block")
+    torch.manual_seed(0)
+    model = pn.Transolver(functional_dim=3, embedding_dim=2, out_dim=3, n_layers=1, n_hidden=256, n_head=8, mlp_ratio=2,
+                          slice_num=32, use_te=False).cuda().train()
+    block = model.blocks[0]
+    x, e = torch.randn(2, 300, 3, device="cuda"), torch.rand(2, 300, 2, device="cuda")
+    rows = 2 * torch.randn(2, 300, 256, device="cuda").bfloat16()
+    runs = (lambda: block(rows.clone().requires_grad_(True)), lambda: model(x, e))
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        for run in runs:
+            want = run()
+            for m in (block.ln_mlp2, *block.ln_mlp2):
+                seen = []
+                handle = m.register_forward_hook(lambda *a: seen.append(1))
+                got = run()
+                handle.remove()
+                assert len(seen) == 1, m
+                assert_rel_l2(got, want, "output with a hook", tol=1e-2)  # a LayerNorm from rounded rows, or unrounded ones
+        block.ln_mlp2[0] = torch.nn.Identity()
+        for run in runs:
+            seen = []
+            handle = block.ln_mlp2[1].register_forward_hook(lambda m, i, o: seen.append((i[0].float(), o.float())))
+            out = run()
+            handle.remove()
+            assert torch.equal(seen[0][1], out.float())
+            std = seen[0][0].std().item()
+            assert not 0.9 < std < 1.1, std  # rows that nothing normalised
+
+
 def test_mlp_module_differentiates_twice_and_forward():
     """An Mlp by itself, float32: gradients of gradients, forward mode, torch.func, and the refusal of another type."""
     announce("second derivatives of the Mlp")
