@@ -668,13 +668,15 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> 
 
 
 def compute_dtype(x: torch.Tensor) -> torch.dtype | None:
-    """The type a Linear of x runs in on the library's training path: bfloat16 under bf16 autocast, x's own float32 or
-    bfloat16 without autocast, None where the modules run as they are (also under torch.func transforms and forward-mode
-    differentiation, which the library's functions do not take part in)."""
+    """The type a Linear of x runs in on the library's training path: bfloat16 under bf16 autocast for the types it casts
+    (float64 and whole numbers it leaves alone), x's own float32 or bfloat16 without autocast, None where the modules run as
+    they are (also under torch.func transforms and forward-mode differentiation, which the library's functions do not take
+    part in)."""
     if not x.is_cuda or torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0:
         return None
     if torch.is_autocast_enabled("cuda"):
-        return torch.bfloat16 if torch.get_autocast_dtype("cuda") == torch.bfloat16 else None
+        cast = x.dtype in (torch.float32, torch.bfloat16, torch.float16)
+        return torch.bfloat16 if cast and torch.get_autocast_dtype("cuda") == torch.bfloat16 else None
     return x.dtype if x.dtype in (torch.bfloat16, torch.float32) else None
 
 

@@ -746,6 +746,19 @@ def test_mlp_module_differentiates_twice_and_forward():
         net(x.bfloat16())
 
 
+def test_mlp_module_under_autocast_leaves_types_that_autocast_leaves():
+    """A float64 Mlp in training under bf16 autocast computes in float64, whole numbers are refused."""
+    announce("Mlp types under autocast")
+    torch.manual_seed(0)
+    net, x = Mlp(4, 64, 8).cuda().double(), torch.randn(500, 4, device="cuda", dtype=torch.float64)
+    want = net.layers(x)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        got = net(x)
+        assert got.dtype == torch.float64 and torch.equal(got, want)
+        with pytest.raises(RuntimeError):
+            net.float()(torch.ones(5, 4, device="cuda", dtype=torch.int64))
+
+
 @pytest.mark.parametrize("plus", [False, True])
 def test_bf16_training_of_a_layer_left_on_the_host(plus):
     """Parameters in host memory are copied to the input's device in the forward; their gradients cannot be delivered there
