@@ -225,13 +225,38 @@ class PhysicsAttentionMfmaFunction(torch.autograd.Function):
         return (dx, None, None) + grads
 
 
-def _through_norm(y, w32, eps, d_y, d_normed, param_dtypes):
+def _keep_parameters(ctx, *params):
+    """For a backward pass that is differentiated again: the parameters themselves, where the saved tensors are copies in the
+    kernels' type.  They are not saved tensors, so that changing one between the passes stays allowed without that."""
+    ctx.kept = [(p, None if p.is_inference() else p._version) for p in params]
+
+
+def _kept_parameters(ctx):
+    if any(version is not None and p._version != version for p, version in ctx.kept):
+        raise RuntimeError("a parameter was modified in place between the forward and a backward pass with create_graph=True")
+    return [p for p, _ in ctx.kept]
+
+
+def _layernorm_backward(ctx, x, dy, w32, eps, add=None):
+    """(dx, d weight, d bias) of LayerNorm, dx with `add`: the library's kernel, or the same formulas as tensor ops on the kept
+    weight where the result is differentiated again."""
+    if not torch.is_grad_enabled():
+        return PF.layernorm_backward(x, dy, w32, eps, add)
+    weight, xf, df = _kept_parameters(ctx)[-1], x.float(), dy.float()
+    centred = xf - xf.mean(-1, keepdim=True)
+    rstd = torch.rsqrt(centred.square().mean(-1, keepdim=True) + eps)
+    xh, g = centred * rstd, df * weight.float()
+    dx = rstd * (g - g.mean(-1, keepdim=True) - xh * (g * xh).mean(-1, keepdim=True))
+    return (dx if add is None else dx + add.float()).to(x.dtype), _rows(df * xh).sum(0), _rows(df).sum(0)
+
+
+def _through_norm(ctx, y, w32, d_y, d_normed):
     """(gradient of y, d weight, d bias) for the outputs y and LayerNorm(y)."""
     if d_normed is None:
         return (None if d_y is None else _aligned(d_y.to(y.dtype))), None, None
     add = None if d_y is None else _aligned(d_y.to(y.dtype))
-    d, dg, db = PF.layernorm_backward(y, _aligned(d_normed.to(y.dtype)), w32, eps, add)
-    return d, dg.to(param_dtypes[0]), db.to(param_dtypes[1])
+    d, dg, db = _layernorm_backward(ctx, y, _aligned(d_normed.to(y.dtype)), w32, ctx.eps, add)
+    return d, dg.to(ctx.ln_dtypes[0]), db.to(ctx.ln_dtypes[1])
 
 
 class LayerResidualNormFunction(torch.autograd.Function):
@@ -246,13 +271,14 @@ class LayerResidualNormFunction(torch.autograd.Function):
         y, saved, normed = PF.layer_train_forward(x, None, kp, dims, residual, w32, _aligned(ln_b.detach().float()), eps)
         ctx.save_for_backward(x, saved, y, w32, *params)
         ctx.dims, ctx.kparams, ctx.eps, ctx.ln_dtypes = dims, kp, eps, (ln_w.dtype, ln_b.dtype)
+        _keep_parameters(ctx, ln_w)
         return y, normed
 
     @staticmethod
     def backward(ctx, d_y, d_normed):
         x, saved, y, w32, *params = ctx.saved_tensors
         need = ctx.needs_input_grad
-        d, dg, db = _through_norm(y, w32, ctx.eps, d_y, d_normed, ctx.ln_dtypes)
+        d, dg, db = _through_norm(ctx, y, w32, d_y, d_normed)
         if d is None:
             return (None,) * (6 + len(params))
         dx, grads = PF.layer_train_backward(x, None, d, saved, ctx.kparams, ctx.dims, need[0])
@@ -639,16 +665,17 @@ class LinearFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias):
         w16 = weight.to(x.dtype)
-        ctx.save_for_backward(x, weight, w16)
+        ctx.save_for_backward(x, w16)
+        _keep_parameters(ctx, weight)
         ctx.param_dtypes = (weight.dtype, bias.dtype if bias is not None else None)
         return torch.nn.functional.linear(x, w16, bias.to(x.dtype) if bias is not None else None)
 
     @staticmethod
     def backward(ctx, dy):
-        x, weight, w16 = ctx.saved_tensors
+        x, w16 = ctx.saved_tensors
         dy = dy.contiguous()
         again = torch.is_grad_enabled()  # create_graph: tensor ops on the inputs themselves, to be differentiated again
-        dx = (dy @ (weight.to(x.dtype) if again else w16)) if ctx.needs_input_grad[0] else None
+        dx = (dy @ (_kept_parameters(ctx)[0].to(x.dtype) if again else w16)) if ctx.needs_input_grad[0] else None
         dw = db = None
         if ctx.needs_input_grad[1] or ctx.needs_input_grad[2]:
             if again:
@@ -714,6 +741,7 @@ class MlpResidualFunction(torch.autograd.Function):
         w1_16, w2_16 = (_aligned(w.detach().to(torch.bfloat16)) for w in (w1, w2))
         b1_32, b2_32 = (_aligned(b.detach().float()) for b in (b1, b2))
         ctx.param_dtypes = tuple(p.dtype for p in (w1, b1, w2, b2))
+        _keep_parameters(ctx, w1, b1, w2, *(() if ln_w is None else (ln_w,)))
         packed = PF.mlp_pack(w1_16, w2_16)
         if ln_w is None:
             ctx.save_for_backward(x, w1_16, b1_32, w2_16)
@@ -731,18 +759,21 @@ class MlpResidualFunction(torch.autograd.Function):
         need = ctx.needs_input_grad
         d_ln = (None, None)
         if norm:
-            dy, *d_ln = _through_norm(norm[0], norm[1], ctx.eps, dy, d_normed, ctx.ln_dtypes)
+            dy, *d_ln = _through_norm(ctx, norm[0], norm[1], dy, d_normed)
         if dy is None:
             return (None,) * 9
         dy16 = _aligned(dy.to(x.dtype))
-        if torch.is_grad_enabled():  # create_graph: the same formulas as tensor ops, which can be differentiated again
-            h = torch.nn.functional.linear(x, w1, b1.to(x.dtype))
+        again = torch.is_grad_enabled()
+        if again:  # create_graph: the same formulas as tensor ops on the parameters, which can be differentiated again
+            w1, b1, w2 = (p.to(x.dtype) for p in _kept_parameters(ctx)[:3])
+            h = torch.nn.functional.linear(x, w1, b1)
             act, dh = torch.nn.functional.gelu(h), torch.ops.aten.gelu_backward(dy16 @ w2, h)
         else:
             act, dh = PF.mlp_backward(x, dy16, w1, b1, w2)
+        product = _wgrad if not again else lambda d, i: (d.float().t() @ i.float(), d.sum(0, dtype=torch.float32))
         dx = dh @ w1 if need[0] else None
-        d_w1, d_b1 = _wgrad(_rows(dh), _rows(x)) if need[2] or need[3] else (None, None)
-        d_w2, d_b2 = _wgrad(_rows(dy16), _rows(act)) if need[4] or need[5] else (None, None)
+        d_w1, d_b1 = product(_rows(dh), _rows(x)) if need[2] or need[3] else (None, None)
+        d_w2, d_b2 = product(_rows(dy16), _rows(act)) if need[4] or need[5] else (None, None)
         grads = (g.to(t) if n else None for g, t, n in zip((d_w1, d_b1, d_w2, d_b2), ctx.param_dtypes, need[2:]))
         return (dx, dy if need[1] else None, *grads, *d_ln, None)
 
@@ -790,21 +821,21 @@ def linear_as_autocast(x: torch.Tensor, lin: torch.nn.Linear) -> torch.Tensor:
 
 class LayerNormFunction(torch.autograd.Function):
     """LayerNorm over the last axis on the library's kernels, forward and backward, in the input's dtype (fp32 or bf16;
-    statistics in fp32).  The backward recomputes the statistics from the saved input."""
+    statistics in fp32); x is contiguous.  The backward recomputes the statistics from the saved input."""
 
     @staticmethod
     def forward(ctx, x, weight, bias, eps):
-        x = x.contiguous()
         w32, b32 = weight.detach().float().contiguous(), bias.detach().float().contiguous()
         _, out = PF.residual_layernorm(x, ln_weight=w32, ln_bias=b32, ln_eps=eps)
         ctx.save_for_backward(x, w32)
+        _keep_parameters(ctx, weight)
         ctx.eps, ctx.param_dtypes = eps, (weight.dtype, bias.dtype)
         return out
 
     @staticmethod
     def backward(ctx, dy):
         x, w32 = ctx.saved_tensors
-        dx, dg, db = PF.layernorm_backward(x, dy.to(x.dtype).contiguous(), w32, ctx.eps)
+        dx, dg, db = _layernorm_backward(ctx, x, dy.to(x.dtype).contiguous(), w32, ctx.eps)
         return dx, dg.to(ctx.param_dtypes[0]), db.to(ctx.param_dtypes[1]), None
 
 
@@ -815,12 +846,7 @@ class LayerNormResidualFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias, eps):
         ctx.set_materialize_grads(False)
-        w32, b32 = weight.detach().float().contiguous(), bias.detach().float().contiguous()
-        rows = x.contiguous()
-        _, out = PF.residual_layernorm(rows, ln_weight=w32, ln_bias=b32, ln_eps=eps)
-        ctx.save_for_backward(rows, w32)
-        ctx.eps, ctx.param_dtypes = eps, (weight.dtype, bias.dtype)
-        return out, x.view_as(x)
+        return LayerNormFunction.forward(ctx, x, weight, bias, eps), x.view_as(x)
 
     @staticmethod
     def backward(ctx, dy, d_pass):
@@ -828,7 +854,7 @@ class LayerNormResidualFunction(torch.autograd.Function):
             return d_pass, None, None, None
         x, w32 = ctx.saved_tensors
         add = None if d_pass is None else _aligned(d_pass.to(x.dtype))
-        dx, dg, db = PF.layernorm_backward(x, dy.to(x.dtype).contiguous(), w32, ctx.eps, add)
+        dx, dg, db = _layernorm_backward(ctx, x, dy.to(x.dtype).contiguous(), w32, ctx.eps, add)
         return dx, dg.to(ctx.param_dtypes[0]), db.to(ctx.param_dtypes[1]), None
 
 
@@ -839,12 +865,12 @@ def _layer_norm_served(x: torch.Tensor, ln: torch.nn.LayerNorm) -> bool:
 def layer_norm_residual(x: torch.Tensor, ln: torch.nn.LayerNorm):
     """(LayerNorm(x), x) for a pre-norm block: use the second element as the residual stream."""
     if _layer_norm_served(x, ln) and x.requires_grad and torch.is_grad_enabled():
-        return LayerNormResidualFunction.apply(x, ln.weight, ln.bias, ln.eps)
+        return LayerNormResidualFunction.apply(x.contiguous(), ln.weight, ln.bias, ln.eps)
     return layer_norm(x, ln), x
 
 
 def layer_norm(x: torch.Tensor, ln: torch.nn.LayerNorm) -> torch.Tensor:
     """Differentiable LayerNorm: the library's kernels where they serve the rows, the module itself otherwise."""
     if _layer_norm_served(x, ln):
-        return LayerNormFunction.apply(x, ln.weight, ln.bias, ln.eps)
+        return LayerNormFunction.apply(x.contiguous(), ln.weight, ln.bias, ln.eps)
     return ln(x)

@@ -590,6 +590,64 @@ def test_mlp_residual_block(rows, F):
     assert_rel_l2(gx.detach(), x64.grad, "dx, create_graph", tol=1e-2)
 
 
+@pytest.mark.parametrize("next_norm", [False, True])
+def test_mlp_residual_block_differentiates_twice(next_norm):
+    """Gradients of a function of the gradient of a bf16 block's MLP, by its input and every parameter of the Linears and of
+    the LayerNorms before and behind, with float32 and with bf16 parameters, against float64.  A parameter that changed
+    between the passes is refused there and only there."""
+    announce("mlp residual twice", next_norm)
+    torch.manual_seed(0)
+    rows, C, F = 300, 256, 128
+    ln, after = torch.nn.LayerNorm(C).cuda(), torch.nn.LayerNorm(C).cuda()
+    layers = torch.nn.Sequential(torch.nn.Linear(C, F), torch.nn.GELU(), torch.nn.Linear(F, C)).cuda()
+    modules = [ln, layers] + ([after] if next_norm else [])
+    with torch.no_grad():
+        for m in modules:
+            for p in m.parameters():
+                p.copy_((p + 0.1 * torch.randn_like(p)).bfloat16().float())
+    x, dy, dn = (torch.randn(rows, C, device="cuda").bfloat16() for _ in range(3))
+
+    def second(mods, x, call):
+        x = x.detach().requires_grad_(True)
+        params = [p for m in mods for p in m.parameters()]
+        grads = torch.autograd.grad(call(x), [x, *params], create_graph=True)
+        return torch.autograd.grad(sum(g.to(x.dtype).float().square().sum() if x.dtype != torch.float64 else g.square().sum()
+                                       for g in grads), [x, *params], allow_unused=True)
+
+    def fused(x):
+        normed, rest = PA.layer_norm_residual(x, ln)
+        y, n = PA.mlp_residual(normed, rest, layers, after if next_norm else None)
+        assert (n is not None) == next_norm
+        return (y * dy).sum() + ((n * dn).sum() if next_norm else 0)
+
+    mods64 = [copy.deepcopy(m).double() for m in modules]
+
+    def plain(x):
+        y = x + mods64[1](mods64[0](x))
+        return (y * dy.double()).sum() + ((mods64[2](y) * dn.double()).sum() if next_norm else 0)
+
+    want = second(mods64, x.double(), plain)
+    names = ["x"] + [f"{k}.{n}" for k, m in enumerate(modules) for n, _ in m.named_parameters()]
+    for dtype in (torch.float32, torch.bfloat16):
+        for m in modules:
+            m.to(dtype)
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=dtype == torch.float32):
+            got = second(modules, x, fused)
+        for name, g, w in zip(names, got, want):
+            if w is None or w.norm() == 0:  # a sum that does not depend on the last bias
+                assert g is None or g.float().norm() <= 1e-6 * want[1].norm()
+                continue
+            # every chain passes the block four times, with some ten bf16 roundings (1.1e-3 of a value each on the average)
+            # of terms that cancel by a few; the parts that used to be missing are of the size of the result
+            assert_rel_l2(g, w, name + " " + str(dtype), tol=4e-2)
+    out = fused(x.detach().requires_grad_(True))
+    with torch.no_grad():
+        layers[0].bias.add_(1.0)
+    params = list(layers.parameters())
+    with pytest.raises(RuntimeError, match="modified"):
+        torch.autograd.grad(out, params, create_graph=True, retain_graph=True)
+
+
 @pytest.mark.parametrize("C,S,B,N,grid", [(256, 64, 2, 1001, None), (128, 16, 1, 33, None), (256, 32, 1, 12 * 9, (12, 9))])
 def test_bf16_blocks_with_fused_tails_train_like_separate_ones(C, S, B, N, grid):
     """A chain of two bf16 blocks and its head: residuals and LayerNorms in the layer's and the MLP's kernels are no
