@@ -455,9 +455,15 @@ int pa_mfma_slice_weighted_sum(const pa_shape *shape, const void *w_pack, const 
                                float *sums, void *stream);
 /* out_x (B, N, H*32) bf16 = deslice of the attended tokens (PA.py:492-495), the input of d W_out = dy^T out_x. */
 int pa_mfma_deslice(const pa_shape *shape, const void *w_pack, const void *tokp, void *out_x, void *stream);
-/* Scratch bytes and gradient floats of pa_point_backward for layers without the Transolver++ temperature. */
+/* Per-point part of the backward pass, as pa_slice_softmax_backward but with the slice weights taken from w_pack.
+ * tables: scratch of pa_mfma_backward_tables_bytes(shape) bytes; d_temperature_partials: float32,
+ * pa_mfma_backward_groups(shape) * H elements (sum over the first index). */
 int64_t pa_mfma_backward_tables_bytes(const pa_shape *shape);
 int64_t pa_mfma_backward_groups(const pa_shape *shape);
+int pa_mfma_slice_softmax_backward(const pa_shape *shape, const pa_params *p, const void *x_mid, const void *fx_mid,
+                                   const void *d_out_x, const void *w_pack, const float *out_slice_token,
+                                   const float *d_num, const float *d_norm, void *tables, void *d_proj, void *d_z,
+                                   float *d_temperature_partials, void *stream);
 
 /* ---- backward pieces for bf16 layers with 32-wide heads (D = 32, C = 32 H in {128, 256, 512}, S in {16, 32, 64, 128}) ----
  * Per-point part: x_mid, fx_mid, d_out_x bf16 rows (B, N, H*32), the attended tokens (NULL: no deslice term), d num and
@@ -609,11 +615,15 @@ int pa_residual_layernorm(int dtype, int64_t rows, int64_t C, void *y, const pa_
 
 /* Backward of LayerNorm over the last axis (TR.py:210, :300-307; the reference relies on autograd): x, dy, dx (rows, C)
  * in the activation dtype, C a multiple of 4 (float32) / 8 (bf16) and <= 1024; the statistics are recomputed from x.
- * dx = add + (gradient through the LayerNorm), add (rows, C) or NULL: the gradient that reaches x past it.
- * grads (2, C) float32: d gamma, d beta; partials: pa_layernorm_backward_groups(rows) * 2 C floats of scratch. */
+ * partials: float32 (pa_layernorm_backward_groups(rows), 2, C): [g][0][:] = that group's share of d gamma,
+ * [g][1][:] of d beta; the caller adds them up over g. */
 int64_t pa_layernorm_backward_groups(int64_t rows);
-int pa_layernorm_backward(int dtype, int64_t rows, int64_t C, const void *x, const void *dy, const void *add,
-                          const float *gamma, float eps, void *dx, float *partials, float *grads, void *stream);
+int pa_layernorm_backward(int dtype, int64_t rows, int64_t C, const void *x, const void *dy, const float *gamma,
+                          float eps, void *dx, float *partials, void *stream);
+/* The same with dx = add + (gradient through the LayerNorm), add (rows, C) or NULL: the gradient that reaches x past it; and
+ * the partial sums added up: grads (2, C) float32 = d gamma, d beta, partials the same scratch. */
+int pa_layernorm_backward_add(int dtype, int64_t rows, int64_t C, const void *x, const void *dy, const void *add,
+                              const float *gamma, float eps, void *dx, float *partials, float *grads, void *stream);
 
 /* ---- whole layer ------------------------------------------------------------------------------ */
 

@@ -30,11 +30,12 @@ EXPORTED = [
     "pa_layer_forward_plus_workspace_bytes", "pa_layer_forward_plus", "pa_flare_forward_mfma_supported",
     "pa_flare_forward_mfma_workspace_bytes", "pa_flare_forward_mfma",
     "pa_mfma_backward_query", "pa_rows_gemm_packed", "pa_mfma_slice_weighted_sum", "pa_mfma_deslice",
-    "pa_mfma_backward_tables_bytes", "pa_mfma_backward_groups", "pa_point_backward_grads",
+    "pa_mfma_backward_tables_bytes", "pa_mfma_backward_groups", "pa_mfma_slice_softmax_backward", "pa_point_backward_grads",
     "pa_point_backward_workspace_bytes", "pa_point_backward", "pa_output_backward_workspace_bytes", "pa_output_backward",
     "pa_layer_train_bytes", "pa_layer_train_forward", "pa_layer_train_backward",
     "pa_cols_gemm_chunks", "pa_cols_gemm", "pa_residual_layernorm",
     "pa_mfma_layer_forward", "pa_rows_gemm_act", "pa_layernorm_backward_groups", "pa_layernorm_backward",
+    "pa_layernorm_backward_add",
     "pa_static_scratch_bytes", "pa_slice_reduce_static",
     "pa_preprocess_query", "pa_preprocess_workspace_bytes", "pa_preprocess_forward",
     "pa_block_query", "pa_block_workspace_bytes", "pa_block_forward", "pa_markers_enabled",
@@ -257,6 +258,8 @@ def load() -> ctypes.CDLL:
     lib.pa_mfma_backward_tables_bytes.argtypes = [ps]
     lib.pa_mfma_backward_groups.restype = c_int64
     lib.pa_mfma_backward_groups.argtypes = [ps]
+    lib.pa_mfma_slice_softmax_backward.restype = c_int
+    lib.pa_mfma_slice_softmax_backward.argtypes = [ps, pp] + [c_void_p] * 12
     pplus = POINTER(PaPlusParams)
     lib.pa_point_backward_grads.restype = c_int64
     lib.pa_point_backward_grads.argtypes = [ps, c_int]
@@ -292,7 +295,9 @@ def load() -> ctypes.CDLL:
     lib.pa_layernorm_backward_groups.restype = c_int64
     lib.pa_layernorm_backward_groups.argtypes = [c_int64]
     lib.pa_layernorm_backward.restype = c_int
-    lib.pa_layernorm_backward.argtypes = [c_int, c_int64, c_int64] + [c_void_p] * 4 + [c_float] + [c_void_p] * 4
+    lib.pa_layernorm_backward.argtypes = [c_int, c_int64, c_int64] + [c_void_p] * 3 + [c_float] + [c_void_p] * 3
+    lib.pa_layernorm_backward_add.restype = c_int
+    lib.pa_layernorm_backward_add.argtypes = [c_int, c_int64, c_int64] + [c_void_p] * 4 + [c_float] + [c_void_p] * 4
     _lib = lib
     return lib
 

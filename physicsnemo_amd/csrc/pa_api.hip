@@ -362,7 +362,7 @@ int mfma_layer(const pa_shape &s, const pa_params &p, const void *blob, const vo
 
 extern "C" {
 
-int pa_version(void) { return 111; }
+int pa_version(void) { return 112; }
 
 int pa_set_compute_units(int n) {
   if (n < 0 || n > 4096) return PA_ERR_DIMS;
@@ -702,8 +702,18 @@ int64_t pa_layernorm_backward_groups(int64_t rows) {
   return pa::general::layernorm_backward_groups(rows);
 }
 
-int pa_layernorm_backward(int dtype, int64_t rows, int64_t C, const void *x, const void *dy, const void *add,
-                          const float *gamma, float eps, void *dx, float *partials, float *grads, void *stream) {
+int pa_layernorm_backward(int dtype, int64_t rows, int64_t C, const void *x, const void *dy, const float *gamma, float eps,
+                          void *dx, float *partials, void *stream) {
+  if (dtype != PA_F32 && dtype != PA_BF16) return PA_ERR_UNSUPPORTED;
+  if (rows <= 0 || C <= 0 || C > 1024) return PA_ERR_DIMS;
+  if (!x || !dy || !gamma || !dx || !partials) return PA_ERR_NULL;
+  if (!aligned16(x) || !aligned16(dy) || !aligned16(dx)) return PA_ERR_ALIGN;
+  return pa::general::layernorm_backward(dtype, rows, C, x, dy, nullptr, gamma, eps, dx, partials, nullptr,
+                                         static_cast<hipStream_t>(stream));
+}
+
+int pa_layernorm_backward_add(int dtype, int64_t rows, int64_t C, const void *x, const void *dy, const void *add,
+                              const float *gamma, float eps, void *dx, float *partials, float *grads, void *stream) {
   if (dtype != PA_F32 && dtype != PA_BF16) return PA_ERR_UNSUPPORTED;
   if (rows <= 0 || C <= 0 || C > 1024) return PA_ERR_DIMS;
   if (!x || !dy || !gamma || !dx || !partials || !grads) return PA_ERR_NULL;
@@ -799,9 +809,19 @@ int pa_mfma_backward_query(const pa_shape *shape) {
   return pa::mfma::backward_supported(*shape) && check_backward_shape(PA_BF16, shape) == PA_OK ? 1 : 0;
 }
 
-int64_t pa_mfma_backward_tables_bytes(const pa_shape *shape) { return pa_point_backward_workspace_bytes(shape, 0); }
+int64_t pa_mfma_backward_tables_bytes(const pa_shape *shape) {
+  int rc = check_shape(PA_BF16, shape);
+  if (rc) return rc;
+  if (!pa::mfma::backward_supported(*shape)) return PA_ERR_UNSUPPORTED;
+  return pa::mfma::backward_tables_bytes(*shape);
+}
 
-int64_t pa_mfma_backward_groups(const pa_shape *shape) { return pa_point_backward_grads(shape, 0); }
+int64_t pa_mfma_backward_groups(const pa_shape *shape) {
+  int rc = check_shape(PA_BF16, shape);
+  if (rc) return rc;
+  if (!pa::mfma::backward_supported(*shape)) return PA_ERR_UNSUPPORTED;
+  return pa::mfma::backward_groups(*shape, compute_units()) * shape->B;
+}
 
 int pa_rows_gemm_packed(const pa_shape *shape, int64_t c_in, const void *in, const void *weight, const float *bias,
                         void *out, void *out_pack, void *stream) {
@@ -837,6 +857,25 @@ int pa_mfma_deslice(const pa_shape *shape, const void *w_pack, const void *tokp,
   if (!w_pack || !tokp || !out_x) return PA_ERR_NULL;
   if (!aligned16(w_pack) || !aligned16(tokp) || !aligned16(out_x)) return PA_ERR_ALIGN;
   return pa::mfma::deslice_natural(*shape, w_pack, tokp, out_x, compute_units(), static_cast<hipStream_t>(stream));
+}
+
+int pa_mfma_slice_softmax_backward(const pa_shape *shape, const pa_params *p, const void *x_mid, const void *fx_mid,
+                                   const void *d_out_x, const void *w_pack, const float *out_slice_token,
+                                   const float *d_num, const float *d_norm, void *tables, void *d_proj, void *d_z,
+                                   float *d_temperature_partials, void *stream) {
+  int rc = check_shape(PA_BF16, shape);
+  if (rc) return rc;
+  if (!pa::mfma::backward_supported(*shape)) return PA_ERR_UNSUPPORTED;
+  if (!p || !p->in_project_slice_weight || !p->in_project_slice_bias || !p->temperature) return PA_ERR_NULL;
+  if (!x_mid || !fx_mid || !d_out_x || !w_pack || !out_slice_token || !d_num || !d_norm || !tables || !d_proj || !d_z ||
+      !d_temperature_partials)
+    return PA_ERR_NULL;
+  if (!aligned16(x_mid) || !aligned16(fx_mid) || !aligned16(d_out_x) || !aligned16(w_pack) || !aligned16(tables) ||
+      !aligned16(d_proj) || !aligned16(d_z))
+    return PA_ERR_ALIGN;
+  return pa::mfma::slice_softmax_backward(*shape, *p, x_mid, fx_mid, d_out_x, w_pack, out_slice_token, d_num, d_norm, tables,
+                                          d_proj, d_z, d_temperature_partials, compute_units(),
+                                          static_cast<hipStream_t>(stream));
 }
 
 static int check_point_backward(const pa_shape *shape) {

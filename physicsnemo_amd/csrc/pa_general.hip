@@ -1365,12 +1365,13 @@ static int layernorm_backward_t(int64_t rows, int C, const void *x, const void *
   return ok ? launch_status() : PA_ERR_UNSUPPORTED;
 }
 
-// grads (2, C): d gamma, d beta; partials: layernorm_backward_groups(rows) * 2 C floats of scratch; add may be NULL
+// partials: layernorm_backward_groups(rows) * 2 C floats; grads (2, C): their sums d gamma, d beta, or NULL (the caller adds
+// them up); add may be NULL
 int layernorm_backward(int dtype, int64_t rows, int64_t C, const void *x, const void *dy, const void *add, const float *gamma,
                        float eps, void *dx, float *partials, float *grads, hipStream_t st) {
   const int rc = dtype == PA_F32 ? layernorm_backward_t<float>(rows, (int)C, x, dy, add, gamma, eps, dx, partials, st)
                                  : layernorm_backward_t<bf16>(rows, (int)C, x, dy, add, gamma, eps, dx, partials, st);
-  return rc ? rc : wgrad::sum_rows(partials, layernorm_backward_groups(rows), 2 * C, grads, st);
+  return rc || !grads ? rc : wgrad::sum_rows(partials, layernorm_backward_groups(rows), 2 * C, grads, st);
 }
 
 int residual_ln(int dtype, const pa_shape &s, void *y, const pa_block_tail &tail, hipStream_t st) {

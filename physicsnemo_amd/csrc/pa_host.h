@@ -250,6 +250,11 @@ int deslice_recompute(const pa_shape &s, const pa_params &p, const void *x_mid, 
                       void *out_x, int num_cu, hipStream_t st);
 bool backward_supported(const pa_shape &s);
 int64_t backward_groups(const pa_shape &s, int num_cu);
+int64_t backward_tables_bytes(const pa_shape &s);
+int slice_softmax_backward(const pa_shape &s, const pa_params &p, const void *x_mid, const void *fx_mid,
+                           const void *d_out_x, const void *w_pack, const float *out_token, const float *d_num,
+                           const float *d_norm, void *tables, void *d_proj, void *d_z, float *dT_part, int num_cu,
+                           hipStream_t st);
 int deslice_natural(const pa_shape &s, const void *w_pack, const void *tokp, void *out_x, int num_cu, hipStream_t st);
 bool point_backward_supported(const pa_shape &s);
 int64_t point_backward_grads(const pa_shape &s, bool plus);

@@ -289,9 +289,10 @@ def layernorm_backward(x, dy, ln_weight, ln_eps=1e-5, add=None):
     partials = torch.empty(int(lib.pa_layernorm_backward_groups(rows)) * 2 * C, dtype=torch.float32, device=x.device)
     grads = torch.empty(2, C, dtype=torch.float32, device=x.device)
     dx = torch.empty_like(x)
-    _lib.check(lib.pa_layernorm_backward(_lib.dtype_code(x.dtype), rows, C, x.data_ptr(), dy.data_ptr(), _lib.ptr(add),
-                                         ln_weight.data_ptr(), float(ln_eps), dx.data_ptr(), partials.data_ptr(),
-                                         grads.data_ptr(), _lib.current_stream_ptr(x.device)), "pa_layernorm_backward")
+    _lib.check(lib.pa_layernorm_backward_add(_lib.dtype_code(x.dtype), rows, C, x.data_ptr(), dy.data_ptr(), _lib.ptr(add),
+                                             ln_weight.data_ptr(), float(ln_eps), dx.data_ptr(), partials.data_ptr(),
+                                             grads.data_ptr(), _lib.current_stream_ptr(x.device)),
+               "pa_layernorm_backward_add")
     return dx, grads[0], grads[1]
 
 
@@ -597,6 +598,24 @@ class MfmaStages:
         _lib.check(self.lib.pa_mfma_deslice(byref(self.shape), self.w_pack.data_ptr(), self.tokp.data_ptr(),
                                             out_x.data_ptr(), self._stream()), "pa_mfma_deslice")
         return out_x
+
+    def slice_softmax_backward(self, x_mid, fx_mid, d_out_x, d_num, d_norm):
+        """Returns (d_proj (B,N,2HD) = [d x_mid | d fx_mid], d_z (B,N,H,S), d clamp(temperature) (H) float32)."""
+        _need_cuda(x_mid, fx_mid, d_out_x, d_num, d_norm)
+        d = self.dims
+        nbytes = self.lib.pa_mfma_backward_tables_bytes(byref(self.shape))
+        groups = self.lib.pa_mfma_backward_groups(byref(self.shape))
+        if nbytes < 0 or groups < 0:
+            _lib.check(int(min(nbytes, groups)), "pa_mfma_backward_tables_bytes")
+        tables = torch.empty(int(nbytes), dtype=torch.uint8, device=self.device)
+        d_proj = torch.empty(d.B, d.N, 2 * d.H * 32, dtype=torch.bfloat16, device=self.device)
+        d_z = torch.empty(d.B, d.N, d.H, d.S, dtype=torch.bfloat16, device=self.device)
+        dT = torch.empty(int(groups), d.H, dtype=torch.float32, device=self.device)
+        _lib.check(self.lib.pa_mfma_slice_softmax_backward(
+            byref(self.shape), byref(self.cparams), x_mid.data_ptr(), fx_mid.data_ptr(), d_out_x.data_ptr(),
+            self.w_pack.data_ptr(), self.tok_out.data_ptr(), d_num.data_ptr(), d_norm.data_ptr(), tables.data_ptr(),
+            d_proj.data_ptr(), d_z.data_ptr(), dT.data_ptr(), self._stream()), "pa_mfma_slice_softmax_backward")
+        return d_proj, d_z, dT.sum(0)
 
     def deslice_project(self, y, residual=None, ln_weight=None, ln_bias=None, ln_eps=1e-5, ln_out=None):
         tail = _c_tail(residual, ln_weight, ln_bias, ln_eps, ln_out)

@@ -9,6 +9,7 @@ import torch
 
 from oracle import torch_oracle as to
 import physicsnemo_amd as pn
+from physicsnemo_amd import _lib
 from physicsnemo_amd import autograd as PA
 from physicsnemo_amd import functional as PF
 from physicsnemo_amd.transolver import Mlp
@@ -529,6 +530,49 @@ def test_layernorm_backward_without_eps(dtype, rows, C):
     for g, want, tol in zip(got, (x64.grad, g64.grad, b64.grad), (4e-3 if dtype == torch.bfloat16 else 1e-6, 1e-5, 1e-5)):
         assert torch.isfinite(g).all()
         assert_rel_l2(g, want, "dx, d gamma, d beta", tol=tol)
+
+
+@pytest.mark.parametrize("C,S,B,N", [(256, 64, 2, 333), (128, 16, 1, 63), (128, 128, 2, 100), (256, 32, 1, 32)])
+def test_point_stages_of_the_bf16_backward_agree(C, S, B, N):
+    """The stage that reads the stored slice weights and leaves d z, and the one that forms the weights again and sums
+    d W_slice: the same gradients."""
+    announce("point stages", C, S, B, N)
+    torch.manual_seed(S)
+    _, hip = make_pair("irregular", C, C // 32, 32, S)
+    x, g = torch.randn(2, B, N, C, device="cuda").bfloat16()
+    dims, kp = hip.layer_dims(x), hip.kernel_params(torch.bfloat16, x.device)
+    st = PF.MfmaStages(kp, dims, x.device)
+    st.pack_params()
+    st.project_softmax(x)
+    st.slice_reduce()
+    st.combine_attention()
+    x_mid, fx_mid = PF.project_inputs(x, kp, dims)
+    d_num = torch.randn(B, dims.H, S, 32, device="cuda")
+    d_norm = torch.randn(B, dims.H, S, device="cuda")
+    d_proj, d_z, d_temp = st.slice_softmax_backward(x_mid, fx_mid, g, d_num, d_norm)
+    want, d_ws, d_bs, want_temp = PF.point_backward(x_mid, fx_mid, g, st.tok_out, d_num, d_norm, kp, dims)
+    # one side reads weights rounded to bf16 (2^-9 of each), both round d z and the result to it
+    assert_rel_l2(d_proj, want, "d x_mid, d fx_mid", tol=6e-3)
+    rows = d_z.float().reshape(-1, S)
+    assert_rel_l2(rows.t() @ x_mid.float().reshape(-1, 32), d_ws, "d W_slice from d z", tol=1e-2)
+    assert_rel_l2(d_temp, want_temp, "d temperature", tol=3e-2)
+
+
+@pytest.mark.parametrize("dtype,rows,C", [(torch.bfloat16, 1003, 256), (torch.float32, 31, 64)])
+def test_layernorm_backward_partial_sums(dtype, rows, C):
+    """pa_layernorm_backward leaves the groups' shares of d gamma and d beta to the caller; their sum and dx are those of
+    the call that adds them up."""
+    announce("layernorm partial sums", dtype, rows, C)
+    x, dy = (torch.randn(rows, C, device="cuda").to(dtype) for _ in range(2))
+    gam, dx = torch.randn(C, device="cuda"), torch.empty_like(x)
+    lib = _lib.load()
+    partials = torch.empty(lib.pa_layernorm_backward_groups(rows), 2, C, device="cuda")
+    _lib.check(lib.pa_layernorm_backward(_lib.dtype_code(dtype), rows, C, x.data_ptr(), dy.data_ptr(), gam.data_ptr(), 1e-5,
+                                         dx.data_ptr(), partials.data_ptr(), _lib.current_stream_ptr(x.device)), "call")
+    want_dx, dg, db = PF.layernorm_backward(x, dy, gam)
+    assert torch.equal(dx, want_dx)
+    for got, want in zip(partials.sum(0), (dg, db)):  # float32 sums in another order
+        assert_rel_l2(got, want, "d gamma, d beta", tol=1e-6)
 
 
 @pytest.mark.parametrize("grid,C,O,B,k", [((3, 5), 64, 256, 2, 3), ((16, 17), 256, 256, 1, 3), ((9, 30), 128, 512, 3, 5),
