@@ -256,6 +256,12 @@ int slice_softmax_backward(const pa_shape &s, const pa_params &p, const void *x_
                            const float *d_norm, void *tables, void *d_proj, void *d_z, float *dT_part, int num_cu,
                            hipStream_t st);
 int deslice_natural(const pa_shape &s, const void *w_pack, const void *tokp, void *out_x, int num_cu, hipStream_t st);
+// out_x and, further down, the whole hand-back on the float32 attended tokens (B, H, S, 32) instead of bf16 fragments
+int deslice_tokens(const pa_shape &s, const void *w_pack, const float *tokens, void *out_x, int num_cu, hipStream_t st);
+bool deslice_project_tokens_supported(const pa_shape &s);
+int deslice_project_tokens(const pa_shape &s, const void *blob, const void *w_pack, const float *tokens, void *y,
+                           const pa_block_tail *tail, int num_cu, hipStream_t st);
+bool float_tables(const pa_shape &s, bool plus);  // training multiplies with float32 tables and tokens, not bf16 ones
 bool point_backward_supported(const pa_shape &s);
 int64_t point_backward_grads(const pa_shape &s, bool plus);
 int64_t point_backward_workspace_bytes(const pa_shape &s, bool plus, int num_cu);

@@ -746,8 +746,10 @@ __global__ __launch_bounds__(64 * ((S + 31) / 32)) void slice_attention_kernel(c
 // operation and issues the next tile's loads right after the last use of the current ones, so every wait
 // counts exactly the younger operations.  MASKED = true: one tile per workgroup, the last `nfull` tiles of each batch: the
 // ragged one, or, where a workgroup per tile fits the chip, all of them in one launch (2 x 1 000 points: 5.9 us against 6.1 + 4.7).
+// SPLIT: tokp is the attended tokens themselves, float32 (B, H, S, 32); each tile is multiplied with bf16(tok') and with the
+// remainder, i.e. with 16 bits of a token (training of the layers that multiplied with float32 tokens before they came here).
 // ------------------------------------------------------------------------------------------------
-template <int C, int S, int TAIL, bool MASKED>
+template <int C, int S, int TAIL, bool MASKED, bool SPLIT>
 __global__ __launch_bounds__(C * 2) void deslice_project_kernel(const u32x4 *__restrict__ blob, const u32x4 *__restrict__ w_pack,
                                                                 const u32x4 *__restrict__ tokp, uint16_t *__restrict__ y,
                                                                 const uint16_t *__restrict__ residual,
@@ -762,7 +764,7 @@ __global__ __launch_bounds__(C * 2) void deslice_project_kernel(const u32x4 *__r
   constexpr int YS = C + 8;           // row stride (floats): rows 4 apart land 32 banks apart
   typedef uint32_t rowvec __attribute__((ext_vector_type(CPL / 2)));  // CPL bf16
   __shared__ u32x4 oxs[H * 2 * 64];
-  __shared__ u32x4 tps[H * NCH * 64];
+  __shared__ u32x4 tps[(SPLIT ? 2 : 1) * H * NCH * 64];  // SPLIT: the remainders behind
   __shared__ float ys[32 * YS];
   const BlobPlan bp = blob_plan(C, S);
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 31, g = lane >> 5;
@@ -821,7 +823,15 @@ __global__ __launch_bounds__(C * 2) void deslice_project_kernel(const u32x4 *__r
   while (true) {
     if (b != b_loaded) {  // workgroup-uniform: (re)load this batch's attended tokens
       __syncthreads();
-      for (int u = tid; u < H * NCH * 64; u += NT) tps[u] = tokp[b * (H * NCH * 64) + u];
+      for (int u = tid; u < H * NCH * 64; u += NT) {
+        if constexpr (SPLIT) {
+          const int ul = u & 63, f = u >> 6;  // fragment (head, 16 slices)
+          const float *src = reinterpret_cast<const float *>(tokp) + (b * (H * NCH) + f) * 512 + (ul & 31);
+          token_fragment(src, ul >> 5, tps[u], tps[H * NCH * 64 + u]);
+        } else {
+          tps[u] = tokp[b * (H * NCH * 64) + u];
+        }
+      }
       __syncthreads();
       b_loaded = b;
     }
@@ -835,6 +845,13 @@ __global__ __launch_bounds__(C * 2) void deslice_project_kernel(const u32x4 *__r
     for (int cq = 0; cq < NCH; cq += 2) {
       ox = mma(tps[(wave * NCH + cq) * 64 + lane], wcur[cq], ox);
       if (cq + 1 < NCH) ox2 = mma(tps[(wave * NCH + cq + 1) * 64 + lane], wcur[cq + 1 < NCH ? cq + 1 : 0], ox2);
+    }
+    if constexpr (SPLIT) {
+#pragma unroll
+      for (int cq = 0; cq < NCH; ++cq) {
+        f32x16 &o = NCH > 1 && cq % 2 ? ox2 : ox;
+        o = mma(tps[((H + wave) * NCH + cq) * 64 + lane], wcur[cq], o);
+      }
     }
     if constexpr (NCH > 1) {
 #pragma unroll
@@ -1278,7 +1295,7 @@ static int slice_reduce_s(const pa_shape &s, const void *w_pack, const void *fx_
   return launch_status();
 }
 
-template <int C, int S, int TAIL>
+template <int C, int S, int TAIL, bool SPLIT>
 static int deslice_project_t(const pa_shape &s, const void *blob, const void *w_pack, const void *tokp, void *y,
                              const pa_block_tail *tail, int num_cu, hipStream_t st) {
   const int64_t tpb = tiles_per_batch(s);
@@ -1295,7 +1312,7 @@ static int deslice_project_t(const pa_shape &s, const void *blob, const void *w_
     static int per_cu = 0;  // resident workgroups per CU for this instantiation
     if (per_cu == 0) {
       int nb = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, deslice_project_kernel<C, S, TAIL, false>, C * 2, 0) !=
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, deslice_project_kernel<C, S, TAIL, false, SPLIT>, C * 2, 0) !=
               hipSuccess || nb < 1)
         nb = 1;
       per_cu = nb;
@@ -1303,14 +1320,14 @@ static int deslice_project_t(const pa_shape &s, const void *blob, const void *w_
     const int64_t total = (int64_t)nfull * s.B;
     int64_t grid = (int64_t)num_cu * per_cu;
     if (grid > total) grid = total;
-    hipLaunchKernelGGL((deslice_project_kernel<C, S, TAIL, false>), dim3((unsigned)grid), dim3(C * 2), 0, st, bl, wp, tp,
+    hipLaunchKernelGGL((deslice_project_kernel<C, S, TAIL, false, SPLIT>), dim3((unsigned)grid), dim3(C * 2), 0, st, bl, wp, tp,
                        yo, res, gm, bt, eps, lo, s.N, (int)tpb, nfull, total);
     int rc = launch_status();
     if (rc) return rc;
   }
   if (ragged) {
     const int per = at_once ? (int)tpb : 1;
-    hipLaunchKernelGGL((deslice_project_kernel<C, S, TAIL, true>), dim3((unsigned)(s.B * per)), dim3(C * 2), 0, st, bl, wp, tp,
+    hipLaunchKernelGGL((deslice_project_kernel<C, S, TAIL, true, SPLIT>), dim3((unsigned)(s.B * per)), dim3(C * 2), 0, st, bl, wp, tp,
                        yo, res, gm, bt, eps, lo, s.N, (int)tpb, per, s.B * per);
     return launch_status();
   }
@@ -1348,14 +1365,27 @@ static int deslice_recompute_project_t(const pa_shape &s, const pa_params &p, co
   return PA_OK;
 }
 
+template <int C, int S, bool SPLIT>
+static int deslice_project_tails(const pa_shape &s, const void *blob, const void *w_pack, const void *tokp, void *y,
+                                 const pa_block_tail *tail, int num_cu, hipStream_t st) {
+  const bool has_res = tail && tail->residual, has_ln = tail && tail->ln_out;
+  if (has_res && has_ln) return deslice_project_t<C, S, 1, SPLIT>(s, blob, w_pack, tokp, y, tail, num_cu, st);
+  if (has_res) return deslice_project_t<C, S, 2, SPLIT>(s, blob, w_pack, tokp, y, tail, num_cu, st);
+  if (has_ln) return deslice_project_t<C, S, 3, SPLIT>(s, blob, w_pack, tokp, y, tail, num_cu, st);
+  return deslice_project_t<C, S, 0, SPLIT>(s, blob, w_pack, tokp, y, tail, num_cu, st);
+}
+
 template <int C, int S>
 static int deslice_project_cs(const pa_shape &s, const void *blob, const void *w_pack, const void *tokp, void *y,
                               const pa_block_tail *tail, int num_cu, hipStream_t st) {
-  const bool has_res = tail && tail->residual, has_ln = tail && tail->ln_out;
-  if (has_res && has_ln) return deslice_project_t<C, S, 1>(s, blob, w_pack, tokp, y, tail, num_cu, st);
-  if (has_res) return deslice_project_t<C, S, 2>(s, blob, w_pack, tokp, y, tail, num_cu, st);
-  if (has_ln) return deslice_project_t<C, S, 3>(s, blob, w_pack, tokp, y, tail, num_cu, st);
-  return deslice_project_t<C, S, 0>(s, blob, w_pack, tokp, y, tail, num_cu, st);
+  return deslice_project_tails<C, S, false>(s, blob, w_pack, tokp, y, tail, num_cu, st);
+}
+
+template <int C, int S>
+static int deslice_project_tokens_cs(const pa_shape &s, const void *blob, const void *w_pack, const float *tokens, void *y,
+                                     const pa_block_tail *tail, int num_cu, hipStream_t st) {
+  if constexpr (S <= 64) return deslice_project_tails<C, S, true>(s, blob, w_pack, tokens, y, tail, num_cu, st);
+  return PA_ERR_UNSUPPORTED;
 }
 
 template <int C>
@@ -1429,6 +1459,15 @@ int combine_attention(const pa_shape &s, const pa_params &p, const float *fx_bia
 int deslice_project(const pa_shape &s, const void *blob, const void *w_pack, const void *tokp, void *y,
                     const pa_block_tail *tail, int num_cu, hipStream_t st) {
   PA_DISPATCH_CS(deslice_project_cs, s, blob, w_pack, tokp, y, tail, num_cu, st);
+}
+
+// the same on the float32 attended tokens (B, H, S, 32); S = 128: both parts of its tokens leave no room in the LDS
+bool deslice_project_tokens_supported(const pa_shape &s) { return s.S <= 64 && (s.C == 128 || s.C == 256); }
+
+int deslice_project_tokens(const pa_shape &s, const void *blob, const void *w_pack, const float *tokens, void *y,
+                           const pa_block_tail *tail, int num_cu, hipStream_t st) {
+  if (!deslice_project_tokens_supported(s)) return PA_ERR_UNSUPPORTED;
+  PA_DISPATCH_CS(deslice_project_tokens_cs, s, blob, w_pack, tokens, y, tail, num_cu, st);
 }
 
 bool deslice_recompute_project_supported(const pa_shape &s) { return s.S == 128 && (s.C == 256 || s.C == 128); }

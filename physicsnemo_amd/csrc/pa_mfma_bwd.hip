@@ -22,8 +22,9 @@ namespace mfma {
 // deslice_natural_kernel: grid (G, B, head groups), one wave per head of the group; wave h walks the batch's tiles
 // g, g + G, ...
 //   out_x^T_h (32 d x 32 pts) = tok'^T_h (A: tokp fragments, registers) . w_h (B: w_pack chunks)
+// SPLIT: tokp is the float32 tokens (B, H, S, 32), multiplied as bf16 and remainder.
 // ------------------------------------------------------------------------------------------------
-template <int S>
+template <int S, bool SPLIT>
 __global__ __launch_bounds__(512) void deslice_natural_kernel(const u32x4 *__restrict__ w_pack,
                                                               const u32x4 *__restrict__ tokp,
                                                               uint16_t *__restrict__ out_x, int64_t N, int tpb, int H) {
@@ -31,9 +32,13 @@ __global__ __launch_bounds__(512) void deslice_natural_kernel(const u32x4 *__res
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 31, g = lane >> 5;
   const int h = blockIdx.z * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(tid >> 6);
   const int b = blockIdx.y;
-  u32x4 tp[NCH];
+  u32x4 tp[NCH], tl[SPLIT ? NCH : 1];
 #pragma unroll
-  for (int cq = 0; cq < NCH; ++cq) tp[cq] = tokp[(((int64_t)b * H + h) * NCH + cq) * 64 + lane];
+  for (int cq = 0; cq < NCH; ++cq) {
+    const int64_t f = ((int64_t)b * H + h) * NCH + cq;
+    if constexpr (SPLIT) token_fragment(reinterpret_cast<const float *>(tokp) + f * 512 + i, g, tp[cq], tl[cq]);
+    else tp[cq] = tokp[f * 64 + lane];
+  }
   for (int t = blockIdx.x; t < tpb; t += gridDim.x) {
     const int64_t gt = (int64_t)b * tpb + t;
     const u32x4 *wsrc = w_pack + ((gt * H + h) * NCH) * 64 + lane;
@@ -41,7 +46,11 @@ __global__ __launch_bounds__(512) void deslice_natural_kernel(const u32x4 *__res
 #pragma unroll
     for (int r = 0; r < 16; ++r) ox[r] = 0.f;
 #pragma unroll
-    for (int cq = 0; cq < NCH; ++cq) ox = mma(tp[cq], load_streaming(wsrc + cq * 64), ox);
+    for (int cq = 0; cq < NCH; ++cq) {
+      const u32x4 w = load_streaming(wsrc + cq * 64);
+      ox = mma(tp[cq], w, ox);
+      if constexpr (SPLIT) ox = mma(tl[SPLIT ? cq : 0], w, ox);
+    }
     const int64_t n = (int64_t)t * 32 + i;
     const bool ok = n < N;
     store_tile_natural(ox, out_x + ((int64_t)b * N + (ok ? n : 0)) * (H * 32) + h * 32, g, ok);
@@ -57,7 +66,7 @@ __global__ __launch_bounds__(512) void deslice_natural_kernel(const u32x4 *__res
 //            dnA[(st*2 + kk)]   = d num[32st + i][16kk + 8g + j]                   A of d w, second half of k
 //            dnT[cq]            = d num[16cq + rowmap(j, g)][i]                     A of d fx_mid
 // Slices >= S read as zero.  SPLIT tables carry the remainders t - bf16(t) in a second set of fragments behind each group,
-// so that products with them keep 16 bits of the table (point_split() says for which layers).
+// so that products with them keep 16 bits of the table (float_tables() says for which layers).
 // ------------------------------------------------------------------------------------------------
 struct BwdTablePlan {
   int st2, nch, group, nshared, nhead;  // fragments: of the two kinds, of a shared group, shared, per (b, h)
@@ -653,7 +662,8 @@ int64_t backward_tables_bytes(const pa_shape &s) {
   return (tp.shared_units + s.B * s.H * tp.per_head_units) * 16;
 }
 
-int deslice_natural(const pa_shape &s, const void *w_pack, const void *tokp, void *out_x, int num_cu, hipStream_t st) {
+template <bool SPLIT>
+static int deslice_natural_t(const pa_shape &s, const void *w_pack, const void *tokp, void *out_x, int num_cu, hipStream_t st) {
   const int waves = (int)(s.H < 8 ? s.H : 8);
   if (s.H % waves != 0) return PA_ERR_UNSUPPORTED;
   const int groups = (int)(s.H / waves);
@@ -664,13 +674,21 @@ int deslice_natural(const pa_shape &s, const void *w_pack, const void *tokp, voi
   uint16_t *ox = static_cast<uint16_t *>(out_x);
   const int tpb = (int)tiles_per_batch(s);
   switch (s.S) {
-    case 16: hipLaunchKernelGGL((deslice_natural_kernel<16>), grid, block, 0, st, wp, tp, ox, s.N, tpb, (int)s.H); break;
-    case 32: hipLaunchKernelGGL((deslice_natural_kernel<32>), grid, block, 0, st, wp, tp, ox, s.N, tpb, (int)s.H); break;
-    case 64: hipLaunchKernelGGL((deslice_natural_kernel<64>), grid, block, 0, st, wp, tp, ox, s.N, tpb, (int)s.H); break;
-    case 128: hipLaunchKernelGGL((deslice_natural_kernel<128>), grid, block, 0, st, wp, tp, ox, s.N, tpb, (int)s.H); break;
+    case 16: hipLaunchKernelGGL((deslice_natural_kernel<16, SPLIT>), grid, block, 0, st, wp, tp, ox, s.N, tpb, (int)s.H); break;
+    case 32: hipLaunchKernelGGL((deslice_natural_kernel<32, SPLIT>), grid, block, 0, st, wp, tp, ox, s.N, tpb, (int)s.H); break;
+    case 64: hipLaunchKernelGGL((deslice_natural_kernel<64, SPLIT>), grid, block, 0, st, wp, tp, ox, s.N, tpb, (int)s.H); break;
+    case 128: hipLaunchKernelGGL((deslice_natural_kernel<128, SPLIT>), grid, block, 0, st, wp, tp, ox, s.N, tpb, (int)s.H); break;
     default: return PA_ERR_UNSUPPORTED;
   }
   return launch_status();
+}
+
+int deslice_natural(const pa_shape &s, const void *w_pack, const void *tokp, void *out_x, int num_cu, hipStream_t st) {
+  return deslice_natural_t<false>(s, w_pack, tokp, out_x, num_cu, st);
+}
+
+int deslice_tokens(const pa_shape &s, const void *w_pack, const float *tokens, void *out_x, int num_cu, hipStream_t st) {
+  return deslice_natural_t<true>(s, w_pack, tokens, out_x, num_cu, st);
 }
 
 int slice_softmax_backward(const pa_shape &s, const pa_params &p, const void *x_mid, const void *fx_mid,
@@ -718,17 +736,17 @@ int64_t point_backward_grads(const pa_shape &s, bool plus) { return point_grads(
 // Irregular layers of 128 and 256 channels multiply with bf16 tables, all others with float32 ones kept as bf16 and its
 // remainder: at 512 channels and 128 slices, 4 096 points, plain bf16 tables leave d b_slice 1.6e-2, d W_slice 1.0e-2 and
 // d W_x 6.9e-3 from float64, the split ones 2.7e-3, 2.2e-3 and 2.5e-3 (as fma loops on float32 tables do).
-static bool point_split(const pa_shape &s, bool plus) { return plus || s.conv_k > 0 || s.C == 512; }
+bool float_tables(const pa_shape &s, bool plus) { return plus || s.conv_k > 0 || s.C == 512; }
 
 static int point_head_waves(const pa_shape &s, bool plus) {  // waves (heads) per workgroup
-  const int most = point_waves((int)s.S, plus, point_split(s, plus));
+  const int most = point_waves((int)s.S, plus, float_tables(s, plus));
   return (int)(s.H < most ? s.H : most);
 }
 
 // workgroups along the points: the chip filled once by the workgroups that fit it (8 waves of 256 or 4 of 512 registers
 // per CU), so that a workgroup's tables and its partial row are paid for once
 static int64_t point_groups(const pa_shape &s, bool plus, int num_cu) {
-  const int w = point_head_waves(s, plus), most = point_waves((int)s.S, plus, point_split(s, plus));
+  const int w = point_head_waves(s, plus), most = point_waves((int)s.S, plus, float_tables(s, plus));
   const int64_t resident = (int64_t)num_cu * (most / w), other = s.B * (s.H / w), tpb = tiles_per_batch(s);
   int64_t g = resident / other;
   if (g > tpb) g = tpb;
@@ -736,7 +754,7 @@ static int64_t point_groups(const pa_shape &s, bool plus, int num_cu) {
 }
 
 int64_t point_backward_workspace_bytes(const pa_shape &s, bool plus, int num_cu) {
-  const BwdTablePlan tp = bwd_table_plan((int)s.S, plus, point_split(s, plus));
+  const BwdTablePlan tp = bwd_table_plan((int)s.S, plus, float_tables(s, plus));
   const int64_t wgs = point_groups(s, plus, num_cu) * s.B * (s.H / point_head_waves(s, plus));
   return (tp.shared_units + s.B * s.H * tp.per_head_units) * 16 + wgs * point_backward_grads(s, plus) * 4;
 }
@@ -748,7 +766,7 @@ int point_backward(const pa_shape &s, const pa_params &p, const pa_plus_params *
                    const float *d_num, const float *d_norm, void *workspace, void *d_proj, float *grads, int num_cu,
                    hipStream_t st) {
   if (!point_backward_supported(s)) return PA_ERR_UNSUPPORTED;
-  const bool split = point_split(s, plus != nullptr);
+  const bool split = float_tables(s, plus != nullptr);
   const BwdTablePlan tp = bwd_table_plan((int)s.S, plus != nullptr, split);
   u32x4 *tabs = static_cast<u32x4 *>(workspace);
   const int64_t table_units = tp.shared_units + s.B * s.H * tp.per_head_units;

@@ -47,6 +47,20 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
   return __builtin_bit_cast(uint32_t, o);
 }
 
+// Operand fragment of 16 slices from float32 rows of 32 channels, `src` at the lane's channel of the first one: element j is
+// slice rowmap(j, g), as bf16 and as the bf16 remainder of that rounding.
+__device__ __forceinline__ void token_fragment(const float *src, int g, u32x4 &hi, u32x4 &lo) {
+  bf16x8 h, l;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float v = src[((j & 3) + 8 * (j >> 2) + 4 * g) * 32];
+    h[j] = (__bf16)v;
+    l[j] = (__bf16)(v - (float)h[j]);
+  }
+  hi = __builtin_bit_cast(u32x4, h);
+  lo = __builtin_bit_cast(u32x4, l);
+}
+
 // Four direct global -> LDS loads of 64 x 16 bytes each (no registers): the wave's lanes read sbase + 1024 q + 16 lane
 // (q = 0..3) and the data land at LDS byte address lds + 1024 q + 16 lane; the instruction offset advances the
 // global and the LDS address alike.  sbase and lds are wave-uniform.  The loads are asynchronous and counted by

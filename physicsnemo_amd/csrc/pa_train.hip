@@ -71,6 +71,17 @@ struct Scratch {
   int64_t work_bytes;
 };
 
+// how the forward hands the attended tokens back to the points
+enum class HandBack {
+  packed,  // kernel (d) on the bf16 tokens the slice attention packs
+  tokens,  // kernel (d) on the float32 tokens
+  apart    // out_x on the float32 tokens, out_linear, tail
+};
+static HandBack hand_back(const pa_shape &s, bool plus) {
+  if (!mfma::float_tables(s, plus)) return HandBack::packed;
+  return mfma::deslice_project_tokens_supported(s) ? HandBack::tokens : HandBack::apart;
+}
+
 static bool fused(const pa_shape &s, bool plus) { return !plus && mfma::supported(PA_BF16, s); }
 
 bool supported(const pa_shape &s, bool plus) {
@@ -117,11 +128,11 @@ static Scratch plan_scratch(const pa_shape &s, bool plus, int num_cu) {
     off += round_up(bytes);
     return at;
   };
-  p.blob = take(s.C <= 256 ? mfma::blob_bytes(s) : 0);
+  p.blob = take(hand_back(s, plus) != HandBack::apart ? mfma::blob_bytes(s) : 0);
   p.fx_pack = take(tiles * s.H * 2 * 1024);
   p.partials = take((forward_groups(s, plus, num_cu) + 1) * BHS * 33 * 4);
   p.tokp = take(mfma::tokp_bytes(s));
-  p.out_x = take(s.C <= 256 ? 0 : M * HD * 2);
+  p.out_x = take(hand_back(s, plus) == HandBack::apart ? M * HD * 2 : 0);
   p.total = off;
 
   off = 0;
@@ -192,6 +203,7 @@ int forward(const pa_shape &s, int weight_dtype, const pa_params &params, const 
         *norm = reinterpret_cast<float *>(sv + sp.norm), *tok_out = reinterpret_cast<float *>(sv + sp.tok_out);
   const int64_t G = forward_groups(s, pl, num_cu);
   const float *fx_bias = nullptr;
+  const HandBack how = hand_back(s, pl);
   if (fused(s, pl)) {
     if ((rc = mfma::pack_params(s, p, blob, st))) return rc;
     const bool one = mfma::fuse_reduce(s);
@@ -218,12 +230,15 @@ int forward(const pa_shape &s, int weight_dtype, const pa_params &params, const 
             : mfma::slice_softmax_pack(s, p, x_mid, w_pack, num_cu, st);
     if (rc) return rc;
     if ((rc = mfma::slice_reduce(s, w_pack, fx_pack, partials, st))) return rc;
-    if (s.C <= 256 && (rc = mfma::pack_out_linear(s, p.out_linear_weight, nullptr, p.out_linear_bias, blob, st))) return rc;
+    if (how != HandBack::apart && (rc = mfma::pack_out_linear(s, p.out_linear_weight, nullptr, p.out_linear_bias, blob, st)))
+      return rc;
   }
   if ((rc = mfma::combine_attention(s, p, fx_bias, partials, G, tok, norm, tok_out, tokp, st))) return rc;
-  if (s.C <= 256) return mfma::deslice_project(s, blob, w_pack, tokp, y, tail, num_cu, st);
-  if ((rc = mfma::deslice_natural(s, w_pack, tokp, ws + sc.out_x, num_cu, st))) return rc;
-  return general::out_linear(PA_BF16, s, p, ws + sc.out_x, y, st);
+  if (how == HandBack::packed) return mfma::deslice_project(s, blob, w_pack, tokp, y, tail, num_cu, st);
+  if (how == HandBack::tokens) return mfma::deslice_project_tokens(s, blob, w_pack, tok_out, y, tail, num_cu, st);
+  if ((rc = mfma::deslice_tokens(s, w_pack, tok_out, ws + sc.out_x, num_cu, st))) return rc;
+  if ((rc = general::out_linear(PA_BF16, s, p, ws + sc.out_x, y, st)) || !tail) return rc;
+  return general::residual_ln(PA_BF16, s, y, *tail, st);
 }
 
 int backward(const pa_shape &s, const pa_params &params, const pa_plus_params *plus, const void *x, const void *uniform,

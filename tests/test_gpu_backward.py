@@ -728,6 +728,34 @@ def test_bf16_blocks_with_fused_tails_train_like_separate_ones(C, S, B, N, grid)
         assert e_got <= 1.3 * e_apart, (e_got, e_apart)
 
 
+@pytest.mark.parametrize("C,S,B,grid", [(256, 64, 2, (21, 17)), (256, 64, 3, (64, 96)), (128, 16, 1, (3, 11)), (256, 32, 1, (8, 4)),
+                                        (128, 128, 2, (9, 30)), (256, 128, 1, (16, 20))])
+def test_structured_training_forward_with_and_without_the_block_tail(C, S, B, grid):
+    """The hand-back on float32 tokens with the residual and LayerNorm in the same call, at full and ragged tiles, several
+    batch elements, more tiles than workgroups, and at 128 slices, where it runs as separate kernels: against the same
+    layer followed by the residual add and LayerNorm in float64."""
+    announce("structured training forward", C, S, B, grid)
+    torch.manual_seed(S)
+    N, H = grid[0] * grid[1], C // 32
+    ref, hip = make_pair("structured2d", C, H, 32, S, spatial=grid, sharpen=3.0)
+    hip.train()
+    ln = torch.nn.LayerNorm(C).cuda()
+    with torch.no_grad():
+        ln.weight.add_(0.3 * torch.randn(C, device="cuda")), ln.bias.add_(0.3 * torch.randn(C, device="cuda"))
+        for m in (ref, hip):
+            m.out_linear.weight.copy_(m.out_linear.weight.bfloat16().float())
+    x, res = torch.randn(2, B, N, C, device="cuda").bfloat16()
+    y = hip(x).detach()
+    fx, normed = (t.detach() for t in hip.forward_block_with_grad(x, res, ln))
+    want = y.double() + res.double()
+    # the tail adds the residual to a result rounded once (2^-9 / sqrt(3) = 1.1e-3), or not at all, and rounds the sum
+    assert_rel_l2(fx, want, "y + residual", tol=3e-3)
+    assert_rel_l2(normed, torch.nn.functional.layer_norm(fx.double(), (C,), ln.weight.double(), ln.bias.double()), "LayerNorm",
+                  tol=3e-3)
+    if C * N <= 100_000:
+        assert_rel_l2(y, ref(x.float().cpu()), "y", tol=1e-2)
+
+
 def test_output_dropout_in_training_matches_the_reference_site():
     """The reference applies nn.Dropout to the layer output in training mode (physics_attention.py:499): kept entries
     are y / (1 - p), the rest zero, gradients flow through the kept entries only; eval mode is the identity."""
