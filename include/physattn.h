@@ -533,6 +533,10 @@ int pa_mlp_forward(int dtype, int64_t rows, int64_t C, int64_t F, const pa_mlp_p
 int pa_mlp_pack(int dtype, int64_t C, int64_t F, const pa_mlp_params *p, void *packed, int64_t packed_bytes, void *stream);
 int pa_mlp_forward_packed(int dtype, int64_t rows, int64_t C, int64_t F, const void *packed, const float *b1,
                           const float *b2, const void *u, void *y, const pa_block_tail *tail, void *stream);
+/* pa_mlp_forward_packed for training: GELU to float32 accuracy (4e-7) as the backward below takes it, where inference uses a
+ * form good to 2.6e-5.  bf16, C = 256. */
+int pa_mlp_train_forward(int dtype, int64_t rows, int64_t C, int64_t F, const void *packed, const float *b1, const float *b2,
+                         const void *u, void *y, const pa_block_tail *tail, void *stream);
 /* The hidden layer's part of the MLP's backward pass, from the layer's input and the output's gradient alone:
  *   act (rows, F) = gelu(w1 u + b1),  d_hidden (rows, F) = (w2^T dy) * gelu'(w1 u + b1);
  * w1 (F, C), w2 (C, F), u, dy (rows, C) and the results bf16, 16-byte aligned; b1 float32; b2 is not read.  The weight

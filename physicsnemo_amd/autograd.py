@@ -745,10 +745,10 @@ class MlpResidualFunction(torch.autograd.Function):
         packed = PF.mlp_pack(w1_16, w2_16)
         if ln_w is None:
             ctx.save_for_backward(x, w1_16, b1_32, w2_16)
-            return PF.mlp_forward_packed(x, packed, b1_32, b2_32, residual=residual)
+            return PF.mlp_forward_packed(x, packed, b1_32, b2_32, residual=residual, train=True)
         w32 = _aligned(ln_w.detach().float())
         y, normed = PF.mlp_forward_packed(x, packed, b1_32, b2_32, residual=residual, ln_weight=w32,
-                                          ln_bias=_aligned(ln_b.detach().float()), ln_eps=eps)
+                                          ln_bias=_aligned(ln_b.detach().float()), ln_eps=eps, train=True)
         ctx.save_for_backward(x, w1_16, b1_32, w2_16, y, w32)
         ctx.eps, ctx.ln_dtypes = eps, (ln_w.dtype, ln_b.dtype)
         return y, normed

@@ -1151,6 +1151,19 @@ int pa_mlp_forward_packed(int dtype, int64_t rows, int64_t C, int64_t F, const v
                           compute_units(), static_cast<hipStream_t>(stream));
 }
 
+int pa_mlp_train_forward(int dtype, int64_t rows, int64_t C, int64_t F, const void *packed, const float *b1, const float *b2,
+                         const void *u, void *y, const pa_block_tail *tail, void *stream) {
+  Range entry("pa_mlp_train_forward");
+  if (rows <= 0 || C <= 0 || F <= 0) return PA_ERR_DIMS;
+  if (dtype != PA_BF16 || !mlp_served(dtype, rows, C, F)) return PA_ERR_UNSUPPORTED;
+  if (!packed || !b1 || !b2 || !u || !y) return PA_ERR_NULL;
+  if (!aligned16(packed) || !aligned16(u) || !aligned16(y)) return PA_ERR_ALIGN;
+  int rc = check_tail(tail);
+  if (rc) return rc;
+  return pa::mlp::train_forward(rows, C, F, packed, b1, b2, u, y, tail_active(tail) ? tail : nullptr, compute_units(),
+                                static_cast<hipStream_t>(stream));
+}
+
 int64_t pa_mlp_backward_workspace_bytes(int dtype, int64_t rows, int64_t C, int64_t F) {
   if (rows <= 0 || C <= 0 || F <= 0) return PA_ERR_DIMS;
   if (dtype != PA_BF16 || rows > PA_MAX_ROWS || !pa::mlp::hidden_backward_supported(rows, C, F)) return PA_ERR_UNSUPPORTED;

@@ -51,16 +51,32 @@ __device__ __forceinline__ float gelu_logistic(float x) {
   return x * __builtin_amdgcn_rcpf(1.f + e);
 }
 
-// Phi(x) of the logistic form above, and the derivative of GELU from it: Phi(x) + x phi(x)
-__device__ __forceinline__ float gelu_logistic_phi(float x) {
-  const float x2 = fminf(x * x, 81.f);
-  float p = fmaf(-3.51902394e-04f * -2.f * kLog2e, x2, 3.70080200e-02f * -2.f * kLog2e);
-  p = fmaf(p, x2, 7.97505275e-01f * -2.f * kLog2e);
-  return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x * p));
+// Phi(x) = 1/2 (1 + erf(x / sqrt 2)) to float32 accuracy for the training kernels, and e^(-x^2 / 2), which the derivative of
+// GELU shares.  1 - Phi(a) = e^(-a^2 / 2) R(1 / (1 + 0.3 a)), a = |x|, R of degree 6 fitted to 0.5 erfcx(a / sqrt 2) for the
+// smallest largest relative error over 0 <= a <= 14: 1.9e-6, so the lower tail keeps its relative accuracy.  GELU is within
+// 3.9e-7 and its derivative within 1.0e-6 of the exact ones everywhere (0.5 x (1 + erff(..)) in float32: 3.9e-7), with two
+// transcendental instructions for both.
+__device__ __forceinline__ float gelu_gauss(float x) { return __builtin_amdgcn_exp2f(x * x * (-0.5f * kLog2e)); }
+__device__ __forceinline__ float gelu_ratio(float x) { return __builtin_amdgcn_rcpf(fmaf(0.3f, fabsf(x), 1.f)); }
+__device__ __forceinline__ float gelu_phi(float x, float e, float t) {  // e, t: the two above
+  float r = fmaf(-8.45932179e-02f, t, 2.40572734e-01f);
+  r = fmaf(r, t, -4.86443127e-02f);
+  r = fmaf(r, t, 1.64764373e-01f);
+  r = fmaf(r, t, 1.06704584e-01f);
+  r = fmaf(r, t, 1.21274687e-01f);
+  r = fmaf(r, t, -7.97878928e-05f);
+  const float q = e * r;
+  return x > 0.f ? 1.f - q : q;
 }
-__device__ __forceinline__ float gelu_grad_from_phi(float x, float phi) {
-  return fmaf(x * 0.3989422804014327f, __builtin_amdgcn_exp2f(x * x * (-0.5f * kLog2e)), phi);
+struct GeluParts {
+  float phi, e;
+};
+__device__ __forceinline__ GeluParts gelu_parts(float x) {
+  const float e = gelu_gauss(x);
+  return {gelu_phi(x, e, gelu_ratio(x)), e};
 }
+__device__ __forceinline__ float gelu_fit(float x) { return x * gelu_parts(x).phi; }
+__device__ __forceinline__ float gelu_grad(float x, const GeluParts &p) { return fmaf(x * 0.3989422804014327f, p.e, p.phi); }
 
 // the derivative of gelu_erf: Phi(v) + v phi(v)
 __device__ __forceinline__ float gelu_erf_grad(float v) {

@@ -312,6 +312,9 @@ struct InputLn {
 bool input_ln_supported(int dtype, int64_t rows, int64_t C, int64_t F);
 int forward(int64_t rows, int64_t C, int64_t F, const void *blob, const float *b1, const float *b2, const void *u,
             void *y, const pa_block_tail *tail, const InputLn &in, int num_cu, hipStream_t st);
+// the same with GELU to float32 accuracy (C = 256)
+int train_forward(int64_t rows, int64_t C, int64_t F, const void *blob, const float *b1, const float *b2, const void *u,
+                  void *y, const pa_block_tail *tail, int num_cu, hipStream_t st);
 // backward of the hidden layer (pa_mlp_bwd.hip): act = gelu(W1 u + b1), dh = (W2^T dy) * gelu'(W1 u + b1), (rows, F) bf16
 bool hidden_backward_supported(int64_t rows, int64_t C, int64_t F);
 int64_t hidden_backward_blob_bytes(int64_t C, int64_t F);

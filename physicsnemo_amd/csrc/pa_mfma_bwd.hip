@@ -441,10 +441,10 @@ __global__ __launch_bounds__((point_waves(S, PLUS, SPLIT) * 64)) void point_back
         hd[st] = mma_shared(1, st * 2 + 0, xm[0], hd[st]);
         hd[st] = mma_shared(1, st * 2 + 1, xm[1], hd[st]);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) a2 = fmaf(w2l[32 * st + rowmap(r, g)], gelu_logistic(hd[st][r]), a2);
+        for (int r = 0; r < 16; ++r) a2 = fmaf(w2l[32 * st + rowmap(r, g)], gelu_fit(hd[st][r]), a2);
       }
       a2 = half_sum(a2) + b2;
-      traw = t_raw + gelu_logistic(a2);
+      traw = t_raw + gelu_fit(a2);
       it = 1.f / bf16_bits_to_f32(f32_to_bf16_bits(fmaxf(traw, 0.01f)));  // the forward rounds it to bf16
     }
     f32x16 z[ST], dw[ST];
@@ -569,9 +569,10 @@ __global__ __launch_bounds__((point_waves(S, PLUS, SPLIT) * 64)) void point_back
       for (int st = 0; st < ST; ++st)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const float v = hd[st][r], phi = gelu_logistic_phi(v);
-          dw2[st][r] = fmaf(d_a2, v * phi, dw2[st][r]);
-          hd[st][r] = d_a2 * w2l[32 * st + rowmap(r, g)] * gelu_grad_from_phi(v, phi);
+          const float v = hd[st][r];
+          const GeluParts p = gelu_parts(v);
+          dw2[st][r] = fmaf(d_a2, v * p.phi, dw2[st][r]);
+          hd[st][r] = d_a2 * w2l[32 * st + rowmap(r, g)] * gelu_grad(v, p);
         }
 #pragma unroll
       for (int cq = 0; cq < NCH; ++cq) dzp[cq] = (cq & 1) ? pack_half<1>(hd[cq >> 1]) : pack_half<0>(hd[cq >> 1]);

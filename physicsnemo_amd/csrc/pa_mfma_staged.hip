@@ -106,7 +106,8 @@ __global__ __launch_bounds__(512) void slice_softmax_pack_kernel(const uint16_t 
 //   w        = softmax_s((logits[s] - log(-log(u[s] + 1e-8) + 1e-8)) / temp)             u: the caller's U[0,1) samples
 // `uniform` (B, N, H, S) bf16 in natural layout: a lane reads its slices (runs of four) with 8-byte loads.
 // ------------------------------------------------------------------------------------------------
-// SPLIT: both weights with their bf16 remainders (training; inference multiplies with the rounded weights)
+// SPLIT: both weights with their bf16 remainders and GELU to float32 accuracy (training; inference multiplies with the
+// rounded weights and takes the logistic form)
 template <int S, bool SPLIT>
 __global__ __launch_bounds__(512) void slice_softmax_pack_plus_kernel(
     const uint16_t *__restrict__ x_mid, const uint16_t *__restrict__ uniform, const float *__restrict__ w_slice,
@@ -162,10 +163,10 @@ __global__ __launch_bounds__(512) void slice_softmax_pack_plus_kernel(
         hd = mma(w1l[((q * ST + st) * 2 + 1) * 64 + lane], xm1, hd);
       }
 #pragma unroll
-      for (int r = 0; r < 16; ++r) a2 = fmaf(w2l[32 * st + rowmap(r, g)], gelu_logistic(hd[r]), a2);
+      for (int r = 0; r < 16; ++r) a2 = fmaf(w2l[32 * st + rowmap(r, g)], SPLIT ? gelu_fit(hd[r]) : gelu_logistic(hd[r]), a2);
     }
     a2 = half_sum(a2) + b2;
-    const float temp = bf16_bits_to_f32(f32_to_bf16_bits(fmaxf(temp_h + gelu_logistic(a2), 0.01f)));
+    const float temp = bf16_bits_to_f32(f32_to_bf16_bits(fmaxf(temp_h + (SPLIT ? gelu_fit(a2) : gelu_logistic(a2)), 0.01f)));
     const float sc = kLog2e * __builtin_amdgcn_rcpf(temp);
     // logits + Gumbel noise
     const uint16_t *urow = uniform + m * HS + h * S;

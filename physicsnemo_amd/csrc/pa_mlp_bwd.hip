@@ -52,8 +52,9 @@ __global__ __launch_bounds__(256) void hidden_backward_pack_kernel(const uint16_
 // Rows past M repeat row M - 1 and write the same values to the same place, so that the number of stores in flight,
 // which the wait at a slot's start counts, is the same for every wave.
 // splits: the hidden units are independent of each other, so short inputs spread them over the chip.
-// Bound by its stores behind the matrix and vector work (4 C + 4 F bytes per row): 262 144 rows, F = 1024: 391 us; without
-// the stores 309; with 64-byte pieces of rows leaving after every slot 492, with ordinary instead of streaming stores 436.
+// Bound by its stores behind the matrix and vector work (4 C + 4 F bytes per row): 262 144 rows, F = 1024: 415 us.  With
+// GELU in the logistic form, good to 2.6e-5, it was 391; of those, without the stores 309, with 64-byte pieces of rows
+// leaving after every slot 492, with ordinary instead of streaming stores 436.
 // ---------------------------------------------------------------------------------------------------------------
 template <int C>
 __global__ __launch_bounds__(512) void hidden_backward_kernel(const u32x4 *__restrict__ blob, const float *__restrict__ b1,
@@ -92,11 +93,13 @@ __global__ __launch_bounds__(512) void hidden_backward_kernel(const u32x4 *__res
   int odd = 0;
   auto activate = [&](auto k_) {
     constexpr int k = decltype(k_)::value, q = k >> 2;
-    const float x = hprev[k], phi = gelu_logistic_phi(x), d = dprev[k] * gelu_grad_from_phi(x, phi);
+    const float x = hprev[k];
+    const GeluParts p = gelu_parts(x);
+    const float d = dprev[k] * gelu_grad(x, p);
     if constexpr (k % 2 == 0) {
-      geven = x * phi, deven = d;
+      geven = x * p.phi, deven = d;
     } else {
-      gp[(k >> 1) & 1] = pack2(geven, x * phi);
+      gp[(k >> 1) & 1] = pack2(geven, x * p.phi);
       dp[(k >> 1) & 1] = pack2(deven, d);
     }
     if constexpr (k % 4 == 3) {

@@ -438,8 +438,9 @@ def mlp_input_ln_supported(dtype: torch.dtype, rows: int, C: int, F: int) -> boo
     return bool(_lib.load().pa_mlp_input_ln_query(_lib.PA_BF16, rows, C, F))
 
 
-def mlp_forward_packed(u, packed, b1, b2, residual=None, ln_weight=None, ln_bias=None, ln_eps=1e-5, in_ln=None):
-    """mlp_forward with the weights already in operand order (mlp_pack); b1 (F), b2 (C) float32.
+def mlp_forward_packed(u, packed, b1, b2, residual=None, ln_weight=None, ln_bias=None, ln_eps=1e-5, in_ln=None, train=False):
+    """mlp_forward with the weights already in operand order (mlp_pack); b1 (F), b2 (C) float32.  train: GELU to float32
+    accuracy (bfloat16 rows of 256 channels, see mlp_backward).
 
     in_ln = (weight, bias, eps), float32: the rows of u are normalised by the kernel on their way in, i.e. the result is
     w2 . gelu(w1 . LayerNorm(u) + b1) + b2 [+ residual] (mlp_input_ln_supported)."""
@@ -457,9 +458,10 @@ def mlp_forward_packed(u, packed, b1, b2, residual=None, ln_weight=None, ln_bias
                                                 b2.data_ptr(), byref(cin), u.data_ptr(), y.data_ptr(), byref(tail),
                                                 _lib.current_stream_ptr(u.device)), "pa_mlp_forward_packed_ln")
     else:
-        _lib.check(lib.pa_mlp_forward_packed(_lib.dtype_code(u.dtype), rows, C, F, packed.data_ptr(), b1.data_ptr(),
-                                             b2.data_ptr(), u.data_ptr(), y.data_ptr(), byref(tail),
-                                             _lib.current_stream_ptr(u.device)), "pa_mlp_forward_packed")
+        call = lib.pa_mlp_train_forward if train else lib.pa_mlp_forward_packed
+        _lib.check(call(_lib.dtype_code(u.dtype), rows, C, F, packed.data_ptr(), b1.data_ptr(), b2.data_ptr(), u.data_ptr(),
+                        y.data_ptr(), byref(tail), _lib.current_stream_ptr(u.device)),
+                   "pa_mlp_train_forward" if train else "pa_mlp_forward_packed")
     return y if ln_out is None else (y, ln_out)
 
 

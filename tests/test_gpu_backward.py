@@ -634,6 +634,30 @@ def test_mlp_residual_block(rows, F):
     assert_rel_l2(gx.detach(), x64.grad, "dx, create_graph", tol=1e-2)
 
 
+def test_gelu_of_the_training_mlp_keeps_its_tail():
+    """The hidden layer at known values over [-9, 9]: GELU and its derivative, forward and backward, are the exact ones
+    rounded to bf16 once (2^-8 of a value at most), far into the lower tail; a fit that is good to 2.6e-5 absolutely is off by
+    a fifth at -4."""
+    announce("GELU of the training MLP")
+    C = F = 256
+    h = torch.linspace(-9, 9, F, device="cuda")
+    rows = 300
+    u = torch.randn(rows, C, device="cuda").bfloat16()
+    w1, eye = torch.zeros(F, C, device="cuda", dtype=torch.bfloat16), torch.eye(C, F, device="cuda").bfloat16()
+    zero = torch.zeros(C, device="cuda")
+    h64 = h.double().requires_grad_(True)
+    want = h64 * 0.5 * torch.erfc(-h64 / 2 ** 0.5)  # erfc keeps the relative accuracy of the tail
+    (slope,) = torch.autograd.grad(want.sum(), h64)
+    want = want.detach()
+    residual = torch.zeros(rows, C, device="cuda", dtype=torch.bfloat16)
+    y = PF.mlp_forward_packed(u, PF.mlp_pack(w1, eye), h, zero, residual=residual, train=True)
+    act, dh = PF.mlp_backward(u, torch.ones(rows, C, device="cuda", dtype=torch.bfloat16), w1, h, eye)
+    for got, exact, slack in ((y, want, 0.0), (act, want, 0.0), (dh, slope, 1.1e-6)):  # the slope passes through zero
+        err = (got.double() - exact).abs()
+        # beside the rounding: the fit's 2e-6 and the exponent's x^2 2^-24 of a value; 1 - Phi is formed in float32
+        assert (err <= 2.0 ** -8 * 1.01 * exact.abs() + slack).all(), (err / exact.abs()).max()
+
+
 @pytest.mark.parametrize("next_norm", [False, True])
 def test_mlp_residual_block_differentiates_twice(next_norm):
     """Gradients of a function of the gradient of a bf16 block's MLP, by its input and every parameter of the Linears and of
