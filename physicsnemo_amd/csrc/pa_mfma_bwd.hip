@@ -296,6 +296,7 @@ __global__ __launch_bounds__(S > 64 ? 256 : 512) void slice_softmax_backward_mfm
 //       bf16 weights instead costs 2 S bytes per point and head, the recomputation none that shows);
 //   dz = (w / T) (dw - sum_s w dw);  dT -= sum dz z / T
 //   d x_mid^T (32 x pts) = W_slice^T . dz^T;  d fx_mid^T = d num^T . w         B = bf16 tiles straight from registers
+//       (SPLIT: dz, and d a1 below, as bf16 and remainder too: 16 bits on both sides)
 //   d W_slice (S x 32) += dz^T . x_mid,  d b_slice += sum dz:  both operands turned around by an exact MFMA product with
 //       0/1 selection matrices (lanes <-> slices / channels, k = points), accumulated in registers over the whole kernel:
 //       d z itself never reaches memory.
@@ -389,6 +390,11 @@ __global__ __launch_bounds__((point_waves(S, PLUS, SPLIT) * 64)) void point_back
   auto mma_shared = [&](int group, int f, u32x4 v, f32x16 acc) {  // W_slice (group 0), W1 (1): ST2 straight, NCH turned
     acc = mma(wsh[(group * GRP + f) * 64 + lane], v, acc);
     if constexpr (SPLIT) acc = mma(wsh[(group * GRP + ST2 + NCH + f) * 64 + lane], v, acc);
+    return acc;
+  };
+  // SPLIT: shared fragment f . what bf16 leaves over of eight registers of v, the third term of the product of both
+  auto mma_rest = [&](int group, int f, const f32x16 &v, int half, f32x16 acc) {
+    if constexpr (SPLIT) acc = mma(wsh[(group * GRP + f) * 64 + lane], half ? pack_half_rest<1>(v) : pack_half_rest<0>(v), acc);
     return acc;
   };
   const float t_raw = a.temperature[h], inv_t = 1.f / clamp_temperature(t_raw);
@@ -528,6 +534,7 @@ __global__ __launch_bounds__((point_waves(S, PLUS, SPLIT) * 64)) void point_back
 #pragma unroll
     for (int cq = 0; cq < NCH; ++cq) {
       dxm = mma_shared(0, ST2 + cq, dzp[cq], dxm);
+      dxm = mma_rest(0, ST2 + cq, dw[cq >> 1], cq & 1, dxm);
       if constexpr (PLUS) dxm = mma_head(2 * ST2 + cq, wq[cq], dxm);
       else dfm = mma_head(2 * ST2 + cq, wq[cq], dfm);
     }
@@ -577,7 +584,10 @@ __global__ __launch_bounds__((point_waves(S, PLUS, SPLIT) * 64)) void point_back
 #pragma unroll
       for (int cq = 0; cq < NCH; ++cq) dzp[cq] = (cq & 1) ? pack_half<1>(hd[cq >> 1]) : pack_half<0>(hd[cq >> 1]);
 #pragma unroll
-      for (int cq = 0; cq < NCH; ++cq) dxm = mma_shared(1, ST2 + cq, dzp[cq], dxm);
+      for (int cq = 0; cq < NCH; ++cq) {
+        dxm = mma_shared(1, ST2 + cq, dzp[cq], dxm);
+        dxm = mma_rest(1, ST2 + cq, hd[cq >> 1], cq & 1, dxm);
+      }
       accumulate(dzp, dw1, csum1);
     }
     uint16_t *pr = a.d_proj + row * (PLUS ? HD : 2 * HD) + h * 32;

@@ -36,6 +36,15 @@ __device__ __forceinline__ u32x4 pack_half(const f32x16 &v, float scale = 1.f) {
   return __builtin_bit_cast(u32x4, o);
 }
 
+// the same for what pack_half leaves over: v - bf16(v)
+template <int HALF>
+__device__ __forceinline__ u32x4 pack_half_rest(const f32x16 &v) {
+  bf16x8 o;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) o[j] = (__bf16)(v[8 * HALF + j] - (float)(__bf16)v[8 * HALF + j]);
+  return __builtin_bit_cast(u32x4, o);
+}
+
 __device__ __forceinline__ uint16_t to_bf16_bits(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 
 // 2 floats -> 2 bf16 (round to nearest even), the first in the low half

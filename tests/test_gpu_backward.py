@@ -558,6 +558,31 @@ def test_point_stages_of_the_bf16_backward_agree(C, S, B, N):
     assert_rel_l2(d_temp, want_temp, "d temperature", tol=3e-2)
 
 
+@pytest.mark.parametrize("C,S,grid", [(256, 64, (20, 33)), (128, 16, (9, 7)), (512, 128, (16, 20)), (256, 32, (8, 4))])
+def test_point_backward_multiplies_float32_gradients(C, S, grid):
+    """d x_mid = d z W_slice of the structured layers from given rows: d z does not lose bits on its way into the product, so
+    the error against float64 is the rounding of the result alone (bf16: 1.7e-3 of a value in the mean square); d z rounded
+    to bf16 first adds as much again, and more where its terms cancel."""
+    announce("point backward, float32 d z", C, S, grid)
+    torch.manual_seed(S)
+    _, hip = make_pair("structured2d", C, C // 32, 32, S, spatial=grid, sharpen=2.0)
+    x = torch.zeros(1, grid[0] * grid[1], C, device="cuda", dtype=torch.bfloat16)
+    dims, kp = hip.layer_dims(x), hip.kernel_params(torch.bfloat16, x.device)
+    N, H = dims.N, dims.H
+    x_mid, fx_mid, g = torch.randn(3, 1, N, C, device="cuda").bfloat16()
+    tok, d_num = torch.randn(2, 1, H, S, 32, device="cuda")
+    d_norm = torch.randn(1, H, S, device="cuda")
+    d_proj, *_ = PF.point_backward(x_mid, fx_mid, g, tok, d_num, d_norm, kp, dims)
+    heads = lambda t: t.double().view(N, H, 32)
+    ws, bs = kp["in_project_slice_weight"].double().view(S, 32), kp["in_project_slice_bias"].double()
+    temp = kp["temperature"].double().clamp(0.5, 5.0).view(1, H, 1)
+    w = torch.softmax((heads(x_mid) @ ws.t() + bs) / temp, -1)
+    dw = (torch.einsum("nhd,hsd->nhs", heads(g), tok[0].double()) +
+          torch.einsum("nhd,hsd->nhs", heads(fx_mid), d_num[0].double()) + d_norm.double())
+    dz = w / temp * (dw - (w * dw).sum(-1, keepdim=True))
+    assert_rel_l2(d_proj[0, :, :C].reshape(N, H, 32), dz @ ws, "d x_mid", tol=1.8e-3)
+
+
 @pytest.mark.parametrize("dtype,rows,C", [(torch.bfloat16, 1003, 256), (torch.float32, 31, 64)])
 def test_layernorm_backward_partial_sums(dtype, rows, C):
     """pa_layernorm_backward leaves the groups' shares of d gamma and d beta to the caller; their sum and dx are those of
