@@ -384,14 +384,15 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(SumArgs a) {
 // token_grad_kernel: what the layer's output gradient says about the slice tokens and out_linear, from the sums
 // P[b][h S + s][c] = sum_n w[n, h, s] dy[n, c] (the packed product above) instead of from per-point d out_x and out_x:
 //   d tok'[b, h, s, d] = sum_c P[b, h, s, c] W_out[c, 32 h + d]              workgroups 0 .. B H ceil(S / 32) - 1
-//   d W_out[c, 32 h + d] = sum_b sum_s P[b, h, s, c] tok'[b, h, s, d]        the others, one per (h, 32 rows c)
+//   d W_out[c, 32 h + d] = sum_b sum_s P[b, h, s, c] tok'[b, h, s, d]        the others, one per (`cb` batch elements, h,
+//                                                                            32 rows c): a partial result per `cb` elements
 // Four waves per 32 x 32 result tile on fp32 MFMA, each a quarter of the reduction, added up in order through LDS.  Bound
 // by latency (P is a few hundred KB): the quarters' loads are all in flight at once, which takes 60 us (one wave per
 // tile) to 15 us at B = 1, S = 64, C = 256.
 // ------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void token_grad_kernel(const float *__restrict__ P, const uint16_t *__restrict__ w_out,
                                                          const float *__restrict__ out_token, float *__restrict__ d_token,
-                                                         float *__restrict__ d_w_out, int B, int H, int S, int C) {
+                                                         float *__restrict__ d_w_out, int B, int H, int S, int C, int cb) {
   typedef float f32x4 __attribute__((ext_vector_type(4)));
   __shared__ float part[3][16][64];
   const int lane = threadIdx.x & 63, i = lane & 31, g = lane >> 5;
@@ -401,7 +402,8 @@ __global__ __launch_bounds__(256) void token_grad_kernel(const float *__restrict
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.f;
   const bool to_token = (int)blockIdx.x < first;
-  const int e = blockIdx.x - first, st = blockIdx.x % ST, bh = blockIdx.x / ST, h = to_token ? bh % H : e % H, c0 = e / H * 32;
+  const int rest = blockIdx.x - first, per = H * (C / 32), chunk = to_token ? 0 : rest / per, e = rest - chunk * per;
+  const int st = blockIdx.x % ST, bh = blockIdx.x / ST, h = to_token ? bh % H : e % H, c0 = e / H * 32;
   if (to_token) {
     const int s = 32 * st + i, cw = C / 4;
     const float *row = P + ((int64_t)bh * S + (s < S ? s : S - 1)) * C + wave * cw + 4 * g;
@@ -415,7 +417,8 @@ __global__ __launch_bounds__(256) void token_grad_kernel(const float *__restrict
     }
   } else {
     const int sw = S / 4;
-    for (int b = 0; b < B; ++b) {
+    const int b_end = (chunk + 1) * cb < B ? (chunk + 1) * cb : B;
+    for (int b = chunk * cb; b < b_end; ++b) {
       const int64_t at = ((int64_t)b * H + h) * S + wave * sw + g;
       const float *p = P + at * C + c0 + i, *tk = out_token + at * 32 + i;
 #pragma unroll 8
@@ -433,7 +436,7 @@ __global__ __launch_bounds__(256) void token_grad_kernel(const float *__restrict
   for (int r = 0; r < 16; ++r) {
     const float v = ((acc[r] + part[0][r][lane]) + part[1][r][lane]) + part[2][r][lane];
     const int row = mfma::rowmap(r, g);
-    if (!to_token) d_w_out[(int64_t)(c0 + row) * HD + 32 * h + i] = v;
+    if (!to_token) d_w_out[((int64_t)chunk * C + c0 + row) * HD + 32 * h + i] = v;
     else if (32 * st + row < S) d_token[((int64_t)bh * S + 32 * st + row) * 32 + i] = v;
   }
 }
@@ -578,40 +581,86 @@ static int64_t output_chunks(const pa_shape &s, int num_cu) {  // row chunks per
   return g < 1 ? 1 : g;
 }
 
-int64_t output_backward_workspace_bytes(const pa_shape &s, int num_cu) {
-  const int64_t G = output_chunks(s, num_cu), n = s.H * s.S * s.C;
-  return (s.B * n * (G + 1) + s.B * G * s.C) * 4;
+// The sums P take n = H S C floats per batch element whatever its number of points, so many small clouds go through in
+// groups that fill the chip once (128 at C = 256, S = 64; up to 64 MB of P), with no copy of P where a batch element is one
+// chunk; and d W_out is formed from `cb` elements per workgroup, 32 partial results at most.  512 clouds of 64 points, 256 / 64:
+// 338 us; all of P at once, copied, and one workgroup walking all clouds 2 731 us.
+struct OutputPlan {
+  int64_t G, Bg, cb, parts, n;                         // chunks and elements per group, elements per d W_out part, parts
+  int64_t P, partials, sums, dw, total;                // floats into the workspace
+};
+static OutputPlan output_plan(const pa_shape &s, int num_cu) {
+  OutputPlan p{};
+  const int64_t HS = s.H * s.S, tiles = ((HS + 255) / 256) * ((s.C + 255) / 256);
+  p.G = output_chunks(s, num_cu), p.n = HS * s.C;
+  p.cb = (s.B + 31) / 32 > 4 ? (s.B + 31) / 32 : 4;
+  p.parts = (s.B + p.cb - 1) / p.cb;
+  p.Bg = (num_cu / tiles + p.cb - 1) / p.cb * p.cb;  // whole parts
+  if (p.Bg < p.cb) p.Bg = p.cb;
+  if (p.Bg > s.B) p.Bg = s.B;
+  p.partials = p.Bg * p.n;
+  p.sums = p.partials + (p.G > 1 ? p.Bg * p.G * p.n : 0);
+  p.dw = p.sums + s.B * p.G * s.C;
+  p.total = p.dw + (p.parts > 1 ? p.parts * s.C * s.H * 32 : 0);
+  return p;
 }
+
+int64_t output_backward_workspace_bytes(const pa_shape &s, int num_cu) { return output_plan(s, num_cu).total * 4; }
 
 // dy (B, N, C) bf16, w_pack and out_token of the forward, w_out (C, H*32) bf16 -> d tok' (B,H,S,32), d W_out, d b_out
 int output_backward(const pa_shape &s, const void *w_pack, const void *dy, const float *out_token, const void *w_out,
                     void *workspace, float *d_out_token, float *d_w_out, float *d_b_out, int num_cu, hipStream_t st) {
-  const int64_t G = output_chunks(s, num_cu), HS = s.H * s.S, n = HS * s.C;
-  float *P = static_cast<float *>(workspace), *partials = P + s.B * n, *sums = partials + s.B * G * n;
+  const OutputPlan p = output_plan(s, num_cu);
+  const int64_t HS = s.H * s.S, tok = HS * 32, HD = s.H * 32, ST = (s.S + 31) / 32;
+  float *ws = static_cast<float *>(workspace), *P = ws + p.P, *partials = p.G > 1 ? ws + p.partials : P, *sums = ws + p.sums,
+        *dw = p.parts > 1 ? ws + p.dw : d_w_out;
   Args a{};
-  a.B = static_cast<const uint16_t *>(dy);
-  a.pack = static_cast<const u32x4 *>(w_pack);
   a.ldb = (int)s.C, a.OA = (int)HS, a.OB = (int)s.C;
   a.M = s.N, a.tpb = (int)((s.N + 31) / 32), a.tile_units = (int)(HS / 16 * 64);
-  a.per = (int)((a.tpb + G - 1) / G);
+  a.per = (int)((a.tpb + p.G - 1) / p.G);
   a.grid = grid_taps(nullptr);
-  a.chunks = (int)G, a.batches = (int)s.B;
+  a.chunks = (int)p.G;
   a.ny = (int)((HS + 255) / 256), a.nz = (int)((s.C + 255) / 256);
-  a.partials = partials, a.col_sums = sums;
+  a.partials = partials;
   const size_t lds = (size_t)kStages * kStageBytes;
   int rc = allow_dynamic_lds(wgrad_kernel<2>, lds);
   if (rc) return rc;
-  hipLaunchKernelGGL(wgrad_kernel<2>, dim3((unsigned)((s.B * G * a.ny * a.nz + 7) / 8 * 8)), dim3(512), lds, st, a);
-  if ((rc = launch_status())) return rc;
+  for (int64_t b0 = 0; b0 < s.B; b0 += p.Bg) {
+    const int64_t nb = s.B - b0 < p.Bg ? s.B - b0 : p.Bg;
+    a.B = static_cast<const uint16_t *>(dy) + b0 * s.N * s.C;
+    a.pack = static_cast<const u32x4 *>(w_pack) + b0 * a.tpb * a.tile_units;
+    a.batches = (int)nb;
+    a.col_sums = sums + b0 * p.G * s.C;
+    hipLaunchKernelGGL(wgrad_kernel<2>, dim3((unsigned)((nb * p.G * a.ny * a.nz + 7) / 8 * 8)), dim3(512), lds, st, a);
+    if ((rc = launch_status())) return rc;
+    if (p.G > 1) {
+      SumArgs sa{};
+      sa.src[0] = partials, sa.dst[0] = P, sa.n[0] = p.n, sa.G[0] = (int)p.G, sa.taps = 1;
+      sa.blocks0 = (p.n + 31) / 32;
+      int64_t blocks = sa.blocks0;
+      if (p.parts == 1) {  // nothing else is to be added up: d b_out here
+        sa.src[1] = sums, sa.dst[1] = d_b_out, sa.n[1] = s.C, sa.G[1] = (int)(s.B * p.G);
+        blocks += (s.C + 31) / 32;
+      }
+      hipLaunchKernelGGL(sum_partials_kernel, dim3((unsigned)blocks, (unsigned)nb), dim3(256), 0, st, sa);
+      if ((rc = launch_status())) return rc;
+    }
+    const int64_t wgs = nb * s.H * ST + s.H * (s.C / 32) * ((nb + p.cb - 1) / p.cb);
+    hipLaunchKernelGGL(token_grad_kernel, dim3((unsigned)wgs), dim3(256), 0, st, P, static_cast<const uint16_t *>(w_out),
+                       out_token + b0 * tok, d_out_token + b0 * tok, dw + b0 / p.cb * s.C * HD, (int)nb, (int)s.H, (int)s.S,
+                       (int)s.C, (int)p.cb);
+    if ((rc = launch_status())) return rc;
+  }
+  if (p.parts == 1 && p.G > 1) return PA_OK;
   SumArgs sa{};
-  sa.src[0] = partials, sa.dst[0] = P, sa.n[0] = n, sa.G[0] = (int)G, sa.taps = 1;
-  sa.blocks0 = (n + 31) / 32;
-  sa.src[1] = sums, sa.dst[1] = d_b_out, sa.n[1] = s.C, sa.G[1] = (int)(s.B * G);
-  hipLaunchKernelGGL(sum_partials_kernel, dim3((unsigned)(sa.blocks0 + (s.C + 31) / 32), (unsigned)s.B), dim3(256), 0, st, sa);
-  if ((rc = launch_status())) return rc;
-  const int64_t wgs = s.B * s.H * ((s.S + 31) / 32) + s.H * (s.C / 32);
-  hipLaunchKernelGGL(token_grad_kernel, dim3((unsigned)wgs), dim3(256), 0, st, P, static_cast<const uint16_t *>(w_out),
-                     out_token, d_out_token, d_w_out, (int)s.B, (int)s.H, (int)s.S, (int)s.C);
+  sa.src[0] = sums, sa.dst[0] = d_b_out, sa.n[0] = s.C, sa.G[0] = (int)(s.B * p.G), sa.taps = 1;
+  sa.blocks0 = (s.C + 31) / 32;
+  int64_t blocks = sa.blocks0;
+  if (p.parts > 1) {
+    sa.src[1] = dw, sa.dst[1] = d_w_out, sa.n[1] = s.C * HD, sa.G[1] = (int)p.parts;
+    blocks += (s.C * HD + 31) / 32;
+  }
+  hipLaunchKernelGGL(sum_partials_kernel, dim3((unsigned)blocks), dim3(256), 0, st, sa);
   return launch_status();
 }
 

@@ -2,6 +2,7 @@
 finite differences in test_oracle_closed_forms.py).  Bars: fp32 gradients rtol 1e-4 with atol = 1e-4 * max|ref|
 per tensor; bf16 gradients rel-L2 <= 3e-2 against the fp32 reference gradients."""
 import copy
+import ctypes
 
 import numpy as np
 import pytest
@@ -299,6 +300,37 @@ def test_bf16_training_gradients_keep_float32_tables(variant, C, S, B, N, grid):
     want, got = run(ref, x.double(), dy.double(), u.double()), run(hip, x.cuda(), dy.cuda(), u.cuda())
     for name in want:
         assert_rel_l2(got[name], want[name], name, tol=1e-2 if want[name].numel() < 16 else 5e-3)
+
+
+@pytest.mark.parametrize("C,S,B,N", [(256, 64, 5, 70), (256, 64, 130, 33), (128, 16, 300, 20), (512, 128, 37, 31),
+                                     (256, 32, 9, 2100)])
+def test_many_clouds_in_one_training_batch(C, S, B, N):
+    """The gradients that come from sums per batch element where those go through in groups, partly filled ones among them,
+    and d W_out is formed in parts: against float64.  The workspace holds one group's sums."""
+    announce("many clouds", C, S, B, N)
+    H = C // 32
+    ref, hip = make_pair("irregular", C, H, 32, S)
+    with torch.no_grad():
+        for m in (ref, hip):
+            for w in (m.in_project_x.weight, m.in_project_fx.weight, m.out_linear.weight):
+                w.copy_(w.bfloat16().float())
+    ref, hip = ref.double().cuda().train(), hip.train()
+    x, dy = torch.randn(2, B, N, C, device="cuda").bfloat16()
+
+    def run(m, x, dy):
+        x = x.clone().requires_grad_(True)
+        m(x).backward(dy)
+        return {"x": x.grad, **{n: p.grad for n, p in m.named_parameters()}}
+
+    want, got = run(ref, x.double(), dy.double()), run(hip, x, dy)
+    # d W_out = dy^T out_x: the weights' bf16 rounding averages out over the points, as for d W_qkv behind the tokens
+    for name in ("out_linear.weight", "out_linear.bias", "qkv_project.weight"):
+        assert_rel_l2(got[name], want[name], name, tol=2e-3)
+    for name in ("x", "in_project_x.weight", "in_project_fx.weight", "in_project_slice.weight"):
+        assert_rel_l2(got[name], want[name], name, tol=2e-2)
+    dims = hip.layer_dims(x)
+    floats = _lib.load().pa_output_backward_workspace_bytes(ctypes.byref(dims.c())) / 4
+    assert floats <= 2 * 256 * 256 * 256 + B * C * 256 + 33 * C * C
 
 
 def test_mfma_deslice_natural_layout():
