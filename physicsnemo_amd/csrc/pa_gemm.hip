@@ -631,7 +631,6 @@ struct ConvTile {  // waves: two along the rows, WC along the outputs; a wave st
   static constexpr int RT = sizeof(T) == 2 ? 2 : 1, WC = sizeof(T) == 2 ? 4 : 2, kWaves = 2 * WC;
   static constexpr int kRows = 64 * RT, kOut = 64 * WC, kStageBytes = (kRows + kOut) * 128, KB = 128 / (int)sizeof(T);
 };
-__device__ const uint32_t kZeroUnit[4] = {0u, 0u, 0u, 0u};
 
 template <typename T>
 __global__ __launch_bounds__((ConvTile<T>::kWaves * 64)) void conv_gemm_kernel(GemmArgs a) {
@@ -679,7 +678,7 @@ __global__ __launch_bounds__((ConvTile<T>::kWaves * 64)) void conv_gemm_kernel(G
     for (int k = 0; k < 2; ++k) {
       const bool ok = ((unsigned)(ci[k] + fu - pad) < (unsigned)a.gh) & ((unsigned)(cj[k] + fv - pad) < (unsigned)a.gw) &
                       ((unsigned)(cl[k] + fz - pad_d) < (unsigned)gd);
-      const T *p = ok ? base[k] + shift : reinterpret_cast<const T *>(kZeroUnit);
+      const T *p = ok ? base[k] + shift : reinterpret_cast<const T *>(&mfma::kZeroUnit);
       mfma::load_unit_to_lds(p, dst + (16 * wave + 8 * k) * 128);
     }
 #pragma unroll

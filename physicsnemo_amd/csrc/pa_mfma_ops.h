@@ -86,6 +86,10 @@ __device__ __forceinline__ void load_4k_to_lds(const void *sbase, unsigned lane1
       : "memory");
 }
 
+// what such a load reads where a convolution's neighbour lies outside the grid; a vector type, so on a 16-byte boundary
+__device__ const u32x4 kZeroUnit = {0u, 0u, 0u, 0u};
+static_assert(alignof(u32x4) == 16, "one 16-byte load");
+
 // One such load with a 16-byte address per lane: lane l's unit lands at dst + 16 l.
 __device__ __forceinline__ void load_unit_to_lds(const void *p, unsigned dst) {  // lane l's 16 bytes land at dst + 16 l
   asm volatile(

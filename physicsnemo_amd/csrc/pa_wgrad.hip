@@ -19,8 +19,6 @@ using mfma::load_unit_to_lds;
 using mfma::u32x2;
 using mfma::u32x4;
 
-__device__ const uint32_t kZeroUnit[4] = {0u, 0u, 0u, 0u};
-
 // ------------------------------------------------------------------------------------------------
 // wgrad_kernel: a workgroup (8 waves, 4 along A's columns x 2 along B's, wave tile 64 x 128) owns a 256 x 256 block of P
 // for its chunk of rows.  32 rows of both operands (32 KB) are one stage; four stages form a ring in LDS, filled by
@@ -135,7 +133,7 @@ __global__ __launch_bounds__(512) void wgrad_kernel(Args a) {
         if constexpr (CONV) {
           const int ii = ci[k] + du, jj = cj[k] + dv, ll = cl[k] + dz;
           const bool in = m < a.M && (unsigned)ii < (unsigned)gh && (unsigned)jj < (unsigned)gw && (unsigned)ll < (unsigned)gd;
-          pb[k] = in ? pb[k] + shift * a.ldb : reinterpret_cast<const uint16_t *>(kZeroUnit);
+          pb[k] = in ? pb[k] + shift * a.ldb : reinterpret_cast<const uint16_t *>(&mfma::kZeroUnit);
           cl[k] += sl;
           cj[k] += sj;
           ci[k] += si;
