@@ -201,9 +201,13 @@ __global__ __launch_bounds__(512) void wgrad_kernel(Args a) {
       for (int u = 0; u < 2; ++u) af[u] = PACKED ? packed_operand(at, ks, wa + 32 * u) : operand(at, ks, wa + 32 * u);
 #pragma unroll
       for (int v = 0; v < 4; ++v) bf[v] = operand(bt, ks, wb + 32 * v);
-      if (!PACKED && valid < 32) {  // the last rows of all: those beyond M hold a repeated row and must not count
+      if (valid < 32) {  // the last rows of all: those beyond M hold a repeated row and must not count, infinite or not
 #pragma unroll
-        for (int u = 0; u < 2; ++u) af[u] = masked(af[u], ks, valid);
+        for (int v = 0; v < 4; ++v) bf[v] = masked(bf[v], ks, valid);
+        if constexpr (!PACKED) {  // the packed weights are zero there
+#pragma unroll
+          for (int u = 0; u < 2; ++u) af[u] = masked(af[u], ks, valid);
+        }
       }
 #pragma unroll
       for (int u = 0; u < 2; ++u)
@@ -212,7 +216,7 @@ __global__ __launch_bounds__(512) void wgrad_kernel(Args a) {
       if (sums) {
         if constexpr (PACKED) {
 #pragma unroll
-          for (int v = 0; v < 4; ++v) add_columns(valid < 32 ? masked(bf[v], ks, valid) : bf[v], csum[v]);
+          for (int v = 0; v < 4; ++v) add_columns(bf[v], csum[v]);
         } else {
 #pragma unroll
           for (int u = 0; u < 2; ++u) add_columns(af[u], csum[u]);

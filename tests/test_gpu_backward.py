@@ -302,6 +302,23 @@ def test_bf16_training_gradients_keep_float32_tables(variant, C, S, B, N, grid):
         assert_rel_l2(got[name], want[name], name, tol=1e-2 if want[name].numel() < 16 else 5e-3)
 
 
+@pytest.mark.parametrize("rows", [1, 33, 2015])
+@pytest.mark.parametrize("ca,cb", [(256, 256), (512, 128), (256, 16)])
+def test_weight_gradient_with_an_infinite_last_row(rows, ca, cb):
+    """An infinity in the last row of a ragged count stays one in the column it belongs to: the rows that only fill the last
+    tile do not turn it into a NaN, nor do they reach other columns."""
+    announce("infinite last row", rows, ca, cb)
+    a, b = (1 + torch.rand(rows, c, device="cuda").bfloat16() for c in (ca, cb))
+    for inf_in_a in (False, True):
+        x, y = a.clone(), b.clone()
+        (x if inf_in_a else y)[-1, 3] = float("inf")
+        got, sums = PF.cols_gemm(x, y, col_sums=True)
+        want = torch.zeros(ca, cb, dtype=torch.bool, device="cuda")
+        (want[3] if inf_in_a else want[:, 3]).fill_(True)
+        assert not got.isnan().any() and torch.equal(got.isinf(), want)
+        assert not sums.isnan().any() and sums.isinf().sum() == int(inf_in_a)
+
+
 @pytest.mark.parametrize("C,S,B,N", [(256, 64, 5, 70), (256, 64, 130, 33), (128, 16, 300, 20), (512, 128, 37, 31),
                                      (256, 32, 9, 2100)])
 def test_many_clouds_in_one_training_batch(C, S, B, N):
