@@ -195,20 +195,18 @@ def _train_params(names, params, device):
 
 def _layer_train_forward(ctx, x, uniform, dims, names, params):
     """Forward of a bf16 layer with 32-wide heads in one library call; ctx keeps what the backward call reads."""
-    x, kp = _aligned(x), _train_params(names, params, x.device)
-    uniform = None if uniform is None else _aligned(uniform)
-    y, saved = PF.layer_train_forward(x, uniform, kp, dims)
-    ctx.save_for_backward(x, uniform, saved, *params)
-    ctx.dims, ctx.names, ctx.kparams = dims, names, kp
+    x, uniform = _aligned(x), None if uniform is None else _aligned(uniform)
+    y, saved = PF.layer_train_forward(x, uniform, _train_params(names, params, x.device), dims)
+    ctx.save_for_backward(x, uniform, saved)
+    ctx.dims, ctx.param_like = dims, [(n, p.shape, p.dtype) for n, p in zip(names, params)]
     return y
 
 
-def _layer_train_backward(ctx, dy, first_param):
-    x, uniform, saved, *params = ctx.saved_tensors
-    dx, grads = PF.layer_train_backward(x, uniform, _aligned(dy.to(x.dtype)), saved, ctx.kparams, ctx.dims,
-                                        ctx.needs_input_grad[0])
-    return dx, tuple(grads[n].view(p.shape).to(p.dtype) if need else None
-                     for n, p, need in zip(ctx.names, params, ctx.needs_input_grad[first_param:]))
+def _layer_train_backward(ctx, x, uniform, dy, saved, need):
+    """(dx, the parameters' gradients); need: which of them are wanted."""
+    dx, grads = PF.layer_train_backward(x, uniform, dy, saved, ctx.dims, ctx.needs_input_grad[0])
+    return dx, tuple(grads[n].view(shape).to(dtype) if wanted else None
+                     for (n, shape, dtype), wanted in zip(ctx.param_like, need))
 
 
 class PhysicsAttentionMfmaFunction(torch.autograd.Function):
@@ -221,7 +219,8 @@ class PhysicsAttentionMfmaFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy):
-        dx, grads = _layer_train_backward(ctx, dy, 3)
+        x, uniform, saved = ctx.saved_tensors
+        dx, grads = _layer_train_backward(ctx, x, uniform, _aligned(dy.to(x.dtype)), saved, ctx.needs_input_grad[3:])
         return (dx, None, None) + grads
 
 
@@ -266,24 +265,24 @@ class LayerResidualNormFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, residual, dims, ln_w, ln_b, eps, *params):
         ctx.set_materialize_grads(False)
-        kp = _train_params(_LAYER_PARAMS, params, x.device)
         w32 = _aligned(ln_w.detach().float())
-        y, saved, normed = PF.layer_train_forward(x, None, kp, dims, residual, w32, _aligned(ln_b.detach().float()), eps)
-        ctx.save_for_backward(x, saved, y, w32, *params)
-        ctx.dims, ctx.kparams, ctx.eps, ctx.ln_dtypes = dims, kp, eps, (ln_w.dtype, ln_b.dtype)
+        y, saved, normed = PF.layer_train_forward(x, None, _train_params(_LAYER_PARAMS, params, x.device), dims, residual, w32,
+                                                  _aligned(ln_b.detach().float()), eps)
+        ctx.save_for_backward(x, saved, y, w32)
+        ctx.dims, ctx.param_like = dims, [(n, p.shape, p.dtype) for n, p in zip(_LAYER_PARAMS, params)]
+        ctx.eps, ctx.ln_dtypes = eps, (ln_w.dtype, ln_b.dtype)
         _keep_parameters(ctx, ln_w)
         return y, normed
 
     @staticmethod
     def backward(ctx, d_y, d_normed):
-        x, saved, y, w32, *params = ctx.saved_tensors
+        x, saved, y, w32 = ctx.saved_tensors
         need = ctx.needs_input_grad
         d, dg, db = _through_norm(ctx, y, w32, d_y, d_normed)
         if d is None:
-            return (None,) * (6 + len(params))
-        dx, grads = PF.layer_train_backward(x, None, d, saved, ctx.kparams, ctx.dims, need[0])
-        return (dx, d if need[1] else None, None, dg, db, None) + tuple(
-            grads[n].view(p.shape).to(p.dtype) if wanted else None for n, p, wanted in zip(_LAYER_PARAMS, params, need[6:]))
+            return (None,) * (6 + len(ctx.param_like))
+        dx, grads = _layer_train_backward(ctx, x, None, d, saved, need[6:])
+        return (dx, d if need[1] else None, None, dg, db, None) + grads
 
 
 class PhysicsAttentionPlusMfmaFunction(torch.autograd.Function):
@@ -295,7 +294,8 @@ class PhysicsAttentionPlusMfmaFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy):
-        dx, grads = _layer_train_backward(ctx, dy, 3)
+        x, uniform, saved = ctx.saved_tensors
+        dx, grads = _layer_train_backward(ctx, x, uniform, _aligned(dy.to(x.dtype)), saved, ctx.needs_input_grad[3:])
         return (dx, None, None) + grads
 
 
@@ -739,7 +739,7 @@ class MlpResidualFunction(torch.autograd.Function):
     def forward(ctx, x, residual, w1, b1, w2, b2, ln_w, ln_b, eps):
         ctx.set_materialize_grads(False)
         w1_16, w2_16 = (_aligned(w.detach().to(torch.bfloat16)) for w in (w1, w2))
-        b1_32, b2_32 = (_aligned(b.detach().float()) for b in (b1, b2))
+        b1_32, b2_32 = _aligned(b1.detach().to(torch.float32, copy=True)), _aligned(b2.detach().float())  # b1: read again
         ctx.param_dtypes = tuple(p.dtype for p in (w1, b1, w2, b2))
         _keep_parameters(ctx, w1, b1, w2, *(() if ln_w is None else (ln_w,)))
         packed = PF.mlp_pack(w1_16, w2_16)

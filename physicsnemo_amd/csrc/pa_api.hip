@@ -981,15 +981,15 @@ int pa_layer_train_backward(const pa_shape *shape, const pa_params *p, const pa_
                             const void *uniform, const void *dy, const void *saved, void *dx, float *grads, void *workspace,
                             int64_t workspace_bytes, void *stream) {
   Range entry("pa_layer_train_backward");
+  (void)p;
   int rc = check_layer_train(shape, plus ? 1 : 0);
   if (rc) return rc;
-  if ((rc = check_train_params(p, plus))) return rc;
   if (!x || (plus && !uniform) || !dy || !saved || !grads || !workspace) return PA_ERR_NULL;
   if (!aligned16(x) || !aligned16(uniform) || !aligned16(dy) || !aligned16(saved) || !aligned16(dx) || !aligned16(grads) ||
       !aligned16(workspace))
     return PA_ERR_ALIGN;
   if (workspace_bytes < pa::train::backward_workspace_bytes(*shape, plus != nullptr, compute_units())) return PA_ERR_WORKSPACE;
-  return pa::train::backward(*shape, *p, plus, x, uniform, dy, saved, dx, grads, workspace, compute_units(),
+  return pa::train::backward(*shape, plus != nullptr, x, uniform, dy, saved, dx, grads, workspace, compute_units(),
                              static_cast<hipStream_t>(stream));
 }
 

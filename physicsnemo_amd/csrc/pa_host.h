@@ -102,8 +102,8 @@ int64_t backward_workspace_bytes(const pa_shape &s, bool plus, int num_cu);
 int64_t grad_floats(const pa_shape &s, bool plus);
 int forward(const pa_shape &s, int weight_dtype, const pa_params &p, const pa_plus_params *plus, const void *x,
             const void *uniform, void *y, const pa_block_tail *tail, void *saved, void *workspace, int num_cu, hipStream_t st);
-int backward(const pa_shape &s, const pa_params &p, const pa_plus_params *plus, const void *x, const void *uniform,
-             const void *dy, const void *saved, void *dx, float *grads, void *workspace, int num_cu, hipStream_t st);
+int backward(const pa_shape &s, bool plus, const void *x, const void *uniform, const void *dy, const void *saved, void *dx,
+             float *grads, void *workspace, int num_cu, hipStream_t st);
 }  // namespace train
 
 namespace general {

@@ -16,11 +16,17 @@ namespace train {
 // torch's layout, 32 x 32 tiles turned around through LDS (grid x: tiles, y: taps):
 //   w_in   [projection][o][tap][c]          w_in_t  [c][taps - 1 - tap][projection HD + o]   (the transposed convolution)
 //   w_out  [c][o]                           w_out_t [o][c]
+// and, in the last kSmallBlocks workgroups, the float32 parameters side by side: the backward pass reads these copies, so that
+// the parameters themselves may change between the two passes.
 // ------------------------------------------------------------------------------------------------
+constexpr int kSmallBlocks = 8, kSmallParams = 10;
 struct PrepareArgs {
   const void *w[3];  // in_project_x, in_project_fx (or NULL), out_linear
   uint16_t *w_in, *w_in_t, *w_out, *w_out_t;
   int C, HD, taps, nproj;
+  const float *small[kSmallParams];
+  int at[kSmallParams + 1], n[kSmallParams];  // where each begins among the copies, its length
+  float *copies;
 };
 
 template <typename T>
@@ -29,8 +35,16 @@ __global__ __launch_bounds__(256) void prepare_weights_kernel(PrepareArgs a) {
   const int t = threadIdx.x, col = t & 31, row0 = t >> 5;
   const int tc = a.C / 32, th = a.HD / 32, per = th * tc;
   int id = blockIdx.x;
-  const int which = id / per;  // 0 .. nproj - 1: an input projection, nproj: out_linear
+  const int which = id / per;  // 0 .. nproj - 1: an input projection, nproj: out_linear, beyond: float32 parameters
   id -= which * per;
+  if (which > a.nproj) {
+    if (blockIdx.y > 0) return;
+    const int k = (int)blockIdx.x - (a.nproj + 1) * per;
+#pragma unroll
+    for (int m = 0; m < kSmallParams; ++m)
+      for (int e = k * 256 + t; a.small[m] && e < a.n[m]; e += kSmallBlocks * 256) a.copies[a.at[m] + e] = a.small[m][e];
+    return;
+  }
   const bool out = which == a.nproj;
   const int tap = blockIdx.y;
   if (out && tap > 0) return;
@@ -63,7 +77,7 @@ static int64_t round_up(int64_t v) { return (v + 255) / 256 * 256; }
 
 // ---- buffer plans ----
 struct Saved {  // kept from the forward to the backward pass
-  int64_t w_in, w_in_t, w_out, w_out_t, w_pack, tok, norm, tok_out, x_mid, fx_mid, total;
+  int64_t w_in, w_in_t, w_out, w_out_t, small, w_pack, tok, norm, tok_out, x_mid, fx_mid, total;
 };
 struct Scratch {
   int64_t blob, fx_pack, partials, tokp, out_x, total;                                     // forward
@@ -90,6 +104,19 @@ bool supported(const pa_shape &s, bool plus) {
   return backward::attention_lds_bytes(s) <= kMaxLdsBytes;
 }
 
+// where the float32 parameters begin among their copies, each on a 16-byte boundary: in_project_slice weight and bias,
+// temperature, qkv_project, the projections' biases, then the four of proj_temperature
+static void small_plan(const pa_shape &s, bool plus, int (&at)[kSmallParams + 1], int *len = nullptr) {
+  const int HD = (int)s.H * 32, S = (int)s.S;
+  const int n[kSmallParams] = {S * 32, S,           (int)s.H,       3 * 32 * 32,  HD, plus ? 0 : HD,
+                               plus ? S * 32 : 0, plus ? S : 0, plus ? S : 0, plus ? 1 : 0};
+  at[0] = 0;
+  for (int m = 0; m < kSmallParams; ++m) {
+    at[m + 1] = at[m] + (n[m] + 3) / 4 * 4;
+    if (len) len[m] = n[m];
+  }
+}
+
 static Saved plan_saved(const pa_shape &s, bool plus) {
   const int64_t HD = s.H * 32, taps = grid_taps(&s).taps, np = plus ? 1 : 2, tiles = s.B * mfma::tiles_per_batch(s);
   Saved p{};
@@ -103,6 +130,9 @@ static Saved plan_saved(const pa_shape &s, bool plus) {
   p.w_in_t = take(np * HD * taps * s.C * 2);
   p.w_out = take(HD * s.C * 2);
   p.w_out_t = take(HD * s.C * 2);
+  int at[kSmallParams + 1];
+  small_plan(s, plus, at);
+  p.small = take((int64_t)at[kSmallParams] * 4);
   p.w_pack = take(tiles * s.H * (s.S / 16) * 1024);
   p.tok = take(s.B * s.H * s.S * 32 * 4);
   p.norm = take(s.B * s.H * s.S * 4);
@@ -170,14 +200,25 @@ int64_t grad_floats(const pa_shape &s, bool plus) {
   return np * HD * s.C * grid_taps(&s).taps + np * HD + s.C * HD + s.C + 3 * 32 * 32 + mfma::point_backward_grads(s, plus);
 }
 
-// `p` for the kernels behind prepare_weights: the bf16 copies in the saved buffer
-static pa_params prepared(const pa_shape &s, const pa_params &p, bool plus, char *sv, const Saved &sp) {
-  pa_params q = p;
-  q.in_project_x_weight = sv + sp.w_in;
-  q.in_project_fx_weight = plus ? nullptr : sv + sp.w_in + s.H * 32 * s.C * grid_taps(&s).taps * 2;
-  q.out_linear_weight = sv + sp.w_out;
-  q.in_project_x_scale = q.in_project_fx_scale = q.out_linear_scale = nullptr;
-  return q;
+// the parameters for the kernels behind prepare_weights: the copies in the saved buffer
+struct Prepared {
+  pa_params p;
+  pa_plus_params q;
+};
+static Prepared prepared(const pa_shape &s, bool plus, char *sv, const Saved &sp) {
+  int at[kSmallParams + 1];
+  small_plan(s, plus, at);
+  const float *small = reinterpret_cast<const float *>(sv + sp.small);
+  Prepared r{};
+  r.p.in_project_x_weight = sv + sp.w_in;
+  r.p.in_project_fx_weight = plus ? nullptr : sv + sp.w_in + s.H * 32 * s.C * grid_taps(&s).taps * 2;
+  r.p.out_linear_weight = sv + sp.w_out;
+  r.p.in_project_slice_weight = small + at[0], r.p.in_project_slice_bias = small + at[1];
+  r.p.temperature = small + at[2], r.p.qkv_project_weight = small + at[3];
+  r.p.in_project_x_bias = small + at[4], r.p.in_project_fx_bias = plus ? nullptr : small + at[5];
+  r.q.proj_temperature_0_weight = small + at[6], r.q.proj_temperature_0_bias = small + at[7];
+  r.q.proj_temperature_2_weight = small + at[8], r.q.proj_temperature_2_bias = small + at[9];
+  return r;
 }
 
 int forward(const pa_shape &s, int weight_dtype, const pa_params &params, const pa_plus_params *plus, const void *x,
@@ -192,12 +233,27 @@ int forward(const pa_shape &s, int weight_dtype, const pa_params &params, const 
   pa.w_in = reinterpret_cast<uint16_t *>(sv + sp.w_in), pa.w_in_t = reinterpret_cast<uint16_t *>(sv + sp.w_in_t);
   pa.w_out = reinterpret_cast<uint16_t *>(sv + sp.w_out), pa.w_out_t = reinterpret_cast<uint16_t *>(sv + sp.w_out_t);
   pa.C = (int)s.C, pa.HD = (int)(s.H * 32), pa.taps = taps, pa.nproj = pl ? 1 : 2;
-  const dim3 grid((unsigned)((pa.nproj + 1) * (s.C / 32) * s.H), (unsigned)taps);
+  const float *small[kSmallParams] = {params.in_project_slice_weight,
+                                      params.in_project_slice_bias,
+                                      params.temperature,
+                                      params.qkv_project_weight,
+                                      params.in_project_x_bias,
+                                      pl ? nullptr : params.in_project_fx_bias,
+                                      pl ? plus->proj_temperature_0_weight : nullptr,
+                                      pl ? plus->proj_temperature_0_bias : nullptr,
+                                      pl ? plus->proj_temperature_2_weight : nullptr,
+                                      pl ? plus->proj_temperature_2_bias : nullptr};
+  for (int m = 0; m < kSmallParams; ++m) pa.small[m] = small[m];
+  small_plan(s, pl, pa.at, pa.n);
+  pa.copies = reinterpret_cast<float *>(sv + sp.small);
+  const dim3 grid((unsigned)((pa.nproj + 1) * (s.C / 32) * s.H + kSmallBlocks), (unsigned)taps);
   if (weight_dtype == PA_F32) hipLaunchKernelGGL(prepare_weights_kernel<float>, grid, dim3(256), 0, st, pa);
   else hipLaunchKernelGGL(prepare_weights_kernel<bf16>, grid, dim3(256), 0, st, pa);
   int rc = launch_status();
   if (rc) return rc;
-  const pa_params p = prepared(s, params, pl, sv, sp);
+  Prepared prep = prepared(s, pl, sv, sp);
+  prep.p.out_linear_bias = params.out_linear_bias;  // read by the forward pass only
+  const pa_params &p = prep.p;
   void *blob = ws + sc.blob, *fx_pack = ws + sc.fx_pack, *tokp = ws + sc.tokp, *w_pack = sv + sp.w_pack;
   float *partials = reinterpret_cast<float *>(ws + sc.partials), *tok = reinterpret_cast<float *>(sv + sp.tok),
         *norm = reinterpret_cast<float *>(sv + sp.norm), *tok_out = reinterpret_cast<float *>(sv + sp.tok_out);
@@ -226,7 +282,7 @@ int forward(const pa_shape &s, int weight_dtype, const pa_params &params, const 
     a.pack_tpb = (int)mfma::tiles_per_batch(s), a.pack_heads = (int)s.H;
     if (!gemm::serves(a, pl ? 1 : 2, 2)) return PA_ERR_UNSUPPORTED;
     if ((rc = gemm::launch(a, pl ? 1 : 2, PA_BF16, st))) return rc;
-    rc = pl ? mfma::slice_softmax_pack_plus(s, p, *plus, x_mid, uniform, w_pack, true, num_cu, st)
+    rc = pl ? mfma::slice_softmax_pack_plus(s, p, prep.q, x_mid, uniform, w_pack, true, num_cu, st)
             : mfma::slice_softmax_pack(s, p, x_mid, w_pack, num_cu, st);
     if (rc) return rc;
     if ((rc = mfma::slice_reduce(s, w_pack, fx_pack, partials, st))) return rc;
@@ -241,13 +297,13 @@ int forward(const pa_shape &s, int weight_dtype, const pa_params &params, const 
   return general::residual_ln(PA_BF16, s, y, *tail, st);
 }
 
-int backward(const pa_shape &s, const pa_params &params, const pa_plus_params *plus, const void *x, const void *uniform,
-             const void *dy, const void *saved, void *dx, float *grads, void *workspace, int num_cu, hipStream_t st) {
-  const bool pl = plus != nullptr;
+int backward(const pa_shape &s, bool pl, const void *x, const void *uniform, const void *dy, const void *saved, void *dx,
+             float *grads, void *workspace, int num_cu, hipStream_t st) {
   const Saved sp = plan_saved(s, pl);
   const Scratch sc = plan_scratch(s, pl, num_cu);
   char *sv = static_cast<char *>(const_cast<void *>(saved)), *ws = static_cast<char *>(workspace);
-  const pa_params p = prepared(s, params, pl, sv, sp);
+  const Prepared prep = prepared(s, pl, sv, sp);
+  const pa_params &p = prep.p;
   const int64_t HD = s.H * 32, M = s.B * s.N, taps = grid_taps(&s).taps, np = pl ? 1 : 2;
   float *d_w_in = grads, *d_b_in = d_w_in + np * HD * s.C * taps, *d_w_out = d_b_in + np * HD, *d_b_out = d_w_out + s.C * HD,
         *d_wqkv = d_b_out + s.C, *small = d_wqkv + 3 * 32 * 32;
@@ -269,7 +325,8 @@ int backward(const pa_shape &s, const pa_params &params, const pa_plus_params *p
     x_mid = ws + sc.x_mid, fx_mid = ws + sc.fx_mid;
     if ((rc = general::project_inputs(PA_BF16, s, p, x, ws + sc.x_mid, ws + sc.fx_mid, st))) return rc;
   }
-  if ((rc = mfma::point_backward(s, p, plus, x_mid, fx_mid, g, uniform, tok_out, d_num, d_norm, work, d_proj, small, num_cu, st)))
+  if ((rc = mfma::point_backward(s, p, pl ? &prep.q : nullptr, x_mid, fx_mid, g, uniform, tok_out, d_num, d_norm, work, d_proj,
+                                 small, num_cu, st)))
     return rc;
   if (dx && (rc = general::rows_gemm(PA_BF16, s, np * HD, s.C, d_proj, sv + sp.w_in_t, nullptr, 0, dx, st))) return rc;
   return wgrad::product(PA_BF16, M, d_proj, np * HD, np * HD, x, s.C, s.C, s.conv_k > 0 ? &s : nullptr, work, d_w_in, d_b_in,

@@ -715,9 +715,10 @@ def layer_train_forward(x, uniform, params: dict, dims: LayerDims, residual=None
     return (y, saved) if ln_out is None else (y, saved, ln_out)
 
 
-def layer_train_backward(x, uniform, dy, saved, params: dict, dims: LayerDims, need_dx: bool = True):
-    """(dx or None, gradients by parameter name, float32 views of one buffer) of `layer_train_forward`."""
-    _need_cuda(x, uniform, dy, saved, *params.values())
+def layer_train_backward(x, uniform, dy, saved, dims: LayerDims, need_dx: bool = True):
+    """(dx or None, gradients by parameter name, float32 views of one buffer) of `layer_train_forward`; the parameters are
+    those of the forward call, kept in `saved`."""
+    _need_cuda(x, uniform, dy, saved)
     lib, shape, plus = _lib.load(), dims.c(), uniform is not None
     nbytes = lib.pa_layer_train_bytes(byref(shape), int(plus), _lib.PA_TRAIN_BACKWARD)
     if nbytes < 0:
@@ -727,8 +728,8 @@ def layer_train_backward(x, uniform, dy, saved, params: dict, dims: LayerDims, n
                         device=x.device)
     dx = torch.empty_like(x) if need_dx else None
     _lib.check(lib.pa_layer_train_backward(
-        byref(shape), byref(_c_params(params)), _c_plus(params) if plus else None, x.data_ptr(), _lib.ptr(uniform),
-        dy.data_ptr(), saved.data_ptr(), _lib.ptr(dx), grads.data_ptr(), workspace.data_ptr(), int(nbytes),
+        byref(shape), None, byref(_lib.PaPlusParams()) if plus else None, x.data_ptr(), _lib.ptr(uniform), dy.data_ptr(),
+        saved.data_ptr(), _lib.ptr(dx), grads.data_ptr(), workspace.data_ptr(), int(nbytes),
         _lib.current_stream_ptr(x.device)), "pa_layer_train_backward")
     C, HD, S, D, H = dims.C, dims.H * dims.D, dims.S, dims.D, dims.H
     taps = dims.conv_k ** (3 if dims.grid_d > 0 else 2) if dims.conv_k > 0 else 1

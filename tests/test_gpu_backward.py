@@ -974,6 +974,45 @@ def test_mlp_module_differentiates_twice_and_forward():
         net(x.bfloat16())
 
 
+@pytest.mark.parametrize("variant", ["irregular", "plus", "structured2d", "block"])
+def test_parameters_may_change_between_the_passes(variant):
+    """The gradients of a bf16 training step are those of the parameters its forward saw, whatever is done to the parameters
+    before the backward."""
+    announce("parameters changed between the passes", variant)
+    torch.manual_seed(0)
+    kw = dict(heads=4, dim_head=32, slice_num=32, use_te=False)
+    if variant == "block":
+        layer = pn.TransolverBlock(8, 256, 0.0, mlp_ratio=2, slice_num=32, use_te=False)
+    elif variant == "structured2d":
+        layer = pn.PhysicsAttentionStructuredMesh2D(128, (9, 15), kernel=3, **kw)
+    else:
+        layer = pn.PhysicsAttentionIrregularMesh(128, plus=variant == "plus", **kw)
+    layer = layer.cuda().train()
+    C = 256 if variant == "block" else 128
+    x, dy = torch.randn(2, 2, 135, C, device="cuda").bfloat16()
+    noise = torch.rand(2, 135, 4, 32, device="cuda").bfloat16()
+    # the LayerNorms' own weights are saved tensors, as in torch
+    params = [p for n, p in layer.named_parameters() if n.split(".")[0] not in ("ln_1",) and not n.startswith("ln_mlp1.0")]
+
+    def step(change):
+        xi = x.clone().requires_grad_(True)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = layer.forward_with_noise(xi, noise) if variant == "plus" else layer(xi)
+        if change:
+            with torch.no_grad():
+                for p in params:
+                    p.add_(1.0)
+        grads = torch.autograd.grad(y, [xi, *params], dy)
+        if change:
+            with torch.no_grad():
+                for p in params:
+                    p.sub_(1.0)
+        return grads
+
+    for a, b in zip(step(False), step(True)):
+        assert torch.equal(a, b)
+
+
 def test_mlp_module_under_autocast_leaves_types_that_autocast_leaves():
     """A float64 Mlp in training under bf16 autocast computes in float64, whole numbers are refused."""
     announce("Mlp types under autocast")
