@@ -747,7 +747,8 @@ __global__ __launch_bounds__(64 * ((S + 31) / 32)) void slice_attention_kernel(c
 // counts exactly the younger operations.  MASKED = true: one tile per workgroup, the last `nfull` tiles of each batch: the
 // ragged one, or, where a workgroup per tile fits the chip, all of them in one launch (2 x 1 000 points: 5.9 us against 6.1 + 4.7).
 // SPLIT: tokp is the attended tokens themselves, float32 (B, H, S, 32); each tile is multiplied with bf16(tok') and with the
-// remainder, i.e. with 16 bits of a token (training of the layers that multiplied with float32 tokens before they came here).
+// remainder, i.e. with 16 bits of a token (training of the layers that multiplied with float32 tokens before they came here):
+// 100 003 points, 256 / 64: 47 us, 15 us more than on packed bf16 tokens.
 // ------------------------------------------------------------------------------------------------
 template <int C, int S, int TAIL, bool MASKED, bool SPLIT>
 __global__ __launch_bounds__(C * 2) void deslice_project_kernel(const u32x4 *__restrict__ blob, const u32x4 *__restrict__ w_pack,
