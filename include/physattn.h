@@ -488,9 +488,9 @@ int pa_output_backward(const pa_shape *shape, const void *w_pack, const void *dy
  * Parameters: the three large weights in `weight_dtype` (PA_F32 or PA_BF16) in torch's layout (convolution weights
  * (H*32, C, k, ..); shape->conv_tap_major must be 1, it names the kernels' order), everything else float32.  The forward
  * leaves in `saved` (PA_TRAIN_SAVED bytes) what the backward reads, copies of the parameters included: they may change
- * between the calls, and the backward call takes of p and plus only whether plus is NULL.  grads (PA_TRAIN_GRADS bytes, float32): d in_project_x.weight, d in_project_fx.weight (not with plus),
- * their biases in the same order, d out_linear.weight, d out_linear.bias, d qkv_project.weight (96, 32), then grads of
- * pa_point_backward.  dx (B, N, C) bf16 or NULL.  tail (NULL, or C <= 256): the block's residual and LayerNorm on y, as in
+ * between the calls, and the backward call takes of p and plus only whether plus is NULL.
+ * grads (PA_TRAIN_GRADS bytes, float32): d in_project_x.weight, d in_project_fx.weight (not with plus), their biases in
+ * the same order, d out_linear.weight, d out_linear.bias, d qkv_project.weight (96, 32), then grads of pa_point_backward.  dx (B, N, C) bf16 or NULL.  tail (NULL, or C <= 256): the block's residual and LayerNorm on y, as in
  * pa_layer_forward; the backward call takes the gradient of y.  Replaces autograd over PA.py:501-558. */
 #define PA_TRAIN_SAVED 0    /* kept from the forward to the backward call */
 #define PA_TRAIN_FORWARD 1  /* workspace of the forward call */
