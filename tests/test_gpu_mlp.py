@@ -61,6 +61,34 @@ def test_mlp_matches_fp32_oracle(rows_shape, C, Fh):
     assert_rel_l2(ln4, F.layer_norm(want, (C,), gamma, beta, 1e-5), "LayerNorm(mlp)")
 
 
+@pytest.mark.parametrize("rows,C,Fh,train", [(*c, t) for c in [
+    (65, 256, 192), (31, 256, 128), (16385, 256, 320), (65536 + 65, 256, 256), (65536 + 32769, 256, 128),
+    (33, 512, 192), (8193, 512, 128), (32768 + 31, 512, 320), (32768 + 16385, 512, 128),
+] for t in (False, True) if not t or c[1] == 256])
+def test_mlp_rows_beyond_whole_rounds_of_the_chip(rows, C, Fh, train):
+    """Rows are split between the kernel that owns its rows and the one whose waves share them (256 compute units: 65 536 rows
+    a round at C = 256, 32 768 at 512): first and last rows of both parts, hidden widths that the four waves share unevenly."""
+    announce("mlp split", rows, C, Fh, train)
+    ref, u, res, gamma, beta, args = _case((rows,), C, Fh)
+    dev = args["u"].device
+    packed = PF.mlp_pack(args["w1"], args["w2"])
+    y, ln = PF.mlp_forward_packed(args["u"], packed, args["b1"], args["b2"], residual=res.to(dev), ln_weight=gamma.to(dev),
+                                  ln_bias=beta.to(dev), train=train)
+    plain = PF.mlp_forward_packed(args["u"], packed, args["b1"], args["b2"], train=train)
+    edge = {0, 1, 63, 64, rows - 66, rows - 33, rows - 2, rows - 1} | {k + d for k in range(0, rows, 32768) for d in (-65, -1, 0, 64)}
+    rows_at = torch.tensor(sorted(r for r in edge if 0 <= r < rows))
+    with torch.no_grad():
+        want = ref(u[rows_at].float())
+        want_sum = want + res[rows_at].float()
+        want_ln = F.layer_norm(want_sum, (C,), gamma, beta, 1e-5)
+    assert torch.isfinite(y.float()).all() and torch.isfinite(ln.float()).all()
+    at = rows_at.to(dev)
+    # each tensor's own rounding to bf16 is 1.7e-3, the hidden layer's less than that behind the sum over it
+    assert_rel_l2(plain[at], want, "mlp output", 5e-3)
+    assert_rel_l2(y[at], want_sum, "mlp + residual", 5e-3)
+    assert_rel_l2(ln[at], want_ln, "LayerNorm(mlp + residual)", 6e-3)
+
+
 def test_mlp_gelu_tails_and_determinism():
     announce("mlp large activations / determinism")
     # large pre-activations exercise both saturated ends of the erf and the sign handling
