@@ -967,61 +967,61 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void mlp_rows2_kernel(
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// mlp_split_kernel: the same MLP for inputs (and remainders of inputs) whose rows do not give every CU a block of the kernels
-// above.  Workgroup = 4 waves, one per SIMD, all on the same rows (64 at C = 256, 32 at C = 512); wave p takes the hidden
-// chunks p, p + 4, ... and sums its share of y^T for all channels (256 accumulation registers), so that a block is a
-// quarter of the serial chain and a CU needs a quarter of the rows.  The rows are B operands in LDS, shared by the waves; a
-// weight fragment is read by one wave of the block, once, so the weights go from the caches straight to registers, 16
-// fragments ahead, with no barrier in the loop.  The shares meet in LDS in float32, a wave finishing every fourth row.
-// Bound by the wave's own chain, of which MFMAs, GELU and the weights' way from L2 (4 C F bytes per block) each are about a
-// half, a quarter and a quarter at C = 256 (4 200 clocks per chunk; 64 MFMAs alone 2 800); at C = 512 by those bytes (51 per
-// clock and CU).  us, before -> after: C = 256, F = 1024: 4 000 rows 57 -> 26, 16 384 rows 61 -> 31; C = 512, F = 2048: 8 192 rows
-// 124 -> 54, 200 003 rows (six whole rounds and 3 395 rows) 951 -> 872.
+// mlp_split_kernel: the same MLP, bit for bit, for inputs (and remainders of inputs) whose rows do not give every CU a block of
+// the kernels above.  Workgroup = 8 waves, two per SIMD, all on the same 64 rows, which lie in LDS as B operands.  In a slot of
+// 256 hidden units wave w
+//   forms 32 of them, h^T = W1[its chunk] . u^T + b1 (two row tiles), leaving gelu(h) as B operands in LDS, and
+//   adds the slot before to its C / 8 output channels, y^T += W2[its channels, slot] . g^T, with the activations behind,
+// so that every sum runs in the order of the row-owning kernels; one barrier per slot.  A weight fragment is read by one wave
+// of the block, once, and feeds both row tiles: the weights go from the caches straight to registers, 16 fragments ahead.
+// Bound by vector issue and the weights' way from L2 (4 C F bytes per block, 40 bytes a clock and CU at C = 512).  us, row-owning
+// kernel -> here: C = 256, F = 1024: 2 000 rows 57 -> 22, 16 384 rows 61 -> 29; C = 512, F = 2048: 8 192 rows 124 -> 59, 16 384
+// rows 129 -> 74; 200 003 rows (six whole rounds of the one, 3 395 rows) 951 -> 877.  Four waves with a quarter of the hidden
+// units each and their sums joined at the end: 26, 31, 54, 104, and other bits than the row-owning kernels'.
 // blob: as packed for mlp_rows2_kernel (C = 256) / mlp_rows_kernel (C = 512).
 // ---------------------------------------------------------------------------------------------------------------
 template <int C>
 struct SplitCfg {
-  static constexpr int RT = 512 / C, ROWS = 32 * RT;  // row tiles, rows of a block
-  static constexpr int NS = C / 16;                   // weight fragments of one product and chunk (both products alike)
-  static constexpr int STEP = C == 256 ? 64 : 128;    // units from one fragment of a product to the next
-  static constexpr int ROUND = 32 * 256 / C;          // rows whose four shares are 128 KB
-  static constexpr int PART_LD = C + 4, PART_BYTES = 4 * ROUND * PART_LD * 4;
+  static constexpr int ROWS = 64, HIDDEN = 256;          // rows of a block, hidden units of a slot
+  static constexpr int LD = C + 8;                       // staged rows: 16 bytes apart in their banks
+  static constexpr int U_BYTES = ROWS * C * 2, G_BYTES = ROWS * HIDDEN * 2, BYTES = U_BYTES + 2 * G_BYTES;
+  static_assert(ROWS * LD * 2 <= BYTES, "the result is staged where the operands were");
 };
 
 template <int C, int TAIL, bool TRAIN>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void mlp_split_kernel(
+__global__ __launch_bounds__(512) void mlp_split_kernel(
     const u32x4 *__restrict__ blob, const float *__restrict__ b1, const float *__restrict__ b2,
     const uint16_t *__restrict__ u, uint16_t *__restrict__ y, const uint16_t *__restrict__ residual,
     const float *__restrict__ ln_gamma, const float *__restrict__ ln_beta, float ln_eps, uint16_t *__restrict__ ln_out,
     int64_t M, int F, const float *__restrict__ in_gamma, const float *__restrict__ in_beta, float in_eps) {
   using K = SplitCfg<C>;
   constexpr bool HAS_RES = TAIL == 1 || TAIL == 2, HAS_LN = TAIL == 1 || TAIL == 3;
-  constexpr int RT = K::RT, NS = K::NS, CT = C / 32, KS = C / 16, RING = 16;
-  static_assert(2 * CT == NS && KS == NS && NS % RING == 0, "both products take NS fragments; ring positions are constants");
+  constexpr int RT = 2, KS = C / 16, CTW = C / 256, RING = 16;  // row tiles, k-steps, channel tiles of a wave
+  // where chunk c's fragments lie: W1's k-step ks at c SLOT + ks STEP, W2's (kk, ct) at c SLOT + W2 + (kk C / 32 + ct) STEP
+  constexpr int STEP = C == 256 ? 64 : 128, SLOT = 2 * KS * 64, W2 = C == 256 ? SLOT + KS * 64 : 2 * SLOT + 64;
+  static_assert(16 * CTW == KS && KS % RING == 0, "both products take KS fragments per slot; ring positions are constants");
   typedef float f32x4 __attribute__((ext_vector_type(4)));
   extern __shared__ u32x4 smem[];
-  u32x4 *rows_lds = smem;                          // [row tile][k-step][lane] B operands
-  float *part = reinterpret_cast<float *>(smem);   // later: [wave][row][C] shares
-  float *b1s = reinterpret_cast<float *>(reinterpret_cast<char *>(smem) + K::PART_BYTES);
+  u32x4 *us = smem, *gs = smem + K::U_BYTES / 16;          // rows [tile][k-step][lane]; gelu(h) [slot & 1][chunk][kk][tile][lane]
+  uint16_t *stage = reinterpret_cast<uint16_t *>(smem);    // later: the result's rows
+  float *b1s = reinterpret_cast<float *>(reinterpret_cast<char *>(smem) + K::BYTES);
   float *b2s = b1s + F, *gams = b2s + C, *bets = gams + C, *igams = bets + C, *ibets = igams + C;
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int NCH = F / 32, mine = (NCH - wave + 3) / 4;  // this wave's chunks, at least one (F >= 128)
+  const int slots = F / K::HIDDEN;
   const int64_t row0 = (int64_t)blockIdx.x * K::ROWS;
 
-  // where the fragments of the two products of this wave's chunk k begin; w1_at past the last chunk: W2's last
-  constexpr int SLOT = C == 256 ? 2 * NS * 64 : 4096;
-  constexpr int W2 = C == 256 ? SLOT + NS * 64 : 2 * SLOT + 64;
-  auto w2_at = [&](int k) -> const u32x4 * { return blob + (int64_t)(wave + 4 * k) * SLOT + W2 + lane; };
-  auto w1_at = [&](int k) -> const u32x4 * {
-    const int past = (mine - 1 - k) >> 31;  // 0 or -1: no branch, which would cut the loop body in two
-    return blob + (int64_t)(wave + 4 * (k + past)) * SLOT + (W2 & past) + lane;
-  };
+  // first fragment of a phase: W1 of this wave's chunk of slot s; W2 of its channels and the slot's first chunk
+  auto w1_at = [&](int s) -> const u32x4 * { return blob + (int64_t)(8 * s + wave) * SLOT + lane; };
+  auto w2_at = [&](int s) -> const u32x4 * { return blob + (int64_t)(8 * s) * SLOT + W2 + wave * CTW * STEP + lane; };
+  // fragment S of them: phase 2 takes (chunk, kk, channel tile), the last the fastest
+  auto off1 = [](int S) { return S * STEP; };
+  auto off2 = [](int S) { return (S / (2 * CTW)) * SLOT + ((S / CTW) % 2) * (C / 32) * STEP + (S % CTW) * STEP; };
   u32x4 fr[RING];
   {
     const u32x4 *w = w1_at(0);
 #pragma unroll
-    for (int q = 0; q < RING; ++q) fr[q] = w[q * K::STEP];
+    for (int q = 0; q < RING; ++q) fr[q] = w[off1(q)];
   }
   {
     u32x4 ub[KS];
@@ -1032,201 +1032,158 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) ub[ks] = *reinterpret_cast<const u32x4 *>(src + 16 * ks);
     }
-    // eight biases per thread are on their way together
-    for (int k0 = tid; k0 < F; k0 += 8 * 256) {
-      float v[8];
+    for (int k0 = tid; k0 < F; k0 += 4 * 512) {  // four biases per thread are on their way together
+      float v[4];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) v[q] = b1[k0 + 256 * q < F ? k0 + 256 * q : k0];
+      for (int q = 0; q < 4; ++q) v[q] = b1[k0 + 512 * q < F ? k0 + 512 * q : k0];
 #pragma unroll
-      for (int q = 0; q < 8; ++q)
-        if (k0 + 256 * q < F) b1s[k0 + 256 * q] = v[q];
+      for (int q = 0; q < 4; ++q)
+        if (k0 + 512 * q < F) b1s[k0 + 512 * q] = v[q];
     }
-#pragma unroll
-    for (int k = tid; k < C; k += 256) {
-      const float v2 = b2[k], vg = HAS_LN ? ln_gamma[k] : 1.f, vb = HAS_LN ? ln_beta[k] : 0.f;
-      const float ig = in_gamma ? in_gamma[k] : 1.f, ib = in_gamma ? in_beta[k] : 0.f;
-      b2s[k] = v2, gams[k] = vg, bets[k] = vb, igams[k] = ig, ibets[k] = ib;
+    if (tid < C) {
+      const float v2 = b2[tid], vg = HAS_LN ? ln_gamma[tid] : 1.f, vb = HAS_LN ? ln_beta[tid] : 0.f;
+      const float ig = in_gamma ? in_gamma[tid] : 1.f, ib = in_gamma ? in_beta[tid] : 0.f;
+      b2s[tid] = v2, gams[tid] = vg, bets[tid] = vb, igams[tid] = ig, ibets[tid] = ib;
     }
     __syncthreads();
     if (wave < RT) {
       if (in_gamma) normalize_operand_rows<C>(ub, igams, ibets, in_eps, g);
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) rows_lds[(wave * KS + ks) * 64 + lane] = ub[ks];
+      for (int ks = 0; ks < KS; ++ks) us[(wave * KS + ks) * 64 + lane] = ub[ks];
     }
   }
   __syncthreads();
 
-  f32x16 yacc[RT][CT];
+  f32x16 yacc[RT][CTW], hacc[RT];  // channel 32 (CTW wave + c) + rowmap(r, g), hidden unit rowmap(r, g) of the chunk; row 32 t + i
 #pragma unroll
   for (int t = 0; t < RT; ++t)
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
+    for (int c = 0; c < CTW; ++c)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) yacc[t][ct][r] = 0.f;
+      for (int r = 0; r < 16; ++r) yacc[t][c][r] = b2s[32 * (CTW * wave + c) + rowmap(r, g)];
 
-  {
-    f32x16 hacc[RT];
-    float hrest[RT][8];
-    u32x4 gop[RT][2], gnew[RT];
-    constexpr int NV = 8 * RT, EVERY = NS / NV;  // evaluations of a phase, steps from one to the next
-    // An evaluation in four parts, so that two of them (RT = 2) take turns behind the MFMAs: one wave per SIMD waits for
-    // whatever its next instruction depends on.  a*: the evaluation that is being started, z*: that is being finished
-    float ax = 0.f, a2 = 0.f, aq = 0.f, ae = 0.f, at = 0.f, zx = 0.f, ze = 0.f, zt = 0.f, zr = 0.f, feven = 0.f;
-    auto start1 = [&](float x) {
-      ax = x;
-      if constexpr (TRAIN) {
-        ae = gelu_gauss(x);
-      } else {
-        a2 = fminf(x * x, 81.f);
-        aq = fmaf(-3.51902394e-04f * -2.f * kLog2e, a2, 3.70080200e-02f * -2.f * kLog2e);
-      }
-    };
-    auto start2 = [&]() {
-      if constexpr (TRAIN) at = gelu_ratio(ax);
-      else ae = __builtin_amdgcn_exp2f(ax * fmaf(aq, a2, 7.97505275e-01f * -2.f * kLog2e));
-    };
-    auto started = [&]() { zx = ax, ze = ae, zt = at; };
-    auto end1 = [&]() {
-      if constexpr (TRAIN) zr = gelu_phi(zx, ze, zt);
-      else zr = __builtin_amdgcn_rcpf(1.f + ze);
-    };
-    auto end2 = [&](auto v_) {
-      constexpr int v = decltype(v_)::value, j = v % 8;
-      const float r = zx * zr;
-      if constexpr (j % 2 == 0) feven = r;
-      else gnew[v / 8][j / 2] = pack2(feven, r);
-    };
-    // what runs behind MFMA t of step S of a phase; value(v): the argument of evaluation v = 8 tile + j
-    auto evaluate = [&](auto S_, auto t_, auto &&value) {
-      constexpr int S = decltype(S_)::value, t = decltype(t_)::value, v = S / EVERY;
-      using V = std::integral_constant<int, v>;
-      if constexpr (EVERY == 1) {
-        if constexpr (t == 0) {
-          start1(value(V{}));
-          if constexpr (S > 0) end1();
-        } else {
-          start2();
-          if constexpr (S > 0) end2(std::integral_constant<int, (S > 0 ? v - 1 : 0)>{});
-          started();
-          if constexpr (S == NS - 1) {
-            end1();
-            end2(V{});
-          }
-        }
-      } else {
-        static_assert(EVERY == 4 || EVERY == 1, "one part per MFMA");
-        if constexpr (S % EVERY == 0) start1(value(V{}));
-        if constexpr (S % EVERY == 1) start2(), started();
-        if constexpr (S % EVERY == 2) end1();
-        if constexpr (S % EVERY == 3) end2(V{});
-      }
-    };
-    auto evaluate_all = [&](auto &&value) {
-      static_for<NV>([&](auto v_) {
-        start1(value(v_));
-        start2();
-        started();
-        end1();
-        end2(v_);
-      });
-    };
-    // the stream of weight fragments is W1(0), W1(1), W2(0), W1(2), W2(1), ...: each one consumed makes room for the one RING
-    // later, of the running phase's fragments (`here`) or of the next phase's
-    auto ahead = [&](auto S_, const u32x4 *here, const u32x4 *next) {
+  u32x4 gop = u32x4{0, 0, 0, 0};
+  float ex[2] = {0.f, 0.f}, ee[2] = {0.f, 0.f}, et[2] = {0.f, 0.f}, feven = 0.f;  // two evaluations in flight
+  u32x4 *gdst = nullptr;
+  auto begin = [&](auto v_) {  // evaluation v: register v % 16 of tile v / 16
+    constexpr int v = decltype(v_)::value;
+    const float x = hacc[v / 16][v % 16];
+    ex[v % 2] = x;
+    if constexpr (TRAIN) {
+      ee[v % 2] = gelu_gauss(x);
+      et[v % 2] = gelu_ratio(x);
+    } else {
+      const float x2 = fminf(x * x, 81.f);
+      float q = fmaf(-3.51902394e-04f * -2.f * kLog2e, x2, 3.70080200e-02f * -2.f * kLog2e);
+      q = fmaf(q, x2, 7.97505275e-01f * -2.f * kLog2e);
+      ee[v % 2] = __builtin_amdgcn_exp2f(x * q);
+    }
+  };
+  auto finish = [&](auto v_) {
+    constexpr int v = decltype(v_)::value, j = v % 8;
+    const float x = ex[v % 2], e = ee[v % 2], t = et[v % 2];
+    const float r = x * (TRAIN ? gelu_phi(x, e, t) : __builtin_amdgcn_rcpf(1.f + e));
+    if constexpr (j % 2 == 0) feven = r;
+    else gop[j / 2] = pack2(feven, r);
+    if constexpr (j == 7) gdst[((v / 8) % 2 * RT + v / 16) * 64] = gop;
+  };
+  // the activations behind unit n of N of a phase: evaluation 32 n / N ends, the next one starts
+  auto activate = [&](auto n_, auto N_) {
+    constexpr int n = decltype(n_)::value, every = decltype(N_)::value / 32;
+    if constexpr (n % every == 0) {
+      constexpr int v = n / every;
+      if constexpr (v + 1 < 32) begin(std::integral_constant<int, v + 1>{});
+      finish(std::integral_constant<int, v>{});
+    }
+  };
+  auto hidden = [&](int s, const u32x4 *here, const u32x4 *next, auto next_is_w1) {
+    const int c = 8 * s + wave;
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) hacc[t][r] = b1s[32 * c + rowmap(r, g)];
+    constexpr int LA = 2;
+    u32x4 bf[LA + 1][RT];
+#pragma unroll
+    for (int q = 0; q < LA; ++q)
+#pragma unroll
+      for (int t = 0; t < RT; ++t) bf[q][t] = us[(t * KS + q) * 64 + lane];
+    static_for<KS>([&](auto S_) {
       constexpr int S = decltype(S_)::value;
-      fr[S % RING] = S + RING < NS ? here[(S + RING) * K::STEP] : next[(S + RING - NS) * K::STEP];
-    };
-    constexpr int LA = 2;  // steps the row operands are read ahead of their MFMAs
-    // the MFMAs that write hacc are unknown to the compiler: its first reader behind them keeps its distance
-    auto settle = [&]() {
+      if constexpr (S + LA < KS) {
 #pragma unroll
-      for (int t = 0; t < RT; ++t) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(hacc[t]));
-    };
-    auto phase1 = [&](auto act_, int k, const u32x4 *here, const u32x4 *next) {
-      constexpr bool ACT = decltype(act_)::value;
-#pragma unroll
-      for (int t = 0; t < RT; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) hacc[t][r] = b1s[32 * (wave + 4 * k) + rowmap(r, g)];
-      // nor are those that read it, so its last vector write keeps its distance from them
-#pragma unroll
-      for (int t = 0; t < RT; ++t) asm volatile("s_nop 7" : "+v"(hacc[t]));
-      u32x4 bf[LA + 1][RT];
-#pragma unroll
-      for (int s = 0; s < LA; ++s)
-#pragma unroll
-        for (int t = 0; t < RT; ++t) bf[s][t] = rows_lds[(t * KS + s) * 64 + lane];
-      static_for<NS>([&](auto S_) {
-        constexpr int S = decltype(S_)::value;
-        if constexpr (S + LA < NS) {
-#pragma unroll
-          for (int t = 0; t < RT; ++t) bf[(S + LA) % (LA + 1)][t] = rows_lds[(t * KS + S + LA) * 64 + lane];
-        }
-        static_for<RT>([&](auto t_) {
-          constexpr int t = decltype(t_)::value;
-          mma_in_vgprs(fr[S % RING], bf[S % (LA + 1)][t], hacc[t]);
-          __builtin_amdgcn_sched_barrier(0);
-          if constexpr (t == RT - 1) ahead(S_, here, next);
-          if constexpr (ACT) evaluate(S_, t_, [&](auto v_) { return hrest[decltype(v_)::value / 8][decltype(v_)::value % 8]; });
-          __builtin_amdgcn_sched_barrier(0);
-        });
-      });
-    };
-    auto phase2 = [&](auto act_, const u32x4 *here, const u32x4 *next) {
-      constexpr bool ACT = decltype(act_)::value;
-      static_for<NS>([&](auto S_) {
-        constexpr int S = decltype(S_)::value, kk = S / CT, ct = S % CT;
-        static_for<RT>([&](auto t_) {
-          constexpr int t = decltype(t_)::value;
-          yacc[t][ct] = mma(fr[S % RING], gop[t][kk], yacc[t][ct]);
-          __builtin_amdgcn_sched_barrier(0);
-          if constexpr (t == RT - 1 && (ACT || S + RING < NS)) ahead(S_, here, next);
-          if constexpr (ACT && t == 0 && S == 0) settle();
-          if constexpr (ACT) evaluate(S_, t_, [&](auto v_) { return hacc[decltype(v_)::value / 8][decltype(v_)::value % 8]; });
-          __builtin_amdgcn_sched_barrier(0);
-        });
-      });
-    };
-    using Yes = std::true_type;
-    using No = std::false_type;
-    // h(k) with the second half of gelu(h(k - 1)) behind it, y += W2 gelu(h(k - 1)) with the first half of gelu(h(k))
-    phase1(No{}, 0, w1_at(0), w1_at(1));
-    settle();
-    evaluate_all([&](auto v_) { return hacc[decltype(v_)::value / 8][decltype(v_)::value % 8]; });
-    auto roll = [&]() {
-#pragma unroll
-      for (int t = 0; t < RT; ++t) {
-        gop[t][0] = gnew[t];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) hrest[t][j] = hacc[t][8 + j];
+        for (int t = 0; t < RT; ++t) bf[(S + LA) % (LA + 1)][t] = us[(t * KS + S + LA) * 64 + lane];
       }
-    };
-    roll();
-    for (int k = 1; k < mine; ++k) {
-      phase1(Yes{}, k, w1_at(k), w2_at(k - 1));
 #pragma unroll
-      for (int t = 0; t < RT; ++t) gop[t][1] = gnew[t];
-      phase2(Yes{}, w2_at(k - 1), w1_at(k + 1));
-      roll();
-    }
-    evaluate_all([&](auto v_) { return hrest[decltype(v_)::value / 8][decltype(v_)::value % 8]; });
+      for (int t = 0; t < RT; ++t) hacc[t] = mma(fr[S % RING], bf[S % (LA + 1)][t], hacc[t]);
+      if constexpr (S + RING < KS) fr[S % RING] = here[off1(S + RING)];
+      else fr[S % RING] = next[decltype(next_is_w1)::value ? off1(S + RING - KS) : off2(S + RING - KS)];
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  auto output = [&](int s, auto act_, const u32x4 *here, const u32x4 *next) {
+    constexpr bool ACT = decltype(act_)::value;
+    const u32x4 *gb = gs + (s & 1) * (K::G_BYTES / 16) + lane;
+    constexpr int LA = 2, NG = 16;  // operand (chunk, kk) pairs
+    u32x4 bf[LA + 1][RT];
 #pragma unroll
-    for (int t = 0; t < RT; ++t) gop[t][1] = gnew[t];
-    phase2(No{}, w2_at(mine - 1), nullptr);
-  }
+    for (int q = 0; q < LA; ++q)
+#pragma unroll
+      for (int t = 0; t < RT; ++t) bf[q][t] = gb[(q * RT + t) * 64];
+    if constexpr (ACT) begin(std::integral_constant<int, 0>{});
+    static_for<KS>([&](auto S_) {
+      constexpr int S = decltype(S_)::value, q = S / CTW, c = S % CTW;
+      if constexpr (c == 0 && q + LA < NG) {
+#pragma unroll
+        for (int t = 0; t < RT; ++t) bf[(q + LA) % (LA + 1)][t] = gb[((q + LA) * RT + t) * 64];
+      }
+      static_for<RT>([&](auto t_) {
+        constexpr int t = decltype(t_)::value;
+        yacc[t][c] = mma(fr[S % RING], bf[q % (LA + 1)][t], yacc[t][c]);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (ACT) activate(std::integral_constant<int, S * RT + t>{}, std::integral_constant<int, KS * RT>{});
+        if constexpr (t == RT - 1) {
+          if constexpr (S + RING < KS) fr[S % RING] = here[off2(S + RING)];
+          else if constexpr (ACT) fr[S % RING] = next[off1(S + RING - KS)];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    });
+  };
+  // where slot s leaves this wave's chunk
+  auto g_at = [&](int s) { return gs + (s & 1) * (K::G_BYTES / 16) + wave * 2 * RT * 64 + lane; };
 
-  // ---- the four shares of ROUND rows at a time, rows 16 bytes apart in their banks ----
-  constexpr int NV = C / 256, ROUND = K::ROUND, LD = K::PART_LD, PER_WAVE = ROUND / 4, NIT = PER_WAVE / 2;
-  const int hl = g, il = i;  // half a wave finishes a row; NIT of them side by side, one wave per SIMD hides no latency
-  f32x4 ga[NV][2], be[NV][2], bo[NV][2];
+  hidden(0, w1_at(0), slots > 1 ? w1_at(1) : w2_at(0), std::true_type{});
+  gdst = g_at(0);
+  begin(std::integral_constant<int, 0>{});
+  static_for<32>([&](auto v_) { activate(v_, std::integral_constant<int, 32>{}); });
+  __syncthreads();
+  for (int s = 1; s < slots; ++s) {
+    hidden(s, w1_at(s), w2_at(s - 1), std::false_type{});
+    gdst = g_at(s);
+    // past the last slot: its own W1 again (read, not used)
+    output(s - 1, std::true_type{}, w2_at(s - 1), w1_at(s + 1 < slots ? s + 1 : s));
+    __syncthreads();
+  }
+  {
+    const u32x4 *w = w2_at(slots - 1);
 #pragma unroll
-  for (int v = 0; v < NV; ++v)
+    for (int q = 0; q < RING; ++q) fr[q] = w[off2(q)];
+    output(slots - 1, std::false_type{}, w, nullptr);
+  }
+  __syncthreads();  // the operands are all read
+
+  // ---- y^T to bf16 rows in LDS; then wave w finishes rows 8 w .. + 7, half a wave per row, four pairs side by side ----
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      ga[v][h] = *reinterpret_cast<const f32x4 *>(gams + 256 * v + 8 * il + 4 * h);
-      be[v][h] = *reinterpret_cast<const f32x4 *>(bets + 256 * v + 8 * il + 4 * h);
-      bo[v][h] = *reinterpret_cast<const f32x4 *>(b2s + 256 * v + 8 * il + 4 * h);
-    }
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int c = 0; c < CTW; ++c)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x16 &a = yacc[t][c];
+        *reinterpret_cast<u32x2 *>(stage + (32 * t + i) * K::LD + 32 * (CTW * wave + c) + 8 * q + 4 * g) =
+            u32x2{pack2(a[4 * q], a[4 * q + 1]), pack2(a[4 * q + 2], a[4 * q + 3])};
+      }
   // Buffer accesses end at the last row by themselves: a branch around the stores would have every wait for a residual row
   // wait for the stores before it as well.
   const int64_t here = M - row0 < K::ROWS ? M - row0 : K::ROWS;
@@ -1234,92 +1191,76 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(static_cast<const uint16_t *>(p)) + row0 * C, 0, (int)here * C * 2,
                                              0x00027000);
   };
-  constexpr int STREAM = 2;  // the non-temporal hint
-  static_for<K::ROWS / ROUND>([&](auto rd_) {
-    constexpr int rd = decltype(rd_)::value, t = rd * ROUND / 32, lo = rd * ROUND % 32;
-    const int at = ((rd * ROUND + wave * PER_WAVE + hl) * C + 8 * il) * 2;  // bytes from the block's first row
-    u32x4 rsd[NIT][NV];
-    if constexpr (HAS_RES) {
-#pragma unroll
-      for (int it = 0; it < NIT; ++it)
-#pragma unroll
-        for (int v = 0; v < NV; ++v)
-          rsd[it][v] = __builtin_amdgcn_raw_buffer_load_b128(rows_of(residual), at + it * 4 * C + 512 * v, 0, STREAM);
-    }
-    __syncthreads();  // the rows' operands, or the shares of the round before, have been read
-    if (ROUND == 32 || (i >= lo && i < lo + ROUND)) {
-      float *dst = part + (wave * ROUND + i - lo) * LD + 4 * g;
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const f32x16 &a = yacc[t][ct];
-          *reinterpret_cast<f32x4 *>(dst + 32 * ct + 8 * q) = f32x4{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
-        }
-    }
-    __syncthreads();
-    float val[NIT][8 * NV];
+  constexpr int NV = C / 256, NIT = K::ROWS / 8 / 2, STREAM = 2;  // STREAM: the non-temporal hint
+  const int hl = g, il = i, at = ((8 * wave + hl) * C + 8 * il) * 2;  // at: bytes from the block's first row
+  u32x4 rsd[NIT][NV];
+  if constexpr (HAS_RES) {
 #pragma unroll
     for (int it = 0; it < NIT; ++it)
 #pragma unroll
-      for (int v = 0; v < NV; ++v) {
-        f32x4 s0 = bo[v][0], s1 = bo[v][1];
+      for (int v = 0; v < NV; ++v)
+        rsd[it][v] = __builtin_amdgcn_raw_buffer_load_b128(rows_of(residual), at + it * 4 * C + 512 * v, 0, STREAM);
+  }
+  __syncthreads();
+  float val[NIT][8 * NV];
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          const float *src = part + (w * ROUND + wave * PER_WAVE + 2 * it + hl) * LD + 256 * v + 8 * il;
-          s0 += *reinterpret_cast<const f32x4 *>(src);
-          s1 += *reinterpret_cast<const f32x4 *>(src + 4);
-        }
-        u32x4 ob;
+  for (int it = 0; it < NIT; ++it)
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          const float a0 = w < 2 ? s0[2 * w] : s1[2 * w - 4], a1 = w < 2 ? s0[2 * w + 1] : s1[2 * w - 3];
-          uint32_t word = pack2(a0, a1);
-          if constexpr (HAS_RES)  // the MLP output is a bf16 tensor; the sum is rounded again
-            word = pack2(__uint_as_float(word << 16) + __uint_as_float(rsd[it][v][w] << 16),
-                         __uint_as_float(word & 0xffff0000u) + __uint_as_float(rsd[it][v][w] & 0xffff0000u));
-          ob[w] = word;
-          val[it][8 * v + 2 * w] = __uint_as_float(word << 16);
-          val[it][8 * v + 2 * w + 1] = __uint_as_float(word & 0xffff0000u);
+    for (int v = 0; v < NV; ++v) {
+      u32x4 ob = *reinterpret_cast<const u32x4 *>(stage + (8 * wave + 2 * it + hl) * K::LD + 256 * v + 8 * il);
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        if constexpr (HAS_RES) {  // the MLP output is a bf16 tensor; the sum is rounded again
+          const uint32_t word = ob[w];
+          ob[w] = pack2(__uint_as_float(word << 16) + __uint_as_float(rsd[it][v][w] << 16),
+                        __uint_as_float(word & 0xffff0000u) + __uint_as_float(rsd[it][v][w] & 0xffff0000u));
         }
-        __builtin_amdgcn_raw_buffer_store_b128(ob, rows_of(y), at + it * 4 * C + 512 * v, 0, STREAM);
+        val[it][8 * v + 2 * w] = __uint_as_float(ob[w] << 16);
+        val[it][8 * v + 2 * w + 1] = __uint_as_float(ob[w] & 0xffff0000u);
       }
-    if constexpr (HAS_LN) {
-      float mean[NIT], rstd[NIT];
+      __builtin_amdgcn_raw_buffer_store_b128(ob, rows_of(y), at + it * 4 * C + 512 * v, 0, STREAM);
+    }
+  if constexpr (HAS_LN) {
+    float mean[NIT], rstd[NIT];
 #pragma unroll
-      for (int it = 0; it < NIT; ++it) {
-        float s1 = 0.f;
+    for (int it = 0; it < NIT; ++it) {
+      float s1 = 0.f;
 #pragma unroll
-        for (int k = 0; k < 8 * NV; ++k) s1 += val[it][k];
-        mean[it] = half_wave_sum(s1) * (1.f / C);
+      for (int k = 0; k < 8 * NV; ++k) s1 += val[it][k];
+      mean[it] = half_wave_sum(s1) * (1.f / C);
+    }
+#pragma unroll
+    for (int it = 0; it < NIT; ++it) {
+      float s2 = 0.f;
+#pragma unroll
+      for (int k = 0; k < 8 * NV; ++k) {
+        const float dl = val[it][k] - mean[it];
+        s2 = fmaf(dl, dl, s2);
       }
+      rstd[it] = rsqrtf(half_wave_sum(s2) * (1.f / C) + ln_eps);
+    }
 #pragma unroll
-      for (int it = 0; it < NIT; ++it) {
-        float s2 = 0.f;
+    for (int v = 0; v < NV; ++v) {
+      f32x4 ga[2], be[2];
 #pragma unroll
-        for (int k = 0; k < 8 * NV; ++k) {
-          const float dl = val[it][k] - mean[it];
-          s2 = fmaf(dl, dl, s2);
-        }
-        rstd[it] = rsqrtf(half_wave_sum(s2) * (1.f / C) + ln_eps);
+      for (int h = 0; h < 2; ++h) {
+        ga[h] = *reinterpret_cast<const f32x4 *>(gams + 256 * v + 8 * il + 4 * h);
+        be[h] = *reinterpret_cast<const f32x4 *>(bets + 256 * v + 8 * il + 4 * h);
       }
 #pragma unroll
       for (int it = 0; it < NIT; ++it) {
         const float r = rstd[it], shift = -mean[it] * r;
+        u32x4 lb;
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
-          u32x4 lb;
-#pragma unroll
-          for (int w = 0; w < 4; ++w) {
-            const int h = w >> 1, e = 2 * (w & 1);
-            lb[w] = pack2(fmaf(fmaf(val[it][8 * v + 2 * w], r, shift), ga[v][h][e], be[v][h][e]),
-                          fmaf(fmaf(val[it][8 * v + 2 * w + 1], r, shift), ga[v][h][e + 1], be[v][h][e + 1]));
-          }
-          __builtin_amdgcn_raw_buffer_store_b128(lb, rows_of(ln_out), at + it * 4 * C + 512 * v, 0, STREAM);
+        for (int w = 0; w < 4; ++w) {
+          const int h = w >> 1, e = 2 * (w & 1);
+          lb[w] = pack2(fmaf(fmaf(val[it][8 * v + 2 * w], r, shift), ga[h][e], be[h][e]),
+                        fmaf(fmaf(val[it][8 * v + 2 * w + 1], r, shift), ga[h][e + 1], be[h][e + 1]));
         }
+        __builtin_amdgcn_raw_buffer_store_b128(lb, rows_of(ln_out), at + it * 4 * C + 512 * v, 0, STREAM);
       }
     }
-  });
+  }
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1955,14 +1896,14 @@ int pack(int64_t C, int64_t F, const void *w1, const float *w1_scale, const void
   return e == hipSuccess ? PA_OK : (int)e;
 }
 
-// LDS of the split kernel: the shares (or the rows' operands), biases and LayerNorm vectors
+// LDS of the split kernel: the operands (later the staged rows), biases and LayerNorm vectors
 template <int C>
 static size_t split_lds(int F) {
-  return (size_t)rows::SplitCfg<C>::PART_BYTES + (size_t)(F + 5 * C) * 4;
+  return (size_t)rows::SplitCfg<C>::BYTES + (size_t)(F + 5 * C) * 4;
 }
-// Rounds of the split kernel that are shorter than one of the owning kernel's.  C = 256, F = 1024 (us): the split kernel 26 - 31
-// / 53 - 58 / 81 - 85 for one / two / three rounds (16 384 rows each), the owning kernel 57 - 67 / 69 - 88 for up to 32 768 / 65 536
-// rows.  C = 512, F = 2048: 51 - 57 / 99 - 112 / 150 - 164 (8 192 rows each) against 120 - 135 / 157.
+// Rounds of the split kernel (64 rows per CU) that are shorter than one of the owning kernel's.  C = 256, F = 1024 (us): the
+// split kernel 22 - 29 / 48 - 53 for one / two rounds, about 78 for three; the owning kernel 57 - 67 for up to 32 768 rows, 73 for
+// 49 152.  C = 512, F = 2048: 50 - 74 / 122 - 150 against 120 - 129 / 131 - 157; F = 128 .. 512 alike.
 template <int C>
 constexpr int64_t kSplitRounds = 2;
 
@@ -1973,7 +1914,7 @@ template <int C>
 static int64_t owned_rows(int64_t rows, int F, int64_t per_round, int num_cu) {
   using K = rows::SplitCfg<C>;
   const int64_t whole = rows / per_round * per_round, rest = rows - whole, split_round = (int64_t)K::ROWS * num_cu;
-  if (rest == 0 || F < 128 || split_lds<C>(F) > kMaxLdsBytes || (rest + split_round - 1) / split_round > kSplitRounds<C>) return rows;
+  if (rest == 0 || F % K::HIDDEN != 0 || split_lds<C>(F) > kMaxLdsBytes || (rest + split_round - 1) / split_round > kSplitRounds<C>) return rows;
   return whole;
 }
 
@@ -1989,7 +1930,7 @@ static int launch_split(int64_t first, int64_t rows, int F, const void *blob, co
   const int64_t n = rows - first, at = first * C;
   auto in16 = [&](const void *p) { return p ? static_cast<const uint16_t *>(p) + at : nullptr; };
   auto out16 = [&](void *p) { return p ? static_cast<uint16_t *>(p) + at : nullptr; };
-  hipLaunchKernelGGL((rows::mlp_split_kernel<C, TAIL, TRAIN>), dim3((unsigned)((n + K::ROWS - 1) / K::ROWS)), dim3(256), lds, st,
+  hipLaunchKernelGGL((rows::mlp_split_kernel<C, TAIL, TRAIN>), dim3((unsigned)((n + K::ROWS - 1) / K::ROWS)), dim3(512), lds, st,
                      static_cast<const u32x4 *>(blob), b1, b2, in16(u), out16(y), tail ? in16(tail->residual) : nullptr,
                      tail ? tail->ln_gamma : nullptr, tail ? tail->ln_beta : nullptr, tail ? tail->ln_eps : 0.f,
                      tail ? out16(tail->ln_out) : nullptr, n, F, in.gamma, in.beta, in.eps);

@@ -62,12 +62,13 @@ def test_mlp_matches_fp32_oracle(rows_shape, C, Fh):
 
 
 @pytest.mark.parametrize("rows,C,Fh,train", [(*c, t) for c in [
-    (65, 256, 192), (31, 256, 128), (16385, 256, 320), (65536 + 65, 256, 256), (65536 + 32769, 256, 128),
-    (33, 512, 192), (8193, 512, 128), (32768 + 31, 512, 320), (32768 + 16385, 512, 128),
+    (65, 256, 256), (31, 256, 512), (16385, 256, 256), (65536 + 65, 256, 256), (65536 + 32769, 256, 256), (65536 + 65, 256, 320),
+    (33, 512, 256), (8193, 512, 768), (32768 + 31, 512, 256), (32768 + 32767, 512, 256), (63, 512, 320),
 ] for t in (False, True) if not t or c[1] == 256])
 def test_mlp_rows_beyond_whole_rounds_of_the_chip(rows, C, Fh, train):
     """Rows are split between the kernel that owns its rows and the one whose waves share them (256 compute units: 65 536 rows
-    a round at C = 256, 32 768 at 512): first and last rows of both parts, hidden widths that the four waves share unevenly."""
+    a round at C = 256, 32 768 at 512), with the same bits from both: first and last rows of both parts, hidden widths of one slot
+    and of several, and one that the second kernel does not take."""
     announce("mlp split", rows, C, Fh, train)
     ref, u, res, gamma, beta, args = _case((rows,), C, Fh)
     dev = args["u"].device
@@ -75,6 +76,8 @@ def test_mlp_rows_beyond_whole_rounds_of_the_chip(rows, C, Fh, train):
     y, ln = PF.mlp_forward_packed(args["u"], packed, args["b1"], args["b2"], residual=res.to(dev), ln_weight=gamma.to(dev),
                                   ln_bias=beta.to(dev), train=train)
     plain = PF.mlp_forward_packed(args["u"], packed, args["b1"], args["b2"], train=train)
+    first = PF.mlp_forward_packed(args["u"][:33].clone(), packed, args["b1"], args["b2"], train=train)
+    assert torch.equal(first, plain[:33])
     edge = {0, 1, 63, 64, rows - 66, rows - 33, rows - 2, rows - 1} | {k + d for k in range(0, rows, 32768) for d in (-65, -1, 0, 64)}
     rows_at = torch.tensor(sorted(r for r in edge if 0 <= r < rows))
     with torch.no_grad():
