@@ -320,8 +320,9 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 
 def current_stream_ptr(device: torch.device) -> int:
-    return int(torch.cuda.current_stream(device).cuda_stream)
+    # the handle alone: torch.cuda.current_stream builds a Stream object around it, 4 us a call against 0.2
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def ptr(t) -> int | None:
-    return None if t is None else int(t.data_ptr())
+    return None if t is None else t.data_ptr()

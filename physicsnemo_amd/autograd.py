@@ -32,8 +32,9 @@ def _wgrad(d_out: torch.Tensor, inp: torch.Tensor):
     """(d W, d b) = (d out^T . in, column sums of d out) over all rows: one pass of the library's MFMA kernel where it
     serves the shape, else the GEMM library and a reduction."""
     d_out, inp = d_out.contiguous(), inp.contiguous()
-    if PF.cols_gemm_supported(d_out, inp):
-        return PF.cols_gemm(d_out, inp, col_sums=True)
+    served = PF.try_cols_gemm(d_out, inp)
+    if served is not None:
+        return served
     ca, cb = d_out.shape[-1], inp.shape[-1]
     rows = d_out.numel() // ca
     fold = 32 // ca if ca < 32 and 32 % ca == 0 else 0
@@ -41,8 +42,9 @@ def _wgrad(d_out: torch.Tensor, inp: torch.Tensor):
         # narrow d out (slice_num 16): `fold` consecutive rows side by side make 32 columns; the wanted product is the
         # sum of the diagonal blocks of the folded one
         a2, b2 = d_out.reshape(rows // fold, 32), inp.reshape(rows // fold, cb * fold)
-        if PF.cols_gemm_supported(a2, b2):
-            p2, s2 = PF.cols_gemm(a2, b2, col_sums=True)
+        folded = PF.try_cols_gemm(a2, b2)
+        if folded is not None:
+            p2, s2 = folded
             dw = sum(p2[k * ca:(k + 1) * ca, k * cb:(k + 1) * cb] for k in range(fold))
             return dw, s2.reshape(fold, ca).sum(0)
     return _rows(d_out).t() @ _rows(inp), _rows(d_out).sum(0, dtype=torch.float32)
@@ -54,8 +56,9 @@ def _conv_weight_grad(d_out: torch.Tensor, x: torch.Tensor, dims):
 
     d_out (B, N, O), x (B, N, C) channels-last over the grid of `dims`.  One pass of the library's kernel where it serves
     the widths; otherwise the GEMM library on the unfolded input (2-D) or tap by tap."""
-    if PF.cols_gemm_supported(d_out, x, dims):
-        return PF.cols_gemm(d_out, x, col_sums=True, grid=dims)
+    served = PF.try_cols_gemm(d_out, x, dims)
+    if served is not None:
+        return served
     k = dims.conv_k
     grid = (dims.grid_h, dims.grid_w) + ((dims.grid_d,) if dims.grid_d > 0 else ())
     d_b = _rows(d_out).sum(0, dtype=torch.float32)
@@ -189,8 +192,13 @@ def _train_params(names, params, device):
     """The parameters as `layer_train_forward` takes them: on the input's device, each on a 16-byte boundary (a view into
     one flat vector of all parameters need not start on one)."""
     large = torch.bfloat16 if all(p.dtype == torch.bfloat16 for n, p in zip(names, params) if n in _LARGE) else torch.float32
-    return {n: _aligned(p.detach().to(device=device, dtype=large if n in _LARGE else torch.float32))
-            for n, p in zip(names, params)}
+    out = {}
+    for n, p in zip(names, params):
+        dtype = large if n in _LARGE else torch.float32
+        if p.dtype != dtype or p.device != device:
+            p = p.detach().to(device=device, dtype=dtype)
+        out[n] = _aligned(p)
+    return out
 
 
 def _layer_train_forward(ctx, x, uniform, dims, names, params):
@@ -198,15 +206,26 @@ def _layer_train_forward(ctx, x, uniform, dims, names, params):
     x, uniform = _aligned(x), None if uniform is None else _aligned(uniform)
     y, saved = PF.layer_train_forward(x, uniform, _train_params(names, params, x.device), dims)
     ctx.save_for_backward(x, uniform, saved)
-    ctx.dims, ctx.param_like = dims, [(n, p.shape, p.dtype) for n, p in zip(names, params)]
+    ctx.dims, ctx.names, ctx.like = dims, names, params
     return y
 
 
+# where a parameter's gradient lies among those of the library call
+_GRADIENT_ORDER = {names: ([names.index(n) for n in order], [order.index(n) for n in names]) for names, order in
+                   ((_LAYER_PARAMS, PF.TRAIN_GRADIENTS), (_PLUS_PARAMS, PF.TRAIN_GRADIENTS_PLUS))}
+
+
 def _layer_train_backward(ctx, x, uniform, dy, saved, need):
-    """(dx, the parameters' gradients); need: which of them are wanted."""
-    dx, grads = PF.layer_train_backward(x, uniform, dy, saved, ctx.dims, ctx.needs_input_grad[0])
-    return dx, tuple(grads[n].view(shape).to(dtype) if wanted else None
-                     for (n, shape, dtype), wanted in zip(ctx.param_like, need))
+    """(dx, the parameters' gradients); need: which of them are wanted.  Of the parameters (`ctx.like`) only sizes and types
+    are read."""
+    dx, grads = PF.layer_train_gradients(x, uniform, dy, saved, ctx.dims, ctx.needs_input_grad[0])
+    to_buffer, from_buffer = _GRADIENT_ORDER[ctx.names]
+    views = torch._utils._unflatten_dense_tensors(grads, [ctx.like[k] for k in to_buffer])
+    out = []
+    for p, k, wanted in zip(ctx.like, from_buffer, need):
+        g = views[k] if wanted else None
+        out.append(g if g is None or p.dtype == torch.float32 else g.to(p.dtype))
+    return dx, tuple(out)
 
 
 class PhysicsAttentionMfmaFunction(torch.autograd.Function):
@@ -269,7 +288,7 @@ class LayerResidualNormFunction(torch.autograd.Function):
         y, saved, normed = PF.layer_train_forward(x, None, _train_params(_LAYER_PARAMS, params, x.device), dims, residual, w32,
                                                   _aligned(ln_b.detach().float()), eps)
         ctx.save_for_backward(x, saved, y, w32)
-        ctx.dims, ctx.param_like = dims, [(n, p.shape, p.dtype) for n, p in zip(_LAYER_PARAMS, params)]
+        ctx.dims, ctx.names, ctx.like = dims, _LAYER_PARAMS, params
         ctx.eps, ctx.ln_dtypes = eps, (ln_w.dtype, ln_b.dtype)
         _keep_parameters(ctx, ln_w)
         return y, normed
@@ -280,7 +299,7 @@ class LayerResidualNormFunction(torch.autograd.Function):
         need = ctx.needs_input_grad
         d, dg, db = _through_norm(ctx, y, w32, d_y, d_normed)
         if d is None:
-            return (None,) * (6 + len(ctx.param_like))
+            return (None,) * (6 + len(ctx.like))
         dx, grads = _layer_train_backward(ctx, x, None, d, saved, need[6:])
         return (dx, d if need[1] else None, None, dg, db, None) + grads
 
@@ -725,6 +744,8 @@ def mlp(x: torch.Tensor, layers: torch.nn.Sequential) -> torch.Tensor:
     dtype = compute_dtype(x)
     if len(layers) != 3 or not unhooked(layers) or not _linears_served(dtype, layers[0], layers[2]):
         return layers(x)
+    if not torch.is_autocast_enabled("cuda"):
+        return linear(layers[1](linear(x, layers[0].weight, layers[0].bias)), layers[2].weight, layers[2].bias)
     with torch.autocast("cuda", enabled=False):
         h = linear(x.to(dtype), layers[0].weight, layers[0].bias)
         return linear(layers[1](h), layers[2].weight, layers[2].bias)
@@ -790,8 +811,7 @@ def mlp_residual(normed: torch.Tensor, x: torch.Tensor, layers: torch.nn.Sequent
         norm = (None, None, 0.0)
         if next_ln is not None and _layer_norm_served(x, next_ln) and tuple(next_ln.normalized_shape) == (C,):
             norm = (next_ln.weight, next_ln.bias, next_ln.eps)
-        with torch.autocast("cuda", enabled=False):
-            out = MlpResidualFunction.apply(_aligned(normed), _aligned(x), lin1.weight, lin1.bias, lin2.weight, lin2.bias, *norm)
+        out = MlpResidualFunction.apply(_aligned(normed), _aligned(x), lin1.weight, lin1.bias, lin2.weight, lin2.bias, *norm)
         return out if norm[0] is not None else (out, None)
     return mlp(normed, layers) + x, None
 
@@ -815,6 +835,8 @@ def linear_as_autocast(x: torch.Tensor, lin: torch.nn.Linear) -> torch.Tensor:
     """lin(x) in training on `linear` where it serves the module, for an x in the type autocast would run it in."""
     if not _linears_served(compute_dtype(x), lin):
         return lin(x)
+    if not torch.is_autocast_enabled("cuda"):
+        return linear(x, lin.weight, lin.bias)
     with torch.autocast("cuda", enabled=False):
         return linear(x, lin.weight, lin.bias)
 

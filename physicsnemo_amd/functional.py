@@ -7,6 +7,7 @@ kernels on torch's current stream.  `params` is the dict produced by
 from __future__ import annotations
 
 from ctypes import byref
+from functools import lru_cache
 from typing import NamedTuple
 
 import torch
@@ -28,7 +29,12 @@ class LayerDims(NamedTuple):
     conv_tap_major: int = 0  # 1: convolution weights are laid out (c_out, k, k[, k], c_in) instead of torch's order
 
     def c(self) -> _lib.PaShape:
-        return _lib.PaShape(*self)
+        return _c_shape(self)
+
+
+@lru_cache(maxsize=256)
+def _c_shape(dims: LayerDims) -> _lib.PaShape:  # the library reads it only
+    return _lib.PaShape(*dims)
 
 
 _PARAM_FIELDS = [f for f, _ in _lib.PaParams._fields_]
@@ -198,35 +204,33 @@ def layer_forward(x, params, dims: LayerDims, residual=None, ln_weight=None, ln_
         if x.dtype != torch.bfloat16:
             raise TypeError("fp8-e4m3 weights need bfloat16 activations")
         code = _lib.PA_BF16_W8
-    shape = dims.c()
-    nbytes = lib.pa_workspace_bytes(code, byref(shape))
+    shape, device, stream = byref(dims.c()), x.device, _lib.current_stream_ptr(x.device)
+    nbytes = lib.pa_workspace_bytes(code, shape)
     if nbytes < 0:
         _lib.check(int(nbytes), "pa_workspace_bytes")
-    workspace = torch.empty(int(nbytes), dtype=torch.uint8, device=x.device)
-    y = torch.empty(dims.B, dims.N, dims.C, dtype=x.dtype, device=x.device)
+    workspace = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    y = torch.empty(dims.B, dims.N, dims.C, dtype=x.dtype, device=device)
     ln_out = torch.empty_like(y) if ln_weight is not None else None
-    tok = (torch.empty(dims.B, dims.H, dims.S, dims.D, dtype=torch.float32, device=x.device)
+    tok = (torch.empty(dims.B, dims.H, dims.S, dims.D, dtype=torch.float32, device=device)
            if return_slice_tokens else None)
-    tail = _c_tail(residual, ln_weight, ln_bias, ln_eps, ln_out)
+    tail = byref(_c_tail(residual, ln_weight, ln_bias, ln_eps, ln_out))
+    c_params = byref(_c_params(params))
     blob = None
-    if code in (_lib.PA_BF16, _lib.PA_BF16_W8) and lib.pa_query_path(code, byref(shape)) == 1:
+    if code != _lib.PA_F32 and lib.pa_query_path(code, shape) == 1:
         # fused MFMA path: the repacked parameters are kept with the parameter set and reused until it changes
         # (fp8-e4m3 weights: the repacking kernel reads the bytes and scales, so they are expanded once, here)
         blob = params.get("_mfma_blob")
         if blob is None:
-            n = lib.pa_mfma_buffer_bytes(byref(shape), _lib.PA_BUF_BLOB)
-            blob = torch.empty(int(n), dtype=torch.uint8, device=x.device)
-            _lib.check(lib.pa_mfma_pack_params(byref(shape), byref(_c_params(params)), blob.data_ptr(),
-                                               _lib.current_stream_ptr(x.device)), "pa_mfma_pack_params")
+            n = lib.pa_mfma_buffer_bytes(shape, _lib.PA_BUF_BLOB)
+            blob = torch.empty(int(n), dtype=torch.uint8, device=device)
+            _lib.check(lib.pa_mfma_pack_params(shape, c_params, blob.data_ptr(), stream), "pa_mfma_pack_params")
             params["_mfma_blob"] = blob
     if blob is not None:
-        _lib.check(lib.pa_mfma_layer_forward(byref(shape), byref(_c_params(params)), blob.data_ptr(), x.data_ptr(),
-                                             y.data_ptr(), byref(tail), _lib.ptr(tok), workspace.data_ptr(), int(nbytes),
-                                             _lib.current_stream_ptr(x.device)), "pa_mfma_layer_forward")
+        _lib.check(lib.pa_mfma_layer_forward(shape, c_params, blob.data_ptr(), x.data_ptr(), y.data_ptr(), tail, _lib.ptr(tok),
+                                             workspace.data_ptr(), nbytes, stream), "pa_mfma_layer_forward")
     else:
-        _lib.check(lib.pa_layer_forward(code, byref(shape), byref(_c_params(params)), x.data_ptr(), y.data_ptr(),
-                                        byref(tail), _lib.ptr(tok), workspace.data_ptr(), int(nbytes),
-                                        _lib.current_stream_ptr(x.device)), "pa_layer_forward")
+        _lib.check(lib.pa_layer_forward(code, shape, c_params, x.data_ptr(), y.data_ptr(), tail, _lib.ptr(tok),
+                                        workspace.data_ptr(), nbytes, stream), "pa_layer_forward")
     out = y if (residual is None and ln_out is None) else (y, ln_out)
     return (out, tok) if return_slice_tokens else out
 
@@ -715,44 +719,66 @@ def layer_train_forward(x, uniform, params: dict, dims: LayerDims, residual=None
     return (y, saved) if ln_out is None else (y, saved, ln_out)
 
 
-def layer_train_backward(x, uniform, dy, saved, dims: LayerDims, need_dx: bool = True):
-    """(dx or None, gradients by parameter name, float32 views of one buffer) of `layer_train_forward`; the parameters are
-    those of the forward call, kept in `saved`."""
+def layer_train_gradients(x, uniform, dy, saved, dims: LayerDims, need_dx: bool = True):
+    """(dx or None, one float32 buffer with the gradients of all parameters in the order of `TRAIN_GRADIENTS` /
+    `TRAIN_GRADIENTS_PLUS`, each in its parameter's layout) of `layer_train_forward`; the parameters are those of the forward
+    call, kept in `saved`."""
     _need_cuda(x, uniform, dy, saved)
-    lib, shape, plus = _lib.load(), dims.c(), uniform is not None
-    nbytes = lib.pa_layer_train_bytes(byref(shape), int(plus), _lib.PA_TRAIN_BACKWARD)
+    lib, shape, plus = _lib.load(), byref(dims.c()), uniform is not None
+    nbytes = lib.pa_layer_train_bytes(shape, int(plus), _lib.PA_TRAIN_BACKWARD)
     if nbytes < 0:
         _lib.check(int(nbytes), "pa_layer_train_bytes")
-    workspace = torch.empty(int(nbytes), dtype=torch.uint8, device=x.device)
-    grads = torch.empty(lib.pa_layer_train_bytes(byref(shape), int(plus), _lib.PA_TRAIN_GRADS) // 4, dtype=torch.float32,
+    workspace = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    grads = torch.empty(lib.pa_layer_train_bytes(shape, int(plus), _lib.PA_TRAIN_GRADS) // 4, dtype=torch.float32,
                         device=x.device)
     dx = torch.empty_like(x) if need_dx else None
     _lib.check(lib.pa_layer_train_backward(
-        byref(shape), None, byref(_lib.PaPlusParams()) if plus else None, x.data_ptr(), _lib.ptr(uniform), dy.data_ptr(),
-        saved.data_ptr(), _lib.ptr(dx), grads.data_ptr(), workspace.data_ptr(), int(nbytes),
+        shape, None, byref(_lib.PaPlusParams()) if plus else None, x.data_ptr(), _lib.ptr(uniform), dy.data_ptr(),
+        saved.data_ptr(), _lib.ptr(dx), grads.data_ptr(), workspace.data_ptr(), nbytes,
         _lib.current_stream_ptr(x.device)), "pa_layer_train_backward")
+    return dx, grads
+
+
+_TRAIN_TAIL = ("out_linear_weight", "out_linear_bias", "qkv_project_weight", "in_project_slice_weight",
+               "in_project_slice_bias", "temperature")
+TRAIN_GRADIENTS = ("in_project_x_weight", "in_project_fx_weight", "in_project_x_bias", "in_project_fx_bias") + _TRAIN_TAIL
+TRAIN_GRADIENTS_PLUS = ("in_project_x_weight", "in_project_x_bias") + _TRAIN_TAIL + (
+    "proj_temperature_0_weight", "proj_temperature_0_bias", "proj_temperature_2_weight", "proj_temperature_2_bias")
+
+
+def layer_train_backward(x, uniform, dy, saved, dims: LayerDims, need_dx: bool = True):
+    """(dx or None, gradients by parameter name, float32 views of one buffer) of `layer_train_forward`."""
+    dx, grads = layer_train_gradients(x, uniform, dy, saved, dims, need_dx)
     C, HD, S, D, H = dims.C, dims.H * dims.D, dims.S, dims.D, dims.H
     taps = dims.conv_k ** (3 if dims.grid_d > 0 else 2) if dims.conv_k > 0 else 1
-    proj = ["in_project_x"] + ([] if plus else ["in_project_fx"])
-    sizes = [(n + "_weight", HD * C * taps) for n in proj] + [(n + "_bias", HD) for n in proj]
-    sizes += [("out_linear_weight", C * HD), ("out_linear_bias", C), ("qkv_project_weight", 3 * D * D),
-              ("in_project_slice_weight", S * D), ("in_project_slice_bias", S), ("temperature", H)]
-    if plus:
-        sizes += [("proj_temperature_0_weight", S * D), ("proj_temperature_0_bias", S), ("proj_temperature_2_weight", S),
-                  ("proj_temperature_2_bias", 1)]
-    parts = grads.split([n for _, n in sizes])
-    return dx, {name: part for (name, _), part in zip(sizes, parts)}
+    size = {"in_project_x_weight": HD * C * taps, "in_project_fx_weight": HD * C * taps, "in_project_x_bias": HD,
+            "in_project_fx_bias": HD, "out_linear_weight": C * HD, "out_linear_bias": C, "qkv_project_weight": 3 * D * D,
+            "in_project_slice_weight": S * D, "in_project_slice_bias": S, "temperature": H, "proj_temperature_0_weight": S * D,
+            "proj_temperature_0_bias": S, "proj_temperature_2_weight": S, "proj_temperature_2_bias": 1}
+    names = TRAIN_GRADIENTS if uniform is None else TRAIN_GRADIENTS_PLUS
+    return dx, dict(zip(names, grads.split([size[n] for n in names])))
+
+
+def _cols_gemm_bytes(a: torch.Tensor, b: torch.Tensor, grid: LayerDims | None) -> int:
+    """Workspace of `cols_gemm` for these operands, 0 or less where it does not serve them."""
+    if not (a.is_cuda and a.dtype == b.dtype and a.dtype in (torch.float32, torch.bfloat16)) or a.numel() == 0:
+        return 0
+    if a.data_ptr() % 16 or b.data_ptr() % 16:
+        return 0
+    ca = a.shape[-1]
+    return _lib.load().pa_weight_grad_workspace_bytes(_lib.dtype_code(a.dtype), a.numel() // ca, ca, b.shape[-1],
+                                                      byref(grid.c()) if grid is not None else None)
 
 
 def cols_gemm_supported(a: torch.Tensor, b: torch.Tensor, grid: LayerDims | None = None) -> bool:
     """True if `cols_gemm` serves d out = a (..., ca), input = b (..., cb) (see pa_weight_grad for the shapes)."""
-    if not (a.is_cuda and a.dtype == b.dtype and a.dtype in (torch.float32, torch.bfloat16)) or a.numel() == 0:
-        return False
-    if a.data_ptr() % 16 or b.data_ptr() % 16:
-        return False
-    ca = a.shape[-1]
-    return _lib.load().pa_weight_grad_workspace_bytes(_lib.dtype_code(a.dtype), a.numel() // ca, ca, b.shape[-1],
-                                                      byref(grid.c()) if grid is not None else None) > 0
+    return _cols_gemm_bytes(a, b, grid) > 0
+
+
+def try_cols_gemm(a: torch.Tensor, b: torch.Tensor, grid: LayerDims | None = None):
+    """`cols_gemm(a, b, col_sums=True, grid=grid)` where it serves the operands, else None."""
+    nbytes = _cols_gemm_bytes(a, b, grid)
+    return _cols_gemm(a, b, True, grid, nbytes) if nbytes > 0 else None
 
 
 def cols_gemm(a: torch.Tensor, b: torch.Tensor, col_sums: bool = False, grid: LayerDims | None = None):
@@ -760,23 +786,27 @@ def cols_gemm(a: torch.Tensor, b: torch.Tensor, col_sums: bool = False, grid: La
     (ca, cb): the weight-gradient product d W = d out^T . in.  With `grid` (the dims of a structured layer) b's rows are
     gathered at every tap of its convolution and the result is (ca, cb, k, ..., k).  With `col_sums` the column sums of
     a (the matching bias gradient) come back as well, from the same pass."""
+    rows = a.numel() // a.shape[-1]
+    nbytes = _lib.load().pa_weight_grad_workspace_bytes(_lib.dtype_code(a.dtype), rows, a.shape[-1], b.shape[-1],
+                                                        byref(grid.c()) if grid is not None else None)
+    if nbytes < 0:
+        _lib.check(int(nbytes), "pa_weight_grad_workspace_bytes")
+    return _cols_gemm(a, b, col_sums, grid, nbytes)
+
+
+def _cols_gemm(a, b, col_sums: bool, grid: LayerDims | None, nbytes: int):
     _need_cuda(a, b)
-    lib = _lib.load()
     ca, cb = a.shape[-1], b.shape[-1]
     rows = a.numel() // ca
     if b.numel() // cb != rows:
         raise ValueError("cols_gemm needs the same number of rows on both sides")
-    code = _lib.dtype_code(a.dtype)
-    geom = byref(grid.c()) if grid is not None else None
-    nbytes = lib.pa_weight_grad_workspace_bytes(code, rows, ca, cb, geom)
-    if nbytes < 0:
-        _lib.check(int(nbytes), "pa_weight_grad_workspace_bytes")
-    workspace = torch.empty(int(nbytes), dtype=torch.uint8, device=a.device)
+    workspace = torch.empty(nbytes, dtype=torch.uint8, device=a.device)
     taps = (grid.conv_k,) * (3 if grid.grid_d > 0 else 2) if grid is not None and grid.conv_k > 0 else ()
     out = torch.empty(ca, cb, *taps, dtype=torch.float32, device=a.device)
     sums = torch.empty(ca, dtype=torch.float32, device=a.device) if col_sums else None
-    _lib.check(lib.pa_weight_grad(code, rows, a.data_ptr(), ca, b.data_ptr(), cb, geom, workspace.data_ptr(), int(nbytes),
-                                  out.data_ptr(), _lib.ptr(sums), _lib.current_stream_ptr(a.device)), "pa_weight_grad")
+    _lib.check(_lib.load().pa_weight_grad(_lib.dtype_code(a.dtype), rows, a.data_ptr(), ca, b.data_ptr(), cb,
+                                          byref(grid.c()) if grid is not None else None, workspace.data_ptr(), nbytes,
+                                          out.data_ptr(), _lib.ptr(sums), _lib.current_stream_ptr(a.device)), "pa_weight_grad")
     return (out, sums) if col_sums else out
 
 

@@ -20,7 +20,7 @@ import torch.nn as nn
 
 from . import functional as PF
 from .autograd import (LayerResidualNormFunction, PhysicsAttentionFunction, PhysicsAttentionMfmaFunction,
-                       PhysicsAttentionPlusFunction, PhysicsAttentionPlusMfmaFunction, _aligned)
+                       PhysicsAttentionPlusFunction, PhysicsAttentionPlusMfmaFunction, _aligned, unhooked)
 
 __all__ = ["PhysicsAttentionBase", "PhysicsAttentionIrregularMesh", "PhysicsAttentionStructuredMesh2D",
            "PhysicsAttentionStructuredMesh3D"]
@@ -30,6 +30,21 @@ def _kernel_layout(p: torch.Tensor) -> torch.Tensor:
     """Convolution weights (O, C, k, k[, k]) -> tap-major (O, k, k[, k], C), the order in which the implicit GEMM
     walks its reduction index (`conv_tap_major` of the shape); everything else unchanged."""
     return p.movedim(1, -1) if p.ndim > 2 else p
+
+
+_LARGE = ("in_project_x_weight", "in_project_fx_weight", "out_linear_weight")
+
+
+def _parameter(module: nn.Module, name: str) -> torch.Tensor:
+    """module.<name>, looked up among its parameters first (nn.Module's own look-up is a Python call)."""
+    p = module._parameters.get(name)
+    return p if p is not None else getattr(module, name)  # parametrised, pruned: an attribute of another kind
+
+
+def _identity_dropout(m: nn.Module) -> bool:
+    """True where calling m returns its argument and nothing else happens."""
+    return (type(m) is nn.Dropout and not (m.training and m.p > 0) and unhooked(m) and
+            not torch.nn.modules.module._has_any_global_hook())
 
 
 class PhysicsAttentionBase(nn.Module):
@@ -80,29 +95,27 @@ class PhysicsAttentionBase(nn.Module):
         return PF.LayerDims(x.shape[0], x.shape[1], self.dim, self.heads, self.dim_head, self.slice_num, gh, gw, k, gd,
                             1 if k > 0 else 0)  # kernel_params() hands convolution weights over tap-major
 
+    def _layer_parameters(self):
+        """(name in the C ABI, module that holds it, attribute) of every parameter."""
+        m = self._modules  # the modules by name, without nn.Module's attribute look-up
+        x, sl, out = m["in_project_x"], m["in_project_slice"], m["out_linear"]
+        if self.plus:
+            pt0, pt2 = self.proj_temperature[0], self.proj_temperature[2]
+            mid = (("proj_temperature_0_weight", pt0, "weight"), ("proj_temperature_0_bias", pt0, "bias"),
+                   ("proj_temperature_2_weight", pt2, "weight"), ("proj_temperature_2_bias", pt2, "bias"))
+        else:
+            fx = m["in_project_fx"]
+            mid = (("in_project_fx_weight", fx, "weight"), ("in_project_fx_bias", fx, "bias"))
+        return (("in_project_x_weight", x, "weight"), ("in_project_x_bias", x, "bias")) + mid + (
+            ("in_project_slice_weight", sl, "weight"), ("in_project_slice_bias", sl, "bias"),
+            ("temperature", self, "temperature"), ("qkv_project_weight", m["qkv_project"], "weight"),
+            ("out_linear_weight", out, "weight"), ("out_linear_bias", out, "bias"))
+
     def kernel_params(self, dtype: torch.dtype, device: torch.device) -> dict:
         """Parameters as the C ABI wants them: the three large weights in ``dtype``, everything else float32,
         contiguous.  Cached until a parameter is modified in place, replaced or moved."""
-        named = [
-            ("in_project_x_weight", self.in_project_x.weight, True),
-            ("in_project_x_bias", self.in_project_x.bias, False),
-        ]
-        if self.plus:
-            named += [("proj_temperature_0_weight", self.proj_temperature[0].weight, False),
-                      ("proj_temperature_0_bias", self.proj_temperature[0].bias, False),
-                      ("proj_temperature_2_weight", self.proj_temperature[2].weight, False),
-                      ("proj_temperature_2_bias", self.proj_temperature[2].bias, False)]
-        else:
-            named += [("in_project_fx_weight", self.in_project_fx.weight, True),
-                      ("in_project_fx_bias", self.in_project_fx.bias, False)]
-        named += [
-            ("in_project_slice_weight", self.in_project_slice.weight, False),
-            ("in_project_slice_bias", self.in_project_slice.bias, False),
-            ("temperature", self.temperature, False),
-            ("qkv_project_weight", self.qkv_project.weight, False),
-            ("out_linear_weight", self.out_linear.weight, True),
-            ("out_linear_bias", self.out_linear.bias, False),
-        ]
+        named = [(name, _parameter(module, attr), attr == "weight" and name in _LARGE)
+                 for name, module, attr in self._layer_parameters()]
         fp8 = self.fp8_weights and dtype == torch.bfloat16
         stamp = (dtype, device, fp8) + tuple((p.data_ptr(), p._version, p.dtype) for _, p, _ in named)
         hit = self._kernel_param_cache.get("stamp")
@@ -219,7 +232,8 @@ class PhysicsAttentionBase(nn.Module):
             return self.forward_with_noise(x, None)
         else:
             y = PF.layer_forward(x, self.kernel_params(x.dtype, x.device), self.layer_dims(x))
-        return self.out_dropout(y)  # identity unless training with dropout > 0 (reference :499)
+        drop = self._modules["out_dropout"]
+        return y if _identity_dropout(drop) else drop(y)  # identity unless training with dropout > 0 (reference :499)
 
     def forward_with_noise(self, x: torch.Tensor, noise_u: torch.Tensor | None, stages: bool = False):
         """Transolver++ forward (reference :166-170, :530-532) through the stage-level kernels.  ``noise_u``
