@@ -613,6 +613,108 @@ __global__ __launch_bounds__(kAttnThreads) void slice_combine_attn_kernel(const 
 }
 
 // ------------------------------------------------------------------------------------------------
+// narrow_combine_attn_kernel<D, S>: combine_partials_kernel and slice_combine_attn_kernel in one launch for narrow heads, with
+// their sums in their order, bit for bit: 32 threads per slice, everything of a (b, h) in registers and LDS, sizes known to
+// the compiler.  Bound by latency: one trip for partials and weights, four barriers.  D = 16, S = 32 (us, the two launches before ->
+// now): 16 workgroups of 128 partials 4.5 + 11.0 -> 9.4, 32 of 64 partials 4.8 + 10.6 -> 7.0.
+// ------------------------------------------------------------------------------------------------
+template <int D, int S>
+__global__ __launch_bounds__(32 * S) void narrow_combine_attn_kernel(const float *__restrict__ partials, int G,
+                                                                    int64_t partial_stride, const float *__restrict__ w_qkv,
+                                                                    float *__restrict__ slice_token,
+                                                                    float *__restrict__ slice_norm,
+                                                                    float *__restrict__ out_token) {
+  constexpr int T = 32 * S, D1 = D + 1, LD = D + 4, NOUT = S * D1, kAhead = 16, KEYS = S / 16;
+  static_assert((S == 16 || S == 32 || S == 64) && D % 4 == 0, "16 threads per slice in the softmax, whole float4 rows");
+  __shared__ float quarter[4][NOUT];
+  __shared__ __align__(16) float tok[S * LD], wq[3 * D * LD], qkv[3][S * LD], prob[S * (S + 1)];
+  const int t = threadIdx.x, bh = blockIdx.x;
+  float w[(3 * D * D + T - 1) / T];
+#pragma unroll
+  for (int k = 0; k < (3 * D * D + T - 1) / T; ++k) w[k] = k * T + t < 3 * D * D ? w_qkv[k * T + t] : 0.f;
+  const int per = (G + 3) / 4;
+  const float *src = partials + (int64_t)bh * NOUT;
+  for (int item = t; item < 4 * NOUT; item += T) {  // kAhead loads in flight, added in index order
+    const int qt = item / NOUT, o = item - qt * NOUT, g0 = qt * per, g1 = min(G, g0 + per);
+    float acc = 0.f;
+    for (int g = g0; g < g1; g += kAhead) {
+      float v[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) v[u] = src[(int64_t)min(g + u, g1 - 1) * partial_stride + o];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) acc += g + u < g1 ? v[u] : 0.f;
+    }
+    quarter[qt][o] = acc;
+  }
+#pragma unroll
+  for (int k = 0; k < (3 * D * D + T - 1) / T; ++k) {
+    const int i = k * T + t;
+    if (i < 3 * D * D) wq[(i / D) * LD + i % D] = w[k];
+  }
+  __syncthreads();
+  auto total = [&](int o) { return ((quarter[0][o] + quarter[1][o]) + quarter[2][o]) + quarter[3][o]; };
+  for (int i = t; i < S * D; i += T) {
+    const int s = i / D, d = i % D;
+    const float cnt = total(s * D1 + D) + kSliceNormEps, val = total(s * D1 + d) / cnt;
+    tok[s * LD + d] = val;
+    if (slice_token) slice_token[(int64_t)bh * S * D + i] = val;
+    if (slice_norm && d == 0) slice_norm[(int64_t)bh * S + s] = cnt;
+  }
+  __syncthreads();
+  auto dot = [](const float *a, const float *b) {  // in index order
+    float acc = 0.f;
+#pragma unroll
+    for (int k = 0; k < D; k += 4) {
+      const float4 x = *reinterpret_cast<const float4 *>(a + k), y = *reinterpret_cast<const float4 *>(b + k);
+      acc = fmaf(x.w, y.w, fmaf(x.z, y.z, fmaf(x.y, y.y, fmaf(x.x, y.x, acc))));
+    }
+    return acc;
+  };
+#pragma unroll
+  for (int i = t; i < S * 3 * D; i += T) {
+    const int s = i % S, e = i / S;
+    qkv[e / D][s * LD + e % D] = dot(tok + s * LD, wq + e * LD);
+  }
+  __syncthreads();
+  // The first half of the workgroup: slice s = t / 16, keys t % 16 + 16 j.  A sum over a slice's keys pairs them as a sum over the
+  // 64 lanes of a wave does.
+  const int s = t >> 4, l = t & 15;
+  float inv = 0.f;
+  if (s < S) {
+    const float scale = rsqrtf((float)D);
+    float e[KEYS], mx = -INFINITY, sum;
+#pragma unroll
+    for (int j = 0; j < KEYS; ++j) {
+      e[j] = dot(qkv[0] + s * LD, qkv[1] + (l + 16 * j) * LD) * scale;
+      asm("" : "+v"(e[j]));  // rounded, as the kernel that stores it has it: no fused multiply-subtract below
+      mx = fmaxf(mx, e[j]);
+    }
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+#pragma unroll
+    for (int j = 0; j < KEYS; ++j) {
+      e[j] = expf(e[j] - mx);
+      prob[s * (S + 1) + l + 16 * j] = e[j];
+    }
+    if constexpr (KEYS == 4) sum = (e[0] + e[2]) + (e[1] + e[3]);
+    else if constexpr (KEYS == 2) sum = e[0] + e[1];
+    else sum = e[0];
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+    inv = 1.f / sum;
+  }
+  __syncthreads();
+  if (s < S) {
+    for (int d = l; d < D; d += 16) {
+      float acc = 0.f;
+#pragma unroll
+      for (int u = 0; u < S; ++u) acc = fmaf(prob[s * (S + 1) + u], qkv[2][u * LD + d], acc);
+      out_token[((int64_t)bh * S + s) * D + d] = acc * inv;
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
 // deslice_kernel: grid (row tiles of R, B-independent; H).  out_x[m, h*D + d] = sum_s w[m, h, s] * tok'[b, h, s, d]
 // A row tile never straddles two batches (the host picks tiles per batch).
 // ------------------------------------------------------------------------------------------------
@@ -1267,8 +1369,24 @@ int combine_partials(const pa_shape &s, const float *partials, int64_t G, const 
   return launch_status();
 }
 
+// Partials of a (b, h) that one workgroup sums itself: 256 of 32 x 17 floats take 3.6 us at the 64 bytes a clock that a CU gets
+// from L2, about what the launch that spreads them over the chip costs with its start.
+constexpr int64_t kFewPartials = 256;
+
+template <int D>
+static int narrow_combine_attention(const pa_shape &s, const pa_params &p, const float *partials, int64_t G, float *slice_token,
+                                    float *slice_norm, float *out_token, hipStream_t st) {
+  hipLaunchKernelGGL((narrow_combine_attn_kernel<D, 32>), dim3((unsigned)(s.B * s.H)), dim3(32 * 32), 0, st, partials, (int)G,
+                     s.B * s.H * s.S * (s.D + 1), p.qkv_project_weight, slice_token, slice_norm, out_token);
+  return launch_status();
+}
+
 int combine_attention(const pa_shape &s, const pa_params &p, const float *partials, int64_t G, float *slice_token,
                       float *slice_norm, float *out_token, hipStream_t st) {
+  if (s.S == 32 && out_token && G > 8 && G <= kFewPartials) {
+    if (s.D == 8) return narrow_combine_attention<8>(s, p, partials, G, slice_token, slice_norm, out_token, st);
+    if (s.D == 16) return narrow_combine_attention<16>(s, p, partials, G, slice_token, slice_norm, out_token, st);
+  }
   size_t lds = combine_attn_lds_bytes(s);
   const size_t wq_bytes = (size_t)3 * s.D * (s.D + 1) * 4;
   const int stage_w = lds + wq_bytes <= 96 * 1024 ? 1 : 0;  // qkv weight rows in LDS when they fit comfortably

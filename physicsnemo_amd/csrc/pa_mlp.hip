@@ -1903,9 +1903,10 @@ static size_t split_lds(int F) {
 }
 // Rounds of the split kernel (64 rows per CU) that are shorter than one of the owning kernel's.  C = 256, F = 1024 (us): the
 // split kernel 22 - 29 / 48 - 53 for one / two rounds, about 78 for three; the owning kernel 57 - 67 for up to 32 768 rows, 73 for
-// 49 152.  C = 512, F = 2048: 50 - 74 / 122 - 150 against 120 - 129 / 131 - 157; F = 128 .. 512 alike.
+// 49 152.  C = 512, F = 2048: 50 - 74 / 122 - 150 against 120 - 129 / 131 - 157, where a second launch's start eats the difference
+// of two rounds (49 512 rows, a model of 7 blocks: 3 763 against 3 703).  F = 128 .. 512 alike.
 template <int C>
-constexpr int64_t kSplitRounds = 2;
+constexpr int64_t kSplitRounds = C == 256 ? 2 : 1;
 
 // The rows for which launch_split is called by the launchers below: whole rounds of the chip stay with the kernel that owns
 // its rows, what is left over (all of it, for small inputs) goes to the split kernel as long as its own rounds are the shorter

@@ -63,7 +63,7 @@ def test_mlp_matches_fp32_oracle(rows_shape, C, Fh):
 
 @pytest.mark.parametrize("rows,C,Fh,train", [(*c, t) for c in [
     (65, 256, 256), (31, 256, 512), (16385, 256, 256), (65536 + 65, 256, 256), (65536 + 32769, 256, 256), (65536 + 65, 256, 320),
-    (33, 512, 256), (8193, 512, 768), (32768 + 31, 512, 256), (32768 + 32767, 512, 256), (63, 512, 320),
+    (33, 512, 256), (8193, 512, 768), (32768 + 31, 512, 256), (32768 + 16384, 512, 256), (32768 + 16385, 512, 256), (63, 512, 320),
 ] for t in (False, True) if not t or c[1] == 256])
 def test_mlp_rows_beyond_whole_rounds_of_the_chip(rows, C, Fh, train):
     """Rows are split between the kernel that owns its rows and the one whose waves share them (256 compute units: 65 536 rows

@@ -466,3 +466,18 @@ def test_fp16_autocast_is_served_and_memory_does_not_grow():
             hip(xb)
         torch.cuda.synchronize()
         assert torch.cuda.memory_allocated() - before < 1 << 20
+
+
+@pytest.mark.parametrize("C,H,N", [(64, 8, 2048), (64, 8, 2049), (64, 4, 2305), (32, 4, 16 * 256 + 17), (32, 4, 256 * 256), (64, 4, 256 * 256 + 1)])
+def test_fp32_narrow_heads_attend_in_one_launch_with_the_same_bits(C, H, N):
+    """float32 heads of 8 / 16 channels, 32 slices: 9 to 256 partial sums (256 points each) are added and attended in one
+    launch, fewer and more in the kernels that the stage entry points run; both give the same bits."""
+    announce("narrow combine + attention", C, H, N)
+    torch.manual_seed(5)
+    layer = pn.PhysicsAttentionIrregularMesh(C, heads=H, dim_head=C // H, slice_num=32, use_te=False).eval().cuda()
+    x = torch.randn(2, N, C, device="cuda")
+    with torch.no_grad():
+        stages = layer.forward_stages(x)
+        y, tok = PF.layer_forward(x, layer.kernel_params(x.dtype, x.device), layer.layer_dims(x), return_slice_tokens=True)
+    assert torch.isfinite(y).all()
+    assert torch.equal(tok, stages["tok"]) and torch.equal(y, stages["y"])
