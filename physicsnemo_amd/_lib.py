@@ -22,6 +22,7 @@ EXPORTED = [
     "pa_mfma_project_softmax", "pa_mfma_slice_reduce", "pa_mfma_project_softmax_reduce", "pa_mfma_partial_groups",
      "pa_mfma_combine_attention", "pa_mfma_deslice_project", "pa_mlp_query", "pa_mlp_workspace_bytes", "pa_mlp_forward", "pa_mlp_pack", "pa_mlp_pack_e4m3", "pa_mlp_input_ln_query", "pa_mlp_forward_packed_ln",
      "pa_mlp_forward_packed", "pa_mlp_train_forward", "pa_mlp_backward_workspace_bytes", "pa_mlp_backward",
+    "pa_norm_mlp_backward_workspace_bytes", "pa_norm_mlp_backward",
     "pa_rows_gemm", "pa_slice_weighted_sum", "pa_backward_query", "pa_backward_point_tiles",
     "pa_slice_attention_backward", "pa_slice_softmax_backward", "pa_slice_softmax_plus",
     "pa_backward_point_tiles_plus", "pa_slice_softmax_plus_backward", "pa_slice_cross_attention_mix",
@@ -162,6 +163,11 @@ def load() -> ctypes.CDLL:
     lib.pa_mlp_backward.restype = c_int
     lib.pa_mlp_backward.argtypes = [c_int, c_int64, c_int64, c_int64, POINTER(PaMlpParams), c_void_p, c_void_p, c_void_p,
                                     c_void_p, c_void_p, c_int64, c_void_p]
+    lib.pa_norm_mlp_backward_workspace_bytes.restype = c_int64
+    lib.pa_norm_mlp_backward_workspace_bytes.argtypes = [c_int, c_int64, c_int64, c_int64]
+    lib.pa_norm_mlp_backward.restype = c_int
+    lib.pa_norm_mlp_backward.argtypes = [c_int, c_int64, c_int64, c_int64, POINTER(PaMlpParams)] + [c_void_p] * 4 + [
+        c_float] + [c_void_p] * 3 + [c_int64, c_void_p]
     lib.pa_mlp_pack.restype = c_int
     lib.pa_mlp_pack.argtypes = [c_int, c_int64, c_int64, POINTER(PaMlpParams), c_void_p, c_int64, c_void_p]
     lib.pa_mlp_input_ln_query.restype = c_int

@@ -260,7 +260,12 @@ def _layernorm_backward(ctx, x, dy, w32, eps, add=None):
     weight where the result is differentiated again."""
     if not torch.is_grad_enabled():
         return PF.layernorm_backward(x, dy, w32, eps, add)
-    weight, xf, df = _kept_parameters(ctx)[-1], x.float(), dy.float()
+    return _layernorm_grad_ops(x, dy, _kept_parameters(ctx)[-1], eps, add)
+
+
+def _layernorm_grad_ops(x, dy, weight, eps, add=None):
+    """(dx + add, d weight, d bias) of LayerNorm as tensor operations that can be differentiated again."""
+    xf, df = x.float(), dy.float()
     centred = xf - xf.mean(-1, keepdim=True)
     rstd = torch.rsqrt(centred.square().mean(-1, keepdim=True) + eps)
     xh, g = centred * rstd, df * weight.float()
@@ -302,6 +307,31 @@ class LayerResidualNormFunction(torch.autograd.Function):
             return (None,) * (6 + len(ctx.like))
         dx, grads = _layer_train_backward(ctx, x, None, d, saved, need[6:])
         return (dx, d if need[1] else None, None, dg, db, None) + grads
+
+
+class LayerResidualFunction(torch.autograd.Function):
+    """(y, LayerNorm(y)) as `LayerResidualNormFunction`, the second without a gradient of its own: for a consumer that takes
+    both and differentiates the LayerNorm itself (`NormMlpResidualFunction`)."""
+
+    @staticmethod
+    def forward(ctx, x, residual, dims, ln_w, ln_b, eps, *params):
+        ctx.set_materialize_grads(False)
+        y, saved, normed = PF.layer_train_forward(x, None, _train_params(_LAYER_PARAMS, params, x.device), dims, residual,
+                                                  _aligned(ln_w.detach().float()), _aligned(ln_b.detach().float()), eps)
+        ctx.save_for_backward(x, saved)
+        ctx.dims, ctx.names, ctx.like = dims, _LAYER_PARAMS, params
+        ctx.mark_non_differentiable(normed)
+        return y, normed
+
+    @staticmethod
+    def backward(ctx, d_y, _):
+        x, saved = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        if d_y is None:
+            return (None,) * (6 + len(ctx.like))
+        d = _aligned(d_y.to(x.dtype))
+        dx, grads = _layer_train_backward(ctx, x, None, d, saved, need[6:])
+        return (dx, d if need[1] else None, None, None, None, None) + grads
 
 
 class PhysicsAttentionPlusMfmaFunction(torch.autograd.Function):
@@ -799,18 +829,95 @@ class MlpResidualFunction(torch.autograd.Function):
         return (dx, dy if need[1] else None, *grads, *d_ln, None)
 
 
+class NormMlpResidualFunction(torch.autograd.Function):
+    """(y, next LayerNorm(y)) for y = x + Linear(gelu(Linear(LayerNorm(x)))) of a bf16 block (next_w None: y alone), given
+    `normed` = LayerNorm(x) from the kernel that formed x; the backward is one library call from dy, x and normed."""
+
+    @staticmethod
+    def forward(ctx, x, normed, ln_w, ln_b, eps, w1, b1, w2, b2, next_w, next_b, next_eps):
+        ctx.set_materialize_grads(False)
+        w1_16, w2_16 = (_aligned(w.detach().to(torch.bfloat16)) for w in (w1, w2))
+        b1_32, b2_32 = _aligned(b1.detach().to(torch.float32, copy=True)), _aligned(b2.detach().float())  # b1: read again
+        ln_w32 = _aligned(ln_w.detach().to(torch.float32, copy=True))
+        ctx.param_dtypes = tuple(p.dtype for p in (w1, b1, w2, b2, ln_w, ln_b))
+        _keep_parameters(ctx, ln_w, ln_b, w1, b1, w2, *(() if next_w is None else (next_w,)))
+        ctx.norm_eps = eps
+        packed = PF.mlp_pack(w1_16, w2_16)
+        if next_w is None:
+            ctx.save_for_backward(x, normed, w1_16, b1_32, w2_16, ln_w32)
+            return PF.mlp_forward_packed(normed, packed, b1_32, b2_32, residual=x, train=True)
+        w32 = _aligned(next_w.detach().float())
+        y, nxt = PF.mlp_forward_packed(normed, packed, b1_32, b2_32, residual=x, ln_weight=w32,
+                                       ln_bias=_aligned(next_b.detach().float()), ln_eps=next_eps, train=True)
+        ctx.save_for_backward(x, normed, w1_16, b1_32, w2_16, ln_w32, y, w32)
+        ctx.eps, ctx.ln_dtypes = next_eps, (next_w.dtype, next_b.dtype)
+        return y, nxt
+
+    @staticmethod
+    def backward(ctx, dy, d_next=None):
+        x, normed, w1, b1, w2, ln_w, *nxt = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        d_nxt = (None, None)
+        if nxt:
+            dy, *d_nxt = _through_norm(ctx, nxt[0], nxt[1], dy, d_next)
+        if dy is None:
+            return (None,) * 12
+        dy16 = _aligned(dy.to(x.dtype))
+        if torch.is_grad_enabled():  # create_graph: the same formulas as tensor ops on the parameters, differentiable again
+            with torch.autocast("cuda", enabled=False):
+                lw, lb, p1, pb1, p2 = _kept_parameters(ctx)[:5]
+                w1, b1, w2 = (p.to(x.dtype) for p in (p1, pb1, p2))
+                u = torch.nn.functional.layer_norm(x.float(), x.shape[-1:], lw.float(), lb.float(), ctx.norm_eps).to(x.dtype)
+                h = torch.nn.functional.linear(u, w1, b1)
+                act, dh = torch.nn.functional.gelu(h), torch.ops.aten.gelu_backward(dy16 @ w2, h)
+                dx, d_ln, d_lb = _layernorm_grad_ops(x, dh @ w1, lw, ctx.norm_eps, dy16)
+                rows = lambda d, i: (_rows(d).float().t() @ _rows(i).float(), _rows(d).sum(0, dtype=torch.float32))
+                grads = (*rows(dh, u), *rows(dy16, act), d_ln, d_lb)
+        else:
+            dx, *grads = PF.norm_mlp_backward(normed, dy16, x, w1, b1, w2, ln_w, ctx.norm_eps)
+        d_w1, d_b1, d_w2, d_b2, d_ln, d_lb = (g.to(t) for g, t in zip(grads, ctx.param_dtypes))
+        return (dx, None, d_ln, d_lb, None, d_w1, d_b1, d_w2, d_b2, *d_nxt, None)
+
+
+def _mlp_fused(dtype, x: torch.Tensor, layers) -> bool:
+    """True where the fused bf16 MLP kernels train `layers` on rows like x's as autocast would run them."""
+    lin1, act, lin2 = layers if len(layers) == 3 else (None,) * 3
+    C = x.shape[-1]
+    return (dtype == x.dtype == torch.bfloat16 and unhooked(layers) and _linears_served(dtype, lin1, lin2) and
+            type(act) is torch.nn.GELU and unhooked(act) and act.approximate == "none" and lin1.bias is not None and
+            lin2.bias is not None and lin1.in_features == lin2.out_features == C and
+            PF.mlp_backward_supported(x.dtype, x.numel() // C, C, lin1.out_features))
+
+
+def _next_norm(x: torch.Tensor, next_ln: torch.nn.LayerNorm | None):
+    """(weight, bias, eps) of a LayerNorm that may ride in the MLP kernel's tail, else Nones."""
+    if next_ln is not None and _layer_norm_served(x, next_ln) and tuple(next_ln.normalized_shape) == (x.shape[-1],):
+        return next_ln.weight, next_ln.bias, next_ln.eps
+    return None, None, 0.0
+
+
+def norm_mlp_fused(x: torch.Tensor, ln: torch.nn.LayerNorm, layers) -> bool:
+    """True where `norm_mlp_residual_of` trains y = x + Mlp(ln(x)) on rows like x's."""
+    C = x.shape[-1]
+    return (type(ln) is torch.nn.LayerNorm and unhooked(ln) and _layer_norm_served(x, ln) and tuple(ln.normalized_shape) == (C,) and
+            _mlp_fused(compute_dtype(x), x, layers) and
+            PF.norm_mlp_backward_supported(x.dtype, x.numel() // C, C, layers[0].out_features))
+
+
+def norm_mlp_residual_of(x: torch.Tensor, normed: torch.Tensor, ln: torch.nn.LayerNorm, layers,
+                         next_ln: torch.nn.LayerNorm | None = None):
+    """(x + Mlp(ln(x)), next_ln of it or None) in training where `norm_mlp_fused`, given normed = ln(x) without a graph."""
+    norm = _next_norm(x, next_ln)
+    out = NormMlpResidualFunction.apply(_aligned(x), _aligned(normed), ln.weight, ln.bias, ln.eps, layers[0].weight,
+                                        layers[0].bias, layers[2].weight, layers[2].bias, *norm)
+    return out if norm[0] is not None else (out, None)
+
+
 def mlp_residual(normed: torch.Tensor, x: torch.Tensor, layers: torch.nn.Sequential, next_ln: torch.nn.LayerNorm | None = None):
     """(x + Mlp(normed), next_ln of it or None) in training, as autocast would run it: on the fused MLP kernels where they
     serve the rows (with the LayerNorm that follows in their tail), else on `mlp`."""
-    C, dtype = x.shape[-1], compute_dtype(normed)
-    lin1, act, lin2 = layers if len(layers) == 3 else (None,) * 3
-    if (dtype == normed.dtype == x.dtype == torch.bfloat16 and unhooked(layers) and _linears_served(dtype, lin1, lin2) and
-            type(act) is torch.nn.GELU and unhooked(act) and act.approximate == "none" and lin1.bias is not None and
-            lin2.bias is not None and lin1.in_features == lin2.out_features == C and
-            PF.mlp_backward_supported(x.dtype, x.numel() // C, C, lin1.out_features)):
-        norm = (None, None, 0.0)
-        if next_ln is not None and _layer_norm_served(x, next_ln) and tuple(next_ln.normalized_shape) == (C,):
-            norm = (next_ln.weight, next_ln.bias, next_ln.eps)
+    if normed.dtype == x.dtype and _mlp_fused(compute_dtype(normed), x, layers):
+        norm, (lin1, _, lin2) = _next_norm(x, next_ln), layers
         out = MlpResidualFunction.apply(_aligned(normed), _aligned(x), lin1.weight, lin1.bias, lin2.weight, lin2.bias, *norm)
         return out if norm[0] is not None else (out, None)
     return mlp(normed, layers) + x, None

@@ -1180,8 +1180,68 @@ int pa_mlp_backward(int dtype, int64_t rows, int64_t C, int64_t F, const pa_mlp_
       !aligned16(workspace))
     return PA_ERR_ALIGN;
   if (workspace_bytes < need) return PA_ERR_WORKSPACE;
-  return pa::mlp::hidden_backward(rows, C, F, p->w1, p->b1, p->w2, u, dy, act, d_hidden, workspace, compute_units(),
+  return pa::mlp::hidden_backward(rows, C, F, p->w1, p->b1, p->w2, u, dy, act, d_hidden, workspace, nullptr, compute_units(),
                                   static_cast<hipStream_t>(stream));
+}
+
+namespace {
+struct NormMlpPlan {
+  int64_t act, dh, blob, w1_t, partials, work, work_bytes, total;
+};
+NormMlpPlan norm_mlp_plan(int64_t rows, int64_t C, int64_t F) {
+  NormMlpPlan p{};
+  int64_t off = 0;
+  auto take = [&](int64_t bytes) {
+    const int64_t at = off;
+    off += round_up(bytes, 256);
+    return at;
+  };
+  p.act = take(rows * F * 2);
+  p.dh = take(rows * F * 2);
+  p.blob = take(pa::mlp::hidden_backward_blob_bytes(C, F));
+  p.w1_t = take(C * F * 2);
+  p.partials = take(pa::norm::rows_ln_backward_groups(rows, compute_units()) * 2 * C * 4);
+  const int64_t w1 = pa::wgrad::workspace_bytes(PA_BF16, rows, F, C, 1, compute_units()),
+                w2 = pa::wgrad::workspace_bytes(PA_BF16, rows, C, F, 1, compute_units());
+  p.work_bytes = w1 <= 0 || w2 <= 0 ? 0 : w1 > w2 ? w1 : w2;
+  p.work = take(p.work_bytes);
+  p.total = p.work_bytes > 0 ? off : 0;
+  return p;
+}
+}  // namespace
+
+int64_t pa_norm_mlp_backward_workspace_bytes(int dtype, int64_t rows, int64_t C, int64_t F) {
+  const int64_t hidden = pa_mlp_backward_workspace_bytes(dtype, rows, C, F);
+  if (hidden < 0) return hidden;
+  if (!pa::norm::rows_ln_backward_supported(rows, C, F)) return PA_ERR_UNSUPPORTED;
+  const int64_t total = norm_mlp_plan(rows, C, F).total;
+  return total > 0 ? total : PA_ERR_UNSUPPORTED;
+}
+
+int pa_norm_mlp_backward(int dtype, int64_t rows, int64_t C, int64_t F, const pa_mlp_params *p, const void *u, const void *dy,
+                         const void *x, const float *ln_gamma, float ln_eps, void *dx, float *grads, void *workspace,
+                         int64_t workspace_bytes, void *stream) {
+  Range entry("pa_norm_mlp_backward");
+  const int64_t need = pa_norm_mlp_backward_workspace_bytes(dtype, rows, C, F);
+  if (need < 0) return (int)need;
+  if (!p || !p->w1 || !p->b1 || !p->w2 || !u || !dy || !x || !ln_gamma || !dx || !grads || !workspace) return PA_ERR_NULL;
+  if (!aligned16(p->w1) || !aligned16(p->w2) || !aligned16(u) || !aligned16(dy) || !aligned16(x) || !aligned16(dx) ||
+      !aligned16(grads) || !aligned16(workspace))
+    return PA_ERR_ALIGN;
+  if (workspace_bytes < need) return PA_ERR_WORKSPACE;
+  const NormMlpPlan w = norm_mlp_plan(rows, C, F);
+  char *ws = static_cast<char *>(workspace);
+  void *act = ws + w.act, *dh = ws + w.dh;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const int cus = compute_units();
+  float *d_w1 = grads, *d_b1 = d_w1 + F * C, *d_w2 = d_b1 + F, *d_b2 = d_w2 + C * F, *d_ln = d_b2 + C;
+  int rc = pa::mlp::hidden_backward(rows, C, F, p->w1, p->b1, p->w2, u, dy, act, dh, ws + w.blob, ws + w.w1_t, cus, st);
+  if (rc) return rc;
+  if ((rc = pa::norm::rows_ln_backward(rows, F, dh, ws + w.w1_t, x, ln_gamma, ln_eps, dy, dx,
+                                       reinterpret_cast<float *>(ws + w.partials), d_ln, cus, st)))
+    return rc;
+  if ((rc = pa::wgrad::product(PA_BF16, rows, dh, F, F, u, C, C, nullptr, ws + w.work, d_w1, d_b1, cus, st))) return rc;
+  return pa::wgrad::product(PA_BF16, rows, dy, C, C, act, F, F, nullptr, ws + w.work, d_w2, d_b2, cus, st);
 }
 
 int pa_mlp_input_ln_query(int dtype, int64_t rows, int64_t C, int64_t F) {

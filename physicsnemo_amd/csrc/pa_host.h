@@ -319,7 +319,7 @@ int train_forward(int64_t rows, int64_t C, int64_t F, const void *blob, const fl
 bool hidden_backward_supported(int64_t rows, int64_t C, int64_t F);
 int64_t hidden_backward_blob_bytes(int64_t C, int64_t F);
 int hidden_backward(int64_t rows, int64_t C, int64_t F, const void *w1, const float *b1, const void *w2, const void *u,
-                    const void *dy, void *act, void *dh, void *blob, int num_cu, hipStream_t st);
+                    const void *dy, void *act, void *dh, void *blob, void *w1_t, int num_cu, hipStream_t st);
 // the preprocess MLP (c_in <= 16 inputs -> F -> C in {256, 512}) with the hidden layer kept on chip; bf16 rows and weights
 bool premlp_supported(int dtype, int64_t rows, int64_t c_in, int64_t F, int64_t C);
 int64_t premlp_blob_bytes(int64_t F, int64_t C);
@@ -346,5 +346,12 @@ int conv_project_packed(int64_t B, int64_t N, int64_t C, int64_t gh, int64_t gw,
                         const void *w_x, const float *b_x, const void *w_fx, const float *b_fx, const void *x,
                         void *xm_pack, void *fx_pack, void *blob, int num_cu, hipStream_t st);
 }  // namespace mlp
+
+namespace norm {
+bool rows_ln_backward_supported(int64_t rows, int64_t C, int64_t K);
+int64_t rows_ln_backward_groups(int64_t rows, int num_cu);
+int rows_ln_backward(int64_t rows, int64_t K, const void *dh, const void *wt, const void *x, const float *gamma, float eps,
+                     const void *add, void *dx, float *partials, float *grads, int num_cu, hipStream_t st);
+}  // namespace norm
 
 }  // namespace pa

@@ -120,6 +120,21 @@ __device__ __forceinline__ float half_sum(float v) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// sum over the 32 lanes of this lane's half of the wave, returned in every lane of the half: DPP steps inside each
+// row of 16 lanes, then v_permlane16_swap pairs the two rows of the half
+__device__ __forceinline__ float half_wave_sum(float v) {
+  auto step = [](float x, auto ctrl) {
+    constexpr int c = decltype(ctrl)::value;
+    return x + __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), c, 0xf, 0xf, true));
+  };
+  v = step(v, std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
+  v = step(v, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+  v = step(v, std::integral_constant<int, 0x141>{});  // row_half_mirror
+  v = step(v, std::integral_constant<int, 0x140>{});  // row_mirror
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 // A 32 x 32 accumulator tile (lane (i, g) <-> point i, register r <-> channel rowmap(r, g)) to bf16 rows in natural
 // layout: `row` points at channel 0 of this lane's point.  Registers 4q..4q+3 hold channels 8q + 4g .. + 3; swapping
 // halves with lane ^ 32 gives each lane 8 consecutive channels (g = 0: 0-7 and 8-15, g = 1: 16-23 and 24-31), so a

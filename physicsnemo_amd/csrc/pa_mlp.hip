@@ -79,22 +79,6 @@ __device__ __forceinline__ u32x4 pack8(const float (&v)[8]) {
   return __builtin_bit_cast(u32x4, o);
 }
 
-// sum over the 32 lanes of this lane's half of the wave, returned in every lane of the half: DPP steps inside each
-// row of 16 lanes, then v_permlane16_swap pairs the two rows of the half
-__device__ __forceinline__ float half_wave_sum(float v) {
-  auto step = [](float x, auto ctrl) {
-    constexpr int c = decltype(ctrl)::value;
-    return x + __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), c, 0xf, 0xf, true));
-  };
-  v = step(v, std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
-  v = step(v, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
-  v = step(v, std::integral_constant<int, 0x141>{});  // row_half_mirror
-  v = step(v, std::integral_constant<int, 0x140>{});  // row_mirror
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-
 template <int C, int TAIL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void mlp_kernel(
     const u32x4 *__restrict__ blob, const float *__restrict__ b1, const float *__restrict__ b2,

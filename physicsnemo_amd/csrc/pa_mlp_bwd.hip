@@ -20,9 +20,10 @@ using mfma::u32x4;
 
 // Chunk c (32 hidden units) of the weight stream: 32 fragments, k-step ks of W1's rows 32 c .. + 31 (fragment 2 ks) and
 // of W2's columns 32 c .. + 31 (fragment 2 ks + 1), both with the reduction index running over the channels
+// and, with w1_t, W1^T (C, F)
 __global__ __launch_bounds__(256) void hidden_backward_pack_kernel(const uint16_t *__restrict__ w1,
                                                                    const uint16_t *__restrict__ w2,
-                                                                   u32x4 *__restrict__ blob, int C, int F) {
+                                                                   u32x4 *__restrict__ blob, u32x4 *__restrict__ w1_t, int C, int F) {
   const int KS = C / 16;
   const int64_t total = (int64_t)F / 32 * 2 * KS * 64;
   for (int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x; u < total; u += (int64_t)gridDim.x * 256) {
@@ -39,6 +40,15 @@ __global__ __launch_bounds__(256) void hidden_backward_pack_kernel(const uint16_
         e[j] = (uint32_t)w2[(int64_t)(col + 2 * j) * F + row] | ((uint32_t)w2[(int64_t)(col + 2 * j + 1) * F + row] << 16);
       blob[u] = e;
     }
+  }
+  if (!w1_t) return;
+  for (int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x; u < (int64_t)C * F / 8; u += (int64_t)gridDim.x * 256) {
+    const int c = (int)(u % C), f = (int)(u / C);  // eight hidden units from 8 f on
+    u32x4 e;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      e[j] = (uint32_t)w1[(int64_t)(8 * f + 2 * j) * C + c] | ((uint32_t)w1[(int64_t)(8 * f + 2 * j + 1) * C + c] << 16);
+    w1_t[((int64_t)c * F + 8 * f) / 8] = e;
   }
 }
 
@@ -185,9 +195,10 @@ bool hidden_backward_supported(int64_t rows, int64_t C, int64_t F) {
 int64_t hidden_backward_blob_bytes(int64_t C, int64_t F) { return 4 * C * F; }
 
 int hidden_backward(int64_t rows, int64_t C, int64_t F, const void *w1, const float *b1, const void *w2, const void *u,
-                    const void *dy, void *act, void *dh, void *blob, int cus, hipStream_t st) {
+                    const void *dy, void *act, void *dh, void *blob, void *w1_t, int cus, hipStream_t st) {
   hidden_backward_pack_kernel<<<(unsigned)(C * F / 4 / 256 < 1024 ? C * F / 4 / 256 : 1024), 256, 0, st>>>(
-      static_cast<const uint16_t *>(w1), static_cast<const uint16_t *>(w2), static_cast<u32x4 *>(blob), (int)C, (int)F);
+      static_cast<const uint16_t *>(w1), static_cast<const uint16_t *>(w2), static_cast<u32x4 *>(blob), static_cast<u32x4 *>(w1_t), (int)C,
+      (int)F);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return (int)e;
   const int64_t blocks = (rows + 255) / 256, chunks = F / 32;

@@ -497,6 +497,35 @@ def mlp_backward(u, dy, w1, b1, w2):
     return act, dh
 
 
+def norm_mlp_backward_supported(dtype: torch.dtype, rows: int, C: int, F: int) -> bool:
+    """True if `norm_mlp_backward` serves this shape (bfloat16, C = 256, F a multiple of 256)."""
+    if dtype != torch.bfloat16 or rows <= 0 or not mlp_supported(dtype, rows, C, F):
+        return False
+    return _lib.load().pa_norm_mlp_backward_workspace_bytes(_lib.PA_BF16, rows, C, F) > 0
+
+
+def norm_mlp_backward(u, dy, x, w1, b1, w2, ln_weight, ln_eps=1e-5):
+    """Backward of y = x + w2 . gelu(w1 . u + b1) + b2, u = LayerNorm(x): (dx, d w1, d b1, d w2, d b2, d ln_weight, d ln_bias),
+    the parameters' gradients float32.  u, dy, x (..., C), w1 (F, C), w2 (C, F) bfloat16; b1, ln_weight float32."""
+    _need_cuda(u, dy, x, w1, b1, w2, ln_weight)
+    lib = _lib.load()
+    C, F = w1.shape[1], w1.shape[0]
+    rows = u.numel() // C
+    nbytes = lib.pa_norm_mlp_backward_workspace_bytes(_lib.PA_BF16, rows, C, F)
+    if nbytes < 0:
+        _lib.check(int(nbytes), "pa_norm_mlp_backward_workspace_bytes")
+    workspace = torch.empty(nbytes, dtype=torch.uint8, device=u.device)
+    grads = torch.empty(2 * F * C + F + 3 * C, dtype=torch.float32, device=u.device)
+    dx = torch.empty_like(x)
+    params = _lib.PaMlpParams(w1.data_ptr(), b1.data_ptr(), w2.data_ptr(), None)
+    _lib.check(lib.pa_norm_mlp_backward(_lib.PA_BF16, rows, C, F, byref(params), u.data_ptr(), dy.data_ptr(), x.data_ptr(),
+                                        ln_weight.data_ptr(), float(ln_eps), dx.data_ptr(), grads.data_ptr(),
+                                        workspace.data_ptr(), nbytes, _lib.current_stream_ptr(u.device)),
+               "pa_norm_mlp_backward")
+    d_w1, d_b1, d_w2, d_b2, d_g, d_b = grads.split([F * C, F, C * F, C, C, C])
+    return dx, d_w1.view(F, C), d_b1, d_w2.view(C, F), d_b2, d_g, d_b
+
+
 class MfmaStages:
     """The bf16 MFMA kernels one by one (pa_mfma_* entry points) with their opaque buffers held as torch tensors.
 

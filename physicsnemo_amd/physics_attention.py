@@ -19,7 +19,7 @@ import torch
 import torch.nn as nn
 
 from . import functional as PF
-from .autograd import (LayerResidualNormFunction, PhysicsAttentionFunction, PhysicsAttentionMfmaFunction,
+from .autograd import (LayerResidualFunction, LayerResidualNormFunction, PhysicsAttentionFunction, PhysicsAttentionMfmaFunction,
                        PhysicsAttentionPlusFunction, PhysicsAttentionPlusMfmaFunction, _aligned, unhooked)
 
 __all__ = ["PhysicsAttentionBase", "PhysicsAttentionIrregularMesh", "PhysicsAttentionStructuredMesh2D",
@@ -300,9 +300,10 @@ class PhysicsAttentionBase(nn.Module):
             ln_weight=ln.weight.detach().float().contiguous(), ln_bias=ln.bias.detach().float().contiguous(),
             ln_eps=ln.eps)
 
-    def forward_block_with_grad(self, x: torch.Tensor, residual: torch.Tensor, ln: nn.LayerNorm):
+    def forward_block_with_grad(self, x: torch.Tensor, residual: torch.Tensor, ln: nn.LayerNorm, apart: bool = False):
         """Training: (self(x) + residual, its LayerNorm) with the add and the LayerNorm in the layer's last kernel, or None
-        where that does not serve the call (other types and widths, Transolver++, dropout, hooks on this module)."""
+        where that does not serve the call (other types and widths, Transolver++, dropout, hooks on this module).  apart:
+        the second without a graph, for `autograd.norm_mlp_residual_of`."""
         hooks = (self._forward_hooks, self._forward_pre_hooks, self._backward_hooks, self._backward_pre_hooks)
         if (type(self).forward is not PhysicsAttentionBase.forward or any(hooks) or self.plus or self.fp8_weights or
                 (self.training and self.out_dropout.p > 0) or not x.is_cuda or x.ndim != 3 or x.numel() == 0 or
@@ -314,7 +315,7 @@ class PhysicsAttentionBase(nn.Module):
         dims = self.layer_dims(x)
         if dims.C > 256 or not PF.layer_train_supported(x.dtype, dims):
             return None
-        return LayerResidualNormFunction.apply(
+        return (LayerResidualFunction if apart else LayerResidualNormFunction).apply(
             _aligned(x), _aligned(residual), dims, ln.weight, ln.bias, ln.eps, self.in_project_x.weight, self.in_project_x.bias,
             self.in_project_fx.weight, self.in_project_fx.bias, self.in_project_slice.weight, self.in_project_slice.bias,
             self.temperature, self.qkv_project.weight, self.out_linear.weight, self.out_linear.bias)

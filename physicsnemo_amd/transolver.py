@@ -235,14 +235,16 @@ class TransolverBlock(nn.Module):
         if self._needs_grad(fx):
             # training: the layer's autograd path, LayerNorms / MLP as differentiable tensor ops (reference :300-303)
             x_in, fx = (normed_in, fx) if normed_in is not None else PA.layer_norm_residual(fx, self.ln_1)
-            pair = None
+            pair, ln2, mlp = None, self.ln_mlp1[0], self.ln_mlp1[1]
+            apart = type(mlp) is Mlp and PA.unhooked(mlp) and PA.norm_mlp_fused(fx, ln2, mlp.layers)
             if isinstance(self.Attn, PhysicsAttentionBase):
-                pair = self.Attn.forward_block_with_grad(x_in, fx, self.ln_mlp1[0])
+                pair = self.Attn.forward_block_with_grad(x_in, fx, ln2, apart)
+            if pair is not None and apart:
+                return PA.norm_mlp_residual_of(*pair, ln2, mlp.layers, next_ln)
             if pair is None:
                 normed, fx1 = PA.layer_norm_residual(self.Attn(x_in) + fx, self.ln_mlp1[0])
             else:
                 fx1, normed = pair
-            mlp = self.ln_mlp1[1]
             if type(mlp) is not Mlp or not PA.unhooked(mlp):
                 return mlp(normed) + fx1, None
             return PA.mlp_residual(normed, fx1, mlp.layers, next_ln)

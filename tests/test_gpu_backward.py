@@ -7,6 +7,7 @@ import ctypes
 import numpy as np
 import pytest
 import torch
+import torch.nn.functional as F
 
 from oracle import torch_oracle as to
 import physicsnemo_amd as pn
@@ -1084,3 +1085,54 @@ def test_row_gemm_of_256_inputs_with_two_workgroups_per_cu(rows, c_out, bias):
     # float32 sums, rounded to bf16 once: at most half a unit in the last place (2^-9) of a value, sums far below it
     err = (y[0].double().cpu() - want).abs()
     assert (err <= 2.0 ** -8 * want.abs() + 1e-3).all()
+
+
+@pytest.mark.parametrize("rows,Fh", [(1, 256), (63, 1024), (64, 320), (65, 256), (2000, 1024), (32768, 256), (32769, 256), (65537, 64),
+                                     (2 * 256 * 128 + 1, 256)])
+def test_norm_mlp_backward_against_float64(rows, Fh):
+    """d x of y = x + Mlp(LayerNorm(x)) with the product that ends in the LayerNorm's backward in one kernel: blocks of 64 rows up
+    to 32 768 rows (256 compute units), of 128 beyond, workgroups with one block and with several, ragged last blocks."""
+    announce("norm mlp backward", rows, Fh)
+    C, eps, dev = 256, 1e-5, torch.device("cuda")
+    assert PF.norm_mlp_backward_supported(torch.bfloat16, rows, C, Fh)
+    gen = torch.Generator().manual_seed(rows + Fh)
+    rnd = lambda *n: torch.randn(*n, generator=gen)
+    x, dy = (2 * rnd(rows, C) + 0.5).bfloat16().to(dev), rnd(rows, C).bfloat16().to(dev)
+    w1, w2 = (rnd(Fh, C) / C ** 0.5).bfloat16().to(dev), (rnd(C, Fh) / Fh ** 0.5).bfloat16().to(dev)
+    b1, gam, bet = (0.1 * rnd(Fh)).to(dev), (0.5 + torch.rand(C, generator=gen)).to(dev), (0.1 * rnd(C)).to(dev)
+    u = F.layer_norm(x.float(), (C,), gam, bet, eps).bfloat16()
+    dx, d_w1, d_b1, d_w2, d_b2, d_g, d_b = PF.norm_mlp_backward(u, dy, x, w1, b1, w2, gam, eps)
+    # the same formulas in float64 from the same bf16 inputs (u as the kernel's producer rounded it)
+    xd, ud, dyd = x.double(), u.double(), dy.double()
+    h = ud @ w1.double().t() + b1.double()
+    phi = 0.5 * (1 + torch.erf(h / 2 ** 0.5))
+    dh = (dyd @ w2.double()) * (phi + h * torch.exp(-h * h / 2) / (2 * torch.pi) ** 0.5)
+    dn = dh @ w1.double()
+    centred = xd - xd.mean(-1, keepdim=True)
+    rstd = torch.rsqrt(centred.square().mean(-1, keepdim=True) + eps)
+    xh, gg = centred * rstd, dn * gam.double()
+    want = rstd * (gg - gg.mean(-1, keepdim=True) - xh * (gg * xh).mean(-1, keepdim=True)) + dyd
+    # dx is rounded once (1.7e-3), dh, gelu(h) and dn before it; sums over rows average those roundings out, but for few rows
+    assert_rel_l2(dx, want, "d x", 4e-3)
+    assert_rel_l2(d_w1, dh.t() @ ud, "d w1", 4e-3)
+    assert_rel_l2(d_b1, dh.sum(0), "d b1", 4e-3)
+    assert_rel_l2(d_w2, dyd.t() @ (h * phi), "d w2", 4e-3)
+    assert_rel_l2(d_b2, dyd.sum(0), "d b2", 1e-5)
+    assert_rel_l2(d_g, (dn * xh).sum(0), "d gamma", 6e-3)
+    assert_rel_l2(d_b, dn.sum(0), "d beta", 6e-3)
+
+
+def test_norm_mlp_backward_of_few_rows_with_infinities_keeps_them_where_they_are():
+    """A row with an infinite gradient leaves the other rows' d x as they are; rows past the end add nothing."""
+    C, Fh, rows, dev = 256, 256, 70, torch.device("cuda")
+    torch.manual_seed(0)
+    x, dy = torch.randn(rows, C, device=dev).bfloat16(), torch.randn(rows, C, device=dev).bfloat16()
+    w1, w2 = (torch.randn(Fh, C, device=dev) / 16).bfloat16(), (torch.randn(C, Fh, device=dev) / 16).bfloat16()
+    b1, gam = torch.zeros(Fh, device=dev), torch.ones(C, device=dev)
+    u = F.layer_norm(x.float(), (C,)).bfloat16()
+    clean = PF.norm_mlp_backward(u, dy, x, w1, b1, w2, gam, 0.0)
+    dy[rows - 1, 3] = float("inf")
+    dirty = PF.norm_mlp_backward(u, dy, x, w1, b1, w2, gam, 0.0)
+    assert all(torch.isfinite(t.float()).all() for t in clean)
+    assert torch.equal(clean[0][:rows - 1], dirty[0][:rows - 1]) and not torch.isfinite(dirty[0][rows - 1].float()).all()
+
