@@ -503,6 +503,14 @@ int pa_layer_train_forward(const pa_shape *shape, int weight_dtype, const pa_par
 int pa_layer_train_backward(const pa_shape *shape, const pa_params *p, const pa_plus_params *plus, const void *x,
                             const void *uniform, const void *dy, const void *saved, void *dx, float *grads, void *workspace,
                             int64_t workspace_bytes, void *stream);
+/* The same for a float32 layer with any head width of the general kernels (irregular or structured; H >= 2, H * S <= 512):
+ * x, y, dy, dx and all parameters float32, grads in the order above with d in_project_slice.weight (S, D), its bias (S) and
+ * d temperature (H) at the end.  pa_layer_train_f32_bytes: as pa_layer_train_bytes. */
+int64_t pa_layer_train_f32_bytes(const pa_shape *shape, int which);
+int pa_layer_train_f32_forward(const pa_shape *shape, const pa_params *p, const void *x, void *y, const pa_block_tail *tail,
+                               void *saved, void *workspace, int64_t workspace_bytes, void *stream);
+int pa_layer_train_f32_backward(const pa_shape *shape, const void *x, const void *dy, const void *saved, void *dx, float *grads,
+                                void *workspace, int64_t workspace_bytes, void *stream);
 
 /* ---- block MLP ---------------------------------------------------------------------------------- */
 

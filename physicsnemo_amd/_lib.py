@@ -34,6 +34,7 @@ EXPORTED = [
     "pa_mfma_backward_tables_bytes", "pa_mfma_backward_groups", "pa_mfma_slice_softmax_backward", "pa_point_backward_grads",
     "pa_point_backward_workspace_bytes", "pa_point_backward", "pa_output_backward_workspace_bytes", "pa_output_backward",
     "pa_layer_train_bytes", "pa_layer_train_forward", "pa_layer_train_backward",
+    "pa_layer_train_f32_bytes", "pa_layer_train_f32_forward", "pa_layer_train_f32_backward",
     "pa_cols_gemm_chunks", "pa_cols_gemm", "pa_residual_layernorm",
     "pa_mfma_layer_forward", "pa_rows_gemm_act", "pa_layernorm_backward_groups", "pa_layernorm_backward",
     "pa_layernorm_backward_add",
@@ -285,6 +286,12 @@ def load() -> ctypes.CDLL:
     lib.pa_layer_train_forward.argtypes = [ps, c_int, pp, pplus] + [c_void_p] * 3 + [pt] + [c_void_p] * 2 + [c_int64, c_void_p]
     lib.pa_layer_train_backward.restype = c_int
     lib.pa_layer_train_backward.argtypes = [ps, pp, pplus] + [c_void_p] * 7 + [c_int64, c_void_p]
+    lib.pa_layer_train_f32_bytes.restype = c_int64
+    lib.pa_layer_train_f32_bytes.argtypes = [ps, c_int]
+    lib.pa_layer_train_f32_forward.restype = c_int
+    lib.pa_layer_train_f32_forward.argtypes = [ps, pp, c_void_p, c_void_p, pt, c_void_p, c_void_p, c_int64, c_void_p]
+    lib.pa_layer_train_f32_backward.restype = c_int
+    lib.pa_layer_train_f32_backward.argtypes = [ps] + [c_void_p] * 6 + [c_int64, c_void_p]
     lib.pa_cols_gemm_chunks.restype = c_int64
     lib.pa_cols_gemm_chunks.argtypes = [c_int64, c_int64]
     lib.pa_weight_grad_workspace_bytes.restype = c_int64

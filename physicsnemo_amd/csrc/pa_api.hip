@@ -993,6 +993,52 @@ int pa_layer_train_backward(const pa_shape *shape, const pa_params *p, const pa_
                              static_cast<hipStream_t>(stream));
 }
 
+static int check_layer_train_f32(const pa_shape *shape) {
+  const int rc = check_backward_shape(PA_F32, shape);
+  if (rc) return rc;
+  return pa::train_f32::supported(*shape, compute_units()) ? PA_OK : PA_ERR_UNSUPPORTED;
+}
+
+int64_t pa_layer_train_f32_bytes(const pa_shape *shape, int which) {
+  const int rc = check_layer_train_f32(shape);
+  if (rc) return rc;
+  switch (which) {
+    case PA_TRAIN_SAVED: return pa::train_f32::saved_bytes(*shape);
+    case PA_TRAIN_FORWARD: return pa::train_f32::forward_workspace_bytes(*shape, compute_units());
+    case PA_TRAIN_BACKWARD: return pa::train_f32::backward_workspace_bytes(*shape, compute_units());
+    case PA_TRAIN_GRADS: return pa::train_f32::grad_floats(*shape) * 4;
+    default: return PA_ERR_UNSUPPORTED;
+  }
+}
+
+int pa_layer_train_f32_forward(const pa_shape *shape, const pa_params *p, const void *x, void *y, const pa_block_tail *tail,
+                               void *saved, void *workspace, int64_t workspace_bytes, void *stream) {
+  Range entry("pa_layer_train_f32_forward");
+  int rc = check_layer_train_f32(shape);
+  if (rc) return rc;
+  if ((rc = check_train_params(p, nullptr))) return rc;
+  if (!x || !y || !saved || !workspace) return PA_ERR_NULL;
+  if (!aligned16(x) || !aligned16(y) || !aligned16(saved) || !aligned16(workspace) || !aligned16(p->in_project_x_weight) ||
+      !aligned16(p->in_project_fx_weight) || !aligned16(p->out_linear_weight))
+    return PA_ERR_ALIGN;
+  if ((rc = check_tail(tail))) return rc;
+  if (workspace_bytes < pa::train_f32::forward_workspace_bytes(*shape, compute_units())) return PA_ERR_WORKSPACE;
+  return pa::train_f32::forward(*shape, *p, x, y, tail_active(tail) ? tail : nullptr, saved, workspace, compute_units(),
+                                static_cast<hipStream_t>(stream));
+}
+
+int pa_layer_train_f32_backward(const pa_shape *shape, const void *x, const void *dy, const void *saved, void *dx, float *grads,
+                                void *workspace, int64_t workspace_bytes, void *stream) {
+  Range entry("pa_layer_train_f32_backward");
+  const int rc = check_layer_train_f32(shape);
+  if (rc) return rc;
+  if (!x || !dy || !saved || !grads || !workspace) return PA_ERR_NULL;
+  if (!aligned16(x) || !aligned16(dy) || !aligned16(saved) || !aligned16(dx) || !aligned16(grads) || !aligned16(workspace))
+    return PA_ERR_ALIGN;
+  if (workspace_bytes < pa::train_f32::backward_workspace_bytes(*shape, compute_units())) return PA_ERR_WORKSPACE;
+  return pa::train_f32::backward(*shape, x, dy, saved, dx, grads, workspace, compute_units(), static_cast<hipStream_t>(stream));
+}
+
 int64_t pa_mfma_buffer_bytes(const pa_shape *shape, int which) {
   int rc = check_shape(PA_BF16, shape);
   if (rc) return rc;

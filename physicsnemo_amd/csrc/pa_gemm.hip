@@ -459,6 +459,8 @@ __global__ __launch_bounds__(512) void cols_gemm_kernel(const uint16_t *__restri
 // operand columns at a time go through LDS (coalesced 16-byte loads, double buffered), wave w multiplies the 64 x 64
 // sub-block (w & 1, w >> 1): per pair of rows 2 + 2 LDS words feed 4 MFMAs.  Row chunks come back as partials
 // P[g][oa][ob] (fixed-order sum by the caller); col_sums[g][oa] = sum_m A[m][oa] from the same pass (blockIdx.z == 0).
+// Bound by the float32 MFMAs, which neighbours found by 64-bit divisions for every row kept waiting: 4 x 85 x 85 grid points, 3 x 3
+// taps, 128 -> 2 x 128 (17 GFLOP) 212 us with them, 182 us with coordinates that are carried from step to step.
 // ------------------------------------------------------------------------------------------------
 constexpr int kF32Tile = 128, kF32Rows = 32;
 
@@ -488,6 +490,21 @@ __global__ __launch_bounds__(256) void cols_gemm_f32_kernel(const float *__restr
   // staging: 32 rows x 128 columns = 1024 float4 per operand, 4 per thread
   const int sr = t >> 5, sc = (t & 31) * 4;  // row 0..7 (+8 k), column of the float4
   float4 pa[4], pb[4];
+  // where the rows fetched next lie in the grid: found by division once, then by steps of 32 rows
+  const bool conv = grid.ks > 0;
+  const int gd = grid.gd > 0 ? grid.gd : 1, gw = conv ? grid.gw : 1, gh = conv ? grid.gh : 1, ksd = grid.gd > 0 ? grid.ks : 1;
+  const int pad = grid.ks / 2, pad_d = grid.gd > 0 ? pad : 0;
+  const int tu = conv ? tap / ksd / grid.ks - pad : 0, tv = conv ? tap / ksd % grid.ks - pad : 0, tz = conv ? tap % ksd - pad_d : 0;
+  const int64_t shift = ((int64_t)tu * gw + tv) * gd + tz;  // the neighbour, from the row
+  int ci[4], cj[4], cl[4];
+  const int step_l = kF32Rows % gd, step_j = kF32Rows / gd % gw, step_i = kF32Rows / gd / gw;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    unsigned n = conv ? (unsigned)((m_begin + sr + 8 * k) % grid.N) : 0u;
+    cl[k] = (int)(n % gd);
+    n /= gd;
+    ci[k] = (int)(n / gw), cj[k] = (int)(n % gw);
+  }
   auto fetch = [&](int64_t m0) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -495,9 +512,20 @@ __global__ __launch_bounds__(256) void cols_gemm_f32_kernel(const float *__restr
       pa[k] = pb[k] = float4{0.f, 0.f, 0.f, 0.f};
       if (m < m_end) {
         if (oa0 + sc < OA) pa[k] = *reinterpret_cast<const float4 *>(A + m * lda + oa0 + sc);
-        const int64_t mb = grid.ks > 0 ? grid_neighbour(grid, m, tap) : m;
-        if (ob0 + sc < OB && mb >= 0) pb[k] = *reinterpret_cast<const float4 *>(B + mb * ldb + ob0 + sc);
+        const bool inside = !conv | (((unsigned)(ci[k] + tu) < (unsigned)gh) & ((unsigned)(cj[k] + tv) < (unsigned)gw) &
+                                     ((unsigned)(cl[k] + tz) < (unsigned)gd));
+        if (ob0 + sc < OB && inside) pb[k] = *reinterpret_cast<const float4 *>(B + (m + shift) * ldb + ob0 + sc);
       }
+    }
+  };
+  auto advance = [&]() {  // the coordinates of the rows 32 further on
+    if (!conv) return;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      cl[k] += step_l, cj[k] += step_j, ci[k] += step_i;
+      if (cl[k] >= gd) cl[k] -= gd, ++cj[k];
+      if (cj[k] >= gw) cj[k] -= gw, ++ci[k];
+      while (ci[k] >= gh) ci[k] -= gh;  // the next batch element
     }
   };
   auto stage = [&](int buf) {
@@ -512,6 +540,7 @@ __global__ __launch_bounds__(256) void cols_gemm_f32_kernel(const float *__restr
   for (int64_t m0 = m_begin; m0 < m_end; m0 += kF32Rows) {
     stage(buf);
     __syncthreads();
+    if (m0 + kF32Rows < m_end) advance();
     fetch(m0 + kF32Rows < m_end ? m0 + kF32Rows : m0);  // the last block re-fetches itself: no branch around the loads
 #pragma unroll 4
     for (int k = 0; k < kF32Rows; k += 2) {

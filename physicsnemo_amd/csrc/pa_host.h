@@ -106,6 +106,19 @@ int backward(const pa_shape &s, bool plus, const void *x, const void *uniform, c
              float *grads, void *workspace, int num_cu, hipStream_t st);
 }  // namespace train
 
+namespace train_f32 {
+// the same for float32 layers: see pa_layer_train_f32_forward / _backward
+bool supported(const pa_shape &s, int num_cu);
+int64_t saved_bytes(const pa_shape &s);
+int64_t forward_workspace_bytes(const pa_shape &s, int num_cu);
+int64_t backward_workspace_bytes(const pa_shape &s, int num_cu);
+int64_t grad_floats(const pa_shape &s);
+int forward(const pa_shape &s, const pa_params &p, const void *x, void *y, const pa_block_tail *tail, void *saved, void *workspace,
+            int num_cu, hipStream_t st);
+int backward(const pa_shape &s, const void *x, const void *dy, const void *saved, void *dx, float *grads, void *workspace,
+             int num_cu, hipStream_t st);
+}  // namespace train_f32
+
 namespace general {
 int dequant_e4m3(const void *in, const float *scale, void *out, int64_t rows, int64_t cols, hipStream_t st);
 int project_inputs(int dtype, const pa_shape &s, const pa_params &p, const void *x, void *x_mid, void *fx_mid,

@@ -718,33 +718,41 @@ def output_backward(w_pack, dy, tok_out, w_out, dims: LayerDims):
     return d_tok, d_w, d_b
 
 
+def _train_bytes(dtype: torch.dtype, shape, plus: bool, which: int) -> int:
+    if dtype == torch.float32 and not plus:
+        return _lib.load().pa_layer_train_f32_bytes(shape, which)
+    return _lib.load().pa_layer_train_bytes(shape, int(plus), which) if dtype == torch.bfloat16 else 0
+
+
 def layer_train_supported(dtype: torch.dtype, dims: LayerDims, plus: bool = False) -> bool:
-    """True where a layer trains in the two library calls below (bf16, 32-wide heads)."""
-    if dtype != torch.bfloat16:
-        return False
-    return _lib.load().pa_layer_train_bytes(byref(dims.c()), 1 if plus else 0, _lib.PA_TRAIN_SAVED) > 0
+    """True where a layer trains in the two library calls below (bf16 with 32-wide heads; float32 without Transolver++)."""
+    return _train_bytes(dtype, byref(dims.c()), plus, _lib.PA_TRAIN_SAVED) > 0
 
 
 def layer_train_forward(x, uniform, params: dict, dims: LayerDims, residual=None, ln_weight=None, ln_bias=None, ln_eps=1e-5):
-    """(y, saved) of a bf16 layer, with ln_weight (y + residual, saved, LayerNorm(y + residual)).  `params`: the layer's own
-    parameters under the names of `pa_params` / `pa_plus_params`, the three large weights all float32 or all bfloat16 in
-    torch's layout, the rest float32."""
+    """(y, saved) of a layer, with ln_weight (y + residual, saved, LayerNorm(y + residual)).  `params`: the layer's own
+    parameters under the names of `pa_params` / `pa_plus_params` in torch's layout, float32; bf16 layers take the three large
+    weights all in bfloat16, too."""
     _need_cuda(x, uniform, residual, ln_weight, ln_bias, *params.values())
     if uniform is not None and (uniform.dtype != x.dtype or uniform.shape != (dims.B, dims.N, dims.H, dims.S)):
         raise ValueError("uniform samples must have the activation dtype and shape (B, N, H, S)")
-    lib, shape, plus = _lib.load(), dims.c(), uniform is not None
-    nbytes = lib.pa_layer_train_bytes(byref(shape), int(plus), _lib.PA_TRAIN_FORWARD)
+    lib, shape, plus = _lib.load(), byref(dims.c()), uniform is not None
+    nbytes = _train_bytes(x.dtype, shape, plus, _lib.PA_TRAIN_FORWARD)
     if nbytes < 0:
         _lib.check(int(nbytes), "pa_layer_train_bytes")
-    saved = torch.empty(lib.pa_layer_train_bytes(byref(shape), int(plus), _lib.PA_TRAIN_SAVED), dtype=torch.uint8, device=x.device)
-    workspace = torch.empty(int(nbytes), dtype=torch.uint8, device=x.device)
+    saved = torch.empty(_train_bytes(x.dtype, shape, plus, _lib.PA_TRAIN_SAVED), dtype=torch.uint8, device=x.device)
+    workspace = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
     y = torch.empty(dims.B, dims.N, dims.C, dtype=x.dtype, device=x.device)
     ln_out = torch.empty_like(y) if ln_weight is not None else None
-    tail = _c_tail(residual, ln_weight, ln_bias, ln_eps, ln_out)
-    _lib.check(lib.pa_layer_train_forward(
-        byref(shape), _lib.dtype_code(params["out_linear_weight"].dtype), byref(_c_params(params)),
-        _c_plus(params) if plus else None, x.data_ptr(), _lib.ptr(uniform), y.data_ptr(), byref(tail), saved.data_ptr(),
-        workspace.data_ptr(), int(nbytes), _lib.current_stream_ptr(x.device)), "pa_layer_train_forward")
+    tail = byref(_c_tail(residual, ln_weight, ln_bias, ln_eps, ln_out))
+    rest = (saved.data_ptr(), workspace.data_ptr(), nbytes, _lib.current_stream_ptr(x.device))
+    if x.dtype == torch.float32:
+        _lib.check(lib.pa_layer_train_f32_forward(shape, byref(_c_params(params)), x.data_ptr(), y.data_ptr(), tail, *rest),
+                   "pa_layer_train_f32_forward")
+    else:
+        _lib.check(lib.pa_layer_train_forward(
+            shape, _lib.dtype_code(params["out_linear_weight"].dtype), byref(_c_params(params)), _c_plus(params) if plus else None,
+            x.data_ptr(), _lib.ptr(uniform), y.data_ptr(), tail, *rest), "pa_layer_train_forward")
     return (y, saved) if ln_out is None else (y, saved, ln_out)
 
 
@@ -754,17 +762,18 @@ def layer_train_gradients(x, uniform, dy, saved, dims: LayerDims, need_dx: bool 
     call, kept in `saved`."""
     _need_cuda(x, uniform, dy, saved)
     lib, shape, plus = _lib.load(), byref(dims.c()), uniform is not None
-    nbytes = lib.pa_layer_train_bytes(shape, int(plus), _lib.PA_TRAIN_BACKWARD)
+    nbytes = _train_bytes(x.dtype, shape, plus, _lib.PA_TRAIN_BACKWARD)
     if nbytes < 0:
         _lib.check(int(nbytes), "pa_layer_train_bytes")
     workspace = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-    grads = torch.empty(lib.pa_layer_train_bytes(shape, int(plus), _lib.PA_TRAIN_GRADS) // 4, dtype=torch.float32,
-                        device=x.device)
+    grads = torch.empty(_train_bytes(x.dtype, shape, plus, _lib.PA_TRAIN_GRADS) // 4, dtype=torch.float32, device=x.device)
     dx = torch.empty_like(x) if need_dx else None
-    _lib.check(lib.pa_layer_train_backward(
-        shape, None, byref(_lib.PaPlusParams()) if plus else None, x.data_ptr(), _lib.ptr(uniform), dy.data_ptr(),
-        saved.data_ptr(), _lib.ptr(dx), grads.data_ptr(), workspace.data_ptr(), nbytes,
-        _lib.current_stream_ptr(x.device)), "pa_layer_train_backward")
+    rest = (saved.data_ptr(), _lib.ptr(dx), grads.data_ptr(), workspace.data_ptr(), nbytes, _lib.current_stream_ptr(x.device))
+    if x.dtype == torch.float32:
+        _lib.check(lib.pa_layer_train_f32_backward(shape, x.data_ptr(), dy.data_ptr(), *rest), "pa_layer_train_f32_backward")
+    else:
+        _lib.check(lib.pa_layer_train_backward(shape, None, byref(_lib.PaPlusParams()) if plus else None, x.data_ptr(),
+                                               _lib.ptr(uniform), dy.data_ptr(), *rest), "pa_layer_train_backward")
     return dx, grads
 
 

@@ -307,13 +307,14 @@ class PhysicsAttentionBase(nn.Module):
         hooks = (self._forward_hooks, self._forward_pre_hooks, self._backward_hooks, self._backward_pre_hooks)
         if (type(self).forward is not PhysicsAttentionBase.forward or any(hooks) or self.plus or self.fp8_weights or
                 (self.training and self.out_dropout.p > 0) or not x.is_cuda or x.ndim != 3 or x.numel() == 0 or
-                not x.dtype == residual.dtype == torch.bfloat16 or self._wants_fp16(x) or x.shape != residual.shape or
+                x.dtype != residual.dtype or x.dtype not in (torch.bfloat16, torch.float32) or self._wants_fp16(x) or
+                (x.dtype == torch.float32 and torch.is_autocast_enabled("cuda")) or x.shape != residual.shape or
                 not (ln.elementwise_affine and ln.bias is not None and tuple(ln.normalized_shape) == (self.dim,))):
             return None
         self._validate(x)
         x = self._prepare_input(x)
         dims = self.layer_dims(x)
-        if dims.C > 256 or not PF.layer_train_supported(x.dtype, dims):
+        if (dims.C > 256 and x.dtype == torch.bfloat16) or not PF.layernorm_supported(x) or not PF.layer_train_supported(x.dtype, dims):
             return None
         return (LayerResidualFunction if apart else LayerResidualNormFunction).apply(
             _aligned(x), _aligned(residual), dims, ln.weight, ln.bias, ln.eps, self.in_project_x.weight, self.in_project_x.bias,

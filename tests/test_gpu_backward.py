@@ -1136,3 +1136,34 @@ def test_norm_mlp_backward_of_few_rows_with_infinities_keeps_them_where_they_are
     assert all(torch.isfinite(t.float()).all() for t in clean)
     assert torch.equal(clean[0][:rows - 1], dirty[0][:rows - 1]) and not torch.isfinite(dirty[0][rows - 1].float()).all()
 
+
+@pytest.mark.parametrize("kind,dim,heads,dim_head,S,grid,kernel,N", [
+    ("irregular", 64, 2, 16, 32, None, 0, 1), ("irregular", 36, 3, 20, 8, None, 0, 333), ("irregular", 128, 8, 16, 64, None, 0, 2500),
+    ("structured2d", 128, 8, 16, 32, (13, 11), 3, 143), ("structured2d", 32, 4, 8, 16, (9, 14), 5, 126),
+    ("structured3d", 64, 4, 16, 32, (5, 6, 7), 3, 210),
+])
+def test_fp32_layer_in_two_calls_against_the_stages(monkeypatch, kind, dim, heads, dim_head, S, grid, kernel, N):
+    """A float32 layer's training step in one library call each way against the same stages called one by one: widths off the
+    tiles of 32 that turn the weights around, every tap, few and many partial sums, temperatures at and beyond the clamp."""
+    announce("fp32 train calls", kind, dim, heads, dim_head, S, grid)
+    temps = [0.2 + 5.6 * i / (heads - 1) for i in range(heads)]
+    temps[-1] = 5.0
+    kw = {} if grid is None else dict(spatial=grid, kernel=kernel)
+    _, hip = make_pair(kind, dim, heads, dim_head, S, sharpen=2.0, temps=temps, **kw)
+    hip.train()
+    x0, dy = torch.randn(2, N, dim, device="cuda"), torch.randn(2, N, dim, device="cuda")
+
+    def step():
+        x = x0.clone().requires_grad_(True)
+        hip.zero_grad(set_to_none=True)
+        y = hip(x)
+        y.backward(dy)
+        return [y.detach(), x.grad] + [p.grad.clone() for p in hip.parameters()]
+
+    assert PF.layer_train_supported(torch.float32, hip.layer_dims(x0))
+    got = step()
+    monkeypatch.setattr(PF, "layer_train_supported", lambda *a, **k: False)
+    want = step()
+    for g, w in zip(got, want):
+        assert_rel_l2(g, w, "two calls against the stages", 2e-6)
+
