@@ -188,16 +188,16 @@ _PLUS_PARAMS = ("in_project_x_weight", "in_project_x_bias", "in_project_slice_we
 _LARGE = ("in_project_x_weight", "in_project_fx_weight", "out_linear_weight")
 
 
-def _train_params(names, params, x):
-    """The parameters as `layer_train_forward` takes them for x: on its device, each on a 16-byte boundary (a view into one flat
-    vector of all parameters need not start on one)."""
-    as_they_are = x.dtype == torch.bfloat16 and all(p.dtype == torch.bfloat16 for n, p in zip(names, params) if n in _LARGE)
+def _train_params(names, params, device, dtype=torch.bfloat16):
+    """The parameters as `layer_train_forward` takes them for an input of `dtype`: on the input's device, each on a 16-byte
+    boundary (a view into one flat vector of all parameters need not start on one)."""
+    as_they_are = dtype == torch.bfloat16 and all(p.dtype == torch.bfloat16 for n, p in zip(names, params) if n in _LARGE)
     large = torch.bfloat16 if as_they_are else torch.float32
     out = {}
     for n, p in zip(names, params):
-        dtype = large if n in _LARGE else torch.float32
-        if p.dtype != dtype or p.device != x.device:
-            p = p.detach().to(device=x.device, dtype=dtype)
+        wanted = large if n in _LARGE else torch.float32
+        if p.dtype != wanted or p.device != device:
+            p = p.detach().to(device=device, dtype=wanted)
         out[n] = _aligned(p)
     return out
 
@@ -205,7 +205,7 @@ def _train_params(names, params, x):
 def _layer_train_forward(ctx, x, uniform, dims, names, params):
     """Forward of a bf16 layer with 32-wide heads in one library call; ctx keeps what the backward call reads."""
     x, uniform = _aligned(x), None if uniform is None else _aligned(uniform)
-    y, saved = PF.layer_train_forward(x, uniform, _train_params(names, params, x), dims)
+    y, saved = PF.layer_train_forward(x, uniform, _train_params(names, params, x.device, x.dtype), dims)
     ctx.save_for_backward(x, uniform, saved)
     ctx.dims, ctx.names, ctx.like = dims, names, params
     return y
@@ -291,8 +291,8 @@ class LayerResidualNormFunction(torch.autograd.Function):
     def forward(ctx, x, residual, dims, ln_w, ln_b, eps, *params):
         ctx.set_materialize_grads(False)
         w32 = _aligned(ln_w.detach().float())
-        y, saved, normed = PF.layer_train_forward(x, None, _train_params(_LAYER_PARAMS, params, x), dims, residual, w32,
-                                                  _aligned(ln_b.detach().float()), eps)
+        kernel_params = _train_params(_LAYER_PARAMS, params, x.device, x.dtype)
+        y, saved, normed = PF.layer_train_forward(x, None, kernel_params, dims, residual, w32, _aligned(ln_b.detach().float()), eps)
         ctx.save_for_backward(x, saved, y, w32)
         ctx.dims, ctx.names, ctx.like = dims, _LAYER_PARAMS, params
         ctx.eps, ctx.ln_dtypes = eps, (ln_w.dtype, ln_b.dtype)
@@ -317,7 +317,8 @@ class LayerResidualFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, residual, dims, ln_w, ln_b, eps, *params):
         ctx.set_materialize_grads(False)
-        y, saved, normed = PF.layer_train_forward(x, None, _train_params(_LAYER_PARAMS, params, x), dims, residual,
+        kernel_params = _train_params(_LAYER_PARAMS, params, x.device, x.dtype)
+        y, saved, normed = PF.layer_train_forward(x, None, kernel_params, dims, residual,
                                                   _aligned(ln_w.detach().float()), _aligned(ln_b.detach().float()), eps)
         ctx.save_for_backward(x, saved)
         ctx.dims, ctx.names, ctx.like = dims, _LAYER_PARAMS, params
