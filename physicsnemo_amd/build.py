@@ -15,7 +15,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 OBJ_DIR = os.path.join(CSRC, "build")
 LIB_PATH = os.path.join(PKG_DIR, "libphysattn.so")
 SOURCES = ["pa_api.hip", "pa_general.hip", "pa_mfma.hip", "pa_mlp.hip", "pa_mlp_bwd.hip", "pa_norm_bwd.hip", "pa_backward.hip", "pa_gemm.hip", "pa_wgrad.hip", "pa_train.hip", "pa_train_f32.hip", "pa_mfma_bwd.hip",
-           "pa_mfma_staged.hip", "pa_gale.hip", "pa_flare.hip", "pa_ball_query.hip", "pa_noalloc.hip", "pa_conv.hip", "pa_rows_f32.hip", "pa_narrow_f32.hip"]
+           "pa_layer_point.hip", "pa_mfma_staged.hip", "pa_gale.hip", "pa_flare.hip", "pa_ball_query.hip", "pa_noalloc.hip", "pa_conv.hip", "pa_rows_f32.hip", "pa_narrow_f32.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -23,6 +23,8 @@ HIPCC_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-function",
 ]
+# flags of single files; the reason stands at the top of the file
+FILE_FLAGS = {"pa_layer_point.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def _headers_mtime() -> float:
@@ -55,7 +57,7 @@ def build(verbose: bool = True, incremental: bool = False, jobs: int | None = No
         fresh = (incremental and os.path.exists(obj) and os.path.getmtime(obj) > os.path.getmtime(src)
                  and os.path.getmtime(obj) > hdr_time)
         if not fresh:
-            todo.append([hipcc, *HIPCC_FLAGS, "-c", src, "-o", obj])
+            todo.append([hipcc, *HIPCC_FLAGS, *FILE_FLAGS.get(s, []), "-c", src, "-o", obj])
     jobs = jobs or min(len(todo) or 1, max(1, min(16, os.cpu_count() or 1)))
     with ThreadPoolExecutor(max_workers=jobs) as pool:
         list(pool.map(lambda c: _run(c, verbose), todo))

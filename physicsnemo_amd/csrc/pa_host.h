@@ -275,6 +275,13 @@ bool deslice_project_tokens_supported(const pa_shape &s);
 int deslice_project_tokens(const pa_shape &s, const void *blob, const void *w_pack, const float *tokens, void *y,
                            const pa_block_tail *tail, int num_cu, hipStream_t st);
 bool float_tables(const pa_shape &s, bool plus);  // training multiplies with float32 tables and tokens, not bf16 ones
+bool layer_point_backward_supported(const pa_shape &s);
+int64_t layer_point_backward_workspace_bytes(const pa_shape &s, int num_cu);
+int layer_point_backward(const pa_shape &s, const pa_params &p, const void *w_out_t, const void *x, const void *dy,
+                         const float *out_token, const float *d_num, const float *d_norm, void *workspace, void *d_proj,
+                         float *grads, int num_cu, hipStream_t st);
+int backward_tables(const pa_shape &s, const float *w_slice, const float *pt_w1, const float *out_token, const float *d_num,
+                    bool split, void *tabs, hipStream_t st);
 bool point_backward_supported(const pa_shape &s);
 int64_t point_backward_grads(const pa_shape &s, bool plus);
 int64_t point_backward_workspace_bytes(const pa_shape &s, bool plus, int num_cu);

@@ -57,33 +57,6 @@ __global__ __launch_bounds__(512) void deslice_natural_kernel(const u32x4 *__res
   }
 }
 
-// ------------------------------------------------------------------------------------------------
-// Operand fragments of the backward kernel (16-byte units, one per lane; lane = 32g + i; j = 0..7):
-//   shared   wsl[(st*2 + kk)]   = W_slice[32st + i][16kk + 8g + j]                 A of the logits (k = d, natural order)
-//            wsT[cq]            = W_slice[16cq + rowmap(j, g)][i]                   A of d x_mid (k = slices, chained order)
-//            (Transolver++: the same two groups for the first Linear of proj_temperature)
-//   per (b,h) tokA[(st*2 + kk)] = tok'[32st + i][16kk + 8g + j]                    A of d w, first half of k
-//            dnA[(st*2 + kk)]   = d num[32st + i][16kk + 8g + j]                   A of d w, second half of k
-//            dnT[cq]            = d num[16cq + rowmap(j, g)][i]                     A of d fx_mid
-// Slices >= S read as zero.  SPLIT tables carry the remainders t - bf16(t) in a second set of fragments behind each group,
-// so that products with them keep 16 bits of the table (float_tables() says for which layers).
-// ------------------------------------------------------------------------------------------------
-struct BwdTablePlan {
-  int st2, nch, group, nshared, nhead;  // fragments: of the two kinds, of a shared group, shared, per (b, h)
-  int64_t shared_units, per_head_units;
-};
-__host__ __device__ inline BwdTablePlan bwd_table_plan(int S, bool plus, bool split) {
-  BwdTablePlan p;
-  p.st2 = 2 * ((S + 31) / 32);
-  p.nch = S / 16;
-  p.group = (p.st2 + p.nch) * (split ? 2 : 1);
-  p.nshared = p.group * (plus ? 2 : 1);
-  p.nhead = (2 * p.st2 + p.nch) * (split ? 2 : 1);
-  p.shared_units = (int64_t)p.nshared * 64;
-  p.per_head_units = (int64_t)p.nhead * 64;
-  return p;
-}
-
 __global__ __launch_bounds__(256) void backward_tables_kernel(const float *__restrict__ w_slice,
                                                               const float *__restrict__ pt_w1,
                                                               const float *__restrict__ out_token,
@@ -323,8 +296,6 @@ struct PointArgs {
   int64_t N;
   int tpb, H;
 };
-
-__host__ __device__ inline int point_grads(int S, int H, bool plus) { return S * 33 + H + (plus ? S * 34 + 1 : 0); }
 
 // heads (waves) per workgroup.  4: one wave per SIMD, 512 registers; 1, 2: what the split tables of S = 128 leave room for
 constexpr int point_waves(int S, bool plus, bool split) { return S > 64 ? (split ? (plus ? 1 : 2) : 4) : plus || (split && S == 64) ? 4 : 8; }
@@ -771,6 +742,16 @@ int64_t point_backward_workspace_bytes(const pa_shape &s, bool plus, int num_cu)
   return (tp.shared_units + s.B * s.H * tp.per_head_units) * 16 + wgs * point_backward_grads(s, plus) * 4;
 }
 
+// the operand fragments of W_slice (Transolver++: and W1), out_token (NULL: zeros) and d_num
+int backward_tables(const pa_shape &s, const float *w_slice, const float *pt_w1, const float *out_token, const float *d_num,
+                    bool split, void *tabs, hipStream_t st) {
+  const BwdTablePlan tp = bwd_table_plan((int)s.S, pt_w1 != nullptr, split);
+  const int64_t grid = (tp.shared_units + s.B * s.H * tp.per_head_units + 255) / 256;
+  hipLaunchKernelGGL(backward_tables_kernel, dim3((unsigned)(grid < 256 ? grid : 256)), dim3(256), 0, st, w_slice, pt_w1,
+                     out_token, d_num, static_cast<u32x4 *>(tabs), (int)(s.B * s.H), (int)s.S, split ? 1 : 0);
+  return launch_status();
+}
+
 // x_mid, fx_mid, d_out_x natural rows (PLUS: fx_mid unused); out_token may be NULL (no deslice term); grads:
 // point_backward_grads() floats
 int point_backward(const pa_shape &s, const pa_params &p, const pa_plus_params *plus, const void *x_mid,
@@ -793,11 +774,8 @@ int point_backward(const pa_shape &s, const pa_params &p, const pa_plus_params *
   a.d_proj = static_cast<uint16_t *>(d_proj);
   a.partials = reinterpret_cast<float *>(tabs + table_units);
   a.N = s.N, a.tpb = (int)tiles_per_batch(s), a.H = (int)s.H;
-  const int64_t tgrid = (table_units + 255) / 256;
-  hipLaunchKernelGGL(backward_tables_kernel, dim3((unsigned)(tgrid < 256 ? tgrid : 256)), dim3(256), 0, st,
-                     p.in_project_slice_weight, plus ? plus->proj_temperature_0_weight : nullptr, out_token, d_num, tabs,
-                     (int)(s.B * s.H), (int)s.S, split ? 1 : 0);
-  int rc = launch_status();
+  int rc = backward_tables(s, p.in_project_slice_weight, plus ? plus->proj_temperature_0_weight : nullptr, out_token, d_num, split,
+                           tabs, st);
   if (rc) return rc;
   const int w = point_head_waves(s, plus != nullptr);
   const int64_t G = point_groups(s, plus != nullptr, num_cu), Z = s.H / w;

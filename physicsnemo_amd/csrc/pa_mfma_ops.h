@@ -99,6 +99,15 @@ __device__ __forceinline__ void load_unit_to_lds(const void *p, unsigned dst) { 
       : "memory");
 }
 
+// The same with a wave-uniform base and a byte offset per lane.
+__device__ __forceinline__ void load_unit_to_lds(const void *sbase, int off, unsigned dst) {
+  asm volatile(
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %0" ::"s"(sbase), "v"(off), "s"(dst)
+      : "memory");
+}
+
 // f(integral_constant<int, 0>{}), ..., f(integral_constant<int, N - 1>{}): a loop whose index is a constant expression
 template <class F, int... I>
 __device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
@@ -139,14 +148,13 @@ __device__ __forceinline__ float half_wave_sum(float v) {
 // layout: `row` points at channel 0 of this lane's point.  Registers 4q..4q+3 hold channels 8q + 4g .. + 3; swapping
 // halves with lane ^ 32 gives each lane 8 consecutive channels (g = 0: 0-7 and 8-15, g = 1: 16-23 and 24-31), so a
 // point's 64 bytes leave as four 16-byte stores.  `nch` = valid channels (32, or 16: the lower half only).
-__device__ __forceinline__ void store_tile_natural(const f32x16 &v, uint16_t *row, int g, bool ok, int nch = 32) {
+__device__ __forceinline__ void tile_natural(const f32x16 &v, u32x4 &s0, u32x4 &s1) {
   uint32_t p[4][2];
 #pragma unroll
   for (int q = 0; q < 4; ++q)
 #pragma unroll
     for (int w = 0; w < 2; ++w)
-      p[q][w] = (uint32_t)to_bf16_bits(v[4 * q + 2 * w]) | ((uint32_t)to_bf16_bits(v[4 * q + 2 * w + 1]) << 16);
-  u32x4 s0, s1;
+      p[q][w] = pack2(v[4 * q + 2 * w], v[4 * q + 2 * w + 1]);
 #pragma unroll
   for (int w = 0; w < 2; ++w) {
     // lower half-wave: (own piece 0, partner's piece 0); upper half-wave: (partner's piece 2, own piece 2)
@@ -157,6 +165,10 @@ __device__ __forceinline__ void store_tile_natural(const f32x16 &v, uint16_t *ro
     s1[w] = b[0];
     s1[2 + w] = b[1];
   }
+}
+__device__ __forceinline__ void store_tile_natural(const f32x16 &v, uint16_t *row, int g, bool ok, int nch = 32) {
+  u32x4 s0, s1;
+  tile_natural(v, s0, s1);
   if (ok && (g == 0 || nch > 16)) {
     *reinterpret_cast<u32x4 *>(row + 16 * g) = s0;
     *reinterpret_cast<u32x4 *>(row + 16 * g + 8) = s1;
@@ -235,6 +247,36 @@ __device__ __forceinline__ void stage_slice_projection(const float *__restrict__
   }
   for (int s = threadIdx.x; s < ST * 32; s += blockDim.x) bsl[s] = s < S ? b_slice[s] : -1e30f;  // slices beyond S: weight 0
 }
+
+// ------------------------------------------------------------------------------------------------
+// Operand fragments of the per-point backward kernels (16-byte units, one per lane; lane = 32g + i; j = 0..7):
+//   shared   wsl[(st*2 + kk)]   = W_slice[32st + i][16kk + 8g + j]                 A of the logits (k = d, natural order)
+//            wsT[cq]            = W_slice[16cq + rowmap(j, g)][i]                   A of d x_mid (k = slices, chained order)
+//            (Transolver++: the same two groups for the first Linear of proj_temperature)
+//   per (b,h) tokA[(st*2 + kk)] = tok'[32st + i][16kk + 8g + j]                    A of d w, first half of k
+//            dnA[(st*2 + kk)]   = d num[32st + i][16kk + 8g + j]                   A of d w, second half of k
+//            dnT[cq]            = d num[16cq + rowmap(j, g)][i]                     A of d fx_mid
+// Slices >= S read as zero.  SPLIT tables carry the remainders t - bf16(t) in a second set of fragments behind each group,
+// so that products with them keep 16 bits of the table (float_tables() says for which layers).
+// ------------------------------------------------------------------------------------------------
+struct BwdTablePlan {
+  int st2, nch, group, nshared, nhead;  // fragments: of the two kinds, of a shared group, shared, per (b, h)
+  int64_t shared_units, per_head_units;
+};
+__host__ __device__ inline BwdTablePlan bwd_table_plan(int S, bool plus, bool split) {
+  BwdTablePlan p;
+  p.st2 = 2 * ((S + 31) / 32);
+  p.nch = S / 16;
+  p.group = (p.st2 + p.nch) * (split ? 2 : 1);
+  p.nshared = p.group * (plus ? 2 : 1);
+  p.nhead = (2 * p.st2 + p.nch) * (split ? 2 : 1);
+  p.shared_units = (int64_t)p.nshared * 64;
+  p.per_head_units = (int64_t)p.nhead * 64;
+  return p;
+}
+
+// floats of a workgroup's row of partial gradients: d W_slice, d b_slice, d T (Transolver++: and d W1, d b1, d w2, d b2)
+__host__ __device__ inline int point_grads(int S, int H, bool plus) { return S * 33 + H + (plus ? S * 34 + 1 : 0); }
 
 }  // namespace mfma
 }  // namespace pa

@@ -98,6 +98,18 @@ static HandBack hand_back(const pa_shape &s, bool plus) {
 
 static bool fused(const pa_shape &s, bool plus) { return !plus && mfma::supported(PA_BF16, s); }
 
+// The projections, d out_x and the per-point stage of the backward pass in one kernel.  Its workgroups, one per CU, read 3 C / 2
+// KB of weights before their first tile.  Many batch elements of one tile each do not pay that back: 2 048 clouds of 16
+// points, C = 256, S = 64, 7 180 us against 7 000 for the whole step; 512 of 64 points 1 250 both ways.  Nor do, at C = 128
+// where the stages move half as much, fewer than four tiles per CU: the kernels of a step at S = 32 take 165 us against 149
+// for 8 192 points, 174 against 163 for 16 384, 189 against 195 for 32 768 and 222 against 246 for 65 536 (C = 256: 187
+// against 193 for 2 000, 223 against 232 for 16 384, 503 against 585 for 131 072).
+static bool points_in_one(const pa_shape &s, bool plus, int num_cu) {
+  if (!fused(s, plus) || !mfma::layer_point_backward_supported(s)) return false;
+  if (s.C == 128 && s.B * mfma::tiles_per_batch(s) < 4 * (int64_t)num_cu) return false;
+  return s.N > 32 || s.B * s.H <= 4 * (int64_t)num_cu;
+}
+
 bool supported(const pa_shape &s, bool plus) {
   if (s.conv_k != 0 && s.conv_tap_major != 1) return false;
   if (!mfma::point_backward_supported(s)) return false;
@@ -167,8 +179,9 @@ static Scratch plan_scratch(const pa_shape &s, bool plus, int num_cu) {
 
   off = 0;
   const int np = plus ? 1 : 2;
-  p.g = take(M * HD * 2);
-  if (fused(s, plus)) {
+  const bool one = points_in_one(s, plus, num_cu);
+  p.g = take(one ? 0 : M * HD * 2);
+  if (fused(s, plus) && !one) {
     p.x_mid = take(M * HD * 2);
     p.fx_mid = take(M * HD * 2);
   }
@@ -181,7 +194,7 @@ static Scratch plan_scratch(const pa_shape &s, bool plus, int num_cu) {
   p.work_bytes = wgrad::workspace_bytes(PA_BF16, M, np * HD, s.C, grid_taps(&s).taps, num_cu);
   auto more = [&](int64_t bytes) { p.work_bytes = bytes > p.work_bytes ? bytes : p.work_bytes; };
   more(wgrad::output_backward_workspace_bytes(s, num_cu));
-  more(mfma::point_backward_workspace_bytes(s, plus, num_cu));
+  more(one ? mfma::layer_point_backward_workspace_bytes(s, num_cu) : mfma::point_backward_workspace_bytes(s, plus, num_cu));
   p.work = take(p.work_bytes);
   p.total_backward = off;
   return p;
@@ -319,15 +332,20 @@ int backward(const pa_shape &s, bool pl, const void *x, const void *uniform, con
   if ((rc = backward::slice_attention(s, p, tok, norm, d_tok, reinterpret_cast<float *>(ws + sc.attn), d_num, d_norm, parts, st)))
     return rc;
   if ((rc = wgrad::sum_rows(parts, s.B * s.H, 3 * 32 * 32, d_wqkv, st))) return rc;
-  if ((rc = general::rows_gemm(PA_BF16, lin, s.C, HD, dy, sv + sp.w_out_t, nullptr, 0, g, st))) return rc;
-  const void *x_mid = sv + sp.x_mid, *fx_mid = pl ? nullptr : sv + sp.fx_mid;
-  if (fused(s, pl)) {
-    x_mid = ws + sc.x_mid, fx_mid = ws + sc.fx_mid;
-    if ((rc = general::project_inputs(PA_BF16, s, p, x, ws + sc.x_mid, ws + sc.fx_mid, st))) return rc;
+  if (points_in_one(s, pl, num_cu)) {
+    if ((rc = mfma::layer_point_backward(s, p, sv + sp.w_out_t, x, dy, tok_out, d_num, d_norm, work, d_proj, small, num_cu, st)))
+      return rc;
+  } else {
+    if ((rc = general::rows_gemm(PA_BF16, lin, s.C, HD, dy, sv + sp.w_out_t, nullptr, 0, g, st))) return rc;
+    const void *x_mid = sv + sp.x_mid, *fx_mid = pl ? nullptr : sv + sp.fx_mid;
+    if (fused(s, pl)) {
+      x_mid = ws + sc.x_mid, fx_mid = ws + sc.fx_mid;
+      if ((rc = general::project_inputs(PA_BF16, s, p, x, ws + sc.x_mid, ws + sc.fx_mid, st))) return rc;
+    }
+    if ((rc = mfma::point_backward(s, p, pl ? &prep.q : nullptr, x_mid, fx_mid, g, uniform, tok_out, d_num, d_norm, work, d_proj,
+                                   small, num_cu, st)))
+      return rc;
   }
-  if ((rc = mfma::point_backward(s, p, pl ? &prep.q : nullptr, x_mid, fx_mid, g, uniform, tok_out, d_num, d_norm, work, d_proj,
-                                 small, num_cu, st)))
-    return rc;
   if (dx && (rc = general::rows_gemm(PA_BF16, s, np * HD, s.C, d_proj, sv + sp.w_in_t, nullptr, 0, dx, st))) return rc;
   return wgrad::product(PA_BF16, M, d_proj, np * HD, np * HD, x, s.C, s.C, s.conv_k > 0 ? &s : nullptr, work, d_w_in, d_b_in,
                         num_cu, st);

@@ -1167,3 +1167,45 @@ def test_fp32_layer_in_two_calls_against_the_stages(monkeypatch, kind, dim, head
     for g, w in zip(got, want):
         assert_rel_l2(g, w, "two calls against the stages", 2e-6)
 
+
+
+@pytest.mark.parametrize("B,N,C,S", [(1, 1, 256, 64), (3, 33, 256, 64), (1, 8229, 256, 32), (17, 40, 256, 16), (130, 33, 256, 64),
+                                     (1, 32_761, 128, 64), (513, 33, 128, 16), (5, 6571, 128, 32), (2, 4127, 256, 16)])
+def test_point_stage_with_its_products_against_the_stages(B, N, C, S):
+    """The irregular layer's backward, whose per-point kernel forms the projections and d out_x itself, against the stages with
+    these in memory: single points, ragged tiles, few and many batch elements, workgroups without a tile, every S.  Both
+    round the three products to bf16 from float32 sums in different orders; where the rounding falls the other way (2^-8 of a
+    value, one in ten at most) the results differ by 2^-8 sqrt(0.1) = 1.2e-3, the sums with cancelling terms by more."""
+    announce("point stage with products", B, N, C, S)
+    from physicsnemo_amd import autograd as PA
+    torch.manual_seed(S + N)
+    H = C // 32
+    _, hip = make_pair("irregular", C, H, 32, S, temps=[0.3 + 0.4 * k for k in range(H)])
+    x, dy = torch.randn(2, B, N, C, device="cuda").bfloat16()
+    dims, kp = hip.layer_dims(x), hip.kernel_params(torch.bfloat16, x.device)
+    names = dict(hip.named_parameters())
+    params = [names[n.replace("_weight", ".weight").replace("_bias", ".bias")] for n in PA._LAYER_PARAMS]
+    xc = x.clone().requires_grad_(True)
+    PA.PhysicsAttentionMfmaFunction.apply(xc, dims, None, *params).backward(dy)
+
+    st = PF.MfmaStages(kp, dims, x.device)
+    st.pack_params()
+    st.project_softmax(x)
+    st.slice_reduce()
+    st.combine_attention()
+    linear = PF.LayerDims(B, N, C, H, 32, S)
+    x_mid, fx_mid = PF.project_inputs(x, kp, dims)
+    g = PF.rows_gemm(dy, kp["out_linear_weight"].view(C, C).t().contiguous(), None, linear, C, C)
+    d_tok, _, _ = PF.output_backward(st.w_pack, dy, st.tok_out, kp["out_linear_weight"], dims)
+    d_num, d_norm, _ = PF.slice_attention_backward(st.tok, st.norm, d_tok, kp, dims)
+    d_proj, d_ws, d_bs, d_temp = PF.point_backward(x_mid, fx_mid, g, st.tok_out, d_num, d_norm, kp, dims)
+    w_t = torch.cat([kp["in_project_x_weight"].view(C, C).t(), kp["in_project_fx_weight"].view(C, C).t()], dim=1).contiguous()
+    assert_rel_l2(xc.grad, PF.rows_gemm(d_proj, w_t, None, linear, 2 * C, C), "dx", tol=4e-3)
+    rows, d_b = d_proj.float().reshape(-1, 2 * C), d_proj.double().reshape(-1, 2 * C).sum(0)
+    d_w = rows.t() @ x.float().reshape(-1, C)
+    assert_rel_l2(hip.in_project_x.weight.grad, d_w[:C], "d W_x", tol=4e-3)
+    assert_rel_l2(hip.in_project_fx.weight.grad, d_w[C:], "d W_fx", tol=4e-3)
+    assert_rel_l2(hip.in_project_fx.bias.grad, d_b[C:], "d b_fx", tol=4e-3)
+    assert_rel_l2(hip.in_project_slice.weight.grad, d_ws.view(S, 32), "d W_slice", tol=4e-3)
+    assert_rel_l2(hip.in_project_slice.bias.grad, d_bs, "d b_slice", tol=2e-2)
+    assert_rel_l2(hip.temperature.grad.reshape(-1), d_temp.reshape(-1), "d temperature", tol=2e-2)
