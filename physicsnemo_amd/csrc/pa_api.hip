@@ -1232,7 +1232,7 @@ int pa_mlp_backward(int dtype, int64_t rows, int64_t C, int64_t F, const pa_mlp_
 
 namespace {
 struct NormMlpPlan {
-  int64_t act, dh, blob, w1_t, partials, work, work_bytes, total;
+  int64_t act, dh, blob, w1_t, partials, work_w1, work_w2, total;
 };
 NormMlpPlan norm_mlp_plan(int64_t rows, int64_t C, int64_t F) {
   NormMlpPlan p{};
@@ -1249,9 +1249,9 @@ NormMlpPlan norm_mlp_plan(int64_t rows, int64_t C, int64_t F) {
   p.partials = take(pa::norm::rows_ln_backward_groups(rows, compute_units()) * 2 * C * 4);
   const int64_t w1 = pa::wgrad::workspace_bytes(PA_BF16, rows, F, C, 1, compute_units()),
                 w2 = pa::wgrad::workspace_bytes(PA_BF16, rows, C, F, 1, compute_units());
-  p.work_bytes = w1 <= 0 || w2 <= 0 ? 0 : w1 > w2 ? w1 : w2;
-  p.work = take(p.work_bytes);
-  p.total = p.work_bytes > 0 ? off : 0;
+  if (w1 <= 0 || w2 <= 0) return p;
+  p.work_w1 = take(w1), p.work_w2 = take(w2);
+  p.total = off;
   return p;
 }
 }  // namespace
@@ -1281,13 +1281,15 @@ int pa_norm_mlp_backward(int dtype, int64_t rows, int64_t C, int64_t F, const pa
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int cus = compute_units();
   float *d_w1 = grads, *d_b1 = d_w1 + F * C, *d_w2 = d_b1 + F, *d_b2 = d_w2 + C * F, *d_ln = d_b2 + C;
+  pa::wgrad::Sums sums;
   int rc = pa::mlp::hidden_backward(rows, C, F, p->w1, p->b1, p->w2, u, dy, act, dh, ws + w.blob, ws + w.w1_t, cus, st);
   if (rc) return rc;
   if ((rc = pa::norm::rows_ln_backward(rows, F, dh, ws + w.w1_t, x, ln_gamma, ln_eps, dy, dx,
-                                       reinterpret_cast<float *>(ws + w.partials), d_ln, cus, st)))
+                                       reinterpret_cast<float *>(ws + w.partials), d_ln, cus, st, sums)))
     return rc;
-  if ((rc = pa::wgrad::product(PA_BF16, rows, dh, F, F, u, C, C, nullptr, ws + w.work, d_w1, d_b1, cus, st))) return rc;
-  return pa::wgrad::product(PA_BF16, rows, dy, C, C, act, F, F, nullptr, ws + w.work, d_w2, d_b2, cus, st);
+  if ((rc = pa::wgrad::product(PA_BF16, rows, dh, F, F, u, C, C, nullptr, ws + w.work_w1, d_w1, d_b1, cus, st, &sums))) return rc;
+  if ((rc = pa::wgrad::product(PA_BF16, rows, dy, C, C, act, F, F, nullptr, ws + w.work_w2, d_w2, d_b2, cus, st, &sums))) return rc;
+  return pa::wgrad::launch_sums(sums, st);
 }
 
 int pa_mlp_input_ln_query(int dtype, int64_t rows, int64_t C, int64_t F) {

@@ -80,10 +80,29 @@ int cols_gemm_f32(const void *A, int64_t lda, int64_t OA, const void *B, int64_t
 }  // namespace gemm
 
 namespace wgrad {
+// Totals of partial results, dst[e] = sum over g < G of src[g][e], collected so that one launch forms several of them: every
+// result's partials stay where they are until then.
+struct Sums {
+  static constexpr int kMost = 8;
+  struct One {
+    const float *src;
+    float *dst;
+    int64_t n, first;     // elements; the launch's first workgroup for them
+    int G, taps, OB;      // taps > 1: src is [oa][tap][ob], dst the order of a convolution's weight, [oa][ob][tap]
+  } r[kMost];
+  int count = 0;
+  int64_t blocks = 0;
+  void add(const float *src, float *dst, int64_t n, int64_t G, int taps = 1, int64_t OB = 1) {
+    r[count++] = One{src, dst, n, blocks, (int)G, taps, (int)OB};
+    blocks += (n + 31) / 32;
+  }
+};
+int launch_sums(const Sums &sums, hipStream_t st);
 // out[oa][ob] (grid: [oa][ob][tap]) = sum_m A[m][oa] B[m][ob] and the column sums of A; `workspace`: workspace_bytes()
 int64_t workspace_bytes(int dtype, int64_t M, int64_t OA, int64_t OB, int taps, int num_cu);
 int product(int dtype, int64_t M, const void *A, int64_t lda, int64_t OA, const void *B, int64_t ldb, int64_t OB,
-            const pa_shape *grid, void *workspace, float *out, float *col_sums, int num_cu, hipStream_t st);
+            const pa_shape *grid, void *workspace, float *out, float *col_sums, int num_cu, hipStream_t st,
+            Sums *later = nullptr);  // later: the totals are left to its launch
 // the bf16 tile kernel alone, G partial results
 int launch_wide(const void *A, int64_t lda, int64_t OA, const void *B, int64_t ldb, int64_t OB, int64_t M, int64_t G,
                 const pa_shape *grid, float *partials, float *col_sums, hipStream_t st);
@@ -279,7 +298,7 @@ bool layer_point_backward_supported(const pa_shape &s);
 int64_t layer_point_backward_workspace_bytes(const pa_shape &s, int num_cu);
 int layer_point_backward(const pa_shape &s, const pa_params &p, const void *w_out_t, const void *x, const void *dy,
                          const float *out_token, const float *d_num, const float *d_norm, void *workspace, void *d_proj,
-                         float *grads, int num_cu, hipStream_t st);
+                         wgrad::Sums &later, float *grads, int num_cu, hipStream_t st);
 int backward_tables(const pa_shape &s, const float *w_slice, const float *pt_w1, const float *out_token, const float *d_num,
                     bool split, void *tabs, hipStream_t st);
 bool point_backward_supported(const pa_shape &s);
@@ -288,7 +307,7 @@ int64_t point_backward_workspace_bytes(const pa_shape &s, bool plus, int num_cu)
 int point_backward(const pa_shape &s, const pa_params &p, const pa_plus_params *plus, const void *x_mid,
                    const void *fx_mid, const void *d_out_x, const void *uniform, const float *out_token,
                    const float *d_num, const float *d_norm, void *workspace, void *d_proj, float *grads, int num_cu,
-                   hipStream_t st);
+                   hipStream_t st, wgrad::Sums *later = nullptr);
 bool supported(int dtype, const pa_shape &s);
 int64_t tiles_per_batch(const pa_shape &s);
 int64_t reduce_groups(const pa_shape &s);
@@ -371,7 +390,7 @@ namespace norm {
 bool rows_ln_backward_supported(int64_t rows, int64_t C, int64_t K);
 int64_t rows_ln_backward_groups(int64_t rows, int num_cu);
 int rows_ln_backward(int64_t rows, int64_t K, const void *dh, const void *wt, const void *x, const float *gamma, float eps,
-                     const void *add, void *dx, float *partials, float *grads, int num_cu, hipStream_t st);
+                     const void *add, void *dx, float *partials, float *grads, int num_cu, hipStream_t st, wgrad::Sums &later);
 }  // namespace norm
 
 }  // namespace pa

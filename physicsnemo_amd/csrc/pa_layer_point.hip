@@ -376,7 +376,7 @@ int64_t layer_point_backward_workspace_bytes(const pa_shape &s, int num_cu) {
 
 int layer_point_backward(const pa_shape &s, const pa_params &p, const void *w_out_t, const void *x, const void *dy,
                          const float *out_token, const float *d_num, const float *d_norm, void *workspace, void *d_proj,
-                         float *grads, int num_cu, hipStream_t st) {
+                         wgrad::Sums &later, float *grads, int num_cu, hipStream_t st) {
   if (!layer_point_backward_supported(s)) return PA_ERR_UNSUPPORTED;
   const BwdTablePlan tp = bwd_table_plan((int)s.S, false, false);
   u32x4 *tabs = static_cast<u32x4 *>(workspace);
@@ -407,7 +407,8 @@ int layer_point_backward(const pa_shape &s, const pa_params &p, const void *w_ou
   PA_LAYER_POINT(256, 64)
 #undef PA_LAYER_POINT
   if ((rc = launch_status())) return rc;
-  return wgrad::sum_rows(a.partials, G * s.B * Z, point_grads((int)s.S, (int)s.H, false), grads, st);
+  later.add(a.partials, grads, point_grads((int)s.S, (int)s.H, false), G * s.B * Z);
+  return PA_OK;
 }
 
 }  // namespace mfma

@@ -757,7 +757,7 @@ int backward_tables(const pa_shape &s, const float *w_slice, const float *pt_w1,
 int point_backward(const pa_shape &s, const pa_params &p, const pa_plus_params *plus, const void *x_mid,
                    const void *fx_mid, const void *d_out_x, const void *uniform, const float *out_token,
                    const float *d_num, const float *d_norm, void *workspace, void *d_proj, float *grads, int num_cu,
-                   hipStream_t st) {
+                   hipStream_t st, wgrad::Sums *later) {
   if (!point_backward_supported(s)) return PA_ERR_UNSUPPORTED;
   const bool split = float_tables(s, plus != nullptr);
   const BwdTablePlan tp = bwd_table_plan((int)s.S, plus != nullptr, split);
@@ -798,7 +798,9 @@ int point_backward(const pa_shape &s, const pa_params &p, const pa_plus_params *
   }
 #undef PA_POINT
   if ((rc = launch_status())) return rc;
-  return wgrad::sum_rows(a.partials, G * s.B * Z, point_backward_grads(s, plus != nullptr), grads, st);
+  wgrad::Sums own, &sums = later ? *later : own;
+  sums.add(a.partials, grads, point_backward_grads(s, plus != nullptr), G * s.B * Z);
+  return later ? PA_OK : wgrad::launch_sums(own, st);
 }
 
 }  // namespace mfma

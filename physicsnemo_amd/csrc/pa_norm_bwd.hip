@@ -212,12 +212,13 @@ static int launch(const Args &a, int64_t groups, hipStream_t st) {
 
 // partials: rows_ln_backward_groups(rows) * 512 floats; grads: d gamma (256), d beta (256)
 int rows_ln_backward(int64_t rows, int64_t K, const void *dh, const void *wt, const void *x, const float *gamma, float eps,
-                     const void *add, void *dx, float *partials, float *grads, int num_cu, hipStream_t st) {
+                     const void *add, void *dx, float *partials, float *grads, int num_cu, hipStream_t st, wgrad::Sums &later) {
   const int64_t per = block_rows(rows, num_cu), groups = rows_ln_backward_groups(rows, num_cu);
   auto in = [](const void *p) { return static_cast<const uint16_t *>(p); };
   const Args a{in(dh), in(wt), in(x), in(add), gamma, static_cast<uint16_t *>(dx), partials, eps, rows, (rows + per - 1) / per, (int)K};
   const int rc = per == 128 ? launch<128>(a, groups, st) : launch<64>(a, groups, st);
-  return rc ? rc : wgrad::sum_rows(partials, groups, 512, grads, st);
+  if (!rc) later.add(partials, grads, 512, groups);
+  return rc;
 }
 
 }  // namespace norm

@@ -81,7 +81,7 @@ struct Saved {  // kept from the forward to the backward pass
 };
 struct Scratch {
   int64_t blob, fx_pack, partials, tokp, out_x, total;                                     // forward
-  int64_t g, x_mid, fx_mid, d_proj, d_tok, d_num, d_norm, attn, parts, work, total_backward;  // backward
+  int64_t g, x_mid, fx_mid, d_proj, d_tok, d_num, d_norm, attn, parts, point, work, total_backward;  // backward
   int64_t work_bytes;
 };
 
@@ -194,7 +194,7 @@ static Scratch plan_scratch(const pa_shape &s, bool plus, int num_cu) {
   p.work_bytes = wgrad::workspace_bytes(PA_BF16, M, np * HD, s.C, grid_taps(&s).taps, num_cu);
   auto more = [&](int64_t bytes) { p.work_bytes = bytes > p.work_bytes ? bytes : p.work_bytes; };
   more(wgrad::output_backward_workspace_bytes(s, num_cu));
-  more(one ? mfma::layer_point_backward_workspace_bytes(s, num_cu) : mfma::point_backward_workspace_bytes(s, plus, num_cu));
+  p.point = take(one ? mfma::layer_point_backward_workspace_bytes(s, num_cu) : mfma::point_backward_workspace_bytes(s, plus, num_cu));
   p.work = take(p.work_bytes);
   p.total_backward = off;
   return p;
@@ -324,16 +324,18 @@ int backward(const pa_shape &s, bool pl, const void *x, const void *uniform, con
               *tok_out = reinterpret_cast<float *>(sv + sp.tok_out);
   float *d_tok = reinterpret_cast<float *>(ws + sc.d_tok), *d_num = reinterpret_cast<float *>(ws + sc.d_num),
         *d_norm = reinterpret_cast<float *>(ws + sc.d_norm), *parts = reinterpret_cast<float *>(ws + sc.parts);
-  void *g = ws + sc.g, *d_proj = ws + sc.d_proj, *work = ws + sc.work;
+  void *g = ws + sc.g, *d_proj = ws + sc.d_proj, *point = ws + sc.point, *work = ws + sc.work;
   pa_shape lin = s;
   lin.conv_k = lin.grid_h = lin.grid_w = lin.grid_d = 0;
   int rc = wgrad::output_backward(s, sv + sp.w_pack, dy, tok_out, p.out_linear_weight, work, d_tok, d_w_out, d_b_out, num_cu, st);
   if (rc) return rc;
   if ((rc = backward::slice_attention(s, p, tok, norm, d_tok, reinterpret_cast<float *>(ws + sc.attn), d_num, d_norm, parts, st)))
     return rc;
-  if ((rc = wgrad::sum_rows(parts, s.B * s.H, 3 * 32 * 32, d_wqkv, st))) return rc;
+  wgrad::Sums sums;  // formed together at the end: what their partial results lie in is not used again until then
+  sums.add(parts, d_wqkv, 3 * 32 * 32, s.B * s.H);
   if (points_in_one(s, pl, num_cu)) {
-    if ((rc = mfma::layer_point_backward(s, p, sv + sp.w_out_t, x, dy, tok_out, d_num, d_norm, work, d_proj, small, num_cu, st)))
+    if ((rc = mfma::layer_point_backward(s, p, sv + sp.w_out_t, x, dy, tok_out, d_num, d_norm, point, d_proj, sums, small,
+                                         num_cu, st)))
       return rc;
   } else {
     if ((rc = general::rows_gemm(PA_BF16, lin, s.C, HD, dy, sv + sp.w_out_t, nullptr, 0, g, st))) return rc;
@@ -342,13 +344,15 @@ int backward(const pa_shape &s, bool pl, const void *x, const void *uniform, con
       x_mid = ws + sc.x_mid, fx_mid = ws + sc.fx_mid;
       if ((rc = general::project_inputs(PA_BF16, s, p, x, ws + sc.x_mid, ws + sc.fx_mid, st))) return rc;
     }
-    if ((rc = mfma::point_backward(s, p, pl ? &prep.q : nullptr, x_mid, fx_mid, g, uniform, tok_out, d_num, d_norm, work, d_proj,
-                                   small, num_cu, st)))
+    if ((rc = mfma::point_backward(s, p, pl ? &prep.q : nullptr, x_mid, fx_mid, g, uniform, tok_out, d_num, d_norm, point, d_proj,
+                                   small, num_cu, st, &sums)))
       return rc;
   }
   if (dx && (rc = general::rows_gemm(PA_BF16, s, np * HD, s.C, d_proj, sv + sp.w_in_t, nullptr, 0, dx, st))) return rc;
-  return wgrad::product(PA_BF16, M, d_proj, np * HD, np * HD, x, s.C, s.C, s.conv_k > 0 ? &s : nullptr, work, d_w_in, d_b_in,
-                        num_cu, st);
+  if ((rc = wgrad::product(PA_BF16, M, d_proj, np * HD, np * HD, x, s.C, s.C, s.conv_k > 0 ? &s : nullptr, work, d_w_in, d_b_in,
+                           num_cu, st, &sums)))
+    return rc;
+  return wgrad::launch_sums(sums, st);
 }
 
 }  // namespace train

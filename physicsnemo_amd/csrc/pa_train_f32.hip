@@ -97,7 +97,8 @@ struct Saved {  // kept from the forward to the backward pass
 };
 struct Scratch {
   int64_t w_in, partials, total;                                                                                    // forward
-  int64_t g, sums, d_tok, d_num, d_norm, attn, parts, d_proj, d_z, d_t, t_sum, heads, work, work_bytes, total_backward;
+  int64_t g, sums, d_tok, d_num, d_norm, attn, parts, d_proj, d_z, d_t, t_sum, heads, work[3], total_backward;
+  bool served;  // by the row-axis products
 };
 struct Taker {
   int64_t off = 0;
@@ -149,8 +150,11 @@ static Scratch plan_scratch(const pa_shape &s, int num_cu) {
   p.heads = back((HS * HD + HS) * 4);
   const int64_t work[3] = {wgrad::workspace_bytes(PA_F32, M, s.C, HD, 1, num_cu), wgrad::workspace_bytes(PA_F32, M, HS, HD, 1, num_cu),
                            wgrad::workspace_bytes(PA_F32, M, 2 * HD, s.C, (int)taps, num_cu)};
-  for (int64_t w : work) p.work_bytes = w <= 0 ? -1 : p.work_bytes < 0 ? -1 : w > p.work_bytes ? w : p.work_bytes;
-  p.work = back(p.work_bytes > 0 ? p.work_bytes : 0);
+  p.served = true;
+  for (int k = 0; k < 3; ++k) {
+    p.served = p.served && work[k] > 0;
+    p.work[k] = back(work[k] > 0 ? work[k] : 0);
+  }
   p.total_backward = back.off;
   return p;
 }
@@ -161,7 +165,7 @@ bool supported(const pa_shape &s, int num_cu) {
   if (s.conv_k != 0 && s.conv_tap_major != 1) return false;
   if (backward::attention_lds_bytes(s) > kMaxLdsBytes || backward::point_tile_rows(s) == 0) return false;
   if (s.H < 2 || s.H * s.S > 512 || s.C % 4 != 0 || s.H * s.D % 4 != 0) return false;
-  return plan_scratch(s, num_cu).work_bytes > 0;
+  return plan_scratch(s, num_cu).served;
 }
 
 int64_t saved_bytes(const pa_shape &s) { return plan_saved(s).total; }
@@ -228,7 +232,7 @@ int backward(const pa_shape &s, const void *x, const void *dy, const void *saved
   const float *tok = f(sv, sp.tok), *norm = f(sv, sp.norm), *tok_out = f(sv, sp.tok_out);
   float *partials = f(ws, sc.partials), *d_tok = f(ws, sc.d_tok), *d_num = f(ws, sc.d_num), *d_norm = f(ws, sc.d_norm),
         *parts = f(ws, sc.parts), *t_tiles = f(ws, sc.d_t), *t_sum = f(ws, sc.t_sum), *heads = f(ws, sc.heads);
-  void *g = ws + sc.g, *d_proj = ws + sc.d_proj, *d_z = ws + sc.d_z, *work = ws + sc.work;
+  void *g = ws + sc.g, *d_proj = ws + sc.d_proj, *d_z = ws + sc.d_z;
   const void *x_mid = sv + sp.x_mid, *fx_mid = sv + sp.fx_mid, *w = sv + sp.w, *out_x = sv + sp.out_x;
   pa_shape lin = s;
   lin.conv_k = lin.grid_h = lin.grid_w = lin.grid_d = 0;
@@ -241,18 +245,23 @@ int backward(const pa_shape &s, const void *x, const void *dy, const void *saved
   hipLaunchKernelGGL(take_tokens_kernel, dim3((unsigned)((BHS * s.D + 255) / 256)), dim3(256), 0, st, sums, d_tok, BHS * s.D, (int)s.D);
   if ((rc = launch_status())) return rc;
   if ((rc = backward::slice_attention(s, p, tok, norm, d_tok, f(ws, sc.attn), d_num, d_norm, parts, st))) return rc;
-  if ((rc = wgrad::sum_rows(parts, s.B * s.H, 3 * s.D * s.D, d_wqkv, st))) return rc;
+  wgrad::Sums totals;  // formed together at the end: what their partial results lie in is not used again until then
+  totals.add(parts, d_wqkv, 3 * s.D * s.D, s.B * s.H);
   // per point: slice softmax, aggregation and deslice adjoints
   if ((rc = backward::slice_softmax(PA_F32, s, p, x_mid, fx_mid, w, g, tok_out, d_num, d_norm, d_proj, d_z, t_tiles, st))) return rc;
-  if ((rc = wgrad::sum_rows(t_tiles, backward::point_tiles(s), s.H, t_sum, st))) return rc;
-  if ((rc = wgrad::product(PA_F32, M, dy, s.C, s.C, out_x, HD, HD, nullptr, work, d_w_out, d_b_out, num_cu, st))) return rc;
-  if ((rc = wgrad::product(PA_F32, M, d_z, HS, HS, x_mid, HD, HD, nullptr, work, heads, heads + HS * HD, num_cu, st))) return rc;
+  totals.add(t_tiles, t_sum, s.H, backward::point_tiles(s));
+  if ((rc = wgrad::product(PA_F32, M, dy, s.C, s.C, out_x, HD, HD, nullptr, ws + sc.work[0], d_w_out, d_b_out, num_cu, st, &totals)))
+    return rc;
+  if ((rc = wgrad::product(PA_F32, M, d_z, HS, HS, x_mid, HD, HD, nullptr, ws + sc.work[1], heads, heads + HS * HD, num_cu, st, &totals)))
+    return rc;
+  if (dx && (rc = general::rows_gemm(PA_F32, s, 2 * HD, s.C, d_proj, sv + sp.w_in_t, nullptr, 0, dx, st))) return rc;
+  if ((rc = wgrad::product(PA_F32, M, d_proj, 2 * HD, 2 * HD, x, s.C, s.C, s.conv_k > 0 ? &s : nullptr, ws + sc.work[2], d_w_in, d_b_in,
+                           num_cu, st, &totals)))
+    return rc;
+  if ((rc = wgrad::launch_sums(totals, st))) return rc;
   hipLaunchKernelGGL(head_sums_kernel, dim3((unsigned)((s.S * s.D + s.S + s.H + 255) / 256)), dim3(256), 0, st, heads, heads + HS * HD,
                      t_sum, small + at[2], d_ws, d_bs, d_t, (int)s.H, (int)s.S, (int)s.D);
-  if ((rc = launch_status())) return rc;
-  if (dx && (rc = general::rows_gemm(PA_F32, s, 2 * HD, s.C, d_proj, sv + sp.w_in_t, nullptr, 0, dx, st))) return rc;
-  return wgrad::product(PA_F32, M, d_proj, 2 * HD, 2 * HD, x, s.C, s.C, s.conv_k > 0 ? &s : nullptr, work, d_w_in, d_b_in, num_cu,
-                        st);
+  return launch_status();
 }
 
 }  // namespace train_f32

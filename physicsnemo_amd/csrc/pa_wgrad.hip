@@ -5,7 +5,7 @@
 //
 //   wgrad_kernel          bf16, up to 256 x 256 of P per workgroup, operands staged by direct global -> LDS loads
 //   narrow_wgrad_kernel   one side with at most 16 columns (input features, output channels), bf16 or fp32
-//   sum_partials_kernel   the fixed-order total, for both results of a call in one launch
+//   sum_partials_kernel   the fixed-order total, for several results in one launch
 // The fp32 tile kernel (cols_gemm_f32_kernel) and the narrower bf16 one (cols_gemm_kernel) are in pa_gemm.hip.
 #include "pa_common.h"
 #include "pa_host.h"
@@ -342,28 +342,26 @@ __global__ __launch_bounds__(256) void narrow_wgrad_kernel(NarrowArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// sum_partials_kernel: dst[e] = sum_g src[g][e], two results in one launch.  A workgroup takes 32 consecutive elements
-// x 8 interleaved eighths of the partials and adds the eighths up through LDS, always in the same order.  blockIdx.y: a
-// batch of such sums of the first result ([batch][g][e] -> [batch][e]); the second one is formed by batch 0.
-// taps > 1: the first result is [oa][tap][ob] and leaves as [oa][ob][tap], the order of a convolution's weight.
+// sum_partials_kernel: dst[e] = sum_g src[g][e], up to eight results in one launch: a backward pass has three to eight of
+// them, each 4 to 6 us for what is mostly too small to fill the chip.  A Transolver++ layer's step over 100 003 points takes
+// 650 us with one launch at the end of its backward pass where it took 658 with three, the float32 grid model's 4 604 with
+// one per layer and 4 653 with five.  A workgroup takes 32 consecutive elements x 8 interleaved eighths of the partials and
+// adds the eighths up through LDS, always in the
+// same order.  blockIdx.y: a batch of such sums of the first result ([batch][g][e] -> [batch][e]); the others are formed by
+// batch 0.
 // ------------------------------------------------------------------------------------------------
-struct SumArgs {
-  const float *src[2];
-  float *dst[2];
-  int64_t n[2];
-  int64_t blocks0;  // workgroups of the first result
-  int G[2], taps, OB;
-};
-
-__global__ __launch_bounds__(256) void sum_partials_kernel(SumArgs a) {
+__global__ __launch_bounds__(256) void sum_partials_kernel(Sums a) {
   __shared__ float part[8][32];
-  const int z = (int64_t)blockIdx.x >= a.blocks0 ? 1 : 0;
-  if (z && blockIdx.y > 0) return;
-  const int64_t e = ((int64_t)blockIdx.x - (z ? a.blocks0 : 0)) * 32 + (threadIdx.x & 31), n = a.n[z];
-  const int part_id = threadIdx.x >> 5, G = a.G[z];
+  Sums::One o = a.r[0];
+#pragma unroll
+  for (int k = 1; k < Sums::kMost; ++k)
+    if (k < a.count && (int64_t)blockIdx.x >= a.r[k].first) o = a.r[k];
+  if (o.first > 0 && blockIdx.y > 0) return;
+  const int64_t e = ((int64_t)blockIdx.x - o.first) * 32 + (threadIdx.x & 31), n = o.n;
+  const int part_id = threadIdx.x >> 5, G = o.G;
   float s = 0.f;
   if (e < n) {
-    const float *p = a.src[z] + (int64_t)blockIdx.y * G * n + e;
+    const float *p = o.src + (int64_t)blockIdx.y * G * n + e;
 #pragma unroll 8
     for (int g = part_id; g < G; g += 8) s += p[(int64_t)g * n];
   }
@@ -374,11 +372,11 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(SumArgs a) {
 #pragma unroll
     for (int k = 1; k < 8; ++k) v += part[k][threadIdx.x];
     int64_t at = (int64_t)blockIdx.y * n + e;
-    if (z == 0 && a.taps > 1) {
-      const int64_t oa = e / (a.taps * (int64_t)a.OB), rest = e - oa * a.taps * a.OB, tap = rest / a.OB, ob = rest - tap * a.OB;
-      at = (oa * a.OB + ob) * a.taps + tap;
+    if (o.taps > 1) {
+      const int64_t oa = e / (o.taps * (int64_t)o.OB), rest = e - oa * o.taps * o.OB, tap = rest / o.OB, ob = rest - tap * o.OB;
+      at = (oa * o.OB + ob) * o.taps + tap;
     }
-    a.dst[z][at] = v;
+    o.dst[at] = v;
   }
 }
 
@@ -528,7 +526,7 @@ int launch_wide(const void *A, int64_t lda, int64_t OA, const void *B, int64_t l
 }
 
 int product(int dtype, int64_t M, const void *A, int64_t lda, int64_t OA, const void *B, int64_t ldb, int64_t OB,
-            const pa_shape *grid, void *workspace, float *out, float *col_sums, int num_cu, hipStream_t st) {
+            const pa_shape *grid, void *workspace, float *out, float *col_sums, int num_cu, hipStream_t st, Sums *later) {
   const int taps = grid_taps(grid).taps;
   const Form f = form_of(dtype, OA, OB, taps);
   if (f == Form::none) return PA_ERR_UNSUPPORTED;
@@ -553,26 +551,23 @@ int product(int dtype, int64_t M, const void *A, int64_t lda, int64_t OA, const 
     }
   }
   if (rc) return rc;
-  SumArgs s{};
-  s.src[0] = partials, s.dst[0] = out, s.n[0] = n;
-  s.blocks0 = (n + 31) / 32;
-  int64_t blocks = s.blocks0;
-  if (col_sums) {
-    s.src[1] = sums, s.dst[1] = col_sums, s.n[1] = OA;
-    blocks += (OA + 31) / 32;
-  }
-  s.G[0] = s.G[1] = (int)G, s.taps = taps, s.OB = (int)OB;
-  hipLaunchKernelGGL(sum_partials_kernel, dim3((unsigned)blocks), dim3(256), 0, st, s);
+  Sums own, &s = later ? *later : own;
+  s.add(partials, out, n, G, taps, OB);
+  if (col_sums) s.add(sums, col_sums, OA, G);
+  return later ? PA_OK : launch_sums(own, st);
+}
+
+static int launch_sums(const Sums &sums, int64_t batches, hipStream_t st) {
+  hipLaunchKernelGGL(sum_partials_kernel, dim3((unsigned)sums.blocks, (unsigned)batches), dim3(256), 0, st, sums);
   return launch_status();
 }
+int launch_sums(const Sums &sums, hipStream_t st) { return launch_sums(sums, 1, st); }
 
 // dst[e] = sum over `rows` rows of n floats
 int sum_rows(const float *src, int64_t rows, int64_t n, float *dst, hipStream_t st) {
-  SumArgs s{};
-  s.src[0] = src, s.dst[0] = dst, s.n[0] = n, s.G[0] = (int)rows, s.taps = 1;
-  s.blocks0 = (n + 31) / 32;
-  hipLaunchKernelGGL(sum_partials_kernel, dim3((unsigned)s.blocks0), dim3(256), 0, st, s);
-  return launch_status();
+  Sums s;
+  s.add(src, dst, n, rows);
+  return launch_sums(s, st);
 }
 
 // ---- the layer's output gradient against the packed slice weights ----
@@ -636,16 +631,10 @@ int output_backward(const pa_shape &s, const void *w_pack, const void *dy, const
     hipLaunchKernelGGL(wgrad_kernel<2>, dim3((unsigned)((nb * p.G * a.ny * a.nz + 7) / 8 * 8)), dim3(512), lds, st, a);
     if ((rc = launch_status())) return rc;
     if (p.G > 1) {
-      SumArgs sa{};
-      sa.src[0] = partials, sa.dst[0] = P, sa.n[0] = p.n, sa.G[0] = (int)p.G, sa.taps = 1;
-      sa.blocks0 = (p.n + 31) / 32;
-      int64_t blocks = sa.blocks0;
-      if (p.parts == 1) {  // nothing else is to be added up: d b_out here
-        sa.src[1] = sums, sa.dst[1] = d_b_out, sa.n[1] = s.C, sa.G[1] = (int)(s.B * p.G);
-        blocks += (s.C + 31) / 32;
-      }
-      hipLaunchKernelGGL(sum_partials_kernel, dim3((unsigned)blocks, (unsigned)nb), dim3(256), 0, st, sa);
-      if ((rc = launch_status())) return rc;
+      Sums sa;
+      sa.add(partials, P, p.n, p.G);
+      if (p.parts == 1) sa.add(sums, d_b_out, s.C, s.B * p.G);  // nothing else is to be added up
+      if ((rc = launch_sums(sa, nb, st))) return rc;
     }
     const int64_t wgs = nb * s.H * ST + s.H * (s.C / 32) * ((nb + p.cb - 1) / p.cb);
     hipLaunchKernelGGL(token_grad_kernel, dim3((unsigned)wgs), dim3(256), 0, st, P, static_cast<const uint16_t *>(w_out),
@@ -654,16 +643,10 @@ int output_backward(const pa_shape &s, const void *w_pack, const void *dy, const
     if ((rc = launch_status())) return rc;
   }
   if (p.parts == 1 && p.G > 1) return PA_OK;
-  SumArgs sa{};
-  sa.src[0] = sums, sa.dst[0] = d_b_out, sa.n[0] = s.C, sa.G[0] = (int)(s.B * p.G), sa.taps = 1;
-  sa.blocks0 = (s.C + 31) / 32;
-  int64_t blocks = sa.blocks0;
-  if (p.parts > 1) {
-    sa.src[1] = dw, sa.dst[1] = d_w_out, sa.n[1] = s.C * HD, sa.G[1] = (int)p.parts;
-    blocks += (s.C * HD + 31) / 32;
-  }
-  hipLaunchKernelGGL(sum_partials_kernel, dim3((unsigned)blocks), dim3(256), 0, st, sa);
-  return launch_status();
+  Sums sa;
+  sa.add(sums, d_b_out, s.C, s.B * p.G);
+  if (p.parts > 1) sa.add(dw, d_w_out, s.C * HD, p.parts);
+  return launch_sums(sa, st);
 }
 
 }  // namespace wgrad
