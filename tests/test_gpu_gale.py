@@ -72,6 +72,28 @@ def test_cross_mix_stage_against_oracle_functions():
         assert_fp32_close(got, want, f"blend {mode}")
 
 
+@pytest.mark.parametrize("mode", ["weighted", "concat_project"])
+@pytest.mark.parametrize("S,Sc,Dc", [(16, 1, 8), (20, 31, 32), (32, 33, 72), (64, 64, 64), (128, 100, 16), (160, 128, 24), (64, 129, 32),
+                                     (64, 40, 36)])
+def test_cross_mix_of_32_wide_heads_against_float64(mode, S, Sc, Dc):
+    """Slice and context tokens off the tiles of 32, more slice tokens than one round of waves, both sides of the limits on the
+    context (128 tokens, rows of eight floats): float32 sums of at most 128 terms, 128 2^-24 = 8e-6 of their magnitudes."""
+    announce("GALE cross mix, 32-wide heads", mode, S, Sc, Dc)
+    torch.manual_seed(S + Sc)
+    B, H, D = 2, 3, 32
+    ref = to.OracleGALE(H * D, heads=H, dim_head=D, slice_num=S, context_dim=Dc, state_mixing_mode=mode)
+    hip = pn.GALE(H * D, heads=H, dim_head=D, slice_num=S, context_dim=Dc, state_mixing_mode=mode, use_te=False)
+    hip.load_state_dict(ref.state_dict())
+    ref.double()
+    tok, self_out, ctx = torch.randn(B, H, S, D), torch.randn(B, H, S, D), 2 * torch.randn(B, H, Sc, Dc)
+    with torch.no_grad():
+        cross = to.gale_cross_attention(tok.double(), ctx.double(), ref.cross_q, ref.cross_k, ref.cross_v)
+        want = to.gale_mix(self_out.double(), cross, mode, getattr(ref, "state_mixing", None), getattr(ref, "concat_project", None))
+    got = PF.slice_cross_attention_mix(tok.cuda(), self_out.cuda(), ctx.cuda(), hip.gale_params(torch.device("cuda")),
+                                       PF.LayerDims(B, 100, H * D, H, D, S))
+    assert_rel_l2(got, want, f"blend {mode}", tol=8e-6)
+
+
 @pytest.mark.parametrize("mode,S,N", [("weighted", 64, 4096), ("concat_project", 32, 5000), ("weighted", 128, 3000)])
 def test_bf16_gale_on_the_mfma_kernels(mode, S, N):
     announce("bf16 GALE MFMA", mode, S, N)
