@@ -173,9 +173,11 @@ __global__ __launch_bounds__(kAttnBwdThreads) void slice_attention_backward_kern
 // 32 x 32 tiles, rows one word longer than a tile multiple so that both the row-wise and the column-wise operand reads
 // fall on 32 different banks; the waves share the output tiles of each step.  P and dSc live in LDS too, or (SCRATCH:
 // S = 128 does not leave room) in the caller's 2 S^2 floats per (b, h), which stay in the L2.
-// Bound by the latency of its ten dependent steps (B * H workgroups, 8 for one sample of an eight-head layer): the
-// kernel above spends 155 us on S = 64, D = 32 at 8 workgroups, where a thread walks its products one fma at a time
-// through LDS reads; the tiles take 35 us (B = 8: 147 -> 30 us; 32 workgroups of S = 32, D = 16: 27 -> 17 us).
+// Bound by the latency of its ten dependent steps (B * H workgroups, 8 for one sample of an eight-head layer) and, each of
+// them running once, by fetching its code: the kernel above spends 155 us on S = 64, D = 32 at 8 workgroups, where a thread
+// walks its products one fma at a time through LDS reads; the tiles take 18 us (S = 32, D = 16: 12).  With a row of the
+// softmax per wave instead of per eight lanes, and d tok as one product of three times the depth, it took 28 (17); with the
+// eight lanes' loops unrolled into registers and a tile product inlined per kind of job, 32 (25).
 // ------------------------------------------------------------------------------------------------
 constexpr int kAttnMfmaWaves = kAttnBwdThreads / 64;
 
@@ -200,9 +202,10 @@ __device__ __forceinline__ mfma::f32x16 tile_product(const float *a, int ar, int
   const int lane = threadIdx.x & 63, i = lane & 31, g = lane >> 5;
   a += i * ar + g * ak;
   b += i * bc + g * bk;
-  for (int k0 = 0; k0 < K; k0 += 32) {  // K: whole tiles
+#pragma unroll 1
+  for (int k0 = 0; k0 < K; k0 += 16) {  // K: whole tiles
 #pragma unroll
-    for (int k = 0; k < 32; k += 2)
+    for (int k = 0; k < 16; k += 2)
       acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[(k0 + k) * ak], b[(k0 + k) * bk], acc, 0, 0, 0);
   }
   return acc;
@@ -256,21 +259,37 @@ __global__ __launch_bounds__(kAttnBwdThreads) void slice_attention_backward_mfma
     put((dp ? dSc : P) + ts * 32 * PS + tu * 32, PS, c, dp ? 1.f : scale);
   }
   __syncthreads();
-  for (int s = wave; s < d.SP; s += kAttnMfmaWaves) {  // softmax rows and their backward; rows and columns beyond S: 0
-    float *pr = P + s * PS, *dr = dSc + s * PS;
-    float mx = -INFINITY;
-    for (int u = lane; u < S; u += 64) mx = fmaxf(mx, pr[u]);
-    mx = wave_max(mx);
-    float sum = 0.f;
-    for (int u = lane; u < S; u += 64) sum += expf(pr[u] - mx);
-    const float inv = s < S ? 1.f / wave_sum(sum) : 0.f;
-    float delta = 0.f;
-    for (int u = lane; u < S; u += 64) delta = fmaf(expf(pr[u] - mx) * inv, dr[u], delta);
-    delta = wave_sum(delta);
-    for (int u = lane; u < d.SP; u += 64) {
-      const float p = u < S ? expf(pr[u] - mx) * inv : 0.f;
-      pr[u] = p;
-      dr[u] = u < S ? p * (dr[u] - delta) * scale : 0.f;
+  // eight lanes per row from here on, each a run of neighbouring elements: all rows of a round at once
+  const int l8 = lane & 7, per = d.SP / 8;
+  auto sum8 = [](float v) {
+    v += __shfl_xor(v, 1, 64);
+    v += __shfl_xor(v, 2, 64);
+    return v + __shfl_xor(v, 4, 64);
+  };
+  for (int s = 8 * wave + (lane >> 3); s < d.SP; s += 8 * kAttnMfmaWaves) {  // softmax and its backward; rows and columns beyond S: 0
+    float *pr = P + s * PS + l8 * per, *dr = dSc + s * PS + l8 * per;
+    const int n = s < S ? (S - l8 * per < per ? S - l8 * per : per) : 0;  // elements of the run within S
+    float mx = -INFINITY, sum = 0.f, delta = 0.f;
+#pragma unroll 2
+    for (int j = 0; j < n; ++j) mx = fmaxf(mx, pr[j]);
+    mx = fmaxf(mx, __shfl_xor(mx, 1, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 2, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 4, 64));
+#pragma unroll 2
+    for (int j = 0; j < n; ++j) {
+      const float e = expf(pr[j] - mx);
+      pr[j] = e;
+      sum += e;
+      delta = fmaf(e, dr[j], delta);
+    }
+    sum = sum8(sum);
+    const float inv = s < S ? 1.f / sum : 0.f;
+    delta = sum8(delta) * inv;
+#pragma unroll 2
+    for (int j = 0; j < per; ++j) {
+      const float p = j < n ? pr[j] * inv : 0.f, dp = j < n ? dr[j] : 0.f;
+      pr[j] = p;
+      dr[j] = p * (dp - delta) * scale;
     }
   }
   __syncthreads();
@@ -282,38 +301,39 @@ __global__ __launch_bounds__(kAttnBwdThreads) void slice_attention_backward_mfma
     put((m == 0 ? dq : m == 1 ? dk : dv) + ts * 32 * D1 + e0, D1, c, 1.f);
   }
   __syncthreads();
-  float *dtok = q;  // q is no longer needed
-  const int njobs = d.nS * d.nD;
-  for (int job = wave; job < njobs + 3 * d.nD * d.nD; job += kAttnMfmaWaves) {
-    if (job < njobs) {  // d tok = dq Wq + dk Wk + dv Wv
-      const int ts = job / d.nD, e0 = (job - ts * d.nD) * 32;
-      f32x16 c = zero;
+  // dW = d(q|k|v)^T tok, then the three terms of d tok = dq Wq + dk Wk + dv Wv (in q, k, v, which are no longer needed), as jobs
+  // of their own; dW, twice as long, has waves to itself where there are enough
+  const int terms = 3 * d.nS * d.nD, weights = 3 * d.nD * d.nD, apart = weights < kAttnMfmaWaves ? weights : 0;
+  const int stride = apart == 0 ? kAttnMfmaWaves : wave < apart ? terms + weights : kAttnMfmaWaves - apart;
+  for (int job = wave; job < terms + weights; job += stride) {
+    const bool term = job >= weights;
+    const int rest = term ? job - weights : job, m = rest % 3, tile = rest / 3, tr = tile / d.nD, tc = tile - tr * d.nD;
+    const float *src = dq + m * SD;
+    const f32x16 c = tile_product(src + tr * 32 * (term ? D1 : 1), term ? D1 : 1, term ? 1 : D1,
+                                  (term ? wq + m * d.DP * D1 : tok) + tc * 32, 1, D1, term ? d.DP : d.SP, zero);
+    if (term) {
+      put(q + m * SD + tr * 32 * D1 + tc * 32, D1, c, 1.f);
+      continue;
+    }
 #pragma unroll
-      for (int m = 0; m < 3; ++m)
-        c = tile_product((m == 0 ? dq : m == 1 ? dk : dv) + ts * 32 * D1, D1, 1, wq + m * d.DP * D1 + e0, 1, D1, d.DP, c);
-      put(dtok + ts * 32 * D1 + e0, D1, c, 1.f);
-    } else {  // dW = d(q|k|v)^T tok
-      const int w = job - njobs, m = w / (d.nD * d.nD), rest = w - m * d.nD * d.nD, te = rest / d.nD, td = rest - te * d.nD;
-      const f32x16 c =
-          tile_product((m == 0 ? dq : m == 1 ? dk : dv) + te * 32, 1, D1, tok + td * 32, 1, D1, d.SP, zero);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int e = te * 32 + mfma::rowmap(r, g), dd = td * 32 + i;
-        if (e < D && dd < D) d_wqkv_part[((int64_t)bh * 3 + m) * D * D + e * D + dd] = c[r];
-      }
+    for (int r = 0; r < 16; ++r) {
+      const int e = tr * 32 + mfma::rowmap(r, g), dd = tc * 32 + i;
+      if (e < D && dd < D) d_wqkv_part[((int64_t)bh * 3 + m) * D * D + e * D + dd] = c[r];
     }
   }
   __syncthreads();
-  for (int u = t; u < S * D; u += kAttnBwdThreads) {
-    const int s = u / D, e = u - s * D;
-    const float inv = slice_norm ? 1.f / slice_norm[(int64_t)bh * S + s] : 1.f;
-    d_num[(int64_t)bh * S * D + u] = dtok[s * D1 + e] * inv;
-  }
-  if (!slice_norm) return;
-  for (int s = t; s < S; s += kAttnBwdThreads) {
+  for (int s = 8 * wave + (lane >> 3); s < d.SP; s += 8 * kAttnMfmaWaves) {  // d num = d tok / nrm,  d nrm = -(d tok . tok) / nrm
+    const bool row = s < S;
+    const float inv = slice_norm && row ? 1.f / slice_norm[(int64_t)bh * S + s] : 1.f;
     float acc = 0.f;
-    for (int e = 0; e < D; ++e) acc = fmaf(dtok[s * D1 + e], tok[s * D1 + e], acc);
-    d_norm[(int64_t)bh * S + s] = -acc / slice_norm[(int64_t)bh * S + s];
+    for (int e = l8; e < D; e += 8) {
+      const int at = s * D1 + e;
+      const float t3 = (q[at] + k[at]) + v[at];
+      acc = fmaf(t3, tok[at], acc);
+      if (row) d_num[((int64_t)bh * S + s) * D + e] = t3 * inv;
+    }
+    acc = sum8(acc);
+    if (slice_norm && row && l8 == 0) d_norm[(int64_t)bh * S + s] = -acc / slice_norm[(int64_t)bh * S + s];
   }
 }
 
