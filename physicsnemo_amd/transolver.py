@@ -10,7 +10,8 @@ and every block MLP the fused kernel does not serve.
 Module names, registration order and state_dict keys match the reference so its checkpoints load unchanged,
 including the legacy ``linear_pre`` / ``linear_post`` MLP keys (:92-97).
 Training (gradients required): the layer runs its differentiable path (stage-level kernels forward, the library's
-backward kernels backward); LayerNorms, MLPs and residual adds are differentiable PyTorch-ROCm tensor ops.
+backward kernels backward); the blocks' LayerNorms and MLPs take the library's functions where these serve the call and are
+differentiable PyTorch-ROCm tensor ops elsewhere.
 """
 from __future__ import annotations
 
@@ -233,7 +234,7 @@ class TransolverBlock(nn.Module):
         """One block inside a chain of blocks: takes LayerNorm_1(fx) if the previous stage already produced it and
         returns (fx_out, next_ln(fx_out) or None).  Same arithmetic as `forward` (reference :300-303)."""
         if self._needs_grad(fx):
-            # training: the layer's autograd path, LayerNorms / MLP as differentiable tensor ops (reference :300-303)
+            # training: the layer's autograd path, LayerNorms / MLP on the library's functions or tensor ops (reference :300-303)
             x_in, fx = (normed_in, fx) if normed_in is not None else PA.layer_norm_residual(fx, self.ln_1)
             pair, ln2, mlp = None, self.ln_mlp1[0], self.ln_mlp1[1]
             apart = type(mlp) is Mlp and PA.unhooked(mlp) and PA.norm_mlp_fused(fx, ln2, mlp.layers)
