@@ -366,15 +366,25 @@ __global__ __launch_bounds__(256) void softmax_rows_plus_vec_kernel(T *__restric
 //   partial[s, d] = sum_n w[n, s] * fx_mid[n, d]   (d < D),   partial[s, D] = sum_n w[n, s]
 // The (S x D+1) output is cut into 4 x 4 register tiles; a thread owns NS of them (tile t + 256 i of its slab of
 // 256 NS tiles) and walks the chunk 64 points at a time through LDS: per point and tile two 16-byte LDS reads
-// (4 slice weights, 4 features) feed 16 FMAs.  LDS rows are padded to multiples of four (zeros; column D of the
+// (4 slice weights, 4 features) feed 16 FMAs.  Up to 256 tiles several groups of threads take every so many points, their
+// sums added up through LDS: S = 32, D = 16 has 40 tiles, 4 x 7 225 points of 8 heads 18 us in six groups, 36 with 216 of
+// 256 threads waiting; S = 64, D = 32 (144 tiles, 65 536 points in bf16) 37 us in three groups of 512 threads, 41 before.
+// LDS rows are padded to multiples of four (zeros; column D of the
 // feature rows holds 1 for the count).  Sums run in a fixed order, so the result is bit-reproducible.
 // ------------------------------------------------------------------------------------------------
 constexpr int kAttnThreads = 1024;  // slice_combine_attn_kernel: 16 waves, one query row per wave at a time
 constexpr int kPartialTile = 64;
 constexpr int kPartialMaxNS = 4;
 
+// threads of a workgroup and the groups of them that share a chunk's points (up to 256 tiles)
+__host__ __device__ inline int partial_threads(int n_tiles) { return n_tiles > 128 ? 512 : 256; }
+__host__ __device__ inline int partial_groups(int n_tiles) {
+  const int g = partial_threads(n_tiles) / n_tiles;
+  return g > 32 ? 32 : g;
+}
+
 template <typename T, int NS>
-__global__ __launch_bounds__(256) void slice_partial_kernel(const T *__restrict__ w, const T *__restrict__ fx_mid,
+__global__ __launch_bounds__(NS == 1 ? 512 : 256) void slice_partial_kernel(const T *__restrict__ w, const T *__restrict__ fx_mid,
                                                             float *__restrict__ partials, int B, int64_t N, int H, int D,
                                                             int S, int64_t chunk) {
   extern __shared__ float4 lds4[];
@@ -387,11 +397,13 @@ __global__ __launch_bounds__(256) void slice_partial_kernel(const T *__restrict_
   const int b = blockIdx.y / H, h = blockIdx.y % H;
   const int n_tiles = SB * DB;
   const int slab0 = blockIdx.z * 256 * NS;
+  const int threads = NS == 1 ? blockDim.x : 256;
+  const int groups = NS == 1 ? partial_groups(n_tiles) : 1, tile0 = NS == 1 ? t % n_tiles : t, group = NS == 1 ? t / n_tiles : 0;
   int sb[NS], db[NS];
   float acc[NS][4][4];
 #pragma unroll
   for (int i = 0; i < NS; ++i) {
-    const int tile = slab0 + t + 256 * i;
+    const int tile = slab0 + tile0 + 256 * i;
     const bool ok = tile < n_tiles;
     sb[i] = ok ? tile % SB : 0;
     db[i] = ok ? tile / SB : 0;
@@ -411,7 +423,7 @@ __global__ __launch_bounds__(256) void slice_partial_kernel(const T *__restrict_
     const int pts = (int)min((int64_t)kPartialTile, n_end - n0);
     if (vec_w) {  // 16-byte loads: the rows are whole numbers of 16-byte units
       const int units = S / UE;
-      for (int i = t; i < kPartialTile * units; i += 256) {
+      for (int i = t; i < kPartialTile * units; i += threads) {
         const int p = i / units, u = i - p * units;
         u32x4 raw = {0u, 0u, 0u, 0u};
         if (p < pts) raw = *reinterpret_cast<const u32x4 *>(w + ((int64_t)b * N + n0 + p) * HS + h * S + u * UE);
@@ -420,14 +432,14 @@ __global__ __launch_bounds__(256) void slice_partial_kernel(const T *__restrict_
         for (int j = 0; j < UE; ++j) wlf[p * (SB * 4) + u * UE + j] = load_as_f32(e + j);
       }
     } else {
-      for (int i = t; i < kPartialTile * SB * 4; i += 256) {
+      for (int i = t; i < kPartialTile * SB * 4; i += threads) {
         const int p = i / (SB * 4), s = i - p * (SB * 4);
         wlf[i] = (p < pts && s < S) ? load_as_f32(w + ((int64_t)b * N + n0 + p) * HS + h * S + s) : 0.f;
       }
     }
     if (vec_f) {
       const int units = D / UE;
-      for (int i = t; i < kPartialTile * units; i += 256) {
+      for (int i = t; i < kPartialTile * units; i += threads) {
         const int p = i / units, u = i - p * units;
         u32x4 raw = {0u, 0u, 0u, 0u};
         if (p < pts) raw = *reinterpret_cast<const u32x4 *>(fx_mid + ((int64_t)b * N + n0 + p) * HD + h * D + u * UE);
@@ -435,12 +447,12 @@ __global__ __launch_bounds__(256) void slice_partial_kernel(const T *__restrict_
 #pragma unroll
         for (int j = 0; j < UE; ++j) flf[p * (DB * 4) + u * UE + j] = load_as_f32(e + j);
       }
-      for (int i = t; i < kPartialTile * (DB * 4 - D); i += 256) {  // the count column and the padding behind it
+      for (int i = t; i < kPartialTile * (DB * 4 - D); i += threads) {  // the count column and the padding behind it
         const int p = i / (DB * 4 - D), d = D + i - p * (DB * 4 - D);
         flf[p * (DB * 4) + d] = (p < pts && d == D) ? 1.f : 0.f;
       }
     } else {
-      for (int i = t; i < kPartialTile * DB * 4; i += 256) {
+      for (int i = t; i < kPartialTile * DB * 4; i += threads) {
         const int p = i / (DB * 4), d = i - p * (DB * 4);
         float v = 0.f;
         if (p < pts && d < D) v = load_as_f32(fx_mid + ((int64_t)b * N + n0 + p) * HD + h * D + d);
@@ -450,7 +462,7 @@ __global__ __launch_bounds__(256) void slice_partial_kernel(const T *__restrict_
     }
     __syncthreads();
 #pragma unroll 2
-    for (int p = 0; p < kPartialTile; ++p) {
+    for (int p = group; p < kPartialTile; p += groups) {
 #pragma unroll
       for (int i = 0; i < NS; ++i) {
         const float4 wv = wl[p * SB + sb[i]];
@@ -464,10 +476,26 @@ __global__ __launch_bounds__(256) void slice_partial_kernel(const T *__restrict_
     }
     __syncthreads();
   }
+  if (groups > 1) {  // the groups' sums added up in order
+    float4 *part = lds4 + ((group - 1) * n_tiles + tile0) * 4;
+    if (group > 0 && group < groups) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) part[u] = float4{acc[0][u][0], acc[0][u][1], acc[0][u][2], acc[0][u][3]};
+    }
+    __syncthreads();
+    if (group > 0) return;
+    for (int q = 1; q < groups; ++q) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float4 v = lds4[((q - 1) * n_tiles + tile0) * 4 + u];
+        acc[0][u][0] += v.x, acc[0][u][1] += v.y, acc[0][u][2] += v.z, acc[0][u][3] += v.w;
+      }
+    }
+  }
   float *dst = partials + (((int64_t)g * B + b) * H + h) * (S * D1);
 #pragma unroll
   for (int i = 0; i < NS; ++i) {
-    if (slab0 + t + 256 * i >= n_tiles) continue;
+    if (slab0 + tile0 + 256 * i >= n_tiles) continue;
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
@@ -1337,15 +1365,16 @@ static int slice_partial_t(const pa_shape &s, const void *w, const void *fx_mid,
   const int64_t chunk = (s.N + G - 1) / G;
   const int SB = (int)((s.S + 3) / 4), DB = (int)((s.D + 1 + 3) / 4);
   const int n_tiles = SB * DB;
-  const size_t lds = (size_t)kPartialTile * (SB + DB) * 16;
+  const size_t rows = (size_t)kPartialTile * (SB + DB) * 16, sums = n_tiles <= 256 ? (size_t)(partial_groups(n_tiles) - 1) * n_tiles * 64 : 0;
+  const size_t lds = rows > sums ? rows : sums;
   const int per_thread = (n_tiles + 255) / 256;
   const int ns = per_thread <= 1 ? 1 : (per_thread <= 2 ? 2 : kPartialMaxNS);
   dim3 grid((unsigned)G, (unsigned)(s.B * s.H), (unsigned)((n_tiles + 256 * ns - 1) / (256 * ns)));
   auto launch = [&](auto kernel) {
     int rc = allow_dynamic_lds(kernel, lds);
     if (rc) return rc;
-    hipLaunchKernelGGL(kernel, grid, dim3(256), lds, st, static_cast<const T *>(w), static_cast<const T *>(fx_mid),
-                       partials, (int)s.B, s.N, (int)s.H, (int)s.D, (int)s.S, chunk);
+    hipLaunchKernelGGL(kernel, grid, dim3(ns == 1 ? partial_threads(n_tiles) : 256), lds, st, static_cast<const T *>(w),
+                       static_cast<const T *>(fx_mid), partials, (int)s.B, s.N, (int)s.H, (int)s.D, (int)s.S, chunk);
     return launch_status();
   };
   if (ns == 1) return launch(slice_partial_kernel<T, 1>);

@@ -481,3 +481,21 @@ def test_fp32_narrow_heads_attend_in_one_launch_with_the_same_bits(C, H, N):
         y, tok = PF.layer_forward(x, layer.kernel_params(x.dtype, x.device), layer.layer_dims(x), return_slice_tokens=True)
     assert torch.isfinite(y).all()
     assert torch.equal(tok, stages["tok"]) and torch.equal(y, stages["y"])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("S,D,N", [(1, 3, 1), (8, 8, 63), (32, 16, 257), (20, 24, 1000), (64, 32, 3001), (64, 60, 130), (64, 64, 300),
+                                   (128, 28, 640)])
+def test_slice_sums_over_groups_of_threads(dtype, S, D, N):
+    """The sums over the points where an output of few tiles is shared by groups of threads: 1 to 256 tiles of 4 x 4 and beyond,
+    ragged chunks.  float32 sums of at most 256 terms per partial result, 256 2^-24 = 1.5e-5."""
+    announce("slice sums", dtype, S, D, N)
+    torch.manual_seed(S + D)
+    B, H = 2, 3
+    w = torch.softmax(torch.randn(B, N, H, S), -1).cuda().to(dtype)
+    f = torch.randn(B, N, H * D).cuda().to(dtype)
+    tok, norm = PF.slice_reduce(w, f, PF.LayerDims(B, N, H * D, H, D, S))
+    count = w.double().sum(1) + 1e-2
+    want = torch.einsum("bnhs,bnhd->bhsd", w.double(), f.double().view(B, N, H, D)) / count[..., None]
+    assert_rel_l2(norm, count, "norm", tol=1.5e-5)
+    assert_rel_l2(tok, want, "tokens", tol=1.5e-5)
