@@ -62,9 +62,11 @@ __global__ __launch_bounds__(256) void hidden_backward_pack_kernel(const uint16_
 // Rows past M repeat row M - 1 and write the same values to the same place, so that the number of stores in flight,
 // which the wait at a slot's start counts, is the same for every wave.
 // splits: the hidden units are independent of each other, so short inputs spread them over the chip.
-// Bound by its stores behind the matrix and vector work (4 C + 4 F bytes per row): 262 144 rows, F = 1024: 415 us.  With
-// GELU in the logistic form, good to 2.6e-5, it was 391; of those, without the stores 309, with 64-byte pieces of rows
-// leaving after every slot 492, with ordinary instead of streaming stores 436.
+// Bound by its vector work (330 vector and 32 transcendental instructions per slot of 32 matrix ones) and the stores
+// behind it (4 C + 4 F bytes per row): 262 144 rows, F = 1024: 405 us, 415 with the accumulators of one chunk copied over for
+// the next instead of two sets taking turns, and 64-bit addresses per store.  Of those 415, GELU in the logistic form, good to
+// 2.6e-5, 24 less; with it 309 without the stores, 492 with 64-byte pieces of rows leaving after every slot, 436 with ordinary
+// instead of streaming stores.
 // ---------------------------------------------------------------------------------------------------------------
 template <int C>
 __global__ __launch_bounds__(512) void hidden_backward_kernel(const u32x4 *__restrict__ blob, const float *__restrict__ b1,
@@ -96,21 +98,20 @@ __global__ __launch_bounds__(512) void hidden_backward_kernel(const u32x4 *__res
       db[ks] = *reinterpret_cast<const u32x4 *>(dy + r * C + 8 * g + 16 * ks);
     }
   };
-  f32x16 hprev, dprev;
+  f32x16 h[2], d[2];  // of an even and of an odd chunk
   uint32_t gp[2], dp[2];
   float geven = 0.f, deven = 0.f;
-  // value k of the chunk before, `odd` its position in its pair; the staged row i holds its 16-byte granule j at j ^ i % 8
-  int odd = 0;
-  auto activate = [&](auto k_) {
-    constexpr int k = decltype(k_)::value, q = k >> 2;
-    const float x = hprev[k];
+  // value k of an even or odd chunk; the staged row i holds its 16-byte granule j at j ^ i % 8
+  auto activate = [&](auto k_, auto odd_) {
+    constexpr int k = decltype(k_)::value, q = k >> 2, odd = decltype(odd_)::value;
+    const float x = h[odd][k];
     const GeluParts p = gelu_parts(x);
-    const float d = dprev[k] * gelu_grad(x, p);
+    const float dv = d[odd][k] * gelu_grad(x, p);
     if constexpr (k % 2 == 0) {
-      geven = x * p.phi, deven = d;
+      geven = x * p.phi, deven = dv;
     } else {
       gp[(k >> 1) & 1] = pack2(geven, x * p.phi);
-      dp[(k >> 1) & 1] = pack2(deven, d);
+      dp[(k >> 1) & 1] = pack2(deven, dv);
     }
     if constexpr (k % 4 == 3) {
       char *at = stage + i * 128 + (((q ^ (i & 7)) << 4) ^ (odd << 6)) + 8 * g;
@@ -118,16 +119,15 @@ __global__ __launch_bounds__(512) void hidden_backward_kernel(const u32x4 *__res
       *reinterpret_cast<u32x2 *>(at + 4096) = u32x2{dp[0], dp[1]};
     }
   };
+  uint32_t row_at[4];  // this lane's pieces of the item's rows, elements from the wave's first row on
   auto store_pair = [&](int64_t row0, int c) {  // chunks c, c + 1; the wave's LDS operations complete in order
+    uint16_t *ga = act + row0 * F + 32 * c, *da = dh + row0 * F + 32 * c;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const int rw = 8 * t + (lane >> 3);
       const char *at = stage + rw * 128 + (((lane & 7) ^ (rw & 7)) << 4);
-      int64_t r = row0 + rw;
-      if (r >= M) r = M - 1;
-      const int64_t off = r * F + 32 * c + 8 * (lane & 7);
-      store_streaming(reinterpret_cast<u32x4 *>(act + off), *reinterpret_cast<const u32x4 *>(at));
-      store_streaming(reinterpret_cast<u32x4 *>(dh + off), *reinterpret_cast<const u32x4 *>(at + 4096));
+      store_streaming(reinterpret_cast<u32x4 *>(ga + row_at[t]), *reinterpret_cast<const u32x4 *>(at));
+      store_streaming(reinterpret_cast<u32x4 *>(da + row_at[t]), *reinterpret_cast<const u32x4 *>(at + 4096));
     }
   };
   // Workgroups go round their chunks from different starts: all at the same one would write the same 128 bytes of every
@@ -139,25 +139,31 @@ __global__ __launch_bounds__(512) void hidden_backward_kernel(const u32x4 *__res
     load_rows(blockIdx.x);
   }
   for (int64_t item = blockIdx.x; item < items; item += gridDim.x) {
-    const int64_t row0 = item / splits * 256 + wave * 32, next = item + gridDim.x < items ? item + gridDim.x : item;
+    // a wave whose rows all lie past M works on the last row
+    const int64_t row = item / splits * 256 + wave * 32, row0 = row < M ? row : M - 1, next = item + gridDim.x < items ? item + gridDim.x : item;
     const int c0 = (int)(item % splits) * CPS, cn = (int)(next % splits) * CPS;
+    const int last = (int)(M - 1 - row0 < 31 ? M - 1 - row0 : 31);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) hprev[r] = dprev[r] = 0.f;
+    for (int t = 0; t < 4; ++t) {
+      const int rw = 8 * t + (lane >> 3);
+      row_at[t] = (uint32_t)((rw < last ? rw : last) * F + 8 * (lane & 7));
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) h[1][r] = d[1][r] = 0.f;
     // the rows are here: said to the compiler, which otherwise waits for them (and all that follows them) in every slot
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
-    for (int c = 0; c < CPS; ++c, ++gs) {
+    auto slot = [&](int c, auto odd_) {
+      constexpr int odd = decltype(odd_)::value;
       // slot gs has landed (every wave waits for its own share, then all meet) and the other buffer is free.  Its loads
       // were issued before the eight stores of an even slot, which may still be in flight.
-      odd = (c & 1) ^ 1;
-      if (odd || c == 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (!odd || c == 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
       __syncthreads();
       const int ch = chunk_of(c0, c);
       fetch(gs + 1, c + 1 < CPS ? chunk_of(c0, c + 1) : chunk_of(cn, 0));
       const u32x4 *wb = wbuf + (gs & 1) * SU + lane;
-      f32x16 h, d;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) h[r] = b1s[32 * ch + rowmap(r, g)], d[r] = 0.f;
+      for (int r = 0; r < 16; ++r) h[odd][r] = b1s[32 * ch + rowmap(r, g)], d[odd][r] = 0.f;
       constexpr int RING = 8, AHEAD = 4;
       u32x4 fr[RING];
       static_for<AHEAD>([&](auto q) { fr[decltype(q)::value] = wb[decltype(q)::value * 64]; });
@@ -167,20 +173,24 @@ __global__ __launch_bounds__(512) void hidden_backward_kernel(const u32x4 *__res
           constexpr int f = 4 * p + decltype(q)::value + AHEAD;
           if constexpr (f < 2 * KS) fr[f % RING] = wb[f * 64];
         });
-        h = mma(fr[(4 * p) % RING], ub[2 * p], h);
-        d = mma(fr[(4 * p + 1) % RING], db[2 * p], d);
-        activate(std::integral_constant<int, 2 * p>{});
-        h = mma(fr[(4 * p + 2) % RING], ub[2 * p + 1], h);
-        d = mma(fr[(4 * p + 3) % RING], db[2 * p + 1], d);
-        activate(std::integral_constant<int, 2 * p + 1>{});
+        constexpr std::integral_constant<int, 1 - odd> before{};
+        h[odd] = mma(fr[(4 * p) % RING], ub[2 * p], h[odd]);
+        d[odd] = mma(fr[(4 * p + 1) % RING], db[2 * p], d[odd]);
+        activate(std::integral_constant<int, 2 * p>{}, before);
+        h[odd] = mma(fr[(4 * p + 2) % RING], ub[2 * p + 1], h[odd]);
+        d[odd] = mma(fr[(4 * p + 3) % RING], db[2 * p + 1], d[odd]);
+        activate(std::integral_constant<int, 2 * p + 1>{}, before);
         __builtin_amdgcn_sched_barrier(0);
       });
-      if (odd && c > 0) store_pair(row0, chunk_of(c0, c - 2));
-      hprev = h, dprev = d;
+      ++gs;
+    };
+    for (int c = 0; c < CPS; c += 2) {
+      slot(c, std::integral_constant<int, 0>{});
+      if (c > 0) store_pair(row0, chunk_of(c0, c - 2));
+      slot(c + 1, std::integral_constant<int, 1>{});
     }
-    odd = 1;
     load_rows(next);
-    static_for<16>(activate);
+    static_for<16>([&](auto k) { activate(k, std::integral_constant<int, 1>{}); });
     store_pair(row0, chunk_of(c0, CPS - 2));
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be landing in LDS when the workgroup ends
