@@ -155,6 +155,8 @@ __global__ __launch_bounds__(kLayerPointWaves * 64) void layer_point_backward_ke
   // Matrix instructions that stay where they are written (the builtin's sink behind all of the softmax), the weights in
   // accumulation registers.  The compiler does not see them as such: `begin` and `finish` keep the distance that vector
   // instructions need to a tile's first and from its last.
+  // In between their operands come from LDS and from registers that
+  // nothing writes inside the loop (in the assembly no vector instruction writes an operand within eight wait states).
   auto multiply = [](const u32x4 &w, const u32x4 &v, f32x16 &acc) {
     asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc) : "a"(w), "v"(v));
   };
