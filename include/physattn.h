@@ -560,6 +560,15 @@ int64_t pa_norm_mlp_backward_workspace_bytes(int dtype, int64_t rows, int64_t C,
 int pa_norm_mlp_backward(int dtype, int64_t rows, int64_t C, int64_t F, const pa_mlp_params *p, const void *u, const void *dy,
                          const void *x, const float *ln_gamma, float ln_eps, void *dx, float *grads, void *workspace,
                          int64_t workspace_bytes, void *stream);
+/* The same for an Mlp of which parts are frozen: `wanted` names the Linears whose weight and bias gradients are formed
+ * (PA_GRAD_LINEAR1 | PA_GRAD_LINEAR2; 0: dx and the LayerNorm's alone), dx NULL: neither dx nor the LayerNorm's.  The places in
+ * grads of what is not formed are left as they are. */
+#define PA_GRAD_LINEAR1 1
+#define PA_GRAD_LINEAR2 2
+int64_t pa_norm_mlp_backward_wanted_workspace_bytes(int dtype, int64_t rows, int64_t C, int64_t F, int wanted);
+int pa_norm_mlp_backward_wanted(int dtype, int64_t rows, int64_t C, int64_t F, int wanted, const pa_mlp_params *p, const void *u,
+                                const void *dy, const void *x, const float *ln_gamma, float ln_eps, void *dx, float *grads,
+                                void *workspace, int64_t workspace_bytes, void *stream);
 /* pa_mlp_forward_packed for rows that still lack the LayerNorm in front of the Mlp: the kernel applies
  * LayerNorm(in_ln) to the rows of u as it turns them into operands, so `ln_mlp1[0]` of TransolverBlock (TR.py:303) costs
  * no pass over memory and its producer (the attention layer's tail) need not write a normalised copy.  With

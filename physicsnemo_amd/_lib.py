@@ -23,6 +23,7 @@ EXPORTED = [
      "pa_mfma_combine_attention", "pa_mfma_deslice_project", "pa_mlp_query", "pa_mlp_workspace_bytes", "pa_mlp_forward", "pa_mlp_pack", "pa_mlp_pack_e4m3", "pa_mlp_input_ln_query", "pa_mlp_forward_packed_ln",
      "pa_mlp_forward_packed", "pa_mlp_train_forward", "pa_mlp_backward_workspace_bytes", "pa_mlp_backward",
     "pa_norm_mlp_backward_workspace_bytes", "pa_norm_mlp_backward",
+    "pa_norm_mlp_backward_wanted_workspace_bytes", "pa_norm_mlp_backward_wanted",
     "pa_rows_gemm", "pa_slice_weighted_sum", "pa_backward_query", "pa_backward_point_tiles",
     "pa_slice_attention_backward", "pa_slice_softmax_backward", "pa_slice_softmax_plus",
     "pa_backward_point_tiles_plus", "pa_slice_softmax_plus_backward", "pa_slice_cross_attention_mix",
@@ -45,6 +46,7 @@ EXPORTED = [
 ]
 
 PA_TRAIN_SAVED, PA_TRAIN_FORWARD, PA_TRAIN_BACKWARD, PA_TRAIN_GRADS = range(4)
+PA_GRAD_LINEAR1, PA_GRAD_LINEAR2 = 1, 2
 PA_BUF_BLOB, PA_BUF_FX_PACK, PA_BUF_W_PACK, PA_BUF_PARTIALS, PA_BUF_TOKP = range(5)
 
 
@@ -168,6 +170,11 @@ def load() -> ctypes.CDLL:
     lib.pa_norm_mlp_backward_workspace_bytes.argtypes = [c_int, c_int64, c_int64, c_int64]
     lib.pa_norm_mlp_backward.restype = c_int
     lib.pa_norm_mlp_backward.argtypes = [c_int, c_int64, c_int64, c_int64, POINTER(PaMlpParams)] + [c_void_p] * 4 + [
+        c_float] + [c_void_p] * 3 + [c_int64, c_void_p]
+    lib.pa_norm_mlp_backward_wanted_workspace_bytes.restype = c_int64
+    lib.pa_norm_mlp_backward_wanted_workspace_bytes.argtypes = [c_int, c_int64, c_int64, c_int64, c_int]
+    lib.pa_norm_mlp_backward_wanted.restype = c_int
+    lib.pa_norm_mlp_backward_wanted.argtypes = [c_int, c_int64, c_int64, c_int64, c_int, POINTER(PaMlpParams)] + [c_void_p] * 4 + [
         c_float] + [c_void_p] * 3 + [c_int64, c_void_p]
     lib.pa_mlp_pack.restype = c_int
     lib.pa_mlp_pack.argtypes = [c_int, c_int64, c_int64, POINTER(PaMlpParams), c_void_p, c_int64, c_void_p]

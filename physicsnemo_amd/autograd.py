@@ -865,6 +865,7 @@ class NormMlpResidualFunction(torch.autograd.Function):
         if dy is None:
             return (None,) * 12
         dy16 = _aligned(dy.to(x.dtype))
+        linear1, linear2 = need[5] or need[6], need[7] or need[8]
         if torch.is_grad_enabled():  # create_graph: the same formulas as tensor ops on the parameters, differentiable again
             with torch.autocast("cuda", enabled=False):
                 lw, lb, p1, pb1, p2 = _kept_parameters(ctx)[:5]
@@ -874,10 +875,12 @@ class NormMlpResidualFunction(torch.autograd.Function):
                 act, dh = torch.nn.functional.gelu(h), torch.ops.aten.gelu_backward(dy16 @ w2, h)
                 dx, d_ln, d_lb = _layernorm_grad_ops(x, dh @ w1, lw, ctx.norm_eps, dy16)
                 rows = lambda d, i: (_rows(d).float().t() @ _rows(i).float(), _rows(d).sum(0, dtype=torch.float32))
-                grads = (*rows(dh, u), *rows(dy16, act), d_ln, d_lb)
+                grads = (*(rows(dh, u) if linear1 else (None, None)), *(rows(dy16, act) if linear2 else (None, None)), d_ln, d_lb)
         else:
-            dx, *grads = PF.norm_mlp_backward(normed, dy16, x, w1, b1, w2, ln_w, ctx.norm_eps)
-        d_w1, d_b1, d_w2, d_b2, d_ln, d_lb = (g.to(t) for g, t in zip(grads, ctx.param_dtypes))
+            dx, *grads = PF.norm_mlp_backward(normed, dy16, x, w1, b1, w2, ln_w, ctx.norm_eps, linear1, linear2,
+                                              need[0] or need[2] or need[3])
+        wanted = need[5:9] + need[2:4]
+        d_w1, d_b1, d_w2, d_b2, d_ln, d_lb = (g.to(t) if n else None for g, t, n in zip(grads, ctx.param_dtypes, wanted))
         return (dx, None, d_ln, d_lb, None, d_w1, d_b1, d_w2, d_b2, *d_nxt, None)
 
 

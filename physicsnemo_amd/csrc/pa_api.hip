@@ -1234,7 +1234,7 @@ namespace {
 struct NormMlpPlan {
   int64_t act, dh, blob, w1_t, partials, work_w1, work_w2, total;
 };
-NormMlpPlan norm_mlp_plan(int64_t rows, int64_t C, int64_t F) {
+NormMlpPlan norm_mlp_plan(int64_t rows, int64_t C, int64_t F, int wanted) {
   NormMlpPlan p{};
   int64_t off = 0;
   auto take = [&](int64_t bytes) {
@@ -1250,32 +1250,36 @@ NormMlpPlan norm_mlp_plan(int64_t rows, int64_t C, int64_t F) {
   const int64_t w1 = pa::wgrad::workspace_bytes(PA_BF16, rows, F, C, 1, compute_units()),
                 w2 = pa::wgrad::workspace_bytes(PA_BF16, rows, C, F, 1, compute_units());
   if (w1 <= 0 || w2 <= 0) return p;
-  p.work_w1 = take(w1), p.work_w2 = take(w2);
+  p.work_w1 = take(wanted & PA_GRAD_LINEAR1 ? w1 : 0), p.work_w2 = take(wanted & PA_GRAD_LINEAR2 ? w2 : 0);
   p.total = off;
   return p;
 }
 }  // namespace
 
-int64_t pa_norm_mlp_backward_workspace_bytes(int dtype, int64_t rows, int64_t C, int64_t F) {
+int64_t pa_norm_mlp_backward_wanted_workspace_bytes(int dtype, int64_t rows, int64_t C, int64_t F, int wanted) {
   const int64_t hidden = pa_mlp_backward_workspace_bytes(dtype, rows, C, F);
   if (hidden < 0) return hidden;
   if (!pa::norm::rows_ln_backward_supported(rows, C, F)) return PA_ERR_UNSUPPORTED;
-  const int64_t total = norm_mlp_plan(rows, C, F).total;
+  const int64_t total = norm_mlp_plan(rows, C, F, wanted).total;
   return total > 0 ? total : PA_ERR_UNSUPPORTED;
 }
 
-int pa_norm_mlp_backward(int dtype, int64_t rows, int64_t C, int64_t F, const pa_mlp_params *p, const void *u, const void *dy,
-                         const void *x, const float *ln_gamma, float ln_eps, void *dx, float *grads, void *workspace,
-                         int64_t workspace_bytes, void *stream) {
+int64_t pa_norm_mlp_backward_workspace_bytes(int dtype, int64_t rows, int64_t C, int64_t F) {
+  return pa_norm_mlp_backward_wanted_workspace_bytes(dtype, rows, C, F, PA_GRAD_LINEAR1 | PA_GRAD_LINEAR2);
+}
+
+int pa_norm_mlp_backward_wanted(int dtype, int64_t rows, int64_t C, int64_t F, int wanted, const pa_mlp_params *p, const void *u,
+                                const void *dy, const void *x, const float *ln_gamma, float ln_eps, void *dx, float *grads,
+                                void *workspace, int64_t workspace_bytes, void *stream) {
   Range entry("pa_norm_mlp_backward");
-  const int64_t need = pa_norm_mlp_backward_workspace_bytes(dtype, rows, C, F);
+  const int64_t need = pa_norm_mlp_backward_wanted_workspace_bytes(dtype, rows, C, F, wanted);
   if (need < 0) return (int)need;
-  if (!p || !p->w1 || !p->b1 || !p->w2 || !u || !dy || !x || !ln_gamma || !dx || !grads || !workspace) return PA_ERR_NULL;
+  if (!p || !p->w1 || !p->b1 || !p->w2 || !u || !dy || !x || !ln_gamma || !grads || !workspace) return PA_ERR_NULL;
   if (!aligned16(p->w1) || !aligned16(p->w2) || !aligned16(u) || !aligned16(dy) || !aligned16(x) || !aligned16(dx) ||
       !aligned16(grads) || !aligned16(workspace))
     return PA_ERR_ALIGN;
   if (workspace_bytes < need) return PA_ERR_WORKSPACE;
-  const NormMlpPlan w = norm_mlp_plan(rows, C, F);
+  const NormMlpPlan w = norm_mlp_plan(rows, C, F, wanted);
   char *ws = static_cast<char *>(workspace);
   void *act = ws + w.act, *dh = ws + w.dh;
   hipStream_t st = static_cast<hipStream_t>(stream);
@@ -1284,12 +1288,27 @@ int pa_norm_mlp_backward(int dtype, int64_t rows, int64_t C, int64_t F, const pa
   pa::wgrad::Sums sums;
   int rc = pa::mlp::hidden_backward(rows, C, F, p->w1, p->b1, p->w2, u, dy, act, dh, ws + w.blob, ws + w.w1_t, cus, st);
   if (rc) return rc;
-  if ((rc = pa::norm::rows_ln_backward(rows, F, dh, ws + w.w1_t, x, ln_gamma, ln_eps, dy, dx,
-                                       reinterpret_cast<float *>(ws + w.partials), d_ln, cus, st, sums)))
+  if (dx && (rc = pa::norm::rows_ln_backward(rows, F, dh, ws + w.w1_t, x, ln_gamma, ln_eps, dy, dx,
+                                             reinterpret_cast<float *>(ws + w.partials), d_ln, cus, st, sums)))
     return rc;
-  if ((rc = pa::wgrad::product(PA_BF16, rows, dh, F, F, u, C, C, nullptr, ws + w.work_w1, d_w1, d_b1, cus, st, &sums))) return rc;
-  if ((rc = pa::wgrad::product(PA_BF16, rows, dy, C, C, act, F, F, nullptr, ws + w.work_w2, d_w2, d_b2, cus, st, &sums))) return rc;
-  return pa::wgrad::launch_sums(sums, st);
+  if (wanted & PA_GRAD_LINEAR1 &&
+      (rc = pa::wgrad::product(PA_BF16, rows, dh, F, F, u, C, C, nullptr, ws + w.work_w1, d_w1, d_b1, cus, st, &sums)))
+    return rc;
+  if (wanted & PA_GRAD_LINEAR2 &&
+      (rc = pa::wgrad::product(PA_BF16, rows, dy, C, C, act, F, F, nullptr, ws + w.work_w2, d_w2, d_b2, cus, st, &sums)))
+    return rc;
+  return sums.count > 0 ? pa::wgrad::launch_sums(sums, st) : PA_OK;
+}
+
+int pa_norm_mlp_backward(int dtype, int64_t rows, int64_t C, int64_t F, const pa_mlp_params *p, const void *u, const void *dy,
+                         const void *x, const float *ln_gamma, float ln_eps, void *dx, float *grads, void *workspace,
+                         int64_t workspace_bytes, void *stream) {
+  if (!dx) {
+    const int64_t need = pa_norm_mlp_backward_workspace_bytes(dtype, rows, C, F);
+    return need < 0 ? (int)need : PA_ERR_NULL;
+  }
+  return pa_norm_mlp_backward_wanted(dtype, rows, C, F, PA_GRAD_LINEAR1 | PA_GRAD_LINEAR2, p, u, dy, x, ln_gamma, ln_eps, dx, grads,
+                                     workspace, workspace_bytes, stream);
 }
 
 int pa_mlp_input_ln_query(int dtype, int64_t rows, int64_t C, int64_t F) {

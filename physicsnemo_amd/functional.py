@@ -504,26 +504,30 @@ def norm_mlp_backward_supported(dtype: torch.dtype, rows: int, C: int, F: int) -
     return _lib.load().pa_norm_mlp_backward_workspace_bytes(_lib.PA_BF16, rows, C, F) > 0
 
 
-def norm_mlp_backward(u, dy, x, w1, b1, w2, ln_weight, ln_eps=1e-5):
+def norm_mlp_backward(u, dy, x, w1, b1, w2, ln_weight, ln_eps=1e-5, linear1=True, linear2=True, through_norm=True):
     """Backward of y = x + w2 . gelu(w1 . u + b1) + b2, u = LayerNorm(x): (dx, d w1, d b1, d w2, d b2, d ln_weight, d ln_bias),
-    the parameters' gradients float32.  u, dy, x (..., C), w1 (F, C), w2 (C, F) bfloat16; b1, ln_weight float32."""
+    the parameters' gradients float32.  u, dy, x (..., C), w1 (F, C), w2 (C, F) bfloat16; b1, ln_weight float32.  `linear1`,
+    `linear2`, `through_norm` (dx and the LayerNorm's): what is not asked for is not formed and comes back as None."""
     _need_cuda(u, dy, x, w1, b1, w2, ln_weight)
     lib = _lib.load()
     C, F = w1.shape[1], w1.shape[0]
     rows = u.numel() // C
-    nbytes = lib.pa_norm_mlp_backward_workspace_bytes(_lib.PA_BF16, rows, C, F)
+    wanted = (_lib.PA_GRAD_LINEAR1 if linear1 else 0) | (_lib.PA_GRAD_LINEAR2 if linear2 else 0)
+    nbytes = lib.pa_norm_mlp_backward_wanted_workspace_bytes(_lib.PA_BF16, rows, C, F, wanted)
     if nbytes < 0:
-        _lib.check(int(nbytes), "pa_norm_mlp_backward_workspace_bytes")
+        _lib.check(int(nbytes), "pa_norm_mlp_backward_wanted_workspace_bytes")
     workspace = torch.empty(nbytes, dtype=torch.uint8, device=u.device)
     grads = torch.empty(2 * F * C + F + 3 * C, dtype=torch.float32, device=u.device)
-    dx = torch.empty_like(x)
+    dx = torch.empty_like(x) if through_norm else None
     params = _lib.PaMlpParams(w1.data_ptr(), b1.data_ptr(), w2.data_ptr(), None)
-    _lib.check(lib.pa_norm_mlp_backward(_lib.PA_BF16, rows, C, F, byref(params), u.data_ptr(), dy.data_ptr(), x.data_ptr(),
-                                        ln_weight.data_ptr(), float(ln_eps), dx.data_ptr(), grads.data_ptr(),
-                                        workspace.data_ptr(), nbytes, _lib.current_stream_ptr(u.device)),
-               "pa_norm_mlp_backward")
+    _lib.check(lib.pa_norm_mlp_backward_wanted(_lib.PA_BF16, rows, C, F, wanted, byref(params), u.data_ptr(), dy.data_ptr(),
+                                               x.data_ptr(), ln_weight.data_ptr(), float(ln_eps), _lib.ptr(dx), grads.data_ptr(),
+                                               workspace.data_ptr(), nbytes, _lib.current_stream_ptr(u.device)),
+               "pa_norm_mlp_backward_wanted")
     d_w1, d_b1, d_w2, d_b2, d_g, d_b = grads.split([F * C, F, C * F, C, C, C])
-    return dx, d_w1.view(F, C), d_b1, d_w2.view(C, F), d_b2, d_g, d_b
+    first = (d_w1.view(F, C), d_b1) if linear1 else (None, None)
+    second = (d_w2.view(C, F), d_b2) if linear2 else (None, None)
+    return (dx, *first, *second, *((d_g, d_b) if through_norm else (None, None)))
 
 
 class MfmaStages:

@@ -1209,3 +1209,44 @@ def test_point_stage_with_its_products_against_the_stages(B, N, C, S):
     assert_rel_l2(hip.in_project_slice.weight.grad, d_ws.view(S, 32), "d W_slice", tol=4e-3)
     assert_rel_l2(hip.in_project_slice.bias.grad, d_bs, "d b_slice", tol=2e-2)
     assert_rel_l2(hip.temperature.grad.reshape(-1), d_temp.reshape(-1), "d temperature", tol=2e-2)
+
+
+@pytest.mark.parametrize("linear1,linear2,through_norm", [(False, False, True), (True, False, True), (False, True, False)])
+def test_frozen_parts_of_a_norm_mlp_are_not_differentiated(monkeypatch, linear1, linear2, through_norm):
+    """Gradients of frozen Linears (and, with LayerNorm and input frozen too, the way through it) are not formed: the call hands
+    back None for them and leaves their memory alone, a block's backward asks for what its parameters need, and what is formed
+    has the same bits."""
+    announce("frozen norm mlp", linear1, linear2, through_norm)
+    torch.manual_seed(3)
+    C, Fh, rows = 256, 512, 3000
+    ln = torch.nn.LayerNorm(C).cuda()
+    layers = torch.nn.Sequential(torch.nn.Linear(C, Fh), torch.nn.GELU(), torch.nn.Linear(Fh, C)).cuda()
+    x, dy = torch.randn(2, rows, C, device="cuda").bfloat16()
+    asked, call = [], PF.norm_mlp_backward
+
+    def spy(*args, **kw):
+        asked.append((args, call(*args, **kw)))
+        return asked[-1][1]
+
+    monkeypatch.setattr(PF, "norm_mlp_backward", spy)
+
+    def step(frozen):
+        for part, on in ((layers[0], linear1), (layers[2], linear2), (ln, through_norm)):
+            part.requires_grad_(on or not frozen)
+        for p in [*ln.parameters(), *layers.parameters()]:
+            p.grad = None
+        xi = x.clone().requires_grad_(through_norm or not frozen)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            normed = torch.nn.functional.layer_norm(x.float(), (C,), ln.weight, ln.bias, ln.eps).detach().bfloat16()
+            assert PA.norm_mlp_fused(xi, ln, layers)
+            y, _ = PA.norm_mlp_residual_of(xi, normed, ln, layers)
+        y.backward(dy)
+        return [xi.grad] + [p.grad for p in [*layers.parameters(), *ln.parameters()]]
+
+    every = step(False)
+    part = step(True)
+    _, formed = asked[-1]
+    on = [through_norm, linear1, linear1, linear2, linear2, through_norm, through_norm]
+    assert [t is not None for t in formed] == on
+    for a, b, wanted in zip(every, part, on):
+        assert (b is None) if not wanted else torch.equal(a, b)
