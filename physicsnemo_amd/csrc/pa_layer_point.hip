@@ -126,7 +126,7 @@ __global__ __launch_bounds__(kLayerPointWaves * 64) void layer_point_backward_ke
     bias[0][tid] = a.b_x[z * kLayerPointWaves * 32 + tid];
     bias[1][tid] = a.b_fx[z * kLayerPointWaves * 32 + tid];
   }
-  const float t_raw = a.temperature[h], inv_t = 1.f / clamp_temperature(t_raw);
+  const float inv_t = 1.f / clamp_temperature(a.temperature[h]);
   const bf16x2 ones = {(__bf16)1.f, (__bf16)1.f};
   f32x16 dws[ST];
   float csum[ST], tsum = 0.f;
@@ -152,13 +152,11 @@ __global__ __launch_bounds__(kLayerPointWaves * 64) void layer_point_backward_ke
       yr[ks % 3] = p[32 * UPR];
     }
   };
-  // Matrix instructions that stay where they are written (the builtin's sink behind all of the softmax), the weights in
-  // accumulation registers.  The compiler does not see them as such: `begin` and `finish` keep the distance that vector
-  // instructions need to a tile's first and from its last.
-  // In between their operands come from LDS and from registers that
-  // nothing writes inside the loop (in the assembly no vector instruction writes an operand within eight wait states).
-  auto multiply = [](const u32x4 &w, const u32x4 &v, f32x16 &acc) {
-    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc) : "a"(w), "v"(v));
+  // Matrix instructions that stay where they are written: the empty statement takes their result, without which they sink
+  // behind all of the softmax.  The distances that vector instructions need to them are the compiler's.
+  auto multiply = [](const u32x4 &w, const u32x4 &v, const f32x16 &onto, f32x16 &acc) {
+    acc = mma(w, v, onto);
+    asm volatile("" : "+v"(acc));
   };
   auto begin = [&](int stage) {
     xs = stages + stage * STAGE;
@@ -168,19 +166,16 @@ __global__ __launch_bounds__(kLayerPointWaves * 64) void layer_point_backward_ke
       px[r] = bias[0][d], pf[r] = bias[1][d];
     }
     static_for<2>(read);
-    asm volatile("s_nop 7" : "+v"(px), "+v"(pf));
   };
   auto product = [&](auto m_) {  // the tile's matrix instruction m
     constexpr int ks = decltype(m_)::value / 3, which = decltype(m_)::value % 3;
     if constexpr (which == 0) {
       read(std::integral_constant<int, ks + 2>{});
-      multiply(wx[ks], xr[ks % 3], px);
+      multiply(wx[ks], xr[ks % 3], px, px);
     } else if constexpr (which == 1) {
-      multiply(wf[ks], xr[ks % 3], pf);
-    } else if constexpr (ks == 0) {
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(pg) : "a"(wg[ks]), "v"(yr[ks % 3]));
+      multiply(wf[ks], xr[ks % 3], pf, pf);
     } else {
-      multiply(wg[ks], yr[ks % 3], pg);
+      multiply(wg[ks], yr[ks % 3], ks == 0 ? f32x16{} : pg, pg);
     }
   };
   // behind piece `done` of E: its share of the products `from` to `to`
@@ -197,7 +192,6 @@ __global__ __launch_bounds__(kLayerPointWaves * 64) void layer_point_backward_ke
   };
   u32x4 xm[2], fm[2], gg[2];
   auto finish = [&] {
-    asm volatile("s_nop 15\n\ts_nop 7" : "+v"(px), "+v"(pf), "+v"(pg));
     xm[0] = pack_half<0>(px), xm[1] = pack_half<1>(px);
     fm[0] = pack_half<0>(pf), fm[1] = pack_half<1>(pf);
     gg[0] = pack_half<0>(pg), gg[1] = pack_half<1>(pg);
@@ -333,6 +327,7 @@ __global__ __launch_bounds__(kLayerPointWaves * 64) void layer_point_backward_ke
     __builtin_amdgcn_raw_buffer_store_b128(s1, rows, out + 2 * HD + 16, 0, 0);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be landing in LDS when the workgroup ends
+  const float t_raw = a.temperature[h];  // read again: no register is left to keep it over the loop
 
   // one row of partial gradients per workgroup: the waves (heads) add up in order
   for (int w = 0; w < kLayerPointWaves; ++w) {

@@ -336,3 +336,14 @@ def test_gale_modules_share_the_reference_state_dict_contract():
         pn.GALE(16, heads=2, dim_head=8, slice_num=4, context_dim=5, state_mixing_mode="sum")
     with pytest.raises(RuntimeError, match="GPU"), torch.no_grad():
         pn.GALE(16, heads=2, dim_head=8, slice_num=4, context_dim=5)((torch.randn(1, 7, 16),), torch.randn(1, 2, 3, 5))
+
+
+def test_matrix_instructions_of_the_per_point_kernel_are_the_compilers():
+    """Where matrix instructions write ordinary registers (a flag of the file) none is written as assembly: the compiler then sees
+    every one and keeps the distances that reads and writes of its registers need."""
+    from physicsnemo_amd import build
+    files = [f for f, flags in build.FILE_FLAGS.items() if "-amdgpu-mfma-vgpr-form" in flags]
+    assert files
+    for name in files:
+        source = open(os.path.join(build.CSRC, name)).read()
+        assert not [s for s in re.findall(r"asm(?:\s+volatile)?\s*\((.*?)\)\s*;", source, re.S) if "mfma" in s], name
