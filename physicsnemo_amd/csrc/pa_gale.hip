@@ -191,6 +191,9 @@ __global__ __launch_bounds__(kThreads) void slice_cross_mix_mfma_kernel(
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[r] = gp.cross_v_bias[i];
       acc = rows_product(cx, gp.cross_v_weight + i * Dc, Dc, g, acc);
+#pragma unroll
+      for (int r = 0; r < 16; ++r)  // rows past the context weigh nothing, which an infinity would not survive
+        if (32 * (n - UT) + mfma::rowmap(r, g) >= Sc) acc[r] = 0.f;
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) tiles[n][q][lane] = f32x4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};

@@ -94,6 +94,31 @@ def test_cross_mix_of_32_wide_heads_against_float64(mode, S, Sc, Dc):
     assert_rel_l2(got, want, f"blend {mode}", tol=8e-6)
 
 
+@pytest.mark.parametrize("Sc", [1, 33, 64, 97])
+def test_cross_mix_of_32_wide_heads_keeps_an_infinite_value_one(Sc):
+    """A context token whose value overflows in one channel makes that channel infinite, as a sum over the tokens there are
+    does, and leaves the others as they are: what fills the last tile of tokens takes no part."""
+    announce("GALE cross mix, infinite value", Sc)
+    torch.manual_seed(Sc)
+    B, H, S, D, Dc = 1, 2, 40, 32, 16
+    hip = pn.GALE(H * D, heads=H, dim_head=D, slice_num=S, context_dim=Dc, use_te=False)
+    with torch.no_grad():
+        hip.cross_v.weight[5, 0] = 3e38
+        hip.cross_k.weight[:, 0] = 0.0
+    params = hip.gale_params(torch.device("cuda"))
+    tok, self_out, ctx = (torch.randn(*s, device="cuda") for s in ((B, H, S, D), (B, H, S, D), (B, H, Sc, Dc)))
+    ctx[..., 0] = 0.0
+    dims = PF.LayerDims(B, 100, H * D, H, D, S)
+    clean = PF.slice_cross_attention_mix(tok, self_out, ctx, params, dims)
+    ctx[:, :, -1, 0] = 10.0
+    params["cross_v_weight"][:5, 0] = 0.0
+    params["cross_v_weight"][6:, 0] = 0.0
+    got = PF.slice_cross_attention_mix(tok, self_out, ctx, params, dims)
+    assert torch.isfinite(clean).all() and torch.isposinf(got[..., 5]).all()
+    others = [e for e in range(D) if e != 5]
+    assert torch.equal(got[..., others], clean[..., others])
+
+
 @pytest.mark.parametrize("mode,S,N", [("weighted", 64, 4096), ("concat_project", 32, 5000), ("weighted", 128, 3000)])
 def test_bf16_gale_on_the_mfma_kernels(mode, S, N):
     announce("bf16 GALE MFMA", mode, S, N)
