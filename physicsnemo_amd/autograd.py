@@ -11,6 +11,7 @@ this is the same gradient, assembled from
 """
 from __future__ import annotations
 
+import functools
 import itertools
 
 import torch
@@ -207,7 +208,7 @@ def _layer_train_forward(ctx, x, uniform, dims, names, params):
     x, uniform = _aligned(x), None if uniform is None else _aligned(uniform)
     y, saved = PF.layer_train_forward(x, uniform, _train_params(names, params, x.device, x.dtype), dims)
     ctx.save_for_backward(x, uniform, saved)
-    ctx.dims, ctx.names, ctx.like = dims, names, params
+    ctx.dims, ctx.names, ctx.like = dims, names, _shapes_and_types(params)
     return y
 
 
@@ -216,16 +217,26 @@ _GRADIENT_ORDER = {names: ([names.index(n) for n in order], [order.index(n) for 
                    ((_LAYER_PARAMS, PF.TRAIN_GRADIENTS), (_PLUS_PARAMS, PF.TRAIN_GRADIENTS_PLUS))}
 
 
+def _shapes_and_types(params):
+    """What the backward pass is to know of the parameters, as they are now: by then they may have been freed, moved or cast."""
+    return tuple(p.shape for p in params), tuple(p.dtype for p in params)
+
+
+@functools.lru_cache(maxsize=64)
+def _of_shapes(shapes):  # tensors without memory, for a call that takes shapes as tensors
+    return [torch.empty(s, device="meta") for s in shapes]
+
+
 def _layer_train_backward(ctx, x, uniform, dy, saved, need):
-    """(dx, the parameters' gradients); need: which of them are wanted.  Of the parameters (`ctx.like`) only sizes and types
-    are read."""
+    """(dx, the parameters' gradients); need: which of them are wanted."""
     dx, grads = PF.layer_train_gradients(x, uniform, dy, saved, ctx.dims, ctx.needs_input_grad[0])
     to_buffer, from_buffer = _GRADIENT_ORDER[ctx.names]
-    views = torch._utils._unflatten_dense_tensors(grads, [ctx.like[k] for k in to_buffer])
+    shapes, dtypes = ctx.like
+    views = torch._utils._unflatten_dense_tensors(grads, _of_shapes(tuple(shapes[k] for k in to_buffer)))
     out = []
-    for p, k, wanted in zip(ctx.like, from_buffer, need):
+    for dtype, k, wanted in zip(dtypes, from_buffer, need):
         g = views[k] if wanted else None
-        out.append(g if g is None or p.dtype == torch.float32 else g.to(p.dtype))
+        out.append(g if g is None or dtype == torch.float32 else g.to(dtype))
     return dx, tuple(out)
 
 
@@ -294,7 +305,7 @@ class LayerResidualNormFunction(torch.autograd.Function):
         kernel_params = _train_params(_LAYER_PARAMS, params, x.device, x.dtype)
         y, saved, normed = PF.layer_train_forward(x, None, kernel_params, dims, residual, w32, _aligned(ln_b.detach().float()), eps)
         ctx.save_for_backward(x, saved, y, w32)
-        ctx.dims, ctx.names, ctx.like = dims, _LAYER_PARAMS, params
+        ctx.dims, ctx.names, ctx.like = dims, _LAYER_PARAMS, _shapes_and_types(params)
         ctx.eps, ctx.ln_dtypes = eps, (ln_w.dtype, ln_b.dtype)
         _keep_parameters(ctx, ln_w)
         return y, normed
@@ -305,7 +316,7 @@ class LayerResidualNormFunction(torch.autograd.Function):
         need = ctx.needs_input_grad
         d, dg, db = _through_norm(ctx, y, w32, d_y, d_normed)
         if d is None:
-            return (None,) * (6 + len(ctx.like))
+            return (None,) * (6 + len(_LAYER_PARAMS))
         dx, grads = _layer_train_backward(ctx, x, None, d, saved, need[6:])
         return (dx, d if need[1] else None, None, dg, db, None) + grads
 
@@ -321,7 +332,7 @@ class LayerResidualFunction(torch.autograd.Function):
         y, saved, normed = PF.layer_train_forward(x, None, kernel_params, dims, residual,
                                                   _aligned(ln_w.detach().float()), _aligned(ln_b.detach().float()), eps)
         ctx.save_for_backward(x, saved)
-        ctx.dims, ctx.names, ctx.like = dims, _LAYER_PARAMS, params
+        ctx.dims, ctx.names, ctx.like = dims, _LAYER_PARAMS, _shapes_and_types(params)
         ctx.mark_non_differentiable(normed)
         return y, normed
 
@@ -330,7 +341,7 @@ class LayerResidualFunction(torch.autograd.Function):
         x, saved = ctx.saved_tensors
         need = ctx.needs_input_grad
         if d_y is None:
-            return (None,) * (6 + len(ctx.like))
+            return (None,) * (6 + len(_LAYER_PARAMS))
         d = _aligned(d_y.to(x.dtype))
         dx, grads = _layer_train_backward(ctx, x, None, d, saved, need[6:])
         return (dx, d if need[1] else None, None, None, None, None) + grads

@@ -1250,3 +1250,31 @@ def test_frozen_parts_of_a_norm_mlp_are_not_differentiated(monkeypatch, linear1,
     assert [t is not None for t in formed] == on
     for a, b, wanted in zip(every, part, on):
         assert (b is None) if not wanted else torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_parameters_may_be_freed_between_the_passes(dtype):
+    """Sharded training frees a layer's parameters between its passes: the gradients have the shapes that the parameters had in
+    the forward pass."""
+    announce("parameters freed between the passes", dtype)
+    torch.manual_seed(0)
+    hip = pn.PhysicsAttentionIrregularMesh(128, heads=4, dim_head=32, slice_num=32, use_te=False).cuda()
+    x, dy = torch.randn(2, 1, 300, 128, device="cuda").to(dtype)
+    params = list(hip.parameters())
+
+    def grads(change):
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=dtype == torch.bfloat16):
+            y = hip(x)
+        kept = [p.data for p in params]
+        change()
+        out = torch.autograd.grad(y, params, dy)
+        for p, k in zip(params, kept):
+            p.data = k
+        return out
+
+    def free():
+        for p in params:
+            p.data = torch.empty(0, device="cuda")
+
+    for g, w, p in zip(grads(free), grads(lambda: None), params):
+        assert g.shape == p.shape and g.dtype == torch.float32 and torch.equal(g, w)
