@@ -43,7 +43,7 @@ def _parameter(module: nn.Module, name: str) -> torch.Tensor:
 
 def _identity_dropout(m: nn.Module) -> bool:
     """True where calling m returns its argument and nothing else happens."""
-    return (type(m) is nn.Dropout and not (m.training and m.p > 0) and unhooked(m) and
+    return (type(m) is nn.Dropout and "forward" not in m.__dict__ and not (m.training and m.p > 0) and unhooked(m) and
             not torch.nn.modules.module._has_any_global_hook())
 
 
@@ -302,11 +302,10 @@ class PhysicsAttentionBase(nn.Module):
 
     def forward_block_with_grad(self, x: torch.Tensor, residual: torch.Tensor, ln: nn.LayerNorm, apart: bool = False):
         """Training: (self(x) + residual, its LayerNorm) with the add and the LayerNorm in the layer's last kernel, or None
-        where that does not serve the call (other types and widths, Transolver++, dropout, hooks on this module).  apart:
-        the second without a graph, for `autograd.norm_mlp_residual_of`."""
-        hooks = (self._forward_hooks, self._forward_pre_hooks, self._backward_hooks, self._backward_pre_hooks)
-        if (type(self).forward is not PhysicsAttentionBase.forward or any(hooks) or self.plus or self.fp8_weights or
-                (self.training and self.out_dropout.p > 0) or not x.is_cuda or x.ndim != 3 or x.numel() == 0 or
+        where that does not serve the call (other types and widths, Transolver++, dropout, hooks on this module or its dropout,
+        another forward).  apart: the second without a graph, for `autograd.norm_mlp_residual_of`."""
+        if (type(self).forward is not PhysicsAttentionBase.forward or "forward" in self.__dict__ or not unhooked(self) or
+                not _identity_dropout(self._modules["out_dropout"]) or self.plus or self.fp8_weights or not x.is_cuda or x.ndim != 3 or x.numel() == 0 or
                 x.dtype != residual.dtype or x.dtype not in (torch.bfloat16, torch.float32) or self._wants_fp16(x) or
                 (x.dtype == torch.float32 and torch.is_autocast_enabled("cuda")) or x.shape != residual.shape or
                 not (ln.elementwise_affine and ln.bias is not None and tuple(ln.normalized_shape) == (self.dim,))):

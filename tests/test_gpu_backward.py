@@ -1278,3 +1278,43 @@ def test_parameters_may_be_freed_between_the_passes(dtype):
 
     for g, w, p in zip(grads(free), grads(lambda: None), params):
         assert g.shape == p.shape and g.dtype == torch.float32 and torch.equal(g, w)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_blocks_in_training_call_what_is_watched_or_replaced(dtype):
+    """A hook on a layer's dropout or on every module, a replaced forward of the dropout or of the layer: a training block calls
+    them, once per pass, and the result is that of the block without them."""
+    announce("watched dropouts", dtype)
+    torch.manual_seed(0)
+    C = 128
+    block = pn.TransolverBlock(4, C, 0.0, mlp_ratio=1, slice_num=32, use_te=False).cuda()
+    attn, drop, seen = block.Attn, block.Attn.out_dropout, []
+    x = torch.randn(2, 700, C, device="cuda").to(dtype).requires_grad_(True)
+
+    def step():
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=dtype == torch.bfloat16):
+            return block(x)
+
+    def watch(m, *_):
+        if m is attn or m is drop:
+            seen.append(m)
+
+    def replaced(m):
+        plain = type(m).forward
+        m.forward = lambda t: (seen.append(m), plain(m, t))[1]
+        return lambda: m.__dict__.pop("forward")
+
+    want = step()
+    everywhere = torch.nn.modules.module.register_module_forward_hook
+    for start, whom in ((lambda: drop.register_forward_hook(watch).remove, [drop]),
+                        (lambda: everywhere(watch).remove, [drop, attn]),
+                        (lambda: replaced(drop), [drop]), (lambda: replaced(attn), [attn])):
+        seen.clear()
+        end = start()
+        try:
+            got = step()
+        finally:
+            end()
+        assert seen == whom
+        assert_rel_l2(got, want, "block", tol=1e-6 if dtype == torch.float32 else 5e-3)  # bf16: LayerNorm from rounded rows
+        got.float().sum().backward()
