@@ -29,12 +29,12 @@ class LayerDims(NamedTuple):
     conv_tap_major: int = 0  # 1: convolution weights are laid out (c_out, k, k[, k], c_in) instead of torch's order
 
     def c(self) -> _lib.PaShape:
-        return _c_shape(self)
+        return _lib.PaShape.from_buffer_copy(_c_shape(self))
 
 
 @lru_cache(maxsize=256)
-def _c_shape(dims: LayerDims) -> _lib.PaShape:  # the library reads it only
-    return _lib.PaShape(*dims)
+def _c_shape(dims: LayerDims) -> bytes:  # callers get a struct of their own
+    return bytes(_lib.PaShape(*dims))
 
 
 _PARAM_FIELDS = [f for f, _ in _lib.PaParams._fields_]

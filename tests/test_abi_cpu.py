@@ -347,3 +347,10 @@ def test_matrix_instructions_of_the_per_point_kernel_are_the_compilers():
     for name in files:
         source = open(os.path.join(build.CSRC, name)).read()
         assert not [s for s in re.findall(r"asm(?:\s+volatile)?\s*\((.*?)\)\s*;", source, re.S) if "mfma" in s], name
+
+
+def test_shape_structs_are_their_callers_own():
+    dims = PF.LayerDims(2, 100, 256, 8, 32, 64)
+    mine = dims.c()
+    mine.N = 7
+    assert [getattr(dims.c(), f) for f, _ in _lib.PaShape._fields_] == list(dims)
