@@ -733,6 +733,9 @@ def layer_train_supported(dtype: torch.dtype, dims: LayerDims, plus: bool = Fals
     return _train_bytes(dtype, byref(dims.c()), plus, _lib.PA_TRAIN_SAVED) > 0
 
 
+_TRAIN_LARGE = ("in_project_x_weight", "in_project_fx_weight", "out_linear_weight")
+
+
 def layer_train_forward(x, uniform, params: dict, dims: LayerDims, residual=None, ln_weight=None, ln_bias=None, ln_eps=1e-5):
     """(y, saved) of a layer, with ln_weight (y + residual, saved, LayerNorm(y + residual)).  `params`: the layer's own
     parameters under the names of `pa_params` / `pa_plus_params` in torch's layout, float32; bf16 layers take the three large
@@ -740,6 +743,13 @@ def layer_train_forward(x, uniform, params: dict, dims: LayerDims, residual=None
     _need_cuda(x, uniform, residual, ln_weight, ln_bias, *params.values())
     if uniform is not None and (uniform.dtype != x.dtype or uniform.shape != (dims.B, dims.N, dims.H, dims.S)):
         raise ValueError("uniform samples must have the activation dtype and shape (B, N, H, S)")
+    large = params["out_linear_weight"].dtype
+    if large not in (x.dtype, torch.float32):
+        raise TypeError(f"{large} weights do not go with {x.dtype} activations")
+    for name, p in params.items():
+        wanted = large if name in _TRAIN_LARGE else torch.float32
+        if p.dtype != wanted:
+            raise TypeError(f"{name}: {p.dtype}, expected {wanted}")
     lib, shape, plus = _lib.load(), byref(dims.c()), uniform is not None
     nbytes = _train_bytes(x.dtype, shape, plus, _lib.PA_TRAIN_FORWARD)
     if nbytes < 0:

@@ -1318,3 +1318,19 @@ def test_blocks_in_training_call_what_is_watched_or_replaced(dtype):
         assert seen == whom
         assert_rel_l2(got, want, "block", tol=1e-6 if dtype == torch.float32 else 5e-3)  # bf16: LayerNorm from rounded rows
         got.float().sum().backward()
+
+
+def test_training_call_refuses_parameters_of_another_type():
+    """The library reads the parameters by the type that goes with the activations: 16-bit ones for float32 activations (half the
+    memory it would read), a 16-bit bias, weights of two types are errors."""
+    announce("training call, parameter types")
+    hip = pn.PhysicsAttentionIrregularMesh(64, heads=2, dim_head=32, slice_num=32, use_te=False).cuda()
+    x = torch.randn(1, 100, 64, device="cuda")
+    dims, names = hip.layer_dims(x), dict(hip.named_parameters())
+    params = {n: names[n.replace("_weight", ".weight").replace("_bias", ".bias")].detach() for n in PA._LAYER_PARAMS}
+    assert torch.isfinite(PF.layer_train_forward(x, None, params, dims)[0]).all()
+    halves = {n: p.bfloat16() if n in PA._LARGE else p for n, p in params.items()}
+    for wrong in (halves, {**params, "out_linear_bias": params["out_linear_bias"].bfloat16()},
+                  {**params, "in_project_x_weight": params["in_project_x_weight"].bfloat16()}):
+        with pytest.raises(TypeError):
+            PF.layer_train_forward(x, None, wrong, dims)
