@@ -641,19 +641,21 @@ __global__ __launch_bounds__(kAttnThreads) void slice_combine_attn_kernel(const 
 }
 
 // ------------------------------------------------------------------------------------------------
-// narrow_combine_attn_kernel<D, S>: combine_partials_kernel and slice_combine_attn_kernel in one launch for narrow heads, with
+// narrow_combine_attn_kernel<D>: combine_partials_kernel and slice_combine_attn_kernel in one launch for narrow heads, with
 // their sums in their order, bit for bit: 32 threads per slice, everything of a (b, h) in registers and LDS, sizes known to
 // the compiler.  Bound by latency: one trip for partials and weights, four barriers.  D = 16, S = 32 (us, the two launches before ->
 // now): 16 workgroups of 128 partials 4.5 + 11.0 -> 9.4, 32 of 64 partials 4.8 + 10.6 -> 7.0.
 // ------------------------------------------------------------------------------------------------
-template <int D, int S>
-__global__ __launch_bounds__(32 * S) void narrow_combine_attn_kernel(const float *__restrict__ partials, int G,
+constexpr int kNarrowSlices = 32;
+
+template <int D>
+__global__ __launch_bounds__(32 * kNarrowSlices) void narrow_combine_attn_kernel(const float *__restrict__ partials, int G,
                                                                     int64_t partial_stride, const float *__restrict__ w_qkv,
                                                                     float *__restrict__ slice_token,
                                                                     float *__restrict__ slice_norm,
                                                                     float *__restrict__ out_token) {
-  constexpr int T = 32 * S, D1 = D + 1, LD = D + 4, NOUT = S * D1, kAhead = 16, KEYS = S / 16;
-  static_assert((S == 16 || S == 32 || S == 64) && D % 4 == 0, "16 threads per slice in the softmax, whole float4 rows");
+  constexpr int S = kNarrowSlices, T = 32 * S, D1 = D + 1, LD = D + 4, NOUT = S * D1, kAhead = 16;
+  static_assert(S == 2 * 16 && D % 4 == 0, "16 threads per slice in the softmax, two keys each; whole float4 rows");
   __shared__ float quarter[4][NOUT];
   __shared__ __align__(16) float tok[S * LD], wq[3 * D * LD], qkv[3][S * LD], prob[S * (S + 1)];
   const int t = threadIdx.x, bh = blockIdx.x;
@@ -704,15 +706,15 @@ __global__ __launch_bounds__(32 * S) void narrow_combine_attn_kernel(const float
     qkv[e / D][s * LD + e % D] = dot(tok + s * LD, wq + e * LD);
   }
   __syncthreads();
-  // The first half of the workgroup: slice s = t / 16, keys t % 16 + 16 j.  A sum over a slice's keys pairs them as a sum over the
+  // The first half of the workgroup: slice s = t / 16, keys t % 16 and t % 16 + 16.  A sum over a slice's keys pairs them as a sum over the
   // 64 lanes of a wave does.
   const int s = t >> 4, l = t & 15;
   float inv = 0.f;
   if (s < S) {
     const float scale = rsqrtf((float)D);
-    float e[KEYS], mx = -INFINITY, sum;
+    float e[2], mx = -INFINITY;
 #pragma unroll
-    for (int j = 0; j < KEYS; ++j) {
+    for (int j = 0; j < 2; ++j) {
       e[j] = dot(qkv[0] + s * LD, qkv[1] + (l + 16 * j) * LD) * scale;
       asm("" : "+v"(e[j]));  // rounded, as the kernel that stores it has it: no fused multiply-subtract below
       mx = fmaxf(mx, e[j]);
@@ -720,13 +722,11 @@ __global__ __launch_bounds__(32 * S) void narrow_combine_attn_kernel(const float
 #pragma unroll
     for (int off = 8; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
 #pragma unroll
-    for (int j = 0; j < KEYS; ++j) {
+    for (int j = 0; j < 2; ++j) {
       e[j] = expf(e[j] - mx);
       prob[s * (S + 1) + l + 16 * j] = e[j];
     }
-    if constexpr (KEYS == 4) sum = (e[0] + e[2]) + (e[1] + e[3]);
-    else if constexpr (KEYS == 2) sum = e[0] + e[1];
-    else sum = e[0];
+    float sum = e[0] + e[1];
 #pragma unroll
     for (int off = 8; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
     inv = 1.f / sum;
@@ -1405,14 +1405,14 @@ constexpr int64_t kFewPartials = 256;
 template <int D>
 static int narrow_combine_attention(const pa_shape &s, const pa_params &p, const float *partials, int64_t G, float *slice_token,
                                     float *slice_norm, float *out_token, hipStream_t st) {
-  hipLaunchKernelGGL((narrow_combine_attn_kernel<D, 32>), dim3((unsigned)(s.B * s.H)), dim3(32 * 32), 0, st, partials, (int)G,
+  hipLaunchKernelGGL(narrow_combine_attn_kernel<D>, dim3((unsigned)(s.B * s.H)), dim3(32 * kNarrowSlices), 0, st, partials, (int)G,
                      s.B * s.H * s.S * (s.D + 1), p.qkv_project_weight, slice_token, slice_norm, out_token);
   return launch_status();
 }
 
 int combine_attention(const pa_shape &s, const pa_params &p, const float *partials, int64_t G, float *slice_token,
                       float *slice_norm, float *out_token, hipStream_t st) {
-  if (s.S == 32 && out_token && G > 8 && G <= kFewPartials) {
+  if (s.S == kNarrowSlices && out_token && G > 8 && G <= kFewPartials) {
     if (s.D == 8) return narrow_combine_attention<8>(s, p, partials, G, slice_token, slice_norm, out_token, st);
     if (s.D == 16) return narrow_combine_attention<16>(s, p, partials, G, slice_token, slice_norm, out_token, st);
   }

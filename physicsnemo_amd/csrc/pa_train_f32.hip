@@ -97,7 +97,7 @@ struct Saved {  // kept from the forward to the backward pass
 };
 struct Scratch {
   int64_t w_in, partials, total;                                                                                    // forward
-  int64_t g, sums, d_tok, d_num, d_norm, attn, parts, d_proj, d_z, d_t, t_sum, heads, work[3], total_backward;
+  int64_t g, d_tok, d_num, d_norm, attn, parts, d_proj, d_z, d_t, t_sum, heads, work[3], total_backward;
   bool served;  // by the row-axis products
 };
 struct Taker {
