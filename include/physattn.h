@@ -555,7 +555,7 @@ int pa_mlp_backward(int dtype, int64_t rows, int64_t C, int64_t F, const pa_mlp_
 /* The whole backward pass of y = x + Mlp(LayerNorm(x)) (TR.py:303) from dy, x and u = LayerNorm(x), the hidden layer and the
  * product with w1 formed on the way, the LayerNorm's backward and the residual's gradient in that product's kernel:
  *   dx (rows, C) bf16;  grads, float32, one behind the other: d w1 (F, C), d b1 (F), d w2 (C, F), d b2 (C), d gamma (C), d beta (C).
- * Types and alignment as pa_mlp_backward; ln_gamma float32; grads 16-byte aligned; F a multiple of 256.  dx may not alias an input. */
+ * Types and alignment as pa_mlp_backward; ln_gamma float32; grads 16-byte aligned; F a multiple of 64 up to 8 192.  dx may not alias an input. */
 int64_t pa_norm_mlp_backward_workspace_bytes(int dtype, int64_t rows, int64_t C, int64_t F);
 int pa_norm_mlp_backward(int dtype, int64_t rows, int64_t C, int64_t F, const pa_mlp_params *p, const void *u, const void *dy,
                          const void *x, const float *ln_gamma, float ln_eps, void *dx, float *grads, void *workspace,

@@ -1885,10 +1885,15 @@ template <int C>
 static size_t split_lds(int F) {
   return (size_t)rows::SplitCfg<C>::BYTES + (size_t)(F + 5 * C) * 4;
 }
-// Rounds of the split kernel (64 rows per CU) that are shorter than one of the owning kernel's.  C = 256, F = 1024 (us): the
-// split kernel 22 - 29 / 48 - 53 for one / two rounds, about 78 for three; the owning kernel 57 - 67 for up to 32 768 rows, 73 for
-// 49 152.  C = 512, F = 2048: 50 - 74 / 122 - 150 against 120 - 129 / 131 - 157, where a second launch's start eats the difference
-// of two rounds (49 512 rows, a model of 7 blocks: 3 763 against 3 703).  F = 128 .. 512 alike.
+// Rounds of the split kernel (64 rows per CU) that are shorter than one of the owning kernel's (us, owning kernel alone -> with the
+// split kernel for the rest, the median of five blocks of launches).
+// C = 256, F = 1024, all rows: 4 000 55 -> 21, 16 384 56 -> 25, 16 960 56 -> 42, 32 768 61 -> 47; three rounds would be 64 -> 63.
+// Behind 1 / 2 / 4 whole rounds: 4 000 rows 130 -> 106, 205 -> 180, 344 -> 318; 16 960 132 -> 128, 205 -> 200, 346 -> 340; 24 576 133 ->
+// 130, 207 -> 203, 347 -> 344; 32 768 135 -> 134, 210 -> 207, 352 -> 351; behind 15, where launches scatter by 10, 1 151 -> 1 129 for
+// 16 384, 1 151 -> 1 146 for 16 960, 1 158 -> 1 155 for 32 768.  In training 152 -> 117 for 4 000 behind one round, 153 -> 141 for
+// 16 960, 155 -> 146 for 32 768.  F = 512: 81 -> 69, 86 -> 85, 89 -> 88; F = 256: 57 -> 51, 62 -> 61, 65 -> 64.
+// C = 512, F = 2048, one round: 8 192 rows 123 -> 56, 16 384 127 -> 75, behind four 681 -> 629, 684 -> 649.  A second one: 32 767 rows alone
+// 131 -> 150, 49 512 rows of a model of 7 blocks 3 703 -> 3 763.
 template <int C>
 constexpr int64_t kSplitRounds = C == 256 ? 2 : 1;
 

@@ -34,7 +34,7 @@ struct Args {
 // of W^T (rows of 64 bytes) form a ring of three stages in LDS, filled two steps ahead by direct global -> LDS loads, one
 // barrier per step.  Position p of row r holds the row's 16-byte unit p ^ (r / 4 % 4): the lanes of an access phase fall on all
 // banks.  g leaves the accumulators through LDS in bf16; half a wave then finishes a row as layernorm_backward_rows_kernel does.
-// Bound by the reach of the ring (24 KB a step and workgroup, W^T two thirds of it) at K = 1 024, by HBM below (2 K + 2 048 bytes
+// Bound by the reach of the ring (24 KB a step and workgroup, W^T two thirds of it) at K = 1 024, by HBM below (2 K + 1 536 bytes
 // per row).  262 144 rows (us), the product and layernorm_backward_rows_kernel -> this: K = 1 024 149 + 99 -> 231, K = 512 96 +
 // 102 -> 149 (the best of 15 launches each), K = 256 94 less in all.  dh as register operands straight from memory instead: 280 at
 // K = 1 024, its 16-byte pieces of rows coming from L2 four times.

@@ -98,7 +98,7 @@ static HandBack hand_back(const pa_shape &s, bool plus) {
 
 static bool fused(const pa_shape &s, bool plus) { return !plus && mfma::supported(PA_BF16, s); }
 
-// The projections, d out_x and the per-point stage of the backward pass in one kernel.  Its workgroups, one per CU, read 3 C / 2
+// The projections, d out_x and the per-point stage of the backward pass in one kernel.  Its workgroups, one per CU, read 3 C / 4
 // KB of weights before their first tile.  Many batch elements of one tile each do not pay that back: 2 048 clouds of 16
 // points, C = 256, S = 64, 7 180 us against 7 000 for the whole step; 512 of 64 points 1 250 both ways.  Nor do, at C = 128
 // where the stages move half as much, fewer than four tiles per CU: the kernels of a step at S = 32 take 165 us against 149

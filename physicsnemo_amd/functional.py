@@ -498,7 +498,7 @@ def mlp_backward(u, dy, w1, b1, w2):
 
 
 def norm_mlp_backward_supported(dtype: torch.dtype, rows: int, C: int, F: int) -> bool:
-    """True if `norm_mlp_backward` serves this shape (bfloat16, C = 256, F a multiple of 256)."""
+    """True if `norm_mlp_backward` serves this shape (bfloat16, C = 256, F a multiple of 64 as `mlp_supported` takes it)."""
     if dtype != torch.bfloat16 or rows <= 0 or not mlp_supported(dtype, rows, C, F):
         return False
     return _lib.load().pa_norm_mlp_backward_workspace_bytes(_lib.PA_BF16, rows, C, F) > 0
