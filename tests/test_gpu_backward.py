@@ -1334,3 +1334,69 @@ def test_training_call_refuses_parameters_of_another_type():
                   {**params, "in_project_x_weight": params["in_project_x_weight"].bfloat16()}):
         with pytest.raises(TypeError):
             PF.layer_train_forward(x, None, wrong, dims)
+
+
+@pytest.mark.parametrize("next_norm", [False, True])
+def test_norm_mlp_block_differentiates_twice(next_norm):
+    """x + Mlp(LayerNorm(x)) in one function, as model blocks of 256 channels train, LayerNorm(x) given without a graph: gradients
+    of a function of its gradient, by x and every parameter of the LayerNorm before, the Linears and the LayerNorm behind,
+    against float64.  A parameter of any of them that changed between the passes is refused there and only there."""
+    announce("norm mlp twice", next_norm)
+    torch.manual_seed(1)
+    rows, C, Fh = 300, 256, 128
+    ln, after = torch.nn.LayerNorm(C, eps=1e-3).cuda(), torch.nn.LayerNorm(C).cuda()
+    layers = torch.nn.Sequential(torch.nn.Linear(C, Fh), torch.nn.GELU(), torch.nn.Linear(Fh, C)).cuda()
+    modules = [ln, layers] + ([after] if next_norm else [])
+    with torch.no_grad():
+        for m in modules:
+            for p in m.parameters():
+                p.copy_((p + 0.1 * torch.randn_like(p)).bfloat16().float())
+    x, dy, dn = (torch.randn(rows, C, device="cuda").bfloat16() for _ in range(3))
+
+    def second(mods, x, call):
+        x = x.detach().requires_grad_(True)
+        params = [p for m in mods for p in m.parameters()]
+        grads = torch.autograd.grad(call(x), [x, *params], create_graph=True)
+        return torch.autograd.grad(sum(g.to(x.dtype).float().square().sum() if x.dtype != torch.float64 else g.square().sum()
+                                       for g in grads), [x, *params], allow_unused=True)
+
+    def fused(x):
+        assert PA.norm_mlp_fused(x, ln, layers)
+        normed = F.layer_norm(x.detach().float(), (C,), ln.weight.detach().float(), ln.bias.detach().float(), ln.eps).bfloat16()
+        y, n = PA.norm_mlp_residual_of(x, normed, ln, layers, after if next_norm else None)
+        assert (n is not None) == next_norm
+        return (y * dy).sum() + ((n * dn).sum() if next_norm else 0)
+
+    mods64 = [copy.deepcopy(m).double() for m in modules]
+
+    def plain(x):
+        y = x + mods64[1](mods64[0](x))
+        return (y * dy.double()).sum() + ((mods64[2](y) * dn.double()).sum() if next_norm else 0)
+
+    want = second(mods64, x.double(), plain)
+    names = ["x"] + [f"{k}.{n}" for k, m in enumerate(modules) for n, _ in m.named_parameters()]
+    for dtype in (torch.float32, torch.bfloat16):
+        for m in modules:
+            m.to(dtype)
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=dtype == torch.float32):
+            got = second(modules, x, fused)
+        for name, g, w in zip(names, got, want):
+            if w is None or w.norm() == 0:  # a sum that does not depend on the last bias
+                assert g is None or g.float().norm() <= 1e-6 * want[1].norm()
+                continue
+            # four passes through the block with some ten bf16 roundings each (1.1e-3 of a value) of terms that cancel by a few
+            assert_rel_l2(g, w, name + " " + str(dtype), tol=4e-2)
+    for m in modules:  # float32 parameters: what the plain backward reads of them are copies in bf16
+        m.float()
+    every = [x.detach().requires_grad_(True), *(p for m in modules for p in m.parameters())]
+    for changed in (ln.weight, ln.bias, layers[0].weight, layers[0].bias, layers[2].weight, *([after.weight] if next_norm else [])):
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            out = fused(every[0])
+        first = torch.autograd.grad(out, every, retain_graph=True)
+        with torch.no_grad():
+            changed.add_(0.5)
+        if changed is not after.weight:
+            for g, w in zip(torch.autograd.grad(out, every, retain_graph=True), first):
+                assert torch.equal(g, w)
+        with pytest.raises(RuntimeError, match="modified"):
+            torch.autograd.grad(out, every, create_graph=True)
