@@ -1400,3 +1400,83 @@ def test_norm_mlp_block_differentiates_twice(next_norm):
                 assert torch.equal(g, w)
         with pytest.raises(RuntimeError, match="modified"):
             torch.autograd.grad(out, every, create_graph=True)
+
+
+def _oracle64_gradients(hip, kind, dim, heads, dim_head, S, x, dy, spatial=None, kernel=3):
+    """x's gradient and the parameters' by autograd over the float64 oracle with the layer's parameters."""
+    if kind == "irregular":
+        ref = to.OraclePhysicsAttentionIrregularMesh(dim, heads=heads, dim_head=dim_head, slice_num=S)
+    else:
+        cls = to.OraclePhysicsAttentionStructuredMesh2D if kind == "structured2d" else to.OraclePhysicsAttentionStructuredMesh3D
+        ref = cls(dim, spatial, heads=heads, dim_head=dim_head, slice_num=S, kernel=kernel)
+    ref = ref.to(x.device).double()
+    ref.load_state_dict({k: v.double() for k, v in hip.state_dict().items()})
+    xd = x.detach().double().requires_grad_(True)
+    ref(xd).backward(dy.double())
+    return {"x": xd.grad, **{n: p.grad for n, p in ref.named_parameters()}}
+
+
+@pytest.mark.parametrize("B,N,C,S", [(2, 3001, 256, 64), (1, 9000, 256, 32), (3, 700, 256, 16), (1, 33_000, 128, 64), (2, 17_000, 128, 16)])
+def test_point_stage_with_its_products_is_as_close_to_float64_as_the_stages(B, N, C, S):
+    """The irregular layer's gradients in bf16 against float64: the kernel that forms x_mid, fx_mid and d out_x itself rounds to
+    bf16 what the stages with these in memory round, so that its errors are theirs but for single roundings that fall the other
+    way (one in a few thousand values, whose float32 sums differ in their last bits): less than 2 % apart over four seeds."""
+    announce("point stage with products against float64", B, N, C, S)
+    H = C // 32
+    names = ["x", "in_project_x.weight", "in_project_x.bias", "in_project_fx.weight", "in_project_fx.bias", "in_project_slice.weight",
+             "in_project_slice.bias", "temperature"]
+    square = {n: [0.0, 0.0] for n in names}
+    for seed in range(4):
+        _, hip = make_pair("irregular", C, H, 32, S, seed=seed, temps=[0.3 + 0.4 * k for k in range(H)])
+        hip.train()
+        x, dy = torch.randn(2, B, N, C, device="cuda").bfloat16()
+        want = _oracle64_gradients(hip, "irregular", C, H, 32, S, x, dy)
+        xr = x.clone().requires_grad_(True)
+        hip.zero_grad(set_to_none=True)
+        hip(xr).backward(dy)
+        one = {"x": xr.grad, **{n: p.grad for n, p in hip.named_parameters()}}
+
+        dims, kp = hip.layer_dims(x), hip.kernel_params(torch.bfloat16, x.device)
+        st = PF.MfmaStages(kp, dims, x.device)
+        st.pack_params()
+        st.project_softmax(x)
+        st.slice_reduce()
+        st.combine_attention()
+        linear = PF.LayerDims(B, N, C, H, 32, S)
+        x_mid, fx_mid = PF.project_inputs(x, kp, dims)
+        g = PF.rows_gemm(dy, kp["out_linear_weight"].view(C, C).t().contiguous(), None, linear, C, C)
+        d_tok, _, _ = PF.output_backward(st.w_pack, dy, st.tok_out, kp["out_linear_weight"], dims)
+        d_num, d_norm, _ = PF.slice_attention_backward(st.tok, st.norm, d_tok, kp, dims)
+        d_proj, d_ws, d_bs, d_t = PF.point_backward(x_mid, fx_mid, g, st.tok_out, d_num, d_norm, kp, dims)
+        w_t = torch.cat([kp["in_project_x_weight"].view(C, C).t(), kp["in_project_fx_weight"].view(C, C).t()], dim=1).contiguous()
+        d_w, d_b = PF.cols_gemm(d_proj, x, col_sums=True)
+        apart = [PF.rows_gemm(d_proj, w_t, None, linear, 2 * C, C), d_w[:C], d_b[:C], d_w[C:], d_b[C:], d_ws, d_bs, d_t]
+        for n, a in zip(names, apart):
+            w = want[n].reshape(-1)
+            for k, got in enumerate((one[n], a)):
+                square[n][k] += ((got.double().reshape(-1) - w).norm() / w.norm()).item() ** 2
+    for n, (one, apart) in square.items():
+        assert one <= 1.02 ** 2 * apart, (n, (one / 4) ** 0.5, (apart / 4) ** 0.5)
+
+
+@pytest.mark.parametrize("kind,dim,heads,dim_head,S,grid,kernel,N", [
+    ("irregular", 64, 2, 16, 32, None, 0, 1), ("irregular", 36, 3, 20, 8, None, 0, 333), ("irregular", 128, 8, 16, 64, None, 0, 2500),
+    ("structured2d", 128, 8, 16, 32, (13, 11), 3, 143), ("structured2d", 32, 4, 8, 16, (9, 14), 5, 126),
+    ("structured3d", 64, 4, 16, 32, (5, 6, 7), 3, 210),
+])
+def test_fp32_layer_in_two_calls_against_float64(kind, dim, heads, dim_head, S, grid, kernel, N):
+    """Every gradient of a float32 layer's training step against float64: up to 1.5e-6 was seen for these shapes, 4.1e-6 for d
+    temperature, whose terms cancel most; four times that."""
+    announce("fp32 train calls against float64", kind, dim, heads, dim_head, S, grid)
+    temps = [0.2 + 5.6 * i / (heads - 1) for i in range(heads)]
+    kw = {} if grid is None else dict(spatial=grid, kernel=kernel)
+    _, hip = make_pair(kind, dim, heads, dim_head, S, sharpen=2.0, temps=temps, **kw)
+    hip.train()
+    x, dy = torch.randn(2, 2, N, dim, device="cuda")
+    assert PF.layer_train_supported(torch.float32, hip.layer_dims(x))
+    want = _oracle64_gradients(hip, kind, dim, heads, dim_head, S, x, dy, **kw)
+    xr = x.clone().requires_grad_(True)
+    hip(xr).backward(dy)
+    for n, got in [("x", xr.grad)] + [(n, p.grad) for n, p in hip.named_parameters()]:
+        err = (got.double() - want[n]).norm() / want[n].norm().clamp(min=1e-30)
+        assert err <= (1.7e-5 if n == "temperature" else 6e-6), (n, err.item())
