@@ -20,7 +20,7 @@ namespace mfma {
 // stores: with one wave per SIMD nothing else would fill the matrix cores meanwhile.  A lane's rows of the weights are
 // taken in the order (bits 2 and 3 of i exchanged) in which the accumulator is an operand with natural channels, what
 // point_backward_kernel loads.  At C = 256 two workgroups share a tile's rows; they are neighbours on one XCD, where the
-// second finds them in L2 (fetched from memory: 0.54 GB of the 1.07 that a million points hold).
+// second finds them in L2 (fetched from memory: 1.08 GB where a million points hold 1.07).
 // Bound by its matrix and vector work (2 500 cycles of each per tile and wave; 5 300 pass, at the 1.5 GHz that the card
 // keeps up under it): 1 048 576 points, C = 256, S = 64: 0.89 ms, in which 4 C bytes per point are read and 4 C written;
 // the products and point_backward_kernel apart took 1.36 ms.  262 144 points in eight
