@@ -891,7 +891,9 @@ int64_t pa_point_backward_grads(const pa_shape *shape, int plus) {
 
 int64_t pa_point_backward_workspace_bytes(const pa_shape *shape, int plus) {
   const int rc = check_point_backward(shape);
-  return rc ? rc : pa::mfma::point_backward_workspace_bytes(*shape, plus != 0, compute_units());
+  if (rc) return rc;
+  return pa::mfma::point_backward_workspace_bytes(*shape, plus != 0, compute_units()) +
+         (plus ? pa::mfma::temperature_hidden_bytes(*shape) : 0);
 }
 
 static bool plus_complete(const pa_plus_params *q) {
@@ -1846,7 +1848,7 @@ int pa_layer_forward_plus(int dtype, const pa_shape *shape, const pa_params *p, 
   a.pack_heads = (int)s.H;
   if (!pa::gemm::serves(a, 1, 2)) return PA_ERR_UNSUPPORTED;
   if ((rc = pa::gemm::launch(a, 1, PA_BF16, st))) return rc;
-  if ((rc = pa::mfma::slice_softmax_pack_plus(s, *p, *plus, x_mid, uniform, wp, false, compute_units(), st))) return rc;
+  if ((rc = pa::mfma::slice_softmax_pack_plus(s, *p, *plus, x_mid, uniform, wp, false, nullptr, compute_units(), st))) return rc;
   if ((rc = pa::mfma::slice_reduce(s, wp, fxp, partials, st))) return rc;
   if ((rc = pa::mfma::combine_attention(s, *p, nullptr, partials, sp.G, tok, norm, tok_out, tokp, st))) return rc;
   if (pa::mfma::supported(dtype, s) && p->out_linear_bias) {

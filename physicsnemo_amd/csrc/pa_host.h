@@ -269,7 +269,7 @@ int ball_query_cells(int64_t B, int64_t Np, int64_t Nq, int64_t K, float radius,
 namespace mfma {
 bool staged_supported(int dtype, const pa_shape &s);
 int slice_softmax_pack_plus(const pa_shape &s, const pa_params &p, const pa_plus_params &pp, const void *x_mid,
-                            const void *uniform, void *w_pack, bool split, int num_cu, hipStream_t st);
+                            const void *uniform, void *w_pack, bool split, float *a2_out, int num_cu, hipStream_t st);
 int slice_softmax_pack(const pa_shape &s, const pa_params &p, const void *x_mid, void *w_pack, int num_cu,
                        hipStream_t st);
 // the same weights recomputed where they are used, never stored: token sums (softmax_reduce_groups partials) and
@@ -304,10 +304,13 @@ int backward_tables(const pa_shape &s, const float *w_slice, const float *pt_w1,
 bool point_backward_supported(const pa_shape &s);
 int64_t point_backward_grads(const pa_shape &s, bool plus);
 int64_t point_backward_workspace_bytes(const pa_shape &s, bool plus, int num_cu);
+// Transolver++: a2 [tile][H][32], what proj_temperature's second Linear gives; without one from the forward pass the workspace
+// ends in as many bytes to form it in
+int64_t temperature_hidden_bytes(const pa_shape &s);
 int point_backward(const pa_shape &s, const pa_params &p, const pa_plus_params *plus, const void *x_mid,
                    const void *fx_mid, const void *d_out_x, const void *uniform, const float *out_token,
                    const float *d_num, const float *d_norm, void *workspace, void *d_proj, float *grads, int num_cu,
-                   hipStream_t st, wgrad::Sums *later = nullptr);
+                   hipStream_t st, wgrad::Sums *later = nullptr, const float *a2 = nullptr);
 bool supported(int dtype, const pa_shape &s);
 int64_t tiles_per_batch(const pa_shape &s);
 int64_t reduce_groups(const pa_shape &s);

@@ -273,7 +273,7 @@ __global__ __launch_bounds__(S > 64 ? 256 : 512) void slice_softmax_backward_mfm
 //   d W_slice (S x 32) += dz^T . x_mid,  d b_slice += sum dz:  both operands turned around by an exact MFMA product with
 //       0/1 selection matrices (lanes <-> slices / channels, k = points), accumulated in registers over the whole kernel:
 //       d z itself never reaches memory.
-// PLUS (Transolver++; fx_mid is x_mid, d_proj holds the sum of both gradients): the softmax argument is
+// PLUS (Transolver++; a2 comes from the forward pass, fx_mid is x_mid, d_proj holds the sum of both gradients): the softmax argument is
 //   (z + Gumbel noise) / temp,  temp = max(temperature[h] + gelu(a2), 0.01),  a2 = b2 + sum_s w2[s] gelu(a1[s]),
 //   a1 = W1 x_mid + b1;  d temp flows back into temperature[h] and through the small MLP (d W1, d b1, d w2, d b2, d x_mid).
 // Rows beyond N repeat the batch's last row: their stores write that row's values again, their sums are masked.
@@ -281,13 +281,14 @@ __global__ __launch_bounds__(S > 64 ? 256 : 512) void slice_softmax_backward_mfm
 // and for PLUS d W1, d b1, d w2, d b2).
 // Bound by HBM, (3 + 2) 64 bytes per point and head, and behind it by the vector work of the softmax and its backward:
 // 1 048 576 points, 8 heads, S = 64: 0.74 ms = 3.7 TB/s; reading the stored weights and writing d z the same step took 1.29 ms,
-// and d W_slice another 0.3 ms behind it.  PLUS is bound by its vector work, 27 instructions to a matrix instruction and one
-// wave per SIMD: 100 003 points 0.219 ms = 1.2 TB/s, against 1.83 ms of the fma kernel on natural layouts; of these the
-// remainder of d z and d a1 takes 0.014 ms, GELU to float32 accuracy 0.010 ms.
+// and d W_slice another 0.3 ms behind it.  PLUS is bound by vector issue (1 900 instructions per tile and head, 9 500 cycles of issue
+// in 11 000 at two waves per SIMD): 100 003 points 0.148 ms.  With one wave per SIMD, the temperature's hidden layer formed once more
+// for a2 and the noise read where it is used it took 0.221 ms; 8 192 points 25 us against 74.
 // ------------------------------------------------------------------------------------------------
 struct PointArgs {
   const uint16_t *x_mid, *fx_mid, *g;  // (B, N, H*32)
   const uint16_t *uniform;             // PLUS: (B, N, H, S)
+  const float *a2;                     // PLUS: [tile][H][32]
   const u32x4 *tabs;
   const float *d_norm, *b_slice, *temperature;
   const float *pt_b1, *pt_w2, *pt_b2;  // PLUS
@@ -297,32 +298,68 @@ struct PointArgs {
   int tpb, H;
 };
 
-// heads (waves) per workgroup.  4: one wave per SIMD, 512 registers; 1, 2: what the split tables of S = 128 leave room for
+// heads per workgroup.  1, 2: what the split tables of S = 128 leave room for
 constexpr int point_waves(int S, bool plus, bool split) { return S > 64 ? (split ? (plus ? 1 : 2) : 4) : plus || (split && S == 64) ? 4 : 8; }
+
+// Waves per head, each with tiles of its own.  PLUS: 2 where the head's sums and one tile's values fit 256 registers (S = 128: the
+// sums alone take 256), so that a SIMD holds two waves; they share the head's tables in LDS, which leave no room for eight heads.
+// The plain form on float32 tables takes 30.6 us with two and 34.1 with one (2 x 16 384 points, S = 64), but the step around it
+// 3 785 us against 3 695: the convolutions behind it then run at a lower clock.
+constexpr int point_streams(int S, bool plus) { return S <= 64 && plus ? 2 : 1; }
 
 // S >= 64: the head's tok' / d num fragments stay in (dynamic) LDS, the registers are needed for z, dw and the sums
 constexpr int point_table_units(int S, bool split) { return S >= 64 ? (4 * ((S + 31) / 32) + S / 16) * 64 * (split ? 2 : 1) : 0; }
 
+// a2 alone, for callers that do not have it from a forward pass: grid (G, B, H), one wave
+template <int S>
+__global__ __launch_bounds__(64) void temperature_hidden_kernel(PointArgs a, float *__restrict__ a2_out) {
+  constexpr int ST = (S + 31) / 32, GRP = (2 * ST + S / 16) * 2;  // fragments of W1 behind those of W_slice, each with remainders
+  const int lane = threadIdx.x, i = lane & 31, g = lane >> 5, b = blockIdx.y, h = blockIdx.z, HD = a.H * 32;
+  const u32x4 *w1 = a.tabs + GRP * 64 + lane;
+  for (int t = blockIdx.x; t < a.tpb; t += gridDim.x) {
+    const int64_t n = (int64_t)t * 32 + i;
+    const uint16_t *row = a.x_mid + ((int64_t)b * a.N + (n < a.N ? n : a.N - 1)) * HD + h * 32 + 8 * g;
+    const u32x4 x0 = *reinterpret_cast<const u32x4 *>(row), x1 = *reinterpret_cast<const u32x4 *>(row + 16);
+    float a2 = 0.f;
+    for (int st = 0; st < ST; ++st) {
+      f32x16 hd;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) hd[r] = 32 * st + rowmap(r, g) < S ? a.pt_b1[32 * st + rowmap(r, g)] : 0.f;
+#pragma unroll
+      for (int lo = 0; lo < 2; ++lo) {
+        hd = mma(w1[(lo * (GRP / 2) + st * 2 + 0) * 64], x0, hd);
+        hd = mma(w1[(lo * (GRP / 2) + st * 2 + 1) * 64], x1, hd);
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (32 * st + rowmap(r, g) < S) a2 = fmaf(a.pt_w2[32 * st + rowmap(r, g)], gelu_fit(hd[r]), a2);
+    }
+    a2 = half_sum(a2) + a.pt_b2[0];
+    if (g == 0) a2_out[(((int64_t)b * a.tpb + t) * a.H + h) * 32 + i] = a2;
+  }
+}
+
+// keeps the phases of a tile apart: the scheduler's freedom to fetch operands of a later one costs registers that are not there
+#define PHASE __builtin_amdgcn_sched_barrier(0)
 template <int S, bool PLUS, bool SPLIT>
-__global__ __launch_bounds__((point_waves(S, PLUS, SPLIT) * 64)) void point_backward_kernel(PointArgs a) {
+__global__ __launch_bounds__((point_waves(S, PLUS, SPLIT) * point_streams(S, PLUS) * 64)) void point_backward_kernel(PointArgs a) {
   constexpr int ST = (S + 31) / 32, NCH = S / 16, ST2 = 2 * ST, GRP = (ST2 + NCH) * (SPLIT ? 2 : 1), NSH = GRP * (PLUS ? 2 : 1);
   constexpr int NTAB = 2 * ST2 + NCH;  // per-head fragments (and as many remainders)
   constexpr int TU = point_table_units(S, SPLIT);
   constexpr bool LDSTAB = TU > 0;
-  extern __shared__ u32x4 tabl[];  // LDSTAB: [wave][TU]
-  constexpr int W = point_waves(S, PLUS, SPLIT);
+  extern __shared__ u32x4 tabl[];  // LDSTAB: [head][TU]; at the end [wave][ST * 32][33] floats
+  constexpr int W = point_waves(S, PLUS, SPLIT), STREAMS = point_streams(S, PLUS);
   constexpr float kLn2 = 0.6931471805599453f;
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
   __shared__ u32x4 wsh[NSH * 64];
   __shared__ u32x4 sel[4 * 64];  // 0, 1: k in kperm order; 2, 3: k in natural order
   __shared__ float bsl[ST * 32], dnl[W][ST * 32], b1l[PLUS ? ST * 32 : 1], w2l[PLUS ? ST * 32 : 1];
-  __shared__ float red[PLUS ? 2 : 1][ST * 32][33];
-  __shared__ float red_t[W];
-  __shared__ float red_w2[PLUS ? ST * 32 : 1], red_b2[W];
+  __shared__ float red_t[W * STREAMS], red_b2[W * STREAMS], red_w2[PLUS ? W * STREAMS : 1][PLUS ? ST * 32 : 1];
   const BwdTablePlan tp = bwd_table_plan(S, PLUS, SPLIT);
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 31, g = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = blockDim.x >> 6;
-  const int h = blockIdx.z * nwaves + wave, b = blockIdx.y, H = a.H, HD = H * 32;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = blockDim.x >> 6, heads = nwaves / STREAMS;
+  const int stream = wave / heads, hw = wave - stream * heads;  // which of the head's waves, head within the workgroup
+  const int h = blockIdx.z * heads + hw, b = blockIdx.y, H = a.H, HD = H * 32;
   const int64_t bh = (int64_t)b * H + h, N = a.N;
 
   for (int u = tid; u < NSH * 64; u += blockDim.x) wsh[u] = a.tabs[u];
@@ -341,9 +378,9 @@ __global__ __launch_bounds__((point_waves(S, PLUS, SPLIT) * 64)) void point_back
       w2l[s] = s < S ? a.pt_w2[s] : 0.f;
     }
   }
-  for (int e = lane; e < ST * 32; e += 64) dnl[wave][e] = e < S ? a.d_norm[bh * S + e] : 0.f;
+  for (int e = lane; e < ST * 32; e += 64) dnl[hw][e] = e < S ? a.d_norm[bh * S + e] : 0.f;
   u32x4 treg[LDSTAB ? 1 : NTAB * (SPLIT ? 2 : 1)];
-  u32x4 *mytab = tabl + wave * TU + lane;
+  u32x4 *mytab = tabl + hw * TU + lane;
   {
     const u32x4 *mine = a.tabs + tp.shared_units + bh * tp.per_head_units + lane;
 #pragma unroll
@@ -370,9 +407,10 @@ __global__ __launch_bounds__((point_waves(S, PLUS, SPLIT) * 64)) void point_back
     return acc;
   };
   const float t_raw = a.temperature[h], inv_t = 1.f / clamp_temperature(t_raw);
-  const float b2 = PLUS ? a.pt_b2[0] : 0.f;
+  const bool odd = lane & 1;
   const bf16x2 ones = {(__bf16)1.f, (__bf16)1.f};
-  f32x16 dws[ST], dw1[PLUS ? ST : 1], dw2[PLUS ? ST : 1];
+  f32x16 dws[ST], dw1[PLUS ? ST : 1];  // this wave's sums
+  float dw2[PLUS ? ST : 1][8];         // d w2: register q of an even lane is slice rowmap(2 q, g), of an odd one rowmap(2 q + 1, g)
   float csum[ST], csum1[PLUS ? ST : 1], tsum = 0.f, b2sum = 0.f;
 #pragma unroll
   for (int st = 0; st < ST; ++st) {
@@ -381,58 +419,79 @@ __global__ __launch_bounds__((point_waves(S, PLUS, SPLIT) * 64)) void point_back
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       dws[st][r] = 0.f;
-      if constexpr (PLUS) dw1[st][r] = dw2[st][r] = 0.f;
+      if constexpr (PLUS) dw1[st][r] = dw2[st][r >> 1] = 0.f;
     }
   }
   __syncthreads();
 
-  u32x4 xm[2], fm[PLUS ? 1 : 2], gg[2];
-  auto row_of = [&](int t) {
-    const int64_t n = (int64_t)t * 32 + i;
-    return (int64_t)b * N + (n < N ? n : N - 1);
+  u32x4 xm[2], fm[PLUS ? 1 : 2], gg[2];  // fetched one tile ahead
+  // a tile's first row (wave-uniform) and this lane's row within it, the last one again beyond N
+  auto tile_row = [&](int t) { return (int64_t)b * N + (int64_t)t * 32; };
+  auto lane_row = [&](int t) {
+    const int64_t last = N - 1 - (int64_t)t * 32;
+    return min(i, (int)(last < 31 ? last : 31));
   };
-  auto load = [&](int t, u32x4(&x)[2], u32x4(&f)[PLUS ? 1 : 2], u32x4(&q)[2]) {
-    const int64_t base = row_of(t) * HD + h * 32 + 8 * g;
+  auto load = [&](const uint16_t *src, int t, u32x4(&v)[2]) {
+    const char *p = reinterpret_cast<const char *>(src + tile_row(t) * HD + h * 32);
+    const unsigned at = (unsigned)(lane_row(t) * HD + 8 * g) * 2u;  // bytes: a scalar base and 32 bits per lane
+    v[0] = *reinterpret_cast<const u32x4 *>(p + at);
+    v[1] = *reinterpret_cast<const u32x4 *>(p + at + 32u);
+  };
+  // PLUS: the noise's samples, slices 32 st + rowmap(4 q .. 4 q + 3, g), and a2
+  uint2 noise[PLUS ? ST : 1][4];
+  float a2_next = 0.f;
+  auto load_noise = [&](int t) {
+    if constexpr (PLUS) {
+      const char *p = reinterpret_cast<const char *>(a.uniform + tile_row(t) * (H * S) + h * S);
+      const unsigned at = (unsigned)(lane_row(t) * (H * S) + 4 * g) * 2u;
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      x[kk] = *reinterpret_cast<const u32x4 *>(a.x_mid + base + 16 * kk);
-      q[kk] = *reinterpret_cast<const u32x4 *>(a.g + base + 16 * kk);
-      if constexpr (!PLUS) f[kk] = *reinterpret_cast<const u32x4 *>(a.fx_mid + base + 16 * kk);
+      for (int st = 0; st < ST; ++st)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (S % 32 == 0 || 32 * st + 8 * q + 4 * g < S)
+            noise[st][q] = *reinterpret_cast<const uint2 *>(p + at + (unsigned)(64 * st + 16 * q));
+      const char *p2 = reinterpret_cast<const char *>(a.a2 + (((int64_t)b * a.tpb + t) * H + h) * 32);
+      a2_next = *reinterpret_cast<const float *>(p2 + (unsigned)i * 4u);
     }
   };
-  if ((int)blockIdx.x < a.tpb) load(blockIdx.x, xm, fm, gg);
+  // streams take turns over the grid, so that few tiles meet as many workgroups as there are
+  const int t0 = blockIdx.x + stream * gridDim.x, tstep = gridDim.x * STREAMS;
+  if (t0 < a.tpb) {
+    load(a.x_mid, t0, xm);
+    load(a.g, t0, gg);
+    if constexpr (!PLUS) load(a.fx_mid, t0, fm);
+    load_noise(t0);
+  }
 
-  for (int t = blockIdx.x; t < a.tpb; t += gridDim.x) {
+  for (int t = t0; t < a.tpb; t += tstep) {
     asm volatile("" ::: "memory");  // the tables are read from LDS where they are used, not kept in registers from here on
     const bool valid = (int64_t)t * 32 + i < N;
-    const int64_t row = row_of(t);
-    u32x4 xn[2], fn[PLUS ? 1 : 2], gn[2];
-    load(t + (int)gridDim.x < a.tpb ? t + gridDim.x : t, xn, fn, gn);  // the tile after this one
+    const int tn = t + tstep < a.tpb ? t + tstep : t;
 
     float it = inv_t, traw = 0.f, a2 = 0.f;  // 1 / temperature of this lane's point
-    f32x16 hd[PLUS ? ST : 1];
+    GeluParts ga2{};
+    auto hidden = [&](int st) {              // the first Linear of proj_temperature, slices 32 st ..
+      f32x16 hd;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) hd[r] = b1l[PLUS ? 32 * st + rowmap(r, g) : 0];
+      hd = mma_shared(1, st * 2 + 0, xm[0], hd);
+      return mma_shared(1, st * 2 + 1, xm[1], hd);
+    };
     if constexpr (PLUS) {
-#pragma unroll
-      for (int st = 0; st < ST; ++st) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) hd[st][r] = b1l[32 * st + rowmap(r, g)];
-        hd[st] = mma_shared(1, st * 2 + 0, xm[0], hd[st]);
-        hd[st] = mma_shared(1, st * 2 + 1, xm[1], hd[st]);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) a2 = fmaf(w2l[32 * st + rowmap(r, g)], gelu_fit(hd[st][r]), a2);
-      }
-      a2 = half_sum(a2) + b2;
-      traw = t_raw + gelu_fit(a2);
-      it = 1.f / bf16_bits_to_f32(f32_to_bf16_bits(fmaxf(traw, 0.01f)));  // the forward rounds it to bf16
+      a2 = a2_next;
+      ga2 = gelu_parts(a2);
+      traw = t_raw + a2 * ga2.phi;
+      it = 1.f / (float)(__bf16)fmaxf(traw, 0.01f);  // the forward rounds it to bf16
     }
     f32x16 z[ST], dw[ST];
     float mx = -INFINITY;
 #pragma unroll
     for (int st = 0; st < ST; ++st) {
+      if constexpr (PLUS) PHASE;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         z[st][r] = bsl[32 * st + rowmap(r, g)];
-        dw[st][r] = dnl[wave][32 * st + rowmap(r, g)];
+        dw[st][r] = dnl[hw][32 * st + rowmap(r, g)];
       }
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
@@ -441,14 +500,13 @@ __global__ __launch_bounds__((point_waves(S, PLUS, SPLIT) * 64)) void point_back
         dw[st] = mma_head(ST2 + st * 2 + kk, PLUS ? xm[kk] : fm[PLUS ? 0 : kk], dw[st]);
       }
       if constexpr (PLUS) {
-        const uint16_t *urow = a.uniform + row * (H * S) + h * S;
+        PHASE;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int s0 = 32 * st + 8 * q + 4 * g;  // slices rowmap(4 q .. 4 q + 3, g)
-          if (S % 32 == 0 || s0 < S) {
-            const uint2 raw = *reinterpret_cast<const uint2 *>(urow + s0);
-            const float uu[4] = {__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xffff0000u),
-                                 __uint_as_float(raw.y << 16), __uint_as_float(raw.y & 0xffff0000u)};
+          if (S % 32 == 0 || 32 * st + 8 * q + 4 * g < S) {
+            const uint2 v = noise[st][q];
+            const float uu[4] = {__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u),
+                                 __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u)};
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
               const float inner = fmaf(-kLn2, __builtin_amdgcn_logf(uu[j] + 1e-8f), 1e-8f);  // -ln(u + eps) + eps
@@ -459,6 +517,11 @@ __global__ __launch_bounds__((point_waves(S, PLUS, SPLIT) * 64)) void point_back
       }
 #pragma unroll
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, z[st][r]);
+    }
+    PHASE;
+    if constexpr (!PLUS) {
+      load(a.g, tn, gg);
+      load(a.fx_mid, tn, fm);
     }
     mx = half_max(mx);
     const float sc = kLog2e * it, off = mx * sc;
@@ -481,15 +544,16 @@ __global__ __launch_bounds__((point_waves(S, PLUS, SPLIT) * 64)) void point_back
     float d_a2 = 0.f;
     if constexpr (PLUS) {
       dlz = half_sum(dlz);
-      const float d_temp = valid && traw >= 0.01f ? -dlz * it * it : 0.f;  // clamp(min): gradient where not clamped
-      d_a2 = d_temp * gelu_erf_grad(a2);
-      if (g == 0) {
+      const float d_temp = traw >= 0.01f ? -dlz * it * it : 0.f;  // clamp(min): gradient where not clamped
+      d_a2 = d_temp * gelu_grad(a2, ga2);  // also in rows beyond N, which write the last row's d x_mid again
+      if (g == 0 && valid) {
         tsum += d_temp;
         b2sum += d_a2;
       }
     } else {
       tsum += valid ? dlz : 0.f;
     }
+    PHASE;
     const float wi = inv * it;
     u32x4 wq[NCH], dzp[NCH];
 #pragma unroll
@@ -503,6 +567,7 @@ __global__ __launch_bounds__((point_waves(S, PLUS, SPLIT) * 64)) void point_back
     f32x16 dxm, dfm;
 #pragma unroll
     for (int r = 0; r < 16; ++r) dxm[r] = dfm[r] = 0.f;
+    PHASE;
 #pragma unroll
     for (int cq = 0; cq < NCH; ++cq) {
       dxm = mma_shared(0, ST2 + cq, dzp[cq], dxm);
@@ -510,6 +575,9 @@ __global__ __launch_bounds__((point_waves(S, PLUS, SPLIT) * 64)) void point_back
       if constexpr (PLUS) dxm = mma_head(2 * ST2 + cq, wq[cq], dxm);
       else dfm = mma_head(2 * ST2 + cq, wq[cq], dfm);
     }
+    u32x4 xn[2];
+    if constexpr (!PLUS) load(a.x_mid, tn, xn);
+    PHASE;
     // x_mid with its points as the reduction index
     f32x16 tr;
 #pragma unroll
@@ -517,112 +585,144 @@ __global__ __launch_bounds__((point_waves(S, PLUS, SPLIT) * 64)) void point_back
     tr = mma(xm[0], sel[2 * 64 + lane], tr);
     tr = mma(xm[1], sel[3 * 64 + lane], tr);
     const u32x4 xt0 = pack_half<0>(tr), xt1 = pack_half<1>(tr);
-    auto accumulate = [&](u32x4(&chunk)[NCH], f32x16(&acc)[ST], float(&cs)[ST]) {
+    // acc += chunks of the slices 32 st .. (lanes <-> points) turned around . x_mid; cs: their sums over the points
+    auto accumulate = [&](u32x4 c0, u32x4 c1, int st, f32x16 &acc, float &cs) {
 #pragma unroll
-      for (int st = 0; st < ST; ++st) {
-        f32x16 tt;
+      for (int j = 0; j < 4; ++j) {
+        c0[j] = valid ? c0[j] : 0u;
+        c1[j] = valid ? c1[j] : 0u;
+      }
+      f32x16 tt;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) tt[r] = 0.f;
+      for (int r = 0; r < 16; ++r) tt[r] = 0.f;
+      tt = mma(c0, sel[lane], tt);
+      if (2 * st + 1 < NCH) tt = mma(c1, sel[64 + lane], tt);
+      const u32x4 t0 = pack_half<0>(tt), t1 = pack_half<1>(tt);
+      acc = mma(t0, xt0, acc);
+      acc = mma(t1, xt1, acc);
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-          if (2 * st + half >= NCH) continue;
-          u32x4 c = chunk[2 * st + half];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) c[j] = valid ? c[j] : 0u;
-          tt = mma(c, sel[half * 64 + lane], tt);
-        }
-        const u32x4 t0 = pack_half<0>(tt), t1 = pack_half<1>(tt);
-        acc[st] = mma(t0, xt0, acc[st]);
-        acc[st] = mma(t1, xt1, acc[st]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t w0 = t0[j], w1 = t1[j];
-          cs[st] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w0), ones, cs[st], false);
-          cs[st] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w1), ones, cs[st], false);
-        }
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t w0 = t0[j], w1 = t1[j];
+        cs = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w0), ones, cs, false);
+        cs = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w1), ones, cs, false);
       }
     };
-    accumulate(dzp, dws, csum);
+#pragma unroll
+    for (int st = 0; st < ST; ++st) {
+      PHASE;
+      accumulate(dzp[2 * st], dzp[2 * st + 1 < NCH ? 2 * st + 1 : 0], st, dws[st], csum[st]);
+    }
     if constexpr (PLUS) {
+      const float d_sum = valid ? d_a2 : 0.f;
 #pragma unroll
-      for (int st = 0; st < ST; ++st)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float v = hd[st][r];
-          const GeluParts p = gelu_parts(v);
-          dw2[st][r] = fmaf(d_a2, v * p.phi, dw2[st][r]);
-          hd[st][r] = d_a2 * w2l[32 * st + rowmap(r, g)] * gelu_grad(v, p);
+      for (int st = 0; st < ST; ++st) {  // the hidden values again: 8 matrix instructions against 32 registers held since a2
+        PHASE;
+        f32x16 hd = hidden(st);
+        if (st == ST - 1) {  // the next tile, under the activations: earlier, its registers would have to be spilled
+          load(a.x_mid, tn, xm);
+          load(a.g, tn, gg);
+          load_noise(tn);
+          PHASE;
         }
 #pragma unroll
-      for (int cq = 0; cq < NCH; ++cq) dzp[cq] = (cq & 1) ? pack_half<1>(hd[cq >> 1]) : pack_half<0>(hd[cq >> 1]);
+        for (int q = 0; q < 8; ++q) {
+          float act[2];
 #pragma unroll
-      for (int cq = 0; cq < NCH; ++cq) {
-        dxm = mma_shared(1, ST2 + cq, dzp[cq], dxm);
-        dxm = mma_rest(1, ST2 + cq, hd[cq >> 1], cq & 1, dxm);
+          for (int k = 0; k < 2; ++k) {
+            const float v = hd[2 * q + k];
+            const GeluParts p = gelu_parts(v);
+            act[k] = d_sum * (v * p.phi);
+            hd[2 * q + k] = d_a2 * w2l[32 * st + rowmap(2 * q + k, g)] * gelu_grad(v, p);
+          }
+          // two lanes share two slices' sums: half the registers
+          const float keep = odd ? act[1] : act[0], give = odd ? act[0] : act[1];
+          dw2[st][q] += keep + __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(give), 0xB1, 0xf, 0xf, true));
+        }
+        const u32x4 c0 = pack_half<0>(hd), c1 = pack_half<1>(hd);
+        dxm = mma_shared(1, ST2 + 2 * st, c0, dxm);
+        dxm = mma_rest(1, ST2 + 2 * st, hd, 0, dxm);
+        if (2 * st + 1 < NCH) {
+          dxm = mma_shared(1, ST2 + 2 * st + 1, c1, dxm);
+          dxm = mma_rest(1, ST2 + 2 * st + 1, hd, 1, dxm);
+        }
+        accumulate(c0, c1, st, dw1[st], csum1[st]);
       }
-      accumulate(dzp, dw1, csum1);
     }
-    uint16_t *pr = a.d_proj + row * (PLUS ? HD : 2 * HD) + h * 32;
+    PHASE;
+    constexpr int NP = PLUS ? 1 : 2;
+    char *pb = reinterpret_cast<char *>(a.d_proj + tile_row(t) * (NP * HD) + h * 32);
+    uint16_t *pr = reinterpret_cast<uint16_t *>(pb + (unsigned)(lane_row(t) * (NP * HD)) * 2u);
     store_tile_natural(dxm, pr, g, true);
     if constexpr (!PLUS) store_tile_natural(dfm, pr + HD, g, true);
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      xm[kk] = xn[kk];
-      gg[kk] = gn[kk];
-      if constexpr (!PLUS) fm[kk] = fn[kk];
-    }
+    if constexpr (!PLUS) xm[0] = xn[0], xm[1] = xn[1];
   }
 
-  // one row of partial gradients per workgroup: the waves (heads) add up in order
-  for (int w = 0; w < nwaves; ++w) {
-    if (wave == w) {
-#pragma unroll
-      for (int st = 0; st < ST; ++st) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          float &at = red[0][32 * st + rowmap(r, g)][i];
-          at = w == 0 ? dws[st][r] : at + dws[st][r];
-          if constexpr (PLUS) {
-            float &a1t = red[PLUS ? 1 : 0][32 * st + rowmap(r, g)][i];
-            a1t = w == 0 ? dw1[st][r] : a1t + dw1[st][r];
-            float v = dw2[st][r];
-#pragma unroll
-            for (int o = 16; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-            if (i == 0) red_w2[32 * st + rowmap(r, g)] = w == 0 ? v : red_w2[32 * st + rowmap(r, g)] + v;
-          }
-        }
-        const float c = half_sum(csum[st]);
-        if (g == 0) red[0][32 * st + i][32] = w == 0 ? c : red[0][32 * st + i][32] + c;
-        if constexpr (PLUS) {
-          const float c1 = half_sum(csum1[st]);
-          if (g == 0) red[PLUS ? 1 : 0][32 * st + i][32] = w == 0 ? c1 : red[PLUS ? 1 : 0][32 * st + i][32] + c1;
-        }
-      }
-      float ts = wave_sum(tsum), bs = PLUS ? wave_sum(b2sum) : 0.f;
-      if constexpr (!PLUS) ts = t_raw >= kTempMin && t_raw <= kTempMax ? -ts * inv_t * inv_t : 0.f;  // clamp's gradient
-      if (lane == 0) {
-        red_t[wave] = ts;
-        red_b2[wave] = bs;
-      }
-    }
-    __syncthreads();
-  }
+  // One row of partial gradients per workgroup.  The waves leave their sums side by side in LDS, over the tables, and all threads
+  // add them up in the waves' order: the waves in turn, each with the shuffles of d w2, took 40 us behind the last tile (8 192
+  // points, S = 64: 74 us, PLUS).
   const int n = point_grads(S, H, PLUS);
   float *dst = a.partials + (((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * n;
-  for (int e = tid; e < S * 32; e += blockDim.x) dst[e] = red[0][e >> 5][e & 31];
-  for (int s = tid; s < S; s += blockDim.x) dst[S * 32 + s] = red[0][s][32];
-  const int h0 = blockIdx.z * nwaves;
-  for (int e = tid; e < H; e += blockDim.x) dst[S * 33 + e] = e >= h0 && e < h0 + nwaves ? red_t[e - h0] : 0.f;
+  float *sums = reinterpret_cast<float *>(tabl);
+  auto total = [&](const f32x16(&acc)[ST], const float(&cs)[ST], float *out) {  // (S, 32) and behind it (S)
+    __syncthreads();
+    float *mine = sums + wave * (ST * 32 * 33);
+#pragma unroll
+    for (int st = 0; st < ST; ++st) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mine[(32 * st + rowmap(r, g)) * 33 + i] = acc[st][r];
+      const float c = half_sum(cs[st]);
+      if (g == 0) mine[(32 * st + i) * 33 + 32] = c;
+    }
+    __syncthreads();
+    for (int e = tid; e < S * 33; e += blockDim.x) {
+      float v = 0.f;
+      for (int w = 0; w < nwaves; ++w) v += sums[w * (ST * 32 * 33) + e];
+      const int sl = e / 33, c = e - sl * 33;
+      out[c < 32 ? sl * 32 + c : S * 32 + sl] = v;
+    }
+  };
+  float ts = wave_sum(tsum), bs = PLUS ? wave_sum(b2sum) : 0.f;
+  if constexpr (!PLUS) ts = t_raw >= kTempMin && t_raw <= kTempMax ? -ts * inv_t * inv_t : 0.f;  // clamp's gradient
+  if (lane == 0) {
+    red_t[wave] = ts;
+    red_b2[wave] = bs;
+  }
+  if constexpr (PLUS) {
+#pragma unroll
+    for (int st = 0; st < ST; ++st)
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {  // over the lanes of this half with the same parity
+        float v = dw2[st][q];
+        auto step = [](float x, auto ctrl) {
+          constexpr int c = decltype(ctrl)::value;
+          return x + __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), c, 0xf, 0xf, true));
+        };
+        v = step(v, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+        v = step(v, std::integral_constant<int, 0x124>{});  // row_ror:4
+        v = step(v, std::integral_constant<int, 0x128>{});  // row_ror:8
+        const auto o = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        if (i < 2) red_w2[wave][32 * st + rowmap(2 * q + i, g)] = __uint_as_float(o[0]) + __uint_as_float(o[1]);
+      }
+  }
+  total(dws, csum, dst);
+  const int h0 = blockIdx.z * heads;
+  for (int e = tid; e < H; e += blockDim.x) {
+    float v = 0.f;
+    if (e >= h0 && e < h0 + heads)
+      for (int q = 0; q < STREAMS; ++q) v += red_t[q * heads + e - h0];
+    dst[S * 33 + e] = v;
+  }
   if constexpr (PLUS) {
     dst += S * 33 + H;
-    for (int e = tid; e < S * 32; e += blockDim.x) dst[e] = red[PLUS ? 1 : 0][e >> 5][e & 31];
+    total(dw1, csum1, dst);
     for (int s = tid; s < S; s += blockDim.x) {
-      dst[S * 32 + s] = red[PLUS ? 1 : 0][s][32];
-      dst[S * 33 + s] = red_w2[s];
+      float v = 0.f;
+      for (int w = 0; w < nwaves; ++w) v += red_w2[w][s];
+      dst[S * 33 + s] = v;
     }
     if (tid == 0) {
-      float v = red_b2[0];
-      for (int w = 1; w < nwaves; ++w) v += red_b2[w];
+      float v = 0.f;
+      for (int w = 0; w < nwaves; ++w) v += red_b2[w];
       dst[S * 34] = v;
     }
   }
@@ -726,8 +826,7 @@ static int point_head_waves(const pa_shape &s, bool plus) {  // waves (heads) pe
   return (int)(s.H < most ? s.H : most);
 }
 
-// workgroups along the points: the chip filled once by the workgroups that fit it (8 waves of 256 or 4 of 512 registers
-// per CU), so that a workgroup's tables and its partial row are paid for once
+// workgroups along the points: the chip filled once by the workgroups that fit it (8 waves of 256 registers or 4 of 512 per CU), so that a workgroup's tables and its partial row are paid for once
 static int64_t point_groups(const pa_shape &s, bool plus, int num_cu) {
   const int w = point_head_waves(s, plus), most = point_waves((int)s.S, plus, float_tables(s, plus));
   const int64_t resident = (int64_t)num_cu * (most / w), other = s.B * (s.H / w), tpb = tiles_per_batch(s);
@@ -741,6 +840,7 @@ int64_t point_backward_workspace_bytes(const pa_shape &s, bool plus, int num_cu)
   const int64_t wgs = point_groups(s, plus, num_cu) * s.B * (s.H / point_head_waves(s, plus));
   return (tp.shared_units + s.B * s.H * tp.per_head_units) * 16 + wgs * point_backward_grads(s, plus) * 4;
 }
+int64_t temperature_hidden_bytes(const pa_shape &s) { return s.B * tiles_per_batch(s) * s.H * 32 * 4; }
 
 // the operand fragments of W_slice (Transolver++: and W1), out_token (NULL: zeros) and d_num
 int backward_tables(const pa_shape &s, const float *w_slice, const float *pt_w1, const float *out_token, const float *d_num,
@@ -757,7 +857,7 @@ int backward_tables(const pa_shape &s, const float *w_slice, const float *pt_w1,
 int point_backward(const pa_shape &s, const pa_params &p, const pa_plus_params *plus, const void *x_mid,
                    const void *fx_mid, const void *d_out_x, const void *uniform, const float *out_token,
                    const float *d_num, const float *d_norm, void *workspace, void *d_proj, float *grads, int num_cu,
-                   hipStream_t st, wgrad::Sums *later) {
+                   hipStream_t st, wgrad::Sums *later, const float *a2) {
   if (!point_backward_supported(s)) return PA_ERR_UNSUPPORTED;
   const bool split = float_tables(s, plus != nullptr);
   const BwdTablePlan tp = bwd_table_plan((int)s.S, plus != nullptr, split);
@@ -768,6 +868,7 @@ int point_backward(const pa_shape &s, const pa_params &p, const pa_plus_params *
   a.fx_mid = static_cast<const uint16_t *>(fx_mid);
   a.g = static_cast<const uint16_t *>(d_out_x);
   a.uniform = static_cast<const uint16_t *>(uniform);
+  a.a2 = a2;
   a.tabs = tabs;
   a.d_norm = d_norm, a.b_slice = p.in_project_slice_bias, a.temperature = p.temperature;
   if (plus) a.pt_b1 = plus->proj_temperature_0_bias, a.pt_w2 = plus->proj_temperature_2_weight, a.pt_b2 = plus->proj_temperature_2_bias;
@@ -777,15 +878,31 @@ int point_backward(const pa_shape &s, const pa_params &p, const pa_plus_params *
   int rc = backward_tables(s, p.in_project_slice_weight, plus ? plus->proj_temperature_0_weight : nullptr, out_token, d_num, split,
                            tabs, st);
   if (rc) return rc;
+  if (plus && !a2) {  // behind the partial gradients
+    float *own = a.partials + point_groups(s, true, num_cu) * s.B * (s.H / point_head_waves(s, true)) * point_backward_grads(s, true);
+    const int64_t gx = a.tpb < 1024 ? a.tpb : 1024;
+    const dim3 grid((unsigned)gx, (unsigned)s.B, (unsigned)s.H);
+    switch (s.S) {
+      case 16: hipLaunchKernelGGL(temperature_hidden_kernel<16>, grid, dim3(64), 0, st, a, own); break;
+      case 32: hipLaunchKernelGGL(temperature_hidden_kernel<32>, grid, dim3(64), 0, st, a, own); break;
+      case 64: hipLaunchKernelGGL(temperature_hidden_kernel<64>, grid, dim3(64), 0, st, a, own); break;
+      default: hipLaunchKernelGGL(temperature_hidden_kernel<128>, grid, dim3(64), 0, st, a, own); break;
+    }
+    if ((rc = launch_status())) return rc;
+    a.a2 = own;
+  }
   const int w = point_head_waves(s, plus != nullptr);
   const int64_t G = point_groups(s, plus != nullptr, num_cu), Z = s.H / w;
-  const dim3 grid((unsigned)G, (unsigned)s.B, (unsigned)Z), block((unsigned)(w * 64));
+  const int streams = point_streams((int)s.S, plus != nullptr);
+  const dim3 grid((unsigned)G, (unsigned)s.B, (unsigned)Z), block((unsigned)(w * streams * 64));
 #define PA_POINT(SS)                                                                             \
   case SS: {                                                                                     \
     auto kernel = plus    ? point_backward_kernel<SS, true, true>                                \
                   : split ? point_backward_kernel<SS, false, true>                               \
                           : point_backward_kernel<SS, false, false>;                             \
-    const size_t lds = (size_t)w * point_table_units(SS, split) * 16;                            \
+    const size_t tables = (size_t)w * point_table_units(SS, split) * 16;                         \
+    const size_t totals = (size_t)w * streams * ((SS + 31) / 32 * 32) * 33 * 4;                  \
+    const size_t lds = tables > totals ? tables : totals;                                        \
     if ((rc = allow_dynamic_lds(kernel, lds))) return rc;                                        \
     hipLaunchKernelGGL(kernel, grid, block, lds, st, a);                                         \
   } break

@@ -113,7 +113,7 @@ __global__ __launch_bounds__(512) void slice_softmax_pack_plus_kernel(
     const uint16_t *__restrict__ x_mid, const uint16_t *__restrict__ uniform, const float *__restrict__ w_slice,
     const float *__restrict__ b_slice, const float *__restrict__ temperature, const float *__restrict__ pt_w1,
     const float *__restrict__ pt_b1, const float *__restrict__ pt_w2, const float *__restrict__ pt_b2,
-    u32x4 *__restrict__ w_pack, int64_t N, int tpb, int H) {
+    u32x4 *__restrict__ w_pack, float *__restrict__ a2_out, int64_t N, int tpb, int H) {
   constexpr int ST = (S + 31) / 32, NCH = S / 16;
   constexpr float kLn2 = 0.6931471805599453f;
   constexpr int NP = SPLIT ? 2 : 1;
@@ -166,6 +166,9 @@ __global__ __launch_bounds__(512) void slice_softmax_pack_plus_kernel(
       for (int r = 0; r < 16; ++r) a2 = fmaf(w2l[32 * st + rowmap(r, g)], SPLIT ? gelu_fit(hd[r]) : gelu_logistic(hd[r]), a2);
     }
     a2 = half_sum(a2) + b2;
+    if constexpr (SPLIT) {  // the backward pass starts from here
+      if (a2_out && g == 0) a2_out[(((int64_t)b * tpb + t) * H + h) * 32 + i] = a2;
+    }
     const float temp = bf16_bits_to_f32(f32_to_bf16_bits(fmaxf(temp_h + (SPLIT ? gelu_fit(a2) : gelu_logistic(a2)), 0.01f)));
     const float sc = kLog2e * __builtin_amdgcn_rcpf(temp);
     // logits + Gumbel noise
@@ -416,7 +419,7 @@ int slice_softmax_pack(const pa_shape &s, const pa_params &p, const void *x_mid,
 }
 
 int slice_softmax_pack_plus(const pa_shape &s, const pa_params &p, const pa_plus_params &pp, const void *x_mid,
-                            const void *uniform, void *w_pack, bool split, int num_cu, hipStream_t st) {
+                            const void *uniform, void *w_pack, bool split, float *a2_out, int num_cu, hipStream_t st) {
   const int waves = (int)(s.H < 8 ? s.H : 8);
   if (s.H % waves != 0) return PA_ERR_UNSUPPORTED;
   const int groups = (int)(s.H / waves);
@@ -430,8 +433,8 @@ int slice_softmax_pack_plus(const pa_shape &s, const pa_params &p, const pa_plus
                      block, 0, st, static_cast<const uint16_t *>(x_mid),                                             \
                      static_cast<const uint16_t *>(uniform), p.in_project_slice_weight, p.in_project_slice_bias,     \
                      p.temperature, pp.proj_temperature_0_weight, pp.proj_temperature_0_bias,                        \
-                     pp.proj_temperature_2_weight, pp.proj_temperature_2_bias, static_cast<u32x4 *>(w_pack), s.N,    \
-                     (int)tpb, (int)s.H)
+                     pp.proj_temperature_2_weight, pp.proj_temperature_2_bias, static_cast<u32x4 *>(w_pack),        \
+                     a2_out, s.N, (int)tpb, (int)s.H)
   switch (s.S) {
     case 16: PA_LAUNCH_SSPP(16); break;
     case 32: PA_LAUNCH_SSPP(32); break;

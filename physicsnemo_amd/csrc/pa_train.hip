@@ -77,7 +77,7 @@ static int64_t round_up(int64_t v) { return (v + 255) / 256 * 256; }
 
 // ---- buffer plans ----
 struct Saved {  // kept from the forward to the backward pass
-  int64_t w_in, w_in_t, w_out, w_out_t, small, w_pack, tok, norm, tok_out, x_mid, fx_mid, total;
+  int64_t w_in, w_in_t, w_out, w_out_t, small, w_pack, tok, norm, tok_out, x_mid, fx_mid, a2, total;
 };
 struct Scratch {
   int64_t blob, fx_pack, partials, tokp, out_x, total;                                     // forward
@@ -153,6 +153,7 @@ static Saved plan_saved(const pa_shape &s, bool plus) {
     p.x_mid = take(s.B * s.N * HD * 2);
     if (!plus) p.fx_mid = take(s.B * s.N * HD * 2);
   }
+  if (plus) p.a2 = take(mfma::temperature_hidden_bytes(s));
   p.total = off;
   return p;
 }
@@ -295,7 +296,7 @@ int forward(const pa_shape &s, int weight_dtype, const pa_params &params, const 
     a.pack_tpb = (int)mfma::tiles_per_batch(s), a.pack_heads = (int)s.H;
     if (!gemm::serves(a, pl ? 1 : 2, 2)) return PA_ERR_UNSUPPORTED;
     if ((rc = gemm::launch(a, pl ? 1 : 2, PA_BF16, st))) return rc;
-    rc = pl ? mfma::slice_softmax_pack_plus(s, p, prep.q, x_mid, uniform, w_pack, true, num_cu, st)
+    rc = pl ? mfma::slice_softmax_pack_plus(s, p, prep.q, x_mid, uniform, w_pack, true, reinterpret_cast<float *>(sv + sp.a2), num_cu, st)
             : mfma::slice_softmax_pack(s, p, x_mid, w_pack, num_cu, st);
     if (rc) return rc;
     if ((rc = mfma::slice_reduce(s, w_pack, fx_pack, partials, st))) return rc;
@@ -345,7 +346,7 @@ int backward(const pa_shape &s, bool pl, const void *x, const void *uniform, con
       if ((rc = general::project_inputs(PA_BF16, s, p, x, ws + sc.x_mid, ws + sc.fx_mid, st))) return rc;
     }
     if ((rc = mfma::point_backward(s, p, pl ? &prep.q : nullptr, x_mid, fx_mid, g, uniform, tok_out, d_num, d_norm, point, d_proj,
-                                   small, num_cu, st, &sums)))
+                                   small, num_cu, st, &sums, pl ? reinterpret_cast<const float *>(sv + sp.a2) : nullptr)))
       return rc;
   }
   if (dx && (rc = general::rows_gemm(PA_BF16, s, np * HD, s.C, d_proj, sv + sp.w_in_t, nullptr, 0, dx, st))) return rc;

@@ -2,11 +2,14 @@
 uniform samples behind the Gumbel noise handed to both sides (deterministic parity), plus a distributional check of the
 self-drawn noise path.  Bars: fp32 rtol 1e-4 (2e-4 for gradients) with atol = rtol * max|ref| per tensor; bf16 output
 rel-L2 2e-2, bf16 gradients rel-L2 5e-2 (1e-1 for the scalar proj_temperature.2.bias) against the fp32 reference."""
+from ctypes import byref
+
 import pytest
 import torch
 
 from oracle import torch_oracle as to
 import physicsnemo_amd as pn
+from physicsnemo_amd import _lib, functional as PF
 from gpu_util import announce, assert_fp32_close, assert_rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -195,3 +198,72 @@ def test_plus_training_forward_draws_noise_and_backpropagates():
     y2.square().mean().backward()
     assert torch.equal(y1, y2) and torch.equal(g1, x.grad)  # same generator state: same noise, same gradient
     assert all(p.grad is not None and torch.isfinite(p.grad).all() for p in hip.parameters())
+
+
+@pytest.mark.parametrize("H,S", [(4, 16), (8, 32), (8, 64), (4, 64), (16, 64), (8, 128)])
+@pytest.mark.parametrize("B,N", [(1, 1), (2, 33), (1, 8000), (3, 700)])
+def test_per_point_backward_entry(H, S, B, N):
+    """pa_point_backward with and without the learned temperature against float64 autograd over what it differentiates,
+    sum_n,h,s w (g . tok' + fx_mid . d num + d nrm): one tile, ragged tiles, fewer tiles than waves and more.  Without a forward
+    pass the Transolver++ form forms the temperature's hidden value itself.  1e-2: bf16 results (2^-9) and bf16 operands of
+    the reductions."""
+    announce("per-point backward", H, S, B, N)
+    gen = torch.Generator().manual_seed(100 * H + S + N)
+    r = lambda *size: torch.randn(*size, generator=gen)
+    x_mid, fx_mid, g = (0.5 * r(B, N, H, 32)).bfloat16(), r(B, N, H, 32).bfloat16(), r(B, N, H, 32).bfloat16()
+    u = torch.rand(B, N, H, S, generator=gen).clamp(max=0.99).bfloat16()  # 1 in bf16 is another noise in float64 than in float32
+    tok, d_num, d_norm = r(B, H, S, 32), 0.3 * r(B, H, S, 32), 0.3 * r(B, H, S)
+    p = {"ws": r(S, 32) / 6, "bs": 0.1 * r(S), "t": 0.4 + 0.2 * torch.rand(H, generator=gen),
+         "w1": r(S, 32) / 6, "b1": 0.1 * r(S), "w2": r(S) / S ** 0.5, "b2": 0.1 * r(1)}
+    dims = PF.LayerDims(B=B, N=N, C=32 * H, H=H, D=32, S=S)
+    lib, shape = _lib.load(), dims.c()
+    dev = {k: v.cuda().contiguous() for k, v in p.items()}
+    for plus in (True, False):
+        if not plus:  # the plain form may multiply with bf16 tables: give it tables that are exact in bf16
+            tok, d_num, p["ws"] = tok.bfloat16().float(), d_num.bfloat16().float(), p["ws"].bfloat16().float()
+            dev["ws"] = p["ws"].cuda()
+        q = {k: v.double().requires_grad_(True) for k, v in p.items()}
+        xm, fm = x_mid.double().requires_grad_(True), fx_mid.double().requires_grad_(True)
+        z = xm @ q["ws"].T + q["bs"]
+        if plus:
+            a2 = torch.nn.functional.gelu(xm @ q["w1"].T + q["b1"]) @ q["w2"] + q["b2"]
+            a2.retain_grad()
+            temp = (q["t"] + torch.nn.functional.gelu(a2)).clamp(min=0.01)[..., None]
+            temp = temp + (temp.bfloat16().double() - temp).detach()  # the forward's temperature is a bf16 value
+            z = z - torch.log(-torch.log(u.double() + 1e-8) + 1e-8)
+        else:
+            temp = q["t"].clamp(0.5, 5.0)[:, None]
+        w = torch.softmax(z / temp, -1)
+        v = xm if plus else fm
+        (torch.einsum("bnhs,bnhd,bhsd->", w, g.double(), tok.double())
+         + torch.einsum("bnhs,bnhd,bhsd->", w, v, d_num.double()) + (w * d_norm.double()[:, None]).sum()).backward()
+
+        params = _lib.PaParams()
+        params.in_project_slice_weight, params.in_project_slice_bias = dev["ws"].data_ptr(), dev["bs"].data_ptr()
+        params.temperature = dev["t"].data_ptr()
+        pp = _lib.PaPlusParams(*[dev[k].data_ptr() for k in ("w1", "b1", "w2", "b2")])
+        nbytes = lib.pa_point_backward_workspace_bytes(byref(shape), int(plus))
+        ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+        grads = torch.full((lib.pa_point_backward_grads(byref(shape), int(plus)),), float("nan"), device="cuda")
+        d_proj = torch.empty(B, N, (1 if plus else 2) * H * 32, dtype=torch.bfloat16, device="cuda")
+        bufs = [t.cuda().contiguous() for t in (x_mid, fx_mid, g, u, tok, d_num, d_norm)]
+        _lib.check(lib.pa_point_backward(
+            byref(shape), byref(params), byref(pp) if plus else None, bufs[0].data_ptr(), None if plus else bufs[1].data_ptr(),
+            bufs[2].data_ptr(), bufs[3].data_ptr() if plus else None, bufs[4].data_ptr(), bufs[5].data_ptr(), bufs[6].data_ptr(),
+            ws.data_ptr(), nbytes, d_proj.data_ptr(), grads.data_ptr(), _lib.current_stream_ptr(d_proj.device)), "pa_point_backward")
+        got = d_proj.view(B, N, -1, H, 32)
+        assert_rel_l2(got[:, :, 0], xm.grad, f"plus={plus} d x_mid", tol=1e-2)
+        if not plus:
+            assert_rel_l2(got[:, :, 1], fm.grad, "d fx_mid", tol=1e-2)
+        names, at = ["ws", "bs", "t"] + (["w1", "b1", "w2"] if plus else []), 0
+        for k in names:
+            n = q[k].numel()
+            part = grads[at:at + n].cpu().double()
+            # sums over the points whose terms cancel: against the size of the terms
+            scale = max(float(q[k].grad.norm()), 0.05 * float(q[{"bs": "ws", "b1": "w1", "t": "ws"}.get(k, k)].grad.norm()))
+            assert float((part - q[k].grad.flatten()).norm()) <= 1e-2 * scale, (plus, k)
+            at += n
+        if plus:
+            assert abs(float(grads[at]) - float(q["b2"].grad)) <= 1e-2 * float(a2.grad.abs().sum())
+            at += 1
+        assert at == grads.numel()
