@@ -453,29 +453,38 @@ __global__ __launch_bounds__(512) void cols_gemm_kernel(const uint16_t *__restri
 // row chunks: about two workgroups per CU over all column groups, and at least 32 blocks of 32 rows per chunk so that
 // ------------------------------------------------------------------------------------------------
 // cols_gemm_f32_kernel: the float32 form of the weight-gradient product  P[oa][ob] = sum_m A[m][oa] * B[m][ob].
-// v_mfma_f32_32x32x2_f32 reduces over two rows m per instruction with lane (i, g) supplying A[m0 + g][oa0 + i] and
-// B[m0 + g][ob0 + i]: consecutive lanes read consecutive columns of a row, so natural row-major operands need no
-// transposition.  A workgroup (4 waves) owns a 128 x 128 block of P for one chunk of rows: 32 rows of its 128 + 128
-// operand columns at a time go through LDS (coalesced 16-byte loads, double buffered), wave w multiplies the 64 x 64
-// sub-block (w & 1, w >> 1): per pair of rows 2 + 2 LDS words feed 4 MFMAs.  Row chunks come back as partials
-// P[g][oa][ob] (fixed-order sum by the caller); col_sums[g][oa] = sum_m A[m][oa] from the same pass (blockIdx.z == 0).
-// Bound by the float32 MFMAs, which neighbours found by 64-bit divisions for every row kept waiting: 4 x 85 x 85 grid points, 3 x 3
-// taps, 128 -> 2 x 128 (17 GFLOP) 212 us with them, 182 us with coordinates that are carried from step to step.
+// v_mfma_f32_32x32x2_f32 reduces over two rows m per instruction with lane (i, g) supplying one value of row m0 + g of either
+// operand: consecutive lanes hold consecutive columns of a row, so natural row-major operands need no transposition.  A workgroup
+// (4 waves) owns a 128 x 128 block of P for one chunk of rows, wave w the 64 x 64 sub-block (w & 1, w >> 1); lane i takes columns
+// 2 i and 2 i + 1 of both operands, one 8-byte load each per pair of rows, for the 4 MFMAs (256 cycles) of the pair.  The operands
+// go straight from memory to registers, 16 pairs (32 rows) ahead: at this rate four waves ask for 8 bytes a cycle, the two waves
+// that share a column meet in the L1, and no wave waits for another.  Rows beyond the chunk and neighbours outside the grid
+// are out of the buffers' range and read as zero.
+// Row chunks come back as partials P[g][oa][ob] (fixed-order sum by the caller); col_sums[g][oa] = sum_m A[m][oa] from the same
+// pass.  Workgroups that share a chunk (the blocks of columns, the taps) run on one XCD, one after the other.
+// Bound by the float32 MFMAs: 4 x 85 x 85 grid points, 3 x 3 taps, 128 -> 2 x 128 (17 GFLOP) 149 us, 128 x 128 over 28 900 rows 16 us;
+// through LDS, one barrier per 32 rows, 176 and 20; with all loads of a block behind its matrix instructions 169 and 20.
 // ------------------------------------------------------------------------------------------------
 constexpr int kF32Tile = 128, kF32Rows = 32;
 
-__global__ __launch_bounds__(256) void cols_gemm_f32_kernel(const float *__restrict__ A, int lda, int OA,
-                                                            const float *__restrict__ B, int ldb, int OB, int64_t M,
-                                                            int64_t rows_per_chunk, GridTaps grid,
-                                                            float *__restrict__ partials, float *__restrict__ col_sums) {
-  __shared__ float As[2][kF32Rows][kF32Tile];
-  __shared__ float Bs[2][kF32Rows][kF32Tile];
+__global__ __launch_bounds__(256, 2) void cols_gemm_f32_kernel(const float *__restrict__ A, int lda, int OA,
+                                                               const float *__restrict__ B, int ldb, int OB, int64_t M,
+                                                               int64_t rows_per_chunk, int chunks, GridTaps grid,
+                                                               float *__restrict__ partials, float *__restrict__ col_sums) {
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  constexpr int kPairs = kF32Rows / 2;
+  constexpr unsigned kOut = 0x80000000u;  // an offset no buffer here reaches
   const int t = threadIdx.x, lane = t & 63, i = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int nob = (OB + kF32Tile - 1) / kF32Tile, tap = blockIdx.z / nob;
-  const int oa0 = blockIdx.y * kF32Tile, ob0 = (blockIdx.z - tap * nob) * kF32Tile;
-  const int64_t m_begin = (int64_t)blockIdx.x * rows_per_chunk;
-  const int64_t m_end = min(M, m_begin + rows_per_chunk);
+  const int noa = (OA + kF32Tile - 1) / kF32Tile, nob = (OB + kF32Tile - 1) / kF32Tile, tiles = noa * nob * grid.taps;
+  // the (chunk, tile) pairs in chunk-major order are dealt out to the XCDs (= workgroup id mod 8) in eight equal runs
+  const int item = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const int chunk = __builtin_amdgcn_readfirstlane(item / tiles), tile = item - chunk * tiles;
+  if (chunk >= chunks) return;
+  const int zt = __builtin_amdgcn_readfirstlane(tile / noa), tap = __builtin_amdgcn_readfirstlane(zt / nob);
+  const int oa0 = (tile - zt * noa) * kF32Tile, ob0 = (zt - tap * nob) * kF32Tile;
+  const int64_t m_begin = (int64_t)chunk * rows_per_chunk;
+  const int64_t m_end = M < m_begin + rows_per_chunk ? M : m_begin + rows_per_chunk;
   const int wa = (wave & 1) * 64, wb = (wave >> 1) * 64;  // this wave's sub-block of the tile
 
   f32x16 acc[2][2];
@@ -487,94 +496,89 @@ __global__ __launch_bounds__(256) void cols_gemm_f32_kernel(const float *__restr
       for (int r = 0; r < 16; ++r) acc[u][v][r] = 0.f;
   float csum[2] = {0.f, 0.f};
 
-  // staging: 32 rows x 128 columns = 1024 float4 per operand, 4 per thread
-  const int sr = t >> 5, sc = (t & 31) * 4;  // row 0..7 (+8 k), column of the float4
-  float4 pa[4], pb[4];
-  // where the rows fetched next lie in the grid: found by division once, then by steps of 32 rows
+  // Convolution: row m's neighbour at this tap is row m + shift where that lies inside the grid.  Lane l looks after row l % 32 of
+  // a block: its grid coordinates are divided out once and then advanced by the 32 rows of a block with carries.
   const bool conv = grid.ks > 0;
   const int gd = grid.gd > 0 ? grid.gd : 1, gw = conv ? grid.gw : 1, gh = conv ? grid.gh : 1, ksd = grid.gd > 0 ? grid.ks : 1;
   const int pad = grid.ks / 2, pad_d = grid.gd > 0 ? pad : 0;
-  const int tu = conv ? tap / ksd / grid.ks - pad : 0, tv = conv ? tap / ksd % grid.ks - pad : 0, tz = conv ? tap % ksd - pad_d : 0;
-  const int64_t shift = ((int64_t)tu * gw + tv) * gd + tz;  // the neighbour, from the row
-  int ci[4], cj[4], cl[4];
+  const int uv = conv ? __builtin_amdgcn_readfirstlane(tap / ksd) : 0, tap_u = conv ? __builtin_amdgcn_readfirstlane(uv / grid.ks) : 0;
+  const int tu = tap_u - pad, tv = uv - tap_u * grid.ks - pad, tz = tap - uv * ksd - pad_d;
+  const int64_t shift = conv ? ((int64_t)tu * gw + tv) * gd + tz : 0;
   const int step_l = kF32Rows % gd, step_j = kF32Rows / gd % gw, step_i = kF32Rows / gd / gw;
+  unsigned n0 = conv ? (unsigned)((m_begin + i) % grid.N) : 0u;
+  int cl = (int)(n0 % gd), cj = (int)(n0 / gd % gw), ci = (int)(n0 / gd / gw);
+  // byte offsets of this lane's columns in the first pair of a block
+  const int ca = oa0 + wa + 2 * i, cb = ob0 + wb + 2 * i;
+  const unsigned a_off = ca < OA ? (unsigned)(g * lda + ca) * 4u : kOut, b_off = cb < OB ? (unsigned)(g * ldb + cb) * 4u : kOut;
+  u32x2 av[kPairs], bv[kPairs];  // the operands of a block of rows
+  const float *pa = A + m_begin * lda, *pb = B + (m_begin + shift) * ldb;  // the block requested next (pb: may lie before B, unread)
+  int left = (int)(m_end - m_begin);                                       // rows from there to the chunk's end
+  unsigned outside = 0;  // bit 2 p: this lane's row of pair p has no neighbour
+  __amdgpu_buffer_rsrc_t ra, rb;
+  auto resource = [](const float *p, int bytes) {  // wave-uniform, and said to be
+    const uint64_t at = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)at), hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32));
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>((uint64_t)hi << 32 | lo), 0,
+                                             __builtin_amdgcn_readfirstlane(bytes), 0x00027000);
+  };
+  auto next_block = [&]() {
+    if (conv) {
+      const bool in = ((unsigned)(ci + tu) < (unsigned)gh) & ((unsigned)(cj + tv) < (unsigned)gw) & ((unsigned)(cl + tz) < (unsigned)gd);
+      outside = ~(unsigned)__builtin_amdgcn_ballot_w64(in) >> g;
+      cl += step_l, cj += step_j, ci += step_i;
+      if (cl >= gd) cl -= gd, ++cj;
+      if (cj >= gw) cj -= gw, ++ci;
+      ci = (int)((unsigned)ci % (unsigned)gh);  // the next batch element; no loop: the loads in flight would be waited for
+    }
+    const int rows = left < 0 ? 0 : left < kF32Rows ? left : kF32Rows;
+    ra = resource(pa, rows * lda * 4), rb = resource(pb, rows * ldb * 4);
+    pa += (int64_t)kF32Rows * lda, pb += (int64_t)kF32Rows * ldb;
+    left -= kF32Rows;
+  };
+  auto request = [&](int p) {
+    av[p] = __builtin_amdgcn_raw_buffer_load_b64(ra, a_off + (unsigned)(8 * p * lda), 0, 0);
+    bv[p] = __builtin_amdgcn_raw_buffer_load_b64(rb, (b_off + (unsigned)(8 * p * ldb)) | ((outside << (31 - 2 * p)) & kOut), 0, 0);
+  };
+  next_block();
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    unsigned n = conv ? (unsigned)((m_begin + sr + 8 * k) % grid.N) : 0u;
-    cl[k] = (int)(n % gd);
-    n /= gd;
-    ci[k] = (int)(n / gw), cj[k] = (int)(n % gw);
+  for (int p = 0; p < kPairs; ++p) {
+    request(p);
+    __builtin_amdgcn_sched_barrier(0);  // in the order in which the loop waits for them
   }
-  auto fetch = [&](int64_t m0) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int64_t m = m0 + sr + 8 * k;
-      pa[k] = pb[k] = float4{0.f, 0.f, 0.f, 0.f};
-      if (m < m_end) {
-        if (oa0 + sc < OA) pa[k] = *reinterpret_cast<const float4 *>(A + m * lda + oa0 + sc);
-        const bool inside = !conv | (((unsigned)(ci[k] + tu) < (unsigned)gh) & ((unsigned)(cj[k] + tv) < (unsigned)gw) &
-                                     ((unsigned)(cl[k] + tz) < (unsigned)gd));
-        if (ob0 + sc < OB && inside) pb[k] = *reinterpret_cast<const float4 *>(B + (m + shift) * ldb + ob0 + sc);
-      }
-    }
-  };
-  auto advance = [&]() {  // the coordinates of the rows 32 further on
-    if (!conv) return;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      cl[k] += step_l, cj[k] += step_j, ci[k] += step_i;
-      if (cl[k] >= gd) cl[k] -= gd, ++cj[k];
-      if (cj[k] >= gw) cj[k] -= gw, ++ci[k];
-      while (ci[k] >= gh) ci[k] -= gh;  // the next batch element
-    }
-  };
-  auto stage = [&](int buf) {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      *reinterpret_cast<float4 *>(&As[buf][sr + 8 * k][sc]) = pa[k];
-      *reinterpret_cast<float4 *>(&Bs[buf][sr + 8 * k][sc]) = pb[k];
-    }
-  };
-  fetch(m_begin);
-  int buf = 0;
   for (int64_t m0 = m_begin; m0 < m_end; m0 += kF32Rows) {
-    stage(buf);
-    __syncthreads();
-    if (m0 + kF32Rows < m_end) advance();
-    fetch(m0 + kF32Rows < m_end ? m0 + kF32Rows : m0);  // the last block re-fetches itself: no branch around the loads
-#pragma unroll 4
-    for (int k = 0; k < kF32Rows; k += 2) {
-      const float a0 = As[buf][k + g][wa + i], a1 = As[buf][k + g][wa + 32 + i];
-      const float b0 = Bs[buf][k + g][wb + i], b1 = Bs[buf][k + g][wb + 32 + i];
+    next_block();  // behind the last one: no rows, every load a zero
+#pragma unroll
+    for (int p = 0; p < kPairs; ++p) {
+      const uint32_t w[4] = {av[p][0], av[p][1], bv[p][0], bv[p][1]};
+      const float a0 = __uint_as_float(w[0]), a1 = __uint_as_float(w[1]), b0 = __uint_as_float(w[2]), b1 = __uint_as_float(w[3]);
       acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b0, acc[0][0], 0, 0, 0);
       acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b1, acc[0][1], 0, 0, 0);
       acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b0, acc[1][0], 0, 0, 0);
       acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b1, acc[1][1], 0, 0, 0);
       csum[0] += a0;
       csum[1] += a1;
+      request(p);
+      __builtin_amdgcn_sched_barrier(0);  // the requests stay between the matrix instructions, a block ahead of their use
     }
-    buf ^= 1;
   }
-  // C/D layout: lane (i, g) holds column ob = i, register r holds row oa = rowmap(r, g)
+  // C/D layout: lane (i, g) holds column 2 i + v, register r holds row 2 rowmap(r, g) + u of the sub-block
   const int64_t ld = (int64_t)grid.taps * OB;
-  float *dst = partials + (int64_t)blockIdx.x * OA * ld + (int64_t)tap * OB;
+  const int row0 = oa0 + wa, rows = OA - row0 < 64 ? OA - row0 : 64;  // of the sub-block
+  if (rows > 0) {
+    const auto out = resource(partials + ((int64_t)chunk * OA + row0) * ld + (int64_t)tap * OB, (int)((rows - 1) * ld + OB) * 4);
+    const unsigned at = cb < OB ? (unsigned)cb * 4u : kOut, step = (unsigned)ld * 4u;
 #pragma unroll
-  for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < 2; ++u)
 #pragma unroll
-    for (int v = 0; v < 2; ++v) {
-      const int ob = ob0 + wb + 32 * v + i;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int oa = oa0 + wa + 32 * u + mfma::rowmap(r, g);
-        if (oa < OA && ob < OB) dst[(int64_t)oa * ld + ob] = acc[u][v][r];
-      }
-    }
-  if (col_sums && blockIdx.z == 0 && (wave >> 1) == 0) {
+      for (int r = 0; r < 16; ++r)  // rows beyond OA are out of range
+        __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(acc[u][0][r]), __float_as_uint(acc[u][1][r])}, out,
+                                              at + (unsigned)(2 * mfma::rowmap(r, g) + u) * step, 0, 0);
+  }
+  if (col_sums && zt == 0 && (wave >> 1) == 0) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const float total = csum[u] + __shfl_xor(csum[u], 32, 64);  // the two row parities
-      const int oa = oa0 + wa + 32 * u + i;
-      if (g == 0 && oa < OA) col_sums[(int64_t)blockIdx.x * OA + oa] = total;
+      if (g == 0 && ca < OA) col_sums[(int64_t)chunk * OA + ca + u] = total;
     }
   }
 }
@@ -599,10 +603,10 @@ int cols_gemm_f32(const void *A, int64_t lda, int64_t OA, const void *B, int64_t
   const int64_t G = cols_gemm_f32_chunks(M, OA, OB * grid_geom.taps, num_cu);
   int64_t per = (M + G - 1) / G;
   per = (per + kF32Rows - 1) / kF32Rows * kF32Rows;
-  const dim3 grid((unsigned)G, (unsigned)((OA + kF32Tile - 1) / kF32Tile),
-                  (unsigned)((OB + kF32Tile - 1) / kF32Tile * grid_geom.taps));
-  hipLaunchKernelGGL(cols_gemm_f32_kernel, grid, dim3(256), 0, st, static_cast<const float *>(A), (int)lda, (int)OA,
-                     static_cast<const float *>(B), (int)ldb, (int)OB, M, per, grid_geom, partials, col_sums);
+  const int64_t wgs = G * ((OA + kF32Tile - 1) / kF32Tile) * ((OB + kF32Tile - 1) / kF32Tile) * grid_geom.taps;
+  hipLaunchKernelGGL(cols_gemm_f32_kernel, dim3((unsigned)((wgs + 7) / 8 * 8)), dim3(256), 0, st, static_cast<const float *>(A),
+                     (int)lda, (int)OA, static_cast<const float *>(B), (int)ldb, (int)OB, M, per, (int)G, grid_geom, partials,
+                     col_sums);
   return launch_status();
 }
 

@@ -1480,3 +1480,38 @@ def test_fp32_layer_in_two_calls_against_float64(kind, dim, heads, dim_head, S, 
     for n, got in [("x", xr.grad)] + [(n, p.grad) for n, p in hip.named_parameters()]:
         err = (got.double() - want[n]).norm() / want[n].norm().clamp(min=1e-30)
         assert err <= (1.7e-5 if n == "temperature" else 6e-6), (n, err.item())
+
+
+@pytest.mark.parametrize("dtype,C,O", [(torch.float32, 128, 132), (torch.float32, 64, 256), (torch.bfloat16, 128, 256)])
+@pytest.mark.parametrize("grid,B", [((1, 1), 70), ((2, 3), 11), ((1, 31), 2), ((32, 1), 3), ((2, 2, 2), 9), ((3, 4, 5), 7)])
+def test_conv_weight_gradient_of_grids_within_a_block_of_rows(dtype, C, O, grid, B):
+    """Grids of fewer points than the 32 rows that a step advances by: several batch elements within one step."""
+    announce("conv weight gradient, tiny grids", dtype, C, O, grid, B)
+    torch.manual_seed(B)
+    N, k = int(np.prod(grid)), 3
+    g, x = torch.randn(B, N, O, device="cuda").to(dtype), torch.randn(B, N, C, device="cuda").to(dtype)
+    dims = PF.LayerDims(B, N, C, 4, 32, 32, grid[0], grid[1], k, grid[2] if len(grid) == 3 else 0, 1)
+    dw, db = PF.cols_gemm(g, x, col_sums=True, grid=dims)
+    w = torch.zeros(O, C, *(k,) * len(grid), dtype=torch.float64, requires_grad=True)
+    conv = torch.nn.functional.conv2d if len(grid) == 2 else torch.nn.functional.conv3d
+    conv(x.double().cpu().transpose(1, 2).reshape(B, C, *grid), w, padding=1).backward(
+        g.double().cpu().transpose(1, 2).reshape(B, O, *grid))
+    assert_fp32_close(dw, w.grad, "d weight")
+    assert_fp32_close(db, g.double().sum((0, 1)), "d bias")
+
+
+@pytest.mark.parametrize("rows,ca,cb", [(1, 128, 128), (33, 132, 64), (2015, 256, 128), (4129, 64, 260)])
+def test_float32_weight_gradient_with_infinities_at_the_ends_of_chunks(rows, ca, cb):
+    """What lies behind a chunk of rows, the next chunk's or nothing, reads as zero: an infinity in the last row stays in its
+    column and one in the first row does too."""
+    announce("float32 infinities", rows, ca, cb)
+    a, b = (1 + torch.rand(rows, c, device="cuda") for c in (ca, cb))
+    for row in (0, rows - 1):
+        for inf_in_a in (False, True):
+            x, y = a.clone(), b.clone()
+            (x if inf_in_a else y)[row, 5] = float("inf")
+            got, sums = PF.cols_gemm(x, y, col_sums=True)
+            want = torch.zeros(ca, cb, dtype=torch.bool, device="cuda")
+            (want[5] if inf_in_a else want[:, 5]).fill_(True)
+            assert not got.isnan().any() and torch.equal(got.isinf(), want)
+            assert not sums.isnan().any() and sums.isinf().sum() == int(inf_in_a)
