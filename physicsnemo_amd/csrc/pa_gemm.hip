@@ -645,33 +645,35 @@ int cols_gemm(const void *A, int64_t lda, int64_t OA, const void *B, int64_t ldb
 // ------------------------------------------------------------------------------------------------
 // conv_gemm_kernel: the grid convolutions as implicit GEMM (rows x taps * channels) . W^T with whole steps of 128 bytes of
 // channels (64 bf16, 32 float32) of one tap.  Workgroup: bf16 8 waves, 128 rows x 256 outputs, wave tile 64 x 64; float32
-// 4 waves, 64 x 128, wave tile 32 x 64 (two workgroups per CU).  One step of both operands (48 / 24 KB) is a stage; three
-// stages form a ring in LDS, filled two steps ahead by direct global -> LDS loads (the neighbours' rows are gathered by
-// their addresses, a unit of zeros outside the grid), one barrier per step.  The loads
+// 128 outputs, wave tile 32 x 64, 8 waves and 128 rows (TALL) or 4 and 64 (conv_tall() below).  One step of both operands (48, 32 or
+// 24 KB) is a stage; three, four or six stages form a ring in LDS, filled one stage less ahead by direct global -> LDS loads (the
+// neighbours' rows are gathered by their addresses, a unit of zeros outside the grid), one barrier per step.  The loads
 // write 8 rows of 128 bytes contiguously, so position p of row r holds the row's 16-byte unit p ^ (r % 8): the eight
 // lanes of an access phase then fall on all banks.
 // Outputs: rows as 16-byte pieces (the product formed as out^T, lanes <-> rows), or with `out_pack` the un-transposed
 // tile, in the packed operand layout and as 2-byte pieces of rows.
-// Bound by LDS reads (one 1 KB fragment per MFMA and wave: 128 bytes a cycle).  32 768 grid points, 3 x 3, 256 -> 2 x 256
-// and 512 -> 256 (77 GFLOP each): 105 and 96 us against 254 and 219 us of rows_gemm_mfma_kernel (registers one step ahead, two
-// barriers per step, no ring); 1 640 points: 40 and 75 us against 107 and 183.
+// bf16: bound by LDS reads (one 1 KB fragment per MFMA and wave: 128 bytes a cycle) and by issue.  32 768 grid points, 3 x 3, 256 -> 2 x
+// 256 and 512 -> 256 (77 GFLOP each): 79 us; 95 with a step's addresses formed in full (64-bit products) ahead of its matrix
+// instructions, 88 with them between these.  rows_gemm_mfma_kernel (registers one step ahead, two barriers per step, no ring): 254
+// and 219 us.
+// float32: bound by v_mfma_f32_32x32x2_f32 and by whole rounds of workgroups: 4 x 85 x 85 points, 128 -> 2 x 128 and 256 -> 128 (17
+// GFLOP each) 162 us against 177 (addresses in full, two 64-row workgroups of three stages per CU: the one that came second took 95 us,
+// the first 75); 57 600 points 322 against 348; 1 600 points 62 against 70.
 // ------------------------------------------------------------------------------------------------
-// float32 is bound by v_mfma_f32_32x32x2_f32 and by whole workgroups per CU: 4 x 85 x 85 points, 128 -> 2 x 128 and
-// 256 -> 128 (17 GFLOP each): 190 and 189 us against 227 and 242; 720 points: 50 and 93 against 192 and 217.
-constexpr int kConvStages = 3;
-template <typename T>
-struct ConvTile {  // waves: two along the rows, WC along the outputs; a wave stages 16 rows and 32 weight rows of a step
-  static constexpr int RT = sizeof(T) == 2 ? 2 : 1, WC = sizeof(T) == 2 ? 4 : 2, kWaves = 2 * WC;
-  static constexpr int kRows = 64 * RT, kOut = 64 * WC, kStageBytes = (kRows + kOut) * 128, KB = 128 / (int)sizeof(T);
+template <typename T, bool TALL>
+struct ConvTile {  // waves: WR along the rows, WC along the outputs; a wave stages 16 rows and OW weight rows of a step
+  static constexpr int RT = sizeof(T) == 2 ? 2 : 1, WR = sizeof(T) == 4 && TALL ? 4 : 2, WC = sizeof(T) == 2 ? 4 : 2, kWaves = WR * WC;
+  static constexpr int kRows = 32 * RT * WR, kOut = 64 * WC, kStageBytes = (kRows + kOut) * 128, KB = 128 / (int)sizeof(T);
+  static constexpr int OW = kOut / kWaves, kLoads = 2 + OW / 8, kStages = sizeof(T) == 2 ? 3 : TALL ? 4 : 6;
 };
 
-template <typename T>
-__global__ __launch_bounds__((ConvTile<T>::kWaves * 64)) void conv_gemm_kernel(GemmArgs a) {
-  using Q = ConvTile<T>;
-  constexpr int RT = Q::RT, UE = Unit<T>::kElems;
+template <typename T, bool TALL>
+__global__ __launch_bounds__((ConvTile<T, TALL>::kWaves * 64)) void conv_gemm_kernel(GemmArgs a) {
+  using Q = ConvTile<T, TALL>;
+  constexpr int RT = Q::RT, UE = Unit<T>::kElems, kConvStages = Q::kStages;
   extern __shared__ u32x4 ring[];  // [stage][kRows input rows | kOut weight rows] of 128 bytes
   const int z = blockIdx.z, t = threadIdx.x, lane = t & 63, i = lane & 31, g = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), wr = (wave & 1) * (32 * RT), wc = (wave >> 1) * 64;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), wr = wave % Q::WR * (32 * RT), wc = wave / Q::WR * 64;
   const T *in = static_cast<const T *>(a.in);
   const int64_t m0 = (int64_t)blockIdx.x * Q::kRows;
   const int o0 = blockIdx.y * Q::kOut;
@@ -684,9 +686,10 @@ __global__ __launch_bounds__((ConvTile<T>::kWaves * 64)) void conv_gemm_kernel(G
     const int64_t end = tpb && (int64_t)(b + 1) * a.N < a.M ? (int64_t)(b + 1) * a.N : a.M, left = end - first;
     count = left < 0 ? 0 : left < 32 ? (int)left : 32;
   };
-  // this wave stages input rows 16 wave + 8 k + lane / 8 (k = 0, 1) and weight rows 32 wave + 8 k + lane / 8 (k = 0 .. 3)
+  // this wave stages input rows 16 wave + 8 k + lane / 8 (k = 0, 1) and weight rows OW wave + 8 k + lane / 8
   const int unit = (lane & 7) ^ (lane >> 3);
-  const T *base[2], *wp = static_cast<const T *>(a.w[z]) + (int64_t)(o0 + 32 * wave + (lane >> 3)) * a.K + UE * unit;
+  const T *base[2], *wu = static_cast<const T *>(a.w[z]) + (int64_t)(o0 + Q::OW * wave) * a.K;  // wu: wave-uniform
+  const int w_off = ((lane >> 3) * a.K + UE * unit) * (int)sizeof(T);
   int ci[2], cj[2], cl[2];
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
@@ -704,30 +707,52 @@ __global__ __launch_bounds__((ConvTile<T>::kWaves * 64)) void conv_gemm_kernel(G
   }
   const int nkb = a.K / Q::KB, cblocks = a.C / Q::KB;
   int fu = 0, fv = 0, fz = 0, fc = 0;  // tap and channel block of the step fetched next
-  auto fetch = [&](int kb) {           // past the last step: that one again, so that every step counts six loads
-    const unsigned dst = (unsigned)(uintptr_t)ring + (unsigned)(kb % kConvStages) * Q::kStageBytes;
-    const int64_t shift = (((int64_t)(fu - pad) * a.gw + fv - pad) * gd + fz - pad_d) * a.C + Q::KB * fc;  // the neighbour, from the row
+  // The addresses of a step are the ones before it plus 128 bytes, but at a new tap: formed in full at every step, 64-bit products
+  // included, they cost as much issue time as the matrix instructions between which they stood.
+  const char *xp[2];
+  int x_step[2];
+  auto enter_tap = [&]() {
+    const int64_t shift = (((int64_t)(fu - pad) * a.gw + fv - pad) * gd + fz - pad_d) * a.C;  // the neighbour, from the row
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const bool ok = ((unsigned)(ci[k] + fu - pad) < (unsigned)a.gh) & ((unsigned)(cj[k] + fv - pad) < (unsigned)a.gw) &
                       ((unsigned)(cl[k] + fz - pad_d) < (unsigned)gd);
-      const T *p = ok ? base[k] + shift : reinterpret_cast<const T *>(&mfma::kZeroUnit);
-      mfma::load_unit_to_lds(p, dst + (16 * wave + 8 * k) * 128);
+      xp[k] = ok ? reinterpret_cast<const char *>(base[k] + shift) : reinterpret_cast<const char *>(&mfma::kZeroUnit);
+      x_step[k] = ok ? 128 : 0;
     }
+  };
+  enter_tap();
+  const unsigned ring0 = (unsigned)(uintptr_t)ring;
+  unsigned slot = 0;  // of the ring, in bytes: where the next step goes
+  // a step's loads in four parts between the matrix instructions; past the last step: that one again, so that every step counts as
+  // many loads
+  auto fetch_part = [&](int kb, auto part_) {
+    constexpr int part = decltype(part_)::value;
+    const unsigned dst = ring0 + slot;
+    if constexpr (part < 2) {
+      mfma::load_unit_to_lds(xp[part], dst + (16 * wave + 8 * part) * 128);
+    } else {
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-      mfma::load_unit_to_lds(wp + (int64_t)8 * k * a.K, dst + Q::kRows * 128 + (32 * wave + 8 * k) * 128);
-    if (kb + 1 < nkb) {
-      wp += Q::KB;
-      if (++fc == cblocks) {
-        fc = 0;
-        if (++fz == ksd) {
-          fz = 0;
-          if (++fv == a.ks) fv = 0, ++fu;
+      for (int k = 2 * part - 4; k < 2 * part - 2 && k < Q::OW / 8; ++k)
+        mfma::load_unit_to_lds(wu + (int64_t)8 * k * a.K, w_off, dst + Q::kRows * 128 + (Q::OW * wave + 8 * k) * 128);
+    }
+    if constexpr (part == 3) {
+      slot = slot == (kConvStages - 1) * Q::kStageBytes ? 0 : slot + Q::kStageBytes;
+      if (kb + 1 < nkb) {
+        wu += Q::KB;
+        xp[0] += x_step[0], xp[1] += x_step[1];
+        if (++fc == cblocks) {
+          fc = 0;
+          if (++fz == ksd) {
+            fz = 0;
+            if (++fv == a.ks) fv = 0, ++fu;
+          }
+          enter_tap();
         }
       }
     }
   };
+  auto fetch = [&](int kb) { mfma::static_for<4>([&](auto part) { fetch_part(kb, part); }); };
   f32x16 acc[2][RT];  // [output tile][row tile]
 #pragma unroll
   for (int u = 0; u < 2; ++u)
@@ -739,27 +764,33 @@ __global__ __launch_bounds__((ConvTile<T>::kWaves * 64)) void conv_gemm_kernel(G
   const int row_off = i * 8, swz = i & 7;
   auto multiply = [&](auto turned_) {
     constexpr bool turned = decltype(turned_)::value;
-    fetch(0);
-    fetch(1);
+    mfma::static_for<kConvStages - 1>([&](auto s) { fetch(decltype(s)::value); });
+    unsigned at_slot = 0;
     for (int kb = 0; kb < nkb; ++kb) {
-      asm volatile("s_waitcnt vmcnt(6)" ::: "memory");  // this wave's share of the step; the next one stays in flight
+      // this wave's share of the step; the younger ones stay in flight
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kConvStages - 2) * Q::kLoads) : "memory");
       __syncthreads();
-      fetch(kb + 2);  // into the stage multiplied one step ago, which every wave is past
-      const u32x4 *xs = ring + (kb % kConvStages) * (Q::kStageBytes / 16) + wr * 8 + row_off;
-      const u32x4 *ws = ring + (kb % kConvStages) * (Q::kStageBytes / 16) + (Q::kRows + wc) * 8 + row_off;
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
+      const u32x4 *xs = ring + at_slot / 16 + wr * 8 + row_off, *ws = ring + at_slot / 16 + (Q::kRows + wc) * 8 + row_off;
+      at_slot = at_slot == (kConvStages - 1) * Q::kStageBytes ? 0 : at_slot + Q::kStageBytes;
+      u32x4 w[2][2], x[2][RT];  // a unit's operands, one unit ahead
+      auto read = [&](int ks) {
         const int at = (2 * ks + g) ^ swz;
-        const u32x4 w[2] = {ws[at], ws[32 * 8 + at]};
-        u32x4 x[RT];
+        w[ks & 1][0] = ws[at], w[ks & 1][1] = ws[32 * 8 + at];
 #pragma unroll
-        for (int v = 0; v < RT; ++v) x[v] = xs[32 * 8 * v + at];
+        for (int v = 0; v < RT; ++v) x[ks & 1][v] = xs[32 * 8 * v + at];
+      };
+      read(0);
+      mfma::static_for<4>([&](auto ks_) {
+        constexpr int ks = decltype(ks_)::value;
+        if constexpr (ks < 3) read(ks + 1);
+        if constexpr (sizeof(T) == 4) __builtin_amdgcn_sched_barrier(0);  // bf16: 84 us so, 79 without
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
           for (int v = 0; v < RT; ++v)
-            acc[u][v] = turned ? mma_unit(in, w[u], x[v], acc[u][v]) : mma_unit(in, x[v], w[u], acc[u][v]);
-      }
+            acc[u][v] = turned ? mma_unit(in, w[ks & 1][u], x[ks & 1][v], acc[u][v]) : mma_unit(in, x[ks & 1][v], w[ks & 1][u], acc[u][v]);
+        fetch_part(kb + kConvStages - 1, ks_);  // into the stage multiplied one step ago, which every wave is past
+      });
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be landing in LDS when the workgroup ends
   };
@@ -816,22 +847,30 @@ __global__ __launch_bounds__((ConvTile<T>::kWaves * 64)) void conv_gemm_kernel(G
 // whole steps of one tap, whole workgroups of outputs; weights in the reduction's order
 template <typename T>
 static bool conv_serves(const GemmArgs &a, int nsets) {
-  using Q = ConvTile<T>;
+  using Q = ConvTile<T, false>;
   if (a.ks <= 0 || a.act != 0 || !a.w_tap_major || a.C % Q::KB != 0 || a.O % Q::kOut != 0 || a.K < 2 * Q::KB) return false;
   for (int z = 0; z < nsets; ++z)
     if (a.out_pack[z] ? sizeof(T) != 2 : !aligned16(a.out[z])) return false;
   return true;
 }
 
-template <typename T>
+template <typename T, bool TALL>
 static int conv_launch(const GemmArgs &a, int nsets, hipStream_t st) {
-  using Q = ConvTile<T>;
+  using Q = ConvTile<T, TALL>;
   const int64_t rows = a.pack_tpb > 0 ? (a.M / a.N) * a.pack_tpb * 32 : a.M;
-  const size_t lds = (size_t)kConvStages * Q::kStageBytes;
-  if (int rc = allow_dynamic_lds(conv_gemm_kernel<T>, lds)) return rc;
+  const size_t lds = (size_t)Q::kStages * Q::kStageBytes;
+  auto kernel = conv_gemm_kernel<T, TALL>;
+  if (int rc = allow_dynamic_lds(kernel, lds)) return rc;
   const dim3 grid((unsigned)((rows + Q::kRows - 1) / Q::kRows), (unsigned)(a.O / Q::kOut), (unsigned)nsets);
-  hipLaunchKernelGGL(conv_gemm_kernel<T>, grid, dim3(Q::kWaves * 64), lds, st, a);
+  hipLaunchKernelGGL(kernel, grid, dim3(Q::kWaves * 64), lds, st, a);
   return launch_status();
+}
+
+// float32: one workgroup per CU in either form, so a round of 128-row workgroups takes twice the matrix time of a round of 64-row
+// ones, 10 % behind that rate with its two waves per SIMD against 20 % with one: whichever needs less for its whole rounds.
+static bool conv_tall(const GemmArgs &a, int nsets) {
+  const int64_t cols = a.O / 128 * nsets, tall = ((a.M + 127) / 128 * cols + 255) / 256, flat = ((a.M + 63) / 64 * cols + 255) / 256;
+  return 2 * 11 * tall <= 12 * flat;
 }
 
 bool serves(const GemmArgs &a, int nsets, size_t elem_bytes) {
@@ -871,8 +910,9 @@ int launch(const GemmArgs &a, int nsets, int dtype, hipStream_t st) {
       cus = 256;
     return linear_launch(a, nsets, cus, st);
   }
-  if (dtype == PA_BF16 && conv_serves<bf16>(a, nsets)) return conv_launch<bf16>(a, nsets, st);
-  if (dtype == PA_F32 && conv_serves<float>(a, nsets)) return conv_launch<float>(a, nsets, st);
+  if (dtype == PA_BF16 && conv_serves<bf16>(a, nsets)) return conv_launch<bf16, false>(a, nsets, st);
+  if (dtype == PA_F32 && conv_serves<float>(a, nsets))
+    return conv_tall(a, nsets) ? conv_launch<float, true>(a, nsets, st) : conv_launch<float, false>(a, nsets, st);
   return dtype == PA_F32 ? launch_n<float>(a, nsets, st) : launch_n<bf16>(a, nsets, st);
 }
 

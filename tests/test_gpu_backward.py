@@ -1515,3 +1515,17 @@ def test_float32_weight_gradient_with_infinities_at_the_ends_of_chunks(rows, ca,
             (want[5] if inf_in_a else want[:, 5]).fill_(True)
             assert not got.isnan().any() and torch.equal(got.isinf(), want)
             assert not sums.isnan().any() and sums.isinf().sum() == int(inf_in_a)
+
+
+@pytest.mark.parametrize("grid,C,O,B", [((110, 140), 32, 256, 1), ((60, 57), 64, 128, 10), ((101, 63), 96, 128, 2)])
+def test_float32_convolution_in_tall_and_flat_tiles(grid, C, O, B):
+    """Row counts on either side of the rule between 128 and 64 rows a workgroup, one to three steps per tap: against float64, to
+    the rounding of the sums (as above)."""
+    announce("float32 conv tiles", grid, C, O, B)
+    torch.manual_seed(C)
+    N = int(np.prod(grid))
+    dims = PF.LayerDims(B, N, C, O // 32, 32, 32, grid[0], grid[1], 3, 0, 1)
+    x, w = torch.randn(B, N, C, device="cuda"), torch.randn(O, C, 3, 3, device="cuda") / (9 * C) ** 0.5
+    got = PF.rows_gemm(x, w.movedim(1, -1).contiguous(), None, dims, C, O)
+    want = torch.nn.functional.conv2d(x.double().transpose(1, 2).reshape(B, C, *grid).cpu(), w.double().cpu(), padding=1)
+    assert_rel_l2(got, want.reshape(B, O, N).transpose(1, 2), "conv", tol=4e-6)
