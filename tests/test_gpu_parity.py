@@ -499,3 +499,20 @@ def test_slice_sums_over_groups_of_threads(dtype, S, D, N):
     want = torch.einsum("bnhs,bnhd->bhsd", w.double(), f.double().view(B, N, H, D)) / count[..., None]
     assert_rel_l2(norm, count, "norm", tol=1.5e-5)
     assert_rel_l2(tok, want, "tokens", tol=1.5e-5)
+
+
+@pytest.mark.parametrize("C,H", [(64, 4), (64, 8), (32, 4), (32, 2)])
+@pytest.mark.parametrize("B,N", [(1, 1), (3, 15), (1, 17), (2, 65), (1, 129), (5, 3277), (4, 4097), (2, 33000)])
+def test_fp32_narrow_block_at_the_edges_of_its_tiles(C, H, B, N):
+    """Tiles of 16 points, workgroups of four and of eight waves, one and several tiles per wave: rows of any count against the
+    float64 block.  1e-6: some tens of float32 roundings (2^-24 each) per value."""
+    announce("fp32 narrow block, edges", C, H, B, N)
+    torch.manual_seed(N)
+    ref = to.OracleTransolverBlock(H, C, mlp_ratio=1, slice_num=32).eval()
+    hip = pn.TransolverBlock(H, C, 0.0, mlp_ratio=1, slice_num=32, use_te=False).eval()
+    hip.load_state_dict(ref.state_dict())
+    hip, ref = hip.cuda(), ref.double().cuda()
+    x = torch.randn(B, N, C, device="cuda")
+    with torch.no_grad():
+        got, want = hip(x), ref(x.double())
+    assert to.rel_l2(got.double(), want) < 1e-6
