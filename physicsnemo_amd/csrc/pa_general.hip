@@ -644,7 +644,8 @@ __global__ __launch_bounds__(kAttnThreads) void slice_combine_attn_kernel(const 
 // narrow_combine_attn_kernel<D>: combine_partials_kernel and slice_combine_attn_kernel in one launch for narrow heads, with
 // their sums in their order, bit for bit: 32 threads per slice, everything of a (b, h) in registers and LDS, sizes known to
 // the compiler.  Bound by latency: one trip for partials and weights, four barriers.  D = 16, S = 32 (us, the two launches before ->
-// now): 16 workgroups of 128 partials 4.5 + 11.0 -> 9.4, 32 of 64 partials 4.8 + 10.6 -> 7.0.
+// now): 16 workgroups of 97 partials 4.5 + 11.0 -> 7.5, of 63 partials 5.9 (with one sum at a time instead of four neighbouring ones
+// 9.5 and 6.5).
 // ------------------------------------------------------------------------------------------------
 constexpr int kNarrowSlices = 32;
 
@@ -654,27 +655,28 @@ __global__ __launch_bounds__(32 * kNarrowSlices) void narrow_combine_attn_kernel
                                                                     float *__restrict__ slice_token,
                                                                     float *__restrict__ slice_norm,
                                                                     float *__restrict__ out_token) {
-  constexpr int S = kNarrowSlices, T = 32 * S, D1 = D + 1, LD = D + 4, NOUT = S * D1, kAhead = 16;
+  constexpr int S = kNarrowSlices, T = 32 * S, D1 = D + 1, LD = D + 4, NOUT = S * D1, NQ = NOUT / 4, kParts = 4, kAhead = 16;
   static_assert(S == 2 * 16 && D % 4 == 0, "16 threads per slice in the softmax, two keys each; whole float4 rows");
-  __shared__ float quarter[4][NOUT];
+  __shared__ __align__(16) float part[kParts][NOUT];
   __shared__ __align__(16) float tok[S * LD], wq[3 * D * LD], qkv[3][S * LD], prob[S * (S + 1)];
   const int t = threadIdx.x, bh = blockIdx.x;
   float w[(3 * D * D + T - 1) / T];
 #pragma unroll
   for (int k = 0; k < (3 * D * D + T - 1) / T; ++k) w[k] = k * T + t < 3 * D * D ? w_qkv[k * T + t] : 0.f;
-  const int per = (G + 3) / 4;
-  const float *src = partials + (int64_t)bh * NOUT;
-  for (int item = t; item < 4 * NOUT; item += T) {  // kAhead loads in flight, added in index order
-    const int qt = item / NOUT, o = item - qt * NOUT, g0 = qt * per, g1 = min(G, g0 + per);
-    float acc = 0.f;
+  // a thread adds up four neighbouring sums of a quarter of the partials in index order, kAhead of them in flight: one trip for 64
+  const int per = (G + kParts - 1) / kParts, pt = t / NQ, o4 = t - pt * NQ, g0 = pt * per, g1 = min(G, g0 + per);
+  if (pt < kParts) {
+    const float4 *src = reinterpret_cast<const float4 *>(partials + (int64_t)bh * NOUT) + o4;  // NOUT and the stride: whole float4
+    float4 acc{0.f, 0.f, 0.f, 0.f};
     for (int g = g0; g < g1; g += kAhead) {
-      float v[kAhead];
+      float4 v[kAhead];
 #pragma unroll
-      for (int u = 0; u < kAhead; ++u) v[u] = src[(int64_t)min(g + u, g1 - 1) * partial_stride + o];
+      for (int u = 0; u < kAhead; ++u) v[u] = src[(int64_t)min(g + u, g1 - 1) * (partial_stride / 4)];
 #pragma unroll
-      for (int u = 0; u < kAhead; ++u) acc += g + u < g1 ? v[u] : 0.f;
+      for (int u = 0; u < kAhead; ++u)
+        if (g + u < g1) acc.x += v[u].x, acc.y += v[u].y, acc.z += v[u].z, acc.w += v[u].w;
     }
-    quarter[qt][o] = acc;
+    reinterpret_cast<float4 *>(part[pt])[o4] = acc;
   }
 #pragma unroll
   for (int k = 0; k < (3 * D * D + T - 1) / T; ++k) {
@@ -682,7 +684,7 @@ __global__ __launch_bounds__(32 * kNarrowSlices) void narrow_combine_attn_kernel
     if (i < 3 * D * D) wq[(i / D) * LD + i % D] = w[k];
   }
   __syncthreads();
-  auto total = [&](int o) { return ((quarter[0][o] + quarter[1][o]) + quarter[2][o]) + quarter[3][o]; };
+  auto total = [&](int o) { return ((part[0][o] + part[1][o]) + part[2][o]) + part[3][o]; };
   for (int i = t; i < S * D; i += T) {
     const int s = i / D, d = i % D;
     const float cnt = total(s * D1 + D) + kSliceNormEps, val = total(s * D1 + d) / cnt;
