@@ -176,6 +176,16 @@ int64_t pa_reduce_partial_count(const pa_shape *shape);
 int pa_slice_reduce(int dtype, const pa_shape *shape, const void *w, const void *fx_mid, float *partials,
                     float *slice_token, float *slice_norm, void *stream);
 
+/* Stages (a) and (b) of a layer whose input has few channels, in one pass over x: slice tokens and norms as
+ * pa_project_inputs, pa_slice_softmax and pa_slice_reduce give them, without x_mid, fx_mid and w in memory.
+ * PA_BF16, conv_k = 0, C <= 16, D = 32, S = 16, 32 or 64, H <= 8 or a multiple of 8; for other shapes
+ * pa_thin_tokens_partial_count returns 0 and pa_thin_tokens PA_ERR_UNSUPPORTED.
+ *   partials: float32 scratch of pa_thin_tokens_partial_count(dtype, shape) * B*H*S*(D+1) elements
+ * Of `p` the three input projections and the temperature are read.  Fixed order (bit-reproducible, no atomics). */
+int64_t pa_thin_tokens_partial_count(int dtype, const pa_shape *shape);
+int pa_thin_tokens(int dtype, const pa_shape *shape, const pa_params *p, const void *x, float *partials,
+                   float *slice_token, float *slice_norm, void *stream);
+
 /* Stage (b) without any device allocation and without a workspace argument.  No counterpart in the reference: it is
  * for callers that cannot allocate device memory -- code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc.  Same kernels, same arguments and bit-identical results as pa_slice_reduce; the per-chunk

@@ -17,7 +17,7 @@ PA_F32, PA_BF16, PA_BF16_W8 = 0, 1, 2
 
 EXPORTED = [
     "pa_version", "pa_set_compute_units", "pa_status_string", "pa_workspace_bytes", "pa_query_path", "pa_project_inputs",
-    "pa_slice_softmax", "pa_reduce_partial_count", "pa_slice_reduce", "pa_slice_attention",
+    "pa_slice_softmax", "pa_reduce_partial_count", "pa_slice_reduce", "pa_thin_tokens_partial_count", "pa_thin_tokens", "pa_slice_attention",
     "pa_deslice_project", "pa_layer_forward", "pa_mfma_buffer_bytes", "pa_mfma_pack_params",
     "pa_mfma_project_softmax", "pa_mfma_slice_reduce", "pa_mfma_project_softmax_reduce", "pa_mfma_partial_groups",
      "pa_mfma_combine_attention", "pa_mfma_deslice_project", "pa_mlp_query", "pa_mlp_workspace_bytes", "pa_mlp_forward", "pa_mlp_pack", "pa_mlp_pack_e4m3", "pa_mlp_input_ln_query", "pa_mlp_forward_packed_ln",
@@ -129,6 +129,10 @@ def load() -> ctypes.CDLL:
     lib.pa_reduce_partial_count.argtypes = [ps]
     lib.pa_slice_reduce.restype = c_int
     lib.pa_slice_reduce.argtypes = [c_int, ps, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]
+    lib.pa_thin_tokens_partial_count.restype = c_int64
+    lib.pa_thin_tokens_partial_count.argtypes = [c_int, ps]
+    lib.pa_thin_tokens.restype = c_int
+    lib.pa_thin_tokens.argtypes = [c_int, ps, pp, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]
     lib.pa_static_scratch_bytes.restype = c_int64
     lib.pa_static_scratch_bytes.argtypes = []
     lib.pa_slice_reduce_static.restype = c_int

@@ -113,6 +113,10 @@ class _SliceToContextMixin:
                 st.slice_reduce()
             st.combine_attention()
             return st.tok
+        if not self.plus:  # few input channels: one pass over x instead of x_mid, fx_mid and the weights through memory
+            tokens = PF.thin_tokens(x, p, dims)
+            if tokens is not None:
+                return tokens[0]
         x_mid, fx_mid = PF.project_inputs(x, p, dims)
         if self.plus:
             u = torch.rand((dims.B, dims.N, dims.H, dims.S), dtype=x.dtype, device=x.device)

@@ -458,6 +458,31 @@ int pa_slice_reduce(int dtype, const pa_shape *shape, const void *w, const void 
                                         slice_norm, nullptr, st);
 }
 
+int64_t pa_thin_tokens_partial_count(int dtype, const pa_shape *shape) {
+  int rc = check_shape(dtype, shape);
+  if (rc) return rc;
+  if (dtype != PA_BF16 || !pa::mfma::thin_tokens_supported(*shape)) return 0;
+  return pa::mfma::softmax_reduce_groups(*shape, compute_units()) + 1;
+}
+
+int pa_thin_tokens(int dtype, const pa_shape *shape, const pa_params *p, const void *x, float *partials,
+                   float *slice_token, float *slice_norm, void *stream) {
+  int rc = check_shape(dtype, shape);
+  if (rc) return rc;
+  if (dtype != PA_BF16 || !pa::mfma::thin_tokens_supported(*shape)) return PA_ERR_UNSUPPORTED;
+  if (!p || !p->in_project_x_weight || !p->in_project_x_bias || !p->in_project_fx_weight || !p->in_project_fx_bias ||
+      !p->in_project_slice_weight || !p->in_project_slice_bias || !p->temperature)
+    return PA_ERR_NULL;
+  if (!x || !partials || !slice_token || !slice_norm) return PA_ERR_NULL;
+  if (!aligned16(x) || !aligned16(partials) || !aligned16(p->in_project_x_weight) || !aligned16(p->in_project_fx_weight))
+    return PA_ERR_ALIGN;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if ((rc = pa::mfma::thin_tokens(*shape, *p, x, partials, compute_units(), st))) return rc;
+  pa_params none{};
+  return pa::general::combine_attention(*shape, none, partials, pa::mfma::softmax_reduce_groups(*shape, compute_units()),
+                                        slice_token, slice_norm, nullptr, st);
+}
+
 int pa_slice_attention(const pa_shape *shape, const pa_params *p, const float *slice_token, float *out_slice_token,
                        void *stream) {
   int rc = check_shape(PA_F32, shape);

@@ -278,6 +278,9 @@ int64_t softmax_reduce_groups(const pa_shape &s, int num_cu);
 // packed_x: x_mid (and out_x) are packed operand tiles [tile][head][2][64 lanes] of 16 bytes instead of rows
 int slice_softmax_reduce(const pa_shape &s, const pa_params &p, const void *x_mid, bool packed_x, const void *fx_pack,
                          float *partials, int num_cu, hipStream_t st);
+// token sums of inputs with few channels, straight from x (softmax_reduce_groups partials)
+bool thin_tokens_supported(const pa_shape &s);
+int thin_tokens(const pa_shape &s, const pa_params &p, const void *x, float *partials, int num_cu, hipStream_t st);
 int deslice_recompute(const pa_shape &s, const pa_params &p, const void *x_mid, bool packed_x, const void *tokp,
                       void *out_x, int num_cu, hipStream_t st);
 bool backward_supported(const pa_shape &s);

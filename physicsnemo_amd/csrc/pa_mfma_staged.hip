@@ -313,6 +313,122 @@ __global__ __launch_bounds__(512) void slice_softmax_reduce_kernel(const uint16_
 }
 
 // ------------------------------------------------------------------------------------------------
+// thin_tokens_kernel: slice-token sums of inputs with few channels (coordinates, global quantities; C <= 16, one k
+// step) in one pass over x: both projections, the slice weights and the first pass of the sums, one wave per head as in
+// slice_softmax_reduce_kernel.  grid (G, B, head groups).
+//   x_mid^T (32 d x 32 pts) = W_x . x^T + b_x       (its bf16 halves are the logits' B operands, k in kperm order)
+//   fx_mid  (32 pts x 32 d) = x . W_fx^T + b_fx     (its bf16 halves are the token sums' A operands: k = points)
+// and from there on the arithmetic of that kernel, with W_slice as two bf16 halves (it is float32 where the stages run one
+// by one).  x_mid, fx_mid, the weights and the token sums are rounded where those stages round them: the first three to
+// bf16, the sums not.
+// What bounds it: the softmax's vector work, S/2 exponentials a lane and tile.  Stage by stage the same work wrote and
+// read 2 x 2 HD + 6 HS bytes a point that it forms here in registers: 65 536 points of 3 channels, 8 heads, 64 slices,
+// with the sum of the partials 259 -> 38 us (of it 20 for the tiles, 3 a launch); 8 points of 16 channels 43 -> 12.
+// ------------------------------------------------------------------------------------------------
+template <int S>
+__global__ __launch_bounds__(512) void thin_tokens_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w_x,
+                                                          const float *__restrict__ b_x,
+                                                          const uint16_t *__restrict__ w_fx,
+                                                          const float *__restrict__ b_fx,
+                                                          const float *__restrict__ w_slice,
+                                                          const float *__restrict__ b_slice,
+                                                          const float *__restrict__ temperature,
+                                                          float *__restrict__ partials, int64_t N, int tpb, int C, int H) {
+  constexpr int ST = (S + 31) / 32, NCH = S / 16, D1 = 33;
+  __shared__ u32x4 wsl[2 * ST * 2 * 64];
+  __shared__ float bsl[ST * 32], bxs[8 * 32];
+  const int tid = threadIdx.x, lane = tid & 63, i = lane & 31, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = blockIdx.z * (blockDim.x >> 6) + wave;
+  const int b = blockIdx.y;
+  // channels 8 g .. 8 g + 7 of a row, zeros from channel C on; a load past the row reads its first channel instead
+  const bool whole = C % 8 == 0;  // rows are whole 16-byte units
+  const int c0 = 8 * g;
+  auto row_part = [&](const uint16_t *row) {
+    u32x4 out = {0u, 0u, 0u, 0u};
+    if (whole) {
+      const u32x4 v = *reinterpret_cast<const u32x4 *>(row + (c0 < C ? c0 : 0));
+      if (c0 < C) out = v;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (j < C) {  // the same for all lanes: the lower half's channel
+          const int c = c0 + j;
+          const uint32_t v = row[c < C ? c : 0];
+          out[j >> 1] |= (c < C ? v : 0u) << (16 * (j & 1));
+        }
+    }
+    return out;
+  };
+  const u32x4 wx = row_part(w_x + (int64_t)(h * 32 + i) * C), wf = row_part(w_fx + (int64_t)(h * 32 + i) * C);
+  if (lane < 32) bxs[wave * 32 + lane] = b_x[h * 32 + lane];  // in LDS: 16 registers a lane otherwise
+  const float bf = b_fx[h * 32 + i];
+  stage_slice_projection<S, true, true>(w_slice, b_slice, wsl, bsl);
+  __syncthreads();
+  const float sc = kLog2e / clamp_temperature(temperature[h]);
+  u32x4 sel[2];
+#pragma unroll
+  for (int par = 0; par < 2; ++par) {
+    bf16x8 s8;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s8[j] = (__bf16)((i == kperm(par, g, j)) ? 1.f : 0.f);
+    sel[par] = __builtin_bit_cast(u32x4, s8);
+  }
+  f32x16 tok[ST];
+  float nrm[ST];
+#pragma unroll
+  for (int st = 0; st < ST; ++st) {
+    nrm[st] = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) tok[st][r] = 0.f;
+  }
+  const uint16_t *xb = x + (int64_t)b * N * C;
+  auto fetch = [&](int t) {  // rows past the last one re-read it; their weights are zero
+    const int64_t n = (int64_t)t * 32 + i;
+    return row_part(xb + (n < N ? n : N - 1) * C);
+  };
+  u32x4 xr = fetch(blockIdx.x);  // the grid is no larger than the number of tiles
+  for (int t = blockIdx.x; t < tpb; t += gridDim.x) {
+    const bool valid = (int64_t)t * 32 + i < N;
+    f32x16 ax, af;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) ax[r] = bxs[wave * 32 + rowmap(r, g)], af[r] = bf;
+    ax = mma(wx, xr, ax);
+    af = mma(xr, wf, af);
+    const u32x4 xm0 = pack_half<0>(ax), xm1 = pack_half<1>(ax), f0 = pack_half<0>(af), f1 = pack_half<1>(af);
+    if (t + (int)gridDim.x < tpb) xr = fetch(t + gridDim.x);  // the next tile's rows under this one's softmax
+    u32x4 chunk[NCH];
+    slice_weights_of_tile<S, false, true>(wsl, bsl, xm0, xm1, sc, valid, lane, g, chunk);
+#pragma unroll
+    for (int st = 0; st < ST; ++st) {
+      f32x16 tr;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) tr[r] = 0.f;
+      tr = mma(chunk[2 * st], sel[0], tr);
+      if (2 * st + 1 < NCH) tr = mma(chunk[2 * st + 1 < NCH ? 2 * st + 1 : 0], sel[1], tr);
+      float s16 = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s16 += tr[r];
+      nrm[st] += s16;
+      // a B operand's k half 0 is the points 0-15 in kperm order, and so is f0's
+      tok[st] = mma(f0, pack_half<0>(tr), tok[st]);
+      tok[st] = mma(f1, pack_half<1>(tr), tok[st]);
+    }
+  }
+  float *dst = partials + (((int64_t)blockIdx.x * gridDim.y + b) * H + h) * (S * D1);
+#pragma unroll
+  for (int st = 0; st < ST; ++st) {
+    const int s = 32 * st + i;
+    const float total = half_sum(nrm[st]);
+    if (s < S) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dst[s * D1 + rowmap(r, g)] = tok[st][r];
+      if (g == 0) dst[s * D1 + 32] = total;
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
 // deslice_recompute_kernel: the attended tokens back to the points, slice weights recomputed from x_mid.
 // grid (G, B, head groups), one wave per head of the group;
 //   out_x^T_h (32 d x 32 pts) = tok'^T_h (A: tokp fragments, registers) . w_h (B: the chunks)
@@ -487,6 +603,31 @@ int slice_softmax_reduce(const pa_shape &s, const pa_params &p, const void *x_mi
   }
 #undef PA_LAUNCH_SSR
 #undef PA_LAUNCH_SSR1
+  return launch_status();
+}
+
+// bf16 layers of 32-channel heads on inputs of at most 16 channels
+bool thin_tokens_supported(const pa_shape &s) {
+  return s.conv_k == 0 && s.C <= 16 && s.D == 32 && (s.S == 16 || s.S == 32 || s.S == 64) && (s.H <= 8 || s.H % 8 == 0);
+}
+
+int thin_tokens(const pa_shape &s, const pa_params &p, const void *x, float *partials, int num_cu, hipStream_t st) {
+  dim3 grid, block;
+  recompute_grid(s, num_cu, &grid, &block);
+  const int tpb = (int)tiles_per_batch(s);
+#define PA_LAUNCH_TT(SS)                                                                                               \
+  hipLaunchKernelGGL((thin_tokens_kernel<SS>), grid, block, 0, st, static_cast<const uint16_t *>(x),                   \
+                     static_cast<const uint16_t *>(p.in_project_x_weight), p.in_project_x_bias,                        \
+                     static_cast<const uint16_t *>(p.in_project_fx_weight), p.in_project_fx_bias,                      \
+                     p.in_project_slice_weight, p.in_project_slice_bias, p.temperature, partials, s.N, tpb, (int)s.C,  \
+                     (int)s.H)
+  switch (s.S) {
+    case 16: PA_LAUNCH_TT(16); break;
+    case 32: PA_LAUNCH_TT(32); break;
+    case 64: PA_LAUNCH_TT(64); break;
+    default: return PA_ERR_UNSUPPORTED;
+  }
+#undef PA_LAUNCH_TT
   return launch_status();
 }
 

@@ -113,6 +113,26 @@ def slice_reduce(w, fx_mid, dims: LayerDims):
     return tok, norm
 
 
+def thin_tokens(x, params, dims: LayerDims):
+    """(slice_token, slice_norm) of a layer whose input has few channels, in one pass over x; None where that pass does
+    not serve the shape (the stages one by one do)."""
+    _need_cuda(x)
+    lib = _lib.load()
+    shape = dims.c()
+    g = lib.pa_thin_tokens_partial_count(_lib.dtype_code(x.dtype), byref(shape))
+    if g < 0:
+        _lib.check(int(g), "pa_thin_tokens_partial_count")
+    if g == 0:
+        return None
+    partials = torch.empty(g * dims.B * dims.H * dims.S * (dims.D + 1), dtype=torch.float32, device=x.device)
+    tok = torch.empty(dims.B, dims.H, dims.S, dims.D, dtype=torch.float32, device=x.device)
+    norm = torch.empty(dims.B, dims.H, dims.S, dtype=torch.float32, device=x.device)
+    _lib.check(lib.pa_thin_tokens(_lib.dtype_code(x.dtype), byref(shape), byref(_c_params(params)), x.data_ptr(),
+                                  partials.data_ptr(), tok.data_ptr(), norm.data_ptr(),
+                                  _lib.current_stream_ptr(x.device)), "pa_thin_tokens")
+    return tok, norm
+
+
 def slice_reduce_static(w, fx_mid, dims: LayerDims, out=None):
     """`slice_reduce` through the entry point that allocates nothing: the partial sums live in the library's static
     device scratch.  `out` = (slice_token, slice_norm) float32 tensors to fill (allocated here when omitted: the

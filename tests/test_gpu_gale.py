@@ -315,6 +315,58 @@ def test_bf16_context_projector_feeds_gale_on_the_mfma_kernels():
         assert_rel_l2(g, p.grad, f"bf16 projector grad {name}", tol=1e-1 if name == "temperature" else 5e-2)
 
 
+@pytest.mark.parametrize("C,H,S,B,N", [
+    (3, 8, 64, 1, 20000), (3, 8, 64, 2, 33), (1, 1, 16, 2, 1), (8, 4, 32, 2, 100), (16, 8, 64, 3, 8), (15, 16, 32, 1, 5000),
+    (16, 3, 16, 1, 64), (7, 2, 64, 1, 8200),
+])
+def test_tokens_of_thin_inputs_in_one_pass(C, H, S, B, N):
+    """One pass and the stages one by one against float64.  Both round x_mid, fx_mid and the weights to bf16, to a part of
+    u = 2^-9.  A logit is then off by e = u sum_d |x_mid_d W_sd| / T at most, a weight by a part of 2 e + u, a token, a
+    mean with those weights, by 2 (2 e + u) + u of the largest |fx_mid|.  Where the errors of many points average out the
+    one pass must be as exact as the stages."""
+    announce("tokens of thin inputs", C, H, S, B, N)
+    torch.manual_seed(C + N)
+    hip = pn.ContextProjector(C, heads=H, dim_head=32, slice_num=S).cuda()
+    with torch.no_grad():
+        hip.in_project_slice.weight.mul_(6.0)
+        hip.in_project_x.weight.copy_(hip.in_project_x.weight.bfloat16())
+        hip.in_project_fx.weight.copy_(hip.in_project_fx.weight.bfloat16())
+        x = torch.randn(B, N, C, device="cuda").bfloat16()
+        dims = hip.layer_dims(x)
+        p = hip.kernel_params(torch.bfloat16, x.device)
+        tok, norm = PF.thin_tokens(x, p, dims)
+        assert torch.equal(hip(x), tok)
+        x_mid, fx_mid = PF.project_inputs(x, p, dims)
+        staged_tok, staged_norm = PF.slice_reduce(PF.slice_softmax(x_mid, p, dims), fx_mid, dims)
+        ref = to.OracleContextProjector(C, heads=H, dim_head=32, slice_num=S)
+        ref.load_state_dict(hip.state_dict())
+        want = ref.double()(x.double().cpu())
+        xm, fx = (ref.__getattr__(m)(x.double().cpu()).reshape(B, N, H, 32) for m in ("in_project_x", "in_project_fx"))
+        u, T = 2.0 ** -9, 0.5
+        e = (u * (xm.abs() @ ref.in_project_slice.weight.abs().T).amax() / T).item()
+        weights = torch.softmax(ref.in_project_slice(xm) / T, -1)
+    assert ((norm.double().cpu() - 1e-2 - weights.sum(1)).abs() <= (2 * e + u) * weights.sum(1) + 1e-6 * N).all()
+    worst = ((tok.double().cpu() - want).abs().max() / fx.abs().max()).item()
+    assert worst <= 2 * (2 * e + u) + u + 1e-6, (worst, e)
+    error = lambda t: ((t.double().cpu() - want).norm() / want.norm()).item()
+    if B * N >= 5000:
+        assert error(tok) <= 1.1 * error(staged_tok), (error(tok), error(staged_tok))
+        assert_rel_l2(norm, staged_norm, "slice norms", tol=u)
+
+
+def test_tokens_of_thin_inputs_refuse_other_shapes():
+    announce("tokens of thin inputs: other shapes")
+    x = torch.randn(1, 64, 3, device="cuda").bfloat16()
+    for kw, dtype in ((dict(heads=12, dim_head=32, slice_num=64), torch.bfloat16),
+                      (dict(heads=8, dim_head=16, slice_num=64), torch.bfloat16),
+                      (dict(heads=8, dim_head=32, slice_num=48), torch.bfloat16),
+                      (dict(heads=8, dim_head=32, slice_num=64), torch.float32)):
+        hip = pn.ContextProjector(3, **kw).cuda()
+        assert PF.thin_tokens(x.to(dtype), hip.kernel_params(dtype, x.device), hip.layer_dims(x)) is None
+        with torch.no_grad():
+            assert torch.isfinite(hip(x.to(dtype))).all()
+
+
 def test_context_projector_plus_and_errors():
     announce("context projector plus / errors")
     ref, hip = _projector_pair("irregular", 16, 4, 8, 8, plus=True)
