@@ -345,39 +345,117 @@ __global__ __launch_bounds__(256) void narrow_wgrad_kernel(NarrowArgs a) {
 // sum_partials_kernel: dst[e] = sum_g src[g][e], up to eight results in one launch: a backward pass has three to eight of
 // them, each 4 to 6 us for what is mostly too small to fill the chip.  A Transolver++ layer's step over 100 003 points takes
 // 650 us with one launch at the end of its backward pass where it took 658 with three, the float32 grid model's 4 604 with
-// one per layer and 4 653 with five.  A workgroup takes 32 consecutive elements x 8 interleaved eighths of the partials and
-// adds the eighths up through LDS, always in the
-// same order.  blockIdx.y: a batch of such sums of the first result ([batch][g][e] -> [batch][e]); the others are formed by
-// batch 0.
+// one per layer and 4 653 with five.  A workgroup takes 4 consecutive elements
+// per lane of its rows, every `parts`-th partial per row of lanes, and adds the parts up through LDS, always in the same
+// order.  Bound by the read of the partials, which the product before has just written.
+// blockIdx.y: a batch of such sums of the first result ([batch][g][e] -> [batch][e]); the others are formed by batch 0.
+// 64 partials of 524 288 elements 25.3 -> 23.4 us (5.7 TB/s), 35 of them 25.7 -> 14.9; 14 of a 3 x 3 convolution's
+// 1 179 648 28.6 -> 15.6; 1 024 of 512 elements 8.2 -> 4.9 (with 32 one-element lanes before).
 // ------------------------------------------------------------------------------------------------
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// sum of load(g) over g = part, part + PARTS, .. < G, AHEAD loads in flight
+template <int PARTS, int AHEAD, class V, class F>
+__device__ __forceinline__ V sum_of_part(int part, int G, F &&load) {
+  V s = {};
+  int g = part;
+  for (; g + (AHEAD - 1) * PARTS < G; g += AHEAD * PARTS) {
+    V r[AHEAD];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) r[u] = load(g + u * PARTS);
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) s += r[u];
+  }
+  for (; g < G; g += AHEAD / 2 * PARTS) {  // the rest, half as many in flight
+    V r[AHEAD / 2];
+#pragma unroll
+    for (int u = 0; u < AHEAD / 2; ++u) r[u] = load(min(g + u * PARTS, G - 1));
+#pragma unroll
+    for (int u = 0; u < AHEAD / 2; ++u) s += g + u * PARTS < G ? r[u] : V{};
+  }
+  return s;
+}
+
+template <int LANES, int V>
+__device__ __forceinline__ void sum_rows_of(const Sums::One &o, int64_t batch, float *part) {
+  constexpr int PARTS = 256 / LANES, PER = LANES * V;
+  typedef float fvec __attribute__((ext_vector_type(V)));
+  const int64_t e0 = ((int64_t)blockIdx.x - o.first) * PER, n = o.n;
+  const int lane = threadIdx.x % LANES, part_id = threadIdx.x / LANES;
+  fvec s = {};
+  if (e0 + lane * V < n) {  // V elements or none: n is a multiple of V
+    const float *p = o.src + batch * o.G * n + e0 + lane * V;
+    s = sum_of_part<PARTS, 8, fvec>(part_id, o.G,
+                                    [&](int g) { return *reinterpret_cast<const fvec *>(p + (int64_t)g * n); });
+  }
+#pragma unroll
+  for (int v = 0; v < V; ++v) part[part_id * PER + lane * V + v] = s[v];
+  __syncthreads();
+  const int64_t e = e0 + threadIdx.x;
+  if (threadIdx.x >= PER || e >= n) return;
+  float v = part[threadIdx.x];
+#pragma unroll
+  for (int k = 1; k < PARTS; ++k) v += part[k * PER + threadIdx.x];
+  int64_t at = batch * n + e;
+  if (o.taps > 1) {
+    const int64_t oa = e / (o.taps * (int64_t)o.OB), rest = e - oa * o.taps * o.OB, tap = rest / o.OB, ob = rest - tap * o.OB;
+    at = (oa * o.OB + ob) * o.taps + tap;
+  }
+  o.dst[at] = v;
+}
+
+// [oa][tap][ob] -> [oa][ob][tap]: 256 neighbouring ob and kTaps taps at a time, so that a workgroup writes whole lines and
+// not 4 bytes in every 4 taps
+__device__ __forceinline__ void sum_taps_of(const Sums::One &o, float *part) {
+  constexpr int PARTS = 4, PER = 256, K = Sums::kTaps;
+  const int per_oa = o.OB / PER;
+  const int64_t block = (int64_t)blockIdx.x - o.first, oa = block / per_oa, n = o.n;
+  const int ob0 = (int)(block - oa * per_oa) * PER;
+  const int lane = threadIdx.x % 64, part_id = threadIdx.x / 64;
+  const float *src = o.src + oa * o.taps * o.OB + ob0 + 4 * lane;
+  float *dst = o.dst + (oa * o.OB + ob0) * o.taps;
+  for (int t0 = 0; t0 < o.taps; t0 += K) {
+    const int nt = min(K, o.taps - t0);
+    f32x4 acc[K] = {};
+    for (int g = part_id; g < o.G; g += PARTS) {  // kTaps loads in flight
+      const float *p = src + (int64_t)g * n + (int64_t)t0 * o.OB;
+      f32x4 r[K];
+#pragma unroll
+      for (int t = 0; t < K; ++t) r[t] = *reinterpret_cast<const f32x4 *>(p + (int64_t)min(t, nt - 1) * o.OB);
+#pragma unroll
+      for (int t = 0; t < K; ++t) acc[t] += r[t];
+    }
+    if (t0 > 0) __syncthreads();
+#pragma unroll
+    for (int t = 0; t < K; ++t) *reinterpret_cast<f32x4 *>(part + (part_id * K + t) * PER + 4 * lane) = acc[t];
+    __syncthreads();
+    for (int e = threadIdx.x; e < PER * nt; e += 256) {
+      const int ob = e / nt, t = e - ob * nt;
+      float v = part[t * PER + ob];
+#pragma unroll
+      for (int k = 1; k < PARTS; ++k) v += part[(k * K + t) * PER + ob];
+      dst[ob * o.taps + t0 + t] = v;
+    }
+  }
+}
+
+// TAPS: some result takes a convolution's taps together (its own instance: it needs twice the registers)
+template <bool TAPS>
 __global__ __launch_bounds__(256) void sum_partials_kernel(Sums a) {
-  __shared__ float part[8][32];
+  extern __shared__ __align__(16) float part[];
   Sums::One o = a.r[0];
 #pragma unroll
   for (int k = 1; k < Sums::kMost; ++k)
     if (k < a.count && (int64_t)blockIdx.x >= a.r[k].first) o = a.r[k];
   if (o.first > 0 && blockIdx.y > 0) return;
-  const int64_t e = ((int64_t)blockIdx.x - o.first) * 32 + (threadIdx.x & 31), n = o.n;
-  const int part_id = threadIdx.x >> 5, G = o.G;
-  float s = 0.f;
-  if (e < n) {
-    const float *p = o.src + (int64_t)blockIdx.y * G * n + e;
-#pragma unroll 8
-    for (int g = part_id; g < G; g += 8) s += p[(int64_t)g * n];
+  if constexpr (TAPS) {
+    if (o.lanes < 0) return sum_taps_of(o, part);
   }
-  part[part_id][threadIdx.x & 31] = s;
-  __syncthreads();
-  if (part_id == 0 && e < n) {
-    float v = s;
-#pragma unroll
-    for (int k = 1; k < 8; ++k) v += part[k][threadIdx.x];
-    int64_t at = (int64_t)blockIdx.y * n + e;
-    if (o.taps > 1) {
-      const int64_t oa = e / (o.taps * (int64_t)o.OB), rest = e - oa * o.taps * o.OB, tap = rest / o.OB, ob = rest - tap * o.OB;
-      at = (oa * o.OB + ob) * o.taps + tap;
-    }
-    o.dst[at] = v;
-  }
+  if (o.lanes == 64) sum_rows_of<64, 4>(o, blockIdx.y, part);
+  else if (o.lanes == 32) sum_rows_of<32, 4>(o, blockIdx.y, part);
+  else if (o.lanes == 16) sum_rows_of<16, 4>(o, blockIdx.y, part);
+  else if (o.lanes == 8) sum_rows_of<8, 4>(o, blockIdx.y, part);
+  else sum_rows_of<32, 1>(o, blockIdx.y, part);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -393,7 +471,6 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(Sums a) {
 __global__ __launch_bounds__(256) void token_grad_kernel(const float *__restrict__ P, const uint16_t *__restrict__ w_out,
                                                          const float *__restrict__ out_token, float *__restrict__ d_token,
                                                          float *__restrict__ d_w_out, int B, int H, int S, int C, int cb) {
-  typedef float f32x4 __attribute__((ext_vector_type(4)));
   __shared__ float part[3][16][64];
   const int lane = threadIdx.x & 63, i = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -558,7 +635,9 @@ int product(int dtype, int64_t M, const void *A, int64_t lda, int64_t OA, const 
 }
 
 static int launch_sums(const Sums &sums, int64_t batches, hipStream_t st) {
-  hipLaunchKernelGGL(sum_partials_kernel, dim3((unsigned)sums.blocks, (unsigned)batches), dim3(256), 0, st, sums);
+  const dim3 grid((unsigned)sums.blocks, (unsigned)batches);
+  if (sums.by_taps) hipLaunchKernelGGL((sum_partials_kernel<true>), grid, dim3(256), 1024 * Sums::kTaps * 4, st, sums);
+  else hipLaunchKernelGGL((sum_partials_kernel<false>), grid, dim3(256), 1024 * 4, st, sums);
   return launch_status();
 }
 int launch_sums(const Sums &sums, hipStream_t st) { return launch_sums(sums, 1, st); }

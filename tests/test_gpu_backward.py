@@ -426,6 +426,21 @@ def test_weight_gradient_shapes(dtype, rows, ca, cb):
     assert torch.equal(got, PF.cols_gemm(a, b))
 
 
+@pytest.mark.parametrize("rows,ca,cb", [
+    (30011, 1024, 256), (9000, 512, 256), (12000, 1024, 256), (70001, 256, 256),  # few / many partials, large / small result
+    (4100, 256, 3), (1000, 3, 20), (65, 5, 16),                                   # results of 4 k and of other numbers of values
+])
+def test_totals_of_partial_products(rows, ca, cb):
+    """The splits of a total among a workgroup's rows of lanes.  Inputs are small whole numbers, so that every float32 sum
+    is exact and the results equal float64's to the bit."""
+    announce("totals of partial products", rows, ca, cb)
+    torch.manual_seed(rows)
+    a, b = (torch.randint(-3, 4, (rows, c), device="cuda").bfloat16() for c in (ca, cb))  # |sums| <= 9 rows < 2^24
+    got, sums = PF.cols_gemm(a, b, col_sums=True)
+    assert torch.equal(got, (a.double().t() @ b.double()).float())
+    assert torch.equal(sums, a.double().sum(0).float())
+
+
 @pytest.mark.parametrize("dtype,C,O", [(torch.bfloat16, 256, 512), (torch.bfloat16, 128, 128), (torch.float32, 128, 256),
                                        (torch.float32, 36, 20)])
 @pytest.mark.parametrize("grid,k", [((13, 9), 3), ((40, 33), 5), ((4, 6, 5), 3), ((1, 50), 3)])
