@@ -230,7 +230,7 @@ StagedPlan plan_staged(const pa_shape &s) {
 // Workspace plan of the Transolver++ layer: the staged kernels with the slice weights stored (their Gumbel noise
 // comes from the caller's samples, which are read once).
 struct PlusPlan {
-  int64_t off_x_mid, off_fx, off_w, off_partials, off_tok, off_norm, off_tok_out, off_tokp, off_blob, total;
+  int64_t off_x_mid, off_w, off_partials, off_tok, off_norm, off_tok_out, off_tokp, off_blob, total;
   int64_t G;
 };
 
@@ -239,10 +239,8 @@ PlusPlan plan_plus(const pa_shape &s) {
   p.G = mfma_groups(s, false);
   const int64_t tiles = s.B * pa::mfma::tiles_per_batch(s);
   int64_t off = 0;
-  p.off_x_mid = off;  // natural (B, N, H*32); reused for out_x once the slice weights exist
+  p.off_x_mid = off;  // natural (B, N, H*32); reused for out_x once the token sums exist
   off += round_up(s.B * s.N * s.H * 32 * 2, 256);
-  p.off_fx = off;
-  off += round_up(tiles * s.H * 2 * 1024, 256);
   p.off_w = off;
   off += round_up(tiles * s.H * (s.S / 16) * 1024, 256);
   p.off_partials = off;
@@ -1848,17 +1846,16 @@ int pa_layer_forward_plus(int dtype, const pa_shape *shape, const pa_params *p, 
   const PlusPlan sp = plan_plus(s);
   if (workspace_bytes < sp.total) return PA_ERR_WORKSPACE;
   char *ws = static_cast<char *>(workspace);
-  void *x_mid = ws + sp.off_x_mid, *fxp = ws + sp.off_fx, *wp = ws + sp.off_w, *tokp = ws + sp.off_tokp;
+  void *x_mid = ws + sp.off_x_mid, *wp = ws + sp.off_w, *tokp = ws + sp.off_tokp;
   float *partials = reinterpret_cast<float *>(ws + sp.off_partials);
   float *tok = slice_token_out ? slice_token_out : reinterpret_cast<float *>(ws + sp.off_tok);
   float *norm = reinterpret_cast<float *>(ws + sp.off_norm);
   float *tok_out = reinterpret_cast<float *>(ws + sp.off_tok_out);
-  pa::GemmArgs a{};  // x -> x_mid, natural layout for the slice weights and packed for the aggregation (fx_mid is x_mid)
+  pa::GemmArgs a{};  // x -> x_mid in natural layout, for the slice weights and the aggregation (fx_mid is x_mid)
   a.in = x;
   a.w[0] = p->in_project_x_weight;
   a.bias[0] = p->in_project_x_bias;
   a.out[0] = x_mid;
-  a.out_pack[0] = fxp;
   a.M = s.B * s.N;
   a.N = (int)s.N;
   a.C = (int)s.C;
@@ -1869,12 +1866,10 @@ int pa_layer_forward_plus(int dtype, const pa_shape *shape, const pa_params *p, 
   a.w_tap_major = (int)s.conv_tap_major;
   a.K = s.conv_k > 0 ? (int)(s.conv_k * s.conv_k * (s.grid_d > 0 ? s.conv_k : 1) * s.C) : (int)s.C;
   a.O = (int)(s.H * 32);
-  a.pack_tpb = (int)pa::mfma::tiles_per_batch(s);
-  a.pack_heads = (int)s.H;
   if (!pa::gemm::serves(a, 1, 2)) return PA_ERR_UNSUPPORTED;
   if ((rc = pa::gemm::launch(a, 1, PA_BF16, st))) return rc;
   if ((rc = pa::mfma::slice_softmax_pack_plus(s, *p, *plus, x_mid, uniform, wp, false, nullptr, compute_units(), st))) return rc;
-  if ((rc = pa::mfma::slice_reduce(s, wp, fxp, partials, st))) return rc;
+  if ((rc = pa::mfma::slice_reduce_rows(s, wp, x_mid, partials, st))) return rc;
   if ((rc = pa::mfma::combine_attention(s, *p, nullptr, partials, sp.G, tok, norm, tok_out, tokp, st))) return rc;
   if (pa::mfma::supported(dtype, s) && p->out_linear_bias) {
     // hand-back, out_linear and the block's tail in kernel (d), which reads the out_linear part of the parameter blob

@@ -349,6 +349,8 @@ int project_softmax(const pa_shape &s, const void *blob, const void *x, void *fx
 int project_softmax_clocked(const pa_shape &s, const void *blob, const void *x, void *w_pack, float *partials,
                             uint64_t *clock_out, int num_cu, hipStream_t st);
 int slice_reduce(const pa_shape &s, const void *w_pack, const void *fx_pack, float *partials, hipStream_t st);
+// the same on fx_mid as (B, N, H*32) rows
+int slice_reduce_rows(const pa_shape &s, const void *w_pack, const void *fx_mid, float *partials, hipStream_t st);
 int combine_attention(const pa_shape &s, const pa_params &p, const float *fx_bias, const float *partials, int64_t G,
                       float *slice_token, float *slice_norm, float *out_token, void *tokp, hipStream_t st);
 int deslice_project(const pa_shape &s, const void *blob, const void *w_pack, const void *tokp, void *y,

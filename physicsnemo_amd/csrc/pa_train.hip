@@ -172,7 +172,7 @@ static Scratch plan_scratch(const pa_shape &s, bool plus, int num_cu) {
     return at;
   };
   p.blob = take(hand_back(s, plus) != HandBack::apart ? mfma::blob_bytes(s) : 0);
-  p.fx_pack = take(tiles * s.H * 2 * 1024);
+  p.fx_pack = take(plus ? 0 : tiles * s.H * 2 * 1024);
   p.partials = take((forward_groups(s, plus, num_cu) + 1) * BHS * 33 * 4);
   p.tokp = take(mfma::tokp_bytes(s));
   p.out_x = take(hand_back(s, plus) == HandBack::apart ? M * HD * 2 : 0);
@@ -287,19 +287,20 @@ int forward(const pa_shape &s, int weight_dtype, const pa_params &params, const 
     a.w[0] = p.in_project_x_weight, a.w[1] = p.in_project_fx_weight;
     a.bias[0] = p.in_project_x_bias, a.bias[1] = p.in_project_fx_bias;
     a.out[0] = x_mid, a.out[1] = fx_mid;
-    a.out_pack[pl ? 0 : 1] = fx_pack;
+    if (!pl) a.out_pack[1] = fx_pack;  // Transolver++: fx_mid is x_mid, read as rows
     a.M = s.B * s.N;
     a.N = (int)s.N, a.C = (int)s.C, a.O = (int)(s.H * 32);
     a.gh = (int)s.grid_h, a.gw = (int)s.grid_w, a.gd = (int)s.grid_d, a.ks = (int)s.conv_k;
     a.w_tap_major = 1;
     a.K = taps * (int)s.C;
-    a.pack_tpb = (int)mfma::tiles_per_batch(s), a.pack_heads = (int)s.H;
+    if (!pl) a.pack_tpb = (int)mfma::tiles_per_batch(s), a.pack_heads = (int)s.H;
     if (!gemm::serves(a, pl ? 1 : 2, 2)) return PA_ERR_UNSUPPORTED;
     if ((rc = gemm::launch(a, pl ? 1 : 2, PA_BF16, st))) return rc;
     rc = pl ? mfma::slice_softmax_pack_plus(s, p, prep.q, x_mid, uniform, w_pack, true, reinterpret_cast<float *>(sv + sp.a2), num_cu, st)
             : mfma::slice_softmax_pack(s, p, x_mid, w_pack, num_cu, st);
     if (rc) return rc;
-    if ((rc = mfma::slice_reduce(s, w_pack, fx_pack, partials, st))) return rc;
+    rc = pl ? mfma::slice_reduce_rows(s, w_pack, x_mid, partials, st) : mfma::slice_reduce(s, w_pack, fx_pack, partials, st);
+    if (rc) return rc;
     if (how != HandBack::apart && (rc = mfma::pack_out_linear(s, p.out_linear_weight, nullptr, p.out_linear_bias, blob, st)))
       return rc;
   }

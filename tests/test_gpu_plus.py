@@ -86,6 +86,13 @@ def test_bf16_plus_layer_on_the_mfma_kernels(dim, heads, S, B, N):
     assert_rel_l2(got, general, "bf16 plus y: MFMA vs general kernels", tol=1e-2)
 
 
+@pytest.mark.parametrize("dim,heads,S,B,N", [(128, 4, 64, 4100, 1), (256, 8, 32, 130, 33), (256, 8, 128, 70, 63),
+                                             (256, 8, 16, 128, 32)])
+def test_bf16_plus_layer_of_one_or_two_tiles(dim, heads, S, B, N):
+    """Token sums from the rows of x_mid where the last tile of a batch element ends early: the same bounds."""
+    test_bf16_plus_layer_on_the_mfma_kernels(dim, heads, S, B, N)
+
+
 def test_bf16_plus_block_tail_on_the_mfma_kernels():
     announce("bf16 plus forward_block")
     ref, hip = _pair("irregular", 256, 8, 32, 64, seed=5)
