@@ -541,13 +541,19 @@ __global__ __launch_bounds__(256) void slice_softmax_backward_kernel(
   for (int off = tpr >> 1; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
   const float inv_sum = 1.f / sum;
   auto weight = [&](int s) { return r_own < rows ? expf(lgl[r_own * S1 + s] * yscale - mx) * inv_sum : 0.f; };
-  float dot = 0.f;
-  for (int s = j_own; s < S; s += tpr) dot = fmaf(weight(s), dwl[r_own * S1 + s], dot);
-  for (int off = tpr >> 1; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64);
+  // d temperature's sum_s d l[s] l[s] takes the l[s] from their weighted mean: as d l sums to zero up to the rounding of `dot`,
+  // that is the same sum without that rounding
+  float dot = 0.f, mean = 0.f;
+  for (int s = j_own; s < S; s += tpr) {
+    const float ws = weight(s);
+    dot = fmaf(ws, dwl[r_own * S1 + s], dot);
+    mean = fmaf(ws, lgl[r_own * S1 + s], mean);
+  }
+  for (int off = tpr >> 1; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64), mean += __shfl_xor(mean, off, 64);
   float tsum = 0.f;
   for (int s = j_own; s < S; s += tpr) {
     const float dl = weight(s) * (dwl[r_own * S1 + s] - dot);
-    tsum = fmaf(dl, lgl[r_own * S1 + s], tsum);
+    tsum = fmaf(dl, lgl[r_own * S1 + s] - mean, tsum);
     dwl[r_own * S1 + s] = dl * inv_temp;
   }
   if constexpr (PLUS) {

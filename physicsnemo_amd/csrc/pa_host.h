@@ -232,6 +232,17 @@ int front(const pa_shape &s, const pa_params &p, const void *x, float *w, float 
 int block_tail(const pa_shape &s, const pa_params &p, const pa_block_mlp &m, const float *w, const float *out_token,
                const void *fx_in, void *fx_out, const pa_block_tail *next, const pa_block_head *head, int num_cu,
                hipStream_t st);
+// float32 training, heads of 16 channels and 32 slices: the slice softmax of x_mid's rows with the token sums of v's (p NULL: the
+// sums alone, of the weights w), point_groups() partials as the general combine kernels read them; and the per-point adjoints
+// with d W_slice | d b_slice | d temperature (masked where clamped), point_backward_rows() partial rows of S 17 + H floats
+bool points_supported(const pa_shape &s);
+int64_t point_groups(const pa_shape &s, int num_cu);
+int64_t point_backward_rows(const pa_shape &s, int num_cu);
+int point_sums(const pa_shape &s, const pa_params *p, const float *x_mid, const float *v, float *w, float *partials, int num_cu,
+               hipStream_t st);
+int point_backward(const pa_shape &s, const pa_params &p, const float *x_mid, const float *fx_mid, const float *g,
+                   const float *out_token, const float *d_num, const float *d_norm, float *d_proj, float *partials, int num_cu,
+                   hipStream_t st);
 }  // namespace narrow
 
 namespace backward {

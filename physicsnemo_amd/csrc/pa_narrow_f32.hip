@@ -12,29 +12,11 @@
 // order 4 g + r, g = 0 .. 3; the other operand is then a float4 per tile of the row-major weight, which lies in LDS as it is
 // (rows four floats apart in the banks).
 #include "pa_host.h"
-#include "pa_mfma_ops.h"
+#include "pa_narrow_ops.h"
 
 namespace pa {
 namespace narrow {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-constexpr int kS = 32, kTilePts = 16;
-
-__device__ __forceinline__ f32x4 mma16(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-// over the four lanes that hold a point's (or a slice's) registers
-__device__ __forceinline__ float group_sum(float v) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return mfma::half_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float group_max(float v) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return mfma::half_max(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
-}
-// a value that is the same in all lanes, in a scalar register
-__device__ __forceinline__ float uniform(float v) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v))); }
-// keeps the LDS reads of a later section from being hoisted into registers here
-__device__ __forceinline__ void section() { asm volatile("" ::: "memory"); }
 __device__ __forceinline__ float4 quad(const float *p) { return *reinterpret_cast<const float4 *>(p); }
 __device__ __forceinline__ float at(const float4 &v, int j) { return j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w; }
 
@@ -150,14 +132,10 @@ __global__ __launch_bounds__(64 * W, C == 64 && D == 8 ? 2 : 4) void front_kerne
   stage_matrices({w_x, C, C, wx}, {w_fx, C, C, wf}, {w_s, kS, D, ws});
   stage_vectors<2>({b_x, b_fx}, {0.f, 0.f}, {bx, bf}, C);
   stage_vectors<1>({b_s}, {0.f}, {bs}, kS);
-  // exp(z / T) = 2^(z sc), sc = log2(e) / T as the sum of two floats: nothing is lost to the rounding of z / T or of its product
   float sc[H], sc_low[H];
 #pragma unroll
   for (int h = 0; h < H; ++h) {
-    const float temp = clamp_temperature(temperature[h]);
-    const float hi = kLog2e / temp;
-    sc[h] = uniform(hi);
-    sc_low[h] = uniform((fmaf(-hi, temp, kLog2e) + 1.92596299e-8f) / temp);  // log2(e) = kLog2e + 1.93e-8
+    exponent_scale(clamp_temperature(temperature[h]), sc[h], sc_low[h]);
   }
   turn += wave * K::kTurn;
   f32x4 tok[H][2];  // lane i <-> channel i of the head's tile, registers <-> slices 16 st + 4 g + r
@@ -203,9 +181,7 @@ __global__ __launch_bounds__(64 * W, C == 64 && D == 8 ? 2 : 4) void front_kerne
         for (int st = 0; st < 2; ++st)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const float z = lg[st][r] - mx, hi = z * sc[h], low = fmaf(z, sc_low[h], fmaf(z, sc[h], -hi));
-            const float e = __builtin_amdgcn_exp2f(hi);
-            lg[st][r] = fmaf(e * 0.69314718f, low, e);
+            lg[st][r] = exponential(lg[st][r] - mx, sc[h], sc_low[h]);
             sum += lg[st][r];
           }
         const float inv = 1.f / group_sum(sum);

@@ -99,6 +99,7 @@ struct Scratch {
   int64_t w_in, partials, total;                                                                                    // forward
   int64_t g, d_tok, d_num, d_norm, attn, parts, d_proj, d_z, d_t, t_sum, heads, work[3], total_backward;
   bool served;  // by the row-axis products
+  bool narrow;  // the per-point stages on the kernels of narrow heads
 };
 struct Taker {
   int64_t off = 0;
@@ -133,11 +134,16 @@ static Saved plan_saved(const pa_shape &s) {
   return p;
 }
 
+static int64_t sum_groups(const pa_shape &s, int num_cu) {  // partial token sums
+  return narrow::points_supported(s) ? narrow::point_groups(s, num_cu) : general::partial_count(s);
+}
+
 static Scratch plan_scratch(const pa_shape &s, int num_cu) {
   const int64_t HD = s.H * s.D, HS = s.H * s.S, M = s.B * s.N, BHS = s.B * HS, taps = grid_taps(&s).taps;
   Scratch p{};
   Taker take;
-  p.partials = take((general::partial_count(s) + 1) * BHS * (s.D + 1) * 4);
+  p.narrow = narrow::points_supported(s);
+  p.partials = take((sum_groups(s, num_cu) + 1) * BHS * (s.D + 1) * 4);
   Taker back = take;
   p.w_in = take(taps > 1 ? 2 * HD * taps * s.C * 4 : 0);
   p.total = take.off;
@@ -145,10 +151,12 @@ static Scratch plan_scratch(const pa_shape &s, int num_cu) {
   p.d_tok = back(BHS * s.D * 4), p.d_num = back(BHS * s.D * 4), p.d_norm = back(BHS * 4);
   p.attn = back(s.B * s.H * 2 * s.S * s.S * 4);
   p.parts = back(s.B * s.H * 3 * s.D * s.D * 4);
-  p.d_proj = back(M * 2 * HD * 4), p.d_z = back(M * HS * 4);
-  p.d_t = back(backward::point_tiles(s) * s.H * 4), p.t_sum = back(s.H * 4);
-  p.heads = back((HS * HD + HS) * 4);
-  const int64_t work[3] = {wgrad::workspace_bytes(PA_F32, M, s.C, HD, 1, num_cu), wgrad::workspace_bytes(PA_F32, M, HS, HD, 1, num_cu),
+  p.d_proj = back(M * 2 * HD * 4), p.d_z = back(p.narrow ? 0 : M * HS * 4);
+  p.d_t = back(p.narrow ? narrow::point_backward_rows(s, num_cu) * (s.S * (s.D + 1) + s.H) * 4 : backward::point_tiles(s) * s.H * 4);
+  p.t_sum = back(s.H * 4);
+  p.heads = back(p.narrow ? 0 : (HS * HD + HS) * 4);
+  const int64_t work[3] = {wgrad::workspace_bytes(PA_F32, M, s.C, HD, 1, num_cu),
+                           p.narrow ? 256 : wgrad::workspace_bytes(PA_F32, M, HS, HD, 1, num_cu),
                            wgrad::workspace_bytes(PA_F32, M, 2 * HD, s.C, (int)taps, num_cu)};
   p.served = true;
   for (int k = 0; k < 3; ++k) {
@@ -206,9 +214,18 @@ int forward(const pa_shape &s, const pa_params &params, const void *x, void *y, 
   float *partials = f(ws, sc.partials), *tok = f(sv, sp.tok), *norm = f(sv, sp.norm), *tok_out = f(sv, sp.tok_out);
   void *x_mid = sv + sp.x_mid, *fx_mid = sv + sp.fx_mid, *w = sv + sp.w, *out_x = sv + sp.out_x;
   if ((rc = general::project_inputs(PA_F32, s, p, x, x_mid, fx_mid, st))) return rc;
-  if ((rc = general::slice_softmax(PA_F32, s, p, x_mid, w, st))) return rc;
-  if ((rc = general::slice_partial(PA_F32, s, w, fx_mid, partials, st))) return rc;
-  if ((rc = general::combine_attention(s, p, partials, general::partial_count(s), tok, norm, tok_out, st))) return rc;
+  if (sc.narrow) {
+    pa_params copies{};  // on their 16-byte boundaries
+    copies.in_project_slice_weight = pa.copies + pa.at[0], copies.in_project_slice_bias = pa.copies + pa.at[1];
+    copies.temperature = pa.copies + pa.at[2];
+    rc = narrow::point_sums(s, &copies, static_cast<float *>(x_mid), static_cast<float *>(fx_mid), static_cast<float *>(w), partials,
+                            num_cu, st);
+  } else {
+    if ((rc = general::slice_softmax(PA_F32, s, p, x_mid, w, st))) return rc;
+    rc = general::slice_partial(PA_F32, s, w, fx_mid, partials, st);
+  }
+  if (rc) return rc;
+  if ((rc = general::combine_attention(s, p, partials, sum_groups(s, num_cu), tok, norm, tok_out, st))) return rc;
   if ((rc = general::deslice(PA_F32, s, w, tok_out, out_x, st))) return rc;
   if ((rc = general::out_linear(PA_F32, s, p, out_x, y, st)) || !tail) return rc;
   return general::residual_ln(PA_F32, s, y, *tail, st);
@@ -240,25 +257,36 @@ int backward(const pa_shape &s, const void *x, const void *dy, const void *saved
   if (rc) return rc;
   // adjoint of the deslice w.r.t. the attended tokens, then the slice attention and the normalisation
   const float *sums = nullptr;
-  if ((rc = general::slice_partial(PA_F32, s, w, g, partials, st))) return rc;
-  if ((rc = general::combine_partials(s, partials, general::partial_count(s), &sums, st))) return rc;
+  rc = sc.narrow ? narrow::point_sums(s, nullptr, nullptr, static_cast<float *>(g), const_cast<float *>(static_cast<const float *>(w)),
+                                      partials, num_cu, st)
+                 : general::slice_partial(PA_F32, s, w, g, partials, st);
+  if (rc) return rc;
+  if ((rc = general::combine_partials(s, partials, sum_groups(s, num_cu), &sums, st))) return rc;
   hipLaunchKernelGGL(take_tokens_kernel, dim3((unsigned)((BHS * s.D + 255) / 256)), dim3(256), 0, st, sums, d_tok, BHS * s.D, (int)s.D);
   if ((rc = launch_status())) return rc;
   if ((rc = backward::slice_attention(s, p, tok, norm, d_tok, f(ws, sc.attn), d_num, d_norm, parts, st))) return rc;
   wgrad::Sums totals;  // formed together at the end: what their partial results lie in is not used again until then
   totals.add(parts, d_wqkv, 3 * s.D * s.D, s.B * s.H);
   // per point: slice softmax, aggregation and deslice adjoints
-  if ((rc = backward::slice_softmax(PA_F32, s, p, x_mid, fx_mid, w, g, tok_out, d_num, d_norm, d_proj, d_z, t_tiles, st))) return rc;
-  totals.add(t_tiles, t_sum, s.H, backward::point_tiles(s));
+  if (sc.narrow) {
+    auto in = [](const void *q) { return static_cast<const float *>(q); };
+    rc = narrow::point_backward(s, p, in(x_mid), in(fx_mid), in(g), tok_out, d_num, d_norm, static_cast<float *>(d_proj), t_tiles, num_cu, st);
+    totals.add(t_tiles, d_ws, s.S * (s.D + 1) + s.H, narrow::point_backward_rows(s, num_cu));  // d_ws, d_bs, d_t
+  } else {
+    rc = backward::slice_softmax(PA_F32, s, p, x_mid, fx_mid, w, g, tok_out, d_num, d_norm, d_proj, d_z, t_tiles, st);
+    totals.add(t_tiles, t_sum, s.H, backward::point_tiles(s));
+  }
+  if (rc) return rc;
   if ((rc = wgrad::product(PA_F32, M, dy, s.C, s.C, out_x, HD, HD, nullptr, ws + sc.work[0], d_w_out, d_b_out, num_cu, st, &totals)))
     return rc;
-  if ((rc = wgrad::product(PA_F32, M, d_z, HS, HS, x_mid, HD, HD, nullptr, ws + sc.work[1], heads, heads + HS * HD, num_cu, st, &totals)))
+  if (!sc.narrow && (rc = wgrad::product(PA_F32, M, d_z, HS, HS, x_mid, HD, HD, nullptr, ws + sc.work[1], heads, heads + HS * HD, num_cu,
+                                         st, &totals)))
     return rc;
   if (dx && (rc = general::rows_gemm(PA_F32, s, 2 * HD, s.C, d_proj, sv + sp.w_in_t, nullptr, 0, dx, st))) return rc;
   if ((rc = wgrad::product(PA_F32, M, d_proj, 2 * HD, 2 * HD, x, s.C, s.C, s.conv_k > 0 ? &s : nullptr, ws + sc.work[2], d_w_in, d_b_in,
                            num_cu, st, &totals)))
     return rc;
-  if ((rc = wgrad::launch_sums(totals, st))) return rc;
+  if ((rc = wgrad::launch_sums(totals, st)) || sc.narrow) return rc;
   hipLaunchKernelGGL(head_sums_kernel, dim3((unsigned)((s.S * s.D + s.S + s.H + 255) / 256)), dim3(256), 0, st, heads, heads + HS * HD,
                      t_sum, small + at[2], d_ws, d_bs, d_t, (int)s.H, (int)s.S, (int)s.D);
   return launch_status();

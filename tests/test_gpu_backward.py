@@ -1497,6 +1497,12 @@ def test_fp32_layer_in_two_calls_against_float64(kind, dim, heads, dim_head, S, 
         assert err <= (1.7e-5 if n == "temperature" else 6e-6), (n, err.item())
 
 
+@pytest.mark.parametrize("dim,heads,N", [(48, 3, 17), (128, 8, 15), (128, 8, 16), (256, 16, 33), (32, 2, 9000), (128, 8, 9000)])
+def test_fp32_layer_of_16_channel_heads_at_the_edges_of_its_tiles(dim, heads, N):
+    """The per-point kernels of 16-channel heads and 32 slices (tiles of 16 points): the same bounds."""
+    test_fp32_layer_in_two_calls_against_float64("irregular", dim, heads, 16, 32, None, 0, N)
+
+
 @pytest.mark.parametrize("dtype,C,O", [(torch.float32, 128, 132), (torch.float32, 64, 256), (torch.bfloat16, 128, 256)])
 @pytest.mark.parametrize("grid,B", [((1, 1), 70), ((2, 3), 11), ((1, 31), 2), ((32, 1), 3), ((2, 2, 2), 9), ((3, 4, 5), 7)])
 def test_conv_weight_gradient_of_grids_within_a_block_of_rows(dtype, C, O, grid, B):
