@@ -202,6 +202,8 @@ bool hidden_backward_supported(int64_t rows, int64_t C, int64_t F) {
   return rows > 0 && C == 256 && F % 64 == 0 && hidden_backward_lds(F) <= 160 * 1024;
 }
 
+constexpr int64_t kItemChunks = 8;
+
 int64_t hidden_backward_blob_bytes(int64_t C, int64_t F) { return 4 * C * F; }
 
 int hidden_backward(int64_t rows, int64_t C, int64_t F, const void *w1, const float *b1, const void *w2, const void *u,
@@ -212,9 +214,14 @@ int hidden_backward(int64_t rows, int64_t C, int64_t F, const void *w1, const fl
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return (int)e;
   const int64_t blocks = (rows + 255) / 256, chunks = F / 32;
-  // two items per CU where the rows alone do not give them; an item of fewer than four chunks is mostly row loads
+  // The split with the shortest way for the busiest CU, its items' chunks and, for each item, the row loads and last stores that
+  // nothing covers: 10 us, three chunks of a full chip; taken as eight, because chunks go faster where CUs are left idle (the
+  // stores bound them).  Against two items per CU wherever the rows do not give them: 14 450 rows 50 -> 40 us, 24 200 72 -> 55,
+  // 32 768 74 -> 65, 60 000 128 -> 99, 100 000 197 -> 177, 2 500 and 8 000 the same; taken as three, 40 000 rows 98 against 87.
   int splits = 1;
-  while (blocks * splits < 2 * cus && chunks % (4 * splits) == 0 && chunks / (2 * splits) >= 4) splits *= 2;
+  auto way = [&](int64_t n) { return (blocks * n + cus - 1) / cus * (chunks / n + kItemChunks); };
+  for (int n = 2; chunks % (2 * n) == 0 && chunks / n >= 4; n *= 2)
+    if (way(n) < way(splits)) splits = n;
   const int64_t items = blocks * splits;
   const int lds = (int)hidden_backward_lds(F);
   e = hipFuncSetAttribute(reinterpret_cast<const void *>(hidden_backward_kernel<256>),

@@ -1102,6 +1102,21 @@ def test_row_gemm_of_256_inputs_with_two_workgroups_per_cu(rows, c_out, bias):
     assert (err <= 2.0 ** -8 * want.abs() + 1e-3).all()
 
 
+@pytest.mark.parametrize("rows,Fh", [(1, 64), (300, 192), (2500, 1024), (14450, 1024), (32768, 1024), (40000, 1024), (70000, 512)])
+def test_hidden_gradients_do_not_depend_on_how_the_hidden_units_are_split(rows, Fh):
+    """Rows choose how many parts the hidden units are taken in; each row's values have the same bits as in a call of few rows."""
+    announce("hidden gradients by split", rows, Fh)
+    C, dev = 256, torch.device("cuda")
+    gen = torch.Generator().manual_seed(rows)
+    rnd = lambda *n: torch.randn(*n, generator=gen)
+    u, dy = rnd(rows, C).bfloat16().to(dev), rnd(rows, C).bfloat16().to(dev)
+    w1, w2, b1 = (rnd(Fh, C) / 16).bfloat16().to(dev), (rnd(C, Fh) / 16).bfloat16().to(dev), (0.1 * rnd(Fh)).to(dev)
+    act, dh = PF.mlp_backward(u, dy, w1, b1, w2)
+    for part in (slice(0, min(rows, 200)), slice(max(0, rows - 300), rows)):
+        few_act, few_dh = PF.mlp_backward(u[part].contiguous(), dy[part].contiguous(), w1, b1, w2)
+        assert torch.equal(act[part], few_act) and torch.equal(dh[part], few_dh)
+
+
 @pytest.mark.parametrize("rows,Fh", [(1, 256), (63, 1024), (64, 320), (65, 256), (2000, 1024), (32768, 256), (32769, 256), (65537, 64),
                                      (2 * 256 * 128 + 1, 256)])
 def test_norm_mlp_backward_against_float64(rows, Fh):
