@@ -316,6 +316,89 @@ __global__ __launch_bounds__(512, LEAN ? 4 : 2) void rows_linear_kernel(GemmArgs
   }
 }
 
+// ------------------------------------------------------------------------------------------------
+// rows_linear_ring_kernel: the same for K = 512 in natural layout, 256 columns per workgroup.  The weights take 128 registers, so one
+// workgroup owns a CU, and what hides memory's latency is what it alone has on its way: the rows go from memory straight into a ring of
+// four 32-row tiles in LDS (33 KB each), three of them in flight while one is multiplied, one barrier per tile.  One load is one row of
+// 1 024 bytes; rows lie 16 bytes more apart, so that the lanes of an access phase (32 rows, one unit) fall on different banks.
+// Loads and stores leave the counter in order: behind a tile's four loads a wave has issued the loads of up to two tiles and the two
+// stores each of up to three.  Bound by HBM: 1 048 576 rows into 256 columns, with rows_linear_kernel / here, in a layer's training step
+// 412 / 297 us (5.4 TB/s); called again and again 4 096 rows 11.1 / 10.4, 30 000 18.3 / 18.5, 65 536 31.4 / 31.6, 131 072 50.4 / 46.0,
+// 262 144 93 / 85 (512 columns 166 / 143).
+// ------------------------------------------------------------------------------------------------
+struct LinearRing {
+  static constexpr int K = 512, KS = K / 16, ROWU = K / 8 + 1, TILE = 32 * ROWU * 16, STAGES = 4, BYTES = STAGES * TILE + 256 * 4;
+};
+
+__global__ __launch_bounds__(512, 2) void rows_linear_ring_kernel(GemmArgs a) {
+  using Q = LinearRing;
+  constexpr int K = Q::K;
+  extern __shared__ u32x4 xs_all[];
+  float *bias_s = reinterpret_cast<float *>(xs_all + Q::STAGES * (Q::TILE / 16));
+  const int z = blockIdx.z;
+  const uint16_t *in = static_cast<const uint16_t *>(a.in);
+  const uint16_t *W = static_cast<const uint16_t *>(a.w[z]);
+  const int tid = threadIdx.x, lane = tid & 63, i = lane & 31, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int o0 = blockIdx.y * 256 + wave * 32;  // this wave's output columns
+
+  const int64_t ntiles = (a.M + 31) / 32, stride = gridDim.x;  // grid.x <= ntiles: a workgroup has a tile
+  auto fetch = [&](int64_t tile, int stage) {
+    if (tile >= ntiles) return;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int row = 4 * wave + k;
+      const int64_t m = tile * 32 + row < a.M ? tile * 32 + row : a.M - 1;  // past the last row: that one
+      mfma::load_unit_to_lds(in + m * K, lane * 16, (unsigned)(uintptr_t)xs_all + stage * Q::TILE + row * (Q::ROWU * 16));
+    }
+  };
+  int64_t tile = blockIdx.x;
+  fetch(tile, 0);
+  const float bias = tid < 256 && a.bias[z] ? a.bias[z][blockIdx.y * 256 + tid] : 0.f;
+  u32x4 wf[Q::KS];  // W[o0 + i][16 ks + 8 g + j]
+#pragma unroll
+  for (int ks = 0; ks < Q::KS; ++ks) wf[ks] = *reinterpret_cast<const u32x4 *>(W + (int64_t)(o0 + i) * K + 16 * ks + 8 * g);
+#pragma unroll
+  for (int ks = 0; ks < Q::KS; ++ks) asm volatile("" : "+v"(wf[ks]));  // they are waited for here and not in the loop
+  if (tid < 256) bias_s[tid] = bias;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // with the first tile: the loop counts from here
+#pragma unroll
+  for (int s = 1; s < Q::STAGES - 1; ++s) fetch(tile + s * stride, s);
+  int stage = 0, done = 0;  // done: tiles whose stores may be on their way, at most three
+  for (; tile < ntiles; tile += stride) {
+    const int later = tile + 2 * stride < ntiles ? 2 : tile + stride < ntiles ? 1 : 0;  // tiles behind this one that are on their way
+    switch (2 * later + done) {
+      case 0: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
+      case 1: asm volatile("s_waitcnt vmcnt(2)" ::: "memory"); break;
+      case 2: asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); break;
+      case 3: asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); break;
+      case 4: asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); break;
+      case 5: asm volatile("s_waitcnt vmcnt(10)" ::: "memory"); break;
+      case 6: asm volatile("s_waitcnt vmcnt(12)" ::: "memory"); break;
+      default: asm volatile("s_waitcnt vmcnt(14)" ::: "memory"); break;
+    }
+    done = done < 3 ? done + 1 : 3;
+    __syncthreads();  // every wave's rows of the tile are there, and every wave is past the tile before
+    fetch(tile + (Q::STAGES - 1) * stride, (stage + Q::STAGES - 1) % Q::STAGES);
+    const u32x4 *xb = xs_all + stage * (Q::TILE / 16) + i * Q::ROWU + g;
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = bias_s[wave * 32 + mfma::rowmap(r, g)];
+#pragma unroll
+    for (int ks = 0; ks < Q::KS; ++ks) acc = mfma::mma(wf[ks], xb[2 * ks], acc);
+    // stores past the last row are dropped by the buffer's range, so that every tile counts two of them
+    const int64_t row0 = tile * 32;
+    const int have = (int)(a.M - row0 < 32 ? a.M - row0 : 32);
+    const auto rows = __builtin_amdgcn_make_buffer_rsrc(static_cast<uint16_t *>(a.out[z]) + row0 * a.O, 0, have * a.O * 2, 0x00027000);
+    u32x4 s0, s1;
+    mfma::tile_natural(acc, s0, s1);
+    const int at = (i * a.O + o0 + 16 * g) * 2;
+    __builtin_amdgcn_raw_buffer_store_b128(s0, rows, at, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(s1, rows, at + 16, 0, 0);
+    stage = (stage + 1) % Q::STAGES;
+  }
+}
+
 bool linear_serves(const GemmArgs &a, int nsets, size_t elem_bytes) {
   if (elem_bytes != 2 || a.ks != 0 || a.act != 0) return false;  // activations: the tiled kernel
   if (a.K != 128 && a.K != 256 && a.K != 512) return false;
@@ -335,12 +418,17 @@ int linear_launch(const GemmArgs &a, int nsets, int num_cu, hipStream_t st) {
   // lean form.  The second one of the lean form pays from eight tiles per CU on, where its weights (128 KB) are covered:
   // 256 -> 256, two against one: 16 384 rows 12.0 / 9.1 us, 32 768 14.5 / 12.5; from 65 536 rows against one of the other
   // form: 19.5 / 20.8, 1 048 576 rows 211 / 227.
-  const bool lean = a.K == 256 && a.O % 256 == 0 && a.pack_tpb == 0 && !a.out_pack[0] && !a.out_pack[nsets - 1];
+  const bool natural = a.O % 256 == 0 && a.pack_tpb == 0 && !a.out_pack[0] && !a.out_pack[nsets - 1], lean = a.K == 256 && natural;
   const int64_t sides = (a.O + 255) / 256 * nsets;
   int64_t gx = (a.K == 128 || (lean && ntiles * sides >= 8 * (int64_t)num_cu) ? 2 : 1) * (int64_t)num_cu / sides;
   if (gx < 1) gx = 1;
   if (gx > ntiles) gx = ntiles;
   const dim3 grid((unsigned)gx, (unsigned)((a.O + 255) / 256), (unsigned)nsets), block((unsigned)(waves * 64));
+  if (a.K == 512 && natural) {
+    if (int rc = allow_dynamic_lds(rows_linear_ring_kernel, LinearRing::BYTES)) return rc;
+    hipLaunchKernelGGL(rows_linear_ring_kernel, grid, block, LinearRing::BYTES, st, a);
+    return launch_status();
+  }
   const size_t lds = (size_t)2 * 32 * (a.K / 8 + 1) * 16;  // only K = 512 exceeds the default limit
   if (int rc = allow_dynamic_lds(rows_linear_kernel<32, false>, a.K == 512 ? lds : 0)) return rc;
   switch (a.K) {

@@ -1102,6 +1102,20 @@ def test_row_gemm_of_256_inputs_with_two_workgroups_per_cu(rows, c_out, bias):
     assert (err <= 2.0 ** -8 * want.abs() + 1e-3).all()
 
 
+@pytest.mark.parametrize("rows,c_out,bias", [(4096, 256, True), (8193, 256, False), (12320, 512, True), (41007, 256, True)])
+def test_row_gemm_of_512_inputs_through_the_ring(rows, c_out, bias):
+    """Half the workgroups of a round, a second round of one row, more tiles per workgroup than the ring has stages (both widths)."""
+    announce("row GEMM, 512 inputs", rows, c_out, bias)
+    torch.manual_seed(rows)
+    x, w = torch.randn(1, rows, 512, device="cuda").bfloat16(), torch.randn(c_out, 512, device="cuda").bfloat16()
+    b = torch.randn(c_out, device="cuda") if bias else None
+    y = PF.rows_gemm(x, w, b, PF.LayerDims(1, rows, 512, 16, 32, 64), 512, c_out)
+    want = x[0].double().cpu() @ w.double().cpu().t() + (b.double().cpu() if bias else 0)
+    # as above: one rounding to bf16
+    err = (y[0].double().cpu() - want).abs()
+    assert (err <= 2.0 ** -8 * want.abs() + 1e-3).all()
+
+
 @pytest.mark.parametrize("rows,Fh", [(1, 64), (300, 192), (2500, 1024), (14450, 1024), (32768, 1024), (40000, 1024), (70000, 512)])
 def test_hidden_gradients_do_not_depend_on_how_the_hidden_units_are_split(rows, Fh):
     """Rows choose how many parts the hidden units are taken in; each row's values have the same bits as in a call of few rows."""
