@@ -458,6 +458,16 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(Sums a) {
   else sum_rows_of<32, 1>(o, blockIdx.y, part);
 }
 
+// f(number of steps, first step) over n steps in batches of eight, four and one: a batch's loads are issued together.  (A loop
+// around matrix instructions whose length is not known when it is compiled is not unrolled, whatever it is asked.)
+template <class F>
+__device__ __forceinline__ void in_batches(int n, F &&f) {
+  int k = 0;
+  for (; k + 8 <= n; k += 8) f(std::integral_constant<int, 8>{}, k);
+  if (k + 4 <= n) f(std::integral_constant<int, 4>{}, k), k += 4;
+  for (; k < n; ++k) f(std::integral_constant<int, 1>{}, k);
+}
+
 // ------------------------------------------------------------------------------------------------
 // token_grad_kernel: what the layer's output gradient says about the slice tokens and out_linear, from the sums
 // P[b][h S + s][c] = sum_n w[n, h, s] dy[n, c] (the packed product above) instead of from per-point d out_x and out_x:
@@ -465,8 +475,8 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(Sums a) {
 //   d W_out[c, 32 h + d] = sum_b sum_s P[b, h, s, c] tok'[b, h, s, d]        the others, one per (`cb` batch elements, h,
 //                                                                            32 rows c): a partial result per `cb` elements
 // Four waves per 32 x 32 result tile on fp32 MFMA, each a quarter of the reduction, added up in order through LDS.  Bound
-// by latency (P is a few hundred KB): the quarters' loads are all in flight at once, which takes 60 us (one wave per
-// tile) to 15 us at B = 1, S = 64, C = 256.
+// by latency (P is a few hundred KB): the quarters took 60 us (one wave per tile) to 14 us at B = 1, S = 64, C = 256,
+// their loads in batches that are issued together (in_batches) to 7.
 // ------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void token_grad_kernel(const float *__restrict__ P, const uint16_t *__restrict__ w_out,
                                                          const float *__restrict__ out_token, float *__restrict__ d_token,
@@ -485,23 +495,39 @@ __global__ __launch_bounds__(256) void token_grad_kernel(const float *__restrict
     const int s = 32 * st + i, cw = C / 4;
     const float *row = P + ((int64_t)bh * S + (s < S ? s : S - 1)) * C + wave * cw + 4 * g;
     const uint16_t *wcol = w_out + (int64_t)(wave * cw + 4 * g) * HD + 32 * h + i;
-#pragma unroll 8
-    for (int c = 0; c < cw; c += 8) {  // lane half g supplies c + 4 g .. + 3, one pair (c + m, c + 4 + m) per MFMA
-      const f32x4 p4 = *reinterpret_cast<const f32x4 *>(row + c);
+    in_batches(cw / 8, [&](auto n_, int k0) {  // lane half g supplies c + 4 g .. + 3, one pair (c + m, c + 4 + m) per MFMA
+      constexpr int n = decltype(n_)::value;
+      f32x4 p4[n];
+      uint16_t w[n][4];
 #pragma unroll
-      for (int m = 0; m < 4; ++m)
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(p4[m], bf16_bits_to_f32(wcol[(int64_t)(c + m) * HD]), acc, 0, 0, 0);
-    }
+      for (int k = 0; k < n; ++k) {
+        const int c = 8 * (k0 + k);
+        p4[k] = *reinterpret_cast<const f32x4 *>(row + c);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) w[k][m] = wcol[(int64_t)(c + m) * HD];
+      }
+      __builtin_amdgcn_sched_barrier(0);  // or the loads move down to their products
+#pragma unroll
+      for (int k = 0; k < n; ++k)
+#pragma unroll
+        for (int m = 0; m < 4; ++m) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(p4[k][m], bf16_bits_to_f32(w[k][m]), acc, 0, 0, 0);
+    });
   } else {
-    const int sw = S / 4;
-    const int b_end = (chunk + 1) * cb < B ? (chunk + 1) * cb : B;
-    for (int b = chunk * cb; b < b_end; ++b) {
-      const int64_t at = ((int64_t)b * H + h) * S + wave * sw + g;
-      const float *p = P + at * C + c0 + i, *tk = out_token + at * 32 + i;
-#pragma unroll 8
-      for (int s = 0; s < sw; s += 2)
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(p[(int64_t)s * C], tk[s * 32], acc, 0, 0, 0);
-    }
+    const int sw = S / 4, steps = sw / 2, b0 = chunk * cb, b_end = b0 + cb < B ? b0 + cb : B;
+    in_batches((b_end - b0) * steps, [&](auto n_, int k0) {  // all batch elements of the chunk in one row of steps
+      constexpr int n = decltype(n_)::value;
+      float p[n], tk[n];
+#pragma unroll
+      for (int k = 0; k < n; ++k) {
+        const int b = b0 + (k0 + k) / steps, s = 2 * ((k0 + k) % steps);
+        const int64_t at = ((int64_t)b * H + h) * S + wave * sw + g + s;
+        p[k] = P[at * C + c0 + i];
+        tk[k] = out_token[at * 32 + i];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < n; ++k) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(p[k], tk[k], acc, 0, 0, 0);
+    });
   }
   if (wave > 0) {
 #pragma unroll
