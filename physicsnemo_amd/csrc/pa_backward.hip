@@ -175,9 +175,10 @@ __global__ __launch_bounds__(kAttnBwdThreads) void slice_attention_backward_kern
 // S = 128 does not leave room) in the caller's 2 S^2 floats per (b, h), which stay in the L2.
 // Bound by the latency of its ten dependent steps (B * H workgroups, 8 for one sample of an eight-head layer) and, each of
 // them running once, by fetching its code: the kernel above spends 155 us on S = 64, D = 32 at 8 workgroups, where a thread
-// walks its products one fma at a time through LDS reads; the tiles take 18 us (S = 32, D = 16: 12).  With a row of the
+// walks its products one fma at a time through LDS reads; the tiles took 18 us (S = 32, D = 16: 12), and with the
+// operands' loads issued together take 14.  With a row of the
 // softmax per wave instead of per eight lanes, and d tok as one product of three times the depth, it took 28 (17); with the
-// eight lanes' loops unrolled into registers and a tile product inlined per kind of job, 32 (25).
+// eight lanes' loops unrolled into registers and a tile product inlined per kind of job, 32 (25), where they took 18.
 // ------------------------------------------------------------------------------------------------
 constexpr int kAttnMfmaWaves = kAttnBwdThreads / 64;
 
@@ -234,15 +235,39 @@ __global__ __launch_bounds__(kAttnBwdThreads) void slice_attention_backward_mfma
     for (int r = 0; r < 16; ++r) dst[mfma::rowmap(r, g) * stride + i] = c[r] * scale;
   };
 
-  for (int u = t; u < d.SP * d.DP; u += kAttnBwdThreads) {
-    const int s = u / d.DP, e = u - s * d.DP;
-    const bool ok = s < S && e < D;
-    tok[s * D1 + e] = ok ? slice_token[((int64_t)bh * S + s) * D + e] : 0.f;
-    dO[s * D1 + e] = ok ? d_out_token[((int64_t)bh * S + s) * D + e] : 0.f;
-  }
-  for (int u = t; u < 3 * d.DP * d.DP; u += kAttnBwdThreads) {
-    const int row = u / d.DP, c = u - row * d.DP, m = row / d.DP, e = row - m * d.DP;
-    wq[row * D1 + c] = (e < D && c < D) ? w_qkv[(int64_t)(m * D + e) * D + c] : 0.f;
+  // thread (column t % 32, row t / 32) of tiles of 16 rows: 64 rows of both token arrays and 32 of each weight per trip, all
+  // fourteen loads on their way together
+  const int tr = t >> 5, trips = (d.SP + 63) / 64 > d.nD ? (d.SP + 63) / 64 : d.nD;
+  const int s_end = 8 * wave + (lane >> 3);  // the first row that this lane finishes
+  float norm = slice_norm && s_end < S ? slice_norm[(int64_t)bh * S + s_end] : 1.f;
+  for (int e = t & 31; e < d.DP; e += 32) {
+    const int ec = e < D ? e : D - 1;  // elements beyond S and D: any that is there, kept as zero
+    for (int x = 0; x < trips; ++x) {
+      float a[4], b[4], w[6];
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+        const int s = 64 * x + 16 * n + tr;
+        const int64_t at = ((int64_t)bh * S + (s < S ? s : S - 1)) * D + ec;
+        a[n] = slice_token[at], b[n] = d_out_token[at];
+      }
+#pragma unroll
+      for (int n = 0; n < 6; ++n) {  // weight n / 2
+        const int row = 32 * x + 16 * (n & 1) + tr;
+        w[n] = w_qkv[((n >> 1) * D + (row < D ? row : D - 1)) * D + ec];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+        const int s = 64 * x + 16 * n + tr;
+        const bool ok = s < S && e < D;
+        if (s < d.SP) tok[s * D1 + e] = ok ? a[n] : 0.f, dO[s * D1 + e] = ok ? b[n] : 0.f;
+      }
+#pragma unroll
+      for (int n = 0; n < 6; ++n) {
+        const int row = 32 * x + 16 * (n & 1) + tr;
+        if (row < d.DP) wq[((n >> 1) * d.DP + row) * D1 + e] = row < D && e < D ? w[n] : 0.f;
+      }
+    }
   }
   __syncthreads();
   for (int job = wave; job < d.nS * 3 * d.nD; job += kAttnMfmaWaves) {  // q | k | v = tok W^T
@@ -322,9 +347,10 @@ __global__ __launch_bounds__(kAttnBwdThreads) void slice_attention_backward_mfma
     }
   }
   __syncthreads();
-  for (int s = 8 * wave + (lane >> 3); s < d.SP; s += 8 * kAttnMfmaWaves) {  // d num = d tok / nrm,  d nrm = -(d tok . tok) / nrm
+  for (int s = s_end; s < d.SP; s += 8 * kAttnMfmaWaves) {  // d num = d tok / nrm,  d nrm = -(d tok . tok) / nrm
     const bool row = s < S;
-    const float inv = slice_norm && row ? 1.f / slice_norm[(int64_t)bh * S + s] : 1.f;
+    if (s != s_end && slice_norm && row) norm = slice_norm[(int64_t)bh * S + s];
+    const float inv = row ? 1.f / norm : 1.f;
     float acc = 0.f;
     for (int e = l8; e < D; e += 8) {
       const int at = s * D1 + e;
@@ -333,7 +359,7 @@ __global__ __launch_bounds__(kAttnBwdThreads) void slice_attention_backward_mfma
       if (row) d_num[((int64_t)bh * S + s) * D + e] = t3 * inv;
     }
     acc = sum8(acc);
-    if (slice_norm && row && l8 == 0) d_norm[(int64_t)bh * S + s] = -acc / slice_norm[(int64_t)bh * S + s];
+    if (slice_norm && row && l8 == 0) d_norm[(int64_t)bh * S + s] = -acc / norm;
   }
 }
 
