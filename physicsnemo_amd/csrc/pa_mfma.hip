@@ -79,12 +79,12 @@ __global__ __launch_bounds__(256) void pack_params_kernel(pa_params p, u32x4 *__
       const int q = (int)((u - bp.wsl) >> 6);
       const int kk = q & 1, st = q >> 1;
       const int s = 32 * st + i;
+      float w[8];  // loaded whether the slice is there or not: a choice each is a trip to memory each
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint16_t lo = s < S ? to_bf16_bits(p.in_project_slice_weight[(int64_t)s * 32 + kperm(kk, g, 2 * j)]) : (uint16_t)0;
-        const uint16_t hi = s < S ? to_bf16_bits(p.in_project_slice_weight[(int64_t)s * 32 + kperm(kk, g, 2 * j + 1)]) : (uint16_t)0;
-        e[j] = (uint32_t)lo | ((uint32_t)hi << 16);
-      }
+      for (int j = 0; j < 8; ++j) w[j] = p.in_project_slice_weight[(int64_t)(s < S ? s : S - 1) * 32 + kperm(kk, g, j)];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        e[j] = s < S ? (uint32_t)to_bf16_bits(w[2 * j]) | ((uint32_t)to_bf16_bits(w[2 * j + 1]) << 16) : 0u;
     } else {
       int q = (int)((u - bp.wout) >> 6);
       const int kk = q & 1;
@@ -621,7 +621,8 @@ __global__ __launch_bounds__(256) void slice_reduce_kernel(const u32x4 *__restri
 // (v_mfma_f32_32x32x2_f32: A lane (i, g) holds A[i][k = g], B lane (i, g) holds B[k = g][i], C/D as above).
 // One workgroup per (b, h), one wave per tile of 32 slices; lane (i, g) of wave w owns slice s = 32w + i.
 //   tok[s][:]  = num[s][:] / (cnt[s] + 1e-2)                                    -> slice_token, slice_norm
-// Bound by latency: the weights come as float4 with the sums, one trip to memory, 9.2 us at S = 64 (as 48 single floats 11.5).
+// Bound by latency: the weights come as float4 with the sums, one trip to memory, 8.8 us at S = 64 (as 48 single floats 11.5,
+// the bias of the sums by a choice per value 9.2).
 //   q^T, k^T, v^T (32 e x 32 s) = Wq|k|v (A) . tok^T (B: lane <-> s, k <-> d = rowmap(r, g))    registers <-> e = rowmap(r, g)
 //   k, v -> LDS; scores^T (keys x queries) = k (A, from LDS) . q^T: register r of q^T is directly the B operand of
 //   the step whose reduction pair is d = rowmap(r, 0 / 1)
@@ -671,11 +672,16 @@ __global__ __launch_bounds__(64 * ((S + 31) / 32)) void slice_attention_kernel(c
   }
   float tk[16];  // tok[s][rowmap(r, g)]
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int d = rowmap(r, g);
-    const float num = fb ? fmaf(fb[d], wsum, src[d]) : src[d];
-    tk[r] = live ? num / cnt : 0.f;
+  for (int r = 0; r < 16; ++r) tk[r] = src[rowmap(r, g)];
+  if (fb) {  // one branch around all of them: sixteen choices of one load or two are sixteen trips to memory
+    float bias[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) bias[r] = fb[rowmap(r, g)];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) tk[r] = fmaf(bias[r], wsum, tk[r]);
   }
+#pragma unroll
+  for (int r = 0; r < 16; ++r) tk[r] = live ? tk[r] / cnt : 0.f;
   if (live) {
     if (slice_token) {
 #pragma unroll

@@ -16,7 +16,7 @@ namespace train {
 // torch's layout, 32 x 32 tiles turned around through LDS (grid x: tiles, y: taps):
 //   w_in   [projection][o][tap][c]          w_in_t  [c][taps - 1 - tap][projection HD + o]   (the transposed convolution)
 //   w_out  [c][o]                           w_out_t [o][c]
-// and, in the last kSmallBlocks workgroups, the float32 parameters side by side: the backward pass reads these copies, so that
+// and, in the last kSmallBlocks x kSmallParams workgroups, the float32 parameters side by side: the backward pass reads these copies, so that
 // the parameters themselves may change between the two passes.
 // ------------------------------------------------------------------------------------------------
 constexpr int kSmallBlocks = 8, kSmallParams = 10;
@@ -39,10 +39,10 @@ __global__ __launch_bounds__(256) void prepare_weights_kernel(PrepareArgs a) {
   id -= which * per;
   if (which > a.nproj) {
     if (blockIdx.y > 0) return;
-    const int k = (int)blockIdx.x - (a.nproj + 1) * per;
-#pragma unroll
-    for (int m = 0; m < kSmallParams; ++m)
-      for (int e = k * 256 + t; a.small[m] && e < a.n[m]; e += kSmallBlocks * 256) a.copies[a.at[m] + e] = a.small[m][e];
+    // kSmallBlocks workgroups for each of them: one after the other they are ten trips to memory
+    const int k = (int)blockIdx.x - (a.nproj + 1) * per, m = k / kSmallBlocks;
+    if (const float *src = a.small[m])
+      for (int e = k % kSmallBlocks * 256 + t; e < a.n[m]; e += kSmallBlocks * 256) a.copies[a.at[m] + e] = src[e];
     return;
   }
   const bool out = which == a.nproj;
@@ -260,7 +260,7 @@ int forward(const pa_shape &s, int weight_dtype, const pa_params &params, const 
   for (int m = 0; m < kSmallParams; ++m) pa.small[m] = small[m];
   small_plan(s, pl, pa.at, pa.n);
   pa.copies = reinterpret_cast<float *>(sv + sp.small);
-  const dim3 grid((unsigned)((pa.nproj + 1) * (s.C / 32) * s.H + kSmallBlocks), (unsigned)taps);
+  const dim3 grid((unsigned)((pa.nproj + 1) * (s.C / 32) * s.H + kSmallBlocks * kSmallParams), (unsigned)taps);
   if (weight_dtype == PA_F32) hipLaunchKernelGGL(prepare_weights_kernel<float>, grid, dim3(256), 0, st, pa);
   else hipLaunchKernelGGL(prepare_weights_kernel<bf16>, grid, dim3(256), 0, st, pa);
   int rc = launch_status();
