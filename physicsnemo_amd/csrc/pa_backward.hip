@@ -176,7 +176,7 @@ __global__ __launch_bounds__(kAttnBwdThreads) void slice_attention_backward_kern
 // Bound by the latency of its ten dependent steps (B * H workgroups, 8 for one sample of an eight-head layer) and, each of
 // them running once, by fetching its code: the kernel above spends 155 us on S = 64, D = 32 at 8 workgroups, where a thread
 // walks its products one fma at a time through LDS reads; the tiles took 18 us (S = 32, D = 16: 12), and with the
-// operands' loads issued together take 14.  With a row of the
+// operands' loads issued together take 15.  With a row of the
 // softmax per wave instead of per eight lanes, and d tok as one product of three times the depth, it took 28 (17); with the
 // eight lanes' loops unrolled into registers and a tile product inlined per kind of job, 32 (25), where they took 18.
 // ------------------------------------------------------------------------------------------------
