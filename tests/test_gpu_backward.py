@@ -1116,6 +1116,21 @@ def test_row_gemm_of_512_inputs_through_the_ring(rows, c_out, bias):
     assert (err <= 2.0 ** -8 * want.abs() + 1e-3).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,c_in,c_out,bias", [(1, 1, 1, True), (63, 3, 5, False), (65, 5, 66, True), (130, 17, 64, True), (200, 33, 30, True)])
+def test_row_gemm_of_odd_inputs(dtype, rows, c_in, c_out, bias):
+    """Rows that are no whole 16-byte units: last rows, inputs and outputs of tiles of 64 x 16 x 64, one block of inputs and more."""
+    announce("row GEMM, odd inputs", dtype, rows, c_in, c_out, bias)
+    torch.manual_seed(rows)
+    x, w = torch.randn(1, rows, c_in, device="cuda").to(dtype), torch.randn(c_out, c_in, device="cuda").to(dtype)
+    b = torch.randn(c_out, device="cuda") if bias else None
+    y = PF.rows_gemm(x, w, b, PF.LayerDims(1, rows, c_in, 1, 1, 1), c_in, c_out)
+    want = x[0].double().cpu() @ w.double().cpu().t() + (b.double().cpu() if bias else 0)
+    # float32 sums of at most 34 terms of a few units each; bf16 results are rounded once
+    err = (y[0].double().cpu() - want).abs()
+    assert (err <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -22) * want.abs() + 1e-4).all()
+
+
 @pytest.mark.parametrize("rows,Fh", [(1, 64), (300, 192), (2500, 1024), (14450, 1024), (32768, 1024), (40000, 1024), (70000, 512)])
 def test_hidden_gradients_do_not_depend_on_how_the_hidden_units_are_split(rows, Fh):
     """Rows choose how many parts the hidden units are taken in; each row's values have the same bits as in a call of few rows."""
