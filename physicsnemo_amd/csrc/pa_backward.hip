@@ -573,13 +573,13 @@ __global__ __launch_bounds__(256) void slice_softmax_backward_kernel(
   for (int s = j_own; s < S; s += tpr) {
     const float ws = weight(s);
     dot = fmaf(ws, dwl[r_own * S1 + s], dot);
-    mean = fmaf(ws, lgl[r_own * S1 + s], mean);
+    if (ws != 0.f) mean = fmaf(ws, lgl[r_own * S1 + s], mean);  // a logit of no weight may be -inf
   }
   for (int off = tpr >> 1; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64), mean += __shfl_xor(mean, off, 64);
   float tsum = 0.f;
   for (int s = j_own; s < S; s += tpr) {
-    const float dl = weight(s) * (dwl[r_own * S1 + s] - dot);
-    tsum = fmaf(dl, lgl[r_own * S1 + s] - mean, tsum);
+    const float ws = weight(s), dl = ws * (dwl[r_own * S1 + s] - dot);
+    if (ws != 0.f) tsum = fmaf(dl, lgl[r_own * S1 + s] - mean, tsum);
     dwl[r_own * S1 + s] = dl * inv_temp;
   }
   if constexpr (PLUS) {

@@ -5,6 +5,8 @@
 // and, one register per step, an operand whose reduction index runs over them in the order 4 g + r, g = 0 .. 3.
 #pragma once
 
+#include <float.h>
+
 #include "pa_mfma_ops.h"
 
 namespace pa {
@@ -36,8 +38,10 @@ __device__ __forceinline__ void exponent_scale(float temp, float &sc, float &sc_
   sc = uniform(hi);
   sc_low = uniform((fmaf(-hi, temp, kLog2e) + 1.92596299e-8f) / temp);  // log2(e) = kLog2e + 1.93e-8
 }
+// z <= 0 or NaN.  Where the power is a normal number, low is below 1e-4; from z sc = -FLT_MAX down it is +inf or, at z = -inf, NaN, and e
+// is 0: fminf makes 1 of either, so that a slice switched off by a bias of -inf or the lowest float has weight 0.
 __device__ __forceinline__ float exponential(float z, float sc, float sc_low) {
-  const float hi = z * sc, low = fmaf(z, sc_low, fmaf(z, sc, -hi)), e = __builtin_amdgcn_exp2f(hi);
+  const float hi = z * sc, low = fminf(fmaf(z, sc_low, fmaf(z, sc, -hi)), 1.f), e = __builtin_amdgcn_exp2f(hi);
   return fmaf(e * 0.69314718f, low, e);
 }
 

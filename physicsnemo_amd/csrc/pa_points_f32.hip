@@ -233,8 +233,9 @@ __global__ __launch_bounds__(512, 4) void point_backward_kernel(PointBackwardArg
     for (int st = 0; st < 2; ++st)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        z[st][r] = w[st][r] - mx;
-        w[st][r] = exponential(z[st][r], sc, sc_low);
+        const float arg = w[st][r] - mx;
+        w[st][r] = exponential(arg, sc, sc_low);
+        z[st][r] = fmaxf(arg, -FLT_MAX);  // 0 z is 0 for a slice of no weight; a NaN is in w
         sum += w[st][r];
         dot = fmaf(w[st][r], dw[st][r], dot);
         mean = fmaf(w[st][r], z[st][r], mean);

@@ -1594,3 +1594,28 @@ def test_float32_convolution_in_tall_and_flat_tiles(grid, C, O, B):
     got = PF.rows_gemm(x, w.movedim(1, -1).contiguous(), None, dims, C, O)
     want = torch.nn.functional.conv2d(x.double().transpose(1, 2).reshape(B, C, *grid).cpu(), w.double().cpu(), padding=1)
     assert_rel_l2(got, want.reshape(B, O, N).transpose(1, 2), "conv", tol=4e-6)
+
+
+@pytest.mark.parametrize("off", [-float("inf"), torch.finfo(torch.float32).min, -1e38])
+@pytest.mark.parametrize("dim,heads,dim_head,S,N", [(128, 8, 16, 32, 333), (48, 3, 16, 32, 17), (64, 4, 16, 64, 333), (96, 3, 32, 32, 65)])
+def test_fp32_training_with_a_slice_switched_off(dim, heads, dim_head, S, N, off):
+    """A slice of no weight adds nothing to any gradient: outputs and gradients are those of float64 with a finite bias that leaves it
+    no weight either (of -inf itself, autograd's d temperature is 0 inf = NaN).  The bounds are those of the layers without one."""
+    announce("fp32 training, a slice off", dim, heads, dim_head, S, N, off)
+    ref, hip = make_pair("irregular", dim, heads, dim_head, S, sharpen=2.0, temps=[0.2 + 5.6 * i / (heads - 1) for i in range(heads)])
+    hip.train()
+    x, dy = torch.randn(2, 2, N, dim, device="cuda")
+    with torch.no_grad():
+        hip.in_project_slice.bias[5] = -1e30
+    want = _oracle64_gradients(hip, "irregular", dim, heads, dim_head, S, x, dy)
+    ref.load_state_dict({k: v.cpu() for k, v in hip.state_dict().items()})
+    with torch.no_grad():
+        want_y = ref.double()(x.double().cpu())
+        hip.in_project_slice.bias[5] = off
+    xr = x.clone().requires_grad_(True)
+    y = hip(xr)
+    y.backward(dy)
+    assert ((y.double().cpu() - want_y).norm() / want_y.norm()).item() <= 6e-6
+    for n, got in [("x", xr.grad)] + [(n, p.grad) for n, p in hip.named_parameters()]:
+        err = (got.double() - want[n]).norm() / want[n].norm().clamp(min=1e-30)
+        assert err <= (1.7e-5 if n == "temperature" else 6e-6), (n, err.item())

@@ -516,3 +516,22 @@ def test_fp32_narrow_block_at_the_edges_of_its_tiles(C, H, B, N):
     with torch.no_grad():
         got, want = hip(x), ref(x.double())
     assert to.rel_l2(got.double(), want) < 1e-6
+
+
+@pytest.mark.parametrize("off", [-float("inf"), torch.finfo(torch.float32).min, -1e38])
+@pytest.mark.parametrize("C,H", [(64, 4), (64, 8), (32, 4), (32, 2)])
+def test_fp32_narrow_block_with_a_slice_switched_off(C, H, off):
+    """A slice bias of -inf, of the lowest float or far below the others gives the slice no weight; the bounds are those of every block."""
+    announce("fp32 narrow block, a slice off", C, H, off)
+    torch.manual_seed(C + H)
+    ref = to.OracleTransolverBlock(H, C, mlp_ratio=1, slice_num=32).eval()
+    hip = pn.TransolverBlock(H, C, 0.0, mlp_ratio=1, slice_num=32, use_te=False).eval()
+    with torch.no_grad():
+        ref.Attn.in_project_slice.bias[5] = off
+        ref.Attn.temperature.copy_(torch.linspace(0.4, 5.2, H).view(1, 1, H, 1))
+    hip.load_state_dict(ref.state_dict())
+    hip, ref = hip.cuda(), ref.double().cuda()
+    x = torch.randn(2, 129, C, device="cuda")
+    with torch.no_grad():
+        got, want = hip(x), ref(x.double())
+    assert torch.isfinite(want).all() and to.rel_l2(got.double(), want) < 1e-6
