@@ -186,8 +186,8 @@ __device__ __forceinline__ void store_tile_natural(const f32x16 &v, uint16_t *ro
 // ------------------------------------------------------------------------------------------------
 // DEFER: the chunks hold bf16(exp2(..)) without the division by their sum; the caller divides what it forms from them
 // by the sum of the same rounded values (one more MFMA column), which saves a pass over the S values per point.
-// SPLIT: wsl holds a second set of fragments behind the first, W_slice - bf16(W_slice).
-template <int S, bool DEFER = false, bool SPLIT = false>
+// PARTS: sets of fragments in wsl, W_slice as that many bf16 values (three hold a float32 value to the last bit).
+template <int S, bool DEFER = false, int PARTS = 1>
 __device__ __forceinline__ void slice_weights_of_tile(const u32x4 *__restrict__ wsl, const float *__restrict__ bsl,
                                                       u32x4 xm0, u32x4 xm1, float sc, bool valid, int lane, int g,
                                                       u32x4 (&chunk)[S / 16]) {
@@ -197,11 +197,10 @@ __device__ __forceinline__ void slice_weights_of_tile(const u32x4 *__restrict__ 
   for (int st = 0; st < ST; ++st) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) lg[st][r] = bsl[32 * st + rowmap(r, g)];
-    lg[st] = mma(wsl[(st * 2 + 0) * 64 + lane], xm0, lg[st]);
-    lg[st] = mma(wsl[(st * 2 + 1) * 64 + lane], xm1, lg[st]);
-    if constexpr (SPLIT) {
-      lg[st] = mma(wsl[((ST + st) * 2 + 0) * 64 + lane], xm0, lg[st]);
-      lg[st] = mma(wsl[((ST + st) * 2 + 1) * 64 + lane], xm1, lg[st]);
+#pragma unroll
+    for (int p = 0; p < PARTS; ++p) {
+      lg[st] = mma(wsl[((p * ST + st) * 2 + 0) * 64 + lane], xm0, lg[st]);
+      lg[st] = mma(wsl[((p * ST + st) * 2 + 1) * 64 + lane], xm1, lg[st]);
     }
   }
   float mx = -INFINITY;
@@ -237,23 +236,27 @@ __device__ __forceinline__ void slice_weights_of_tile(const u32x4 *__restrict__ 
 
 // W_slice as A operands and the slice bias in LDS, as slice_weights_of_tile reads them; the reduction index runs over
 // d in natural order (x_mid read from its rows) or in kperm order (PACKED_X: x_mid read as packed operand tiles);
-// SPLIT: followed by the fragments of what the rounding to bf16 left over
-template <int S, bool PACKED_X, bool SPLIT = false>
+// PARTS: followed by the fragments of what the rounding to bf16 left over, and of what that one's left
+template <int S, bool PACKED_X, int PARTS = 1>
 __device__ __forceinline__ void stage_slice_projection(const float *__restrict__ w_slice, const float *__restrict__ b_slice,
                                                        u32x4 *wsl, float *bsl) {
   constexpr int ST = (S + 31) / 32;
   for (int u = threadIdx.x; u < ST * 2 * 64; u += blockDim.x) {
     const int ul = u & 63, ui = ul & 31, ug = ul >> 5, f = u >> 6, st = f >> 1, kk = f & 1;
     const int s = 32 * st + ui;
-    bf16x8 e, rest;
+    float v[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float v = s < S ? w_slice[s * 32 + (PACKED_X ? kperm(kk, ug, j) : 16 * kk + 8 * ug + j)] : 0.f;
-      e[j] = (__bf16)v;
-      rest[j] = (__bf16)(v - (float)e[j]);
+    for (int j = 0; j < 8; ++j) v[j] = s < S ? w_slice[s * 32 + (PACKED_X ? kperm(kk, ug, j) : 16 * kk + 8 * ug + j)] : 0.f;
+#pragma unroll
+    for (int p = 0; p < PARTS; ++p) {
+      bf16x8 e;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        e[j] = (__bf16)v[j];
+        v[j] = isinf((float)e[j]) ? 0.f : v[j] - (float)e[j];  // nothing is left of an infinity
+      }
+      wsl[p * ST * 2 * 64 + u] = __builtin_bit_cast(u32x4, e);
     }
-    wsl[u] = __builtin_bit_cast(u32x4, e);
-    if constexpr (SPLIT) wsl[ST * 2 * 64 + u] = __builtin_bit_cast(u32x4, rest);
   }
   for (int s = threadIdx.x; s < ST * 32; s += blockDim.x) bsl[s] = s < S ? b_slice[s] : -1e30f;  // slices beyond S: weight 0
 }

@@ -327,12 +327,14 @@ __global__ __launch_bounds__(512) void slice_softmax_reduce_kernel(const uint16_
 // slice_softmax_reduce_kernel.  grid (G, B, head groups).
 //   x_mid^T (32 d x 32 pts) = W_x . x^T + b_x       (its bf16 halves are the logits' B operands, k in kperm order)
 //   fx_mid  (32 pts x 32 d) = x . W_fx^T + b_fx     (its bf16 halves are the token sums' A operands: k = points)
-// and from there on the arithmetic of that kernel, with W_slice as two bf16 halves (it is float32 where the stages run one
-// by one).  x_mid, fx_mid, the weights and the token sums are rounded where those stages round them: the first three to
-// bf16, the sums not.
+// and from there on the arithmetic of that kernel, with W_slice as three bf16 parts, all bits of the float32 value that the
+// stages multiply.  x_mid, fx_mid, the weights and the token sums are rounded where those stages round them: the first three
+// to bf16, the sums not; the logits, which the stages store as bf16, stay float32: tokens 0.50-0.64 as far from float64.
+// Against a float64 computation with the same roundings they are 4e-7 to 4e-6 off, with two parts 3e-6 to 5e-5.
 // What bounds it: the softmax's vector work, S/2 exponentials a lane and tile.  Stage by stage the same work wrote and
 // read 2 x 2 HD + 6 HS bytes a point that it forms here in registers: 65 536 points of 3 channels, 8 heads, 64 slices,
-// with the sum of the partials 259 -> 38 us (of it 20 for the tiles, 3 a launch); 8 points of 16 channels 43 -> 12.
+// with the sum of the partials 259 -> 38 us (of it 20 for the tiles, 3 a launch); 8 points of 16 channels 43 -> 12.  This
+// kernel alone, two parts of W_slice / three: 65 536 points 26.9 / 27.4, 262 144 points 66 / 70.
 // ------------------------------------------------------------------------------------------------
 template <int S>
 __global__ __launch_bounds__(512) void thin_tokens_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w_x,
@@ -344,7 +346,7 @@ __global__ __launch_bounds__(512) void thin_tokens_kernel(const uint16_t *__rest
                                                           const float *__restrict__ temperature,
                                                           float *__restrict__ partials, int64_t N, int tpb, int C, int H) {
   constexpr int ST = (S + 31) / 32, NCH = S / 16, D1 = 33;
-  __shared__ u32x4 wsl[2 * ST * 2 * 64];
+  __shared__ u32x4 wsl[3 * ST * 2 * 64];
   __shared__ float bsl[ST * 32], bxs[8 * 32];
   const int tid = threadIdx.x, lane = tid & 63, i = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -372,7 +374,7 @@ __global__ __launch_bounds__(512) void thin_tokens_kernel(const uint16_t *__rest
   const u32x4 wx = row_part(w_x + (int64_t)(h * 32 + i) * C), wf = row_part(w_fx + (int64_t)(h * 32 + i) * C);
   if (lane < 32) bxs[wave * 32 + lane] = b_x[h * 32 + lane];  // in LDS: 16 registers a lane otherwise
   const float bf = b_fx[h * 32 + i];
-  stage_slice_projection<S, true, true>(w_slice, b_slice, wsl, bsl);
+  stage_slice_projection<S, true, 3>(w_slice, b_slice, wsl, bsl);
   __syncthreads();
   const float sc = kLog2e / clamp_temperature(temperature[h]);
   u32x4 sel[2];
@@ -407,7 +409,7 @@ __global__ __launch_bounds__(512) void thin_tokens_kernel(const uint16_t *__rest
     const u32x4 xm0 = pack_half<0>(ax), xm1 = pack_half<1>(ax), f0 = pack_half<0>(af), f1 = pack_half<1>(af);
     if (t + (int)gridDim.x < tpb) xr = fetch(t + gridDim.x);  // the next tile's rows under this one's softmax
     u32x4 chunk[NCH];
-    slice_weights_of_tile<S, false, true>(wsl, bsl, xm0, xm1, sc, valid, lane, g, chunk);
+    slice_weights_of_tile<S, false, 3>(wsl, bsl, xm0, xm1, sc, valid, lane, g, chunk);
 #pragma unroll
     for (int st = 0; st < ST; ++st) {
       f32x16 tr;
