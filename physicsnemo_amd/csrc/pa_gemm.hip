@@ -956,9 +956,9 @@ static int conv_launch(const GemmArgs &a, int nsets, hipStream_t st) {
 
 // float32: one workgroup per CU in either form, so a round of 128-row workgroups takes twice the matrix time of a round of 64-row
 // ones, 10 % behind that rate with its two waves per SIMD against 20 % with one: whichever needs less for its whole rounds.
-static bool conv_tall(const GemmArgs &a, int nsets) {
-  const int64_t cols = a.O / 128 * nsets, tall = ((a.M + 127) / 128 * cols + 255) / 256, flat = ((a.M + 63) / 64 * cols + 255) / 256;
-  return 2 * 11 * tall <= 12 * flat;
+static bool conv_tall(const GemmArgs &a, int nsets, int num_cu) {
+  auto rounds = [&](int64_t rows) { return ((a.M + rows - 1) / rows * (a.O / 128) * nsets + num_cu - 1) / num_cu; };
+  return 2 * 11 * rounds(128) <= 12 * rounds(64);
 }
 
 bool serves(const GemmArgs &a, int nsets, size_t elem_bytes) {
@@ -990,17 +990,19 @@ static int launch_n(const GemmArgs &a, int nsets, hipStream_t st) {
   return launch_t<T, 2>(a, nsets, st);
 }
 
+static int device_cus() {
+  int dev = 0, cus = 256;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    cus = 256;
+  return cus;
+}
+
 int launch(const GemmArgs &a, int nsets, int dtype, hipStream_t st) {
-  if (dtype == PA_BF16 && linear_serves(a, nsets, 2)) {
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-      cus = 256;
-    return linear_launch(a, nsets, cus, st);
-  }
+  if (dtype == PA_BF16 && linear_serves(a, nsets, 2)) return linear_launch(a, nsets, device_cus(), st);
   if (dtype == PA_BF16 && conv_serves<bf16>(a, nsets)) return conv_launch<bf16, false>(a, nsets, st);
   if (dtype == PA_F32 && conv_serves<float>(a, nsets))
-    return conv_tall(a, nsets) ? conv_launch<float, true>(a, nsets, st) : conv_launch<float, false>(a, nsets, st);
+    return conv_tall(a, nsets, device_cus()) ? conv_launch<float, true>(a, nsets, st) : conv_launch<float, false>(a, nsets, st);
   return dtype == PA_F32 ? launch_n<float>(a, nsets, st) : launch_n<bf16>(a, nsets, st);
 }
 
