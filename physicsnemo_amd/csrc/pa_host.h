@@ -100,9 +100,11 @@ struct Sums {
   // few elements; small results have too few elements to fill the chip and split the partials instead, 32 ways.
   void add(const float *src, float *dst, int64_t n, int64_t G, int taps = 1, int64_t OB = 1) {
     const bool units = n % 4 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0;
-    // A workgroup takes 256 neighbouring ob of one oa, all taps, where there are enough of those: 512 x 256 x 9 elements
-    // 15.6 us against 20.1 by rows, 256 x 128 x 9 19.1 against 15.7 (lanes < 0)
-    if (units && taps > 1 && OB % 256 == 0 && n >= 1 << 20) {
+    // A workgroup takes 256 neighbouring ob of one oa, all taps, where there are enough of those (lanes < 0): three for every two
+    // CUs.  By taps / by rows, us, results of 256, 320, 384, 448, 512 workgroups: 9 taps, 14 partials 11.6 / 10.3, 13.1 / 11.9,
+    // 13.8 / 13.9, 14.2 / 17.2, 15.2 / 18.4; 25 taps 19.6 / 19.6, 21.2 / 21.8, 22.5 / 25.3 (OB = 512: 22.4 / 20.5), 24.2 / 29.5,
+    // 26.1 / 33.0; 27 taps 24.9 / 23.7, 17.5 / 21.4, 19.0 / 25.9, 20.2 / 28.9, 22.2 / 32.6.  With 128 they take 1.7 to 1.9 times as long.
+    if (units && taps > 1 && OB % 256 == 0 && n / (taps * 256) >= 384) {
       r[count++] = One{src, dst, n, blocks, (int)G, taps, (int)OB, -1};
       blocks += n / (taps * 256);
       by_taps = true;
