@@ -323,8 +323,9 @@ __global__ __launch_bounds__(512, LEAN ? 4 : 2) void rows_linear_kernel(GemmArgs
 // 1 024 bytes; rows lie 16 bytes more apart, so that the lanes of an access phase (32 rows, one unit) fall on different banks.
 // Loads and stores leave the counter in order: behind a tile's four loads a wave has issued the loads of up to two tiles and the two
 // stores each of up to three.  Bound by HBM: 1 048 576 rows into 256 columns, with rows_linear_kernel / here, in a layer's training step
-// 412 / 297 us (5.4 TB/s); called again and again 4 096 rows 11.1 / 10.4, 30 000 18.3 / 18.5, 65 536 31.4 / 31.6, 131 072 50.4 / 46.0,
-// 262 144 93 / 85 (512 columns 166 / 143).
+// 412 / 297 us (5.4 TB/s); called again and again, the two in turn, 4 096 rows (the fewest that come here) 11.1 / 10.5, 12 000 13.5 / 13.3,
+// 30 000 18.3 / 18.5, 65 536 27.3 / 27.0, 131 072 49.2 / 45.0, 262 144 94 / 85; into 512 columns 11.4 / 10.9, 16.4 / 15.5, 26.9 / 24.8,
+// 44.4 / 41.7, 86 / 76, 168 / 147: 1 % slower at one of twelve sizes (30 000 x 256), which is no reason for a line.
 // ------------------------------------------------------------------------------------------------
 struct LinearRing {
   static constexpr int K = 512, KS = K / 16, ROWU = K / 8 + 1, TILE = 32 * ROWU * 16, STAGES = 4, BYTES = STAGES * TILE + 256 * 4;
@@ -545,9 +546,9 @@ __global__ __launch_bounds__(512) void cols_gemm_kernel(const uint16_t *__restri
 // operand: consecutive lanes hold consecutive columns of a row, so natural row-major operands need no transposition.  A workgroup
 // (4 waves) owns a 128 x 128 block of P for one chunk of rows, wave w the 64 x 64 sub-block (w & 1, w >> 1); lane i takes columns
 // 2 i and 2 i + 1 of both operands, one 8-byte load each per pair of rows, for the 4 MFMAs (256 cycles) of the pair.  The operands
-// go straight from memory to registers, 16 pairs (32 rows) ahead: at this rate four waves ask for 8 bytes a cycle, the two waves
-// that share a column meet in the L1, and no wave waits for another.  Rows beyond the chunk and neighbours outside the grid
-// are out of the buffers' range and read as zero.
+// go straight from memory to registers, 16 pairs (32 rows) ahead: at this rate four waves ask for 16 bytes a cycle, 8 of them
+// beyond the L1 where the two waves that share a column meet there, and no wave waits for another.  Rows beyond the chunk and
+// neighbours outside the grid are out of the buffers' range and read as zero.
 // Row chunks come back as partials P[g][oa][ob] (fixed-order sum by the caller); col_sums[g][oa] = sum_m A[m][oa] from the same
 // pass.  Workgroups that share a chunk (the blocks of columns, the taps) run on one XCD, one after the other.
 // Bound by the float32 MFMAs: 4 x 85 x 85 grid points, 3 x 3 taps, 128 -> 2 x 128 (17 GFLOP) 149 us, 128 x 128 over 28 900 rows 16 us;

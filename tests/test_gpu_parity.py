@@ -535,3 +535,40 @@ def test_fp32_narrow_block_with_a_slice_switched_off(C, H, off):
     with torch.no_grad():
         got, want = hip(x), ref(x.double())
     assert torch.isfinite(want).all() and to.rel_l2(got.double(), want) < 1e-6
+
+
+@pytest.mark.parametrize("kind,dim,heads,dim_head,S,plus,dtype", [
+    ("irregular", 256, 8, 32, 64, False, torch.bfloat16), ("irregular", 128, 4, 32, 16, False, torch.bfloat16),   # one launch
+    ("irregular", 256, 8, 32, 128, False, torch.bfloat16), ("irregular", 512, 16, 32, 64, False, torch.bfloat16),  # staged
+    ("structured2d", 256, 8, 32, 64, False, torch.bfloat16), ("structured2d", 128, 8, 16, 32, False, torch.float32),
+    ("irregular", 256, 8, 32, 64, True, torch.bfloat16), ("irregular", 64, 4, 16, 32, True, torch.bfloat16),
+    ("irregular", 128, 4, 32, 48, False, torch.bfloat16), ("irregular", 96, 3, 32, 32, False, torch.float32),      # general
+])
+def test_slice_switched_off_by_bias(kind, dim, heads, dim_head, S, plus, dtype):
+    """A bias of -1e30, -1e38, the lowest float or -inf leaves a slice no weight in any of the softmax kernels, served and trained: the
+    same bits.  (-inf in training: test_fp32_training_with_a_slice_switched_off; in bf16, d temperature is autograd's 0 inf = NaN.)"""
+    announce("slice switched off", kind, dim, heads, dim_head, S, plus, dtype)
+    torch.manual_seed(dim + S)
+    kw = dict(heads=heads, dim_head=dim_head, slice_num=S, use_te=False, plus=plus)
+    hip = (pn.PhysicsAttentionIrregularMesh(dim, **kw) if kind == "irregular" else pn.PhysicsAttentionStructuredMesh2D(dim, (20, 17), **kw)).cuda()
+    x, dy = torch.randn(2, 2, 340, dim, device="cuda").to(dtype)
+    u = torch.rand(2, 340, heads, S, device="cuda").to(dtype)
+    lowest, first = torch.finfo(torch.float32).min, None
+    for off in (-1e30, -1e38, lowest, -float("inf")):
+        with torch.no_grad():
+            hip.in_project_slice.bias[5] = off
+            hip.temperature.copy_(torch.linspace(0.55, 4.5, heads).view_as(hip.temperature))
+        got = {}
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=dtype == torch.bfloat16):
+            with torch.no_grad():
+                got["served"] = hip.forward_with_noise(x, u) if plus else hip(x)
+            if off >= lowest:
+                xr = x.clone().requires_grad_(True)
+                hip.zero_grad(set_to_none=True)
+                got["y"] = hip.forward_with_noise(xr, u) if plus else hip(xr)
+        if off >= lowest:
+            got["y"].backward(dy)
+            got.update(x=xr.grad, **{n: p.grad for n, p in hip.named_parameters()})
+        first = first or got
+        for n, v in got.items():
+            assert torch.isfinite(v).all() and torch.equal(v, first[n]), (off, n)
