@@ -46,7 +46,7 @@ struct SumsArgs {
 
 // grid (groups, B, head groups), a wave per head of the group; a wave keeps its head's sums in registers over the tiles
 // blockIdx.x, + gridDim.x, ...  Bound by memory (x_mid and v read, w written: 256 bytes a point and head).
-// 4 x 7 225 points of eight heads 15.5 us, where a product, a softmax over rows and the general sums took 22 + 12 + 18; with the
+// 4 x 7 225 points of eight heads 15.8 us, where a product, a softmax over rows and the general sums took 22 + 12 + 18; with the
 // weights given 11.4 against 18.
 template <bool GIVEN>
 __global__ __launch_bounds__(512, 4) void point_sums_kernel(SumsArgs a) {
