@@ -376,6 +376,20 @@ __device__ __forceinline__ V sum_of_part(int part, int G, F &&load) {
   return s;
 }
 
+// sum of load(k) over k < PARTS (a power of two), halves added to halves: one after the other 32 parts of random signs were 1.3 to 1.6
+// times as far from float64
+template <int PARTS, class F>
+__device__ __forceinline__ float sum_of_parts(F &&load) {
+  float v[PARTS];
+#pragma unroll
+  for (int k = 0; k < PARTS; ++k) v[k] = load(k);
+#pragma unroll
+  for (int half = PARTS / 2; half > 0; half /= 2)
+#pragma unroll
+    for (int k = 0; k < half; ++k) v[k] += v[k + half];
+  return v[0];
+}
+
 template <int LANES, int V>
 __device__ __forceinline__ void sum_rows_of(const Sums::One &o, int64_t batch, float *part) {
   constexpr int PARTS = 256 / LANES, PER = LANES * V;
@@ -393,9 +407,7 @@ __device__ __forceinline__ void sum_rows_of(const Sums::One &o, int64_t batch, f
   __syncthreads();
   const int64_t e = e0 + threadIdx.x;
   if (threadIdx.x >= PER || e >= n) return;
-  float v = part[threadIdx.x];
-#pragma unroll
-  for (int k = 1; k < PARTS; ++k) v += part[k * PER + threadIdx.x];
+  const float v = sum_of_parts<PARTS>([&](int k) { return part[k * PER + threadIdx.x]; });
   int64_t at = batch * n + e;
   if (o.taps > 1) {
     const int64_t oa = e / (o.taps * (int64_t)o.OB), rest = e - oa * o.taps * o.OB, tap = rest / o.OB, ob = rest - tap * o.OB;
@@ -431,10 +443,7 @@ __device__ __forceinline__ void sum_taps_of(const Sums::One &o, float *part) {
     __syncthreads();
     for (int e = threadIdx.x; e < PER * nt; e += 256) {
       const int ob = e / nt, t = e - ob * nt;
-      float v = part[t * PER + ob];
-#pragma unroll
-      for (int k = 1; k < PARTS; ++k) v += part[(k * K + t) * PER + ob];
-      dst[ob * o.taps + t0 + t] = v;
+      dst[ob * o.taps + t0 + t] = sum_of_parts<PARTS>([&](int k) { return part[(k * K + t) * PER + ob]; });
     }
   }
 }

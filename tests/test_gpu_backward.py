@@ -441,6 +441,21 @@ def test_totals_of_partial_products(rows, ca, cb):
     assert torch.equal(sums, a.double().sum(0).float())
 
 
+@pytest.mark.parametrize("rows,ca,cb", [(30011, 256, 64), (32768, 1024, 256), (50000, 512, 256)])
+def test_totals_add_their_parts_in_halves(rows, ca, cb):
+    """Sums of random values over the rows, in up to 32 parts: 6.1e-8 to 6.5e-8 off float64 with halves added to halves, 1.0e-7 to
+    1.1e-7 with one part after the other, whose roundings a sum of that many values of one size adds up (7.0e-8 to 7.5e-8: eight
+    parts)."""
+    announce("totals in halves", rows, ca, cb)
+    square = 0.0
+    for seed in range(6):
+        torch.manual_seed(seed)
+        a, b = (torch.randn(rows, c, device="cuda").bfloat16() for c in (ca, cb))
+        want = a.double().sum(0)
+        square += ((PF.cols_gemm(a, b, col_sums=True)[1] - want).norm() / want.norm()).item() ** 2 / 6
+    assert square ** 0.5 <= 7.5e-8, square ** 0.5
+
+
 @pytest.mark.parametrize("dtype,C,O", [(torch.bfloat16, 256, 512), (torch.bfloat16, 128, 128), (torch.float32, 128, 256),
                                        (torch.float32, 36, 20)])
 @pytest.mark.parametrize("grid,k", [((13, 9), 3), ((40, 33), 5), ((4, 6, 5), 3), ((1, 50), 3)])
