@@ -527,9 +527,8 @@ __global__ __launch_bounds__(NS == 1 ? 512 : 256) void slice_partial_kernel(cons
 
 // ------------------------------------------------------------------------------------------------
 // combine_partials_kernel: second pass of the reduction, parallel over outputs.  grid (ceil(n_out/64), B*H);
-// 64 outputs x 4 quarter-ranges of the G partials per workgroup; each thread adds its quarter in four sums, every fourth partial
-// each, (a0 + a1) + (a2 + a3), and the quarters are then added in a fixed order ((q0 + q1) + q2) + q3: bit-reproducible, no
-// atomics.  (As one sum a quarter of 512 partials is a chain of 128 roundings.)
+// 64 outputs x 4 quarter-ranges of the G partials per workgroup; each thread adds its quarter in index order,
+// the four quarter sums are then added in a fixed order ((q0 + q1) + q2) + q3: bit-reproducible, no atomics.
 // Bound by the latency of the partials, which other XCDs wrote: 16 of a thread's loads are in flight at once.  256 partials
 // of 8 x 2 112 floats 5.1 us; one load at a time 17.5.
 // ------------------------------------------------------------------------------------------------
@@ -543,18 +542,18 @@ __global__ __launch_bounds__(256) void combine_partials_kernel(const float *__re
   const int bh = blockIdx.y;
   const int per = (G + 3) / 4;
   const int g0 = q * per, g1 = min(G, g0 + per);
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  float acc = 0.f;
   if (o < n_out) {
     const float *src = partials + (int64_t)bh * n_out + o;
-    for (int g = g0; g < g1; g += kAhead) {  // kAhead loads in flight
+    for (int g = g0; g < g1; g += kAhead) {  // kAhead loads in flight, added in index order
       float v[kAhead];
 #pragma unroll
       for (int u = 0; u < kAhead; ++u) v[u] = src[(int64_t)min(g + u, g1 - 1) * partial_stride];
 #pragma unroll
-      for (int u = 0; u < kAhead; ++u) acc[u & 3] += g + u < g1 ? v[u] : 0.f;
+      for (int u = 0; u < kAhead; ++u) acc += g + u < g1 ? v[u] : 0.f;
     }
   }
-  quarter[q][l] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+  quarter[q][l] = acc;
   __syncthreads();
   if (q == 0 && o < n_out)
     combined[(int64_t)bh * n_out + o] = ((quarter[0][l] + quarter[1][l]) + quarter[2][l]) + quarter[3][l];
@@ -683,21 +682,20 @@ __global__ __launch_bounds__(32 * kNarrowSlices) void narrow_combine_attn_kernel
   float w[(3 * D * D + T - 1) / T];
 #pragma unroll
   for (int k = 0; k < (3 * D * D + T - 1) / T; ++k) w[k] = k * T + t < 3 * D * D ? w_qkv[k * T + t] : 0.f;
-  // a thread adds up four neighbouring sums of a quarter of the partials, kAhead of them in flight: one trip for 64
+  // a thread adds up four neighbouring sums of a quarter of the partials in index order, kAhead of them in flight: one trip for 64
   const int per = (G + kParts - 1) / kParts, pt = t / NQ, o4 = t - pt * NQ, g0 = pt * per, g1 = min(G, g0 + per);
   if (pt < kParts) {
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
-    const f32x4 *src = reinterpret_cast<const f32x4 *>(partials + (int64_t)bh * NOUT) + o4;  // NOUT and the stride: whole ones
-    f32x4 acc[4] = {};
+    const float4 *src = reinterpret_cast<const float4 *>(partials + (int64_t)bh * NOUT) + o4;  // NOUT and the stride: whole float4
+    float4 acc{0.f, 0.f, 0.f, 0.f};
     for (int g = g0; g < g1; g += kAhead) {
-      f32x4 v[kAhead];
+      float4 v[kAhead];
 #pragma unroll
       for (int u = 0; u < kAhead; ++u) v[u] = src[(int64_t)min(g + u, g1 - 1) * (partial_stride / 4)];
 #pragma unroll
       for (int u = 0; u < kAhead; ++u)
-        if (g + u < g1) acc[u & 3] += v[u];
+        if (g + u < g1) acc.x += v[u].x, acc.y += v[u].y, acc.z += v[u].z, acc.w += v[u].w;
     }
-    reinterpret_cast<f32x4 *>(part[pt])[o4] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    reinterpret_cast<float4 *>(part[pt])[o4] = acc;
   }
 #pragma unroll
   for (int k = 0; k < (3 * D * D + T - 1) / T; ++k) {
