@@ -1,7 +1,7 @@
 // Weight gradients: products over the row axis  P[oa][ob] = sum_m A[m][oa] B[m][ob]  with A = d out, B = the layer's
 // input (or, for a grid convolution, its neighbours: one product per tap), plus the column sums of A (the bias
 // gradient).  The row axis is cut into chunks, each leaves one partial result, and one small kernel adds the partials up
-// in index order, so results do not depend on the launch.
+// in a fixed order, so results do not depend on the launch.
 //
 //   wgrad_kernel          bf16, up to 256 x 256 of P per workgroup, operands staged by direct global -> LDS loads
 //   narrow_wgrad_kernel   one side with at most 16 columns (input features, output channels), bf16 or fp32

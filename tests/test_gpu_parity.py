@@ -572,3 +572,20 @@ def test_slice_switched_off_by_bias(kind, dim, heads, dim_head, S, plus, dtype):
         first = first or got
         for n, v in got.items():
             assert torch.isfinite(v).all() and torch.equal(v, first[n]), (off, n)
+
+
+@pytest.mark.parametrize("S,D,N,tokens,norms", [(32, 16, 131072, 2.4e-7, 7.3e-8), (64, 32, 1048576, 4.5e-7, 1.2e-7)])
+def test_slice_sums_of_many_partials(S, D, N, tokens, norms):
+    """512 and 4 096 partial sums against float64.  A quarter of them in four sums: tokens 2.0e-7 and 3.3e-7 off, norms 5.4e-8 and 6.9e-8;
+    as one chain of 128 and 1 024 roundings 2.7e-7 and 6.0e-7, 9.2e-8 and 2.1e-7.  The bounds lie between."""
+    announce("slice sums of many partials", S, D, N)
+    square = [0.0, 0.0]
+    for seed in range(4):
+        torch.manual_seed(seed)
+        w, f = torch.rand(1, N, 1, S, device="cuda"), torch.randn(1, N, D, device="cuda")
+        got = PF.slice_reduce(w, f, PF.LayerDims(1, N, 16, 1, D, S))
+        count = w.double().sum(1) + 1e-2
+        want = (torch.einsum("bnhs,bnhd->bhsd", w.double(), f.double().view(1, N, 1, D)) / count[..., None], count)
+        for k in range(2):
+            square[k] += ((got[k].double() - want[k]).norm() / want[k].norm()).item() ** 2 / 4
+    assert square[0] ** 0.5 <= tokens and square[1] ** 0.5 <= norms, [v ** 0.5 for v in square]
